@@ -6,9 +6,21 @@
 
 #include "../../include/exhip.h"
 
+// Pinned chunks that host <-> device copies of a context go through (transfer.hip), taken when first needed.
+struct exhip_staging {
+    static constexpr int kChunks = 4;
+    void* chunk[kChunks] = {};
+    void* event[kChunks] = {};    // uploads: behind the last reader of the chunk; downloads: behind the copy into it
+    bool pending[kChunks] = {};   // uploads: the event has been recorded and not been waited for
+    int at = -1;                  // uploads: the chunk being filled, and how much of it is
+    size_t used = 0;
+};
+
 struct exhip_ctx {
     int device;
     hipStream_t stream;
+    exhip_staging up, down;
+    unsigned download_number = 0;  // of the last small download, the value its flag takes
     // scratch of the convolution's split reduction, grown on demand and kept until the context is destroyed
     int* split_acc = nullptr;
     size_t split_acc_bytes = 0;
@@ -23,6 +35,8 @@ constexpr int kSplitGroups = 256;
 int exhip_split_scratch(exhip_ctx* ctx, size_t acc_bytes, size_t tiles, int** acc, unsigned** count);
 
 void exhip_set_error(const char* fmt, ...);
+
+void exhip_release_staging(exhip_ctx* ctx);  // the stream has been drained
 
 // How exhip_conv_pack_weights lays this layer's weights out: output channels per slab, and whether it is the packed
 // first-layer form (4- or 8-byte pixels, one k-step per filter row).

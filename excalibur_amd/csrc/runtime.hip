@@ -76,6 +76,7 @@ extern "C" int exhip_init(int device, exhip_ctx** out) {
 extern "C" int exhip_destroy(exhip_ctx* ctx) {
     if (!ctx) return 0;
     (void)hipStreamSynchronize(ctx->stream);
+    exhip_release_staging(ctx);
     if (ctx->split_acc) (void)hipFree(ctx->split_acc);
     if (ctx->split_count) (void)hipFree(ctx->split_count);
     (void)hipStreamDestroy(ctx->stream);
@@ -108,24 +109,6 @@ extern "C" int exhip_free(exhip_ctx* ctx, void* dptr) {
 extern "C" int exhip_memset(exhip_ctx* ctx, void* dptr, int value, size_t bytes) {
     EXHIP_REQUIRE(ctx && (dptr || !bytes), "exhip_memset: NULL argument");
     if (bytes) EXHIP_CHECK(hipMemsetAsync(dptr, value, bytes, ctx->stream));
-    return 0;
-}
-
-extern "C" int exhip_memcpy_h2d(exhip_ctx* ctx, void* dst, const void* src, size_t bytes) {
-    EXHIP_REQUIRE(ctx && ((dst && src) || !bytes), "exhip_memcpy_h2d: NULL argument");
-    if (bytes) {
-        EXHIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
-        EXHIP_CHECK(hipStreamSynchronize(ctx->stream));  // src may be pageable and reused by the caller
-    }
-    return 0;
-}
-
-extern "C" int exhip_memcpy_d2h(exhip_ctx* ctx, void* dst, const void* src, size_t bytes) {
-    EXHIP_REQUIRE(ctx && ((dst && src) || !bytes), "exhip_memcpy_d2h: NULL argument");
-    if (bytes) {
-        EXHIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
-        EXHIP_CHECK(hipStreamSynchronize(ctx->stream));
-    }
     return 0;
 }
 

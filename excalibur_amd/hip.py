@@ -41,6 +41,10 @@ def lib():
         L.exhip_last_error.restype = ctypes.c_char_p
         L.exhip_conv_packed_bytes.restype = ctypes.c_size_t
         L.exhip_static_scratch_bytes.restype = ctypes.c_size_t
+        L.exhip_host_alloc.restype = ctypes.c_void_p
+        L.exhip_host_alloc.argtypes = [ctypes.c_size_t]
+        L.exhip_host_free.restype = None
+        L.exhip_host_free.argtypes = [ctypes.c_void_p]
         _lib = L
     return _lib
 

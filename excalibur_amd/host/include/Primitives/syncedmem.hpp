@@ -30,10 +30,16 @@ public:
     const Dtype* gpu_data();
     Dtype* mutable_cpu_data();
     Dtype* mutable_gpu_data();
+    // Replaces the contents by host bytes, on the device alone: returns when `src` has been read; the calling slot's stream
+    // finds the new contents. And the first `count` values as host bytes, without keeping a host copy.
+    void upload(const Dtype* src);
+    void download(Dtype* out, size_t count);
 
 private:
     void to_cpu();
     void to_gpu(bool will_overwrite);
+    void to_gpu_block();
+    void fetch(Dtype* out, size_t count);
     Dtype* cpu_ptr_ = nullptr;
     Dtype* gpu_ptr_ = nullptr;
     size_t size_;

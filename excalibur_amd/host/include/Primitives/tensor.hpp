@@ -29,6 +29,8 @@ public:
     const Dtype* gpu_data() const { return data_->gpu_data(); }
     Dtype* mutable_cpu_data() const { return data_->mutable_cpu_data(); }
     Dtype* mutable_gpu_data() const { return data_->mutable_gpu_data(); }
+    void upload(const Dtype* src) const { data_->upload(src); }    // see syncedmem
+    void download(Dtype* out) const { data_->download(out, static_cast<size_t>(count())); }
     unsigned long long writes() const { return data_->writes(); }  // mutable_*_data() calls so far
     void copy_from(const void* data, size_t size);
 

@@ -36,8 +36,7 @@ template <typename T>
 void set_input(std::shared_ptr<tensor<T>>& slot, int device, const void* data, const int* shape) {
     const std::vector<int> s{shape[0], shape[1], shape[2], shape[3]};
     if (!slot || slot->data_shape() != s) slot = std::make_shared<tensor<T>>(s, device, glasssix::memory::NCHW);
-    std::memcpy(slot->mutable_cpu_data(), data, sizeof(T) * static_cast<size_t>(slot->count()));
-    slot->gpu_data();  // upload now, so that timed runs start with the input resident in HBM
+    slot->upload(static_cast<const T*>(data));  // straight to the device: a forward finds its input there
 }
 
 template <typename T, typename P, typename M>
@@ -49,7 +48,7 @@ long get_blob(P& pipe, M& outs, const char* name, void* out, long capacity, int*
     const std::vector<int> s = t->data_shape();
     for (int i = 0; i < 4; ++i) shape[i] = s[i];
     const long n = t->count();
-    if (out && n <= capacity) std::memcpy(out, t->cpu_data(), sizeof(T) * static_cast<size_t>(n));
+    if (out && n <= capacity) t->download(static_cast<T*>(out));
     return n;
 }
 }  // namespace
@@ -165,8 +164,8 @@ extern "C" long exc_pipeline_get_kept(exc_pipeline* p, int back, const char* nam
     for (int i = 0; i < 4; ++i) shape[i] = s[i];
     const long n = t32 ? t32->count() : t16->count();
     if (out && n <= capacity) {
-        if (t32) std::memcpy(out, t32->cpu_data(), sizeof(float) * static_cast<size_t>(n));
-        else std::memcpy(out, t16->cpu_data(), sizeof(unsigned short) * static_cast<size_t>(n));
+        if (t32) t32->download(static_cast<float*>(out));
+        else t16->download(static_cast<unsigned short*>(out));
     }
     return n;
 }

@@ -129,14 +129,41 @@ void syncedmem<Dtype>::to_cpu() {
         break;
     case HEAD_AT_GPU:
         if (!cpu_ptr_) cpu_ptr_ = static_cast<Dtype*>(std::aligned_alloc(64, (bytes + 63) / 64 * 64 + 64));
-        // synchronises the stream of the slot the block was taken in (a pipeline's outputs: the pipeline's); a reader working
-        // in another slot may have queued the writer there, so that stream is drained as well
-        if (stream_slot() != slot_) EXHIP_FATAL(exhip_sync(device_context(device_)));
-        EXHIP_FATAL(exhip_memcpy_d2h(device_context(device_, slot_), cpu_ptr_, gpu_ptr_, bytes));
+        fetch(cpu_ptr_, size_);
         head_ = SYNCED;
         break;
     default: break;
     }
+}
+
+template <typename Dtype>
+void syncedmem<Dtype>::fetch(Dtype* out, size_t count) {
+    // synchronises the stream of the slot the block was taken in (a pipeline's outputs: the pipeline's); a reader working
+    // in another slot may have queued the writer there, so that stream is drained as well
+    if (stream_slot() != slot_) EXHIP_FATAL(exhip_sync(device_context(device_)));
+    EXHIP_FATAL(exhip_memcpy_d2h(device_context(device_, slot_), out, gpu_ptr_, count * sizeof(Dtype)));
+}
+
+template <typename Dtype>
+void syncedmem<Dtype>::upload(const Dtype* src) {
+    to_gpu_block();
+    EXHIP_FATAL(exhip_upload(device_context(device_), gpu_ptr_, src, size_ * sizeof(Dtype)));
+    head_ = HEAD_AT_GPU;
+    ++writes_;
+}
+
+template <typename Dtype>
+void syncedmem<Dtype>::download(Dtype* out, size_t count) {
+    if (head_ == HEAD_AT_GPU) fetch(out, count);
+    else std::memcpy(out, cpu_data(), count * sizeof(Dtype));
+}
+
+template <typename Dtype>
+void syncedmem<Dtype>::to_gpu_block() {
+    if (device_ < 0) LOG(FATAL) << "gpu_data() on a tensor created without a device";
+    if (gpu_ptr_) return;
+    slot_ = stream_slot();  // the block comes from, is first used in, and returns to the slot of this call
+    gpu_ptr_ = static_cast<Dtype*>(device_alloc(device_, size_ * sizeof(Dtype)));
 }
 
 // will_overwrite: the caller asks for the buffer to write all of it (mutable_gpu_data of a fresh blob, which is how every
@@ -144,21 +171,16 @@ void syncedmem<Dtype>::to_cpu() {
 // (gpu_data first) still yields zeros.
 template <typename Dtype>
 void syncedmem<Dtype>::to_gpu(bool will_overwrite) {
-    if (device_ < 0) LOG(FATAL) << "gpu_data() on a tensor created without a device";
+    if (head_ != UNINITIALIZED && head_ != HEAD_AT_CPU) return;
     const size_t bytes = size_ * sizeof(Dtype);
+    to_gpu_block();
     exhip_ctx* ctx = device_context(device_);
     switch (head_) {
     case UNINITIALIZED:
-        slot_ = stream_slot();  // the block comes from, is first used in, and returns to the slot of this call
-        gpu_ptr_ = static_cast<Dtype*>(device_alloc(device_, bytes));
         if (!will_overwrite) EXHIP_FATAL(exhip_memset(ctx, gpu_ptr_, 0, bytes));
         head_ = HEAD_AT_GPU;
         break;
     case HEAD_AT_CPU:
-        if (!gpu_ptr_) {
-            slot_ = stream_slot();
-            gpu_ptr_ = static_cast<Dtype*>(device_alloc(device_, bytes));
-        }
         EXHIP_FATAL(exhip_memcpy_h2d(ctx, gpu_ptr_, cpu_ptr_, bytes));
         head_ = SYNCED;
         break;

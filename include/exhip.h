@@ -42,6 +42,13 @@ int exhip_memset(exhip_ctx* ctx, void* dptr, int value, size_t bytes);
 int exhip_memcpy_h2d(exhip_ctx* ctx, void* dst, const void* src, size_t bytes);
 int exhip_memcpy_d2h(exhip_ctx* ctx, void* dst, const void* src, size_t bytes);
 int exhip_memcpy_d2d(exhip_ctx* ctx, void* dst, const void* src, size_t bytes);
+/* Host to device like exhip_memcpy_h2d, but returns as soon as src has been read (it goes through pinned staging): work
+ * queued on the context's stream afterwards finds the bytes, other streams have to wait for this one first. */
+int exhip_upload(exhip_ctx* ctx, void* dst, const void* src, size_t bytes);
+/* Pinned host memory for results (1 MiB and more), which exhip_memcpy_d2h fills without a copy by the host. Blocks are cached
+ * process-wide (at most 512 MiB idle, 1 GiB in all); NULL where there is none: use memory of your own then. Any thread. */
+void* exhip_host_alloc(size_t bytes);
+void exhip_host_free(void* ptr);
 int exhip_sync(exhip_ctx* ctx);
 const char* exhip_last_error(void);
 /* Switches for tests and development (no counterpart in the reference; the library reads nothing from the environment):

@@ -1,0 +1,85 @@
+"""Host <-> device copies (csrc/transfer.hip): every size class and its edges, unaligned ends, uploads queued without a
+wait, several threads at once, and results in pinned blocks of the pool."""
+import ctypes
+import threading
+
+import numpy as np
+import pytest
+
+from excalibur_amd import hip
+from excalibur_amd import pipeline as xp
+
+pytestmark = pytest.mark.gpu
+KB, MB = 1 << 10, 1 << 20
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = hip.Ctx(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("size", [1, 15, 4096, 64 * KB, 64 * KB + 1, 256 * KB, 256 * KB + 1, MB, 2 * MB + 5, 4 * MB, 4 * MB + 1, 19 * MB + 3])
+@pytest.mark.parametrize("offset", [0, 3])
+def test_bytes_arrive_in_both_directions(ctx, size, offset):
+    want = np.random.default_rng(size).integers(0, 256, size, dtype=np.uint8)
+    d = ctx.array(np.zeros(size + 64, np.uint8))
+    at, L = d.at(offset), hip.lib()
+    hip._check(L.exhip_memcpy_h2d(ctx.h, at.ptr, want.ctypes.data_as(ctypes.c_void_p), ctypes.c_size_t(size)))
+    got = np.zeros(size, np.uint8)
+    hip._check(L.exhip_memcpy_d2h(ctx.h, got.ctypes.data_as(ctypes.c_void_p), at.ptr, ctypes.c_size_t(size)))
+    assert np.array_equal(got, want)
+    whole = d.download()
+    assert np.array_equal(whole[offset:offset + size], want) and not whole[:offset].any() and not whole[offset + size:].any()
+    d.free()
+
+
+def test_uploads_do_not_wait_and_the_source_may_change_at_once(ctx):
+    """More uploads than the staging ring holds, queued behind each other from one reused host buffer."""
+    L, n, size = hip.lib(), 40, 900 * KB + 8
+    host, parts = np.empty(size, np.uint8), [ctx.empty((size,), np.uint8) for _ in range(n)]
+    for i, p in enumerate(parts):
+        host[:] = i + 1
+        hip._check(L.exhip_upload(ctx.h, p.ptr, host.ctypes.data_as(ctypes.c_void_p), ctypes.c_size_t(size)))
+    for i, p in enumerate(parts):
+        assert (p.download() == i + 1).all()
+        p.free()
+
+
+def test_threads_with_a_context_each_copy_at_once():
+    bad = []
+
+    def work(seed):
+        c = hip.Ctx(0)
+        for k in range(6):
+            want = np.random.default_rng(seed * 10 + k).integers(0, 256, 9 * MB + seed, dtype=np.uint8)
+            d = c.array(want)
+            if not np.array_equal(d.download(), want):
+                bad.append((seed, k))
+            d.free()
+        c.close()
+
+    threads = [threading.Thread(target=work, args=(s,)) for s in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+
+
+def test_results_in_pool_blocks_stay_their_holder_s(ctx):
+    xp.lib()
+    d = ctx.array(np.arange(MB, dtype=np.float32))
+    first = xp._host_array((MB,), np.float32)
+    hip._check(hip.lib().exhip_memcpy_d2h(ctx.h, first.ctypes.data_as(ctypes.c_void_p), d.ptr, ctypes.c_size_t(d.nbytes)))
+    second = xp._host_array((MB,), np.float32)   # the first block is still held: another one
+    second[:] = -1
+    assert np.array_equal(first, np.arange(MB, dtype=np.float32))
+    view = first[10:20]
+    del first
+    third = xp._host_array((MB,), np.float32)    # a view holds it as well
+    third[:] = -2
+    assert np.array_equal(view, np.arange(10, 20, dtype=np.float32))
+    assert hip.lib().exhip_host_alloc((1 << 30) + 1) is None   # beyond the bound: the caller's own memory
+    d.free()
