@@ -68,286 +68,226 @@ struct PwParams {
     int step[kMaxDirectSteps];   // offset | tap << kTapShift
 };
 
-__device__ __forceinline__ float fast_activation(float v, int act) {
-    if (act == 1) return (0.f > v) ? 0.f : v;
-    if (act == 3) { const float d = (0.f > v) ? 0.f : v; return d <= 6.f ? d : 0.f; }
-    return v;
-}
 __device__ __noinline__ float slow_activation(float v, int act) { return exhip_act(v, act); }
 
-template <int OP>
-__device__ __forceinline__ void post_activation_op(float (&v)[16], float alpha, float beta) {
-#pragma unroll
-    for (int e = 0; e < 16; ++e) v[e] = unary_value<OP>(exhip_h2f(exhip_f2h(v[e])), alpha, beta);
-}
+// ---- epilogue ----
+// What bounds a short launch is the length of one wave's chain, and the epilogue was half of it (stamps inside a 256 -> 256
+// layer on a 20 x 20 map, 19 000 cycles in all: 3 000 for 32 conditional one-word bias loads, 4 200 - 8 200 for the arithmetic
+// with a test per value and per lane, against 7 000 for the products). So: the per-channel parameters (scale, bias, BatchNorm,
+// PReLU slopes) are requested at the kernel's start, one coalesced load each with zeros beyond K, wait in the wave's own LDS
+// slice and are read back four channels at a time; layer kinds are one wave-uniform branch per 32 x 32 block with straight
+// code behind it, and tests against K exist only in a block that holds the ragged end; results leave through the same slice,
+// so that every store instruction writes whole rows of MT * 32 channels (128-byte runs for 64 half channels).
+constexpr int kParams = 3;                      // scale / bias / (BatchNorm a, PReLU slope): BatchNorm b is the fourth
+constexpr int kParamBytes(int mt) { return (kParams + 1) * mt * 32 * 4; }
+constexpr int kTileBytes(int mt) { return 32 * ((mt * 64 > 128 ? mt * 64 : 128) + 16); }
+constexpr int kWaveBytes(int mt) { return kParamBytes(mt) + kTileBytes(mt); }
 
-// The bias values of a lane's 16 channels per 32-channel block (zeros beyond K).
 template <int MT>
-__device__ __forceinline__ void load_bias(const PwParams& p, int kb0, int lane, float (&bi)[MT][16]) {
+__device__ __forceinline__ void read16(const char* lds, int which, int m, int half, float (&v)[16]) {
+    const v4f* src = reinterpret_cast<const v4f*>(lds + (which * MT * 32 + m * 32 + half * 16) * 4);
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        const int ch0 = (kb0 + m) * 32 + (lane >> 5) * 16;
+    for (int q = 0; q < 4; ++q) {
+        const v4f t = src[q];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) bi[m][e] = (p.bias && ch0 + e < p.K) ? p.bias[ch0 + e] : 0.f;
+        for (int e = 0; e < 4; ++e) v[q * 4 + e] = t[e];
     }
 }
 
-// Epilogue of one wave tile: a lane holds 16 consecutive channels of its pixel per 32-channel block.
-template <int MT, int NT>
-__device__ __forceinline__ void pw_epilogue(const PwParams& p, const v16f (&acc)[MT][NT], const unsigned (&pix)[NT], int kb0, int lane,
-                                            const float (&bi)[MT][16]) {
-    const bool odd = lane & 1;
+// An activation layer on 16 values. HALF: the layer reads the half the convolution layer stored.
+template <int OP, bool HALF>
+__device__ __forceinline__ void unary16(float (&v)[16], float alpha, float beta) {
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        const int ch0 = (kb0 + m) * 32 + (lane >> 5) * 16;
-        if (ch0 >= p.kstride && ch0 >= p.K) continue;
+    for (int e = 0; e < 16; ++e) v[e] = unary_value<OP>(HALF ? exhip_h2f(exhip_f2h(v[e])) : v[e], alpha, beta);
+}
+
+template <bool HALF, int MT>
+__device__ __forceinline__ void post_layer(const PwParams& p, const char* lds, int m, int half, float (&v)[16]) {
+    if (!p.post_op) return;
+    if (p.post_op == 1 + EXHIP_UNARY_HARDSWISH) {
+        unary16<0, HALF>(v, p.post_alpha, p.post_beta);
+    } else if (p.post_op == EXHIP_POST_PRELU) {
+        float slope[16];
+        read16<MT>(lds, 2, m, half, slope);
 #pragma unroll
-        for (int n = 0; n < NT; ++n) {
-            const bool valid = pix[n] < p.pixels;
-            float v[16];
-#pragma unroll
-            for (int e = 0; e < 16; ++e) v[e] = acc[m][n][e] + bi[m][e];
-            if (p.act >= 4) {
-#pragma unroll 1
-                for (int e = 0; e < 16; ++e) v[e] = slow_activation(v[e], p.act);
-            } else if (p.act) {
-#pragma unroll
-                for (int e = 0; e < 16; ++e) v[e] = fast_activation(v[e], p.act);
-            }
-            auto add_shortcut = [&]() {
-                // the add layer behind this one reads the stored (rounded) half
-                const uint16_t* r = p.residual + (size_t)pix[n] * p.kstride + ch0;
-                if (ch0 + 16 <= p.K) {
-                    const v4i r0 = reinterpret_cast<const v4i*>(r)[0], r1 = reinterpret_cast<const v4i*>(r)[1];
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) {
-                        const int word = e < 8 ? r0[e >> 1] : r1[(e - 8) >> 1];
-                        v[e] = exhip_h2f(exhip_f2h(v[e])) + exhip_h2f((uint16_t)(((uint32_t)word >> ((e & 1) * 16)) & 0xffff));
-                    }
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 16; ++e)
-                        if (ch0 + e < p.K) v[e] = exhip_h2f(exhip_f2h(v[e])) + exhip_h2f(r[e]);
-                }
-            };
-            if (p.residual && valid && !p.residual_last) add_shortcut();
-            if (p.post_relu) {
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    v[e] = exhip_h2f(exhip_f2h(v[e]));
-                    v[e] = (0.f > v[e]) ? 0.f : v[e];
-                }
-            }
-            if (p.post_op == EXHIP_POST_PRELU) {
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    const float t = exhip_h2f(exhip_f2h(v[e]));
-                    const float slope = p.post_slope[p.post_slope_shared || ch0 + e >= p.K ? 0 : ch0 + e];
-                    v[e] = t >= 0.f ? t : slope * t;
-                }
-            } else if (p.post_op) {
-                switch (p.post_op - 1) {
-                case EXHIP_UNARY_HARDSWISH: post_activation_op<0>(v, p.post_alpha, p.post_beta); break;
-                case EXHIP_UNARY_LEAKYRELU: post_activation_op<1>(v, p.post_alpha, p.post_beta); break;
-                case EXHIP_UNARY_HARDSIGMOID: post_activation_op<3>(v, p.post_alpha, p.post_beta); break;
-                default: post_activation_op<4>(v, p.post_alpha, p.post_beta); break;
-                }
-            }
-            if (p.residual && valid && p.residual_last) add_shortcut();
-#pragma unroll
-            for (int e = 0; e < 16; ++e)
-                if (ch0 + e >= p.K) v[e] = 0.f;  // pad channels hold zeros
-            v4i o[2];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const uint32_t lo = exhip_f2h(v[2 * e]), hi = exhip_f2h(v[2 * e + 1]);
-                o[e >> 2][e & 3] = (int)(lo | (hi << 16));
-            }
-            char* const yb = reinterpret_cast<char*>(p.y) + ch0 * 2;
-            if (ch0 + 16 <= p.kstride) {
-                if (__builtin_amdgcn_ballot_w64(valid) == ~0ull) {
-                    // the whole wave stores: a lane's 32 bytes and its neighbour's trade halves, so that four lanes (p,
-                    // p + 1 and the same two of the other half-wave) write 64 contiguous bytes of one pixel per instruction
-                    pair_exchange4(o[0], o[1], odd);
-                    const unsigned mine = pix[n], other = (unsigned)lane_neighbour((int)mine);
-                    const size_t even_pix = odd ? other : mine, odd_pix = odd ? mine : other;
-                    const int sub = odd ? 16 : 0;
-                    *reinterpret_cast<v4i*>(yb + even_pix * p.kstride * 2 + sub) = o[0];
-                    *reinterpret_cast<v4i*>(yb + odd_pix * p.kstride * 2 + sub) = o[1];
-                } else if (valid) {
-                    v4i* y = reinterpret_cast<v4i*>(yb + (size_t)pix[n] * p.kstride * 2);
-                    y[0] = o[0];
-                    y[1] = o[1];
-                }
-            } else if (valid) {
-                uint16_t* y = reinterpret_cast<uint16_t*>(yb + (size_t)pix[n] * p.kstride * 2);
-#pragma unroll
-                for (int e = 0; e < 16; ++e)
-                    if (ch0 + e < p.kstride) y[e] = (uint16_t)(((uint32_t)o[e >> 3][(e >> 1) & 3] >> ((e & 1) * 16)) & 0xffff);
-            }
-            // one 32 x 32 block at a time: interleaving the blocks buys nothing (they do not depend on each other's loads)
-            // and costs the registers of their temporaries
-            __builtin_amdgcn_sched_barrier(0);
+        for (int e = 0; e < 16; ++e) {
+            const float t = HALF ? exhip_h2f(exhip_f2h(v[e])) : v[e];
+            v[e] = t >= 0.f ? t : slope[e] * t;
         }
+    } else if (p.post_op == 1 + EXHIP_UNARY_LEAKYRELU) {
+        unary16<1, HALF>(v, p.post_alpha, p.post_beta);
+    } else if (p.post_op == 1 + EXHIP_UNARY_HARDSIGMOID) {
+        unary16<3, HALF>(v, p.post_alpha, p.post_beta);
+    } else {
+        unary16<4, HALF>(v, p.post_alpha, p.post_beta);
     }
 }
 
-// The int8 layer's epilogue: the general kernel's, value by value.
-template <int MT, int NT>
-__device__ __forceinline__ void pw_epilogue_i8(const PwParams& p, const v16i (&acc)[MT][NT], const unsigned (&pix)[NT], int kb0, int lane) {
+__device__ __forceinline__ void activation16(const PwParams& p, float (&v)[16]) {
+    if (p.act == 1) {
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        const int ch0 = (kb0 + m) * 32 + (lane >> 5) * 16;
-        if (ch0 >= p.K && (p.exact || ch0 >= p.kstride)) continue;
-        // FULL: every channel of the block exists (wave-uniform), and the per-value tests against K fall away
-        auto block = [&](auto full_c) {
-        constexpr bool FULL = decltype(full_c)::value;
-        float sc[16], bi[16];
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            sc[e] = (FULL || ch0 + e < p.K) ? p.scale[ch0 + e] : 0.f;
-            bi[e] = (p.bias && (FULL || ch0 + e < p.K)) ? p.bias[ch0 + e] : 0.f;
-        }
-        const bool vec_ok = ch0 + 16 <= p.kstride;
-        float bna[16], bnb[16];  // the BatchNorm's parameters of these channels (identity beyond K)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            bna[e] = (p.post_bn_a && (FULL || ch0 + e < p.K)) ? p.post_bn_a[ch0 + e] : 0.f;
-            bnb[e] = (p.post_bn_a && (FULL || ch0 + e < p.K)) ? p.post_bn_b[ch0 + e] : 1.f;
-        }
-#pragma unroll
-        for (int n = 0; n < NT; ++n) {
-            const bool valid = pix[n] < p.pixels;
-            const size_t at = (size_t)pix[n] * p.kstride + ch0;
-            float v[16];
-#pragma unroll
-            for (int e = 0; e < 16; ++e) v[e] = __builtin_fmaf((float)acc[m][n][e], sc[e], bi[e]);
-            if (p.act >= 4) {
+        for (int e = 0; e < 16; ++e) v[e] = (0.f > v[e]) ? 0.f : v[e];
+    } else if (p.act) {
 #pragma unroll 1
-                for (int e = 0; e < 16; ++e) v[e] = slow_activation(v[e], p.act);
-            } else if (p.act) {
+        for (int e = 0; e < 16; ++e) v[e] = slow_activation(v[e], p.act);
+    }
+}
+
+// Rows of a wave tile from its LDS slice to memory: CHUNKS 16-byte pieces per row of 32, neighbouring lanes on neighbouring
+// pieces. `y` is the tensor at the tile's first pixel and first channel, `rows` the pixels that exist, `bytes` how far the
+// tensor's channels reach from there.
+template <int CHUNKS>
+__device__ __forceinline__ void store_rows(const char* tile, int pitch, char* y, size_t row_bytes, int rows, int bytes, int lane) {
 #pragma unroll
-                for (int e = 0; e < 16; ++e) v[e] = fast_activation(v[e], p.act);
+    for (int j = 0; j < CHUNKS / 2; ++j) {
+        const int at = j * 64 + lane, row = at / CHUNKS, col = (at % CHUNKS) * 16;
+        const v4i t = *reinterpret_cast<const v4i*>(tile + row * pitch + col);
+        if (row < rows && col < bytes) *reinterpret_cast<v4i*>(y + row * row_bytes + col) = t;
+    }
+}
+
+template <int DT, int MT, int NT, typename ACC>
+__device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[MT][NT], unsigned pix0, int kb0, int lane, char* lds) {
+    constexpr bool I8 = DT == EXHIP_I8;
+    const int half = lane >> 5, row = lane & 31;
+    char* const tile = lds + kParamBytes(MT);
+    const int k_end = p.exact ? p.K : p.kstride > p.K ? p.kstride : p.K;  // channels from here on are not written
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        const unsigned first = pix0 + n * 32;
+        const int rows = first >= p.pixels ? 0 : p.pixels - first < 32 ? (int)(p.pixels - first) : 32;
+        if (rows == 0) continue;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const int kb = kb0 + m, ch0 = kb * 32 + half * 16;
+            if (kb * 32 >= k_end) continue;
+            const bool full = kb * 32 + 32 <= p.K;  // wave-uniform: every channel of the block exists
+            const size_t at = (size_t)(first + row) * p.kstride + ch0;
+            float v[16], t[16];
+            if constexpr (I8) {
+                read16<MT>(lds, 0, m, half, t);
+                float b[16];
+                read16<MT>(lds, 1, m, half, b);
+#pragma unroll
+                for (int e = 0; e < 16; ++e) v[e] = __builtin_fmaf((float)acc[m][n][e], t[e], b[e]);
+            } else {
+                read16<MT>(lds, 1, m, half, t);
+#pragma unroll
+                for (int e = 0; e < 16; ++e) v[e] = acc[m][n][e] + t[e];
             }
+            activation16(p, v);
             float r[16];
-            if (p.residual_f) {
+            const bool shortcut = I8 ? p.residual_f != nullptr : p.residual != nullptr;
+            if (shortcut) {
+                if constexpr (I8) {
 #pragma unroll
-                for (int e = 0; e < 16; ++e) r[e] = 0.f;
-                if (valid && (FULL || ch0 + 16 <= p.K)) {
+                    for (int e = 0; e < 16; ++e) r[e] = 0.f;
+                    if (row < rows) {
+                        if (full) {
 #pragma unroll
-                    for (int e4 = 0; e4 < 4; ++e4) {
-                        const v4f t = *reinterpret_cast<const v4f*>(p.residual_f + at + e4 * 4);
+                            for (int q = 0; q < 4; ++q) {
+                                const v4f x = *reinterpret_cast<const v4f*>(p.residual_f + at + q * 4);
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) r[e4 * 4 + e] = t[e];
-                    }
-                } else if (valid) {
+                                for (int e = 0; e < 4; ++e) r[q * 4 + e] = x[e];
+                            }
+                        } else {
 #pragma unroll
-                    for (int e = 0; e < 16; ++e)
-                        if (ch0 + e < p.K) r[e] = p.residual_f[at + e];
-                }
-            }
-            if (p.residual_f && !p.residual_last) {
-#pragma unroll
-                for (int e = 0; e < 16; ++e)
-                    if (FULL || ch0 + e < p.K) v[e] += r[e];
-            }
-            if (p.post_relu) {
-#pragma unroll
-                for (int e = 0; e < 16; ++e) v[e] = (0.f > v[e]) ? 0.f : v[e];
-            }
-            if (p.post_bn_a) {  // the BatchNorm layer between this layer (through a Concat) and its activation layer
-#pragma unroll
-                for (int e = 0; e < 16; ++e) v[e] = __builtin_fmaf(bnb[e], v[e], bna[e]);
-            }
-            if (p.post_op == EXHIP_POST_PRELU) {
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    const float slope = p.post_slope[p.post_slope_shared || (!FULL && ch0 + e >= p.K) ? 0 : ch0 + e];
-                    v[e] = v[e] >= 0.f ? v[e] : slope * v[e];
-                }
-            } else if (p.post_op) {
-                auto apply = [&](auto op) {
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) v[e] = unary_value<decltype(op)::value>(v[e], p.post_alpha, p.post_beta);
-                };
-                switch (p.post_op - 1) {
-                case EXHIP_UNARY_HARDSWISH: apply(std::integral_constant<int, 0>{}); break;
-                case EXHIP_UNARY_LEAKYRELU: apply(std::integral_constant<int, 1>{}); break;
-                case EXHIP_UNARY_HARDSIGMOID: apply(std::integral_constant<int, 3>{}); break;
-                default: apply(std::integral_constant<int, 4>{}); break;
-                }
-            }
-            if (p.residual_f && p.residual_last) {
-#pragma unroll
-                for (int e = 0; e < 16; ++e)
-                    if (FULL || ch0 + e < p.K) v[e] += r[e];
-            }
-#pragma unroll
-            for (int e = 0; e < 16; ++e)
-                if (!FULL && ch0 + e >= p.K) v[e] = 0.f;  // pad channels hold zeros
-            if (p.y_f && (kb0 + m) * 32 + 32 <= p.kstride && __builtin_amdgcn_ballot_w64(valid) == ~0ull) {
-                // the whole wave stores a whole 32-channel block: the two half-waves trade 16-byte pieces and neighbouring
-                // lanes trade pixels, so that four lanes (p, p + 1 and the same two of the other half-wave) write 64
-                // contiguous bytes of one pixel per instruction instead of 16-byte pieces of 64 pixels
-                v4i o4[4];
-#pragma unroll
-                for (int e4 = 0; e4 < 4; ++e4) {
-                    const v4f o = {v[e4 * 4], v[e4 * 4 + 1], v[e4 * 4 + 2], v[e4 * 4 + 3]};
-                    o4[e4] = __builtin_bit_cast(v4i, o);
-                }
-                const bool odd = lane & 1;
-                half_swap4(o4[0], o4[1]);   // o4[0], o4[2]: channels 0-7 and 8-15 of the block; o4[1], o4[3]: 16-23 and 24-31
-                half_swap4(o4[2], o4[3]);
-                pair_exchange4(o4[0], o4[2], odd);
-                pair_exchange4(o4[1], o4[3], odd);
-                const unsigned mine = pix[n], other = (unsigned)lane_neighbour((int)mine);
-                const size_t even_pix = odd ? other : mine, odd_pix = odd ? mine : other;
-                char* const yb = reinterpret_cast<char*>(p.y_f) + (size_t)(kb0 + m) * 128 + (odd ? 32 : 0) + (lane >> 5) * 16;
-                *reinterpret_cast<v4i*>(yb + even_pix * p.kstride * 4) = o4[0];
-                *reinterpret_cast<v4i*>(yb + even_pix * p.kstride * 4 + 64) = o4[1];
-                *reinterpret_cast<v4i*>(yb + odd_pix * p.kstride * 4) = o4[2];
-                *reinterpret_cast<v4i*>(yb + odd_pix * p.kstride * 4 + 64) = o4[3];
-            } else if (p.y_f && valid) {
-                float* y = p.y_f + at;
-                if (vec_ok) {
-#pragma unroll
-                    for (int e4 = 0; e4 < 4; ++e4) {
-                        const v4f o = {v[e4 * 4], v[e4 * 4 + 1], v[e4 * 4 + 2], v[e4 * 4 + 3]};
-                        *reinterpret_cast<v4f*>(y + e4 * 4) = o;
+                            for (int e = 0; e < 16; ++e)
+                                if (ch0 + e < p.K) r[e] = p.residual_f[at + e];
+                        }
                     }
                 } else {
+                    v4i x[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+                    if (row < rows) {
+                        if (full) {
+                            x[0] = reinterpret_cast<const v4i*>(p.residual + at)[0];
+                            x[1] = reinterpret_cast<const v4i*>(p.residual + at)[1];
+                        } else {
 #pragma unroll
-                    for (int e = 0; e < 16; ++e)
-                        if (ch0 + e < p.kstride) y[e] = v[e];
+                            for (int e = 0; e < 16; ++e)
+                                if (ch0 + e < p.K) x[e >> 3][(e >> 1) & 3] |= (int)((uint32_t)p.residual[at + e] << ((e & 1) * 16));
+                        }
+                    }
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) r[e] = exhip_h2f((uint16_t)(((uint32_t)x[e >> 3][(e >> 1) & 3] >> ((e & 1) * 16)) & 0xffff));
                 }
             }
-            if (p.y_q && valid && vec_ok) {
-                v4i o;
+            auto add_shortcut = [&]() {  // half layers: the sum reads the half the layer in front of it stored
 #pragma unroll
-                for (int e4 = 0; e4 < 4; ++e4) {
-                    uint32_t w = 0;
+                for (int e = 0; e < 16; ++e) v[e] = (I8 ? v[e] : exhip_h2f(exhip_f2h(v[e]))) + r[e];
+            };
+            if (shortcut && !p.residual_last) add_shortcut();
+            if (p.post_relu) {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) w |= (uint32_t)(exhip_q8(v[e4 * 4 + e] * p.fs_out) & 0xff) << (8 * e);
-                    o[e4] = (int)w;
+                for (int e = 0; e < 16; ++e) {
+                    const float x = I8 ? v[e] : exhip_h2f(exhip_f2h(v[e]));
+                    v[e] = (0.f > x) ? 0.f : x;
                 }
-                *reinterpret_cast<v4i*>(p.y_q + at) = o;
             }
+            if constexpr (I8) {
+                if (p.post_bn_a) {  // the BatchNorm layer between this layer (through a Concat) and its activation layer
+                    float a[16], b[16];
+                    read16<MT>(lds, 2, m, half, a);
+                    read16<MT>(lds, 3, m, half, b);
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) v[e] = __builtin_fmaf(b[e], v[e], a[e]);
+                }
+            }
+            post_layer<!I8, MT>(p, lds, m, half, v);
+            if (shortcut && p.residual_last) add_shortcut();
+            if (!full) {  // pad channels hold zeros
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    if (ch0 + e >= p.K) v[e] = 0.f;
+            }
+            if constexpr (I8) {
+                if (p.y_f) {  // one block at a time: 128 bytes per pixel
+                    constexpr int pitch = 128 + 16;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const v4f o = {v[q * 4], v[q * 4 + 1], v[q * 4 + 2], v[q * 4 + 3]};
+                        *reinterpret_cast<v4f*>(tile + row * pitch + half * 64 + q * 16) = o;
+                    }
+                    store_rows<8>(tile, pitch, reinterpret_cast<char*>(p.y_f + (size_t)first * p.kstride + kb * 32), (size_t)p.kstride * 4, rows,
+                                  (k_end - kb * 32) * 4, lane);
+                }
+                if (p.y_q) {
+                    v4i o;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        uint32_t w = 0;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) w |= (uint32_t)(exhip_q8(v[q * 4 + e] * p.fs_out) & 0xff) << (8 * e);
+                        o[q] = (int)w;
+                    }
+                    if (row < rows && ch0 < k_end) *reinterpret_cast<v4i*>(p.y_q + at) = o;
+                }
+            } else {
+                constexpr int pitch = MT * 64 + 16;
+                v4i o[2];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const uint32_t lo = exhip_f2h(v[2 * e]), hi = exhip_f2h(v[2 * e + 1]);
+                    o[e >> 2][e & 3] = (int)(lo | (hi << 16));
+                }
+                *reinterpret_cast<v4i*>(tile + row * pitch + m * 64 + half * 32) = o[0];
+                *reinterpret_cast<v4i*>(tile + row * pitch + m * 64 + half * 32 + 16) = o[1];
+            }
+            // one 32 x 32 block at a time: interleaving the blocks buys nothing and costs the registers of their temporaries
             __builtin_amdgcn_sched_barrier(0);
         }
-        };
-        // (the 64 x 64 tile keeps the one general form: with both its epilogue no longer fits the register file)
-        if constexpr (MT + NT < 4 || MT == 1) {
-            if ((kb0 + m) * 32 + 32 <= p.K) block(std::true_type{});
-            else block(std::false_type{});
-        } else {
-            block(std::false_type{});
+        if constexpr (!I8) {
+            constexpr int pitch = MT * 64 + 16;
+            store_rows<MT * 4>(tile, pitch, reinterpret_cast<char*>(p.y + (size_t)first * p.kstride + kb0 * 32), (size_t)p.kstride * 2, rows,
+                               (k_end - kb0 * 32) * 2, lane);
         }
     }
 }
 
-template <int DT, int MT, int NT, bool TAPS>
+// U: k-steps per request round; two rounds are in flight.
+template <int DT, int MT, int NT, int U, bool TAPS>
 __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
-    constexpr int U = MT + NT > 4 ? 2 : 4;  // k-steps fetched per request round; two rounds are in flight
+    __shared__ __attribute__((aligned(16))) char lds_all[4 * kWaveBytes(MT)];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // workgroup ids are dealt round-robin to the 8 XCDs: give each XCD one contiguous run of items, so that the channel
     // groups of a pixel tile (and the weights' re-reads) share that XCD's L2
@@ -360,34 +300,34 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
     if (item >= p.items) return;  // wave-uniform; the kernel has no barrier
     const unsigned tile = __builtin_amdgcn_readfirstlane(item / p.ch_groups);
     const int kb0 = __builtin_amdgcn_readfirstlane((int)(item - tile * p.ch_groups) * MT);  // first 32-channel block
+    char* const lds = lds_all + wave * kWaveBytes(MT);
 
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.x), 0, (int)p.x_bytes, kRsrcWord3);
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.wp), 0, (int)p.w_bytes, kRsrcWord3);
 
     // pixel fragments: lane = pixel (lane & 31), 16-byte half (lane >> 5) of each 32-byte k-step
-    unsigned pix[NT];
     int xoff[NT];
     unsigned taps_in[NT];  // TAPS: bit r * kw + q set where that tap of the pixel lies inside the image
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-        pix[nt] = (tile * NT + nt) * 32 + (lane & 31);
+        const unsigned pix = (tile * NT + nt) * 32 + (lane & 31);
         if constexpr (TAPS) {
             // the filter's top-left input pixel; its offset may lie in front of the tensor (padding), the taps inside the
             // image never do, and 32-bit wrap-around of the sum gives their offsets
             const unsigned per_image = (unsigned)(p.out_h * p.out_w);
-            const unsigned img = pix[nt] / per_image, rem = pix[nt] - img * per_image;
+            const unsigned img = pix / per_image, rem = pix - img * per_image;
             const int oy = (int)(rem / (unsigned)p.out_w), ox = (int)(rem - (unsigned)oy * (unsigned)p.out_w);
             const int iy = oy * p.stride - p.pad_t, ix = ox * p.stride - p.pad_l;
             xoff[nt] = (((int)img * p.in_h + iy) * p.in_w + ix) * p.xs_b + (lane >> 5) * 16;
             unsigned m = 0;
-            if (pix[nt] < p.pixels) {
+            if (pix < p.pixels) {
                 for (int r = 0; r < p.kh; ++r)
                     for (int q = 0; q < p.kw; ++q)
                         if ((unsigned)(iy + r) < (unsigned)p.in_h && (unsigned)(ix + q) < (unsigned)p.in_w) m |= 1u << (r * p.kw + q);
             }
             taps_in[nt] = m;
         } else {
-            xoff[nt] = pix[nt] < p.pixels ? (int)(pix[nt] * (unsigned)p.xs_b) + (lane >> 5) * 16 : kOutOfRange;
+            xoff[nt] = pix < p.pixels ? (int)(pix * (unsigned)p.xs_b) + (lane >> 5) * 16 : kOutOfRange;
         }
     }
     // weight fragments: block kb of slab kb / mts lies at ((slab * n_ksteps + ks) * mts + kb % mts) KiB; the MT blocks
@@ -407,64 +347,77 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
 
     v4i a[2][U][MT], b[2][U][NT];
     const int nks = p.n_ksteps;
+    // The request behind an odd last k-step reads the next row or block (or zeros beyond the view) and is not used.
     auto request = [&](auto buf_c, int ks0) {
         constexpr int buf = decltype(buf_c)::value;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            if (ks0 + u < nks) {
+            if (ks0 + (u & ~1) >= nks) continue;
 #pragma unroll
-                for (int m = 0; m < MT; ++m)
-                    a[buf][u][m] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, woff + m * 1024, w_base + (ks0 + u) * w_step, 0));
-                if constexpr (TAPS) {
-                    const int entry = p.step[ks0 + u];
-                    const int off = entry & ((1 << kTapShift) - 1);
-                    const unsigned bit = 1u << ((unsigned)entry >> kTapShift);
+            for (int m = 0; m < MT; ++m)
+                a[buf][u][m] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, woff + m * 1024, w_base + (ks0 + u) * w_step, 0));
+            if constexpr (TAPS) {
+                const int entry = p.step[ks0 + u < kMaxDirectSteps ? ks0 + u : 0];
+                const int off = entry & ((1 << kTapShift) - 1);
+                const unsigned bit = 1u << ((unsigned)entry >> kTapShift);
 #pragma unroll
-                    for (int n = 0; n < NT; ++n)
-                        b[buf][u][n] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(xr, (taps_in[n] & bit) ? xoff[n] + off : kOutOfRange, 0, 0));
-                } else {
+                for (int n = 0; n < NT; ++n)
+                    b[buf][u][n] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(xr, (taps_in[n] & bit) ? xoff[n] + off : kOutOfRange, 0, 0));
+            } else {
 #pragma unroll
-                    for (int n = 0; n < NT; ++n)
-                        b[buf][u][n] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(xr, xoff[n], (ks0 + u) * 32, 0));
-                }
+                for (int n = 0; n < NT; ++n)
+                    b[buf][u][n] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(xr, xoff[n], (ks0 + u) * 32, 0));
             }
         }
     };
-    auto compute = [&](auto buf_c, int ks0) {
+    auto step = [&](auto buf_c, int u) {
         constexpr int buf = decltype(buf_c)::value;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (ks0 + u < nks) {
+        for (int m = 0; m < MT; ++m)
 #pragma unroll
-                for (int m = 0; m < MT; ++m)
-#pragma unroll
-                    for (int n = 0; n < NT; ++n) {
-                        if constexpr (DT == EXHIP_I8)
-                            acc[m][n] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[buf][u][m], b[buf][u][n], acc[m][n], 0, 0, 0);
-                        else
-                            acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a[buf][u][m]), __builtin_bit_cast(v8h, b[buf][u][n]),
-                                                                               acc[m][n], 0, 0, 0);
-                    }
+            for (int n = 0; n < NT; ++n) {
+                if constexpr (DT == EXHIP_I8)
+                    acc[m][n] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[buf][u][m], b[buf][u][n], acc[m][n], 0, 0, 0);
+                else
+                    acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a[buf][u][m]), __builtin_bit_cast(v8h, b[buf][u][n]),
+                                                                       acc[m][n], 0, 0, 0);
             }
-        }
     };
     using B0 = std::integral_constant<int, 0>;
     using B1 = std::integral_constant<int, 1>;
     request(B0{}, 0);
-    for (int ks0 = 0; ks0 < nks; ks0 += 2 * U) {
-        request(B1{}, ks0 + U);
-        compute(B0{}, ks0);
+    // the channels' parameters: lane = channel of the wave's MT * 32, zeros beyond K
+    float par[kParams + 1] = {0.f, 0.f, 0.f, 0.f};
+    {
+        const int ch = kb0 * 32 + lane;
+        const bool in = ch < p.K && lane < MT * 32;
+        if (DT == EXHIP_I8 && in) par[0] = p.scale[ch];
+        if (p.bias && in) par[1] = p.bias[ch];
+        if (p.post_slope && in) par[2] = p.post_slope[p.post_slope_shared ? 0 : ch];
+        if (DT == EXHIP_I8 && p.post_bn_a && in) { par[2] = p.post_bn_a[ch]; par[3] = p.post_bn_b[ch]; }
+    }
+    request(B1{}, U);
+    int ks0 = 0;
+    for (; ks0 + 2 * U < nks; ks0 += 2 * U) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) step(B0{}, u);
         request(B0{}, ks0 + 2 * U);
-        compute(B1{}, ks0 + U);
+#pragma unroll
+        for (int u = 0; u < U; ++u) step(B1{}, u);
+        request(B1{}, ks0 + 3 * U);
     }
-
-    if constexpr (DT == EXHIP_I8) {
-        pw_epilogue_i8<MT, NT>(p, acc, pix, kb0, lane);
-    } else {
-        float bi[MT][16];
-        load_bias<MT>(p, kb0, lane, bi);
-        pw_epilogue<MT, NT>(p, acc, pix, kb0, lane, bi);
+    // (the loop leaves with both rounds of the last 2 * U k-steps requested)
+    if (lane < MT * 32) {
+#pragma unroll
+        for (int i = 0; i <= kParams; ++i) *reinterpret_cast<float*>(lds + (i * MT * 32 + lane) * 4) = par[i];
     }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (ks0 + u < nks) step(B0{}, u);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (ks0 + U + u < nks) step(B1{}, u);
+    pw_epilogue<DT, MT, NT>(p, acc, tile * NT * 32, kb0, lane, lds);
 }
 
 template <int DT, int MT, int NT, bool TAPS = false>
@@ -475,7 +428,12 @@ int launch(exhip_ctx* ctx, PwParams& p, int kblocks) {
     if (items >= (1ll << 31)) return EXHIP_ERR_UNSUPPORTED;
     p.items = (unsigned)items;
     const unsigned grid = (unsigned)((items + 3) / 4);
-    hipLaunchKernelGGL((conv1x1_pw_kernel<DT, MT, NT, TAPS>), dim3(grid), dim3(256), 0, ctx->stream, p);
+    // A launch of at most two waves per SIMD is as long as one wave's chain of load round trips: eight k-steps per round.
+    // Larger ones hide each other's round trips and want the registers for more waves.
+    if (MT + NT == 3 && items <= 2048)
+        hipLaunchKernelGGL((conv1x1_pw_kernel<DT, MT, NT, MT + NT == 3 ? 8 : 2, TAPS>), dim3(grid), dim3(256), 0, ctx->stream, p);
+    else
+        hipLaunchKernelGGL((conv1x1_pw_kernel<DT, MT, NT, MT + NT == 3 ? 4 : 2, TAPS>), dim3(grid), dim3(256), 0, ctx->stream, p);
     EXHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -534,7 +492,7 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
             for (int q = 0; q < t.kw; ++q)
                 for (int j = 0; j < t.chunk_b / 32; ++j)
                     p.step[s++] = ((r * t.in_w + q) * g.c_bytes + cc * t.chunk_b + j * 32) | (int)((unsigned)(r * t.kw + q) << kTapShift);
-    if (kblocks == 1) return launch<DT, 1, 4, true>(ctx, p, kblocks);
+    if (kblocks == 1) return launch<DT, 1, 2, true>(ctx, p, kblocks);
     const long long waves64 = ((g.pixels + 63) / 64) * ((kblocks + 1) / 2);
     if (waves64 < 2048 || small_tile<DT>()) return launch<DT, 2, 1, true>(ctx, p, kblocks);
     return launch<DT, 2, 2, true>(ctx, p, kblocks);
@@ -589,7 +547,7 @@ int run_pw(exhip_ctx* ctx, const exhip_pw_geom& g, PwParams& p, int es, bool has
     const int kblocks = std::min(g.slabs * g.slab_blocks, (out_channels + 31) / 32);
     // 64 x 64 per wave unless that leaves SIMDs without a wave: then 64 channels x 32 pixels; a lone 32-channel block
     // takes 128 pixels per wave
-    if (kblocks == 1) return launch<DT, 1, 4>(ctx, p, kblocks);
+    if (kblocks == 1) return launch<DT, 1, 2>(ctx, p, kblocks);
     const long long waves64 = ((g.pixels + 63) / 64) * ((kblocks + 1) / 2);
     if (waves64 < 2048 || small_tile<DT>()) return launch<DT, 2, 1>(ctx, p, kblocks);
     return launch<DT, 2, 2>(ctx, p, kblocks);
