@@ -56,6 +56,8 @@ struct PwParams {
     int exact;                // channels [0, K) only: blocks past K are not written (the results lie inside a wider tensor)
     unsigned pixels, x_bytes, w_bytes;
     unsigned items, ch_groups;   // waves with work; 32 * MT channel groups per pixel tile
+    unsigned groups_magic, image_magic, width_magic;  // divide() by ch_groups, out_h * out_w, out_w
+    int groups_shift, image_shift, width_shift;
     int xs_b;                    // bytes per input pixel
     int n_ksteps;                // 32-byte k-steps per pixel
     int mts;                     // 32-channel blocks per packed slab
@@ -73,15 +75,26 @@ __device__ __noinline__ float slow_activation(float v, int act) { return exhip_a
 // ---- epilogue ----
 // What bounds a short launch is the length of one wave's chain, and the epilogue was half of it (stamps inside a 256 -> 256
 // layer on a 20 x 20 map, 19 000 cycles in all: 3 000 for 32 conditional one-word bias loads, 4 200 - 8 200 for the arithmetic
-// with a test per value and per lane, against 7 000 for the products). So: the per-channel parameters (scale, bias, BatchNorm,
-// PReLU slopes) are requested at the kernel's start, one coalesced load each with zeros beyond K, wait in the wave's own LDS
-// slice and are read back four channels at a time; layer kinds are one wave-uniform branch per 32 x 32 block with straight
-// code behind it, and tests against K exist only in a block that holds the ragged end; results leave through the same slice,
-// so that every store instruction writes whole rows of MT * 32 channels (128-byte runs for 64 half channels).
-constexpr int kParams = 3;                      // scale / bias / (BatchNorm a, PReLU slope): BatchNorm b is the fourth
-constexpr int kParamBytes(int mt) { return (kParams + 1) * mt * 32 * 4; }
-constexpr int kTileBytes(int mt) { return 32 * ((mt * 64 > 128 ? mt * 64 : 128) + 16); }
-constexpr int kWaveBytes(int mt) { return kParamBytes(mt) + kTileBytes(mt); }
+// with a test per value, per lane and per layer kind, most of it instruction fetch, against 7 000 for the products). So:
+//  * the per-channel parameters (scale, bias, BatchNorm, PReLU slopes) are requested at the kernel's start, one coalesced
+//    load each with zeros beyond K, wait in the wave's own LDS slice and are read back four channels at a time;
+//  * the layers behind the convolution are template constants (Ep) for the combinations the networks are made of, so the
+//    epilogue is straight code; any other combination runs the one instantiation that looks at run time (Any);
+//  * results leave through the LDS slice, so that every store instruction writes whole rows of MT * 32 channels.
+enum { kPostNone, kPostRelu, kPostHardSwish, kPostLeaky, kPostPrelu, kPostHardSigmoid, kPostClip };
+template <int ACT, int POST, int RES, bool BN, bool ANY>
+struct EpT {
+    static constexpr int act = ACT, post = POST, res = RES;  // res: 0 no shortcut, 1 added in front of the layers behind, 2 behind them
+    static constexpr bool bn = BN, any = ANY;
+};
+template <int ACT, int POST, int RES, bool BN = false>
+using Ep = EpT<ACT, POST, RES, BN, false>;
+using EpAny = EpT<0, 0, 0, false, true>;
+
+constexpr int kParams = 4;  // scale / bias / BatchNorm a or PReLU slope / BatchNorm b
+constexpr int param_bytes(int mt) { return kParams * mt * 32 * 4; }
+constexpr int tile_bytes(int dt, int mt) { return 32 * ((dt == EXHIP_I8 ? 128 : mt * 64) + 16); }  // int8 layers: one float32 block
+constexpr int wave_bytes(int dt, int mt) { return param_bytes(mt) + tile_bytes(dt, mt); }
 
 template <int MT>
 __device__ __forceinline__ void read16(const char* lds, int which, int m, int half, float (&v)[16]) {
@@ -94,79 +107,96 @@ __device__ __forceinline__ void read16(const char* lds, int which, int m, int ha
     }
 }
 
-// An activation layer on 16 values. HALF: the layer reads the half the convolution layer stored.
-template <int OP, bool HALF>
-__device__ __forceinline__ void unary16(float (&v)[16], float alpha, float beta) {
-#pragma unroll
-    for (int e = 0; e < 16; ++e) v[e] = unary_value<OP>(HALF ? exhip_h2f(exhip_f2h(v[e])) : v[e], alpha, beta);
+// Two float32 values rounded to nearest-even halves, one instruction. (Written out: left to itself the compiler may round a
+// product to half in one step, which is another value than the float32 product rounded.)
+__device__ __forceinline__ unsigned round_pair(float lo, float hi) {
+    unsigned d;
+    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(d) : "v"(lo), "v"(hi));
+    return d;
 }
 
-template <bool HALF, int MT>
-__device__ __forceinline__ void post_layer(const PwParams& p, const char* lds, int m, int half, float (&v)[16]) {
-    if (!p.post_op) return;
-    if (p.post_op == 1 + EXHIP_UNARY_HARDSWISH) {
-        unary16<0, HALF>(v, p.post_alpha, p.post_beta);
-    } else if (p.post_op == EXHIP_POST_PRELU) {
-        float slope[16];
-        read16<MT>(lds, 2, m, half, slope);
+// ROUND: the layer behind reads the halves that the layer in front of it stored.
+template <bool ROUND>
+__device__ __forceinline__ void stored16(float (&v)[16]) {
+    if constexpr (ROUND) {
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const float t = HALF ? exhip_h2f(exhip_f2h(v[e])) : v[e];
-            v[e] = t >= 0.f ? t : slope[e] * t;
+        for (int e = 0; e < 16; e += 2) {
+            const unsigned d = round_pair(v[e], v[e + 1]);
+            v[e] = exhip_h2f((uint16_t)(d & 0xffff));
+            v[e + 1] = exhip_h2f((uint16_t)(d >> 16));
         }
-    } else if (p.post_op == 1 + EXHIP_UNARY_LEAKYRELU) {
-        unary16<1, HALF>(v, p.post_alpha, p.post_beta);
-    } else if (p.post_op == 1 + EXHIP_UNARY_HARDSIGMOID) {
-        unary16<3, HALF>(v, p.post_alpha, p.post_beta);
-    } else {
-        unary16<4, HALF>(v, p.post_alpha, p.post_beta);
     }
 }
 
-__device__ __forceinline__ void activation16(const PwParams& p, float (&v)[16]) {
-    if (p.act == 1) {
+template <int OP, bool ROUND>
+__device__ __forceinline__ void unary16(float (&v)[16], float alpha, float beta) {
+    stored16<ROUND>(v);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) v[e] = (0.f > v[e]) ? 0.f : v[e];
-    } else if (p.act) {
-#pragma unroll 1
-        for (int e = 0; e < 16; ++e) v[e] = slow_activation(v[e], p.act);
-    }
+    for (int e = 0; e < 16; ++e) v[e] = unary_value<OP>(v[e], alpha, beta);
+}
+
+template <bool ROUND>
+__device__ __forceinline__ void relu16(float (&v)[16]) {
+    stored16<ROUND>(v);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) v[e] = (0.f > v[e]) ? 0.f : v[e];
 }
 
 // Rows of a wave tile from its LDS slice to memory: CHUNKS 16-byte pieces per row of 32, neighbouring lanes on neighbouring
-// pieces. `y` is the tensor at the tile's first pixel and first channel, `rows` the pixels that exist, `bytes` how far the
-// tensor's channels reach from there.
+// pieces. The view starts at the tile's first pixel and channel and ends behind its last pixel's row; `bytes`: how far the
+// tensor's channels reach from the tile's first one.
 template <int CHUNKS>
-__device__ __forceinline__ void store_rows(const char* tile, int pitch, char* y, size_t row_bytes, int rows, int bytes, int lane) {
+__device__ __forceinline__ void store_rows(const char* tile, int pitch, __amdgpu_buffer_rsrc_t y, int row_bytes, int bytes, int lane) {
+    const int row = lane / CHUNKS, col = (lane % CHUNKS) * 16;
+    const int at = col < bytes ? row * row_bytes + col : kOutOfRange;
 #pragma unroll
     for (int j = 0; j < CHUNKS / 2; ++j) {
-        const int at = j * 64 + lane, row = at / CHUNKS, col = (at % CHUNKS) * 16;
-        const v4i t = *reinterpret_cast<const v4i*>(tile + row * pitch + col);
-        if (row < rows && col < bytes) *reinterpret_cast<v4i*>(y + row * row_bytes + col) = t;
+        const v4i t = *reinterpret_cast<const v4i*>(tile + (j * (64 / CHUNKS) + row) * pitch + col);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(__attribute__((ext_vector_type(4))) unsigned int, t), y, at, j * (64 / CHUNKS) * row_bytes, 0);
     }
 }
 
-template <int DT, int MT, int NT, typename ACC>
+// A view of a pixel-major tensor from pixel `first` and channel ch0 on, `rows` pixels long.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_view(const void* base, unsigned first, int row_bytes, int ch_bytes, int rows) {
+    char* p = const_cast<char*>(static_cast<const char*>(base)) + (size_t)first * (unsigned)row_bytes + ch_bytes;
+    return __builtin_amdgcn_make_buffer_rsrc(p, 0, rows * row_bytes - ch_bytes, kRsrcWord3);
+}
+
+template <int DT, int MT, int NT, typename EP, typename ACC>
 __device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[MT][NT], unsigned pix0, int kb0, int lane, char* lds) {
-    constexpr bool I8 = DT == EXHIP_I8;
+    constexpr bool I8 = DT == EXHIP_I8, ANY = EP::any;
+    constexpr int ES = I8 ? 4 : 2;  // bytes per value of the shortcut tensor
     const int half = lane >> 5, row = lane & 31;
-    char* const tile = lds + kParamBytes(MT);
+    char* const tile = lds + param_bytes(MT);
     const int k_end = p.exact ? p.K : p.kstride > p.K ? p.kstride : p.K;  // channels from here on are not written
+    const bool shortcut = ANY ? (I8 ? p.residual_f != nullptr : p.residual != nullptr) : EP::res != 0;
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
         const unsigned first = pix0 + n * 32;
-        const int rows = first >= p.pixels ? 0 : p.pixels - first < 32 ? (int)(p.pixels - first) : 32;
-        if (rows == 0) continue;
+        if (n > 0 && first >= p.pixels) continue;
+        const int rows = p.pixels - first < 32 ? (int)(p.pixels - first) : 32;
+        v4i r[MT][ES];
+        if (shortcut) {
+            // a channel group beyond the tensor's stride reads zeros; pad channels inside it read what lies there and are
+            // overwritten with zeros below
+            const __amdgpu_buffer_rsrc_t rr = tile_view(I8 ? (const void*)p.residual_f : (const void*)p.residual, first, p.kstride * ES, kb0 * 32 * ES, rows);
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int q = 0; q < ES; ++q) {
+                    const int ch = m * 32 + half * 16 + q * (16 / ES);
+                    const int at = kb0 * 32 + ch < p.kstride ? row * p.kstride * ES + ch * ES : kOutOfRange;
+                    r[m][q] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rr, at, 0, 0));
+                }
+        }
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
             const int kb = kb0 + m, ch0 = kb * 32 + half * 16;
-            if (kb * 32 >= k_end) continue;
-            const bool full = kb * 32 + 32 <= p.K;  // wave-uniform: every channel of the block exists
-            const size_t at = (size_t)(first + row) * p.kstride + ch0;
+            if (m > 0 && kb * 32 >= k_end) continue;
             float v[16], t[16];
             if constexpr (I8) {
-                read16<MT>(lds, 0, m, half, t);
                 float b[16];
+                read16<MT>(lds, 0, m, half, t);
                 read16<MT>(lds, 1, m, half, b);
 #pragma unroll
                 for (int e = 0; e < 16; ++e) v[e] = __builtin_fmaf((float)acc[m][n][e], t[e], b[e]);
@@ -175,57 +205,24 @@ __device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[
 #pragma unroll
                 for (int e = 0; e < 16; ++e) v[e] = acc[m][n][e] + t[e];
             }
-            activation16(p, v);
-            float r[16];
-            const bool shortcut = I8 ? p.residual_f != nullptr : p.residual != nullptr;
-            if (shortcut) {
-                if constexpr (I8) {
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) r[e] = 0.f;
-                    if (row < rows) {
-                        if (full) {
-#pragma unroll
-                            for (int q = 0; q < 4; ++q) {
-                                const v4f x = *reinterpret_cast<const v4f*>(p.residual_f + at + q * 4);
-#pragma unroll
-                                for (int e = 0; e < 4; ++e) r[q * 4 + e] = x[e];
-                            }
-                        } else {
-#pragma unroll
-                            for (int e = 0; e < 16; ++e)
-                                if (ch0 + e < p.K) r[e] = p.residual_f[at + e];
-                        }
-                    }
-                } else {
-                    v4i x[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
-                    if (row < rows) {
-                        if (full) {
-                            x[0] = reinterpret_cast<const v4i*>(p.residual + at)[0];
-                            x[1] = reinterpret_cast<const v4i*>(p.residual + at)[1];
-                        } else {
-#pragma unroll
-                            for (int e = 0; e < 16; ++e)
-                                if (ch0 + e < p.K) x[e >> 3][(e >> 1) & 3] |= (int)((uint32_t)p.residual[at + e] << ((e & 1) * 16));
-                        }
-                    }
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) r[e] = exhip_h2f((uint16_t)(((uint32_t)x[e >> 3][(e >> 1) & 3] >> ((e & 1) * 16)) & 0xffff));
-                }
+            if (ANY ? p.act == 1 : EP::act == 1) relu16<false>(v);
+            if (ANY && p.act > 1) {
+#pragma unroll 1
+                for (int e = 0; e < 16; ++e) v[e] = slow_activation(v[e], p.act);
             }
-            auto add_shortcut = [&]() {  // half layers: the sum reads the half the layer in front of it stored
-#pragma unroll
-                for (int e = 0; e < 16; ++e) v[e] = (I8 ? v[e] : exhip_h2f(exhip_f2h(v[e]))) + r[e];
-            };
-            if (shortcut && !p.residual_last) add_shortcut();
-            if (p.post_relu) {
+            auto add_shortcut = [&]() {
+                stored16<!I8>(v);
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
-                    const float x = I8 ? v[e] : exhip_h2f(exhip_f2h(v[e]));
-                    v[e] = (0.f > x) ? 0.f : x;
+                    const int word = r[m][I8 ? e >> 2 : e >> 3][I8 ? e & 3 : (e >> 1) & 3];  // (a bit cast of the element itself takes the vector's first)
+                    if constexpr (I8) v[e] += __builtin_bit_cast(float, word);
+                    else v[e] += exhip_h2f((uint16_t)(((uint32_t)word >> ((e & 1) * 16)) & 0xffff));
                 }
-            }
+            };
+            if (ANY ? shortcut && !p.residual_last : EP::res == 1) add_shortcut();
+            if (ANY ? p.post_relu != 0 : EP::post == kPostRelu) relu16<!I8>(v);
             if constexpr (I8) {
-                if (p.post_bn_a) {  // the BatchNorm layer between this layer (through a Concat) and its activation layer
+                if (ANY ? p.post_bn_a != nullptr : EP::bn) {  // the BatchNorm layer between this layer (through a Concat) and its activation layer
                     float a[16], b[16];
                     read16<MT>(lds, 2, m, half, a);
                     read16<MT>(lds, 3, m, half, b);
@@ -233,9 +230,18 @@ __device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[
                     for (int e = 0; e < 16; ++e) v[e] = __builtin_fmaf(b[e], v[e], a[e]);
                 }
             }
-            post_layer<!I8, MT>(p, lds, m, half, v);
-            if (shortcut && p.residual_last) add_shortcut();
-            if (!full) {  // pad channels hold zeros
+            if (ANY ? p.post_op == 1 + EXHIP_UNARY_HARDSWISH : EP::post == kPostHardSwish) unary16<0, !I8>(v, p.post_alpha, p.post_beta);
+            if (ANY ? p.post_op == 1 + EXHIP_UNARY_LEAKYRELU : EP::post == kPostLeaky) unary16<1, !I8>(v, p.post_alpha, p.post_beta);
+            if (ANY && p.post_op == 1 + EXHIP_UNARY_HARDSIGMOID) unary16<3, !I8>(v, p.post_alpha, p.post_beta);
+            if (ANY && p.post_op == 1 + EXHIP_UNARY_CLIP) unary16<4, !I8>(v, p.post_alpha, p.post_beta);
+            if (ANY ? p.post_op == EXHIP_POST_PRELU : EP::post == kPostPrelu) {
+                read16<MT>(lds, 2, m, half, t);
+                stored16<!I8>(v);
+#pragma unroll
+                for (int e = 0; e < 16; ++e) v[e] = v[e] >= 0.f ? v[e] : t[e] * v[e];
+            }
+            if (ANY ? shortcut && p.residual_last : EP::res == 2) add_shortcut();
+            if (kb * 32 + 32 > p.K) {  // pad channels hold zeros (wave-uniform: only the block with the ragged end looks)
 #pragma unroll
                 for (int e = 0; e < 16; ++e)
                     if (ch0 + e >= p.K) v[e] = 0.f;
@@ -248,8 +254,7 @@ __device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[
                         const v4f o = {v[q * 4], v[q * 4 + 1], v[q * 4 + 2], v[q * 4 + 3]};
                         *reinterpret_cast<v4f*>(tile + row * pitch + half * 64 + q * 16) = o;
                     }
-                    store_rows<8>(tile, pitch, reinterpret_cast<char*>(p.y_f + (size_t)first * p.kstride + kb * 32), (size_t)p.kstride * 4, rows,
-                                  (k_end - kb * 32) * 4, lane);
+                    store_rows<8>(tile, pitch, tile_view(p.y_f, first, p.kstride * 4, kb * 128, rows), p.kstride * 4, (k_end - kb * 32) * 4, lane);
                 }
                 if (p.y_q) {
                     v4i o;
@@ -260,34 +265,34 @@ __device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[
                         for (int e = 0; e < 4; ++e) w |= (uint32_t)(exhip_q8(v[q * 4 + e] * p.fs_out) & 0xff) << (8 * e);
                         o[q] = (int)w;
                     }
-                    if (row < rows && ch0 < k_end) *reinterpret_cast<v4i*>(p.y_q + at) = o;
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(__attribute__((ext_vector_type(4))) unsigned int, o),
+                                                           tile_view(p.y_q, first, p.kstride, kb * 32, rows),
+                                                           ch0 < k_end ? row * p.kstride + half * 16 : kOutOfRange, 0, 0);
                 }
             } else {
                 constexpr int pitch = MT * 64 + 16;
                 v4i o[2];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const uint32_t lo = exhip_f2h(v[2 * e]), hi = exhip_f2h(v[2 * e + 1]);
-                    o[e >> 2][e & 3] = (int)(lo | (hi << 16));
-                }
+                for (int e = 0; e < 8; ++e) o[e >> 2][e & 3] = (int)round_pair(v[2 * e], v[2 * e + 1]);
                 *reinterpret_cast<v4i*>(tile + row * pitch + m * 64 + half * 32) = o[0];
                 *reinterpret_cast<v4i*>(tile + row * pitch + m * 64 + half * 32 + 16) = o[1];
             }
             // one 32 x 32 block at a time: interleaving the blocks buys nothing and costs the registers of their temporaries
             __builtin_amdgcn_sched_barrier(0);
         }
-        if constexpr (!I8) {
-            constexpr int pitch = MT * 64 + 16;
-            store_rows<MT * 4>(tile, pitch, reinterpret_cast<char*>(p.y + (size_t)first * p.kstride + kb0 * 32), (size_t)p.kstride * 2, rows,
-                               (k_end - kb0 * 32) * 2, lane);
-        }
+        if constexpr (!I8)
+            store_rows<MT * 4>(tile, MT * 64 + 16, tile_view(p.y, first, p.kstride * 2, kb0 * 64, rows), p.kstride * 2, (k_end - kb0 * 32) * 2, lane);
     }
 }
 
+__device__ __forceinline__ unsigned divide(unsigned n, unsigned d, unsigned magic, int shift) {  // n < 2^31, magic of host_divisor()
+    return d == 1 ? n : __umulhi(n, magic) >> shift;
+}
+
 // U: k-steps per request round; two rounds are in flight.
-template <int DT, int MT, int NT, int U, bool TAPS>
+template <int DT, int MT, int NT, int U, bool TAPS, typename EP>
 __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
-    __shared__ __attribute__((aligned(16))) char lds_all[4 * kWaveBytes(MT)];
+    __shared__ __attribute__((aligned(16))) char lds_all[4 * wave_bytes(DT, MT)];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // workgroup ids are dealt round-robin to the 8 XCDs: give each XCD one contiguous run of items, so that the channel
     // groups of a pixel tile (and the weights' re-reads) share that XCD's L2
@@ -298,9 +303,9 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
     }
     const unsigned item = __builtin_amdgcn_readfirstlane(bid * 4 + wave);
     if (item >= p.items) return;  // wave-uniform; the kernel has no barrier
-    const unsigned tile = __builtin_amdgcn_readfirstlane(item / p.ch_groups);
+    const unsigned tile = __builtin_amdgcn_readfirstlane(divide(item, p.ch_groups, p.groups_magic, p.groups_shift));
     const int kb0 = __builtin_amdgcn_readfirstlane((int)(item - tile * p.ch_groups) * MT);  // first 32-channel block
-    char* const lds = lds_all + wave * kWaveBytes(MT);
+    char* const lds = lds_all + wave * wave_bytes(DT, MT);
 
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.x), 0, (int)p.x_bytes, kRsrcWord3);
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.wp), 0, (int)p.w_bytes, kRsrcWord3);
@@ -315,8 +320,8 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
             // the filter's top-left input pixel; its offset may lie in front of the tensor (padding), the taps inside the
             // image never do, and 32-bit wrap-around of the sum gives their offsets
             const unsigned per_image = (unsigned)(p.out_h * p.out_w);
-            const unsigned img = pix / per_image, rem = pix - img * per_image;
-            const int oy = (int)(rem / (unsigned)p.out_w), ox = (int)(rem - (unsigned)oy * (unsigned)p.out_w);
+            const unsigned img = divide(pix, per_image, p.image_magic, p.image_shift), rem = pix - img * per_image;
+            const int oy = (int)divide(rem, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = (int)(rem - (unsigned)oy * (unsigned)p.out_w);
             const int iy = oy * p.stride - p.pad_t, ix = ox * p.stride - p.pad_l;
             xoff[nt] = (((int)img * p.in_h + iy) * p.in_w + ix) * p.xs_b + (lane >> 5) * 16;
             unsigned m = 0;
@@ -331,9 +336,9 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
         }
     }
     // weight fragments: block kb of slab kb / mts lies at ((slab * n_ksteps + ks) * mts + kb % mts) KiB; the MT blocks
-    // of a wave are neighbours in one slab (mts is a multiple of MT)
-    const int w_step = p.mts * 1024;
-    const int w_base = __builtin_amdgcn_readfirstlane(((kb0 / p.mts) * p.n_ksteps * p.mts + kb0 % p.mts) * 1024);
+    // of a wave are neighbours in one slab (mts, 2 or 4, is a multiple of MT)
+    const int w_step = p.mts * 1024, slab = kb0 >> (p.mts >> 1);
+    const int w_base = (slab * p.n_ksteps * p.mts + (kb0 & (p.mts - 1))) * 1024;
     const int woff = lane * 16;
 
     typedef typename std::conditional<DT == EXHIP_I8, v16i, v16f>::type acc_t;
@@ -386,15 +391,21 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
     using B0 = std::integral_constant<int, 0>;
     using B1 = std::integral_constant<int, 1>;
     request(B0{}, 0);
-    // the channels' parameters: lane = channel of the wave's MT * 32, zeros beyond K
-    float par[kParams + 1] = {0.f, 0.f, 0.f, 0.f};
+    // the channels' parameters: lane = channel of the wave's MT * 32, zeros beyond K and for an absent array
+    float par[kParams] = {};
     {
-        const int ch = kb0 * 32 + lane;
-        const bool in = ch < p.K && lane < MT * 32;
-        if (DT == EXHIP_I8 && in) par[0] = p.scale[ch];
-        if (p.bias && in) par[1] = p.bias[ch];
-        if (p.post_slope && in) par[2] = p.post_slope[p.post_slope_shared ? 0 : ch];
-        if (DT == EXHIP_I8 && p.post_bn_a && in) { par[2] = p.post_bn_a[ch]; par[3] = p.post_bn_b[ch]; }
+        const int at = (kb0 * 32 + lane) * 4;
+        auto load = [&](const float* src, int offset, int count) {
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src), 0, src ? count * 4 : 0, kRsrcWord3);
+            return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, offset, 0, 0));
+        };
+        if constexpr (DT == EXHIP_I8) par[0] = load(p.scale, at, p.K);
+        par[1] = load(p.bias, at, p.K);
+        if (EP::any || EP::post == kPostPrelu) par[2] = load(p.post_slope, p.post_slope_shared ? 0 : at, p.post_slope_shared ? 1 : p.K);
+        if (DT == EXHIP_I8 && (EP::any ? p.post_bn_a != nullptr : EP::bn)) {
+            par[2] = load(p.post_bn_a, at, p.K);
+            par[3] = load(p.post_bn_b, at, p.K);
+        }
     }
     request(B1{}, U);
     int ks0 = 0;
@@ -407,9 +418,9 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
         request(B1{}, ks0 + 3 * U);
     }
     // (the loop leaves with both rounds of the last 2 * U k-steps requested)
-    if (lane < MT * 32) {
+    if (MT == 2 || lane < 32) {
 #pragma unroll
-        for (int i = 0; i <= kParams; ++i) *reinterpret_cast<float*>(lds + (i * MT * 32 + lane) * 4) = par[i];
+        for (int i = 0; i < kParams; ++i) *reinterpret_cast<float*>(lds + (i * MT * 32 + lane) * 4) = par[i];
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
@@ -417,7 +428,57 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
         if (ks0 + U + u < nks) step(B1{}, u);
-    pw_epilogue<DT, MT, NT>(p, acc, tile * NT * 32, kb0, lane, lds);
+    pw_epilogue<DT, MT, NT, EP>(p, acc, tile * NT * 32, kb0, lane, lds);
+}
+
+// magic and shift of divide() for divisors from 2 on: with s = ceil(log2 d) and magic = ceil(2^(31 + s) / d) < 2^32,
+// n * magic >> (31 + s) is n / d for every n < 2^31 (the rounding of magic adds less than n / 2^31 < 1 part of d)
+void host_divisor(unsigned d, unsigned* magic, int* shift) {
+    *magic = 0;
+    *shift = 0;
+    if (d <= 1) return;
+    int s = 0;
+    while ((1ull << s) < d) ++s;
+    *magic = (unsigned)(((1ull << (31 + s)) + d - 1) / d);
+    *shift = s - 1;
+}
+
+template <int DT, int MT, int NT, int U, bool TAPS, typename EP>
+int go(exhip_ctx* ctx, const PwParams& p) {
+    hipLaunchKernelGGL((conv1x1_pw_kernel<DT, MT, NT, U, TAPS, EP>), dim3((p.items + 3) / 4), dim3(256), 0, ctx->stream, p);
+    EXHIP_LAUNCH_CHECK();
+    return 0;
+}
+
+// The layers behind the convolution, as template constants where a network of this library's kind has the combination.
+template <int DT, int MT, int NT, int U, bool TAPS>
+int pick_epilogue(exhip_ctx* ctx, const PwParams& p) {
+    const bool shortcut = DT == EXHIP_I8 ? p.residual_f != nullptr : p.residual != nullptr;
+    const int res = !shortcut ? 0 : p.residual_last ? 2 : 1;
+    int post = p.post_relu ? kPostRelu : kPostNone;
+    if (p.post_op) {
+        const int op = p.post_op == EXHIP_POST_PRELU ? kPostPrelu
+                       : p.post_op == 1 + EXHIP_UNARY_HARDSWISH ? kPostHardSwish
+                       : p.post_op == 1 + EXHIP_UNARY_LEAKYRELU ? kPostLeaky : -1;
+        post = post == kPostNone ? op : -1;
+    }
+    const bool bn = p.post_bn_a != nullptr;
+    auto is = [&](int a, int q, int r, bool b) { return p.act == a && post == q && res == r && bn == b; };
+    if (is(0, kPostNone, 0, false)) return go<DT, MT, NT, U, TAPS, Ep<0, kPostNone, 0>>(ctx, p);
+    if (is(0, kPostHardSwish, 0, false)) return go<DT, MT, NT, U, TAPS, Ep<0, kPostHardSwish, 0>>(ctx, p);
+    if (is(0, kPostRelu, 0, false)) return go<DT, MT, NT, U, TAPS, Ep<0, kPostRelu, 0>>(ctx, p);
+    if (is(1, kPostNone, 0, false)) return go<DT, MT, NT, U, TAPS, Ep<1, kPostNone, 0>>(ctx, p);
+    if (is(0, kPostHardSwish, 2, false)) return go<DT, MT, NT, U, TAPS, Ep<0, kPostHardSwish, 2>>(ctx, p);
+    if (is(0, kPostRelu, 1, false)) return go<DT, MT, NT, U, TAPS, Ep<0, kPostRelu, 1>>(ctx, p);
+    if constexpr (DT == EXHIP_F16) {
+        if (is(0, kPostPrelu, 0, false)) return go<DT, MT, NT, U, TAPS, Ep<0, kPostPrelu, 0>>(ctx, p);
+        if (is(0, kPostNone, 1, false)) return go<DT, MT, NT, U, TAPS, Ep<0, kPostNone, 1>>(ctx, p);
+    } else {
+        if (is(0, kPostRelu, 2, false)) return go<DT, MT, NT, U, TAPS, Ep<0, kPostRelu, 2>>(ctx, p);
+        if constexpr (!TAPS)
+            if (is(0, kPostLeaky, 0, true)) return go<DT, MT, NT, U, TAPS, Ep<0, kPostLeaky, 0, true>>(ctx, p);
+    }
+    return go<DT, MT, NT, U == 8 ? 4 : U, TAPS, EpAny>(ctx, p);
 }
 
 template <int DT, int MT, int NT, bool TAPS = false>
@@ -425,17 +486,14 @@ int launch(exhip_ctx* ctx, PwParams& p, int kblocks) {
     const long long tiles = ((long long)p.pixels + 32 * NT - 1) / (32 * NT);
     p.ch_groups = (unsigned)((kblocks + MT - 1) / MT);
     const long long items = tiles * p.ch_groups;
-    if (items >= (1ll << 31)) return EXHIP_ERR_UNSUPPORTED;
+    if (items >= (1ll << 31) - 4) return EXHIP_ERR_UNSUPPORTED;
     p.items = (unsigned)items;
-    const unsigned grid = (unsigned)((items + 3) / 4);
-    // A launch of at most two waves per SIMD is as long as one wave's chain of load round trips: eight k-steps per round.
-    // Larger ones hide each other's round trips and want the registers for more waves.
-    if (MT + NT == 3 && items <= 2048)
-        hipLaunchKernelGGL((conv1x1_pw_kernel<DT, MT, NT, MT + NT == 3 ? 8 : 2, TAPS>), dim3(grid), dim3(256), 0, ctx->stream, p);
-    else
-        hipLaunchKernelGGL((conv1x1_pw_kernel<DT, MT, NT, MT + NT == 3 ? 4 : 2, TAPS>), dim3(grid), dim3(256), 0, ctx->stream, p);
-    EXHIP_LAUNCH_CHECK();
-    return 0;
+    host_divisor(p.ch_groups, &p.groups_magic, &p.groups_shift);
+    if constexpr (MT + NT > 3) return go<DT, MT, NT, 2, TAPS, EpAny>(ctx, p);
+    // A launch of at most two waves per SIMD is as long as one wave's chain of load round trips: sixteen k-steps in flight
+    // where there are more than eight. Larger ones hide each other's round trips and want the registers for more waves.
+    else if (MT == 2 && items <= 2048 && p.n_ksteps > 8) return pick_epilogue<DT, MT, NT, 8, TAPS>(ctx, p);
+    else return pick_epilogue<DT, MT, NT, 4, TAPS>(ctx, p);
 }
 
 }  // namespace
@@ -486,6 +544,8 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
     p.post_alpha = g.post_alpha; p.post_beta = g.post_beta;
     p.in_h = t.in_h; p.in_w = t.in_w; p.out_h = t.out_h; p.out_w = t.out_w; p.stride = t.stride; p.pad_t = t.pad_t; p.pad_l = t.pad_l;
     p.kh = t.kh; p.kw = t.kw;
+    host_divisor((unsigned)(t.out_h * t.out_w), &p.image_magic, &p.image_shift);
+    host_divisor((unsigned)t.out_w, &p.width_magic, &p.width_shift);
     int s = 0;
     for (int cc = 0; cc < t.n_chunks; ++cc)
         for (int r = 0; r < t.kh; ++r)
