@@ -92,6 +92,7 @@ struct exhip_options {
     int pw = 1;              // 1x1 stride-1 fp16 layers with an NHWC result: 1 the pointwise kernel where it measured faster, 2 wherever it can run, 0 never
 };
 extern exhip_options g_exhip_options;
+extern unsigned g_exhip_options_version;  // counts exhip_set_option calls: what was planned under other options is planned again
 
 // Cache policy bits of the float32 result stores of the int8 kernels (the aux operand of the raw buffer store builtins).
 #ifndef EXHIP_F32_STORE_AUX

@@ -1349,9 +1349,7 @@ int validate(const exhip_conv_desc* d, int dt) {
 
 // Picks the tile variant, patch shape and staging split for a layer. Maximises the share of issued
 // MFMA work that is useful, subject to the per-thread staging limits and the LDS size.
-int make_plan(const exhip_conv_desc* d, int dt, Plan* out, const PoolSpec* pool = nullptr) {
-    int rc = validate(d, dt);
-    if (rc) return rc;
+int search_plan(const exhip_conv_desc* d, int dt, Plan* out, const PoolSpec* pool) {
     Plan best;
     double best_score = -1e30;
     bool found = false;
@@ -1595,6 +1593,36 @@ int launch_variant(exhip_ctx* ctx, const Plan& pl, const ConvParams& p, int grid
     case 1: return launch_shape<DT, 2, 2, 4, PACKED, EPI>(ctx, pl, p, grid);
     default: return launch_shape<DT, 2, 2, 2, PACKED, EPI>(ctx, pl, p, grid);
     }
+}
+
+// The search above walks hundreds of patch shapes, 2 - 6 us of a call's host time, and its answer depends on the layer's
+// shape and the library's options alone: a thread keeps its last answers (direct mapped; a short launch then costs the host
+// 3 us instead of 6, which is what bounds a network at batch 1).
+int make_plan(const exhip_conv_desc* d, int dt, Plan* out, const PoolSpec* pool = nullptr) {
+    const int rc = validate(d, dt);
+    if (rc) return rc;
+    constexpr int kKey = 20, kSlots = 512;
+    const int key[kKey] = {dt, d->n, d->c, d->h, d->w, d->k, d->kh, d->kw, d->sh, d->pt, d->pb, d->pl, d->pr, d->c_stride,
+                           pool ? pool->pt : -1, pool ? pool->pl : -1, pool ? pool->oh : -1, pool ? pool->ow : -1, (int)g_exhip_options_version, 1};
+    struct Entry {
+        int key[kKey];
+        Plan plan;
+    };
+    static thread_local std::vector<Entry> cache;
+    if (cache.empty()) cache.resize(kSlots);  // zeroed keys: no layer has the key's last word 0
+    uint32_t h = 2166136261u;
+    for (int v : key) h = (h ^ (uint32_t)v) * 16777619u;
+    Entry& e = cache[(h ^ (h >> 15)) % kSlots];
+    if (memcmp(e.key, key, sizeof(key)) != 0) {
+        const int found = search_plan(d, dt, &e.plan, pool);
+        if (found) {
+            e.key[kKey - 1] = 0;
+            return found;
+        }
+        memcpy(e.key, key, sizeof(key));
+    }
+    *out = e.plan;
+    return 0;
 }
 
 // The plan assumes the largest epilogue so that the weight packing does not depend on a call's outputs; the number of

@@ -18,10 +18,12 @@ void exhip_set_error(const char* fmt, ...) {
 extern "C" const char* exhip_last_error(void) { return g_err; }
 
 exhip_options g_exhip_options;
+unsigned g_exhip_options_version = 0;
 
 extern "C" int exhip_set_option(const char* name, int value) {
     EXHIP_REQUIRE(name, "exhip_set_option: NULL name");
     exhip_options& o = g_exhip_options;
+    ++g_exhip_options_version;
     if (!strcmp(name, "force_variant")) o.force_variant = value;
     else if (!strcmp(name, "force_chunk")) o.force_chunk = value;
     else if (!strcmp(name, "force_rs")) o.force_rs = value;
