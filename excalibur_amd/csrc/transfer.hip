@@ -24,6 +24,8 @@ namespace {
 constexpr size_t kChunk = (size_t)4 << 20;       // staging chunk: 50 GB/s on the link with one copy each (38 at 1 MiB), short enough to start early
 constexpr size_t kPiece = (size_t)512 << 10;     // what one thread copies at a time
 constexpr size_t kUploadKernel = (size_t)256 << 10;   // up to here a kernel reads the staging memory; the copy engine is as fast from 1 MiB on
+constexpr size_t kSmallRing = (size_t)512 << 10;      // small uploads turn in this much of each chunk, so that the GPU's translations of it stay
+                                                      // cached (75 KB from pages not seen lately take the kernel 31 us)
 constexpr size_t kDownloadKernel = (size_t)64 << 10;  // up to here one group writes the host's memory and a flag
 constexpr int kSmallThreads = 1024;
 
@@ -240,7 +242,7 @@ extern "C" int exhip_upload(exhip_ctx* ctx, void* dst, const void* src, size_t b
     while (bytes) {
         exhip_staging& s = ctx->up;
         const size_t now = bytes < kChunk ? bytes : kChunk;
-        if (s.at < 0 || s.used + now > kChunk) {
+        if (s.at < 0 || s.used + now > (now <= kUploadKernel ? kSmallRing : kChunk)) {
             const int rc = next_chunk(ctx);
             if (rc == EXHIP_ERR_UNSUPPORTED) {  // no pinned memory left: the runtime's own way
                 EXHIP_CHECK(hipMemcpyAsync(to, from, bytes, hipMemcpyHostToDevice, ctx->stream));
