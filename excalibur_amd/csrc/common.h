@@ -89,6 +89,7 @@ struct exhip_options {
     int direct = 1;          // layers with a filter, a stride or padding and NHWC results on the pointwise kernel's tapped form: 1 where it measured
                              // faster, 2 wherever it can run, 0 never
     int pw_tile = 0;         // that kernel's wave tile for more than 32 output channels: 0 = 32 pixels x 64 channels, 2 = 64 x 64 from 2048 waves on
+    int f32_tile = 0;        // the float32 convolution's wave tile and split: 0 by its rule, n = the n-th of its list
     int pw = 1;              // 1x1 stride-1 fp16 layers with an NHWC result: 1 the pointwise kernel where it measured faster, 2 wherever it can run, 0 never
 };
 extern exhip_options g_exhip_options;
@@ -98,6 +99,22 @@ extern unsigned g_exhip_options_version;  // counts exhip_set_option calls: what
 #ifndef EXHIP_F32_STORE_AUX
 #define EXHIP_F32_STORE_AUX 0
 #endif
+
+// Division by a launch constant: n / d for n < 2^31, with magic and shift of exhip_host_divisor(d).
+__device__ __forceinline__ unsigned exhip_divide(unsigned n, unsigned d, unsigned magic, int shift) {
+    return d == 1 ? n : __umulhi(n, magic) >> shift;
+}
+// With s = ceil(log2 d) and magic = ceil(2^(31 + s) / d) < 2^32, n * magic >> (31 + s) is n / d for every n < 2^31 (the
+// rounding of magic adds less than n / 2^31 < 1 part of d).
+inline void exhip_host_divisor(unsigned d, unsigned* magic, int* shift) {
+    *magic = 0;
+    *shift = 0;
+    if (d <= 1) return;
+    int s = 0;
+    while ((1ull << s) < d) ++s;
+    *magic = (unsigned)(((1ull << (31 + s)) + d - 1) / d);
+    *shift = s - 1;
+}
 
 // ---- device helpers shared by the kernels ----
 typedef int exhip_v4i __attribute__((ext_vector_type(4)));

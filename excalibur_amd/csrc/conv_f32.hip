@@ -1,0 +1,559 @@
+// conv_f32_kernel: the float32 convolution, any filter, stride and padding, on NHWC input with v_mfma_f32_32x32x2_f32.
+//
+// float32 products run at a sixteenth of the half-precision rate (157 TFLOP/s), so operands are cheap next to the
+// arithmetic: one 32-byte step of a 64-channel x 32-pixel wave tile fetches 3 KiB for 512 matrix cycles. Nothing is staged
+// therefore: a wave owns 32 * NT output pixels x 32 * MT output channels and loads its fragments straight into registers,
+// 16 bytes per lane and step -- the weights from a packing in which a 32-channel block is one contiguous stream, the
+// pixels from the NHWC rows around each output pixel, taps outside the image reading zeros. The pixels of all images form
+// one list, so ragged maps waste no lanes. No barrier in the main loop, no tile geometry, no patch to plan.
+//
+// What bounds it otherwise is a small launch: a 3x3 layer of 64 channels on one 56 x 56 map is 98 wave tiles for 1024 SIMDs,
+// each with a chain of 72 steps. WK waves of a group therefore share a tile: each reduces its run of the steps, the parts are
+// added through LDS in a fixed order (the same bits every time) and the waves share the tile's blocks in the epilogue.
+//
+// Arithmetic: float32 products and sums, bias, activation, the optional shortcut in front of or behind the layers behind the
+// convolution, BatchNorm, activation layer.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+#include <cstdint>
+#include <cstring>
+#include <type_traits>
+
+#include "conv_f32.h"
+
+namespace {
+
+typedef exhip_v4i v4i;
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
+
+constexpr unsigned kRsrcWord3 = 0x00020000u;      // raw buffer: out-of-range loads return 0, such stores are dropped
+constexpr unsigned kOutOfRange = 0xfffff000u;     // a lane offset beyond every view
+constexpr int kMaxSplit = 8;
+
+// How a step's 32 bytes lie in the input: kPoint one tap, always inside the image (1x1 filters without padding); kTaps 8
+// channels of one tap; kPair two neighbouring taps of 16-byte pixels (layers of at most four channels).
+enum { kPoint, kTaps, kPair };
+
+struct F32Params {
+    const char* x;
+    const char* wp;
+    const float *bias, *residual, *slope, *bn_a, *bn_b;
+    float *y, *y_nchw;
+    unsigned pixels, x_bytes, w_bytes, tiles, items, ch_groups;
+    unsigned groups_magic, image_magic, width_magic;  // exhip_divide() by ch_groups, out_h * out_w, out_w
+    int groups_shift, image_shift, width_shift;
+    int in_h, in_w, out_h, out_w, stride, pad_t, pad_l, kh, kw;
+    int xs_b, row_b;               // bytes per input pixel and input row
+    int csteps, n_ksteps;          // steps per tap (kPair: 1) and in all
+    int start_r[kMaxSplit + 1], start_q[kMaxSplit + 1], start_c[kMaxSplit + 1], start_s[kMaxSplit + 1];  // where each wave of a tile begins
+    int K, kstride, k_end;         // channels from k_end on are not written
+    int act, post_relu, post_op, slope_shared, residual_last;
+    float alpha, beta;
+    int vector_rows;               // output (and shortcut) rows take 16-byte accesses
+};
+
+__device__ __forceinline__ v4f load4(__amdgpu_buffer_rsrc_t r, unsigned voff, int soff) {
+    return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, soff, 0));
+}
+
+// A view of a pixel-major float tensor from pixel `first` and channel ch0 on, `rows` pixels long.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_view(const float* base, unsigned first, int stride, int ch0, int rows) {
+    float* p = const_cast<float*>(base) + (size_t)first * (unsigned)stride + ch0;
+    return __builtin_amdgcn_make_buffer_rsrc(p, 0, (rows * stride - ch0) * 4, kRsrcWord3);
+}
+
+template <int MT>
+__device__ __forceinline__ void read16(const char* lds, int which, int m, int half, float (&v)[16]) {
+    const v4f* src = reinterpret_cast<const v4f*>(lds + (which * MT * 32 + m * 32 + half * 16) * 4);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const v4f t = src[q];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[q * 4 + e] = t[e];
+    }
+}
+
+template <int OP>
+__device__ __forceinline__ void unary16(float (&v)[16], float alpha, float beta) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) v[e] = unary_value<OP>(v[e], alpha, beta);
+}
+__device__ __forceinline__ void relu16(float (&v)[16]) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) v[e] = (0.f > v[e]) ? 0.f : v[e];
+}
+
+constexpr int kParams = 4;                // bias / PReLU slope / BatchNorm a / b
+constexpr int kTilePitch = 128 + 16;      // one pixel's 32 channels and padding
+constexpr int wave_lds(int mt) { return kParams * mt * 32 * 4 + 32 * kTilePitch; }
+
+// One 32-pixel x 32-channel block: lane = pixel (lane & 31) and sixteen neighbouring channels. Straight code per layer kind
+// under wave-uniform branches; what is not taken is not fetched.
+template <int MT, bool SLOW>
+__device__ __forceinline__ void epilogue_block(const F32Params& p, const v16f& acc, unsigned first, int kb, int m, int lane, char* lds) {
+    const int half = lane >> 5, row = lane & 31, ch0 = kb * 32 + half * 16;
+    if (first >= p.pixels || kb * 32 >= p.k_end) return;
+    const int rows = p.pixels - first < 32 ? (int)(p.pixels - first) : 32;
+    char* const tile = lds + kParams * MT * 32 * 4;
+    float v[16], t[16], res[16];
+    if (p.residual) {
+        const __amdgpu_buffer_rsrc_t rr = rows_view(p.residual, first, p.kstride, kb * 32, rows);
+        if (p.vector_rows) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const v4f r = load4(rr, ch0 + q * 4 < p.kstride ? (unsigned)(row * p.kstride + half * 16 + q * 4) * 4 : kOutOfRange, 0);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) res[q * 4 + e] = r[e];
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                res[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                       rr, ch0 + e < p.K ? (row * p.kstride + half * 16 + e) * 4 : (int)kOutOfRange, 0, 0));
+        }
+    }
+    read16<MT>(lds, 0, m, half, t);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) v[e] = acc[e] + t[e];
+    if (p.act == 1) relu16(v);
+    if constexpr (SLOW) {  // double-precision functions: through LDS, one value at a time, so that their registers are needed once
+        float* const own = reinterpret_cast<float*>(tile) + (row * kTilePitch / 4 + half * 16);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) own[e] = v[e];
+#pragma unroll 1
+        for (int e = 0; e < 16; ++e) own[e] = exhip_act(own[e], p.act);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] = own[e];
+    } else if (p.act == 3) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] = exhip_act(v[e], 3);
+    }
+    if (p.residual && !p.residual_last) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] += res[e];
+    }
+    if (p.post_relu) relu16(v);
+    if (p.bn_a) {
+        read16<MT>(lds, 2, m, half, t);
+        float b[16];
+        read16<MT>(lds, 3, m, half, b);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] = __builtin_fmaf(b[e], v[e], t[e]);
+    }
+    switch (p.post_op) {
+    case 0: break;
+    case 1 + EXHIP_UNARY_HARDSWISH: unary16<0>(v, p.alpha, p.beta); break;
+    case 1 + EXHIP_UNARY_LEAKYRELU: unary16<1>(v, p.alpha, p.beta); break;
+    case 1 + EXHIP_UNARY_HARDSIGMOID: unary16<3>(v, p.alpha, p.beta); break;
+    case 1 + EXHIP_UNARY_CLIP: unary16<4>(v, p.alpha, p.beta); break;
+    default:
+        read16<MT>(lds, 1, m, half, t);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] = v[e] >= 0.f ? v[e] : t[e] * v[e];
+    }
+    if (p.residual && p.residual_last) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] += res[e];
+    }
+    if (p.y) {
+        if (kb * 32 + 32 > p.K) {  // pad channels hold zeros
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                if (ch0 + e >= p.K) v[e] = 0.f;
+        }
+        const __amdgpu_buffer_rsrc_t yr = rows_view(p.y, first, p.kstride, kb * 32, rows);
+        if (p.vector_rows) {  // through LDS: eight neighbouring lanes write one pixel's 128 bytes
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const v4f o = {v[q * 4], v[q * 4 + 1], v[q * 4 + 2], v[q * 4 + 3]};
+                *reinterpret_cast<v4f*>(tile + row * kTilePitch + half * 64 + q * 16) = o;
+            }
+            const int scol = (lane & 7) * 16;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int srow = j * 8 + (lane >> 3);
+                const v4u o = *reinterpret_cast<const v4u*>(tile + srow * kTilePitch + scol);
+                const bool in = srow < rows && scol < (p.k_end - kb * 32) * 4;
+                __builtin_amdgcn_raw_buffer_store_b128(o, yr, in ? srow * p.kstride * 4 + scol : (int)kOutOfRange, 0, 0);
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v[e]), yr,
+                                                      row < rows && ch0 + e < p.k_end ? (row * p.kstride + half * 16 + e) * 4 : (int)kOutOfRange, 0, 0);
+        }
+    }
+    if (p.y_nchw && row < rows) {  // 32 neighbouring pixels of a channel per store instruction and half-wave
+        const unsigned per_image = (unsigned)(p.out_h * p.out_w);
+        const unsigned pix = first + row, img = exhip_divide(pix, per_image, p.image_magic, p.image_shift);
+        float* const dst = p.y_nchw + ((size_t)img * p.K + ch0) * per_image + (pix - img * per_image);
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+            if (ch0 + e < p.K) dst[(size_t)e * per_image] = v[e];
+    }
+}
+
+// R: requested steps in flight.
+template <int MT, int NT, int WK, int R, int MODE, bool SLOW>
+__global__ __launch_bounds__(WK > 4 ? 64 * WK : 256, 2) void conv_f32_kernel(const F32Params p) {
+    constexpr int WAVES = WK > 4 ? WK : 4, ITEMS = WAVES / WK;  // tiles per group
+    constexpr int RED = WK > 1 ? WAVES * MT * NT * 4096 : 0;    // the waves' partial sums
+    constexpr int OWNERS = MT * NT < WK ? MT * NT : WK;         // waves of a tile that run the epilogue
+    __shared__ __attribute__((aligned(16))) char lds_all[RED + ITEMS * OWNERS * wave_lds(MT)];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int part = wave % WK;
+    // workgroup ids are dealt round-robin to the 8 XCDs: give each XCD one contiguous run of items, so that the channel
+    // groups of a pixel tile, neighbouring tiles and the weights' re-reads share that XCD's L2
+    unsigned bid = blockIdx.x;
+    {
+        const unsigned per = gridDim.x >> 3;
+        if (bid < (per << 3)) bid = (bid & 7) * per + (bid >> 3);
+    }
+    const unsigned item = __builtin_amdgcn_readfirstlane(bid * ITEMS + wave / WK);
+    if (WK == 1 && item >= p.items) return;  // wave-uniform; that form has no barrier
+    const bool on = item < p.items;
+    const unsigned tile = __builtin_amdgcn_readfirstlane(exhip_divide(item, p.ch_groups, p.groups_magic, p.groups_shift));
+    const int kb0 = __builtin_amdgcn_readfirstlane((int)(item - tile * p.ch_groups) * MT);  // first 32-channel block
+    char* const lds = lds_all + RED + (wave / WK * OWNERS + (part < OWNERS ? part : 0)) * wave_lds(MT);
+
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.x), 0, (int)p.x_bytes, kRsrcWord3);
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.wp), 0, (int)p.w_bytes, kRsrcWord3);
+
+    // pixel fragments: lane = pixel (lane & 31), 16-byte half (lane >> 5) of each step
+    unsigned xoff[NT];
+    int iy[NT], ix[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        const unsigned pix = (tile * NT + n) * 32 + (lane & 31);
+        const bool in = on && pix < p.pixels;
+        if (MODE == kPoint && p.stride == 1) {
+            xoff[n] = in ? pix * (unsigned)p.xs_b + (lane >> 5) * 16 : kOutOfRange;
+        } else {
+            // the filter's top-left input pixel; its offset may lie in front of the tensor (padding), the taps inside the
+            // image never do, and 32-bit wrap-around of the sum gives their offsets
+            const unsigned per_image = (unsigned)(p.out_h * p.out_w);
+            const unsigned img = exhip_divide(pix, per_image, p.image_magic, p.image_shift), rem = pix - img * per_image;
+            const int oy = (int)exhip_divide(rem, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = (int)(rem - (unsigned)oy * (unsigned)p.out_w);
+            iy[n] = oy * p.stride - p.pad_t;
+            ix[n] = ox * p.stride - p.pad_l;
+            xoff[n] = (unsigned)((((int)img * p.in_h + iy[n]) * p.in_w + ix[n]) * p.xs_b + (lane >> 5) * 16);
+            if (MODE == kPair) ix[n] += lane >> 5;
+            if (!in) {
+                iy[n] = -0x40000000;
+                if (MODE == kPoint) xoff[n] = kOutOfRange;
+            }
+        }
+    }
+    const int s_first = p.start_s[part], steps = on ? p.start_s[part + 1] - s_first : 0;
+    // the next step to request: its weights, its filter row and tap, and how far it lies behind the tap's first channel
+    int w_at = s_first * 1024, r_at = p.start_r[part], q_at = p.start_q[part], c_at = p.start_c[part] * 32;
+    const int w_last = (p.n_ksteps - 1) * 1024, c_end = p.csteps * 32;
+    // a block past the packed ones (pad channels of a wide stride, the second half of a last pair) reads zeros
+    const int wbase = kb0 * p.n_ksteps * 1024;
+    unsigned woff[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) woff[m] = (kb0 + m) * 32 < p.K ? (unsigned)(m * p.n_ksteps * 1024 + lane * 16) : kOutOfRange;
+    unsigned xcur[NT];  // the lane's offset at the tap, out of range where the tap lies outside the image
+    auto enter_tap = [&]() {
+        const int off = r_at * p.row_b + q_at * p.xs_b;
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            const bool in = (unsigned)(iy[n] + r_at) < (unsigned)p.in_h && (unsigned)(ix[n] + q_at) < (unsigned)p.in_w &&
+                            (MODE != kPair || q_at + (lane >> 5) < p.kw);
+            xcur[n] = in ? xoff[n] + (unsigned)off : kOutOfRange;
+        }
+    };
+    if constexpr (MODE == kPoint) {
+#pragma unroll
+        for (int n = 0; n < NT; ++n) xcur[n] = xoff[n];
+    } else {
+        enter_tap();
+    }
+
+    v16f acc[MT][NT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[m][n][e] = 0.f;
+
+    v4f a[R][MT], b[R][NT];  // a ring of requested steps
+    // Requests are unconditional, so that the waits in front of the products count exactly what is in flight (behind a branch
+    // the compiler has to wait for everything: 510 cycles a step instead of 420). Those past this wave's run read what lies
+    // there -- the next part's operands, the last step's again -- and are not used. A step costs a handful of scalar
+    // instructions; where a tap ends, a branch without memory accesses finds the next one's offsets (evaluated in every
+    // step, the tap's tests stretched a step by 150 cycles where a SIMD has one wave).
+    auto request = [&](int u) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) a[u][m] = load4(wr, woff[m], wbase + w_at);
+#pragma unroll
+        for (int n = 0; n < NT; ++n) b[u][n] = load4(xr, xcur[n], c_at);
+        w_at = w_at + 1024 < w_last ? w_at + 1024 : w_last;
+        c_at += 32;
+        if constexpr (MODE == kPoint) {
+            c_at = c_at < c_end - 32 ? c_at : c_end - 32;
+        } else if (c_at == c_end) {
+            c_at = 0;
+            q_at += MODE == kPair ? 2 : 1;
+            if (q_at >= p.kw) {
+                q_at = 0;
+                ++r_at;
+            }
+            enter_tap();
+        }
+    };
+    auto step = [&](int u) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int n = 0; n < NT; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][m][e], b[u][n][e], acc[m][n], 0, 0, 0);
+    };
+#pragma unroll
+    for (int u = 0; u < R / 2; ++u) request(u);
+    // the channels' parameters: lane = channel of the wave's MT * 32, zeros beyond K and for an absent array
+    float par[kParams] = {};
+    {
+        auto load = [&](const float* src, unsigned offset, int count) {
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src), 0, src ? count * 4 : 0, kRsrcWord3);
+            return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)offset, 0, 0));
+        };
+        const unsigned at = (unsigned)(kb0 * 32 + lane) * 4;
+        par[0] = load(p.bias, at, p.K);
+        par[1] = load(p.slope, p.slope_shared ? 0 : at, p.slope_shared ? 1 : p.K);
+        par[2] = load(p.bn_a, at, p.K);
+        par[3] = load(p.bn_b, at, p.K);
+    }
+#pragma unroll
+    for (int u = R / 2; u < R; ++u) request(u);
+    int s = 0;
+    for (; s + R < steps; s += R) {
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            step(u);
+            request(u);
+            __builtin_amdgcn_sched_barrier(0);  // each slot is requested again as soon as its products have been issued
+        }
+    }
+    // (the loop leaves with the last steps, at most R, requested)
+    if (part < OWNERS && (MT == 2 || lane < 32)) {
+#pragma unroll
+        for (int i = 0; i < kParams; ++i) *reinterpret_cast<float*>(lds + (i * MT * 32 + lane) * 4) = par[i];
+    }
+#pragma unroll
+    for (int u = 0; u < R; ++u)
+        if (s + u < steps) step(u);
+    if constexpr (WK == 1) {
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                epilogue_block<MT, SLOW>(p, acc[m][n], (tile * NT + n) * 32, kb0 + m, m, lane, lds);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+    } else {
+        // wave `part` finishes the tile's blocks part, part + WK, ...: the others leave it their sums
+        constexpr int BLOCKS = MT * NT;
+        char* const red = lds_all + (wave - part) * BLOCKS * 4096;
+#pragma unroll
+        for (int blk = 0; blk < BLOCKS; ++blk) {
+            if (blk % WK == part) continue;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const v16f& c = acc[blk % MT][blk / MT];
+                const v4f o = {c[q * 4], c[q * 4 + 1], c[q * 4 + 2], c[q * 4 + 3]};
+                *reinterpret_cast<v4f*>(red + (part * BLOCKS + blk) * 4096 + q * 1024 + lane * 16) = o;
+            }
+        }
+        __syncthreads();
+        if (!on) return;
+#pragma unroll
+        for (int blk = 0; blk < BLOCKS; ++blk) {
+            if (blk % WK != part) continue;
+            v16f sum = acc[blk % MT][blk / MT];
+#pragma unroll
+            for (int w = 0; w < WK; ++w) {
+                if (w == blk % WK) continue;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const v4f o = *reinterpret_cast<const v4f*>(red + (w * BLOCKS + blk) * 4096 + q * 1024 + lane * 16);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) sum[q * 4 + e] += o[e];
+                }
+            }
+            epilogue_block<MT, SLOW>(p, sum, (tile * NT + blk / MT) * 32, kb0 + blk % MT, blk % MT, lane, lds);
+        }
+    }
+}
+
+template <int MT, int NT, int WK, int R, int MODE, bool SLOW>
+int go(exhip_ctx* ctx, F32Params& p, int kblocks) {
+    const long long tiles = ((long long)p.pixels + 32 * NT - 1) / (32 * NT);
+    p.tiles = (unsigned)tiles;
+    p.ch_groups = (unsigned)((kblocks + MT - 1) / MT);
+    const long long items = tiles * p.ch_groups;
+    EXHIP_REQUIRE(items < (1ll << 31) - 4, "conv: grid too large");
+    p.items = (unsigned)items;
+    exhip_host_divisor(p.ch_groups, &p.groups_magic, &p.groups_shift);
+    const int taps_w = MODE == kPair ? (p.kw + 1) / 2 : p.kw;
+    for (int i = 0; i <= WK; ++i) {
+        const int s = (int)((long long)p.n_ksteps * i / WK), tap = s / p.csteps;
+        p.start_s[i] = s;
+        p.start_c[i] = s % p.csteps;
+        p.start_r[i] = tap / taps_w;
+        p.start_q[i] = tap % taps_w * (MODE == kPair ? 2 : 1);
+    }
+    constexpr int WAVES = WK > 4 ? WK : 4, ITEMS = WAVES / WK;
+    hipLaunchKernelGGL((conv_f32_kernel<MT, NT, WK, R, MODE, SLOW>), dim3((p.items + ITEMS - 1) / ITEMS), dim3(64 * WAVES), 0, ctx->stream, p);
+    EXHIP_LAUNCH_CHECK();
+    return 0;
+}
+
+template <int MODE>
+int pick(exhip_ctx* ctx, F32Params& p, int kblocks) {
+    if (p.act == 4 || p.act == 5) return go<1, 1, 1, 8, MODE, true>(ctx, p, kblocks);
+    // The tile and the split that a model of the launch says are shortest, in microseconds: rounds of groups on 256 CUs, each
+    // as long as its waves' products (0.028 a product and SIMD), the blocks' epilogue (1 each, shared by the waves of a tile) and
+    // the exchange of a split (0.4), or the time the operands take at 12 TB/s where that is longer. Over 28 layers from
+    // 1 x 64 x 8 x 4 to 30 GFLOP its choice is within 1 % of the fastest form of the list on average.
+    struct Config { int mt, nt, wk; };
+    static constexpr Config kConfigs[] = {{2, 2, 1}, {2, 1, 1}, {2, 1, 2}, {2, 1, 4}, {1, 1, 4}, {1, 1, 8}, {1, 2, 1}, {1, 1, 2}};
+    constexpr int kCount = (int)(sizeof(kConfigs) / sizeof(kConfigs[0]));
+    int best = 0;
+    double best_cost = 0;
+    for (int i = 0; i < kCount; ++i) {
+        const Config& c = kConfigs[i];
+        if (c.wk > p.n_ksteps) continue;
+        const int blocks = c.mt * c.nt, waves = std::max(4, c.wk), steps = (p.n_ksteps + c.wk - 1) / c.wk;
+        const double tiles = (double)(((long long)p.pixels + 32 * c.nt - 1) / (32 * c.nt) * ((kblocks + c.mt - 1) / c.mt));
+        const double rounds = std::ceil(std::ceil(tiles * c.wk / waves) / 256) * (waves / 4);
+        const double round = steps * blocks * 4 * 0.0278 + (double)blocks / std::min(c.wk, blocks) + (c.wk > 1 ? 0.4 : 0);
+        const double cost = std::max(rounds * round, tiles * c.wk * steps * (c.mt + c.nt) * 1024 / 12e6);
+        if (i == 0 || cost < best_cost) {
+            best_cost = cost;
+            best = i;
+        }
+    }
+    if (g_exhip_options.f32_tile > 0) best = std::min(g_exhip_options.f32_tile, kCount) - 1;
+    switch (best) {
+    case 0: return go<2, 2, 1, 4, MODE, false>(ctx, p, kblocks);
+    case 1: return go<2, 1, 1, 6, MODE, false>(ctx, p, kblocks);
+    case 2: return go<2, 1, 2, 6, MODE, false>(ctx, p, kblocks);
+    case 3: return go<2, 1, 4, 6, MODE, false>(ctx, p, kblocks);
+    case 4: return go<1, 1, 4, 8, MODE, false>(ctx, p, kblocks);
+    case 5: return go<1, 1, 8, 8, MODE, false>(ctx, p, kblocks);
+    case 6: return go<1, 2, 1, 6, MODE, false>(ctx, p, kblocks);
+    default: return go<1, 1, 2, 8, MODE, false>(ctx, p, kblocks);
+    }
+}
+
+int taps_steps(const exhip_conv_desc* d) { return d->c_stride == 4 ? d->kh * ((d->kw + 1) / 2) : d->kh * d->kw * ((d->c + 7) / 8); }
+
+}  // namespace
+
+int exhip_conv_f32_validate(const exhip_conv_desc* d) {
+    EXHIP_REQUIRE(d, "conv: NULL descriptor");
+    EXHIP_REQUIRE(d->n > 0 && d->c > 0 && d->h > 0 && d->w > 0 && d->k > 0, "conv: empty shape");
+    EXHIP_REQUIRE(d->kh > 0 && d->kw > 0 && d->sh > 0 && d->sw > 0, "conv: bad kernel/stride");
+    EXHIP_REQUIRE(d->sh == d->sw, "conv: MFMA path needs equal strides (got %dx%d)", d->sh, d->sw);
+    EXHIP_REQUIRE(d->pt >= 0 && d->pb >= 0 && d->pl >= 0 && d->pr >= 0, "conv: negative padding");
+    EXHIP_REQUIRE(d->h + d->pt + d->pb >= d->kh && d->w + d->pl + d->pr >= d->kw, "conv: kernel larger than padded input");
+    EXHIP_REQUIRE(d->c_stride >= d->c, "conv: c_stride %d < c %d", d->c_stride, d->c);
+    EXHIP_REQUIRE(d->c_stride == 4 || d->c_stride % 8 == 0, "conv: input pixel is %d bytes; need a multiple of 32, or 16", d->c_stride * 4);
+    EXHIP_REQUIRE((long long)d->h * d->w * d->c_stride * 4 < (1ll << 31), "conv: one input image exceeds 2 GiB");
+    EXHIP_REQUIRE((long long)((d->k + 31) / 32) * taps_steps(d) * 1024 < (1ll << 31), "conv: the packed weights exceed 2 GiB");
+    return 0;
+}
+
+size_t exhip_conv_f32_packed_bytes(const exhip_conv_desc* d) {
+    if (exhip_conv_f32_validate(d)) return 0;
+    return (size_t)((d->k + 31) / 32) * taps_steps(d) * 1024;
+}
+
+// [32-channel block][step: filter row, tap, 8 channels (or 2 taps x 4 channels)][lane][4 floats]; the accumulator of
+// v_mfma_f32_32x32x2_f32 then holds sixteen neighbouring channels per lane.
+int exhip_conv_f32_pack_weights(const exhip_conv_desc* d, const float* w, float* out) {
+    const int rc = exhip_conv_f32_validate(d);
+    if (rc) return rc;
+    const bool pair = d->c_stride == 4;
+    const int C = d->c, K = d->k, KH = d->kh, KW = d->kw, csteps = pair ? 1 : (C + 7) / 8;
+    for (int kb = 0; kb < (K + 31) / 32; ++kb)
+        for (int r = 0; r < KH; ++r)
+            for (int q0 = 0; q0 < KW; q0 += pair ? 2 : 1)
+                for (int j = 0; j < csteps; ++j)
+                    for (int lane = 0; lane < 64; ++lane) {
+                        const int rr = lane % 32, h = lane / 32;
+                        const int k = kb * 32 + ((rr / 4) % 2) * 16 + (rr / 8) * 4 + rr % 4;
+                        const int q = pair ? q0 + h : q0;
+                        for (int e = 0; e < 4; ++e) {
+                            const int c = pair ? e : j * 8 + h * 4 + e;
+                            *out++ = k < K && c < C && q < KW ? w[(((size_t)k * C + c) * KH + r) * KW + q] : 0.f;
+                        }
+                    }
+    return 0;
+}
+
+extern "C" int exhip_conv2d_f32(exhip_ctx* ctx, const exhip_conv_desc* d, const float* x, const void* wp,
+                                const float* bias, const float* residual, float* y_f32_nhwc, float* y_f32_nchw) {
+    EXHIP_REQUIRE(y_f32_nhwc || y_f32_nchw, "exhip_conv2d_f32: no output requested");
+    EXHIP_REQUIRE(ctx, "conv: NULL ctx");
+    const int rc = exhip_conv_f32_validate(d);
+    if (rc) return rc;
+    EXHIP_REQUIRE(x && wp, "conv: NULL input or weights");
+    EXHIP_REQUIRE(d->k_stride >= d->k || (!y_f32_nhwc && !residual), "conv: k_stride %d < k %d", d->k_stride, d->k);
+    EXHIP_REQUIRE(!bias || (uintptr_t)bias % 16 == 0, "conv: scale and bias arrays must be 16-byte aligned");
+    EXHIP_REQUIRE((uintptr_t)x % 16 == 0 && (uintptr_t)wp % 16 == 0, "conv: input and weights must be 16-byte aligned");
+    EXHIP_REQUIRE((d->post_op >= 0 && d->post_op <= 1 + EXHIP_UNARY_CLIP && d->post_op != 1 + EXHIP_UNARY_SIGMOID) ||
+                      (d->post_op == EXHIP_POST_PRELU && d->post_slope),
+                  "conv: post_op %d is not an activation the epilogue applies", d->post_op);
+    EXHIP_REQUIRE((d->post_bn_a == nullptr) == (d->post_bn_b == nullptr), "conv: half a BatchNorm");
+    F32Params p = {};
+    const int oh = (d->h + d->pt + d->pb - d->kh) / d->sh + 1, ow = (d->w + d->pl + d->pr - d->kw) / d->sw + 1;
+    p.wp = static_cast<const char*>(wp);
+    p.bias = bias; p.bn_a = d->post_bn_a; p.bn_b = d->post_bn_b;
+    p.slope = d->post_op == EXHIP_POST_PRELU ? d->post_slope : nullptr;
+    p.in_h = d->h; p.in_w = d->w; p.out_h = oh; p.out_w = ow;
+    p.stride = d->sh; p.pad_t = d->pt; p.pad_l = d->pl; p.kh = d->kh; p.kw = d->kw;
+    p.xs_b = d->c_stride * 4;
+    p.row_b = d->w * p.xs_b;
+    const bool pair = d->c_stride == 4;
+    p.csteps = pair ? 1 : (d->c + 7) / 8;
+    p.n_ksteps = taps_steps(d);
+    const int kblocks = (d->k + 31) / 32;
+    p.w_bytes = (unsigned)((size_t)kblocks * p.n_ksteps * 1024);
+    p.K = d->k;
+    p.kstride = d->k_stride;
+    p.k_end = d->exact_k || !y_f32_nhwc ? d->k : std::max(d->k, d->k_stride);
+    p.act = d->act; p.post_relu = d->post_relu; p.post_op = d->post_op; p.slope_shared = d->post_slope_shared;
+    p.residual_last = d->residual_last;
+    p.alpha = d->post_alpha; p.beta = d->post_beta;
+    p.vector_rows = d->k_stride % 4 == 0 && (uintptr_t)y_f32_nhwc % 16 == 0 && (uintptr_t)residual % 16 == 0 && p.k_end % 4 == 0;
+    exhip_host_divisor((unsigned)(oh * ow), &p.image_magic, &p.image_shift);
+    exhip_host_divisor((unsigned)ow, &p.width_magic, &p.width_shift);
+    // blocks past the last channel's (pad channels of a wider stride) get zeros too: weights beyond the view read zero
+    const int write_blocks = (p.k_end + 31) / 32;
+    const long long img_bytes = (long long)d->h * p.row_b, per_image = (long long)oh * ow;
+    EXHIP_REQUIRE(per_image < (1ll << 31) - 256, "conv: more than 2^31 output pixels in an image");
+    // input offsets are 32-bit: as many images per launch as fit below 4 GiB and 2^31 pixels
+    const long long most = std::max(1ll, std::min((0x7fff0000ll) / img_bytes, ((1ll << 31) - 256) / per_image));
+    for (long long n0 = 0; n0 < d->n; n0 += most) {
+        const long long n = std::min<long long>(most, d->n - n0);
+        p.x = reinterpret_cast<const char*>(x) + n0 * img_bytes;
+        p.x_bytes = (unsigned)(n * img_bytes);
+        p.pixels = (unsigned)(n * per_image);
+        p.residual = residual ? residual + n0 * per_image * d->k_stride : nullptr;
+        p.y = y_f32_nhwc ? y_f32_nhwc + n0 * per_image * d->k_stride : nullptr;
+        p.y_nchw = y_f32_nchw ? y_f32_nchw + n0 * per_image * d->k : nullptr;
+        const int go_rc = pair ? pick<kPair>(ctx, p, write_blocks)
+                          : d->kh == 1 && d->kw == 1 && !d->pt && !d->pb && !d->pl && !d->pr ? pick<kPoint>(ctx, p, write_blocks)
+                                                                                             : pick<kTaps>(ctx, p, write_blocks);
+        if (go_rc) return go_rc;
+    }
+    return 0;
+}

@@ -9,7 +9,7 @@
 // halo tile. The next stage's global loads are issued before the current stage's MFMAs and written to
 // LDS afterwards.
 //
-// One k-step is 32 bytes of reduction per pixel: 32 int8 / 16 half / 8 float input channels of one
+// One k-step is 32 bytes of reduction per pixel: 32 int8 / 16 half input channels of one
 // tap ("generic" form), or, for first layers with <= 4 channels, one whole filter row of up to 8 (int8)
 // or 4 (half) neighbouring pixels ("packed-row" form), which keeps the 7x7x3 stem from being padded
 // out to 32 channels.
@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "common.h"
+#include "conv_f32.h"
 #include "conv_i8_lean.h"
 #include "conv_pw.h"
 
@@ -67,8 +68,8 @@ struct ConvParams {
     const float* scale;
     const float* bias;
     const void* residual;
-    void* y_q;       // i8: int8 NHWC ; f16: half NHWC ; f32: unused
-    void* y_nhwc;    // f32 NHWC (i8 and f32 kernels)
+    void* y_q;       // i8: int8 NHWC ; f16: half NHWC
+    void* y_nhwc;    // f32 NHWC (i8 kernel)
     void* y_nchw;    // f32 NCHW
     void* y_nchw_h;  // half NCHW (f16 kernel)
     int32_t* acc_nchw;
@@ -121,18 +122,13 @@ struct ConvParams {
 
 template <int DT> struct Acc { typedef v16i type; };
 template <> struct Acc<EXHIP_F16> { typedef v16f type; };
-template <> struct Acc<EXHIP_F32> { typedef v16f type; };
 
 template <int DT>
 __device__ __forceinline__ void mma(typename Acc<DT>::type& acc, const v4i& a, const v4i& b) {
     if constexpr (DT == EXHIP_I8) {
         acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, acc, 0, 0, 0);
-    } else if constexpr (DT == EXHIP_F16) {
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, b), acc, 0, 0, 0);
     } else {
-        const v4f af = __builtin_bit_cast(v4f, a), bf = __builtin_bit_cast(v4f, b);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(af[e], bf[e], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, b), acc, 0, 0, 0);
     }
 }
 
@@ -1906,6 +1902,7 @@ extern "C" int exhip_conv_out_hw(const exhip_conv_desc* d, int* oh, int* ow) {
 }
 
 extern "C" size_t exhip_conv_packed_bytes(const exhip_conv_desc* d, int dtype) {
+    if (dtype == EXHIP_F32) return exhip_conv_f32_packed_bytes(d);
     Plan pl;
     if (dtype < 0 || dtype > 2 || make_plan(d, dtype, &pl)) return 0;
     return (size_t)pl.ktiles * pl.n_chunks * d->kh * pl.KWe * pl.KS * (pl.TM / 32) * 1024;
@@ -1914,12 +1911,12 @@ extern "C" size_t exhip_conv_packed_bytes(const exhip_conv_desc* d, int dtype) {
 extern "C" int exhip_conv_pack_weights(const exhip_conv_desc* d, int dtype, const void* w, void* packed) {
     EXHIP_REQUIRE(w && packed, "exhip_conv_pack_weights: NULL argument");
     EXHIP_REQUIRE(dtype >= 0 && dtype <= 2, "exhip_conv_pack_weights: bad dtype %d", dtype);
+    if (dtype == EXHIP_F32) return exhip_conv_f32_pack_weights(d, (const float*)w, (float*)packed);
     Plan pl;
     int rc = make_plan(d, dtype, &pl);
     if (rc) return rc;
     if (dtype == EXHIP_I8) pack_weights_t<int8_t>(d, dtype, pl, (const int8_t*)w, (char*)packed);
-    else if (dtype == EXHIP_F16) pack_weights_t<uint16_t>(d, dtype, pl, (const uint16_t*)w, (char*)packed);
-    else pack_weights_t<float>(d, dtype, pl, (const float*)w, (char*)packed);
+    else pack_weights_t<uint16_t>(d, dtype, pl, (const uint16_t*)w, (char*)packed);
     return 0;
 }
 
@@ -2008,13 +2005,4 @@ extern "C" int exhip_conv2d_f16(exhip_ctx* ctx, const exhip_conv_desc* d, const 
     p.x = (const char*)x; p.wp = (const char*)wp; p.bias = bias; p.residual = residual;
     p.y_q = y_f16_nhwc; p.y_nchw_h = y_f16_nchw; p.y_nchw = y_f32_nchw;
     return run_conv<EXHIP_F16>(ctx, d, p);
-}
-
-extern "C" int exhip_conv2d_f32(exhip_ctx* ctx, const exhip_conv_desc* d, const float* x, const void* wp,
-                                const float* bias, const float* residual, float* y_f32_nhwc, float* y_f32_nchw) {
-    EXHIP_REQUIRE(y_f32_nhwc || y_f32_nchw, "exhip_conv2d_f32: no output requested");
-    ConvParams p = {};
-    p.x = (const char*)x; p.wp = (const char*)wp; p.bias = bias; p.residual = residual;
-    p.y_nhwc = y_f32_nhwc; p.y_nchw = y_f32_nchw;
-    return run_conv<EXHIP_F32>(ctx, d, p);
 }

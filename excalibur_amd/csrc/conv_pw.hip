@@ -56,7 +56,7 @@ struct PwParams {
     int exact;                // channels [0, K) only: blocks past K are not written (the results lie inside a wider tensor)
     unsigned pixels, x_bytes, w_bytes;
     unsigned items, ch_groups;   // waves with work; 32 * MT channel groups per pixel tile
-    unsigned groups_magic, image_magic, width_magic;  // divide() by ch_groups, out_h * out_w, out_w
+    unsigned groups_magic, image_magic, width_magic;  // exhip_divide() by ch_groups, out_h * out_w, out_w
     int groups_shift, image_shift, width_shift;
     int xs_b;                    // bytes per input pixel
     int n_ksteps;                // 32-byte k-steps per pixel
@@ -285,10 +285,6 @@ __device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[
     }
 }
 
-__device__ __forceinline__ unsigned divide(unsigned n, unsigned d, unsigned magic, int shift) {  // n < 2^31, magic of host_divisor()
-    return d == 1 ? n : __umulhi(n, magic) >> shift;
-}
-
 // U: k-steps per request round; two rounds are in flight.
 template <int DT, int MT, int NT, int U, bool TAPS, typename EP>
 __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
@@ -303,7 +299,7 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
     }
     const unsigned item = __builtin_amdgcn_readfirstlane(bid * 4 + wave);
     if (item >= p.items) return;  // wave-uniform; the kernel has no barrier
-    const unsigned tile = __builtin_amdgcn_readfirstlane(divide(item, p.ch_groups, p.groups_magic, p.groups_shift));
+    const unsigned tile = __builtin_amdgcn_readfirstlane(exhip_divide(item, p.ch_groups, p.groups_magic, p.groups_shift));
     const int kb0 = __builtin_amdgcn_readfirstlane((int)(item - tile * p.ch_groups) * MT);  // first 32-channel block
     char* const lds = lds_all + wave * wave_bytes(DT, MT);
 
@@ -320,8 +316,8 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
             // the filter's top-left input pixel; its offset may lie in front of the tensor (padding), the taps inside the
             // image never do, and 32-bit wrap-around of the sum gives their offsets
             const unsigned per_image = (unsigned)(p.out_h * p.out_w);
-            const unsigned img = divide(pix, per_image, p.image_magic, p.image_shift), rem = pix - img * per_image;
-            const int oy = (int)divide(rem, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = (int)(rem - (unsigned)oy * (unsigned)p.out_w);
+            const unsigned img = exhip_divide(pix, per_image, p.image_magic, p.image_shift), rem = pix - img * per_image;
+            const int oy = (int)exhip_divide(rem, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = (int)(rem - (unsigned)oy * (unsigned)p.out_w);
             const int iy = oy * p.stride - p.pad_t, ix = ox * p.stride - p.pad_l;
             xoff[nt] = (((int)img * p.in_h + iy) * p.in_w + ix) * p.xs_b + (lane >> 5) * 16;
             unsigned m = 0;
@@ -431,18 +427,6 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
     pw_epilogue<DT, MT, NT, EP>(p, acc, tile * NT * 32, kb0, lane, lds);
 }
 
-// magic and shift of divide() for divisors from 2 on: with s = ceil(log2 d) and magic = ceil(2^(31 + s) / d) < 2^32,
-// n * magic >> (31 + s) is n / d for every n < 2^31 (the rounding of magic adds less than n / 2^31 < 1 part of d)
-void host_divisor(unsigned d, unsigned* magic, int* shift) {
-    *magic = 0;
-    *shift = 0;
-    if (d <= 1) return;
-    int s = 0;
-    while ((1ull << s) < d) ++s;
-    *magic = (unsigned)(((1ull << (31 + s)) + d - 1) / d);
-    *shift = s - 1;
-}
-
 template <int DT, int MT, int NT, int U, bool TAPS, typename EP>
 int go(exhip_ctx* ctx, const PwParams& p) {
     hipLaunchKernelGGL((conv1x1_pw_kernel<DT, MT, NT, U, TAPS, EP>), dim3((p.items + 3) / 4), dim3(256), 0, ctx->stream, p);
@@ -488,7 +472,7 @@ int launch(exhip_ctx* ctx, PwParams& p, int kblocks) {
     const long long items = tiles * p.ch_groups;
     if (items >= (1ll << 31) - 4) return EXHIP_ERR_UNSUPPORTED;
     p.items = (unsigned)items;
-    host_divisor(p.ch_groups, &p.groups_magic, &p.groups_shift);
+    exhip_host_divisor(p.ch_groups, &p.groups_magic, &p.groups_shift);
     if constexpr (MT + NT > 3) return go<DT, MT, NT, 2, TAPS, EpAny>(ctx, p);
     // A launch of at most two waves per SIMD is as long as one wave's chain of load round trips: sixteen k-steps in flight
     // where there are more than eight. Larger ones hide each other's round trips and want the registers for more waves.
@@ -544,8 +528,8 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
     p.post_alpha = g.post_alpha; p.post_beta = g.post_beta;
     p.in_h = t.in_h; p.in_w = t.in_w; p.out_h = t.out_h; p.out_w = t.out_w; p.stride = t.stride; p.pad_t = t.pad_t; p.pad_l = t.pad_l;
     p.kh = t.kh; p.kw = t.kw;
-    host_divisor((unsigned)(t.out_h * t.out_w), &p.image_magic, &p.image_shift);
-    host_divisor((unsigned)t.out_w, &p.width_magic, &p.width_shift);
+    exhip_host_divisor((unsigned)(t.out_h * t.out_w), &p.image_magic, &p.image_shift);
+    exhip_host_divisor((unsigned)t.out_w, &p.width_magic, &p.width_shift);
     int s = 0;
     for (int cc = 0; cc < t.n_chunks; ++cc)
         for (int r = 0; r < t.kh; ++r)

@@ -1,0 +1,68 @@
+"""The float32 convolution kernel (conv_f32.hip): every wave tile and split of its list on ragged shapes, against the CPU
+oracle's layers; and what surrounds the products -- pad channels, odd channel strides, four-channel pixels, the shortcut."""
+import numpy as np
+import pytest
+
+from excalibur_amd import hip
+from oracle import port
+from tests import cases
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = hip.Ctx(0)
+    yield c
+    c.close()
+
+
+@pytest.fixture(params=range(9))
+def tile(request):
+    hip.set_option("f32_tile", request.param)
+    yield request.param
+    hip.set_option("f32_tile", 0)
+
+
+SHAPES = [
+    # seed, n, c, h, w, k, kernel, stride, pad, c_stride, k_stride, shortcut
+    (900, 1, 8, 1, 1, 1, 1, 1, 0, 8, 1, False),             # one pixel, one step, one channel: splits find too few steps
+    (901, 2, 24, 9, 7, 33, 3, 1, 1, 24, 33, True),          # ragged pixels and channels, rows without 16-byte alignment
+    (902, 1, 3, 17, 19, 40, 3, 2, 1, 4, 64, False),         # 16-byte pixels (two taps a step), a pad block and pad channels
+    (903, 1, 4, 12, 11, 32, (1, 4), 1, 0, 4, 32, False),    # the same with an even row of taps
+    (904, 3, 40, 13, 13, 255, 1, 1, 0, 48, 256, True),      # a head: one pad channel
+    (905, 2, 72, 10, 14, 96, 1, 2, 0, 72, 96, False),       # strided 1x1: single taps, never outside
+    (906, 1, 64, 20, 21, 64, 3, 1, 1, 64, 64, True),        # 72 steps
+    (907, 1, 16, 15, 15, 32, 9, 2, 4, 16, 32, False),       # 81 taps
+    (908, 1, 136, 6, 5, 160, (2, 3), 1, (0, 1, 2, 0), 136, 160, True),  # uneven padding
+]
+
+
+@pytest.mark.parametrize("args", SHAPES, ids=[f"s{a[0]}" for a in SHAPES])
+def test_conv_f32_tiles_and_splits(ctx, tile, args):
+    seed, n, c, h, w, k, kernel, stride, pad, cs, ks, shortcut = args
+    case = cases.conv_f32_case(seed, n, c, h, w, k, kernel, stride, pad, act=0)
+    want = cases.oracle_eval(case)
+    r = np.random.default_rng(seed)
+    res = r.uniform(-1, 1, want.shape).astype(np.float32)
+    d = ctx.conv_desc(n, c, h, w, k, kernel, stride, pad, 0, cs, ks, int(shortcut))
+    oh, ow = ctx.conv_out_hw(d)
+    x = np.zeros((n, h, w, cs), np.float32)
+    x[..., :c] = case["x"].transpose(0, 2, 3, 1)
+    guard = 64  # floats behind the tensor that must keep their value
+    y = ctx.array(np.full(n * oh * ow * ks + guard, 7.0, np.float32))
+    planar = ctx.array(np.full(want.size + guard, 7.0, np.float32))
+    rd = None
+    if shortcut:
+        padded = np.zeros((n, oh, ow, ks), np.float32)
+        padded[..., :k] = res.transpose(0, 2, 3, 1)
+        rd = ctx.array(padded)
+        want = port.relu(port.binaryop_add(want, res))
+    ctx.conv2d_f32(d, ctx.array(x), ctx.pack_conv_weights(d, hip.F32, case["wt"]), ctx.array(case["bias"]), rd, y, planar)
+    ctx.sync()
+    got, flat = y.download(), planar.download()
+    assert (got[-guard:] == 7.0).all() and (flat[-guard:] == 7.0).all()
+    got = got[:-guard].reshape(n, oh, ow, ks)
+    assert cases.check_value(got[..., :k].transpose(0, 3, 1, 2), want, 1e-5) == 0
+    assert not got[..., k:].any()
+    assert np.array_equal(flat[:-guard].reshape(want.shape), got[..., :k].transpose(0, 3, 1, 2))
