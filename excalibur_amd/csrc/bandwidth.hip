@@ -2239,6 +2239,11 @@ static int dw_nhwc_f16(exhip_ctx* ctx, const uint16_t* x, const float* w9, const
         const size_t want = (size_t)256 * 14 * 64;
         int bands = (int)std::min<size_t>((size_t)std::max(1, oh / 7), std::max<size_t>((oh + 13) / 14, (want + per_band - 1) / per_band));
         int band_rows = (oh + bands - 1) / bands;
+        // A launch with at most one wave per SIMD is as long as one wave's chain of rows (about 0.9 us each at stride 1):
+        // the shortest of 1, 2 and 4 rows with which it stays one (1 x 128 x 28 x 28: 10.0 us with seven rows, 4.9 with one;
+        // 16 x 256 x 28 x 28: 10.9, with four 8.2, with one -- three waves per SIMD -- 11.2)
+        for (int rows = 4; rows >= 1; rows /= 2)
+            if (rows < band_rows && per_band / 64 * ((oh + rows - 1) / rows) <= 1024) band_rows = rows;
         if (env_rows > 0) band_rows = std::min(env_rows, oh);
         bands = (oh + band_rows - 1) / band_rows;
         const size_t total = per_band * bands;
