@@ -464,24 +464,27 @@ __global__ __launch_bounds__(kBlock) void dwconv3x3_nhwc_f16_kernel(const uint16
     *reinterpret_cast<v4i*>(y + ((n * OH + oy) * OW + ox) * cs + g * 8) = o;
 }
 
-// Strip form of the same layer for stride 1 and 2 and the activations that need no transcendental: a thread owns
-// 4 channels (8 bytes) of a strip of PX output pixels and walks a band of output rows, keeping the three input
-// rows it needs as stored (two halves to a register), so every input value is fetched once per band and the 36
+// Strip form of the same layer, on half or float storage, for stride 1 and 2 and the activations that need no transcendental: a
+// thread owns 4 channels of a strip of PX output pixels and walks a band of output rows, keeping the three input
+// rows it needs as stored (two halves or one float to a register), so every input value is fetched once per band and the 36
 // weights once per thread. The next step's rows are requested before the current outputs are computed. Loads and
 // stores go through buffer descriptors over the whole tensors: a tap outside the image, or an output pixel beyond
 // the row's end, gets an offset beyond the descriptor's range and reads as zero / is dropped. The kernel is bound
 // by vector ALU issue as much as by memory, hence the template on the activation and the masked, packed stores.
 // Arithmetic order per output is that of dw_pixel.
-template <int STRIDE, int PX, int ACT>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 4))) void dwconv3x3_nhwc_f16_strip_kernel(const uint16_t* __restrict__ x,
+template <typename T, int STRIDE, int PX, int ACT>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 4))) void dwconv3x3_nhwc_strip_kernel(const T* __restrict__ x,
                                                                           const float* __restrict__ w,
                                                                           const float* __restrict__ bias,
-                                                                          uint16_t* __restrict__ y, int C, int H, int W,
+                                                                          T* __restrict__ y, int C, int H, int W,
                                                                           int cs, int OH, int OW, int pt, int pl,
                                                                           int band_rows, int bands, int strips,
                                                                           unsigned x_bytes, unsigned y_bytes, size_t total,
                                                                           const float* __restrict__ slope, int slope_shared) {
-    constexpr int NC = (PX - 1) * STRIDE + 3, KEEP = 3 - STRIDE;
+    constexpr bool HALF = sizeof(T) == 2;
+    constexpr int ES = sizeof(T);
+    typedef typename std::conditional<HALF, v4h, v4f>::type vec;
+    constexpr int NC = (PX - 1) * STRIDE + 3;
     // out-of-range markers: a tensor is at most 2^30 bytes, so a valid row offset plus the column marker, the row
     // marker plus anything, and both markers together all land beyond the descriptor's range without wrapping
     constexpr unsigned kRowOutside = 0x80000000u, kColOutside = 0x40000000u;
@@ -517,24 +520,24 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 4))) 
 #pragma unroll
         for (int e = 0; e < 4; ++e) sl[e] = slope[slope_shared ? 0 : min(c0 + e, C - 1)];
     }
-    // channels of the padding are stored as zero halves
+    // channels of the padding are stored as zeros
     const int keep_lo = (c0 < C ? 0xffff : 0) | (c0 + 1 < C ? 0xffff0000 : 0);
     const int keep_hi = (c0 + 2 < C ? 0xffff : 0) | (c0 + 3 < C ? 0xffff0000 : 0);
     const bool ragged_c = (C & 3) != 0 || cs != C;  // uniform over the launch: whole groups of four channels need no masks
     const int oy0 = band * band_rows, oy1 = min(OH, oy0 + band_rows);
     const int ox0 = xs * PX, ix0 = ox0 * STRIDE - pl;
-    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x), 0, (int)x_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(x), 0, (int)x_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc(y, 0, (int)y_bytes, 0x00020000);
-    const int row_b = W * cs * 2, orow_b = OW * cs * 2;
-    const int img_off = n * H * row_b + c0 * 2;
+    const int row_b = W * cs * ES, orow_b = OW * cs * ES;
+    const int img_off = n * H * row_b + c0 * ES;
     unsigned col_off[NC], ocol_off[PX];  // byte offsets within a row, or the marker
 #pragma unroll
     for (int cidx = 0; cidx < NC; ++cidx) {
         const int ix = ix0 + cidx;
-        col_off[cidx] = ix >= 0 && ix < W ? (unsigned)(ix * cs * 2) : kColOutside;
+        col_off[cidx] = ix >= 0 && ix < W ? (unsigned)(ix * cs * ES) : kColOutside;
     }
 #pragma unroll
-    for (int px = 0; px < PX; ++px) ocol_off[px] = ox0 + px < OW ? (unsigned)((ox0 + px) * cs * 2) : kColOutside;
+    for (int px = 0; px < PX; ++px) ocol_off[px] = ox0 + px < OW ? (unsigned)((ox0 + px) * cs * ES) : kColOutside;
     // The input rows live in a ring of 3 + D * STRIDE register rows: output row t reads ring slots (t * STRIDE + a) % R,
     // a = 0 .. 2, while the rows the next D output rows add are already on their way into the slots behind them. The
     // row loop is unrolled over one turn of the ring, so every slot index is a constant and no row is ever copied.
@@ -542,16 +545,17 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 4))) 
     // cover the memory latency with three waves per SIMD).
     constexpr int D = STRIDE == 1 ? 2 : 1;
     constexpr int R = 3 + D * STRIDE, TURN = R;  // R and STRIDE are coprime (4 or 5 and 1, 5 and 2): a turn is R output rows
-    v4h r[R][NC];
-    auto fetch = [&](int iy, v4h (&dst)[NC]) {
+    vec r[R][NC];
+    auto fetch = [&](int iy, vec (&dst)[NC]) {
         const unsigned row_off = iy >= 0 && iy < H ? (unsigned)(img_off + iy * row_b) : kRowOutside;
 #pragma unroll
         for (int cidx = 0; cidx < NC; ++cidx)
-            dst[cidx] = __builtin_bit_cast(v4h, __builtin_amdgcn_raw_buffer_load_b64(xr, (int)(row_off + col_off[cidx]), 0, 0));
+            if constexpr (HALF) dst[cidx] = __builtin_bit_cast(v4h, __builtin_amdgcn_raw_buffer_load_b64(xr, (int)(row_off + col_off[cidx]), 0, 0));
+            else dst[cidx] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(row_off + col_off[cidx]), 0, 0));
     };
 #pragma unroll
     for (int a = 0; a < (D - 1) * STRIDE + 3; ++a) fetch(oy0 * STRIDE - pt + a, r[a]);
-    unsigned orow_off = (unsigned)((n * OH + oy0) * orow_b + c0 * 2);
+    unsigned orow_off = (unsigned)((n * OH + oy0) * orow_b + c0 * ES);
     // one output row, PH = its position in the turn
     auto row = [&](auto ph, int oy) {
         constexpr int PH = decltype(ph)::value;
@@ -575,7 +579,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 4))) 
                 }
                 // activations 0 (none), 1 (ReLU), 3 (ReLU6 as the reference writes it)
                 if (ACT == kDwPrelu) {
-                    sum = exhip_h2f(exhip_f2h(sum));  // the PReLU layer reads the stored half
+                    if (HALF) sum = exhip_h2f(exhip_f2h(sum));  // the PReLU layer reads the stored half
                     sum = sum >= 0.f ? sum : sl[e] * sum;
                 } else if (ACT != 0) {
                     sum = (0.f > sum) ? 0.f : sum;
@@ -583,12 +587,20 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 4))) 
                 if (ACT == 3) sum = sum <= 6.f ? sum : 0.f;
                 res[e] = sum;
             }
-            v2i o = __builtin_bit_cast(v2i, __builtin_convertvector(res, v4h));
-            if (ragged_c) {
-                o[0] &= keep_lo;
-                o[1] &= keep_hi;
+            if constexpr (HALF) {
+                v2i o = __builtin_bit_cast(v2i, __builtin_convertvector(res, v4h));
+                if (ragged_c) {
+                    o[0] &= keep_lo;
+                    o[1] &= keep_hi;
+                }
+                __builtin_amdgcn_raw_buffer_store_b64(o, yr, (int)(orow_off + ocol_off[px]), 0, 0);
+            } else {
+                if (ragged_c) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) res[e] = c0 + e < C ? res[e] : 0.f;
+                }
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, res), yr, (int)(orow_off + ocol_off[px]), 0, 0);
             }
-            __builtin_amdgcn_raw_buffer_store_b64(o, yr, (int)(orow_off + ocol_off[px]), 0, 0);
         }
         orow_off += orow_b;
     };
@@ -1129,6 +1141,77 @@ __global__ __launch_bounds__(kBlock) void global_avgpool_nhwc_f16_kernel(const u
     }
 }
 
+// Pooling on NHWC float storage, four channels per thread; the tensors may be slices of wider ones (xs, ys: their channel
+// strides). Window clipping, divisor and summation order are those of the NCHW kernel. Window taps hit in the caches: the
+// kernel is bound by its loads' latency on the small maps it runs on, so a row of the window is requested at once.
+template <int TYPE>
+__global__ __launch_bounds__(kBlock) void pool2d_nhwc_f32_kernel(const float* __restrict__ x, float* __restrict__ y, int xs, int ys, int H, int W,
+                                                                 int OH, int OW, int kh, int kw, int sh, int sw, int pt, int pb, int pl, int pr,
+                                                                 int include_pad, unsigned C4, unsigned total) {
+    const unsigned i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= total) return;
+    const unsigned pix = i / C4, c = (i - pix * C4) * 4;
+    const unsigned t = pix / (unsigned)OW;
+    const int pw = (int)(pix - t * (unsigned)OW);
+    const unsigned n = t / (unsigned)OH;
+    const int ph = (int)(t - n * (unsigned)OH);
+    int hs = ph * sh - pt, ws = pw * sw - pl;
+    int he = min(hs + kh, H + (TYPE ? pb : 0)), we = min(ws + kw, W + (TYPE ? pr : 0));
+    int pool = (he - hs) * (we - ws);
+    hs = max(hs, 0);
+    ws = max(ws, 0);
+    he = min(he, H);
+    we = min(we, W);
+    const float* const src = x + (size_t)n * H * W * xs + c;
+    v4f v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = TYPE ? 0.f : -FLT_MAX;
+    for (int a = hs; a < he; ++a) {
+        const float* const row = src + (size_t)a * W * xs;
+#pragma unroll 5
+        for (int b = ws; b < we; ++b) {
+            const v4f u = *reinterpret_cast<const v4f*>(row + (size_t)b * xs);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = TYPE ? v[e] + u[e] : (v[e] < u[e] ? u[e] : v[e]);
+        }
+    }
+    if (TYPE) {
+        if (!include_pad) pool = (he - hs) * (we - ws);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] /= (float)pool;
+    }
+    *reinterpret_cast<v4f*>(y + (size_t)pix * ys + c) = v;
+}
+
+// Global average pooling on NHWC float storage: a group per image and 16 channels. The sums are those of the NCHW kernel below:
+// pixels l, l + 64, ... for l = 0 .. 63, then a tree over the 64 partial sums.
+__global__ __launch_bounds__(kBlock) void global_avgpool_nhwc_f32_kernel(const float* __restrict__ x, float* __restrict__ y, int C, int xs, int ys, int HW) {
+    __shared__ v4f part[64][4];
+    const int q = threadIdx.x & 3, l = threadIdx.x >> 2, c = blockIdx.x * 16 + q * 4;
+    v4f s = {0.f, 0.f, 0.f, 0.f};
+    if (c < C)
+        for (int p = l; p < HW; p += 64) {
+            const v4f u = *reinterpret_cast<const v4f*>(x + ((size_t)blockIdx.y * HW + p) * xs + c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] += u[e];
+        }
+    part[l][q] = s;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+        __syncthreads();
+        if (l < d) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) part[l][q][e] += part[l + d][q][e];
+        }
+    }
+    if (l == 0 && c < C) {
+        v4f o = part[0][q];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] /= (float)HW;
+        *reinterpret_cast<v4f*>(y + (size_t)blockIdx.y * ys + c) = o;
+    }
+}
+
 // NCHW float: one wave per plane; lane l adds elements l, l + 64, ..., then the 64 partial sums are folded
 // 32 + 32, 16 + 16, ... in a fixed tree.
 __global__ __launch_bounds__(kBlock) void global_avgpool_nchw_f32_kernel(const float* __restrict__ x, float* __restrict__ y, int HW,
@@ -1579,6 +1662,19 @@ __global__ __launch_bounds__(kBlock) void interp_nearest_nhwc_f16_kernel(const u
     reinterpret_cast<v4i*>(y)[i] = reinterpret_cast<const v4i*>(x)[((n * H + iy) * W + ix) * C8 + v];
 }
 
+// The same on NHWC float storage, slices of wider tensors included, four channels per thread.
+__global__ __launch_bounds__(kBlock) void interp_nearest_nhwc_f32_kernel(const float* __restrict__ x, float* __restrict__ y, int xs, int ys, int H, int W,
+                                                                         int OH, int OW, float hs, float ws, unsigned C4, unsigned total) {
+    const unsigned i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= total) return;
+    const unsigned pix = i / C4, c = (i - pix * C4) * 4, t = pix / (unsigned)OW, n = t / (unsigned)OH;
+    const int ox = (int)(pix - t * (unsigned)OW), oy = (int)(t - n * (unsigned)OH);
+    int iy = (int)(oy * hs), ix = (int)(ox * ws);
+    iy = iy > H - 1 ? H - 1 : iy;
+    ix = ix > W - 1 ? W - 1 : ix;
+    *reinterpret_cast<v4f*>(y + (size_t)pix * ys + c) = *reinterpret_cast<const v4f*>(x + (((size_t)n * H + iy) * W + ix) * xs + c);
+}
+
 // One direction of a stride-1 "same" max pooling on NHWC half storage (window K, padding K / 2, taps outside the image
 // do not count): the K x K maximum is the maximum over rows of the maxima over columns, so two launches of 2K taps
 // replace K * K. ALONG_W: the window runs along x, else along y.
@@ -1669,6 +1765,39 @@ __global__ __launch_bounds__(kBlock) void input_focus_quantize_kernel(const floa
     v4i* dst = reinterpret_cast<v4i*>(y + i * 32);
     dst[0] = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
     dst[1] = v4i{0, 0, 0, 0};
+}
+
+// The layers in front of a float network's first convolution -- Input, (x - mean) * scale per channel, and YoloV5Focus -- and
+// the NHWC layout its kernel reads, one pixel of the result per thread. FOCUS: channel g * C + c of pixel (y, x) is channel c of
+// pixel (2 y + g % 2, 2 x + g / 2).
+template <int CS, bool FOCUS>
+__global__ __launch_bounds__(kBlock) void input_nhwc_f32_kernel(const float* __restrict__ x, float* __restrict__ y, int C, int H, int W, FrontArgs a,
+                                                                unsigned total) {
+    const unsigned i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= total) return;
+    const int OW = FOCUS ? W / 2 : W, OH = FOCUS ? H / 2 : H;
+    const unsigned t = i / (unsigned)OW, n = t / (unsigned)OH;
+    const int ox = (int)(i - t * (unsigned)OW), oy = (int)(t - n * (unsigned)OH);
+    float v[CS];
+#pragma unroll
+    for (int k = 0; k < CS; ++k) v[k] = 0.f;
+    const float* const src = x + (size_t)n * C * H * W;
+    if constexpr (FOCUS) {  // three channels
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                const float* const row = src + ((size_t)c * H + 2 * oy + r) * W + 2 * ox;
+                v[r * 3 + c] = (row[0] - a.mean[c]) * a.scale[c];
+                v[(r + 2) * 3 + c] = (row[1] - a.mean[c]) * a.scale[c];
+            }
+    } else {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            if (c < C) v[c] = (src[((size_t)c * H + oy) * W + ox] - a.mean[c]) * a.scale[c];
+    }
+#pragma unroll
+    for (int k = 0; k < CS; k += 4) *reinterpret_cast<v4f*>(y + (size_t)i * CS + k) = v4f{v[k], v[k + 1], v[k + 2], v[k + 3]};
 }
 
 // A detection head's Reshape + Transpose on the convolution's float32 NHWC result: y[n][g][pixel][j] = x[n][pixel][g * J + j]
@@ -2216,15 +2345,17 @@ extern "C" int exhip_dwconv3x3_nchw_f32_prelu(exhip_ctx* ctx, const float* x, co
     return dw_nchw_f32(ctx, x, w9, bias, y, n, c, h, w, stride, pt, pb, pl, pr, 0, slope, slope_shared);
 }
 
-static int dw_nhwc_f16(exhip_ctx* ctx, const uint16_t* x, const float* w9, const float* bias, uint16_t* y, int n, int c, int h,
+template <typename T>
+static int dw_nhwc(exhip_ctx* ctx, const T* x, const float* w9, const float* bias, T* y, int n, int c, int h,
                        int w, int cs, int stride, int pt, int pb, int pl, int pr, int act, const float* slope,
                        int slope_shared) {
-    REQ_CTX("exhip_dwconv3x3_nhwc_f16");
-    EXHIP_REQUIRE(x && w9 && y && n > 0 && c > 0 && cs >= c && cs % 8 == 0, "exhip_dwconv3x3_nhwc_f16: bad argument (c_stride %% 8)");
+    constexpr bool HALF = sizeof(T) == 2;
+    REQ_CTX("exhip_dwconv3x3_nhwc");
+    EXHIP_REQUIRE(x && w9 && y && n > 0 && c > 0 && cs >= c && cs % 8 == 0, "exhip_dwconv3x3_nhwc: bad argument (c_stride %% 8)");
     int oh, ow;
     int rc = dw_out(h, w, stride, pt, pb, pl, pr, &oh, &ow);
     if (rc) return rc;
-    const size_t x_bytes = (size_t)n * h * w * cs * 2, y_bytes = (size_t)n * oh * ow * cs * 2;
+    const size_t x_bytes = (size_t)n * h * w * cs * sizeof(T), y_bytes = (size_t)n * oh * ow * cs * sizeof(T);
     const size_t desc_limit = (size_t)1 << 30;
     if ((stride == 1 || stride == 2) && (act == 0 || act == 1 || act == 3) && x_bytes <= desc_limit && y_bytes <= desc_limit) {
         // bands of output rows: about fourteen rows each (the per-thread set-up and the two halo rows are worth several
@@ -2232,7 +2363,8 @@ static int dw_nhwc_f16(exhip_ctx* ctx, const uint16_t* x, const float* w9, const
         // seven rows (measured at 64x128x56x56: 7 rows beat 4, 10, 14 and 28 at both strides)
         // stride 2: strips of two pixels (five input columns a row); three pixels (seven columns) sit at the register
         // limit of four waves per SIMD, spill with the PReLU epilogue, and measured slower without it
-        const int px = stride == 1 ? 4 : 2;
+        // float storage: two pixels at either stride, its rows take twice the registers
+        const int px = stride == 1 && HALF ? 4 : 2;
         const int strips = (ow + px - 1) / px;
         const size_t per_band = (size_t)n * strips * (cs / 4);
         const int env_rows = g_exhip_options.dw_band_rows;
@@ -2248,14 +2380,14 @@ static int dw_nhwc_f16(exhip_ctx* ctx, const uint16_t* x, const float* w9, const
         bands = (oh + band_rows - 1) / band_rows;
         const size_t total = per_band * bands;
 #define EXHIP_DW_STRIP(S, P, A)                                                                                          \
-    hipLaunchKernelGGL((dwconv3x3_nhwc_f16_strip_kernel<S, P, A>), dim3(blocks_for(total)), dim3(kBlock), 0, ctx->stream, \
+    hipLaunchKernelGGL((dwconv3x3_nhwc_strip_kernel<T, S, P, A>), dim3(blocks_for(total)), dim3(kBlock), 0, ctx->stream, \
                        x, w9, bias, y, c, h, w, cs, oh, ow, pt, pl, band_rows, bands, strips, (unsigned)x_bytes,        \
                        (unsigned)y_bytes, total, slope, slope_shared)
         if (stride == 1) {
-            if (slope) EXHIP_DW_STRIP(1, 4, kDwPrelu);
-            else if (act == 0) EXHIP_DW_STRIP(1, 4, 0);
-            else if (act == 1) EXHIP_DW_STRIP(1, 4, 1);
-            else EXHIP_DW_STRIP(1, 4, 3);
+            if (slope) EXHIP_DW_STRIP(1, (HALF ? 4 : 2), kDwPrelu);
+            else if (act == 0) EXHIP_DW_STRIP(1, (HALF ? 4 : 2), 0);
+            else if (act == 1) EXHIP_DW_STRIP(1, (HALF ? 4 : 2), 1);
+            else EXHIP_DW_STRIP(1, (HALF ? 4 : 2), 3);
         } else {
             if (slope) EXHIP_DW_STRIP(2, 2, kDwPrelu);
             else if (act == 0) EXHIP_DW_STRIP(2, 2, 0);
@@ -2267,27 +2399,38 @@ static int dw_nhwc_f16(exhip_ctx* ctx, const uint16_t* x, const float* w9, const
         return 0;
     }
     if (slope) {
-        exhip_set_error("exhip_dwconv3x3_nhwc_f16_prelu: this shape runs the general kernel, which has no PReLU epilogue");
+        exhip_set_error("exhip_dwconv3x3_nhwc_prelu: this shape runs the general kernel, which has no PReLU epilogue");
         return EXHIP_ERR_UNSUPPORTED;
     }
-    const size_t total = (size_t)n * oh * ow * (cs / 8);
-    hipLaunchKernelGGL(dwconv3x3_nhwc_f16_kernel, dim3(blocks_for(total)), dim3(kBlock), 0, ctx->stream, x, w9, bias, y, c, h, w,
-                       cs, oh, ow, stride, pt, pl, act, total);
-    EXHIP_LAUNCH_CHECK();
-    return 0;
+    if constexpr (HALF) {
+        const size_t total = (size_t)n * oh * ow * (cs / 8);
+        hipLaunchKernelGGL(dwconv3x3_nhwc_f16_kernel, dim3(blocks_for(total)), dim3(kBlock), 0, ctx->stream, x, w9, bias, y, c, h, w,
+                           cs, oh, ow, stride, pt, pl, act, total);
+        EXHIP_LAUNCH_CHECK();
+        return 0;
+    } else {
+        exhip_set_error("exhip_dwconv3x3_nhwc_f32: activation %d or tensors beyond 1 GiB are not taken", act);
+        return EXHIP_ERR_UNSUPPORTED;
+    }
 }
 
 extern "C" int exhip_dwconv3x3_nhwc_f16(exhip_ctx* ctx, const uint16_t* x, const float* w9, const float* bias, uint16_t* y,
                                         int n, int c, int h, int w, int cs, int stride, int pt, int pb, int pl, int pr,
                                         int act) {
-    return dw_nhwc_f16(ctx, x, w9, bias, y, n, c, h, w, cs, stride, pt, pb, pl, pr, act, nullptr, 0);
+    return dw_nhwc(ctx, x, w9, bias, y, n, c, h, w, cs, stride, pt, pb, pl, pr, act, nullptr, 0);
 }
 
 extern "C" int exhip_dwconv3x3_nhwc_f16_prelu(exhip_ctx* ctx, const uint16_t* x, const float* w9, const float* bias,
                                               const float* slope, int slope_shared, uint16_t* y, int n, int c, int h, int w,
                                               int cs, int stride, int pt, int pb, int pl, int pr) {
     EXHIP_REQUIRE(slope, "exhip_dwconv3x3_nhwc_f16_prelu: NULL slopes");
-    return dw_nhwc_f16(ctx, x, w9, bias, y, n, c, h, w, cs, stride, pt, pb, pl, pr, 0, slope, slope_shared);
+    return dw_nhwc(ctx, x, w9, bias, y, n, c, h, w, cs, stride, pt, pb, pl, pr, 0, slope, slope_shared);
+}
+
+extern "C" int exhip_dwconv3x3_nhwc_f32(exhip_ctx* ctx, const float* x, const float* w9, const float* bias, const float* slope, int slope_shared,
+                                        float* y, int n, int c, int h, int w, int cs, int stride, int pt, int pb, int pl, int pr, int act) {
+    EXHIP_REQUIRE(!slope || act == 0, "exhip_dwconv3x3_nhwc_f32: an activation and PReLU slopes");
+    return dw_nhwc(ctx, x, w9, bias, y, n, c, h, w, cs, stride, pt, pb, pl, pr, act, slope, slope_shared);
 }
 
 extern "C" int exhip_dw_dequant_weights(exhip_ctx* ctx, const int8_t* w, const float* ws, float* wf, int k, int per_group) {
@@ -2976,6 +3119,60 @@ extern "C" int exhip_input_focus_quantize_nchw_f32_to_nhwc_i8(exhip_ctx* ctx, co
     for (int i = 0; i < c; ++i) { a.mean[i] = means[i]; a.scale[i] = scales[i]; }
     const size_t total = (size_t)n * (h / 2) * (w / 2);
     hipLaunchKernelGGL(input_focus_quantize_kernel<3>, dim3(blocks_for(total)), dim3(kBlock), 0, ctx->stream, x, y, h, w, a, fs, total);
+    EXHIP_LAUNCH_CHECK();
+    return 0;
+}
+
+extern "C" int exhip_input_nchw_f32_to_nhwc_f32(exhip_ctx* ctx, const float* x, int n, int c, int h, int w, const float* means, const float* scales,
+                                                int focus, int c_stride, float* y) {
+    REQ_CTX("exhip_input_nchw_f32_to_nhwc_f32");
+    EXHIP_REQUIRE(x && y && means && scales && n > 0 && c > 0 && h > 0 && w > 0, "exhip_input_nchw_f32_to_nhwc_f32: bad argument");
+    const long long total = focus ? (long long)n * (h / 2) * (w / 2) : (long long)n * h * w;
+    if ((reinterpret_cast<uintptr_t>(y) & 15) != 0 || total >= (1ll << 31) || total == 0) return EXHIP_ERR_UNSUPPORTED;
+    if (focus ? c != 3 || c_stride != 16 || (h & 1) || (w & 1) : c > 4 || c_stride != 4) return EXHIP_ERR_UNSUPPORTED;
+    FrontArgs a = {};
+    for (int i = 0; i < c; ++i) { a.mean[i] = means[i]; a.scale[i] = scales[i]; }
+    if (focus)
+        hipLaunchKernelGGL((input_nhwc_f32_kernel<16, true>), dim3(blocks_for((size_t)total)), dim3(kBlock), 0, ctx->stream, x, y, c, h, w, a, (unsigned)total);
+    else
+        hipLaunchKernelGGL((input_nhwc_f32_kernel<4, false>), dim3(blocks_for((size_t)total)), dim3(kBlock), 0, ctx->stream, x, y, c, h, w, a, (unsigned)total);
+    EXHIP_LAUNCH_CHECK();
+    return 0;
+}
+
+extern "C" int exhip_pool2d_nhwc_f32(exhip_ctx* ctx, const float* x, int x_stride, float* y, int y_stride, int n, int c, int h, int w, int oh, int ow,
+                                     int type, int kh, int kw, int sh, int sw, int pt, int pb, int pl, int pr, int count_include_pad) {
+    REQ_CTX("exhip_pool2d_nhwc_f32");
+    EXHIP_REQUIRE(x && y && n > 0 && c > 0 && h > 0 && w > 0 && oh > 0 && ow > 0 && kh > 0 && kw > 0 && (type == 0 || type == 1),
+                  "exhip_pool2d_nhwc_f32: bad argument");
+    const long long total = (long long)n * oh * ow * ((c + 3) / 4);
+    if (x_stride % 4 != 0 || y_stride % 4 != 0 || (c + 3) / 4 * 4 > std::min(x_stride, y_stride) || ((uintptr_t)x & 15) || ((uintptr_t)y & 15) ||
+        total >= (1ll << 31))
+        return EXHIP_ERR_UNSUPPORTED;
+    if (type == 1 && oh == 1 && ow == 1 && kh == h && kw == w && !pt && !pb && !pl && !pr && n <= 65535) {
+        hipLaunchKernelGGL(global_avgpool_nhwc_f32_kernel, dim3((unsigned)((c + 15) / 16), (unsigned)n), dim3(kBlock), 0, ctx->stream, x, y, (c + 3) / 4 * 4,
+                           x_stride, y_stride, h * w);
+    } else if (type == 0) {
+        hipLaunchKernelGGL(pool2d_nhwc_f32_kernel<0>, dim3(blocks_for((size_t)total)), dim3(kBlock), 0, ctx->stream, x, y, x_stride, y_stride, h, w, oh, ow, kh,
+                           kw, sh, sw, pt, pb, pl, pr, count_include_pad, (unsigned)((c + 3) / 4), (unsigned)total);
+    } else {
+        hipLaunchKernelGGL(pool2d_nhwc_f32_kernel<1>, dim3(blocks_for((size_t)total)), dim3(kBlock), 0, ctx->stream, x, y, x_stride, y_stride, h, w, oh, ow, kh,
+                           kw, sh, sw, pt, pb, pl, pr, count_include_pad, (unsigned)((c + 3) / 4), (unsigned)total);
+    }
+    EXHIP_LAUNCH_CHECK();
+    return 0;
+}
+
+extern "C" int exhip_interp_nearest_nhwc_f32(exhip_ctx* ctx, const float* x, int x_stride, float* y, int y_stride, int n, int c, int h, int w, int oh,
+                                             int ow) {
+    REQ_CTX("exhip_interp_nearest_nhwc_f32");
+    EXHIP_REQUIRE(x && y && n > 0 && c > 0 && h > 0 && w > 0 && oh > 0 && ow > 0, "exhip_interp_nearest_nhwc_f32: bad argument");
+    const long long total = (long long)n * oh * ow * ((c + 3) / 4);
+    if (x_stride % 4 != 0 || y_stride % 4 != 0 || (c + 3) / 4 * 4 > std::min(x_stride, y_stride) || ((uintptr_t)x & 15) || ((uintptr_t)y & 15) ||
+        total >= (1ll << 31))
+        return EXHIP_ERR_UNSUPPORTED;
+    hipLaunchKernelGGL(interp_nearest_nhwc_f32_kernel, dim3(blocks_for((size_t)total)), dim3(kBlock), 0, ctx->stream, x, y, x_stride, y_stride, h, w, oh, ow,
+                       (float)h / oh, (float)w / ow, (unsigned)((c + 3) / 4), (unsigned)total);
     EXHIP_LAUNCH_CHECK();
     return 0;
 }

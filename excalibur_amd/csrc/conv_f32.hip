@@ -51,9 +51,11 @@ struct F32Params {
     int csteps, n_ksteps;          // steps per tap (kPair: 1) and in all
     int start_r[kMaxSplit + 1], start_q[kMaxSplit + 1], start_c[kMaxSplit + 1], start_s[kMaxSplit + 1];  // where each wave of a tile begins
     int K, kstride, k_end;         // channels from k_end on are not written
-    int act, post_relu, post_op, slope_shared, residual_last;
+    int act, post_relu, bn_relu, post_op, slope_shared, residual_last;
     float alpha, beta;
     int vector_rows;               // output (and shortcut) rows take 16-byte accesses
+    int rstride, res_shift;        // the shortcut's channel stride; log2 of how many output pixels per axis share one of its pixels
+    int layout, group;             // EXHIP_PLACE_*; grouped: channels per group, shuffled: channels of an upsampled pixel
 };
 
 __device__ __forceinline__ v4f load4(__amdgpu_buffer_rsrc_t r, unsigned voff, int soff) {
@@ -100,20 +102,31 @@ __device__ __forceinline__ void epilogue_block(const F32Params& p, const v16f& a
     const int rows = p.pixels - first < 32 ? (int)(p.pixels - first) : 32;
     char* const tile = lds + kParams * MT * 32 * 4;
     float v[16], t[16], res[16];
+    // where the lane's pixel lies: its image and the pixel inside it, for the forms that place pixels or read them elsewhere
+    const unsigned per_image = (unsigned)(p.out_h * p.out_w), pix = first + row;
+    unsigned img = 0, in_image = 0;
+    if (p.res_shift || p.y_nchw || p.layout != EXHIP_PLACE_ROWS) {
+        img = exhip_divide(pix, per_image, p.image_magic, p.image_shift);
+        in_image = pix - img * per_image;
+    }
     if (p.residual) {
-        const __amdgpu_buffer_rsrc_t rr = rows_view(p.residual, first, p.kstride, kb * 32, rows);
+        unsigned from = pix;
+        if (p.res_shift) {
+            const unsigned oy = exhip_divide(in_image, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = in_image - oy * (unsigned)p.out_w;
+            from = (img * ((unsigned)p.out_h >> p.res_shift) + (oy >> p.res_shift)) * ((unsigned)p.out_w >> p.res_shift) + (ox >> p.res_shift);
+        }
+        const float* const src = p.residual + (size_t)from * (unsigned)p.rstride + ch0;
         if (p.vector_rows) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const v4f r = load4(rr, ch0 + q * 4 < p.kstride ? (unsigned)(row * p.kstride + half * 16 + q * 4) * 4 : kOutOfRange, 0);
+                v4f r = {0.f, 0.f, 0.f, 0.f};
+                if (row < rows && ch0 + q * 4 < p.K) r = reinterpret_cast<const v4f*>(src)[q];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) res[q * 4 + e] = r[e];
             }
         } else {
 #pragma unroll
-            for (int e = 0; e < 16; ++e)
-                res[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                                       rr, ch0 + e < p.K ? (row * p.kstride + half * 16 + e) * 4 : (int)kOutOfRange, 0, 0));
+            for (int e = 0; e < 16; ++e) res[e] = row < rows && ch0 + e < p.K ? src[e] : 0.f;
         }
     }
     read16<MT>(lds, 0, m, half, t);
@@ -143,6 +156,7 @@ __device__ __forceinline__ void epilogue_block(const F32Params& p, const v16f& a
         read16<MT>(lds, 3, m, half, b);
 #pragma unroll
         for (int e = 0; e < 16; ++e) v[e] = __builtin_fmaf(b[e], v[e], t[e]);
+        if (p.bn_relu) relu16(v);
     }
     switch (p.post_op) {
     case 0: break;
@@ -165,32 +179,67 @@ __device__ __forceinline__ void epilogue_block(const F32Params& p, const v16f& a
             for (int e = 0; e < 16; ++e)
                 if (ch0 + e >= p.K) v[e] = 0.f;
         }
-        const __amdgpu_buffer_rsrc_t yr = rows_view(p.y, first, p.kstride, kb * 32, rows);
-        if (p.vector_rows) {  // through LDS: eight neighbouring lanes write one pixel's 128 bytes
+        if (p.vector_rows || p.layout == EXHIP_PLACE_GROUPED) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const v4f o = {v[q * 4], v[q * 4 + 1], v[q * 4 + 2], v[q * 4 + 3]};
                 *reinterpret_cast<v4f*>(tile + row * kTilePitch + half * 64 + q * 16) = o;
             }
-            const int scol = (lane & 7) * 16;
+        }
+        if (p.layout == EXHIP_PLACE_GROUPED) {
+            // y[img][group][pixel][member]: a half-wave writes the block's 32 channels of one pixel, runs of neighbouring floats
+            const int ch = kb * 32 + row, g = ch / p.group, member = ch - g * p.group;
+            const unsigned lane_at = img * (unsigned)p.K * per_image + in_image * (unsigned)p.group;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int srow = j * 8 + (lane >> 3);
-                const v4u o = *reinterpret_cast<const v4u*>(tile + srow * kTilePitch + scol);
-                const bool in = srow < rows && scol < (p.k_end - kb * 32) * 4;
-                __builtin_amdgcn_raw_buffer_store_b128(o, yr, in ? srow * p.kstride * 4 + scol : (int)kOutOfRange, 0, 0);
+            for (int j = 0; j < 16; ++j) {
+                const int srow = j * 2 + half;
+                const unsigned at = (unsigned)__builtin_amdgcn_ds_bpermute(srow * 4, (int)lane_at) + (unsigned)g * per_image * (unsigned)p.group + member;
+                if (srow < rows && ch < p.K) p.y[at] = *reinterpret_cast<const float*>(tile + srow * kTilePitch + row * 4);
+            }
+        } else if (p.layout == EXHIP_PLACE_SHUFFLED) {
+            // channel pos * group + k of pixel (y, x) is channel k of pixel (2 y + pos / 2, 2 x + pos % 2) of a map twice as large
+            const unsigned oy = exhip_divide(in_image, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = in_image - oy * (unsigned)p.out_w;
+            const unsigned corner = (img * 2 * (unsigned)p.out_h + 2 * oy) * 2 * (unsigned)p.out_w + 2 * ox;
+            if (p.vector_rows) {  // whole blocks belong to one of the four
+                const int pos = kb * 32 / p.group, k0 = kb * 32 - pos * p.group;
+                const unsigned step = (unsigned)(pos >> 1) * 2 * (unsigned)p.out_w + (pos & 1);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int srow = j * 8 + (lane >> 3);
+                    const unsigned to = (unsigned)__builtin_amdgcn_ds_bpermute(srow * 4, (int)corner) + step;
+                    if (srow < rows)
+                        *reinterpret_cast<v4f*>(p.y + (size_t)to * (unsigned)p.kstride + k0 + (lane & 7) * 4) =
+                            *reinterpret_cast<const v4f*>(tile + srow * kTilePitch + (lane & 7) * 16);
+                }
+            } else if (row < rows) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const int pos = (ch0 + e) / p.group, k = ch0 + e - pos * p.group;
+                    if (ch0 + e < p.K)
+                        p.y[(size_t)(corner + (unsigned)(pos >> 1) * 2 * (unsigned)p.out_w + (pos & 1)) * (unsigned)p.kstride + k] = v[e];
+                }
             }
         } else {
+            const __amdgpu_buffer_rsrc_t yr = rows_view(p.y, first, p.kstride, kb * 32, rows);
+            if (p.vector_rows) {  // through LDS: eight neighbouring lanes write one pixel's 128 bytes
+                const int scol = (lane & 7) * 16;
 #pragma unroll
-            for (int e = 0; e < 16; ++e)
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v[e]), yr,
-                                                      row < rows && ch0 + e < p.k_end ? (row * p.kstride + half * 16 + e) * 4 : (int)kOutOfRange, 0, 0);
+                for (int j = 0; j < 4; ++j) {
+                    const int srow = j * 8 + (lane >> 3);
+                    const v4u o = *reinterpret_cast<const v4u*>(tile + srow * kTilePitch + scol);
+                    const bool in = srow < rows && scol < (p.k_end - kb * 32) * 4;
+                    __builtin_amdgcn_raw_buffer_store_b128(o, yr, in ? srow * p.kstride * 4 + scol : (int)kOutOfRange, 0, 0);
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v[e]), yr,
+                                                          row < rows && ch0 + e < p.k_end ? (row * p.kstride + half * 16 + e) * 4 : (int)kOutOfRange, 0, 0);
+            }
         }
     }
     if (p.y_nchw && row < rows) {  // 32 neighbouring pixels of a channel per store instruction and half-wave
-        const unsigned per_image = (unsigned)(p.out_h * p.out_w);
-        const unsigned pix = first + row, img = exhip_divide(pix, per_image, p.image_magic, p.image_shift);
-        float* const dst = p.y_nchw + ((size_t)img * p.K + ch0) * per_image + (pix - img * per_image);
+        float* const dst = p.y_nchw + ((size_t)img * p.K + ch0) * per_image + in_image;
 #pragma unroll
         for (int e = 0; e < 16; ++e)
             if (ch0 + e < p.K) dst[(size_t)e * per_image] = v[e];
@@ -499,14 +548,15 @@ int exhip_conv_f32_pack_weights(const exhip_conv_desc* d, const float* w, float*
     return 0;
 }
 
-extern "C" int exhip_conv2d_f32(exhip_ctx* ctx, const exhip_conv_desc* d, const float* x, const void* wp,
-                                const float* bias, const float* residual, float* y_f32_nhwc, float* y_f32_nchw) {
-    EXHIP_REQUIRE(y_f32_nhwc || y_f32_nchw, "exhip_conv2d_f32: no output requested");
+static int run_conv_f32(exhip_ctx* ctx, const exhip_conv_desc* d, const exhip_conv_place* place, const float* x, const void* wp, const float* bias,
+                        const float* residual, float* y, float* y_nchw) {
+    EXHIP_REQUIRE(y || y_nchw, "exhip_conv2d_f32: no output requested");
     EXHIP_REQUIRE(ctx, "conv: NULL ctx");
     const int rc = exhip_conv_f32_validate(d);
     if (rc) return rc;
     EXHIP_REQUIRE(x && wp, "conv: NULL input or weights");
-    EXHIP_REQUIRE(d->k_stride >= d->k || (!y_f32_nhwc && !residual), "conv: k_stride %d < k %d", d->k_stride, d->k);
+    const int layout = place ? place->layout : EXHIP_PLACE_ROWS, group = place ? place->group : 0;
+    EXHIP_REQUIRE(layout != EXHIP_PLACE_ROWS || d->k_stride >= d->k || (!y && !residual), "conv: k_stride %d < k %d", d->k_stride, d->k);
     EXHIP_REQUIRE(!bias || (uintptr_t)bias % 16 == 0, "conv: scale and bias arrays must be 16-byte aligned");
     EXHIP_REQUIRE((uintptr_t)x % 16 == 0 && (uintptr_t)wp % 16 == 0, "conv: input and weights must be 16-byte aligned");
     EXHIP_REQUIRE((d->post_op >= 0 && d->post_op <= 1 + EXHIP_UNARY_CLIP && d->post_op != 1 + EXHIP_UNARY_SIGMOID) ||
@@ -515,6 +565,20 @@ extern "C" int exhip_conv2d_f32(exhip_ctx* ctx, const exhip_conv_desc* d, const 
     EXHIP_REQUIRE((d->post_bn_a == nullptr) == (d->post_bn_b == nullptr), "conv: half a BatchNorm");
     F32Params p = {};
     const int oh = (d->h + d->pt + d->pb - d->kh) / d->sh + 1, ow = (d->w + d->pl + d->pr - d->kw) / d->sw + 1;
+    p.layout = layout;
+    p.group = group;
+    p.rstride = d->k_stride;
+    if (place) {
+        EXHIP_REQUIRE(layout >= EXHIP_PLACE_ROWS && layout <= EXHIP_PLACE_SHUFFLED && place->residual_shift >= 0 && place->residual_shift <= 4,
+                      "conv: unknown placement");
+        EXHIP_REQUIRE(layout == EXHIP_PLACE_ROWS || (group > 0 && d->k % group == 0 && y && !y_nchw), "conv: %d channels do not make groups of %d", d->k, group);
+        EXHIP_REQUIRE(layout != EXHIP_PLACE_SHUFFLED || (d->k == 4 * group && d->k_stride >= group), "conv: a shuffled layer has four groups");
+        EXHIP_REQUIRE(!residual || (place->residual_stride >= d->k && oh % (1 << place->residual_shift) == 0 && ow % (1 << place->residual_shift) == 0),
+                      "conv: the shortcut does not fit the output");
+        p.rstride = place->residual_stride;
+        p.res_shift = residual ? place->residual_shift : 0;
+        p.bn_relu = place->bn_relu;
+    }
     p.wp = static_cast<const char*>(wp);
     p.bias = bias; p.bn_a = d->post_bn_a; p.bn_b = d->post_bn_b;
     p.slope = d->post_op == EXHIP_POST_PRELU ? d->post_slope : nullptr;
@@ -525,35 +589,50 @@ extern "C" int exhip_conv2d_f32(exhip_ctx* ctx, const exhip_conv_desc* d, const 
     const bool pair = d->c_stride == 4;
     p.csteps = pair ? 1 : (d->c + 7) / 8;
     p.n_ksteps = taps_steps(d);
-    const int kblocks = (d->k + 31) / 32;
-    p.w_bytes = (unsigned)((size_t)kblocks * p.n_ksteps * 1024);
+    p.w_bytes = (unsigned)((size_t)((d->k + 31) / 32) * p.n_ksteps * 1024);
     p.K = d->k;
     p.kstride = d->k_stride;
-    p.k_end = d->exact_k || !y_f32_nhwc ? d->k : std::max(d->k, d->k_stride);
+    p.k_end = d->exact_k || !y || layout != EXHIP_PLACE_ROWS ? d->k : std::max(d->k, d->k_stride);
     p.act = d->act; p.post_relu = d->post_relu; p.post_op = d->post_op; p.slope_shared = d->post_slope_shared;
     p.residual_last = d->residual_last;
     p.alpha = d->post_alpha; p.beta = d->post_beta;
-    p.vector_rows = d->k_stride % 4 == 0 && (uintptr_t)y_f32_nhwc % 16 == 0 && (uintptr_t)residual % 16 == 0 && p.k_end % 4 == 0;
+    p.vector_rows = d->k_stride % 4 == 0 && (uintptr_t)y % 16 == 0 && p.k_end % 4 == 0 &&
+                    (!residual || ((uintptr_t)residual % 16 == 0 && p.rstride % 4 == 0 && (d->k + 3) / 4 * 4 <= p.rstride));
+    if (layout == EXHIP_PLACE_SHUFFLED && group % 32 != 0) p.vector_rows = 0;
     exhip_host_divisor((unsigned)(oh * ow), &p.image_magic, &p.image_shift);
     exhip_host_divisor((unsigned)ow, &p.width_magic, &p.width_shift);
     // blocks past the last channel's (pad channels of a wider stride) get zeros too: weights beyond the view read zero
     const int write_blocks = (p.k_end + 31) / 32;
     const long long img_bytes = (long long)d->h * p.row_b, per_image = (long long)oh * ow;
-    EXHIP_REQUIRE(per_image < (1ll << 31) - 256, "conv: more than 2^31 output pixels in an image");
-    // input offsets are 32-bit: as many images per launch as fit below 4 GiB and 2^31 pixels
-    const long long most = std::max(1ll, std::min((0x7fff0000ll) / img_bytes, ((1ll << 31) - 256) / per_image));
+    EXHIP_REQUIRE(per_image < (1ll << 29) && (layout != EXHIP_PLACE_GROUPED || per_image * d->k < (1ll << 31)), "conv: too many output pixels in an image");
+    // input offsets are 32-bit, pixel numbers 31-bit, offsets of grouped results 32-bit: as many images per launch as fit
+    long long most = std::min(0x7fff0000ll / img_bytes, ((1ll << (layout == EXHIP_PLACE_SHUFFLED ? 29 : 31)) - 256) / per_image);
+    if (layout == EXHIP_PLACE_GROUPED) most = std::min(most, (1ll << 32) / (per_image * d->k) - 1);
+    most = std::max(1ll, most);
+    const long long y_image = layout == EXHIP_PLACE_SHUFFLED ? per_image * 4 * d->k_stride : layout == EXHIP_PLACE_GROUPED ? per_image * d->k : per_image * d->k_stride;
     for (long long n0 = 0; n0 < d->n; n0 += most) {
         const long long n = std::min<long long>(most, d->n - n0);
         p.x = reinterpret_cast<const char*>(x) + n0 * img_bytes;
         p.x_bytes = (unsigned)(n * img_bytes);
         p.pixels = (unsigned)(n * per_image);
-        p.residual = residual ? residual + n0 * per_image * d->k_stride : nullptr;
-        p.y = y_f32_nhwc ? y_f32_nhwc + n0 * per_image * d->k_stride : nullptr;
-        p.y_nchw = y_f32_nchw ? y_f32_nchw + n0 * per_image * d->k : nullptr;
+        p.residual = residual ? residual + n0 * (per_image >> (2 * p.res_shift)) * p.rstride : nullptr;
+        p.y = y ? y + n0 * y_image : nullptr;
+        p.y_nchw = y_nchw ? y_nchw + n0 * per_image * d->k : nullptr;
         const int go_rc = pair ? pick<kPair>(ctx, p, write_blocks)
                           : d->kh == 1 && d->kw == 1 && !d->pt && !d->pb && !d->pl && !d->pr ? pick<kPoint>(ctx, p, write_blocks)
                                                                                              : pick<kTaps>(ctx, p, write_blocks);
         if (go_rc) return go_rc;
     }
     return 0;
+}
+
+extern "C" int exhip_conv2d_f32(exhip_ctx* ctx, const exhip_conv_desc* d, const float* x, const void* wp,
+                                const float* bias, const float* residual, float* y_f32_nhwc, float* y_f32_nchw) {
+    return run_conv_f32(ctx, d, nullptr, x, wp, bias, residual, y_f32_nhwc, y_f32_nchw);
+}
+
+extern "C" int exhip_conv2d_f32_placed(exhip_ctx* ctx, const exhip_conv_desc* d, const exhip_conv_place* place, const float* x, const void* wp,
+                                       const float* bias, const float* residual, float* y, float* y_f32_nchw) {
+    EXHIP_REQUIRE(place, "exhip_conv2d_f32_placed: NULL placement");
+    return run_conv_f32(ctx, d, place, x, wp, bias, residual, y, y_f32_nchw);
 }

@@ -465,11 +465,23 @@ public:
     template <typename T>
     using tensor_list = typename operation<Dtype>::template tensor_list<T>;
     explicit operation_deconvolution(const operation_param& param) : operation_general_conv<Dtype>(param) {}
+    ~operation_deconvolution() override;
     int init_weights() override;
     int init_weights(FILE* fp) override;
+    // A 2x2 stride-2 layer without padding gives every output pixel one input pixel and one tap: four 1x1 convolutions whose
+    // results interleave (EXHIP_PLACE_SHUFFLED). Their packed weights and their bias, made once.
+    bool four_pointwise() const;
+    int deconv_input_channels() const { return this->weight_data_size_ / (this->output_channel_ * this->kernel_size_h_ * this->kernel_size_w_); }
+    const void* pointwise_weights(const exhip_conv_desc& d);
+    const float* pointwise_bias();
 
 protected:
     void forward_gpu_f32(const tensor_list<float>& bottoms, tensor_list<float>& tops) override;
+
+private:
+    void* pointwise_ = nullptr;
+    size_t pointwise_bytes_ = 0;
+    std::shared_ptr<memory::tensor<float>> pointwise_bias_;
 };
 
 }  // namespace excalibur

@@ -113,7 +113,7 @@ unsigned short half_bits_rne(float f) {
 // input channel stride (elements) the MFMA convolution wants for a dtype / kernel width
 int conv_in_stride(int c, int dtype, int kw) {
     const int es = dtype == EXHIP_I8 ? 1 : dtype == EXHIP_F16 ? 2 : 4;
-    if (c <= 4 && ((dtype == EXHIP_I8 && kw <= 8) || (dtype == EXHIP_F16 && kw <= 4))) return 4;
+    if (c <= 4 && ((dtype == EXHIP_I8 && kw <= 8) || (dtype == EXHIP_F16 && kw <= 4) || dtype == EXHIP_F32)) return 4;
     return pad_to(c * es, 32) / es;
 }
 
@@ -1713,6 +1713,50 @@ int operation_deconvolution<Dtype>::init_weights() {
 }
 
 template <typename Dtype>
+operation_deconvolution<Dtype>::~operation_deconvolution() {
+    if (pointwise_) memory::device_release(this->params_.device_, pointwise_, pointwise_bytes_);
+}
+
+template <typename Dtype>
+bool operation_deconvolution<Dtype>::four_pointwise() const {
+    const int k = this->output_channel_;
+    return this->group_ == 1 && this->dilation_h_ == 1 && this->dilation_w_ == 1 && this->kernel_size_h_ == 2 && this->kernel_size_w_ == 2 &&
+           this->stride_h_ == 2 && this->stride_w_ == 2 && !this->pad_top_ && !this->pad_bottom_ && !this->pad_left_ && !this->pad_right_ &&
+           (k == 1 || k % 8 == 0) && !this->weights_f32_.empty();
+}
+
+template <typename Dtype>
+const void* operation_deconvolution<Dtype>::pointwise_weights(const exhip_conv_desc& d) {
+    if (pointwise_) return pointwise_;
+    // blob [C][K][2][2] -> OIHW [4 K][C][1][1], output channel pos * K + k
+    const int c = d.c, k = this->output_channel_;
+    const float* w = this->weights_f32_[0]->cpu_data();
+    std::vector<float> rows(static_cast<size_t>(4) * k * c);
+    for (int pos = 0; pos < 4; ++pos)
+        for (int o = 0; o < k; ++o)
+            for (int i = 0; i < c; ++i) rows[(static_cast<size_t>(pos) * k + o) * c + i] = w[(static_cast<size_t>(i) * k + o) * 4 + pos];
+    pointwise_bytes_ = exhip_conv_packed_bytes(&d, EXHIP_F32);
+    if (pointwise_bytes_ == 0) LOG(FATAL) << "layer " << this->params_.name_ << ": " << exhip_last_error();
+    std::vector<char> packed(pointwise_bytes_);
+    EXHIP_FATAL(exhip_conv_pack_weights(&d, EXHIP_F32, rows.data(), packed.data()));
+    pointwise_ = memory::device_alloc(this->params_.device_, pointwise_bytes_);
+    EXHIP_FATAL(exhip_memcpy_h2d(this->ctx(), pointwise_, packed.data(), pointwise_bytes_));
+    return pointwise_;
+}
+
+template <typename Dtype>
+const float* operation_deconvolution<Dtype>::pointwise_bias() {
+    if (!this->bias_term_) return nullptr;
+    if (!pointwise_bias_) {
+        const int k = this->output_channel_;
+        pointwise_bias_ = vec_tensor<float>(4 * k, this->params_.device_);
+        float* b = pointwise_bias_->mutable_cpu_data();
+        for (int pos = 0; pos < 4; ++pos) std::memcpy(b + pos * k, this->weights_f32_[1]->cpu_data(), k * sizeof(float));
+    }
+    return pointwise_bias_->gpu_data();
+}
+
+template <typename Dtype>
 void operation_deconvolution<Dtype>::forward_gpu_f32(const tensor_list<float>& bottoms, tensor_list<float>& tops) {
     CHECK_EQ(bottoms.size(), 1);
     CHECK_EQ(tops.size(), 1);
@@ -1724,6 +1768,29 @@ void operation_deconvolution<Dtype>::forward_gpu_f32(const tensor_list<float>& b
     const int oh = (b->height() - 1) * this->stride_h_ + this->kernel_size_h_ - (this->pad_top_ + this->pad_bottom_);
     const int ow = (b->width() - 1) * this->stride_w_ + this->kernel_size_w_ - (this->pad_left_ + this->pad_right_);
     tops[0] = new_tensor<float>({b->num(), this->output_channel_, oh, ow}, this->params_.device_);
+    if (four_pointwise()) {
+        const int n = b->num(), h = b->height(), w = b->width(), k = this->output_channel_, dev = this->params_.device_;
+        exhip_conv_desc d;
+        std::memset(&d, 0, sizeof(d));
+        d.n = n; d.c = c; d.h = h; d.w = w; d.k = 4 * k; d.kh = d.kw = d.sh = d.sw = 1;
+        d.c_stride = pad_to(c, 8); d.k_stride = k;
+        exhip_conv_place how;
+        std::memset(&how, 0, sizeof(how));
+        how.layout = EXHIP_PLACE_SHUFFLED;
+        how.group = k;
+        auto x = new_tensor<float>({n, h, w, d.c_stride}, dev);
+        EXHIP_FATAL(exhip_nchw_f32_to_nhwc_f32(this->ctx(), b->gpu_data(), n, c, h, w, d.c_stride, x->mutable_gpu_data()));
+        if (k == 1) {  // one channel: the layouts are the same
+            EXHIP_FATAL(exhip_conv2d_f32_placed(this->ctx(), &d, &how, x->gpu_data(), pointwise_weights(d), pointwise_bias(), nullptr,
+                                                tops[0]->mutable_gpu_data(), nullptr));
+            return;
+        }
+        auto y = new_tensor<float>({n, oh, ow, k}, dev);
+        EXHIP_FATAL(exhip_conv2d_f32_placed(this->ctx(), &d, &how, x->gpu_data(), pointwise_weights(d), pointwise_bias(), nullptr,
+                                            y->mutable_gpu_data(), nullptr));
+        EXHIP_FATAL(exhip_nhwc_f32_to_nchw_f32(this->ctx(), y->gpu_data(), n, k, oh, ow, k, tops[0]->mutable_gpu_data()));
+        return;
+    }
     EXHIP_FATAL(exhip_deconv2d_f32(this->ctx(), b->gpu_data(), this->weights_f32_[0]->gpu_data(),
                                    this->bias_term_ ? this->weights_f32_[1]->gpu_data() : nullptr, tops[0]->mutable_gpu_data(), b->num(), c,
                                    b->height(), b->width(), this->output_channel_, this->kernel_size_h_, this->kernel_size_w_, this->stride_h_,

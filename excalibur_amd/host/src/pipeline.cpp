@@ -329,7 +329,7 @@ public:
         if (profile_) {
             exhip_sync(memory::device_context(device_));
             last_ms_ = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-            LOG(INFO) << name_ << ": forward " << last_ms_ << " ms (" << (last_fused_ ? "fused int8 plan" : "per-layer") << ")";
+            LOG(INFO) << name_ << ": forward " << last_ms_ << " ms (" << (last_fused_ ? "fused int8 plan" : plan_ && fusion_ ? "float plan" : "per-layer") << ")";
         }
         return results;
     }
@@ -499,6 +499,7 @@ private:
     bool try_fused(const tensor_ptr& input, blob_map* results);
     bool build_block_plan(const tensor_ptr& input, const std::vector<int>& shape);  // residual networks: Convolution / max Pooling / Split / add / ReLU
     bool build_graph_plan(const tensor_ptr& input, const std::vector<int>& shape);  // + activation layers, Concat, BatchNorm, Interp, Focus
+    bool build_float_plan(const tensor_ptr& input, const std::vector<int>& shape);  // float32 networks of those layers
     struct fused_plan;
     std::shared_ptr<fused_plan> plan_;
     bool fused_unsupported_ = false;
@@ -540,6 +541,7 @@ private:
 template <typename Dtype>
 struct pipeline<Dtype>::impl::fused_plan {
     std::vector<int> in_shape;
+    bool int8 = true;  // what fused() reports; the float plan keeps the name "per-layer" for its values, which are the layers'
     std::vector<dev_buffer> buffers;
     std::vector<std::function<void()>> launches;
     // Results: the launches write through `slot` into `t`, which forward() hands out. A result the caller still holds
@@ -593,6 +595,10 @@ template <>
 bool pipeline<unsigned short>::impl::build_graph_plan(const tensor_ptr&, const std::vector<int>&) { return false; }
 template <>
 bool pipeline<double>::impl::build_graph_plan(const tensor_ptr&, const std::vector<int>&) { return false; }
+template <>
+bool pipeline<unsigned short>::impl::build_float_plan(const tensor_ptr&, const std::vector<int>&) { return false; }
+template <>
+bool pipeline<double>::impl::build_float_plan(const tensor_ptr&, const std::vector<int>&) { return false; }
 
 template <>
 bool pipeline<float>::impl::build_block_plan(const tensor_ptr& input, const std::vector<int>& shape) {
@@ -1590,13 +1596,675 @@ bool pipeline<float>::impl::build_graph_plan(const tensor_ptr& input, const std:
     return true;
 }
 
+// The planner for float32 networks: every tensor between layers is float32 NHWC in the plan's own buffers, and the layers
+// between convolutions either run in a convolution's kernel or where its operands lie:
+//   * Convolution [-> activation layer / ReLU / PReLU] [-> add] [-> ReLU / activation layer] is one launch, a depthwise 3x3
+//     layer with its PReLU or ReLU too; a nearest Interp in front of the add (a feature pyramid's top-down path) is read through;
+//   * Concat costs nothing: its inputs' producers write their channels of the joined tensor. BatchNorm and the activation
+//     layer behind it run in the producers' epilogues where those are plain convolutions, else as one launch over the result;
+//   * a 2x2 stride-2 Deconvolution [-> BatchNorm] [-> ReLU] is four 1x1 layers in one launch;
+//   * Input and YoloV5Focus make the NHWC tensor the first convolution reads; a detection head's Reshape -> Transpose is how its
+//     convolution stores; anything behind the last planned layer runs as a layer on the NCHW results (the tail).
+// Values are those of the layers run one by one, bit for bit: the same kernels in the same order of sums. Anything else in the
+// topology returns false (the per-layer executor runs). What it replaces cost a layout conversion per convolution and a launch
+// per layer: 293 kernels for a yolov5s_simp forward, now 78.
+template <>
+bool pipeline<float>::impl::build_float_plan(const tensor_ptr& input, const std::vector<int>& shape) {
+    auto refuse = [&](int line) {
+        if (std::getenv("EXCALIBUR_PLAN_DEBUG")) LOG(INFO) << name_ << ": float plan not used (the check at pipeline.cpp:" << line << ")";
+        return false;
+    };
+    using conv_t = operation_convolution<float>;
+    const int n_ops = static_cast<int>(operations_.size());
+    const int n_blobs = static_cast<int>(blob_names_.size());
+    if (input->order() != memory::NCHW || shape.size() != 4 || input_names_.size() != 1) return refuse(__LINE__);
+
+    // ---- classify; blobs must be written once ----
+    // c convolution, d depthwise 3x3, v 2x2 deconvolution, u activation, r relu, q prelu, s split, a add, k concat, b batchnorm, i interp,
+    // p pooling, n input, f focus, t tail
+    std::vector<int> alias(n_blobs), producer(n_blobs, -1);
+    for (int b = 0; b < n_blobs; ++b) alias[b] = b;
+    std::vector<char> kind(n_ops, 't');
+    for (int i = 0; i < n_ops; ++i) {
+        operation<float>* op = operations_[i].get();
+        for (int o : op_outputs_[i]) {
+            if (producer[o] >= 0 || o == blob_index_[input_names_[0]]) return refuse(__LINE__);
+            producer[o] = i;
+        }
+        if (auto* d = dynamic_cast<operation_convolutiondepthwise<float>*>(op)) {
+            if (d->param().int8_quantization_) return refuse(__LINE__);
+            if (d->kernel_size_h_ == 3 && d->kernel_size_w_ == 3 && d->stride_h_ == d->stride_w_ && (d->stride_h_ == 1 || d->stride_h_ == 2) &&
+                d->dilation_h_ == 1 && d->dilation_w_ == 1 && d->output_channel_ == d->group_ &&
+                (d->activation_type_ == 0 || d->activation_type_ == 1 || d->activation_type_ == 3))
+                kind[i] = 'd';
+        } else if (auto* c = dynamic_cast<conv_t*>(op)) {
+            if (c->param().int8_quantization_) return refuse(__LINE__);
+            if (c->group_ == 1 && c->stride_h_ == c->stride_w_ && c->dilation_h_ == 1 && c->dilation_w_ == 1 && !c->weights_f32().empty()) kind[i] = 'c';
+        } else if (auto* v = dynamic_cast<operation_deconvolution<float>*>(op)) {
+            if (v->four_pointwise()) kind[i] = 'v';
+        } else if (auto* u = dynamic_cast<operation_unary<float>*>(op)) {
+            if (u->op_ != EXHIP_UNARY_SIGMOID) kind[i] = 'u';
+        } else if (dynamic_cast<operation_relu<float>*>(op)) {
+            kind[i] = 'r';
+        } else if (dynamic_cast<operation_prelu<float>*>(op)) {
+            kind[i] = 'q';
+        } else if (dynamic_cast<operation_split<float>*>(op)) {
+            kind[i] = 's';
+            for (int o : op_outputs_[i]) alias[o] = alias[op_inputs_[i][0]];
+        } else if (auto* b = dynamic_cast<operation_binaryop<float>*>(op)) {
+            if (b->op_type_ == 0 && !b->with_scalar_ && op_inputs_[i].size() == 2) kind[i] = 'a';
+        } else if (auto* e = dynamic_cast<operation_eltwise<float>*>(op)) {
+            if (e->type_ == 1 && op_inputs_[i].size() == 2 && e->coeffs_.size() == 2 && e->coeffs_[0] == 1.f && e->coeffs_[1] == 1.f) kind[i] = 'a';
+        } else if (auto* k = dynamic_cast<operation_concat<float>*>(op)) {
+            if (k->axis_ + 2 == 1 && op_inputs_[i].size() <= 8) kind[i] = 'k';
+        } else if (dynamic_cast<operation_batchnorm<float>*>(op)) {
+            kind[i] = 'b';
+        } else if (auto* ip = dynamic_cast<operation_interp<float>*>(op)) {
+            if (ip->resize_type_ == 1 && ip->align_corner_ == 0) kind[i] = 'i';
+        } else if (auto* p = dynamic_cast<operation_pooling<float>*>(op)) {
+            if (p->type_ == 0 || p->type_ == 1) kind[i] = 'p';
+        } else if (dynamic_cast<operation_input<float>*>(op)) {
+            kind[i] = 'n';
+        } else if (dynamic_cast<operation_yolov5focus<float>*>(op)) {
+            kind[i] = 'f';
+        }
+        if (kind[i] == 't' || kind[i] == 's') continue;
+        if (op_outputs_[i].size() != 1 || (kind[i] != 'a' && kind[i] != 'k' && op_inputs_[i].size() != 1)) return refuse(__LINE__);
+    }
+    auto root = [&](int b) { return alias[b]; };
+    std::vector<std::vector<int>> consumers(n_blobs);
+    for (int i = 0; i < n_ops; ++i)
+        if (kind[i] != 's')
+            for (int b : op_inputs_[i]) consumers[root(b)].push_back(i);
+    std::vector<char> is_output(n_blobs, 0);
+    for (const std::string& o : output_names_) is_output[root(blob_index_[o])] = 1;
+    const int in_value = root(blob_index_[input_names_[0]]);
+
+    // ---- the layers in front ----
+    auto plan = std::make_shared<fused_plan>();
+    plan->in_shape = shape;
+    plan->int8 = false;
+    std::vector<char> where(n_blobs, 0);  // 0 a value of the plan, 1 an NCHW blob of the front chain, 2 a blob of the tail
+    where[in_value] = 1;
+    int front_value = in_value;
+    std::vector<int> front_shape = shape;
+    for (int i = 0; i < n_ops; ++i) {
+        if (kind[i] != 'n' && kind[i] != 'f') continue;
+        if (root(op_inputs_[i][0]) != front_value || consumers[front_value].size() != 1 || is_output[front_value]) return refuse(__LINE__);
+        plan->front_ops.push_back(i);
+        front_value = root(op_outputs_[i][0]);
+        where[front_value] = 1;
+        if (kind[i] == 'f') front_shape = {front_shape[0], front_shape[1] * 4, front_shape[2] / 2, front_shape[3] / 2};
+    }
+    if (is_output[front_value] || consumers[front_value].empty()) return refuse(__LINE__);
+    for (int c : consumers[front_value])
+        if (kind[c] != 'c') return refuse(__LINE__);
+
+    // ---- nodes ----
+    struct node {
+        char kind;  // c, d, v as above; g glue (Concat / BatchNorm / activation), r, a, i, p
+        int op, at;
+        std::vector<int> in;
+        int res = -1, out = -1;
+        int unary = -1, bn = -1, prelu = -1;  // layer numbers of absorbed layers
+        bool post_relu = false, residual_last = false, bn_relu = false;
+        int head_reshape = -1;                // convolution: the Reshape layer of a detection head (Reshape -> Transpose) it absorbs
+        int cascade = -1, cascade_k = 0;      // max pooling: the value of a smaller pool of the same input to pool again
+        enum { launch, placed, joined } join = launch;  // Concat: how its result comes about
+        int into = -1, into_offset = 0;       // convolution: the joined Concat's node and the first channel there
+    };
+    std::vector<node> nodes;
+    std::vector<char> absorbed(n_ops, 0);
+    auto sole = [&](int v, char want) -> int {  // the single reader of v if it is an unclaimed layer of kind `want`
+        if (is_output[v] || consumers[v].size() != 1) return -1;
+        const int c = consumers[v][0];
+        return (kind[c] == want && !absorbed[c]) ? c : -1;
+    };
+    for (int i = 0; i < n_ops; ++i) {
+        if (absorbed[i] || kind[i] == 's' || kind[i] == 'n' || kind[i] == 'f' || kind[i] == 't') continue;
+        node nd;
+        nd.kind = kind[i] == 'k' || kind[i] == 'b' || kind[i] == 'u' ? 'g' : kind[i];
+        nd.op = nd.at = i;
+        for (int b : op_inputs_[i]) nd.in.push_back(root(b));
+        nd.out = root(op_outputs_[i][0]);
+        auto absorb = [&](int layer) {
+            absorbed[layer] = 1;
+            nd.at = layer;
+            nd.out = root(op_outputs_[layer][0]);
+        };
+        if (kind[i] == 'c') {
+            auto* c = static_cast<conv_t*>(operations_[i].get());
+            int act = -1;
+            if ((act = sole(nd.out, 'u')) >= 0) {
+                nd.unary = act;
+            } else if ((act = sole(nd.out, 'r')) >= 0) {
+                nd.post_relu = true;
+            } else if ((act = sole(nd.out, 'q')) >= 0) {
+                auto* q = static_cast<operation_prelu<float>*>(operations_[act].get());
+                if (!q->share_channel_ && q->num_slope_ != c->output_channel_) return refuse(__LINE__);
+                nd.prelu = act;
+            }
+            if (act >= 0) absorb(act);
+            const int rs = act < 0 ? sole(nd.out, 't') : -1;  // a detection head: Reshape (channels into groups) -> Transpose of the last two axes
+            if (rs >= 0 && dynamic_cast<operation_reshape<float>*>(operations_[rs].get())) {
+                const int tp = sole(root(op_outputs_[rs][0]), 't');
+                auto* transpose = tp >= 0 ? dynamic_cast<operation_transpose<float>*>(operations_[tp].get()) : nullptr;
+                if (transpose && transpose->perms_.size() == 3 && transpose->perms_[0] == 1 && transpose->perms_[1] == 0 && transpose->perms_[2] == 2) {
+                    nd.head_reshape = rs;
+                    absorb(rs);
+                    absorb(tp);
+                }
+            }
+            const int sum = nd.head_reshape < 0 ? sole(nd.out, 'a') : -1;
+            if (sum >= 0) {
+                const int x = root(op_inputs_[sum][0]), y = root(op_inputs_[sum][1]);
+                // the other operand must be there by then, and be another value
+                if (x != y) {
+                    nd.res = x == nd.out ? y : x;
+                    nd.residual_last = act >= 0;
+                    absorb(sum);
+                    if (act < 0) {  // the activation behind the sum
+                        int behind = sole(nd.out, 'r');
+                        if (behind >= 0) {
+                            nd.post_relu = true;
+                            absorb(behind);
+                        } else if ((behind = sole(nd.out, 'u')) >= 0) {
+                            nd.unary = behind;
+                            absorb(behind);
+                        }
+                    }
+                }
+            }
+        } else if (kind[i] == 'd') {
+            auto* d = static_cast<operation_convolutiondepthwise<float>*>(operations_[i].get());
+            int act = -1;
+            if (d->activation_type_ == 0) {
+                if ((act = sole(nd.out, 'q')) >= 0) {
+                    auto* q = static_cast<operation_prelu<float>*>(operations_[act].get());
+                    if (!q->share_channel_ && q->num_slope_ != d->output_channel_) return refuse(__LINE__);
+                    nd.prelu = act;
+                } else if ((act = sole(nd.out, 'r')) >= 0) {
+                    nd.post_relu = true;
+                }
+                if (act >= 0) absorb(act);
+            }
+        } else if (kind[i] == 'v') {
+            const int bn = sole(nd.out, 'b');
+            if (bn >= 0) {
+                nd.bn = bn;
+                absorb(bn);
+            }
+            const int relu = sole(nd.out, 'r');
+            if (relu >= 0) {
+                (bn >= 0 ? nd.bn_relu : nd.post_relu) = true;
+                absorb(relu);
+            }
+        } else if (nd.kind == 'g') {
+            if (kind[i] == 'b') nd.bn = i;
+            if (kind[i] == 'u') nd.unary = i;
+            if (kind[i] == 'k') {
+                const int bn = sole(nd.out, 'b');
+                if (bn >= 0) {
+                    nd.bn = bn;
+                    absorb(bn);
+                }
+            }
+            if (kind[i] != 'u') {
+                const int act = sole(nd.out, 'u');
+                if (act >= 0) {
+                    nd.unary = act;
+                    absorb(act);
+                }
+            }
+        } else if (kind[i] == 'q') {
+            return refuse(__LINE__);  // a PReLU no convolution's epilogue takes
+        }
+        nodes.push_back(nd);
+    }
+    std::stable_sort(nodes.begin(), nodes.end(), [](const node& a, const node& b) { return a.at < b.at; });
+    if (nodes.empty()) return refuse(__LINE__);
+    for (int i = 0; i < n_ops; ++i) {
+        if (absorbed[i]) continue;
+        if (kind[i] == 't') {
+            for (int b : op_inputs_[i])
+                if (where[root(b)] == 1) return refuse(__LINE__);  // the front chain's blobs are not kept
+            plan->tail_ops.push_back(i);
+            for (int o : op_outputs_[i]) where[root(o)] = 2;
+        } else if (kind[i] == 's' && where[root(op_inputs_[i][0])] == 2) {
+            plan->tail_ops.push_back(i);
+        }
+    }
+    for (const node& nd : nodes) {  // nothing but the tail reads the tail, nothing but convolutions the front
+        if (where[nd.out] != 0 || (nd.res >= 0 && where[nd.res] != 0)) return refuse(__LINE__);
+        for (int v : nd.in)
+            if (where[v] == 2 || (where[v] == 1 && nd.kind != 'c')) return refuse(__LINE__);
+    }
+
+    // ---- values ----
+    struct value_info {
+        bool rows = false, nchw_wanted = false;  // read by a planned layer as NHWC; leaves as NCHW
+        int n = 0, c = 0, h = 0, w = 0, cs = 0;
+        float* p = nullptr;
+        int parent = -1, offset = 0;             // a slice of a Concat's result
+        int through = -1, shift = 0;             // a nearest Interp that its only reader looks through: its input and log2 of the factor
+    };
+    std::vector<value_info> vals(n_blobs);
+    std::vector<int> node_of(n_blobs, -1);
+    for (size_t i = 0; i < nodes.size(); ++i) node_of[nodes[i].out] = static_cast<int>(i);
+    for (int b = 0; b < n_blobs; ++b)
+        if (is_output[b] && where[b] == 0) vals[b].nchw_wanted = true;
+    for (int t : plan->tail_ops)
+        for (int b : op_inputs_[t])
+            if (where[root(b)] == 0) vals[root(b)].nchw_wanted = true;
+    vals[front_value].c = front_shape[1];
+    for (const node& nd : nodes) {  // channel counts are known from the layers alone
+        int c = vals[nd.in[0]].c;
+        if (nd.kind == 'c') c = static_cast<conv_t*>(operations_[nd.op].get())->output_channel_;
+        else if (nd.kind == 'v') c = static_cast<operation_deconvolution<float>*>(operations_[nd.op].get())->output_channel_;
+        else if (nd.kind == 'g')
+            for (size_t j = 1; j < nd.in.size(); ++j) c += vals[nd.in[j]].c;
+        vals[nd.out].c = c;
+        for (int v : nd.in) vals[v].rows = true;
+        if (nd.res >= 0) vals[nd.res].rows = true;
+    }
+    // Concat: its inputs' producers write their channels of the joined tensor where each is a planned layer's result that
+    // lies in no other Concat and starts and ends on whole 32-byte steps
+    for (size_t i = 0; i < nodes.size(); ++i) {
+        node& nd = nodes[i];
+        if (nd.kind != 'g' || kind[nd.op] != 'k') continue;
+        bool can = true, plain = true;
+        std::set<int> seen;
+        for (int v : nd.in) {
+            const int pn = node_of[v];
+            can = can && pn >= 0 && vals[v].parent < 0 && vals[v].c % 8 == 0 && seen.insert(v).second;
+            if (!can) break;
+            const node& pr = nodes[pn];
+            can = pr.kind == 'c' || pr.kind == 'i' || pr.kind == 'p' || pr.kind == 'g';
+            plain = plain && pr.kind == 'c' && pr.unary < 0 && pr.prelu < 0 && !pr.post_relu && pr.res < 0 && pr.head_reshape < 0 && pr.into < 0 &&
+                    !is_output[v] && consumers[v].size() == 1;
+        }
+        if (!can) continue;
+        nd.join = plain && (nd.bn >= 0 || nd.unary >= 0) ? node::joined : node::placed;
+        int offset = 0;
+        for (int v : nd.in) {
+            vals[v].parent = nd.out;
+            vals[v].offset = offset;
+            if (nd.join == node::joined) {
+                nodes[node_of[v]].into = static_cast<int>(i);
+                nodes[node_of[v]].into_offset = offset;
+            }
+            offset += vals[v].c;
+        }
+    }
+
+    // ---- shapes, buffers, launches ----
+    exhip_ctx* ctx = memory::device_context(device_);
+    const int dev = device_;
+    auto alloc = [&](size_t floats) {
+        plan->buffers.emplace_back(dev, floats * sizeof(float));
+        return static_cast<float*>(plan->buffers.back().ptr);
+    };
+    auto upload = [&](const std::vector<float>& host) {
+        float* p = alloc(host.size());
+        EXHIP_FATAL(exhip_memcpy_h2d(ctx, p, host.data(), host.size() * sizeof(float)));
+        return p;
+    };
+    auto blobs_of = [&](int value) {  // the names a tail layer may read the value by
+        std::vector<int> ids;
+        for (int b = 0; b < n_blobs; ++b)
+            if (root(b) == value) ids.push_back(b);
+        return ids;
+    };
+    std::vector<float**> slot_of(n_blobs, nullptr);
+    auto nchw_result = [&](int value) {
+        const value_info& v = vals[value];
+        slot_of[value] = plan->new_result({v.n, v.c, v.h, v.w}, dev);
+        plan->outputs.back().blobs = blobs_of(value);
+        return slot_of[value];
+    };
+    // the NHWC buffer of a value whose shape is known: its own, or its place in the Concat it belongs to
+    std::function<bool(int)> place = [&](int value) {
+        value_info& v = vals[value];
+        if (v.p) return true;
+        if (v.parent < 0) {
+            v.cs = pad_to(v.c, 8);
+            v.p = alloc(static_cast<size_t>(v.n) * v.h * v.w * v.cs);
+            return true;
+        }
+        value_info& up = vals[v.parent];
+        if (up.n == 0) { up.n = v.n; up.h = v.h; up.w = v.w; }
+        if (up.n != v.n || up.h != v.h || up.w != v.w || !place(v.parent)) return false;
+        v.cs = vals[v.parent].cs;
+        v.p = vals[v.parent].p + v.offset;
+        return true;
+    };
+    auto nchw_from_rows = [&](int value) {  // a value that leaves as NCHW from a layer other than a convolution
+        if (!vals[value].nchw_wanted) return;
+        float** slot = nchw_result(value);
+        const value_info v = vals[value];
+        plan->launches.push_back([=]() { EXHIP_FATAL(exhip_nhwc_f32_to_nchw_f32(ctx, v.p, v.n, v.c, v.h, v.w, v.cs, *slot)); });
+    };
+    {
+        value_info& v = vals[front_value];
+        v.n = front_shape[0]; v.h = front_shape[2]; v.w = front_shape[3];
+        v.cs = v.c <= 4 ? 4 : pad_to(v.c, 8);
+        v.p = alloc(static_cast<size_t>(v.n) * v.h * v.w * v.cs);
+        fused_plan* pl = plan.get();
+        float* y = v.p;
+        const int cs = v.cs, ch = shape[1], n0 = shape[0], h0 = shape[2], w0 = shape[3];
+        bool one_kernel = false;
+        const size_t n_front = plan->front_ops.size();
+        if (n_front >= 1 && n_front <= 2 && kind[plan->front_ops[0]] == 'n' && (n_front == 1 || kind[plan->front_ops[1]] == 'f')) {
+            auto* in_op = static_cast<operation_input<float>*>(operations_[plan->front_ops[0]].get());
+            if ((ch == 1 || ch == 3) && static_cast<int>(in_op->means_.size()) == ch && static_cast<int>(in_op->vars_.size()) >= ch) {
+                std::array<float, 4> means{}, scales{};
+                for (int c = 0; c < ch; ++c) { means[c] = in_op->means_[c]; scales[c] = in_op->vars_[c]; }
+                const int focus = n_front == 2;
+                const int rc = exhip_input_nchw_f32_to_nhwc_f32(ctx, input->gpu_data(), n0, ch, h0, w0, means.data(), scales.data(), focus, cs, y);  // trial launch
+                if (rc == 0) {
+                    one_kernel = true;
+                    plan->front_ops.clear();
+                    plan->launches.push_back([=]() {
+                        EXHIP_FATAL(exhip_input_nchw_f32_to_nhwc_f32(ctx, pl->input_ptr, n0, ch, h0, w0, means.data(), scales.data(), focus, cs, y));
+                    });
+                } else if (rc != EXHIP_ERR_UNSUPPORTED) {
+                    EXHIP_FATAL(rc);
+                }
+            }
+        }
+        const value_info vi = v;
+        if (!one_kernel)
+            plan->launches.push_back([=]() { EXHIP_FATAL(exhip_nchw_f32_to_nhwc_f32(ctx, pl->input_ptr, vi.n, vi.c, vi.h, vi.w, cs, y)); });
+    }
+    for (const node& nd : nodes) {
+        const value_info in = vals[nd.in[0]];
+        value_info& out = vals[nd.out];
+        if (in.n == 0) return refuse(__LINE__);
+        if (nd.kind == 'c') {
+            auto* c = static_cast<conv_t*>(operations_[nd.op].get());
+            if (in.c != c->input_channels() || !in.p) return refuse(__LINE__);
+            exhip_conv_desc d = c->describe(in.n, in.h, in.w, in.cs, pad_to(c->output_channel_, 8));
+            int oh, ow;
+            EXHIP_FATAL(exhip_conv_out_hw(&d, &oh, &ow));
+            out.n = in.n; out.h = oh; out.w = ow;
+            d.post_relu = nd.post_relu ? 1 : 0;
+            d.residual_last = nd.residual_last ? 1 : 0;
+            exhip_conv_place how;
+            std::memset(&how, 0, sizeof(how));
+            if (nd.unary >= 0) {
+                auto* u = static_cast<operation_unary<float>*>(operations_[nd.unary].get());
+                d.post_op = 1 + u->op_; d.post_alpha = u->alpha_; d.post_beta = u->beta_;
+            }
+            if (nd.prelu >= 0) {
+                auto* q = static_cast<operation_prelu<float>*>(operations_[nd.prelu].get());
+                d.post_op = EXHIP_POST_PRELU;
+                d.post_slope = q->weights_f32()[0]->gpu_data();
+                d.post_slope_shared = q->share_channel_ ? 1 : 0;
+            }
+            if (nd.into >= 0) {  // its channels' BatchNorm and activation of the Concat it belongs to
+                const node& jn = nodes[nd.into];
+                if (jn.bn >= 0) {
+                    auto* bn = static_cast<operation_batchnorm<float>*>(operations_[jn.bn].get());
+                    if (bn->channels_ != vals[jn.out].c || !bn->a_ || !bn->b_) return refuse(__LINE__);
+                    d.post_bn_a = bn->a_->gpu_data() + nd.into_offset;
+                    d.post_bn_b = bn->b_->gpu_data() + nd.into_offset;
+                }
+                if (jn.unary >= 0) {
+                    auto* u = static_cast<operation_unary<float>*>(operations_[jn.unary].get());
+                    d.post_op = 1 + u->op_; d.post_alpha = u->alpha_; d.post_beta = u->beta_;
+                }
+            }
+            const float* res = nullptr;
+            if (nd.res >= 0) {
+                const value_info& sum = vals[nd.res];
+                const value_info& r = sum.through >= 0 ? vals[sum.through] : sum;
+                if (!r.p || sum.n != out.n || sum.h != oh || sum.w != ow || r.c != out.c) return refuse(__LINE__);
+                res = r.p;
+                how.residual_stride = r.cs;
+                how.residual_shift = sum.through >= 0 ? sum.shift : 0;
+            }
+            float *y = nullptr, **slot = nullptr;
+            bool slot_is_rows = false;  // the launch's first output is the result slot
+            if (nd.head_reshape >= 0) {
+                // [n, K, oh, ow] -> Reshape [n, G, J, oh * ow] -> Transpose [n, G, oh * ow, J]
+                auto* rs = static_cast<operation_reshape<float>*>(operations_[nd.head_reshape].get());
+                const std::vector<int> to = rs->new_shape({in.n, c->output_channel_, oh, ow}, in.n * c->output_channel_ * oh * ow);
+                if (to.size() != 4 || to[0] != in.n || to[1] * to[2] != c->output_channel_ || to[3] != oh * ow) return refuse(__LINE__);
+                if (out.rows || !out.nchw_wanted || out.parent >= 0) return refuse(__LINE__);
+                how.layout = EXHIP_PLACE_GROUPED;
+                how.group = to[2];
+                out.c = to[1]; out.h = oh * ow; out.w = to[2];
+                slot = nchw_result(nd.out);
+                slot_is_rows = true;
+            } else {
+                if (out.rows || out.parent >= 0 || !out.nchw_wanted) {
+                    if (!place(nd.out)) return refuse(__LINE__);
+                    y = out.p;
+                    d.k_stride = out.cs;
+                    d.exact_k = out.parent >= 0 ? 1 : 0;
+                }
+                if (out.nchw_wanted) slot = nchw_result(nd.out);
+            }
+            const void* wp = c->pin_packed_weights(EXHIP_F32, d);  // the launch keeps this pointer
+            plan->pinned.emplace_back([c, wp]() { c->unpin_packed_weights(wp); });
+            const float *bias = c->bias_gpu(), *x = in.p;
+            plan->launches.push_back([=]() {
+                EXHIP_FATAL(exhip_conv2d_f32_placed(ctx, &d, &how, x, wp, bias, res, slot_is_rows ? *slot : y, slot && !slot_is_rows ? *slot : nullptr));
+            });
+        } else if (nd.kind == 'd') {
+            auto* c = static_cast<operation_convolutiondepthwise<float>*>(operations_[nd.op].get());
+            if (in.c != c->output_channel_ || !in.p || out.parent >= 0) return refuse(__LINE__);
+            out.n = in.n;
+            out.h = (in.h + c->pad_top_ + c->pad_bottom_ - 3) / c->stride_h_ + 1;
+            out.w = (in.w + c->pad_left_ + c->pad_right_ - 3) / c->stride_w_ + 1;
+            if (out.h < 1 || out.w < 1 || !place(nd.out) || out.cs != in.cs) return refuse(__LINE__);
+            const float *w9 = c->weights_f32()[0]->gpu_data(), *bias = c->bias_gpu(), *slope = nullptr;
+            int shared = 0;
+            if (nd.prelu >= 0) {
+                auto* q = static_cast<operation_prelu<float>*>(operations_[nd.prelu].get());
+                slope = q->weights_f32()[0]->gpu_data();
+                shared = q->share_channel_ ? 1 : 0;
+            }
+            const int act = nd.post_relu ? 1 : c->activation_type_, stride = c->stride_h_;
+            const int pt = c->pad_top_, pb = c->pad_bottom_, pl = c->pad_left_, pr = c->pad_right_;
+            const float* x = in.p;
+            float* y = out.p;
+            const int rc = exhip_dwconv3x3_nhwc_f32(ctx, x, w9, bias, slope, shared, y, in.n, in.c, in.h, in.w, in.cs, stride, pt, pb, pl, pr, act);  // trial
+            if (rc == EXHIP_ERR_UNSUPPORTED) return refuse(__LINE__);
+            EXHIP_FATAL(rc);
+            plan->launches.push_back([=]() {
+                EXHIP_FATAL(exhip_dwconv3x3_nhwc_f32(ctx, x, w9, bias, slope, shared, y, in.n, in.c, in.h, in.w, in.cs, stride, pt, pb, pl, pr, act));
+            });
+            nchw_from_rows(nd.out);
+        } else if (nd.kind == 'v') {
+            auto* c = static_cast<operation_deconvolution<float>*>(operations_[nd.op].get());
+            const int k = c->output_channel_;
+            if (in.c != c->deconv_input_channels() || !in.p || out.parent >= 0) return refuse(__LINE__);
+            exhip_conv_desc d;
+            std::memset(&d, 0, sizeof(d));
+            d.n = in.n; d.c = in.c; d.h = in.h; d.w = in.w; d.k = 4 * k; d.kh = d.kw = d.sh = d.sw = 1;
+            d.c_stride = in.cs;
+            d.post_relu = nd.post_relu ? 1 : 0;
+            exhip_conv_place how;
+            std::memset(&how, 0, sizeof(how));
+            how.layout = EXHIP_PLACE_SHUFFLED;
+            how.group = k;
+            how.bn_relu = nd.bn_relu ? 1 : 0;
+            if (nd.bn >= 0) {
+                auto* bn = static_cast<operation_batchnorm<float>*>(operations_[nd.bn].get());
+                if (bn->channels_ != k || !bn->a_ || !bn->b_) return refuse(__LINE__);
+                std::vector<float> a, b;
+                for (int pos = 0; pos < 4; ++pos) {
+                    a.insert(a.end(), bn->a_->cpu_data(), bn->a_->cpu_data() + k);
+                    b.insert(b.end(), bn->b_->cpu_data(), bn->b_->cpu_data() + k);
+                }
+                d.post_bn_a = upload(a);
+                d.post_bn_b = upload(b);
+            }
+            out.n = in.n; out.h = 2 * in.h; out.w = 2 * in.w;
+            float* y = nullptr;
+            float** slot = nullptr;
+            if (k == 1 && !out.rows && out.nchw_wanted) {  // one channel: NHWC and NCHW are the same
+                slot = nchw_result(nd.out);
+                d.k_stride = 1;
+            } else {
+                if (!place(nd.out)) return refuse(__LINE__);
+                if (out.cs != k) return refuse(__LINE__);  // pad channels would be left unwritten
+                y = out.p;
+                d.k_stride = out.cs;
+            }
+            const void* wp = c->pointwise_weights(d);
+            const float *bias = c->pointwise_bias(), *x = in.p;
+            plan->launches.push_back([=]() { EXHIP_FATAL(exhip_conv2d_f32_placed(ctx, &d, &how, x, wp, bias, nullptr, slot ? *slot : y, nullptr)); });
+            if (!slot) nchw_from_rows(nd.out);
+        } else if (nd.kind == 'g') {
+            int total = 0;
+            std::vector<const float*> ptrs;
+            std::vector<int> channels, strides;
+            for (int v : nd.in) {
+                const value_info& s = vals[v];
+                if (!s.p || s.n != in.n || s.h != in.h || s.w != in.w) return refuse(__LINE__);
+                ptrs.push_back(s.p);
+                channels.push_back(s.c);
+                strides.push_back(s.cs);
+                total += s.c;
+            }
+            out.n = in.n; out.h = in.h; out.w = in.w;
+            if (!place(nd.out)) return refuse(__LINE__);
+            const bool work = nd.join == node::launch || (nd.join == node::placed && (nd.bn >= 0 || nd.unary >= 0));
+            if (work) {
+                if (out.parent >= 0 || total % 4 != 0) return refuse(__LINE__);
+                for (int ch : channels)
+                    if (ch % 4 != 0) return refuse(__LINE__);
+                if (nd.join == node::placed) {  // the joined tensor is there: one pass over it
+                    ptrs = {out.p};
+                    channels = {total};
+                    strides = {out.cs};
+                }
+                const float *bn_a = nullptr, *bn_b = nullptr;
+                if (nd.bn >= 0) {
+                    auto* bn = static_cast<operation_batchnorm<float>*>(operations_[nd.bn].get());
+                    if (bn->channels_ != total || !bn->a_ || !bn->b_) return refuse(__LINE__);
+                    bn_a = bn->a_->gpu_data();
+                    bn_b = bn->b_->gpu_data();
+                }
+                int uop = -1;
+                float alpha = 0.f, beta = 0.f;
+                if (nd.unary >= 0) {
+                    auto* u = static_cast<operation_unary<float>*>(operations_[nd.unary].get());
+                    uop = u->op_; alpha = u->alpha_; beta = u->beta_;
+                }
+                const size_t pixels = static_cast<size_t>(out.n) * out.h * out.w;
+                float* y = out.p;
+                const int cs = out.cs, n_in = static_cast<int>(ptrs.size());
+                plan->launches.push_back([=]() {
+                    EXHIP_FATAL(exhip_concat_batchnorm_unary_nhwc_f32(ctx, ptrs.data(), channels.data(), strides.data(), n_in, pixels, bn_a, bn_b, uop, alpha,
+                                                                      beta, cs, y, nullptr, 0.f));
+                });
+            }
+            nchw_from_rows(nd.out);
+        } else if (nd.kind == 'a' || nd.kind == 'r') {  // a sum or ReLU no convolution's epilogue takes: over whole buffers
+            out.n = in.n; out.h = in.h; out.w = in.w;
+            if (!in.p || in.parent >= 0 || out.parent >= 0 || !place(nd.out) || out.cs != in.cs) return refuse(__LINE__);
+            const size_t count = static_cast<size_t>(out.n) * out.h * out.w * out.cs;
+            const float* x = in.p;
+            float* y = out.p;
+            if (nd.kind == 'r') {
+                plan->launches.push_back([=]() { EXHIP_FATAL(exhip_relu_f32(ctx, x, y, count)); });
+            } else {
+                const value_info& o = vals[nd.in[1]];
+                if (!o.p || o.parent >= 0 || o.n != in.n || o.c != in.c || o.h != in.h || o.w != in.w || o.cs != in.cs) return refuse(__LINE__);
+                const float* x2 = o.p;
+                plan->launches.push_back([=]() { EXHIP_FATAL(exhip_add_f32(ctx, x, x2, y, count, 0)); });
+            }
+            nchw_from_rows(nd.out);
+        } else if (nd.kind == 'i') {
+            auto* ip = static_cast<operation_interp<float>*>(operations_[nd.op].get());
+            int oh = ip->output_height_, ow = ip->output_width_;
+            if (oh == 0 || ow == 0) {
+                oh = static_cast<int>(in.h * ip->height_scale_);
+                ow = static_cast<int>(in.w * ip->width_scale_);
+            }
+            if (oh <= 0 || ow <= 0 || !in.p) return refuse(__LINE__);
+            out.n = in.n; out.h = oh; out.w = ow;
+            // read through by the convolution that adds it, if that is its only reader and the factor a power of two
+            bool through = false;
+            if (out.parent < 0 && !is_output[nd.out] && consumers[nd.out].size() == 1)
+                for (const node& reader : nodes)
+                    if (reader.kind == 'c' && reader.res == nd.out)
+                        for (int s = 1; s <= 4; ++s)
+                            if (oh == in.h << s && ow == in.w << s) {
+                                through = true;
+                                out.through = nd.in[0];
+                                out.shift = s;
+                            }
+            if (through) continue;
+            if (!place(nd.out)) return refuse(__LINE__);
+            const value_info o = out;
+            if (in.cs % 4 != 0 || o.cs % 4 != 0) return refuse(__LINE__);
+            const int ch = pad_to(in.c, 8);  // with the pad channels (a slice has none)
+            plan->launches.push_back([=]() {
+                EXHIP_FATAL(exhip_interp_nearest_nhwc_f32(ctx, in.p, in.cs, o.p, o.cs, in.n, ch, in.h, in.w, oh, ow));
+            });
+            nchw_from_rows(nd.out);
+        } else {
+            auto* p = static_cast<operation_pooling<float>*>(operations_[nd.op].get());
+            int kh, kw, sh, sw, pt, pb, pl, pr, oh, ow;
+            p->geometry(in.h, in.w, &kh, &kw, &sh, &sw, &pt, &pb, &pl, &pr, &oh, &ow);
+            out.n = in.n; out.h = oh; out.w = ow;
+            if (!in.p || !place(nd.out)) return refuse(__LINE__);
+            // A pyramid of stride-1 "same" max pools over one tensor: the maximum over a window of k is the maximum over a window
+            // of k - k' + 1 of the maxima over windows of k' (taps outside the image count in neither)
+            value_info src = in;
+            auto same_window = [&](const operation_pooling<float>* q) {
+                const int k = q->kernel_size_w_;
+                const bool same = q->type_ == 0 && !q->global_pooling_ && k == q->kernel_size_h_ && (k & 1) && q->stride_w_ == 1 && q->stride_h_ == 1 &&
+                                  q->pad_left_ == k / 2 && q->pad_right_ == k / 2 && q->pad_top_ == k / 2 && q->pad_bottom_ == k / 2;
+                return same ? k : 0;
+            };
+            const int k = same_window(p);
+            int best = 0;
+            if (k > 0 && oh == in.h && ow == in.w)
+                for (const node& q : nodes) {
+                    if (q.kind != 'p' || q.op == nd.op || q.at > nd.at || q.in[0] != nd.in[0]) continue;
+                    const int kq = same_window(static_cast<operation_pooling<float>*>(operations_[q.op].get()));
+                    const value_info& qv = vals[q.out];
+                    if (kq > best && kq < k && qv.p && qv.h == in.h && qv.w == in.w) {
+                        best = kq;
+                        src = qv;
+                        kh = kw = k - kq + 1;
+                        pt = pb = pl = pr = (k - kq + 1) / 2;
+                    }
+                }
+            const value_info o = out;
+            const int type = p->type_, include_pad = p->avgpool_count_include_pad_, ch = pad_to(in.c, 8);  // with the pad channels (a slice has none)
+            const int rc = exhip_pool2d_nhwc_f32(ctx, src.p, src.cs, o.p, o.cs, in.n, ch, in.h, in.w, oh, ow, type, kh, kw, sh, sw, pt, pb, pl, pr, include_pad);
+            if (rc == EXHIP_ERR_UNSUPPORTED) return refuse(__LINE__);
+            EXHIP_FATAL(rc);
+            plan->launches.push_back([=]() {
+                EXHIP_FATAL(exhip_pool2d_nhwc_f32(ctx, src.p, src.cs, o.p, o.cs, in.n, ch, in.h, in.w, oh, ow, type, kh, kw, sh, sw, pt, pb, pl, pr, include_pad));
+            });
+            nchw_from_rows(nd.out);
+        }
+    }
+    for (const std::string& o : output_names_) {
+        const int v = root(blob_index_[o]);
+        if (where[v] == 2) continue;
+        if (where[v] != 0 || !slot_of[v]) return refuse(__LINE__);
+        for (auto& r : plan->outputs)
+            if (&r.slot == slot_of[v]) r.name += (r.name.empty() ? "" : "\n") + o;
+    }
+    plan_ = plan;
+    return true;
+}
+
 template <>
 bool pipeline<float>::impl::try_fused(const tensor_ptr& input, blob_map* results) {
     if (!fusion_ || fused_unsupported_) return false;
     const std::vector<int> shape = input->data_shape();
     if (!plan_ || plan_->in_shape != shape) {
         plan_.reset();
-        if (!build_block_plan(input, shape) && !build_graph_plan(input, shape)) {
+        if (!build_block_plan(input, shape) && !build_graph_plan(input, shape) && !build_float_plan(input, shape)) {
             fused_unsupported_ = true;  // the per-layer executor from now on
             plan_.reset();
             return false;
@@ -1669,7 +2337,7 @@ bool pipeline<float>::impl::try_fused(const tensor_ptr& input, blob_map* results
     }
     if (timed) ++span_count_;
     ++plan_->forwards;
-    last_fused_ = true;
+    last_fused_ = plan_->int8;
     for (auto& r : plan_->outputs) {
         r.t->mutable_gpu_data();  // the kernels just wrote it: the device copy is the newest
         for (int b : r.blobs) featmaps_[b] = r.t;

@@ -212,6 +212,22 @@ int exhip_conv2d_f16(exhip_ctx* ctx, const exhip_conv_desc* d, const uint16_t* x
 int exhip_conv2d_f32(exhip_ctx* ctx, const exhip_conv_desc* d, const float* x_nhwc, const void* w_packed,
                      const float* bias, const float* residual_nhwc, float* y_f32_nhwc, float* y_f32_nchw);
 
+/* The same with layers behind the convolution that move values folded into where they are read and written (the executor of
+ * src/Excalibur/pipeline.cpp:326-392 runs each as a layer of its own). The input may be a slice of a wider NHWC tensor
+ * (c_stride > c), the output too (k_stride > k with exact_k); d->post_bn_a / post_bn_b apply here, in front of post_op. */
+#define EXHIP_PLACE_ROWS 0     /* NHWC */
+#define EXHIP_PLACE_GROUPED 1  /* a detection head's Reshape + Transpose (operation_reshape.cpp, operation_transpose.cpp): [n][k / group][pixel][group] */
+#define EXHIP_PLACE_SHUFFLED 2 /* a 2x2 stride-2 Deconvolution (operation_deconvolution.cpp) as four 1x1 layers: output channel pos * group + k
+                                * is channel k of output pixel (2 y + pos / 2, 2 x + pos % 2); k == 4 * group, k_stride that map's stride */
+typedef struct exhip_conv_place {
+    int layout, group;
+    int residual_stride;   /* the shortcut's channel stride */
+    int residual_shift;    /* its map is 2^shift times smaller in each direction: a nearest Interp (operation_interp.cpp:247-268) in front of the sum */
+    int bn_relu;           /* ReLU behind the BatchNorm */
+} exhip_conv_place;
+int exhip_conv2d_f32_placed(exhip_ctx* ctx, const exhip_conv_desc* d, const exhip_conv_place* place, const float* x_nhwc, const void* w_packed,
+                            const float* bias, const float* residual_nhwc, float* y, float* y_f32_nchw);
+
 /* Any geometry incl. groups, straight from the definition on NCHW f32 (slow; used for shapes the
  * MFMA path does not take). int8 mode when w_i8 != NULL: quantizes x with fs on the fly and applies
  * fmaf(acc, scale[k], bias[k]); otherwise f32 weights. */
@@ -237,6 +253,10 @@ int exhip_dwconv3x3_nchw_f32_prelu(exhip_ctx* ctx, const float* x, const float* 
 int exhip_dwconv3x3_nhwc_f16_prelu(exhip_ctx* ctx, const uint16_t* x, const float* w9, const float* bias, const float* slope,
                                    int slope_shared, uint16_t* y, int n, int c, int h, int w, int cs, int stride, int pt, int pb,
                                    int pl, int pr);
+/* ... and on NHWC f32 (c_stride a multiple of 8), with the PReLU layer behind it where slope is not NULL (act 0 then). act 0, 1
+ * or 3; EXHIP_ERR_UNSUPPORTED for the others and for tensors beyond 1 GiB. */
+int exhip_dwconv3x3_nhwc_f32(exhip_ctx* ctx, const float* x, const float* w9, const float* bias, const float* slope, int slope_shared,
+                             float* y, int n, int c, int h, int w, int c_stride, int stride, int pt, int pb, int pl, int pr, int act);
 int exhip_dw_dequant_weights(exhip_ctx* ctx, const int8_t* w, const float* ws, float* wf, int k, int per_group);
 
 /* operation_pooling::forward_cpu_f32 (src/Excalibur/operation_pooling.cpp:80-208). type 0 max, 1 average.
@@ -246,6 +266,17 @@ int exhip_pool_out_hw(int h, int w, int kh, int kw, int sh, int sw, int pt, int 
 int exhip_pool2d_nchw_f32(exhip_ctx* ctx, const float* x, float* y, int n, int c, int h, int w, int oh, int ow,
                           int type, int kh, int kw, int sh, int sw, int pt, int pb, int pl, int pr,
                           int count_include_pad);
+/* The same on NHWC f32 tensors, which may be slices of wider ones (x_stride, y_stride: their channel strides, multiples of 4). */
+int exhip_pool2d_nhwc_f32(exhip_ctx* ctx, const float* x, int x_stride, float* y, int y_stride, int n, int c, int h, int w, int oh, int ow,
+                          int type, int kh, int kw, int sh, int sw, int pt, int pb, int pl, int pr, int count_include_pad);
+/* Nearest Interp (operation_interp.cpp:247-268) on such tensors. */
+int exhip_interp_nearest_nhwc_f32(exhip_ctx* ctx, const float* x, int x_stride, float* y, int y_stride, int n, int c, int h, int w, int oh,
+                                  int ow);
+/* What stands in front of a float network's first convolution: the Input layer (operation_input.cpp:61-151) with host arrays of c
+ * means and scales, YoloV5Focus (operation_yolov5focus.cpp) if focus != 0, and NHWC: c_stride 4 for c <= 4, 16 for the twelve
+ * channels of the focus. EXHIP_ERR_UNSUPPORTED for other shapes. */
+int exhip_input_nchw_f32_to_nhwc_f32(exhip_ctx* ctx, const float* x, int n, int c, int h, int w, const float* means, const float* scales,
+                                     int focus, int c_stride, float* y);
 /* NHWC variants used between fused layers. The int8 one exists because max commutes with the
  * (monotone) quantizer; the f32 one can also emit the requantized int8 copy (y_i8 may be NULL). */
 int exhip_maxpool2d_nhwc_f32(exhip_ctx* ctx, const float* x, float* y, int8_t* y_i8, float fs_out, int n, int c,

@@ -1,0 +1,116 @@
+"""The float32 plan (pipeline.cpp, build_float_plan): NHWC tensors between the layers, Concats written in place, layers folded
+into the convolutions around them. Every blob it gives equals the per-layer executor's bit for bit."""
+import os
+import tempfile
+
+import numpy as np
+import pytest
+
+from excalibur_amd import modelfile as mf
+from excalibur_amd import pipeline as xp
+
+pytestmark = pytest.mark.gpu
+
+
+def network(focus):
+    r = np.random.default_rng(71)
+    lines, blobs = ["Input data 0 1 data 0=32 1=32 2=3 3=3,2,1 4=0.5"], []
+
+    def conv(bottom, top, cin, k, kernel=1, stride=1, groups=1, act=0):
+        w = r.normal(0, np.sqrt(2.0 / (cin // groups * kernel * kernel)), (k, cin // groups, kernel, kernel)).astype(np.float32)
+        kind = "Convolution" if groups == 1 else "ConvolutionDepthWise"
+        lines.append(mf.conv_line(kind, top + "_l", bottom, top, k, kernel, stride, kernel // 2, True, w.size, groups, act=act))
+        blobs.append(mf.conv_blob_f32(w, r.normal(0, 0.5, (k,)).astype(np.float32)))
+
+    def batchnorm(bottom, top, c):
+        lines.append(f"BatchNorm {top}_l 1 1 {bottom} {top} 0={c}")
+        blobs.append(b"".join(mf.floats_blob(v.astype(np.float32)) for v in (r.normal(1, .2, c), r.normal(0, .5, c), r.uniform(.5, 2, c), r.normal(0, .5, c))))
+
+    def prelu(bottom, top, c):
+        lines.append(f"PReLU {top}_l 1 1 {bottom} {top} 0={c}")
+        blobs.append(mf.floats_blob(r.uniform(-.5, .5, max(1, c)).astype(np.float32)))
+
+    def split(bottom, n):
+        lines.append(f"Split {bottom}_sp 1 {n} {bottom} " + " ".join(f"{bottom}{j}" for j in range(n)))
+
+    def add(kind, bottoms, top, params=""):
+        lines.append(f"{kind} {top}_l {len(bottoms)} 1 {' '.join(bottoms)} {top} {params}")
+
+    if focus:
+        add("YoloV5Focus", ["data"], "front")
+        conv("front", "c0", 12, 24, 3)
+    else:
+        conv("data", "c0", 3, 24, 3, 2)
+    prelu("c0", "p0", 24)
+    conv("p0", "d1", 24, 24, 3, 1, groups=24)           # depthwise + PReLU, shared slope
+    prelu("d1", "p1", 1)
+    conv("p1", "d2", 24, 24, 3, 2, groups=24)           # depthwise + ReLU, stride 2
+    add("ReLU", ["d2"], "r2")
+    split("r2", 3)
+    conv("r20", "c3", 24, 20)                            # 20 channels: pad channels travel with the tensor
+    add("HardSwish", ["c3"], "a3", "0=1.666667e-01 1=5.000000e-01")
+    conv("a3", "c4", 20, 24, 3)
+    add("Eltwise", ["r21", "c4"], "s4", "0=1")           # sum behind a plain convolution, ReLU behind the sum
+    add("ReLU", ["s4"], "s4r")
+    split("s4r", 4)
+    conv("s4r0", "y1", 24, 16)                           # Concat -> BatchNorm -> LeakyRelu in two plain producers
+    conv("r22", "y2", 24, 32)
+    add("Concat", ["y1", "y2"], "cat", "0=-1")
+    batchnorm("cat", "catbn", 48)
+    add("LeakyRelu", ["catbn"], "cata", "0=1.000000e-01")
+    conv("cata", "c5", 48, 32, act=1)
+    split("c5", 3)
+    for j, k in enumerate((5, 9)):                       # pools of a pool, written into a Concat beside their input's copy
+        add("Pooling", ["c50" if j else "c51"], f"mp{k}", f"0=0 1={k} 11={k} 2=1 12=1 3={k // 2} 13={k // 2} 14={k // 2} 15={k // 2} 5=1 4=0")
+    add("Concat", ["c52", "mp5", "mp9"], "spp", "0=-1")
+    conv("spp", "c6", 96, 24, 3, 2)
+    split("c6", 2)
+    add("Interp", ["c60"], "up", "0=1 1=2.000000e+00 2=2.000000e+00")
+    conv("s4r1", "lat", 24, 24)
+    add("BinaryOp", ["up", "lat"], "fpn", "0=0")         # the upsampled map is read through by the sum
+    add("Interp", ["c61"], "up2", "0=1 1=2.000000e+00 2=2.000000e+00")
+    add("Pooling", ["s4r2"], "av", "0=1 1=3 11=3 2=1 12=1 3=1 13=1 14=1 15=1 5=1 4=0 6=1")
+    add("Concat", ["fpn", "up2", "av"], "wide", "0=-1")  # nothing plain about its producers: BatchNorm as a pass over it
+    batchnorm("wide", "widebn", 72)
+    split("widebn", 3)
+    conv("widebn0", "c7", 72, 42, 1)                     # a head: [n][3 x 14] -> [n][3][pixels][14]
+    add("Reshape", ["c7"], "hr", "0=64 1=14 2=3")
+    add("Transpose", ["hr"], "head", "0=1,0,2")
+    wd = r.normal(0, .2, (72, 8, 2, 2)).astype(np.float32)
+    lines.append(f"Deconvolution dc1 1 1 widebn1 dc 0=8 1=2 11=2 2=1 12=1 3=2 13=2 4=0 14=0 15=0 16=0 5=1 6={wd.size} 7=1")
+    blobs.append(mf.conv_blob_f32(wd, r.normal(0, .5, (8,)).astype(np.float32)))
+    batchnorm("dc", "dcbn", 8)
+    add("ReLU", ["dcbn"], "dcr")
+    w1 = r.normal(0, .5, (8, 1, 2, 2)).astype(np.float32)
+    lines.append(f"Deconvolution dc2 1 1 dcr dm 0=1 1=2 11=2 2=1 12=1 3=2 13=2 4=0 14=0 15=0 16=0 5=1 6={w1.size} 7=1")
+    blobs.append(mf.conv_blob_f32(w1, r.normal(0, .5, (1,)).astype(np.float32)))
+    add("Sigmoid", ["dm"], "map")
+    lines.append(mf.pool_line("gap", "widebn2", "gap", 1, global_pool=True))
+    wf = r.normal(0, .2, (10, 72)).astype(np.float32)
+    lines.append(f"InnerProduct fc 1 1 gap fc 0=10 1=1 2={wf.size}")
+    blobs.append(mf.fc_blob_f32(wf, r.normal(0, .5, (10,)).astype(np.float32)))
+    return lines, blobs, ["head", "map", "fc", "s4r3"]
+
+
+@pytest.mark.parametrize("focus", [False, True])
+def test_float_plan_equals_the_layers_bit_for_bit(focus):
+    lines, blobs, outs = network(focus)
+    with tempfile.NamedTemporaryFile(suffix=".racy", delete=False) as f:
+        path = f.name
+    mf.write_model(path, blobs)
+    planned, plain = (xp.Pipeline(mf.topology(lines, "float"), path, 0, fusion=on) for on in (True, False))
+    try:
+        for n, seed in ((1, 1), (3, 2), (3, 3)):
+            x = np.random.default_rng(seed).uniform(-4, 4, (n, 3, 32, 32)).astype(np.float32)
+            planned.forward(x)
+            plain.forward(x)
+            assert planned.stored("head") and not planned.stored("c0") and plain.stored("c0")
+            for o in outs:
+                got, want = planned.get(o), plain.get(o)
+                assert np.isfinite(want).all() and np.ptp(want) > 0
+                assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (o, n)
+            assert np.array_equal(planned.get("spp"), plain.get("spp"))  # a blob the plan never made: by the rerun
+    finally:
+        planned.close()
+        plain.close()
+        os.unlink(path)
