@@ -532,19 +532,23 @@ int exhip_conv_f32_pack_weights(const exhip_conv_desc* d, const float* w, float*
     if (rc) return rc;
     const bool pair = d->c_stride == 4;
     const int C = d->c, K = d->k, KH = d->kh, KW = d->kw, csteps = pair ? 1 : (C + 7) / 8;
-    for (int kb = 0; kb < (K + 31) / 32; ++kb)
-        for (int r = 0; r < KH; ++r)
-            for (int q0 = 0; q0 < KW; q0 += pair ? 2 : 1)
-                for (int j = 0; j < csteps; ++j)
-                    for (int lane = 0; lane < 64; ++lane) {
-                        const int rr = lane % 32, h = lane / 32;
-                        const int k = kb * 32 + ((rr / 4) % 2) * 16 + (rr / 8) * 4 + rr % 4;
-                        const int q = pair ? q0 + h : q0;
-                        for (int e = 0; e < 4; ++e) {
-                            const int c = pair ? e : j * 8 + h * 4 + e;
-                            *out++ = k < K && c < C && q < KW ? w[(((size_t)k * C + c) * KH + r) * KW + q] : 0.f;
+    const int taps_w = pair ? (KW + 1) / 2 : KW;
+    const size_t tap_step = (size_t)csteps * 256;  // floats between a lane's vectors of neighbouring taps
+    for (int kb = 0; kb < (K + 31) / 32; ++kb, out += KH * taps_w * tap_step)
+        for (int j = 0; j < csteps; ++j)
+            for (int lane = 0; lane < 64; ++lane) {
+                const int rr = lane % 32, h = lane / 32;
+                const int k = kb * 32 + ((rr / 4) % 2) * 16 + (rr / 8) * 4 + rr % 4;
+                const int c = pair ? 0 : j * 8 + h * 4, n = k < K ? std::max(0, std::min(4, C - c)) : 0;
+                float* const o = out + (j * 64 + lane) * 4;
+                const float* const src = n ? w + ((size_t)k * C + c) * KH * KW : w;
+                for (int e = 0; e < 4; ++e)  // a channel's taps lie side by side in the OIHW weights
+                    for (int r = 0; r < KH; ++r)
+                        for (int q = 0; q < taps_w; ++q) {
+                            const int tap = pair ? 2 * q + h : q;
+                            o[(r * taps_w + q) * tap_step + e] = e < n && tap < KW ? src[(e * KH + r) * KW + tap] : 0.f;
                         }
-                    }
+            }
     return 0;
 }
 
