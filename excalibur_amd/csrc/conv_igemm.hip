@@ -1721,7 +1721,8 @@ int run_conv(exhip_ctx* ctx, const exhip_conv_desc* d, ConvParams p, const PoolS
         // split keeps more CUs busy). EXHIP_ERR_UNSUPPORTED leaves the layer to this kernel.
         const int min_chunks_ = (3 + pl.n_rg - 1) / pl.n_rg;
         const bool would_split = g_exhip_options.force_splits != 1 && pl.n_chunks / min_chunks_ >= 2 && kCUs / tiles >= 2;
-        if ((tiles >= 16 || !would_split) && g_exhip_options.force_splits <= 1) {
+        const bool deep = !pl.packed && exhip_pw_splits_f16((long long)d->n * pl.OH * pl.OW, d->k, d->k_stride, pl.n_chunks * d->kh * d->kw * (pl.chunk_b / 32));
+        if ((tiles >= 16 || !would_split) && g_exhip_options.force_splits <= 1 && !deep) {
             if (!pl.packed && !pool && d->kh == 3 && d->kw == 3 && d->sh == 1 && d->sw == 1 && pl.variant == 0 && pl.chunk_b == 64 &&
                 pl.RS == 1 && p.cstride_b % 64 == 0 && d->k % 64 == 0 && d->k_stride == d->k && d->act <= 1 && p.y_q && !p.y_nchw_h && !p.y_nchw &&
                 d->post_op != EXHIP_POST_PRELU) {

@@ -36,6 +36,7 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 constexpr unsigned kRsrcWord3 = 0x00020000u;  // raw buffer: out-of-range loads return 0
 constexpr int kOutOfRange = 0x7ffff000;       // a lane offset beyond every view
 constexpr int kMaxDirectSteps = 40;           // k-steps of a layer with a filter (taps x 32-byte steps per pixel)
+constexpr int kSplit = 4;                     // waves that share a tile's k-steps in the split form
 constexpr int kTapShift = 27;                 // a step's table entry: byte offset below, tap number above
 
 struct PwParams {
@@ -67,7 +68,12 @@ struct PwParams {
     // the form with a filter (TAPS): output pixel (img, oy, ox) reads input pixel (oy * stride - pt + r, ox * stride - pl + q)
     // for k-step s of tap r * kw + q, that many bytes behind its top-left input pixel
     int in_h, in_w, out_h, out_w, stride, pad_t, pad_l, kh, kw;
-    int step[kMaxDirectSteps];   // offset | tap << kTapShift
+    int step[kMaxDirectSteps];   // offset | tap << kTapShift (not used by the split form)
+    // the split form: where each wave of a tile begins in that order -- its first k-step, bytes behind the top-left input pixel,
+    // filter row, tap and bytes left of the chunk -- and what leads from behind a row's last tap to the next row, and from
+    // behind the last row to the next chunk
+    int start_s[kSplit + 1], start_b[kSplit + 1], start_r[kSplit + 1], start_q[kSplit + 1], start_left[kSplit + 1];
+    int chunk_b, row_end_b, chunk_end_b;
 };
 
 __device__ __noinline__ float slow_activation(float v, int act) { return exhip_act(v, act); }
@@ -427,9 +433,175 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
     pw_epilogue<DT, MT, NT, EP>(p, acc, tile * NT * 32, kb0, lane, lds);
 }
 
+// The split form, for launches of few tiles and many k-steps (one image, deep layers), where the kernel above is as long as one
+// wave's chain: 0.17 us a k-step, 16 us for 256 -> 256 3x3 int8 on a 20 x 20 map. WK waves share a tile of 32 pixels x 32 * MT
+// channels: each takes its run of the k-steps, the sums meet in LDS (exactly for int8; in a fixed order, so the same bits
+// every time, for fp16), wave m finishes block m. Every request in the loop is unconditional, so that the waits count what is in
+// flight; those past a wave's run ask for operands it does not use.
+template <int DT, int MT, int WK, bool TAPS, typename EP>
+__global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParams p) {
+    constexpr int R = 8;  // k-steps in flight
+    constexpr int RED = WK * MT * 4096;
+    static_assert(MT <= WK && WK <= kSplit, "a wave per block");
+    __shared__ __attribute__((aligned(16))) char lds_all[RED + MT * wave_bytes(DT, 1)];
+    const int lane = threadIdx.x & 63, part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    unsigned item = blockIdx.x;
+    {
+        const unsigned per = gridDim.x >> 3;
+        if (item < (per << 3)) item = (item & 7) * per + (item >> 3);
+    }
+    const unsigned tile = __builtin_amdgcn_readfirstlane(exhip_divide(item, p.ch_groups, p.groups_magic, p.groups_shift));
+    const int kb0 = __builtin_amdgcn_readfirstlane((int)(item - tile * p.ch_groups) * MT);
+    char* const lds = lds_all + RED + (part < MT ? part : 0) * wave_bytes(DT, 1);
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.x), 0, (int)p.x_bytes, kRsrcWord3);
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.wp), 0, (int)p.w_bytes, kRsrcWord3);
+
+    const unsigned pix = tile * 32 + (lane & 31);
+    int xoff, iy = 0, ix = 0;
+    if constexpr (TAPS) {
+        const unsigned per_image = (unsigned)(p.out_h * p.out_w);
+        const unsigned img = exhip_divide(pix, per_image, p.image_magic, p.image_shift), rem = pix - img * per_image;
+        const int oy = (int)exhip_divide(rem, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = (int)(rem - (unsigned)oy * (unsigned)p.out_w);
+        iy = oy * p.stride - p.pad_t;
+        ix = ox * p.stride - p.pad_l;
+        xoff = (((int)img * p.in_h + iy) * p.in_w + ix) * p.xs_b + (lane >> 5) * 16;
+        if (pix >= p.pixels) iy = -0x40000000;
+    } else {
+        xoff = pix < p.pixels ? (int)(pix * (unsigned)p.xs_b) + (lane >> 5) * 16 : kOutOfRange;
+    }
+    const int s_first = p.start_s[part], steps = p.start_s[part + 1] - s_first, s_last = p.n_ksteps - 1;
+    const int w_step = p.mts * 1024, slab = kb0 >> (p.mts >> 1);
+    const int w_base = (slab * p.n_ksteps * p.mts + (kb0 & (p.mts - 1))) * 1024;
+    int s_at = s_first, b_at = p.start_b[part], r_at = p.start_r[part], q_at = p.start_q[part], left = p.start_left[part];
+    int xcur = xoff;
+    auto enter_tap = [&]() {  // the lane's offset at the tap, out of range outside the image
+        const bool in = (unsigned)(iy + r_at) < (unsigned)p.in_h && (unsigned)(ix + q_at) < (unsigned)p.in_w;
+        xcur = in ? xoff + b_at : kOutOfRange;
+    };
+    if constexpr (TAPS) enter_tap();
+
+    typedef typename std::conditional<DT == EXHIP_I8, v16i, v16f>::type acc_t;
+    acc_t acc[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[m][e] = 0;
+    v4i a[R][MT], b[R];
+    auto request = [&](int u) {
+        const int s_in = s_at < s_last ? s_at : s_last;
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+            a[u][m] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, lane * 16 + m * 1024, w_base + s_in * w_step, 0));
+        b[u] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(xr, xcur, TAPS ? 0 : s_in * 32, 0));
+        ++s_at;
+        if constexpr (TAPS) {
+            b_at += 32;
+            left -= 32;
+            if (left == 0) {  // the next tap (no memory accesses under the branch)
+                left = p.chunk_b;
+                b_at += p.xs_b - p.chunk_b;
+                if (++q_at == p.kw) {
+                    q_at = 0;
+                    b_at += p.row_end_b;
+                    if (++r_at == p.kh) {
+                        r_at = 0;
+                        b_at += p.chunk_end_b;
+                    }
+                }
+                enter_tap();
+            } else {
+                xcur += xcur == kOutOfRange ? 0 : 32;
+            }
+        }
+    };
+    auto step = [&](int u) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            if constexpr (DT == EXHIP_I8) acc[m] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[u][m], b[u], acc[m], 0, 0, 0);
+            else acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a[u][m]), __builtin_bit_cast(v8h, b[u]), acc[m], 0, 0, 0);
+        }
+    };
+    float par[kParams] = {};
+    auto load_parameters = [&]() {  // of the block this wave will finish: lane = channel
+        const int at = lane < 32 ? ((kb0 + part) * 32 + lane) * 4 : kOutOfRange;
+        auto load = [&](const float* src, int offset, int count) {
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src), 0, src ? count * 4 : 0, kRsrcWord3);
+            return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, offset, 0, 0));
+        };
+        if constexpr (DT == EXHIP_I8) par[0] = load(p.scale, at, p.K);
+        par[1] = load(p.bias, at, p.K);
+        if (EP::any || EP::post == kPostPrelu) par[2] = load(p.post_slope, p.post_slope_shared ? 0 : at, p.post_slope_shared ? 1 : p.K);
+        if (DT == EXHIP_I8 && (EP::any ? p.post_bn_a != nullptr : EP::bn)) {
+            par[2] = load(p.post_bn_a, at, p.K);
+            par[3] = load(p.post_bn_b, at, p.K);
+        }
+    };
+    if (steps > R) {
+#pragma unroll
+        for (int u = 0; u < R; ++u) request(u);
+        int k = 0;
+        for (; k + R < steps; k += R) {
+#pragma unroll
+            for (int u = 0; u < R; ++u) {
+                step(u);
+                request(u);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (part < MT) load_parameters();
+#pragma unroll
+        for (int u = 0; u < R; ++u)
+            if (k + u < steps) step(u);
+    } else {
+#pragma unroll
+        for (int u = 0; u < R; ++u)
+            if (u < steps) request(u);
+        if (part < MT) load_parameters();
+#pragma unroll
+        for (int u = 0; u < R; ++u)
+            if (u < steps) step(u);
+    }
+    // the waves' sums: 16 words a lane and block, 16 bytes side by side per lane
+    auto word4 = [](const acc_t& c, int q) {
+        if constexpr (DT == EXHIP_I8) return v4i{c[q * 4], c[q * 4 + 1], c[q * 4 + 2], c[q * 4 + 3]};
+        else return __builtin_bit_cast(v4i, v4f{c[q * 4], c[q * 4 + 1], c[q * 4 + 2], c[q * 4 + 3]});
+    };
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        if (m == part) continue;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) *reinterpret_cast<v4i*>(lds_all + (part * MT + m) * 4096 + q * 1024 + lane * 16) = word4(acc[m], q);
+    }
+    __syncthreads();
+    if (part >= MT) return;
+    if (lane < 32) {
+#pragma unroll
+        for (int i = 0; i < kParams; ++i) *reinterpret_cast<float*>(lds + (i * 32 + lane) * 4) = par[i];
+    }
+    acc_t sum[1][1];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+        if (m == part) sum[0][0] = acc[m];
+    for (int w = 0; w < WK; ++w) {
+        if (w == part) continue;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const v4i t = *reinterpret_cast<const v4i*>(lds_all + (w * MT + part) * 4096 + q * 1024 + lane * 16);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if constexpr (DT == EXHIP_I8) sum[0][0][q * 4 + e] += t[e];
+                else sum[0][0][q * 4 + e] += __builtin_bit_cast(v4f, t)[e];
+            }
+        }
+    }
+    pw_epilogue<DT, 1, 1, EP>(p, sum, tile * 32, kb0 + part, lane, lds);
+}
+
+// U < 0: the split form with -U waves to a tile
 template <int DT, int MT, int NT, int U, bool TAPS, typename EP>
 int go(exhip_ctx* ctx, const PwParams& p) {
-    hipLaunchKernelGGL((conv1x1_pw_kernel<DT, MT, NT, U, TAPS, EP>), dim3((p.items + 3) / 4), dim3(256), 0, ctx->stream, p);
+    if constexpr (U < 0) hipLaunchKernelGGL((conv_pw_split_kernel<DT, MT, -U, TAPS, EP>), dim3(p.items), dim3(64 * -U), 0, ctx->stream, p);
+    else hipLaunchKernelGGL((conv1x1_pw_kernel<DT, MT, NT, U, TAPS, EP>), dim3((p.items + 3) / 4), dim3(256), 0, ctx->stream, p);
     EXHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -465,6 +637,19 @@ int pick_epilogue(exhip_ctx* ctx, const PwParams& p) {
     return go<DT, MT, NT, U == 8 ? 4 : U, TAPS, EpAny>(ctx, p);
 }
 
+// Whether a launch takes the split form: few enough wave tiles that their chains, not their sum, set the time, and k-steps enough
+// to share. Measured on the layers of yolov5s_simp at 1, 2, 4, 8 and 16 images (us, unsplit -> split): int8 256 -> 512 3x3 stride 2
+// from 40 x 40 at one image 24.5 -> 6.8, 128 -> 128 3x3 at 40 x 40 9.5 -> 5.5, 1024 -> 512 at 20 x 20 8.4 -> 4.6, fp16 13.1 -> 5.5. The
+// lines: up to 800 blocks of 32 pixels x 32 channels from 8 k-steps on (128 -> 128 3x3 int8 at 800 blocks 9.7 -> 8.3, at 1600
+// 10.0 -> 13.2; four k-steps gain nothing); int8 layers with a filter and 64 k-steps, which otherwise run the staged kernel, up to
+// 1600 (26.7 -> 18.6; 3200: 30.4 -> 29.7). A lone 32-channel block would leave half of every tile unused.
+bool split_wins(int dt, bool taps, long long pixels, int kblocks, int n_ksteps) {
+    if (g_exhip_options.force_splits == 1 || g_exhip_options.pw_split == 0 || kblocks < 2) return false;
+    if (g_exhip_options.pw_split == 2) return true;
+    const long long blocks = (pixels + 31) / 32 * kblocks;
+    return n_ksteps >= 8 && blocks <= (dt == EXHIP_I8 && taps && n_ksteps >= 64 ? 1664 : 832);
+}
+
 template <int DT, int MT, int NT, bool TAPS = false>
 int launch(exhip_ctx* ctx, PwParams& p, int kblocks) {
     const long long tiles = ((long long)p.pixels + 32 * NT - 1) / (32 * NT);
@@ -478,6 +663,28 @@ int launch(exhip_ctx* ctx, PwParams& p, int kblocks) {
     // where there are more than eight. Larger ones hide each other's round trips and want the registers for more waves.
     else if (MT == 2 && items <= 2048 && p.n_ksteps > 8) return pick_epilogue<DT, MT, NT, 8, TAPS>(ctx, p);
     else return pick_epilogue<DT, MT, NT, 4, TAPS>(ctx, p);
+}
+
+template <int DT, bool TAPS>
+int launch_split(exhip_ctx* ctx, PwParams& p, int kblocks) {
+    p.ch_groups = (unsigned)((kblocks + 1) / 2);
+    const long long items = ((long long)p.pixels + 31) / 32 * p.ch_groups;
+    if (items >= (1ll << 31) - 4) return EXHIP_ERR_UNSUPPORTED;
+    p.items = (unsigned)items;
+    exhip_host_divisor(p.ch_groups, &p.groups_magic, &p.groups_shift);
+    for (int i = 0; i <= kSplit; ++i) {
+        const int s = (int)((long long)p.n_ksteps * i / kSplit);
+        p.start_s[i] = s;
+        if (TAPS) {
+            const int per_tap = p.chunk_b / 32, per_row = p.kw * per_tap, per_chunk = p.kh * per_row;
+            const int chunk = s / per_chunk, in_chunk = s % per_chunk, row = in_chunk / per_row, tap = in_chunk % per_row / per_tap, j = in_chunk % per_tap;
+            p.start_r[i] = row;
+            p.start_q[i] = tap;
+            p.start_b[i] = (row * p.in_w + tap) * p.xs_b + chunk * p.chunk_b + j * 32;
+            p.start_left[i] = p.chunk_b - j * 32;
+        }
+    }
+    return pick_epilogue<DT, 2, 1, -kSplit, TAPS>(ctx, p);
 }
 
 }  // namespace
@@ -499,7 +706,7 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
     if (g.post_bn_a || g.post_bn_b || g.exact_k) return EXHIP_ERR_UNSUPPORTED;
     const long long n_ksteps = (long long)t.n_chunks * t.kh * t.kw * (t.chunk_b / 32);
     if (g.pixels <= 0 || g.c_bytes <= 0 || g.c_bytes % 32 != 0 || t.chunk_b % 32 != 0 || t.n_chunks * t.chunk_b != g.c_bytes ||
-        (g.slab_blocks != 2 && g.slab_blocks != 4) || g.k_stride % 8 != 0 || n_ksteps > kMaxDirectSteps || t.kh * t.kw > (1 << (32 - kTapShift)) || t.stride < 1 || t.pad_t < 0 || t.pad_l < 0)
+        (g.slab_blocks != 2 && g.slab_blocks != 4) || g.k_stride % 8 != 0 || (n_ksteps > kMaxDirectSteps && !split_wins(DT, true, g.pixels, (std::max(g.k, g.k_stride) + 31) / 32, (int)n_ksteps)) || t.kh * t.kw > (1 << (32 - kTapShift)) || t.stride < 1 || t.pad_t < 0 || t.pad_l < 0)
         return EXHIP_ERR_UNSUPPORTED;
     const long long x_bytes = (long long)t.n * t.in_h * t.in_w * g.c_bytes;
     const long long w_bytes = (long long)g.slabs * n_ksteps * g.slab_blocks * 1024;
@@ -515,10 +722,11 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
     // and 1.83 -> 1.81 ms per forward of the detection networks); of the int8 layers only a few deep ones are (3x3
     // stride 2 from 40 x 40: 29 -> 23 us) while the wide first layers lose (12 -> 32 channels at 320 x 320: 81 -> 94 us),
     // so int8 layers stay with the staged kernels unless the option asks.
-    // A lone 32-channel block (its 128-pixel tile with the tap bookkeeping fills the register file) never wins: 12 -> 32
-    // at 16 x 320 x 320 78 against 80 us, 16 -> 32 stride 2 at 224 x 224 11.5 against 9 us in either data type.
-    const bool take = kblocks > 1 && (DT == EXHIP_F16 || g.c_bytes == 32 || (g.pixels <= 32768 && kblocks <= 4) || g.pixels <= 6400);
-    if (g_exhip_options.direct != 2 && !take) return EXHIP_ERR_UNSUPPORTED;
+    // A lone 32-channel block wins whatever its size (12 -> 32 at 16 x 320 x 320: int8 71 -> 46 us, fp16 66 -> 45; 32 -> 32 at
+    // 160 x 160: one image 8.1 -> 5.3 us, sixteen 24.9 -> 15.8).
+    const bool take = kblocks == 1 || DT == EXHIP_F16 || g.c_bytes == 32 || (g.pixels <= 32768 && kblocks <= 4) || g.pixels <= 6400;
+    const bool split = split_wins(DT, true, g.pixels, kblocks, (int)n_ksteps);
+    if (g_exhip_options.direct != 2 && !take && !split) return EXHIP_ERR_UNSUPPORTED;
     p.post_slope = g.post_slope;
     p.pixels = (unsigned)g.pixels; p.x_bytes = (unsigned)x_bytes; p.w_bytes = (unsigned)w_bytes;
     p.xs_b = g.c_bytes; p.n_ksteps = (int)n_ksteps; p.mts = g.slab_blocks;
@@ -530,6 +738,10 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
     p.kh = t.kh; p.kw = t.kw;
     exhip_host_divisor((unsigned)(t.out_h * t.out_w), &p.image_magic, &p.image_shift);
     exhip_host_divisor((unsigned)t.out_w, &p.width_magic, &p.width_shift);
+    p.chunk_b = t.chunk_b;
+    p.row_end_b = (t.in_w - t.kw) * g.c_bytes;
+    p.chunk_end_b = t.chunk_b - t.kh * t.in_w * g.c_bytes;
+    if (split) return launch_split<DT, true>(ctx, p, kblocks);
     int s = 0;
     for (int cc = 0; cc < t.n_chunks; ++cc)
         for (int r = 0; r < t.kh; ++r)
@@ -591,6 +803,7 @@ int run_pw(exhip_ctx* ctx, const exhip_pw_geom& g, PwParams& p, int es, bool has
     const int kblocks = std::min(g.slabs * g.slab_blocks, (out_channels + 31) / 32);
     // 64 x 64 per wave unless that leaves SIMDs without a wave: then 64 channels x 32 pixels; a lone 32-channel block
     // takes 128 pixels per wave
+    if (split_wins(DT, false, g.pixels, kblocks, (int)n_ksteps)) return launch_split<DT, false>(ctx, p, kblocks);
     if (kblocks == 1) return launch<DT, 1, 2>(ctx, p, kblocks);
     const long long waves64 = ((g.pixels + 63) / 64) * ((kblocks + 1) / 2);
     if (waves64 < 2048 || small_tile<DT>()) return launch<DT, 2, 1>(ctx, p, kblocks);
@@ -614,4 +827,8 @@ int exhip_conv1x1_i8_pw(exhip_ctx* ctx, const exhip_pw_geom& g, const int8_t* x,
     p.residual_f = residual; p.y_f = y_f32; p.y_q = y_i8; p.fs_out = g.fs_out;
     p.post_bn_a = g.post_bn_a; p.post_bn_b = g.post_bn_b; p.exact = g.exact_k;
     return run_pw<EXHIP_I8>(ctx, g, p, 1, residual != nullptr, taps);
+}
+
+bool exhip_pw_splits_f16(long long pixels, int k, int k_stride, int n_ksteps) {
+    return g_exhip_options.pw != 0 && g_exhip_options.direct != 0 && split_wins(EXHIP_F16, true, pixels, (std::max(k, k_stride) + 31) / 32, n_ksteps);
 }

@@ -62,7 +62,8 @@ const char* exhip_last_error(void);
  * layers (0 = the general kernel), "pw" the fp16 / int8 kernel without staging for pointwise layers and "direct" its
  * form for layers with a filter (1 where it measured faster, 2 wherever it can run, 0 never), "pw_tile" that kernel's wave
  * tile (0 = 32 pixels x 64 channels, 2 = 64 x 64 for large launches), "stem" the one-kernel stem: every form computes
- * the same values. "f32_tile" pins the float32 convolution's wave tile and split (0 = its rule).
+ * the same values. "pw_split" chooses that kernel's split form (1 by its rule, 2 wherever it can run, 0 never; fp16 sums then run
+ * in another order). "f32_tile" pins the float32 convolution's wave tile and split (0 = its rule).
  * Process-wide; packed weights depend on the first three, so set them before packing. */
 int exhip_set_option(const char* name, int value);
 int exhip_device_name(exhip_ctx* ctx, char* buf, size_t len);
