@@ -279,6 +279,93 @@ extern "C" int exhip_memcpy_h2d(exhip_ctx* ctx, void* dst, const void* src, size
     return 0;
 }
 
+extern "C" int exhip_mark(exhip_ctx* ctx, void** mark) {
+    EXHIP_REQUIRE(ctx && mark, "exhip_mark: NULL argument");
+    if (!*mark) {
+        hipEvent_t e;
+        EXHIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        *mark = (void*)e;
+    }
+    EXHIP_CHECK(hipEventRecord((hipEvent_t)*mark, ctx->stream));
+    return 0;
+}
+
+extern "C" int exhip_mark_destroy(void* mark) {
+    if (mark) EXHIP_CHECK(hipEventDestroy((hipEvent_t)mark));
+    return 0;
+}
+
+// Everything but small results: through pinned chunks, or straight into a pinned block.
+static int download(exhip_ctx* ctx, hipStream_t stream, void* dst, const void* src, size_t bytes) {
+    exhip_staging& s = ctx->down;
+    auto chunk = [&](int i) {
+        if (!s.chunk[i]) s.chunk[i] = take_chunk();
+        return static_cast<char*>(s.chunk[i]);
+    };
+    if (is_result_block(dst, bytes) || bytes <= kUploadKernel || !chunk(0) || !chunk(1)) {
+        EXHIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream));
+        EXHIP_CHECK(hipStreamSynchronize(stream));
+        return 0;
+    }
+    int chunks = 2;
+    while (chunks < exhip_staging::kChunks && (size_t)chunks * kChunk < bytes && chunk(chunks)) ++chunks;
+    for (int i = 0; i < chunks; ++i)
+        if (!s.event[i]) {
+            hipEvent_t e;
+            EXHIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+            s.event[i] = e;
+        }
+    copy_crew::session crew(bytes >= 4 * kPiece);
+    const size_t total = (bytes + kChunk - 1) / kChunk;
+    auto request = [&](size_t i) -> int {
+        const size_t o = i * kChunk, n = bytes - o < kChunk ? bytes - o : kChunk;
+        EXHIP_CHECK(hipMemcpyAsync(s.chunk[i % chunks], static_cast<const char*>(src) + o, n, hipMemcpyDeviceToHost, stream));
+        EXHIP_CHECK(hipEventRecord((hipEvent_t)s.event[i % chunks], stream));
+        return 0;
+    };
+    for (size_t i = 0; i < total && i < (size_t)chunks; ++i)
+        if (const int rc = request(i)) return rc;
+    for (size_t i = 0; i < total; ++i) {
+        const size_t o = i * kChunk, n = bytes - o < kChunk ? bytes - o : kChunk;
+        EXHIP_CHECK(hipEventSynchronize((hipEvent_t)s.event[i % chunks]));
+        crew.copy(static_cast<char*>(dst) + o, s.chunk[i % chunks], n);
+        if (i + chunks < total)
+            if (const int rc = request(i + chunks)) return rc;
+    }
+    return 0;
+}
+
+
+// Streams for copies beside a context's own, cached for the process: one per copy in flight, kept until it ends.
+namespace {
+std::mutex g_side_mu;
+std::map<int, std::vector<hipStream_t>> g_side;  // idle streams by device
+}  // namespace
+
+extern "C" int exhip_memcpy_d2h_from(exhip_ctx* ctx, void* mark, void* dst, const void* src, size_t bytes) {
+    EXHIP_REQUIRE(ctx && mark && ((dst && src) || !bytes), "exhip_memcpy_d2h_from: NULL argument");
+    if (!bytes) return 0;
+    hipStream_t side = nullptr;
+    {
+        std::lock_guard<std::mutex> g(g_side_mu);
+        auto& idle = g_side[ctx->device];
+        if (!idle.empty()) {
+            side = idle.back();
+            idle.pop_back();
+        }
+    }
+    if (!side) {
+        EXHIP_CHECK(hipSetDevice(ctx->device));
+        EXHIP_CHECK(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
+    }
+    int rc = (int)hipStreamWaitEvent(side, (hipEvent_t)mark, 0);
+    if (rc == 0) rc = download(ctx, side, dst, src, bytes);
+    else exhip_set_error("exhip_memcpy_d2h_from: hipStreamWaitEvent failed: %s", hipGetErrorString((hipError_t)rc));
+    std::lock_guard<std::mutex> g(g_side_mu);
+    g_side[ctx->device].push_back(side);  // download() has waited for it
+    return rc;
+}
+
 extern "C" int exhip_memcpy_d2h(exhip_ctx* ctx, void* dst, const void* src, size_t bytes) {
     EXHIP_REQUIRE(ctx && ((dst && src) || !bytes), "exhip_memcpy_d2h: NULL argument");
     if (!bytes) return 0;
@@ -306,37 +393,7 @@ extern "C" int exhip_memcpy_d2h(exhip_ctx* ctx, void* dst, const void* src, size
         memcpy(dst, stage, bytes);
         return 0;
     }
-    if (is_result_block(dst, bytes) || bytes <= kUploadKernel || !chunk(0) || !chunk(1)) {
-        EXHIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
-        EXHIP_CHECK(hipStreamSynchronize(ctx->stream));
-        return 0;
-    }
-    int chunks = 2;
-    while (chunks < exhip_staging::kChunks && (size_t)chunks * kChunk < bytes && chunk(chunks)) ++chunks;
-    for (int i = 0; i < chunks; ++i)
-        if (!s.event[i]) {
-            hipEvent_t e;
-            EXHIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-            s.event[i] = e;
-        }
-    copy_crew::session crew(bytes >= 4 * kPiece);
-    const size_t total = (bytes + kChunk - 1) / kChunk;
-    auto request = [&](size_t i) -> int {
-        const size_t o = i * kChunk, n = bytes - o < kChunk ? bytes - o : kChunk;
-        EXHIP_CHECK(hipMemcpyAsync(s.chunk[i % chunks], static_cast<const char*>(src) + o, n, hipMemcpyDeviceToHost, ctx->stream));
-        EXHIP_CHECK(hipEventRecord((hipEvent_t)s.event[i % chunks], ctx->stream));
-        return 0;
-    };
-    for (size_t i = 0; i < total && i < (size_t)chunks; ++i)
-        if (const int rc = request(i)) return rc;
-    for (size_t i = 0; i < total; ++i) {
-        const size_t o = i * kChunk, n = bytes - o < kChunk ? bytes - o : kChunk;
-        EXHIP_CHECK(hipEventSynchronize((hipEvent_t)s.event[i % chunks]));
-        crew.copy(static_cast<char*>(dst) + o, s.chunk[i % chunks], n);
-        if (i + chunks < total)
-            if (const int rc = request(i + chunks)) return rc;
-    }
-    return 0;
+    return download(ctx, ctx->stream, dst, src, bytes);
 }
 
 // A pinned host block for results of a megabyte and more: the copy engine writes it directly. Blocks are cached for reuse

@@ -34,6 +34,9 @@ public:
     // finds the new contents. And the first `count` values as host bytes, without keeping a host copy.
     void upload(const Dtype* src);
     void download(Dtype* out, size_t count);
+    // The device contents are what the work queued so far on the calling slot's stream makes them: a download then waits for
+    // that much of the stream only. Until the next write.
+    void mark_ready();
 
 private:
     void to_cpu();
@@ -43,6 +46,8 @@ private:
     Dtype* cpu_ptr_ = nullptr;
     Dtype* gpu_ptr_ = nullptr;
     size_t size_;
+    void* ready_ = nullptr;   // the mark, and the write it belongs to
+    unsigned long long ready_at_ = 0;
     SyncedHead head_ = UNINITIALIZED;
     unsigned long long writes_ = 0;
     int device_;

@@ -31,6 +31,7 @@ public:
     Dtype* mutable_gpu_data() const { return data_->mutable_gpu_data(); }
     void upload(const Dtype* src) const { data_->upload(src); }    // see syncedmem
     void download(Dtype* out) const { data_->download(out, static_cast<size_t>(count())); }
+    void mark_ready() const { data_->mark_ready(); }
     unsigned long long writes() const { return data_->writes(); }  // mutable_*_data() calls so far
     void copy_from(const void* data, size_t size);
 

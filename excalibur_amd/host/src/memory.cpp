@@ -112,6 +112,7 @@ syncedmem<Dtype>::syncedmem(size_t size, int device) : size_(size), device_(devi
 template <typename Dtype>
 syncedmem<Dtype>::~syncedmem() {
     if (cpu_ptr_) std::free(cpu_ptr_);
+    if (ready_) exhip_mark_destroy(ready_);
     // Kernels using this buffer may still be queued, and that is fine: every device operation of a slot (kernels,
     // copies, fills) goes through that slot's one stream, and the block returns to the cache of the slot it was taken
     // from, so whatever touches the recycled block is queued behind them.
@@ -137,7 +138,17 @@ void syncedmem<Dtype>::to_cpu() {
 }
 
 template <typename Dtype>
+void syncedmem<Dtype>::mark_ready() {
+    EXHIP_FATAL(exhip_mark(device_context(device_), &ready_));
+    ready_at_ = writes_;
+}
+
+template <typename Dtype>
 void syncedmem<Dtype>::fetch(Dtype* out, size_t count) {
+    if (ready_ && ready_at_ == writes_) {
+        EXHIP_FATAL(exhip_memcpy_d2h_from(device_context(device_, slot_), ready_, out, gpu_ptr_, count * sizeof(Dtype)));
+        return;
+    }
     // synchronises the stream of the slot the block was taken in (a pipeline's outputs: the pipeline's); a reader working
     // in another slot may have queued the writer there, so that stream is drained as well
     if (stream_slot() != slot_) EXHIP_FATAL(exhip_sync(device_context(device_)));

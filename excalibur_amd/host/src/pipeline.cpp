@@ -114,6 +114,7 @@ public:
             CHECK_EQ(std::fclose(fp), 0) << "Cannot close " << path;
         }
 
+        hoist_results();
         // blob table, producers, consumers
         std::map<std::string, int> produced_by;
         for (size_t i = 0; i < op_params_.size(); ++i)
@@ -145,6 +146,56 @@ public:
         if (input_names_.empty()) LOG(FATAL) << "the topology has no input blob";
         featmaps_.resize(blob_names_.size());
         find_activation_pairs();
+    }
+
+    // A layer chain that ends in a result of the network and that nothing else reads (a detection head: Convolution -> Reshape ->
+    // Transpose) moves to right behind the layer that makes its input. Files list such chains last; run early, their results can
+    // leave for the host while the rest of the network runs. Layers are moved as whole chains, so neighbours stay neighbours.
+    void hoist_results() {
+        const int n = static_cast<int>(op_params_.size());
+        std::map<std::string, int> made_by, readers;
+        for (int i = 0; i < n; ++i) {
+            for (const std::string& o : op_params_[i].output_featmaps_)
+                if (!made_by.emplace(o, i).second) return;  // a blob written over: the order of the file matters
+            for (const std::string& b : op_params_[i].input_featmaps_) ++readers[b];
+        }
+        auto simple = [&](int i) { return op_params_[i].input_featmaps_.size() == 1 && op_params_[i].output_featmaps_.size() == 1; };
+        std::vector<std::vector<int>> behind(n);  // chains to run right behind layer i
+        std::vector<char> moved(n, 0);
+        for (int last = 0; last < n; ++last) {
+            if (!simple(last) || readers.count(op_params_[last].output_featmaps_[0])) continue;
+            std::vector<int> chain{last};
+            int source = -1;
+            for (;;) {
+                const std::string& b = op_params_[chain.back()].input_featmaps_[0];
+                auto it = made_by.find(b);
+                if (it == made_by.end()) { chain.clear(); break; }  // down to the network's input
+                source = it->second;
+                if (!simple(source) || readers[b] != 1 || source + 1 != chain.back()) break;
+                chain.push_back(source);
+            }
+            if (chain.size() < 2 || source + 1 >= chain.back()) continue;  // a lone layer, or where it belongs already
+            for (auto it = chain.rbegin(); it != chain.rend(); ++it) {
+                behind[source].push_back(*it);
+                moved[*it] = 1;
+            }
+        }
+        std::vector<int> order;
+        std::function<void(int)> put = [&](int i) {
+            order.push_back(i);
+            for (int j : behind[i]) order.push_back(j);
+        };
+        for (int i = 0; i < n; ++i)
+            if (!moved[i]) put(i);
+        if (static_cast<int>(order.size()) != n) return;  // a chain behind a moved layer: leave the file's order
+        std::vector<operation_param> params;
+        std::vector<std::shared_ptr<operation<Dtype>>> ops;
+        for (int i : order) {
+            params.push_back(op_params_[i]);
+            ops.push_back(operations_[i]);
+        }
+        op_params_.swap(params);
+        operations_.swap(ops);
     }
 
     // A convolution whose only reader is the activation layer on the next line runs that layer in its epilogue: the
@@ -485,6 +536,10 @@ private:
             }
             operations_[i]->forward_gpu(in, out);
             for (size_t j = 0; j < out.size(); ++j) featmaps_[op_outputs_[i][j]] = out[j];
+            if (fusion_ && i + kMarkAhead < operations_.size() && out.size() == 1 && out[0]->order() == memory::NCHW &&
+                out[0]->count() * sizeof(Dtype) >= kMarkBytes &&
+                std::find(output_names_.begin(), output_names_.end(), blob_names_[op_outputs_[i][0]]) != output_names_.end())
+                out[0]->mark_ready();
         }
         blob_map results;
         for (const std::string& o : output_names_) {
@@ -494,6 +549,10 @@ private:
         }
         return results;
     }
+
+    // A result of this many bytes with at least so many layers (launches of a plan) left behind it is marked, so that it can
+    // leave while they run. The mark and the wait for it cost 10 us or so; a megabyte takes the link 18 us.
+    static constexpr size_t kMarkBytes = (size_t)1 << 20, kMarkAhead = 4;
 
     // ---------------------------------------------------------------- fused int8 executor
     bool try_fused(const tensor_ptr& input, blob_map* results);
@@ -552,6 +611,7 @@ struct pipeline<Dtype>::impl::fused_plan {
         std::shared_ptr<tensor<float>> t;
         std::vector<int> shape;
         float* slot = nullptr;
+        int launch = -1;          // the launch that completes it
     };
     std::deque<result> outputs;  // stable addresses: the launches keep pointers to the slots
     // Layers in front of the first convolution that work on the caller's NCHW tensor (Input, YoloV5Focus) and layers
@@ -1360,7 +1420,12 @@ bool pipeline<float>::impl::build_graph_plan(const tensor_ptr& input, const std:
         }
         return true;
     };
+    auto results_complete = [&]() {  // the results made so far are complete with the last launch
+        for (auto& r : plan->outputs)
+            if (r.launch < 0) r.launch = static_cast<int>(plan->launches.size()) - 1;
+    };
     for (const node& nd : nodes) {
+        results_complete();
         const value_info in = vals[nd.in[0]];
         value_info& out = vals[nd.out];
         if (in.n == 0) return refuse(__LINE__);
@@ -1584,6 +1649,7 @@ bool pipeline<float>::impl::build_graph_plan(const tensor_ptr& input, const std:
         }
         if (!more_forms(out)) return refuse(__LINE__);
     }
+    results_complete();
     // the network's outputs: results of the plan by name (Split copies share their tensor), the rest comes from the tail
     for (const std::string& o : output_names_) {
         const int v = root(blob_index_[o]);
@@ -1976,7 +2042,12 @@ bool pipeline<float>::impl::build_float_plan(const tensor_ptr& input, const std:
         if (!one_kernel)
             plan->launches.push_back([=]() { EXHIP_FATAL(exhip_nchw_f32_to_nhwc_f32(ctx, pl->input_ptr, vi.n, vi.c, vi.h, vi.w, cs, y)); });
     }
+    auto results_complete = [&]() {  // the results made so far are complete with the last launch
+        for (auto& r : plan->outputs)
+            if (r.launch < 0) r.launch = static_cast<int>(plan->launches.size()) - 1;
+    };
     for (const node& nd : nodes) {
+        results_complete();
         const value_info in = vals[nd.in[0]];
         value_info& out = vals[nd.out];
         if (in.n == 0) return refuse(__LINE__);
@@ -2247,6 +2318,7 @@ bool pipeline<float>::impl::build_float_plan(const tensor_ptr& input, const std:
             nchw_from_rows(nd.out);
         }
     }
+    results_complete();
     for (const std::string& o : output_names_) {
         const int v = root(blob_index_[o]);
         if (where[v] == 2) continue;
@@ -2294,6 +2366,7 @@ bool pipeline<float>::impl::try_fused(const tensor_ptr& input, blob_map* results
             r.t->reshape(r.shape);  // a Reshape layer behind it gave the tensor another shape in the last forward
         }
     }
+    for (auto& r : plan_->outputs) r.t->mutable_gpu_data();  // the launches below write it: the device copy is the newest
     exhip_ctx* const ctx = memory::device_context(device_);
     const int n_launches = static_cast<int>(plan_->launches.size());
     const int span_first = span_first_ == -2 ? plan_->first_conv_launch : span_first_;  // -2: from the first convolution on
@@ -2332,14 +2405,18 @@ bool pipeline<float>::impl::try_fused(const tensor_ptr& input, blob_map* results
         EXHIP_FATAL(exhip_event_record(ctx, span_ev[1]));
         span_launches_ = n_launches - span_first;
     } else {
-        for (auto& launch : plan_->launches) launch();
+        for (int i = 0; i < n_launches; ++i) {
+            plan_->launches[i]();
+            if (i + static_cast<int>(kMarkAhead) < n_launches)
+                for (auto& r : plan_->outputs)
+                    if (r.launch == i && r.t->count() * sizeof(float) >= kMarkBytes) r.t->mark_ready();
+        }
         span_launches_ = 0;
     }
     if (timed) ++span_count_;
     ++plan_->forwards;
     last_fused_ = plan_->int8;
     for (auto& r : plan_->outputs) {
-        r.t->mutable_gpu_data();  // the kernels just wrote it: the device copy is the newest
         for (int b : r.blobs) featmaps_[b] = r.t;
         if (r.name.empty()) continue;
         for (const std::string& name : split_string(r.name, "\n")) {

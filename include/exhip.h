@@ -45,6 +45,11 @@ int exhip_memcpy_d2d(exhip_ctx* ctx, void* dst, const void* src, size_t bytes);
 /* Host to device like exhip_memcpy_h2d, but returns as soon as src has been read (it goes through pinned staging): work
  * queued on the context's stream afterwards finds the bytes, other streams have to wait for this one first. */
 int exhip_upload(exhip_ctx* ctx, void* dst, const void* src, size_t bytes);
+/* A point of the context's stream: exhip_mark records it into *mark (made there if NULL), exhip_memcpy_d2h_from copies what was
+ * written before it while the stream goes on with what was queued behind it. */
+int exhip_mark(exhip_ctx* ctx, void** mark);
+int exhip_mark_destroy(void* mark);
+int exhip_memcpy_d2h_from(exhip_ctx* ctx, void* mark, void* dst, const void* src, size_t bytes);
 /* Pinned host memory for results (1 MiB and more), which exhip_memcpy_d2h fills without a copy by the host. Blocks are cached
  * process-wide (at most 512 MiB idle, 1 GiB in all); NULL where there is none: use memory of your own then. Any thread. */
 void* exhip_host_alloc(size_t bytes);
