@@ -1659,10 +1659,11 @@ inline bool fused_epilogue_ok(const exhip_conv_desc* d, const ConvParams& p, lon
 }
 
 template <int DT>
-int run_conv(exhip_ctx* ctx, const exhip_conv_desc* d, ConvParams p, const PoolSpec* pool = nullptr, const exhip_lean_proj* proj = nullptr) {
+int run_conv(exhip_ctx* ctx, const exhip_conv_desc* d, ConvParams p, const PoolSpec* pool = nullptr, const exhip_lean_proj* proj = nullptr, int group = 0) {
+    const bool joined = d->post_bn_a || d->post_bn_b || d->exact_k || group;  // what only the pointwise kernel does
     EXHIP_REQUIRE(ctx, "conv: NULL ctx");
-    // a BatchNorm in the epilogue and writes limited to the layer's own channels: int8 pointwise layers only (below)
-    if ((d->post_bn_a || d->post_bn_b || d->exact_k) && (DT != EXHIP_I8 || pool || proj)) return EXHIP_ERR_UNSUPPORTED;
+    // a BatchNorm in the epilogue, writes limited to the layer's own channels and grouped results: pointwise layers only (below)
+    if (joined && (pool || proj)) return EXHIP_ERR_UNSUPPORTED;
     Plan pl;
     int rc = make_plan(d, DT, &pl, pool);
     if (rc) return rc;
@@ -1778,11 +1779,12 @@ int run_conv(exhip_ctx* ctx, const exhip_conv_desc* d, ConvParams p, const PoolS
             g.post_alpha = d->post_alpha; g.post_beta = d->post_beta; g.post_slope = d->post_slope; g.residual_last = d->residual_last;
             g.fs_out = d->fs_out;
             g.post_bn_a = d->post_bn_a; g.post_bn_b = d->post_bn_b; g.exact_k = d->exact_k;
+            g.group = group; g.map_h = d->h; g.map_w = d->w;
             rc = exhip_conv1x1_i8_pw(ctx, g, reinterpret_cast<const int8_t*>(p.x), p.wp, p.scale, p.bias, reinterpret_cast<const float*>(p.residual),
                                      reinterpret_cast<int8_t*>(p.y_q), reinterpret_cast<float*>(p.y_nhwc));
             if (rc != EXHIP_ERR_UNSUPPORTED) return rc;
         }
-        if (d->post_bn_a || d->post_bn_b || d->exact_k) return EXHIP_ERR_UNSUPPORTED;  // only the pointwise kernel has these
+        if (joined) return EXHIP_ERR_UNSUPPORTED;
         if (!pl.packed && !proj && !p.acc_nchw && !p.y_nchw && (p.y_q || p.y_nhwc) && pl.KWe == d->kw) {
             // a layer with a filter on that kernel's tapped form, where it takes the layer
             exhip_pw_geom g = {};
@@ -1833,9 +1835,13 @@ int run_conv(exhip_ctx* ctx, const exhip_conv_desc* d, ConvParams p, const PoolS
             g.slab_blocks = pl.TM / 32; g.slabs = pl.ktiles;
             g.act = d->act; g.post_relu = d->post_relu; g.post_op = d->post_op; g.post_slope_shared = d->post_slope_shared;
             g.post_alpha = d->post_alpha; g.post_beta = d->post_beta; g.post_slope = d->post_slope; g.residual_last = d->residual_last;
+            g.post_bn_a = d->post_bn_a; g.post_bn_b = d->post_bn_b; g.exact_k = d->exact_k;
+            g.group = group; g.map_h = d->h; g.map_w = d->w;
             rc = exhip_conv1x1_f16_pw(ctx, g, reinterpret_cast<const uint16_t*>(p.x), p.wp, p.bias, reinterpret_cast<const uint16_t*>(p.residual),
                                       reinterpret_cast<uint16_t*>(p.y_q));
-            if (rc != EXHIP_ERR_UNSUPPORTED) return rc;
+            if (rc != EXHIP_ERR_UNSUPPORTED || joined) return rc;
+        } else if (joined) {
+            return EXHIP_ERR_UNSUPPORTED;
         } else if (!pl.packed && !pool && p.y_q && !p.y_nchw_h && !p.y_nchw && pl.KWe == d->kw) {
             // a layer with a filter on that kernel's tapped form, where it takes the layer
             exhip_pw_geom g = {};
@@ -2011,4 +2017,20 @@ extern "C" int exhip_conv2d_f16(exhip_ctx* ctx, const exhip_conv_desc* d, const 
     p.x = (const char*)x; p.wp = (const char*)wp; p.bias = bias; p.residual = residual;
     p.y_q = y_f16_nhwc; p.y_nchw_h = y_f16_nchw; p.y_nchw = y_f32_nchw;
     return run_conv<EXHIP_F16>(ctx, d, p);
+}
+
+extern "C" int exhip_conv2d_i8_grouped(exhip_ctx* ctx, const exhip_conv_desc* d, int group, const int8_t* x, const void* wp, const float* scale,
+                                       const float* bias, float* y) {
+    EXHIP_REQUIRE(scale && y && group > 0, "exhip_conv2d_i8_grouped: bad argument");
+    ConvParams p = {};
+    p.x = (const char*)x; p.wp = (const char*)wp; p.scale = scale; p.bias = bias; p.y_nhwc = y;
+    return run_conv<EXHIP_I8>(ctx, d, p, nullptr, nullptr, group);
+}
+
+extern "C" int exhip_conv2d_f16_grouped(exhip_ctx* ctx, const exhip_conv_desc* d, int group, const uint16_t* x, const void* wp, const float* bias,
+                                        uint16_t* y) {
+    EXHIP_REQUIRE(y && group > 0, "exhip_conv2d_f16_grouped: bad argument");
+    ConvParams p = {};
+    p.x = (const char*)x; p.wp = (const char*)wp; p.bias = bias; p.y_q = y;
+    return run_conv<EXHIP_F16>(ctx, d, p, nullptr, nullptr, group);
 }

@@ -54,6 +54,7 @@ struct PwParams {
     float fs_out;
     const float* post_bn_a;   // BatchNorm in front of post_op: fmaf(post_bn_b[ch], v, post_bn_a[ch])
     const float* post_bn_b;
+    int group;                // a detection head: results go to [image][channel / group][pixel][channel % group] (0: rows)
     int exact;                // channels [0, K) only: blocks past K are not written (the results lie inside a wider tensor)
     unsigned pixels, x_bytes, w_bytes;
     unsigned items, ch_groups;   // waves with work; 32 * MT channel groups per pixel tile
@@ -176,6 +177,20 @@ __device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[
     char* const tile = lds + param_bytes(MT);
     const int k_end = p.exact ? p.K : p.kstride > p.K ? p.kstride : p.K;  // channels from here on are not written
     const bool shortcut = ANY ? (I8 ? p.residual_f != nullptr : p.residual != nullptr) : EP::res != 0;
+    // grouped results: every half-wave writes the 32 channels of one pixel of a block, runs of neighbouring values (a head of 128 -> 255
+    // channels at 16 x 80 x 80 takes 37 us, the memory's time for its 104 MB is 20; without this form, 41 us and a second launch over them)
+    auto store_grouped = [&](auto* y, int pitch, int at0, unsigned first, int rows, int kb) {
+        typedef typename std::remove_pointer<decltype(y)>::type T;
+        const unsigned per_image = (unsigned)(p.out_h * p.out_w), img = exhip_divide(first + row, per_image, p.image_magic, p.image_shift);
+        const unsigned lane_at = img * (unsigned)p.K * per_image + (first + row - img * per_image) * (unsigned)p.group;
+        const int ch = kb * 32 + row, g = ch / p.group, member = ch - g * p.group;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int srow = j * 2 + half;
+            const unsigned at = (unsigned)__builtin_amdgcn_ds_bpermute(srow * 4, (int)lane_at) + (unsigned)g * per_image * (unsigned)p.group + member;
+            if (srow < rows && ch < p.K) y[at] = *reinterpret_cast<const T*>(tile + srow * pitch + at0 + row * (int)sizeof(T));
+        }
+    };
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
         const unsigned first = pix0 + n * 32;
@@ -227,14 +242,13 @@ __device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[
             };
             if (ANY ? shortcut && !p.residual_last : EP::res == 1) add_shortcut();
             if (ANY ? p.post_relu != 0 : EP::post == kPostRelu) relu16<!I8>(v);
-            if constexpr (I8) {
-                if (ANY ? p.post_bn_a != nullptr : EP::bn) {  // the BatchNorm layer between this layer (through a Concat) and its activation layer
-                    float a[16], b[16];
-                    read16<MT>(lds, 2, m, half, a);
-                    read16<MT>(lds, 3, m, half, b);
+            if (ANY ? p.post_bn_a != nullptr : EP::bn) {  // the BatchNorm layer between this layer (through a Concat) and its activation layer
+                float a[16], b[16];
+                read16<MT>(lds, 2, m, half, a);
+                read16<MT>(lds, 3, m, half, b);
+                stored16<!I8>(v);
 #pragma unroll
-                    for (int e = 0; e < 16; ++e) v[e] = __builtin_fmaf(b[e], v[e], a[e]);
-                }
+                for (int e = 0; e < 16; ++e) v[e] = __builtin_fmaf(b[e], v[e], a[e]);
             }
             if (ANY ? p.post_op == 1 + EXHIP_UNARY_HARDSWISH : EP::post == kPostHardSwish) unary16<0, !I8>(v, p.post_alpha, p.post_beta);
             if (ANY ? p.post_op == 1 + EXHIP_UNARY_LEAKYRELU : EP::post == kPostLeaky) unary16<1, !I8>(v, p.post_alpha, p.post_beta);
@@ -260,7 +274,8 @@ __device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[
                         const v4f o = {v[q * 4], v[q * 4 + 1], v[q * 4 + 2], v[q * 4 + 3]};
                         *reinterpret_cast<v4f*>(tile + row * pitch + half * 64 + q * 16) = o;
                     }
-                    store_rows<8>(tile, pitch, tile_view(p.y_f, first, p.kstride * 4, kb * 128, rows), p.kstride * 4, (k_end - kb * 32) * 4, lane);
+                    if (ANY && p.group) store_grouped(p.y_f, pitch, 0, first, rows, kb);
+                    else store_rows<8>(tile, pitch, tile_view(p.y_f, first, p.kstride * 4, kb * 128, rows), p.kstride * 4, (k_end - kb * 32) * 4, lane);
                 }
                 if (p.y_q) {
                     v4i o;
@@ -285,6 +300,13 @@ __device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[
             }
             // one 32 x 32 block at a time: interleaving the blocks buys nothing and costs the registers of their temporaries
             __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (!I8) {
+            if (ANY && p.group) {
+#pragma unroll
+                for (int m = 0; m < MT; ++m) store_grouped(p.y, MT * 64 + 16, m * 64, first, rows, kb0 + m);
+                continue;
+            }
         }
         if constexpr (!I8)
             store_rows<MT * 4>(tile, MT * 64 + 16, tile_view(p.y, first, p.kstride * 2, kb0 * 64, rows), p.kstride * 2, (k_end - kb0 * 32) * 2, lane);
@@ -404,7 +426,7 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
         if constexpr (DT == EXHIP_I8) par[0] = load(p.scale, at, p.K);
         par[1] = load(p.bias, at, p.K);
         if (EP::any || EP::post == kPostPrelu) par[2] = load(p.post_slope, p.post_slope_shared ? 0 : at, p.post_slope_shared ? 1 : p.K);
-        if (DT == EXHIP_I8 && (EP::any ? p.post_bn_a != nullptr : EP::bn)) {
+        if (EP::any ? p.post_bn_a != nullptr : EP::bn) {
             par[2] = load(p.post_bn_a, at, p.K);
             par[3] = load(p.post_bn_b, at, p.K);
         }
@@ -531,7 +553,7 @@ __global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParam
         if constexpr (DT == EXHIP_I8) par[0] = load(p.scale, at, p.K);
         par[1] = load(p.bias, at, p.K);
         if (EP::any || EP::post == kPostPrelu) par[2] = load(p.post_slope, p.post_slope_shared ? 0 : at, p.post_slope_shared ? 1 : p.K);
-        if (DT == EXHIP_I8 && (EP::any ? p.post_bn_a != nullptr : EP::bn)) {
+        if (EP::any ? p.post_bn_a != nullptr : EP::bn) {
             par[2] = load(p.post_bn_a, at, p.K);
             par[3] = load(p.post_bn_b, at, p.K);
         }
@@ -619,6 +641,7 @@ int pick_epilogue(exhip_ctx* ctx, const PwParams& p) {
         post = post == kPostNone ? op : -1;
     }
     const bool bn = p.post_bn_a != nullptr;
+    if (p.group) return go<DT, MT, NT, U == 8 ? 4 : U, TAPS, EpAny>(ctx, p);
     auto is = [&](int a, int q, int r, bool b) { return p.act == a && post == q && res == r && bn == b; };
     if (is(0, kPostNone, 0, false)) return go<DT, MT, NT, U, TAPS, Ep<0, kPostNone, 0>>(ctx, p);
     if (is(0, kPostHardSwish, 0, false)) return go<DT, MT, NT, U, TAPS, Ep<0, kPostHardSwish, 0>>(ctx, p);
@@ -629,6 +652,8 @@ int pick_epilogue(exhip_ctx* ctx, const PwParams& p) {
     if constexpr (DT == EXHIP_F16) {
         if (is(0, kPostPrelu, 0, false)) return go<DT, MT, NT, U, TAPS, Ep<0, kPostPrelu, 0>>(ctx, p);
         if (is(0, kPostNone, 1, false)) return go<DT, MT, NT, U, TAPS, Ep<0, kPostNone, 1>>(ctx, p);
+        if constexpr (!TAPS)
+            if (is(0, kPostLeaky, 0, true)) return go<DT, MT, NT, U, TAPS, Ep<0, kPostLeaky, 0, true>>(ctx, p);
     } else {
         if (is(0, kPostRelu, 2, false)) return go<DT, MT, NT, U, TAPS, Ep<0, kPostRelu, 2>>(ctx, p);
         if constexpr (!TAPS)
@@ -703,7 +728,7 @@ bool small_tile() { return g_exhip_options.pw_tile != 2; }
 template <int DT>
 int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwParams& p, bool has_residual) {
     if (g_exhip_options.direct == 0) return EXHIP_ERR_UNSUPPORTED;
-    if (g.post_bn_a || g.post_bn_b || g.exact_k) return EXHIP_ERR_UNSUPPORTED;
+    if (g.post_bn_a || g.post_bn_b || g.exact_k || g.group) return EXHIP_ERR_UNSUPPORTED;
     const long long n_ksteps = (long long)t.n_chunks * t.kh * t.kw * (t.chunk_b / 32);
     if (g.pixels <= 0 || g.c_bytes <= 0 || g.c_bytes % 32 != 0 || t.chunk_b % 32 != 0 || t.n_chunks * t.chunk_b != g.c_bytes ||
         (g.slab_blocks != 2 && g.slab_blocks != 4) || g.k_stride % 8 != 0 || (n_ksteps > kMaxDirectSteps && !split_wins(DT, true, g.pixels, (std::max(g.k, g.k_stride) + 31) / 32, (int)n_ksteps)) || t.kh * t.kw > (1 << (32 - kTapShift)) || t.stride < 1 || t.pad_t < 0 || t.pad_l < 0)
@@ -767,9 +792,19 @@ int run_pw(exhip_ctx* ctx, const exhip_pw_geom& g, PwParams& p, int es, bool has
     // 64-byte store runs against the general epilogue's 16-byte pieces: 41 against 60 us on a 128 -> 255 head at
     // 16 x 80 x 80). Beyond that the general kernel's staged tiles re-read less and win (128 -> 128 at 80 x 80).
     // Option pw = 2 takes every layer the kernel can (tests), 0 none.
-    const bool joined = g.post_bn_a || g.exact_k;  // only this kernel has those: it takes the layer whatever its size
-    if (joined && (DT != EXHIP_I8 || (g.post_bn_a == nullptr) != (g.post_bn_b == nullptr) || (g.exact_k && g.k % 32 != 0))) return EXHIP_ERR_UNSUPPORTED;
-    const int out_channels = g.exact_k ? g.k : std::max(g.k, g.k_stride);  // channels this launch writes
+    const bool joined = g.post_bn_a || g.exact_k || g.group;  // only this kernel has those: it takes the layer whatever its size
+    if (joined && ((g.post_bn_a == nullptr) != (g.post_bn_b == nullptr) || (g.post_bn_a && g.post_op == EXHIP_POST_PRELU) || (g.exact_k && g.k % 32 != 0)))
+        return EXHIP_ERR_UNSUPPORTED;
+    if (g.group) {
+        if (g.group < 0 || g.k % g.group != 0 || g.pixels % ((long long)g.map_h * g.map_w) != 0 || g.pixels * g.k >= (1ll << 32) || p.y_q || has_residual)
+            return EXHIP_ERR_UNSUPPORTED;
+        p.group = g.group;
+        p.out_h = g.map_h;
+        p.out_w = g.map_w;
+        exhip_host_divisor((unsigned)(g.map_h * g.map_w), &p.image_magic, &p.image_shift);
+    }
+    p.post_bn_a = g.post_bn_a; p.post_bn_b = g.post_bn_b; p.exact = g.exact_k || g.group;
+    const int out_channels = g.exact_k || g.group ? g.k : std::max(g.k, g.k_stride);  // channels this launch writes
     const int blocks_needed = (out_channels + 31) / 32;
     const double flop = 2.0 * (double)g.pixels * (g.c_bytes / es) * g.k;
     bool take = joined || blocks_needed == 1 || (flop <= 8.0e9 && g.pixels <= 32768);
@@ -825,7 +860,6 @@ int exhip_conv1x1_i8_pw(exhip_ctx* ctx, const exhip_pw_geom& g, const int8_t* x,
     PwParams p = {};
     p.x = reinterpret_cast<const char*>(x); p.wp = reinterpret_cast<const char*>(wp); p.bias = bias; p.scale = scale;
     p.residual_f = residual; p.y_f = y_f32; p.y_q = y_i8; p.fs_out = g.fs_out;
-    p.post_bn_a = g.post_bn_a; p.post_bn_b = g.post_bn_b; p.exact = g.exact_k;
     return run_pw<EXHIP_I8>(ctx, g, p, 1, residual != nullptr, taps);
 }
 

@@ -262,6 +262,13 @@ class Ctx:
         _check(lib().exhip_conv2d_f16(self.h, ctypes.byref(d), x.ptr, wp.ptr, _ptr(bias), _ptr(residual), _ptr(y_f16_nhwc),
                                       _ptr(y_f16_nchw), _ptr(y_f32_nchw)))
 
+    def conv2d_grouped(self, d, group, x, wp, bias, y, scale=None):
+        """A detection head (y: n x k / group x pixels x group): int8 with `scale`, else fp16."""
+        if scale is not None:
+            _check(lib().exhip_conv2d_i8_grouped(self.h, ctypes.byref(d), group, x.ptr, wp.ptr, scale.ptr, _ptr(bias), y.ptr))
+        else:
+            _check(lib().exhip_conv2d_f16_grouped(self.h, ctypes.byref(d), group, x.ptr, wp.ptr, _ptr(bias), y.ptr))
+
     def conv2d_f32(self, d, x, wp, bias=None, residual=None, y_f32_nhwc=None, y_f32_nchw=None):
         _check(lib().exhip_conv2d_f32(self.h, ctypes.byref(d), x.ptr, wp.ptr, _ptr(bias), _ptr(residual), _ptr(y_f32_nhwc),
                                       _ptr(y_f32_nchw)))

@@ -1483,18 +1483,24 @@ bool pipeline<float>::impl::build_graph_plan(const tensor_ptr& input, const std:
             }
             if (nd.head_reshape >= 0) {
                 // [n, K, oh, ow] -> Reshape [n, G, J, oh * ow] -> Transpose [n, G, oh * ow, J]: the convolution writes float32
-                // NHWC and one kernel regroups the channels of every pixel
+                // NHWC and one kernel regroups the channels of every pixel where the convolution cannot store them so itself
                 auto* rs = static_cast<operation_reshape<float>*>(operations_[nd.head_reshape].get());
                 const std::vector<int> to = rs->new_shape({in.n, c->output_channel_, oh, ow}, in.n * c->output_channel_ * oh * ow);
                 if (to.size() != 4 || to[0] != in.n || to[1] * to[2] != c->output_channel_ || to[3] != oh * ow) return refuse(__LINE__);
                 if (out.need_i8 || out.need_f32 || !out.need_nchw || nd.res >= 0) return refuse(__LINE__);
                 const int groups = to[1], per_group = to[2], hw = oh * ow, n0 = in.n;
                 out.n = in.n; out.c = groups; out.h = hw; out.w = per_group; out.cs = 0;
-                float* mid = static_cast<float*>(alloc(elems * sizeof(float)));
                 float** slot = nchw_result(out, nd.out);
                 const void* wp = c->pin_packed_weights(EXHIP_I8, d);
                 plan->pinned.emplace_back([c, wp]() { c->unpin_packed_weights(wp); });
                 const float *scale = c->scale_gpu(), *bias = c->bias_gpu();
+                const int rc = exhip_conv2d_i8_grouped(ctx, &d, per_group, x, wp, scale, bias, *slot);  // trial launch
+                if (rc == 0) {
+                    plan->launches.push_back([=]() { EXHIP_FATAL(exhip_conv2d_i8_grouped(ctx, &d, per_group, x, wp, scale, bias, *slot)); });
+                    continue;
+                }
+                if (rc != EXHIP_ERR_UNSUPPORTED) EXHIP_FATAL(rc);
+                float* mid = static_cast<float*>(alloc(elems * sizeof(float)));
                 plan->launches.push_back([=]() {
                     EXHIP_FATAL(exhip_conv2d_i8(ctx, &d, x, wp, scale, bias, nullptr, nullptr, mid, nullptr, nullptr));
                     EXHIP_FATAL(exhip_nhwc_f32_to_grouped_f32(ctx, mid, n0, hw, groups, per_group, ks, *slot));

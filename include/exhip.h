@@ -133,7 +133,7 @@ typedef struct exhip_conv_desc {
     int post_slope_shared;
     int residual_last;          /* 1: the shortcut is added behind post_relu / post_op instead of in front of them (a sum
                                  * layer behind the activation layer that follows the convolution) */
-    /* exhip_conv2d_i8, 1x1 stride-1 layers with NHWC results only: the BatchNorm layer (operation_batchnorm.cpp:122-156)
+    /* exhip_conv2d_i8 and exhip_conv2d_f16, 1x1 stride-1 layers with NHWC results only: the BatchNorm layer (operation_batchnorm.cpp:122-156)
      * that follows the layer through a Concat, applied in front of post_op: v = fmaf(post_bn_b[k], v, post_bn_a[k]) with
      * device arrays of k floats (the layer's a / b for this convolution's channels); both NULL = none */
     const float* post_bn_a;
@@ -204,6 +204,14 @@ int exhip_stem_f32_conv_i8_maxpool3x3s2(exhip_ctx* ctx, const exhip_conv_desc* d
                                         int pool_ow, const float* x_f32_nchw, float fs_in, const void* w_packed,
                                         const float* scale, int scales_nonnegative, const float* bias, int8_t* y_i8_nhwc,
                                         float* y_f32_nhwc);
+
+/* A detection head: the 1x1 convolution, the Reshape of its channels into groups and the Transpose of the last two axes
+ * (operation_reshape.cpp, operation_transpose.cpp) as one launch, y[n][k / group][pixel][group] (float32 of an int8 layer, halves).
+ * EXHIP_ERR_UNSUPPORTED, with nothing launched, where the pointwise kernel cannot take the layer. */
+int exhip_conv2d_i8_grouped(exhip_ctx* ctx, const exhip_conv_desc* d, int group, const int8_t* x_nhwc, const void* w_packed, const float* scale,
+                            const float* bias, float* y);
+int exhip_conv2d_f16_grouped(exhip_ctx* ctx, const exhip_conv_desc* d, int group, const uint16_t* x_nhwc, const void* w_packed, const float* bias,
+                             uint16_t* y);
 
 /* operation_convolution::forward_cpu_f32 (src/Excalibur/operation_convolution.cpp:251-329) with fp16
  * storage and f32 accumulation (include/Excalibur/operation.hpp:234-260 describes the fp16 layer):

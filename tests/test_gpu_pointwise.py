@@ -242,6 +242,32 @@ def test_batchnorm_and_exact_channels_are_refused_outside_the_int8_pointwise_ker
         ctx.conv2d_i8(d, xq, wp, ctx.array(dequant_scales(case1["ws"], case1["fs"], 48)), None, None, y)
 
 
+@pytest.mark.parametrize("dtype", ["int8", "f16"])
+@pytest.mark.parametrize("n,c,h,w,k,group", [(1, 32, 5, 7, 6, 3), (2, 64, 9, 11, 255, 85), (3, 256, 6, 6, 96, 1), (1, 64, 33, 31, 64, 64), (1, 1056, 4, 8, 40, 5)],
+                         ids=lambda v: str(v))
+def test_grouped_results_are_the_layers_own_rearranged(ctx, dtype, n, c, h, w, k, group):
+    """Groups that straddle 32-channel blocks, images that begin inside a 32-pixel tile, the split form (1056 channels)."""
+    r = np.random.default_rng(c + k)
+    ks = hip.pad_to(k, 32)
+    d = ctx.conv_desc(n, c, h, w, k, 1, c_stride=c, k_stride=ks)
+    bias = ctx.array(r.normal(0, 0.5, k).astype(np.float32))
+    if dtype == "int8":
+        x, wp = ctx.array(r.integers(-127, 128, (n, h, w, c), dtype=np.int8)), ctx.pack_conv_weights(d, hip.I8, r.integers(-127, 128, (k, c, 1, 1), dtype=np.int8))
+        scale = ctx.array(r.uniform(1e-4, 1e-3, k).astype(np.float32))
+        rows, y = ctx.empty((n, h, w, ks), np.float32), ctx.array(np.full((n, k // group, h * w, group), np.nan, np.float32))
+        ctx.conv2d_i8(d, x, wp, scale, bias, None, None, rows)
+        ctx.conv2d_grouped(d, group, x, wp, bias, y, scale)
+    else:
+        x = ctx.array(r.normal(0, 1, (n, h, w, c)).astype(np.float16).view(np.uint16))
+        wp = ctx.pack_conv_weights(d, hip.F16, r.normal(0, 0.05, (k, c, 1, 1)).astype(np.float16).view(np.uint16))
+        rows, y = ctx.empty((n, h, w, ks), np.uint16), ctx.array(np.full((n, k // group, h * w, group), 0x7e00, np.uint16))
+        ctx.conv2d_f16(d, x, wp, bias, None, rows)
+        ctx.conv2d_grouped(d, group, x, wp, bias, y)
+    ctx.sync()
+    want = rows.download()[..., :k].reshape(n, h * w, k // group, group).transpose(0, 2, 1, 3)
+    assert np.array_equal(y.download(), want) and np.count_nonzero(want) > want.size // 2
+
+
 TAP_SHAPES = [
     # seed, n, c, h, w, k, kernel, stride, pad, shortcut (0 none, 1 in front, 2 behind), act, post_relu, post_op
     (800, 2, 12, 40, 36, 32, 3, 1, 1, 0, 0, 0, "hardswish"),       # a first layer behind Focus: 12 channels in a 32-byte pixel
