@@ -1659,8 +1659,9 @@ inline bool fused_epilogue_ok(const exhip_conv_desc* d, const ConvParams& p, lon
 }
 
 template <int DT>
-int run_conv(exhip_ctx* ctx, const exhip_conv_desc* d, ConvParams p, const PoolSpec* pool = nullptr, const exhip_lean_proj* proj = nullptr, int group = 0) {
-    const bool joined = d->post_bn_a || d->post_bn_b || d->exact_k || group;  // what only the pointwise kernel does
+int run_conv(exhip_ctx* ctx, const exhip_conv_desc* d, ConvParams p, const PoolSpec* pool = nullptr, const exhip_lean_proj* proj = nullptr, int group = 0,
+             const exhip_pw_depthwise* dw = nullptr) {
+    const bool joined = d->post_bn_a || d->post_bn_b || d->exact_k || group || dw;  // what only the pointwise kernel does
     EXHIP_REQUIRE(ctx, "conv: NULL ctx");
     // a BatchNorm in the epilogue, writes limited to the layer's own channels and grouped results: pointwise layers only (below)
     if (joined && (pool || proj)) return EXHIP_ERR_UNSUPPORTED;
@@ -1838,7 +1839,7 @@ int run_conv(exhip_ctx* ctx, const exhip_conv_desc* d, ConvParams p, const PoolS
             g.post_bn_a = d->post_bn_a; g.post_bn_b = d->post_bn_b; g.exact_k = d->exact_k;
             g.group = group; g.map_h = d->h; g.map_w = d->w;
             rc = exhip_conv1x1_f16_pw(ctx, g, reinterpret_cast<const uint16_t*>(p.x), p.wp, p.bias, reinterpret_cast<const uint16_t*>(p.residual),
-                                      reinterpret_cast<uint16_t*>(p.y_q));
+                                      reinterpret_cast<uint16_t*>(p.y_q), nullptr, dw);
             if (rc != EXHIP_ERR_UNSUPPORTED || joined) return rc;
         } else if (joined) {
             return EXHIP_ERR_UNSUPPORTED;
@@ -2033,4 +2034,17 @@ extern "C" int exhip_conv2d_f16_grouped(exhip_ctx* ctx, const exhip_conv_desc* d
     ConvParams p = {};
     p.x = (const char*)x; p.wp = (const char*)wp; p.bias = bias; p.y_q = y;
     return run_conv<EXHIP_F16>(ctx, d, p, nullptr, nullptr, group);
+}
+
+extern "C" int exhip_dw_pw_f16(exhip_ctx* ctx, const exhip_depthwise_desc* dw, const exhip_conv_desc* d, const void* wp, const float* bias,
+                               const uint16_t* residual, uint16_t* y) {
+    EXHIP_REQUIRE(dw && d && dw->x && dw->w9 && y, "exhip_dw_pw_f16: NULL argument");
+    EXHIP_REQUIRE(dw->n == d->n && dw->h > 0 && dw->w > 0 && dw->stride > 0 && dw->pt >= 0 && dw->pl >= 0 && dw->pb >= 0 && dw->pr >= 0 &&
+                      (dw->h + dw->pt + dw->pb - 3) / dw->stride + 1 == d->h && (dw->w + dw->pl + dw->pr - 3) / dw->stride + 1 == d->w &&
+                      d->c_stride == d->c && dw->h + dw->pt + dw->pb >= 3 && dw->w + dw->pl + dw->pr >= 3,
+                  "exhip_dw_pw_f16: the layers' maps do not fit");
+    const exhip_pw_depthwise g = {dw->x, dw->w9, dw->bias, dw->slope, dw->slope_shared, dw->act, dw->n, dw->h, dw->w, d->h, d->w, dw->stride, dw->pt, dw->pl};
+    ConvParams p = {};
+    p.x = (const char*)dw->x; p.wp = (const char*)wp; p.bias = bias; p.residual = (const char*)residual; p.y_q = y;
+    return run_conv<EXHIP_F16>(ctx, d, p, nullptr, nullptr, 0, &g);
 }

@@ -32,10 +32,21 @@ struct exhip_pw_taps {
     int n_chunks, chunk_b;             // the packing: channel chunks of chunk_b bytes (a multiple of 32), n_chunks * chunk_b bytes per pixel
 };
 
+// The depthwise 3x3 layer in front of a pointwise layer, in the same kernel: its NHWC input, weights [channel][9], bias or NULL,
+// PReLU slopes or NULL, activation 0, 1 or 3; out_h x out_w are the pointwise layer's map.
+struct exhip_pw_depthwise {
+    const uint16_t* x;
+    const float* w9;
+    const float* bias;
+    const float* slope;
+    int slope_shared, act;
+    int n, in_h, in_w, out_h, out_w, stride, pad_t, pad_l;
+};
+
 // Returns 0 when launched, EXHIP_ERR_UNSUPPORTED when the geometry is outside what the kernel takes (the caller then
 // runs the general kernel), another code on failure. Semantics as exhip_conv2d_f16 with only the NHWC half output.
 int exhip_conv1x1_f16_pw(exhip_ctx* ctx, const exhip_pw_geom& g, const uint16_t* x, const void* wp, const float* bias,
-                         const uint16_t* residual, uint16_t* y, const exhip_pw_taps* taps = nullptr);
+                         const uint16_t* residual, uint16_t* y, const exhip_pw_taps* taps = nullptr, const exhip_pw_depthwise* dw = nullptr);
 // The int8 layer: semantics as exhip_conv2d_i8 with the NHWC results only (y_i8 and / or y_f32; k_stride a multiple of 16).
 int exhip_conv1x1_i8_pw(exhip_ctx* ctx, const exhip_pw_geom& g, const int8_t* x, const void* wp, const float* scale, const float* bias,
                         const float* residual, int8_t* y_i8, float* y_f32, const exhip_pw_taps* taps = nullptr);

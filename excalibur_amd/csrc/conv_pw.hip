@@ -75,6 +75,12 @@ struct PwParams {
     // behind the last row to the next chunk
     int start_s[kSplit + 1], start_b[kSplit + 1], start_r[kSplit + 1], start_q[kSplit + 1], start_left[kSplit + 1];
     int chunk_b, row_end_b, chunk_end_b;
+    // the depthwise 3x3 layer in front (dw_pw_kernel; geometry in in_h .. pad_l above, x is its input): weights, bias and PReLU slopes,
+    // activation 0, 1 or 3; 32-pixel tiles of a group and output blocks of a group
+    const float* dw_w;
+    const float* dw_bias;
+    const float* dw_slope;
+    int dw_act, dw_slope_shared, dw_tiles, dw_kblocks, dw_split, kblocks;
 };
 
 __device__ __noinline__ float slow_activation(float v, int act) { return exhip_act(v, act); }
@@ -619,6 +625,168 @@ __global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParam
     pw_epilogue<DT, 1, 1, EP>(p, sum, tile * 32, kb0 + part, lane, lds);
 }
 
+// A depthwise 3x3 layer and the pointwise layer that alone reads it, the depthwise results staying in LDS. A group computes
+// all C channels of 32 * dw_tiles output pixels -- a thread owns four channels of strips of PX pixels, the arithmetic and roundings
+// of dwconv3x3_nhwc_strip_kernel -- and its four waves then take the tile's 32 x 32 output blocks, pixel fragments from LDS, weight
+// fragments from L2 with R k-steps in flight. A small launch deals the output channels over several groups, each with depthwise
+// results of its own. A layer that the split form above would take (dw_split) adds its four runs of k-steps in that form's order.
+// Bound by a launch's fixed cost where it is small, by the depthwise loads where it is large: 64 x 128 x 56 x 56 takes 43 us (61 as two
+// launches), 1 x 64 x 56 x 56 takes 4.6 us (9.0).
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+typedef int v2i __attribute__((ext_vector_type(2)));
+
+template <int S, int PX, typename EP>
+__global__ __launch_bounds__(256, 3) void dw_pw_kernel(const PwParams p) {
+    constexpr int R = 4, NC = (PX - 1) * S + 3;
+    constexpr unsigned kRowOutside = 0x80000000u, kColOutside = 0x40000000u;  // tensors of at most 2^30 bytes: beyond the view, alone or together
+    extern __shared__ __attribute__((aligned(16))) char lds_dyn[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    unsigned item0 = blockIdx.x;
+    {
+        const unsigned per = gridDim.x >> 3;
+        if (item0 < (per << 3)) item0 = (item0 & 7) * per + (item0 >> 3);
+    }
+    const unsigned tile = __builtin_amdgcn_readfirstlane(exhip_divide(item0, p.ch_groups, p.groups_magic, p.groups_shift));
+    const int kb_first = __builtin_amdgcn_readfirstlane((int)(item0 - tile * p.ch_groups) * p.dw_kblocks);
+    const unsigned pix0 = tile * 32 * p.dw_tiles;
+    char* const lds = lds_dyn + wave * wave_bytes(EXHIP_F16, 1);
+    char* const mid = lds_dyn + 4 * wave_bytes(EXHIP_F16, 1);
+    const int mid_pitch = p.xs_b + 16;
+    {
+        const int groups = p.xs_b >> 3, g = threadIdx.x % groups, lanes = 256 / groups, first = threadIdx.x / groups;
+        const int strips = first < lanes ? 32 * p.dw_tiles / PX : 0;
+        const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.x), 0, (int)p.x_bytes, kRsrcWord3);
+        float k[36], b[4] = {0.f, 0.f, 0.f, 0.f}, sl[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < 9; ++q) {
+            const v4f t = reinterpret_cast<const v4f*>(p.dw_w + g * 36)[q];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) k[q * 4 + e] = t[e];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (p.dw_bias) b[e] = p.dw_bias[g * 4 + e];
+            if (p.dw_slope) sl[e] = p.dw_slope[p.dw_slope_shared ? 0 : g * 4 + e];
+        }
+        const unsigned per_image = (unsigned)(p.out_h * p.out_w);
+        const int row_b = p.in_w * p.xs_b;
+        for (int st = first; st < strips; st += lanes) {
+            const unsigned pix = pix0 + st * PX;
+            const unsigned img = exhip_divide(pix, per_image, p.image_magic, p.image_shift), rem = pix - img * per_image;
+            const int oy = (int)exhip_divide(rem, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = (int)(rem - (unsigned)oy * (unsigned)p.out_w);
+            const int iy = pix < p.pixels ? oy * S - p.pad_t : -4, ix = ox * S - p.pad_l;
+            const unsigned at = img * (unsigned)(p.in_h * row_b) + g * 8;
+            unsigned row_off[3], col_off[NC];
+#pragma unroll
+            for (int a = 0; a < 3; ++a) row_off[a] = (unsigned)(iy + a) < (unsigned)p.in_h ? at + (unsigned)((iy + a) * row_b) : kRowOutside;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) col_off[c] = (unsigned)(ix + c) < (unsigned)p.in_w ? (unsigned)((ix + c) * p.xs_b) : kColOutside;
+            v4h r[3][NC];
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+#pragma unroll
+                for (int c = 0; c < NC; ++c) r[a][c] = __builtin_bit_cast(v4h, __builtin_amdgcn_raw_buffer_load_b64(xr, (int)(row_off[a] + col_off[c]), 0, 0));
+#pragma unroll
+            for (int px = 0; px < PX; ++px) {
+                v4f res;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float sum = b[e];
+#pragma unroll
+                    for (int j = 0; j < 3; ++j) {
+                        float s = 0.f;
+#pragma unroll
+                        for (int a = 0; a < 3; ++a) s = __builtin_fmaf((float)r[a][px * S + j][e], k[e * 9 + a * 3 + j], s);
+                        sum += s;
+                    }
+                    res[e] = sum;
+                }
+                if (p.dw_slope) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float h = exhip_h2f(exhip_f2h(res[e]));
+                        res[e] = h >= 0.f ? h : sl[e] * h;
+                    }
+                } else if (p.dw_act != 0) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        res[e] = (0.f > res[e]) ? 0.f : res[e];
+                        if (p.dw_act == 3) res[e] = res[e] <= 6.f ? res[e] : 0.f;
+                    }
+                }
+                const v2i o = {(int)round_pair(res[0], res[1]), (int)round_pair(res[2], res[3])};
+                *reinterpret_cast<v2i*>(mid + (st * PX + px) * mid_pitch + g * 8) = o;
+            }
+        }
+    }
+    __syncthreads();
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.wp), 0, (int)p.w_bytes, kRsrcWord3);
+    const int blocks = p.kblocks - kb_first < p.dw_kblocks ? p.kblocks - kb_first : p.dw_kblocks;
+    const int nks = p.n_ksteps, w_step = p.mts * 1024;
+    for (int item = wave; item < blocks * p.dw_tiles; item += 4) {
+        const int sub = item & (p.dw_tiles - 1), kb = kb_first + (item >> (p.dw_tiles - 1));
+        const unsigned first = pix0 + sub * 32;
+        if (first >= p.pixels) continue;  // wave-uniform; no barrier follows
+        const int w_base = ((kb >> (p.mts >> 1)) * nks * p.mts + (kb & (p.mts - 1))) * 1024;
+        v4i a[R];
+        auto request = [&](int u, int s) {
+            a[u] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, lane * 16, w_base + (s < nks ? s : nks - 1) * w_step, 0));
+        };
+#pragma unroll
+        for (int u = 0; u < R; ++u) request(u, u);
+        float par[kParams] = {};
+        {
+            const int at = lane < 32 ? (kb * 32 + lane) * 4 : kOutOfRange;
+            auto load = [&](const float* src, int offset, int count) {
+                const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src), 0, src ? count * 4 : 0, kRsrcWord3);
+                return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, offset, 0, 0));
+            };
+            par[1] = load(p.bias, at, p.K);
+            if (EP::any || EP::post == kPostPrelu) par[2] = load(p.post_slope, p.post_slope_shared ? 0 : at, p.post_slope_shared ? 1 : p.K);
+        }
+        v16f acc, sum[1][1];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[e] = sum[0][0][e] = 0.f;
+        const char* src = mid + (sub * 32 + (lane & 31)) * mid_pitch + (lane >> 5) * 16;
+        int run = 1, end = p.dw_split ? p.start_s[1] : nks;
+        for (int s = 0; s < nks; s += R) {
+#pragma unroll
+            for (int u = 0; u < R; ++u) {
+                if (s + u < nks) {
+                    if (s + u == end) {
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) sum[0][0][e] += acc[e], acc[e] = 0.f;
+                        do end = p.start_s[++run]; while (end == s + u);
+                    }
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a[u]), *reinterpret_cast<const v8h*>(src + (s + u) * 32), acc, 0, 0, 0);
+                }
+                request(u, s + R + u);
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sum[0][0][e] += acc[e];
+        if (lane < 32) {
+#pragma unroll
+            for (int i = 0; i < kParams; ++i) *reinterpret_cast<float*>(lds + (i * 32 + lane) * 4) = par[i];
+        }
+        pw_epilogue<EXHIP_F16, 1, 1, EP>(p, sum, first, kb, lane, lds);
+    }
+}
+
+template <int S, int PX>
+int go_dw(exhip_ctx* ctx, const PwParams& p) {
+    const int lds = 4 * wave_bytes(EXHIP_F16, 1) + 32 * p.dw_tiles * (p.xs_b + 16);
+    auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(p.items), dim3(256), lds, ctx->stream, p);
+        EXHIP_LAUNCH_CHECK();
+        return 0;
+    };
+    const int res = !p.residual ? 0 : p.residual_last ? 2 : 1;
+    if (!p.post_relu && !p.post_op && p.act == 0 && res < 2) return res ? run(dw_pw_kernel<S, PX, Ep<0, kPostNone, 1>>) : run(dw_pw_kernel<S, PX, Ep<0, kPostNone, 0>>);
+    if (!p.post_relu && p.act == 0 && p.post_op == EXHIP_POST_PRELU && res == 0) return run(dw_pw_kernel<S, PX, Ep<0, kPostPrelu, 0>>);
+    return run(dw_pw_kernel<S, PX, EpAny>);
+}
+
 // U < 0: the split form with -U waves to a tile
 template <int DT, int MT, int NT, int U, bool TAPS, typename EP>
 int go(exhip_ctx* ctx, const PwParams& p) {
@@ -779,10 +947,46 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
     return launch<DT, 2, 2, true>(ctx, p, kblocks);
 }
 
+// The pointwise layer p behind the depthwise layer dw.
+int run_depthwise(exhip_ctx* ctx, const exhip_pw_depthwise& dw, PwParams& p, int kblocks, bool split) {
+    if (g_exhip_options.dw_pw == 0) return EXHIP_ERR_UNSUPPORTED;
+    const long long x_bytes = (long long)dw.n * dw.in_h * dw.in_w * p.xs_b;
+    if (p.xs_b > 1024 || x_bytes > (1ll << 30) || (dw.stride != 1 && dw.stride != 2) || (dw.act != 0 && dw.act != 1 && dw.act != 3) ||
+        (long long)dw.n * dw.out_h * dw.out_w != (long long)p.pixels)
+        return EXHIP_ERR_UNSUPPORTED;
+    p.x = reinterpret_cast<const char*>(dw.x); p.x_bytes = (unsigned)x_bytes;
+    p.in_h = dw.in_h; p.in_w = dw.in_w; p.out_h = dw.out_h; p.out_w = dw.out_w; p.stride = dw.stride; p.pad_t = dw.pad_t; p.pad_l = dw.pad_l;
+    p.dw_w = dw.w9; p.dw_bias = dw.bias; p.dw_slope = dw.slope; p.dw_slope_shared = dw.slope_shared; p.dw_act = dw.act;
+    exhip_host_divisor((unsigned)(dw.out_h * dw.out_w), &p.image_magic, &p.image_shift);
+    exhip_host_divisor((unsigned)dw.out_w, &p.width_magic, &p.width_shift);
+    const long long tiles32 = ((long long)p.pixels + 31) / 32;
+    // A thread that computes more than four strips of a tile one behind the other makes the depthwise half the longer one (1 x 512 x 22 x 22
+    // at stride 2: 15.6 against 9.5 us for two launches; 1 x 256 x 22 x 22: 10.3 against 11.0; 64 x 512 x 14 x 14 at stride 2: 20.6
+    // against 16.6). Beyond 128 tiles, where a launch's fixed 4 us no longer count, a widening layer loses as well: its depthwise half
+    // waits behind the stores of the wider result (64 x 32 x 112 x 112 -> 64: 81 against 67 us). The others win (64 x 128 x 56 x 56: 43
+    // against 61 us).
+    const int pixels = dw.stride == 2 ? 2 - dw.out_w % 2 : dw.out_w % 4 == 0 ? 4 : 2 - dw.out_w % 2;
+    const bool long_strips = 32 / pixels * (p.xs_b >> 3) > 4 * 256;
+    if (g_exhip_options.dw_pw != 2 && (long_strips || (tiles32 > 128 && kblocks * 64 > p.xs_b))) return EXHIP_ERR_UNSUPPORTED;
+    p.dw_tiles = p.xs_b <= 512 && tiles32 >= 1024 ? 2 : 1;
+    const long long tiles = (tiles32 + p.dw_tiles - 1) / p.dw_tiles;
+    int groups = 1;
+    while (groups * 4 < kblocks * p.dw_tiles && tiles * groups * 2 <= 512) groups *= 2;
+    p.kblocks = kblocks;
+    p.dw_kblocks = (kblocks + groups - 1) / groups;
+    p.ch_groups = (unsigned)((kblocks + p.dw_kblocks - 1) / p.dw_kblocks);
+    p.items = (unsigned)(tiles * p.ch_groups);
+    exhip_host_divisor(p.ch_groups, &p.groups_magic, &p.groups_shift);
+    p.dw_split = split;
+    for (int i = 0; i <= kSplit; ++i) p.start_s[i] = (int)((long long)p.n_ksteps * i / kSplit);
+    if (dw.stride == 2) return pixels == 2 ? go_dw<2, 2>(ctx, p) : go_dw<2, 1>(ctx, p);
+    return pixels == 4 ? go_dw<1, 4>(ctx, p) : pixels == 2 ? go_dw<1, 2>(ctx, p) : go_dw<1, 1>(ctx, p);
+}
+
 // Geometry checks and the wave tile, shared by the two data types. `es`: bytes per input element.
 template <int DT>
-int run_pw(exhip_ctx* ctx, const exhip_pw_geom& g, PwParams& p, int es, bool has_residual, const exhip_pw_taps* t = nullptr) {
-    if (g_exhip_options.pw == 0) return EXHIP_ERR_UNSUPPORTED;
+int run_pw(exhip_ctx* ctx, const exhip_pw_geom& g, PwParams& p, int es, bool has_residual, const exhip_pw_taps* t = nullptr, const exhip_pw_depthwise* dw = nullptr) {
+    if (g_exhip_options.pw == 0 || (dw && (t || g.post_bn_a || g.exact_k || g.group))) return EXHIP_ERR_UNSUPPORTED;
     if (t) return run_taps<DT>(ctx, g, *t, p, has_residual);
     // Measured per layer against the general kernel inside a detection and two mobile networks (16 and 64 images, kernel
     // traces): this form wins where a launch is short -- every layer of at most 32 768 pixels up to about 7 GFLOP (twice
@@ -836,6 +1040,8 @@ int run_pw(exhip_ctx* ctx, const exhip_pw_geom& g, PwParams& p, int es, bool has
     // every packed block that holds a channel below max(k, k_stride): pad channels of the output are written as zeros
     // (exact_k: only the blocks of the k channels themselves)
     const int kblocks = std::min(g.slabs * g.slab_blocks, (out_channels + 31) / 32);
+    if constexpr (DT == EXHIP_F16)
+        if (dw) return run_depthwise(ctx, *dw, p, kblocks, split_wins(DT, false, g.pixels, kblocks, (int)n_ksteps));
     // 64 x 64 per wave unless that leaves SIMDs without a wave: then 64 channels x 32 pixels; a lone 32-channel block
     // takes 128 pixels per wave
     if (split_wins(DT, false, g.pixels, kblocks, (int)n_ksteps)) return launch_split<DT, false>(ctx, p, kblocks);
@@ -848,10 +1054,10 @@ int run_pw(exhip_ctx* ctx, const exhip_pw_geom& g, PwParams& p, int es, bool has
 }  // namespace
 
 int exhip_conv1x1_f16_pw(exhip_ctx* ctx, const exhip_pw_geom& g, const uint16_t* x, const void* wp, const float* bias,
-                         const uint16_t* residual, uint16_t* y, const exhip_pw_taps* taps) {
+                         const uint16_t* residual, uint16_t* y, const exhip_pw_taps* taps, const exhip_pw_depthwise* dw) {
     PwParams p = {};
     p.x = reinterpret_cast<const char*>(x); p.wp = reinterpret_cast<const char*>(wp); p.bias = bias; p.residual = residual; p.y = y;
-    return run_pw<EXHIP_F16>(ctx, g, p, 2, residual != nullptr, taps);
+    return run_pw<EXHIP_F16>(ctx, g, p, 2, residual != nullptr, taps, dw);
 }
 
 int exhip_conv1x1_i8_pw(exhip_ctx* ctx, const exhip_pw_geom& g, const int8_t* x, const void* wp, const float* scale, const float* bias,

@@ -35,6 +35,9 @@ public:
 };
 
 template <typename Dtype>
+class operation_convolutiondepthwise;
+
+template <typename Dtype>
 class operation_convolution : public operation_general_conv<Dtype> {
 public:
     template <typename T>
@@ -75,6 +78,9 @@ public:
         post_sum_ = other; post_sum_used_ = false; post_sum_last_ = behind_activation;
     }
     bool post_sum_used() const { return post_sum_used_; }
+    // fp16: this layer, a pointwise one, with the 3x3 depthwise layer that it alone reads in front of it in one kernel, each with
+    // the layers set behind it; `bottoms` are the depthwise layer's. False, with nothing done, where the pair runs as two layers.
+    bool forward_behind_depthwise(operation_convolutiondepthwise<Dtype>& dw, const tensor_list<unsigned short>& bottoms, tensor_list<unsigned short>& tops);
     // int8 layers on the MFMA kernel. The next forward calls also write the int8 NHWC form of the output that a reader
     // quantizing with `fs` into `stride` channels per pixel would make of it (attached to the top blob as its
     // `quantized` copy), and with `only` leave the float data unwritten; fs = 0 switches it off. False where this
@@ -88,6 +94,7 @@ protected:
     void forward_gpu_i8(const tensor_list<float>& bottoms, tensor_list<float>& tops) override;
     void forward_gpu_f16(const tensor_list<unsigned short>& bottoms, tensor_list<unsigned short>& tops) override;
     bool mfma_path_ok() const;
+    const unsigned short* sum_operand(const tensor_list<unsigned short>& tops, exhip_conv_desc* d);
     int post_op_ = 0;
     float post_alpha_ = 0.f, post_beta_ = 0.f;
     bool post_relu_ = false;
@@ -118,6 +125,7 @@ public:
     void quantized_input(float* fs, int* stride) const override { *fs = 0.f; *stride = 0; }
 
 protected:
+    friend class operation_convolution<Dtype>;
     void forward_gpu_f32(const tensor_list<float>& bottoms, tensor_list<float>& tops) override;
     void forward_gpu_i8(const tensor_list<float>& bottoms, tensor_list<float>& tops) override;
     void forward_gpu_f16(const tensor_list<unsigned short>& bottoms, tensor_list<unsigned short>& tops) override;

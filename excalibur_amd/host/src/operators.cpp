@@ -552,15 +552,44 @@ void operation_convolution<Dtype>::forward_gpu_f16(const tensor_list<unsigned sh
     tops[0] = out_nhwc ? new_tensor<unsigned short>({n, oh, ow, this->output_channel_}, dev, memory::NHWC)
                        : new_tensor<unsigned short>({n, this->output_channel_, oh, ow}, dev);
     unsigned short* y = tops[0]->mutable_gpu_data();
-    const unsigned short* residual = nullptr;
-    if (post_sum_ && out_nhwc && post_sum_->order() == memory::NHWC && post_sum_->data_shape() == tops[0]->data_shape() &&
-        (post_sum_last_ || (!post_op_ && !post_relu_))) {
-        residual = post_sum_->gpu_data();
-        d.residual_last = post_sum_last_ ? 1 : 0;
-        post_sum_used_ = true;
-    }
+    const unsigned short* residual = out_nhwc ? sum_operand(tops, &d) : nullptr;
     EXHIP_FATAL(exhip_conv2d_f16(this->ctx(), &d, x->gpu_data(), packed_weights(EXHIP_F16, d), bias_gpu(), residual,
                                  out_nhwc ? y : nullptr, out_nhwc ? nullptr : y, nullptr));
+}
+
+// The operand of the sum layer behind this one where the epilogue can add it to the NHWC result tops[0], else NULL.
+template <typename Dtype>
+const unsigned short* operation_convolution<Dtype>::sum_operand(const tensor_list<unsigned short>& tops, exhip_conv_desc* d) {
+    if (!post_sum_ || post_sum_->order() != memory::NHWC || post_sum_->data_shape() != tops[0]->data_shape() ||
+        !(post_sum_last_ || (!post_op_ && !post_relu_)))
+        return nullptr;
+    d->residual_last = post_sum_last_ ? 1 : 0;
+    post_sum_used_ = true;
+    return post_sum_->gpu_data();
+}
+
+template <typename Dtype>
+bool operation_convolution<Dtype>::forward_behind_depthwise(operation_convolutiondepthwise<Dtype>& dw, const tensor_list<unsigned short>& bottoms,
+                                                            tensor_list<unsigned short>& tops) {
+    const int dev = this->params_.device_, c = this->input_channels();
+    if (bottoms[0]->order() != memory::NHWC || bottoms[0]->channels() != c || dw.output_channel_ != c || dw.group_ != c || !dw.fast3x3() ||
+        !nhwc_channels_ok(c) || !mfma_path_ok() || this->output_channel_ % 16 != 0)
+        return false;
+    const int n = bottoms[0]->num(), h = bottoms[0]->height(), w = bottoms[0]->width();
+    const int oh = (h + dw.pad_top_ + dw.pad_bottom_ - 3) / dw.stride_h_ + 1, ow = (w + dw.pad_left_ + dw.pad_right_ - 3) / dw.stride_w_ + 1;
+    exhip_conv_desc d = describe(n, oh, ow, c, this->output_channel_);
+    if (d.kh != 1 || d.kw != 1 || d.sh != 1 || d.sw != 1 || d.pt || d.pb || d.pl || d.pr || conv_in_stride(c, EXHIP_F16, 1) != c) return false;
+    const exhip_depthwise_desc q = {bottoms[0]->gpu_data(), dw.weights_f32_[0]->gpu_data(), dw.bias_gpu(), dw.post_slope_, dw.post_slope_shared_,
+                                    dw.activation_type_, n, h, w, dw.stride_h_, dw.pad_top_, dw.pad_bottom_, dw.pad_left_, dw.pad_right_};
+    tops[0] = new_tensor<unsigned short>({n, oh, ow, this->output_channel_}, dev, memory::NHWC);
+    const unsigned short* residual = sum_operand(tops, &d);
+    const int rc = exhip_dw_pw_f16(this->ctx(), &q, &d, packed_weights(EXHIP_F16, d), bias_gpu(), residual, tops[0]->mutable_gpu_data());
+    if (rc == EXHIP_ERR_UNSUPPORTED) {
+        post_sum_used_ = false;
+        return false;
+    }
+    EXHIP_FATAL(rc);
+    return true;
 }
 
 // ------------------------------------------------------------------ depthwise convolution

@@ -234,7 +234,32 @@ public:
         }
         find_quantized_links();
         find_sum_pairs();
+        find_depthwise_pairs();
         find_glue_chains();
+    }
+
+    // fp16 pipeline: a depthwise layer (with its PReLU layer) whose only reader is the convolution behind it: where that is a
+    // pointwise layer one kernel runs both, and the blob between them is never stored.
+    void find_depthwise_pairs() {
+        behind_depthwise_.assign(operations_.size(), -1);
+        if constexpr (std::is_same_v<Dtype, unsigned short>) {
+            std::vector<int> readers(blob_names_.size(), 0);
+            for (const auto& in : op_inputs_)
+                for (int b : in) ++readers[b];
+            for (size_t i = 0; i + 1 < operations_.size(); ++i) {
+                if (!dynamic_cast<operation_convolutiondepthwise<Dtype>*>(operations_[i].get())) continue;
+                const size_t last = pair_[i].on ? i + 1 : i;
+                if (last + 1 >= operations_.size() || op_outputs_[last].size() != 1 || op_inputs_[last + 1].size() != 1) continue;
+                const int mid = op_outputs_[last][0];
+                auto* conv = dynamic_cast<operation_convolution<Dtype>*>(operations_[last + 1].get());
+                if (!conv || dynamic_cast<operation_convolutiondepthwise<Dtype>*>(conv) || op_inputs_[last + 1][0] != mid) continue;
+                // an activation writing over its input reads the blob as well
+                const int own_readers = pair_[i].on && op_outputs_[i][0] == mid ? 2 : 1;
+                if (readers[mid] != own_readers || op_outputs_[last + 1].size() != 1 || op_outputs_[last + 1][0] == mid) continue;
+                if (std::find(output_names_.begin(), output_names_.end(), blob_names_[mid]) != output_names_.end()) continue;
+                behind_depthwise_[i] = static_cast<int>(last + 1);
+            }
+        }
     }
 
     // fp16 pipeline: a convolution whose only reader is the two-input sum on the next line (Eltwise SUM with unit
@@ -466,14 +491,35 @@ private:
                 if (!featmaps_[b]) LOG(FATAL) << "layer " << op_params_[i].name_ << " reads blob " << blob_names_[b] << " before it is produced";
                 in.push_back(featmaps_[b]);
             }
+            auto set_paired_activation = [&](size_t layer) {
+                auto* conv = static_cast<operation_convolution<Dtype>*>(operations_[layer].get());
+                const post_activation& pa = pair_[layer];
+                if (pa.on && pa.prelu) conv->set_post_prelu(pa.prelu->weights_f32()[0]->gpu_data(), pa.prelu->share_channel_);
+                else if (pa.on) conv->set_post_activation(pa.post_op, pa.alpha, pa.beta, pa.relu);
+                return conv;
+            };
+            if constexpr (std::is_same_v<Dtype, unsigned short>) {
+                if (fusion_ && behind_depthwise_[i] >= 0) {
+                    const size_t j = behind_depthwise_[i];
+                    auto* dw = static_cast<operation_convolutiondepthwise<Dtype>*>(set_paired_activation(i));
+                    auto* conv = set_paired_activation(j);
+                    if (sum_other_[j] >= 0 && featmaps_[sum_other_[j]]) conv->set_post_sum(featmaps_[sum_other_[j]], pair_[j].on);
+                    const bool ran = conv->forward_behind_depthwise(*dw, in, out), summed = conv->post_sum_used();
+                    dw->clear_post();
+                    conv->clear_post();
+                    if (ran) {
+                        const size_t done = j + (pair_[j].on ? 1 : 0) + (summed ? 1 : 0);  // the last layer whose work the launch did
+                        for (size_t k = i; k < done; ++k) featmaps_[op_outputs_[k][0]] = nullptr;
+                        featmaps_[op_outputs_[done][0]] = out[0];
+                        i = done;
+                        continue;
+                    }
+                }
+            }
             if constexpr (std::is_same_v<Dtype, unsigned short>) {
                 if (fusion_ && sum_other_[i] >= 0 && featmaps_[sum_other_[i]]) {
-                    auto* conv = static_cast<operation_convolution<Dtype>*>(operations_[i].get());
                     const bool paired = pair_[i].on;  // the activation layer between the convolution and the sum
-                    if (paired && pair_[i].prelu)
-                        conv->set_post_prelu(pair_[i].prelu->weights_f32()[0]->gpu_data(), pair_[i].prelu->share_channel_);
-                    else if (paired)
-                        conv->set_post_activation(pair_[i].post_op, pair_[i].alpha, pair_[i].beta, pair_[i].relu);
+                    auto* conv = set_paired_activation(i);
                     conv->set_post_sum(featmaps_[sum_other_[i]], paired);
                     conv->forward_gpu(in, out);
                     const bool summed = conv->post_sum_used();
@@ -516,11 +562,7 @@ private:
                 }
             }
             if (fusion_ && (pair_[i].on || link_[i].on)) {
-                auto* conv = static_cast<operation_convolution<Dtype>*>(operations_[i].get());
-                if (pair_[i].on && pair_[i].prelu)
-                    conv->set_post_prelu(pair_[i].prelu->weights_f32()[0]->gpu_data(), pair_[i].prelu->share_channel_);
-                else if (pair_[i].on)
-                    conv->set_post_activation(pair_[i].post_op, pair_[i].alpha, pair_[i].beta, pair_[i].relu);
+                auto* conv = set_paired_activation(i);
                 if (link_[i].on) conv->set_quantized_output(link_[i].fs, link_[i].stride, link_[i].only);
                 conv->forward_gpu(in, out);
                 conv->clear_post();
@@ -588,6 +630,7 @@ private:
         int stride = 0;
     };
     std::vector<int> sum_other_;         // per layer: the other operand's blob of the sum layer this convolution absorbs, or -1
+    std::vector<int> behind_depthwise_;  // per layer: the pointwise layer that runs in this depthwise layer's kernel, or -1
     struct glue_chain {
         int bn = -1, unary = -1, last = -1;  // layer numbers of the absorbed BatchNorm / activation, and of the last absorbed layer
     };

@@ -205,6 +205,21 @@ int exhip_stem_f32_conv_i8_maxpool3x3s2(exhip_ctx* ctx, const exhip_conv_desc* d
                                         const float* scale, int scales_nonnegative, const float* bias, int8_t* y_i8_nhwc,
                                         float* y_f32_nhwc);
 
+/* A depthwise 3x3 layer (stride 1 or 2, activation 0, 1 or 3 or the PReLU layer behind it) and the pointwise layer d that alone reads
+ * it (operation_convolutiondepthwise.cpp, operation_convolution.cpp) as one launch on NHWC halves: d is the pointwise layer on the
+ * depthwise layer's map, c_stride == c. Values are those of the two layers run one after the other, bit for bit.
+ * EXHIP_ERR_UNSUPPORTED, with nothing launched, where the pair runs as two launches. */
+typedef struct exhip_depthwise_desc {
+    const uint16_t* x; /* n x h x w x d->c */
+    const float* w9;   /* 9 per channel */
+    const float* bias; /* or NULL */
+    const float* slope; /* of a PReLU layer behind it, or NULL */
+    int slope_shared, act;
+    int n, h, w, stride, pt, pb, pl, pr;
+} exhip_depthwise_desc;
+int exhip_dw_pw_f16(exhip_ctx* ctx, const exhip_depthwise_desc* dw, const exhip_conv_desc* d, const void* w_packed, const float* bias,
+                    const uint16_t* residual_nhwc, uint16_t* y_nhwc);
+
 /* A detection head: the 1x1 convolution, the Reshape of its channels into groups and the Transpose of the last two axes
  * (operation_reshape.cpp, operation_transpose.cpp) as one launch, y[n][k / group][pixel][group] (float32 of an int8 layer, halves).
  * EXHIP_ERR_UNSUPPORTED, with nothing launched, where the pointwise kernel cannot take the layer. */
