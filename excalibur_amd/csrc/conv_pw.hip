@@ -24,6 +24,7 @@
 #include <type_traits>
 
 #include "conv_pw.h"
+#include "pw_rows.h"
 
 namespace {
 
@@ -34,7 +35,7 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 constexpr unsigned kRsrcWord3 = 0x00020000u;  // raw buffer: out-of-range loads return 0
-constexpr int kOutOfRange = 0x7ffff000;       // a lane offset beyond every view
+constexpr int kOutOfRange = kPwOutOfRange;    // a lane offset beyond every view
 constexpr int kMaxDirectSteps = 40;           // k-steps of a layer with a filter (taps x 32-byte steps per pixel)
 constexpr int kSplit = 4;                     // waves that share a tile's k-steps in the split form
 constexpr int kTapShift = 27;                 // a step's table entry: byte offset below, tap number above
@@ -161,7 +162,7 @@ __device__ __forceinline__ void relu16(float (&v)[16]) {
 template <int CHUNKS>
 __device__ __forceinline__ void store_rows(const char* tile, int pitch, __amdgpu_buffer_rsrc_t y, int row_bytes, int bytes, int lane) {
     const int row = lane / CHUNKS, col = (lane % CHUNKS) * 16;
-    const int at = col < bytes ? row * row_bytes + col : kOutOfRange;
+    const int at = pw_lane_offset(row, row_bytes, col, bytes);
 #pragma unroll
     for (int j = 0; j < CHUNKS / 2; ++j) {
         const v4i t = *reinterpret_cast<const v4i*>(tile + (j * (64 / CHUNKS) + row) * pitch + col);
@@ -172,7 +173,7 @@ __device__ __forceinline__ void store_rows(const char* tile, int pitch, __amdgpu
 // A view of a pixel-major tensor from pixel `first` and channel ch0 on, `rows` pixels long.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_view(const void* base, unsigned first, int row_bytes, int ch_bytes, int rows) {
     char* p = const_cast<char*>(static_cast<const char*>(base)) + (size_t)first * (unsigned)row_bytes + ch_bytes;
-    return __builtin_amdgcn_make_buffer_rsrc(p, 0, rows * row_bytes - ch_bytes, kRsrcWord3);
+    return __builtin_amdgcn_make_buffer_rsrc(p, 0, pw_view_bytes(rows, row_bytes, ch_bytes), kRsrcWord3);
 }
 
 template <int DT, int MT, int NT, typename EP, typename ACC>
@@ -181,7 +182,7 @@ __device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[
     constexpr int ES = I8 ? 4 : 2;  // bytes per value of the shortcut tensor
     const int half = lane >> 5, row = lane & 31;
     char* const tile = lds + param_bytes(MT);
-    const int k_end = p.exact ? p.K : p.kstride > p.K ? p.kstride : p.K;  // channels from here on are not written
+    const int k_end = pw_channel_end(p.K, p.kstride, p.exact);
     const bool shortcut = ANY ? (I8 ? p.residual_f != nullptr : p.residual != nullptr) : EP::res != 0;
     // grouped results: every half-wave writes the 32 channels of one pixel of a block, runs of neighbouring values (a head of 128 -> 255
     // channels at 16 x 80 x 80 takes 37 us, the memory's time for its 104 MB is 20; without this form, 41 us and a second launch over them)
@@ -212,14 +213,14 @@ __device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[
 #pragma unroll
                 for (int q = 0; q < ES; ++q) {
                     const int ch = m * 32 + half * 16 + q * (16 / ES);
-                    const int at = kb0 * 32 + ch < p.kstride ? row * p.kstride * ES + ch * ES : kOutOfRange;
+                    const int at = pw_lane_offset(row, p.kstride * ES, ch * ES, (p.kstride - kb0 * 32) * ES);
                     r[m][q] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rr, at, 0, 0));
                 }
         }
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
             const int kb = kb0 + m, ch0 = kb * 32 + half * 16;
-            if (m > 0 && kb * 32 >= k_end) continue;
+            if (m > 0 && !pw_block_exists(kb, k_end)) continue;
             float v[16], t[16];
             if constexpr (I8) {
                 float b[16];
@@ -294,7 +295,7 @@ __device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[
                     }
                     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(__attribute__((ext_vector_type(4))) unsigned int, o),
                                                            tile_view(p.y_q, first, p.kstride, kb * 32, rows),
-                                                           ch0 < k_end ? row * p.kstride + half * 16 : kOutOfRange, 0, 0);
+                                                           pw_lane_offset(row, p.kstride, half * 16, k_end - kb * 32), 0, 0);
                 }
             } else {
                 constexpr int pitch = MT * 64 + 16;
@@ -601,7 +602,8 @@ __global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParam
         for (int q = 0; q < 4; ++q) *reinterpret_cast<v4i*>(lds_all + (part * MT + m) * 4096 + q * 1024 + lane * 16) = word4(acc[m], q);
     }
     __syncthreads();
-    if (part >= MT) return;
+    // the wave of a second block that does not exist (an odd number of blocks) is done too
+    if (part >= MT || !pw_block_exists(kb0 + part, pw_channel_end(p.K, p.kstride, p.exact))) return;
     if (lane < 32) {
 #pragma unroll
         for (int i = 0; i < kParams; ++i) *reinterpret_cast<float*>(lds + (i * 32 + lane) * 4) = par[i];
@@ -899,7 +901,7 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
     if (g.post_bn_a || g.post_bn_b || g.exact_k || g.group) return EXHIP_ERR_UNSUPPORTED;
     const long long n_ksteps = (long long)t.n_chunks * t.kh * t.kw * (t.chunk_b / 32);
     if (g.pixels <= 0 || g.c_bytes <= 0 || g.c_bytes % 32 != 0 || t.chunk_b % 32 != 0 || t.n_chunks * t.chunk_b != g.c_bytes ||
-        (g.slab_blocks != 2 && g.slab_blocks != 4) || g.k_stride % 8 != 0 || (n_ksteps > kMaxDirectSteps && !split_wins(DT, true, g.pixels, (std::max(g.k, g.k_stride) + 31) / 32, (int)n_ksteps)) || t.kh * t.kw > (1 << (32 - kTapShift)) || t.stride < 1 || t.pad_t < 0 || t.pad_l < 0)
+        (g.slab_blocks != 2 && g.slab_blocks != 4) || g.k_stride % 8 != 0 || !pw_row_fits(4ll * g.k_stride) || (n_ksteps > kMaxDirectSteps && !split_wins(DT, true, g.pixels, (std::max(g.k, g.k_stride) + 31) / 32, (int)n_ksteps)) || t.kh * t.kw > (1 << (32 - kTapShift)) || t.stride < 1 || t.pad_t < 0 || t.pad_l < 0)
         return EXHIP_ERR_UNSUPPORTED;
     const long long x_bytes = (long long)t.n * t.in_h * t.in_w * g.c_bytes;
     const long long w_bytes = (long long)g.slabs * n_ksteps * g.slab_blocks * 1024;
@@ -1021,7 +1023,7 @@ int run_pw(exhip_ctx* ctx, const exhip_pw_geom& g, PwParams& p, int es, bool has
     if (DT == EXHIP_F16 && g_exhip_options.pw_tile != 2) take = true;
     if (DT == EXHIP_F16 && ((g.c_bytes <= 128 && g.pixels <= 524288) || (g.c_bytes <= 256 && g.k <= 64 && g.pixels <= 131072))) take = true;
     if (g_exhip_options.pw != 2 && !take) return EXHIP_ERR_UNSUPPORTED;
-    if (g.pixels <= 0 || g.c_bytes <= 0 || g.c_bytes % 32 != 0 || (g.slab_blocks != 2 && g.slab_blocks != 4) || g.k_stride % 8 != 0)
+    if (g.pixels <= 0 || g.c_bytes <= 0 || g.c_bytes % 32 != 0 || (g.slab_blocks != 2 && g.slab_blocks != 4) || g.k_stride % 8 != 0 || !pw_row_fits(4ll * g.k_stride))
         return EXHIP_ERR_UNSUPPORTED;
     // lane offsets are 32-bit: the input tensor and the packed weights must stay below the out-of-range sentinel
     const long long x_bytes = g.pixels * g.c_bytes;

@@ -79,3 +79,82 @@ def test_fp16_split_against_the_oracle(ctx, options, args):
     got = runs[0].view(np.float16).astype(np.float32)
     assert cases.check_value(got[..., :k].transpose(0, 3, 1, 2), want, 2e-3) == 0
     assert not got[..., k:].any()
+
+
+# An odd number of 32-channel blocks leaves the last pair with one: 80 and 144 channels at a stride of their own, maps whose last
+# tile holds one or two pixels.
+ODD = [
+    # seed, c, h, w, k, kernel
+    (960, 128, 1, 1, 80, 1),
+    (961, 128, 15, 15, 144, 1),    # 225 pixels: 7 * 32 + 1
+    (962, 160, 1, 34, 80, 1),
+    (963, 32, 3, 11, 80, 3),       # 33 pixels, nine steps or more
+    (964, 128, 2, 1, 144, 3),
+    (965, 512, 17, 17, 272, 1),
+]
+
+
+def whole_numbers(seed, c, h, w, k, kernel, bound):
+    """Inputs and weights whose sums are exact in every precision, and the layer's result [h, w, k] with padding kernel // 2."""
+    rng = np.random.default_rng(seed)
+    x, wt = rng.integers(-3, 4, (h, w, c)), rng.integers(-3, 4, (k, c, kernel, kernel))
+    p = kernel // 2
+    padded = np.pad(x, ((p, p), (p, p), (0, 0)))
+    y = sum(padded[r:r + h, q:q + w] @ wt[:, :, r, q].T for r in range(kernel) for q in range(kernel))
+    assert np.abs(y).max() < bound
+    return x, wt, y
+
+
+def guarded(ctx, shape, dtype, fill):
+    """An array in the middle of a larger one: (the operand, a function that returns its values once nothing beside it changed)."""
+    size, row = int(np.prod(shape)), int(shape[-1])
+    guard = 64 * row
+    whole = ctx.array(np.full(size + 2 * guard, fill, dtype))
+
+    def read():
+        got = whole.download()
+        assert (got[:guard] == fill).all() and (got[-guard:] == fill).all()
+        return got[guard:-guard].reshape(shape)
+
+    return whole.at(guard * np.dtype(dtype).itemsize), read
+
+
+@pytest.mark.parametrize("shortcut", [0, 1])
+@pytest.mark.parametrize("split", [0, 1, 2])
+@pytest.mark.parametrize("args", ODD, ids=[f"s{a[0]}" for a in ODD])
+def test_fp16_split_of_an_odd_number_of_blocks(ctx, options, args, split, shortcut):
+    seed, c, h, w, k, kernel = args
+    x, wt, want = whole_numbers(seed, c, h, w, k, kernel, 1900)   # whole numbers up to 2048 are halves
+    d = ctx.conv_desc(1, c, h, w, k, kernel, 1, kernel // 2, 0, c, k)
+    res = np.random.default_rng(seed + 1).integers(-99, 100, (h, w, k)) if shortcut else None
+    options("pw_split", split)
+    options("direct", 2)
+    y, read = guarded(ctx, (h, w, k), np.uint16, 0x7e00)
+    xd, wp = ctx.array(x.astype(np.float16).view(np.uint16)), ctx.pack_conv_weights(d, hip.F16, wt.astype(np.float16).view(np.uint16))
+    rd = ctx.array(res.astype(np.float16).view(np.uint16)) if shortcut else None
+    ctx.conv2d_f16(d, xd, wp, None, rd, y)
+    ctx.sync()
+    assert np.array_equal(read().view(np.float16).astype(np.int64), want + res if shortcut else want)
+
+
+@pytest.mark.parametrize("shortcut", [0, 1])
+@pytest.mark.parametrize("split", [0, 1, 2])
+@pytest.mark.parametrize("args", ODD, ids=[f"s{a[0]}" for a in ODD])
+def test_int8_split_of_an_odd_number_of_blocks(ctx, options, args, split, shortcut):
+    seed, c, h, w, k, kernel = args
+    x, wt, want = whole_numbers(seed, c, h, w, k, kernel, 1 << 20)
+    d = ctx.conv_desc(1, c, h, w, k, kernel, 1, kernel // 2, 0, c, k, fs_out=0.25)
+    res = np.random.default_rng(seed + 1).integers(-99, 100, (h, w, k)) if shortcut else None
+    options("pw_split", split)
+    options("direct", 2)
+    options("pw", 2)
+    y_f, read_f = guarded(ctx, (h, w, k), np.float32, np.float32(7))
+    y_q, read_q = guarded(ctx, (h, w, k), np.int8, 77)
+    xd, wp = ctx.array(x.astype(np.int8)), ctx.pack_conv_weights(d, hip.I8, wt.astype(np.int8))
+    rd = ctx.array(res.astype(np.float32)) if shortcut else None
+    ctx.conv2d_i8(d, xd, wp, ctx.array(np.ones(k, np.float32)), None, rd, y_q, y_f)
+    ctx.sync()
+    want = want + res if shortcut else want
+    assert np.array_equal(read_f().astype(np.int64), want)
+    t = want * 0.25
+    assert np.array_equal(read_q().astype(np.int64), np.clip(np.trunc(t + np.copysign(0.5, t)), -128, 127).astype(np.int64))
