@@ -4,6 +4,8 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include <mutex>
+
 #include "../../include/exhip.h"
 
 // Pinned chunks that host <-> device copies of a context go through (transfer.hip), taken when first needed.
@@ -21,11 +23,10 @@ struct exhip_ctx {
     hipStream_t stream;
     exhip_staging up, down;
     unsigned download_number = 0;  // of the last small download, the value its flag takes
-    // scratch of the convolution's split reduction, grown on demand and kept until the context is destroyed
+    // scratch of the convolution's split reduction, allocated when first needed and kept until the context is destroyed
+    std::mutex split_mu;
     int* split_acc = nullptr;
-    size_t split_acc_bytes = 0;
     unsigned* split_count = nullptr;
-    size_t split_count_n = 0;
 };
 
 // The context's split-reduction scratch (partial accumulators, and one zeroed arrival counter per tile): allocated on first

@@ -205,24 +205,26 @@ int exhip_split_scratch(exhip_ctx* ctx, size_t acc_bytes, size_t tiles, int** ac
     constexpr size_t kAccBytes = (size_t)kSplitGroups * 512 * 256, kCounters = kSplitGroups;
     EXHIP_REQUIRE(acc_bytes <= kAccBytes && tiles <= kCounters, "split reduction: %zu bytes for %zu tiles exceed the scratch's fixed size", acc_bytes,
                   tiles);
+    // threads that share a stream slot may come here at once: whoever finds the accumulators finds zeroed counters too
+    std::lock_guard<std::mutex> lock(ctx->split_mu);
     if (!ctx->split_acc) {
         hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
         EXHIP_CHECK(hipStreamIsCapturing(ctx->stream, &capturing));
         EXHIP_REQUIRE(capturing == hipStreamCaptureStatusNone,
                       "split reduction: its scratch cannot be allocated while the stream records a graph; run the launch once before recording");
-        EXHIP_CHECK(hipMalloc(reinterpret_cast<void**>(&ctx->split_acc), kAccBytes));
-        ctx->split_acc_bytes = kAccBytes;
-        hipError_t e = hipMalloc(reinterpret_cast<void**>(&ctx->split_count), kCounters * sizeof(unsigned));
-        if (e == hipSuccess) e = hipMemset(ctx->split_count, 0, kCounters * sizeof(unsigned));  // every launch leaves its counters at zero
+        int* parts = nullptr;
+        unsigned* counters = nullptr;
+        EXHIP_CHECK(hipMalloc(reinterpret_cast<void**>(&parts), kAccBytes));
+        hipError_t e = hipMalloc(reinterpret_cast<void**>(&counters), kCounters * sizeof(unsigned));
+        if (e == hipSuccess) e = hipMemset(counters, 0, kCounters * sizeof(unsigned));  // every launch leaves its counters at zero
         if (e != hipSuccess) {
-            (void)hipFree(ctx->split_acc);
-            if (ctx->split_count) (void)hipFree(ctx->split_count);
-            ctx->split_acc = nullptr;
-            ctx->split_count = nullptr;
+            (void)hipFree(parts);
+            if (counters) (void)hipFree(counters);
             exhip_set_error("split reduction: allocating the arrival counters failed: %s", hipGetErrorString(e));
             return (int)e;
         }
-        ctx->split_count_n = kCounters;
+        ctx->split_acc = parts;
+        ctx->split_count = counters;
     }
     *acc = ctx->split_acc;
     *count = ctx->split_count;
