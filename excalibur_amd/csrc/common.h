@@ -8,7 +8,8 @@
 
 #include "../../include/exhip.h"
 
-// Pinned chunks that host <-> device copies of a context go through (transfer.hip), taken when first needed.
+// Pinned chunks that host <-> device copies of a context go through (transfer.hip), taken when first needed. A copy has one
+// of these to itself while it runs.
 struct exhip_staging {
     static constexpr int kChunks = 4;
     void* chunk[kChunks] = {};
@@ -16,13 +17,22 @@ struct exhip_staging {
     bool pending[kChunks] = {};   // uploads: the event has been recorded and not been waited for
     int at = -1;                  // uploads: the chunk being filled, and how much of it is
     size_t used = 0;
+    unsigned number = 0;          // downloads: of the last small one, the value its flag takes
+};
+
+// Those of a context that no copy uses, in one direction. Pipelines of one stream slot share a context whatever thread runs
+// them, so copies of several threads may be under way on it at once.
+struct exhip_staging_pool {
+    static constexpr int kIdle = 4;  // kept for the next copies; one thread only ever needs one
+    std::mutex mu;
+    exhip_staging* idle[kIdle] = {};
+    int n_idle = 0;
 };
 
 struct exhip_ctx {
     int device;
     hipStream_t stream;
-    exhip_staging up, down;
-    unsigned download_number = 0;  // of the last small download, the value its flag takes
+    exhip_staging_pool up, down;
     // scratch of the convolution's split reduction, allocated when first needed and kept until the context is destroyed
     std::mutex split_mu;
     int* split_acc = nullptr;

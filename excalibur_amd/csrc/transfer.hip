@@ -14,6 +14,7 @@
 #include <condition_variable>
 #include <map>
 #include <mutex>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -201,9 +202,46 @@ __global__ void __launch_bounds__(kSmallThreads) download_kernel(const char* __r
 
 int is_wide(const void* a, const void* b) { return ((uintptr_t)a | (uintptr_t)b) % 16 == 0; }
 
+void release(exhip_staging* s) {
+    for (int i = 0; i < exhip_staging::kChunks; ++i) {
+        give_chunk(s->chunk[i]);
+        if (s->event[i]) (void)hipEventDestroy((hipEvent_t)s->event[i]);
+    }
+    delete s;
+}
+
+// One copy's staging: the pool's last returned one (a thread that copies alone meets the same chunks again and again) or a new
+// one, NULL where the host has no memory for it. More than the pool keeps are only there while as many copies run; `reader` is
+// the stream whose queued work may still read the chunks when the loan ends.
+class staging_loan {
+public:
+    explicit staging_loan(exhip_staging_pool& pool, hipStream_t reader = nullptr) : pool_(pool), reader_(reader) {
+        std::lock_guard<std::mutex> g(pool_.mu);
+        staging = pool_.n_idle > 0 ? pool_.idle[--pool_.n_idle] : new (std::nothrow) exhip_staging();
+    }
+    ~staging_loan() {
+        if (!staging) return;
+        {
+            std::lock_guard<std::mutex> g(pool_.mu);
+            if (pool_.n_idle < exhip_staging_pool::kIdle) {
+                pool_.idle[pool_.n_idle++] = staging;
+                return;
+            }
+        }
+        if (reader_) (void)hipStreamSynchronize(reader_);
+        release(staging);
+    }
+    staging_loan(const staging_loan&) = delete;
+    staging_loan& operator=(const staging_loan&) = delete;
+    exhip_staging* staging;
+
+private:
+    exhip_staging_pool& pool_;
+    const hipStream_t reader_;
+};
+
 // Moves on to the next upload chunk (allocating it the first time round) and waits until its last readers are done.
-int next_chunk(exhip_ctx* ctx) {
-    exhip_staging& s = ctx->up;
+int next_chunk(exhip_ctx* ctx, exhip_staging& s) {
     if (s.at >= 0 && s.used) {
         EXHIP_CHECK(hipEventRecord((hipEvent_t)s.event[s.at], ctx->stream));
         s.pending[s.at] = true;
@@ -238,12 +276,14 @@ extern "C" int exhip_upload(exhip_ctx* ctx, void* dst, const void* src, size_t b
         EXHIP_CHECK(hipStreamSynchronize(ctx->stream));
         return 0;
     }
+    staging_loan loan(ctx->up, ctx->stream);
+    EXHIP_REQUIRE(loan.staging, "exhip_upload: no host memory");
+    exhip_staging& s = *loan.staging;
     copy_crew::session crew(bytes >= 4 * kPiece);
     while (bytes) {
-        exhip_staging& s = ctx->up;
         const size_t now = bytes < kChunk ? bytes : kChunk;
         if (s.at < 0 || s.used + now > (now <= kUploadKernel ? kSmallRing : kChunk)) {
-            const int rc = next_chunk(ctx);
+            const int rc = next_chunk(ctx, s);
             if (rc == EXHIP_ERR_UNSUPPORTED) {  // no pinned memory left: the runtime's own way
                 EXHIP_CHECK(hipMemcpyAsync(to, from, bytes, hipMemcpyHostToDevice, ctx->stream));
                 EXHIP_CHECK(hipStreamSynchronize(ctx->stream));
@@ -296,8 +336,7 @@ extern "C" int exhip_mark_destroy(void* mark) {
 }
 
 // Everything but small results: through pinned chunks, or straight into a pinned block.
-static int download(exhip_ctx* ctx, hipStream_t stream, void* dst, const void* src, size_t bytes) {
-    exhip_staging& s = ctx->down;
+static int download_through(exhip_staging& s, hipStream_t stream, void* dst, const void* src, size_t bytes) {
     auto chunk = [&](int i) {
         if (!s.chunk[i]) s.chunk[i] = take_chunk();
         return static_cast<char*>(s.chunk[i]);
@@ -335,6 +374,13 @@ static int download(exhip_ctx* ctx, hipStream_t stream, void* dst, const void* s
     return 0;
 }
 
+static int download(exhip_ctx* ctx, hipStream_t stream, void* dst, const void* src, size_t bytes) {
+    staging_loan loan(ctx->down);
+    EXHIP_REQUIRE(loan.staging, "download: no host memory");
+    const int rc = download_through(*loan.staging, stream, dst, src, bytes);
+    if (rc != 0) (void)hipStreamSynchronize(stream);  // requests may still be writing to its chunks
+    return rc;
+}
 
 // Streams for copies beside a context's own, cached for the process: one per copy in flight, kept until it ends.
 namespace {
@@ -369,31 +415,29 @@ extern "C" int exhip_memcpy_d2h_from(exhip_ctx* ctx, void* mark, void* dst, cons
 extern "C" int exhip_memcpy_d2h(exhip_ctx* ctx, void* dst, const void* src, size_t bytes) {
     EXHIP_REQUIRE(ctx && ((dst && src) || !bytes), "exhip_memcpy_d2h: NULL argument");
     if (!bytes) return 0;
-    exhip_staging& s = ctx->down;
-    auto chunk = [&](int i) {
-        if (!s.chunk[i]) s.chunk[i] = take_chunk();
-        return static_cast<char*>(s.chunk[i]);
-    };
-    if (bytes <= kDownloadKernel && chunk(0)) {
-        // the flag's line and the bytes behind it
-        auto* flag = reinterpret_cast<unsigned*>(chunk(0));
-        char* stage = chunk(0) + 256;
-        const unsigned value = ++ctx->download_number;
-        __atomic_store_n(flag, value - 1, __ATOMIC_RELAXED);
-        download_kernel<<<1, kSmallThreads, 0, ctx->stream>>>(static_cast<const char*>(src), stage, (unsigned)bytes, is_wide(src, stage), flag, value);
-        EXHIP_LAUNCH_CHECK();
-        const auto start = std::chrono::steady_clock::now();
-        for (int i = 0; __atomic_load_n(flag, __ATOMIC_ACQUIRE) != value; ++i) {
-            __builtin_ia32_pause();
-            if (i % 256 == 255 && std::chrono::steady_clock::now() - start > std::chrono::milliseconds(2)) {
-                EXHIP_CHECK(hipStreamSynchronize(ctx->stream));  // a long queue in front (or an error): wait without spinning
-                break;
-            }
+    if (bytes > kDownloadKernel) return download(ctx, ctx->stream, dst, src, bytes);
+    staging_loan loan(ctx->down);
+    EXHIP_REQUIRE(loan.staging, "exhip_memcpy_d2h: no host memory");
+    exhip_staging& s = *loan.staging;
+    if (!s.chunk[0]) s.chunk[0] = take_chunk();
+    if (!s.chunk[0]) return download_through(s, ctx->stream, dst, src, bytes);
+    // the flag's line and the bytes behind it
+    auto* flag = static_cast<unsigned*>(s.chunk[0]);
+    char* stage = static_cast<char*>(s.chunk[0]) + 256;
+    const unsigned value = ++s.number;
+    __atomic_store_n(flag, value - 1, __ATOMIC_RELAXED);
+    download_kernel<<<1, kSmallThreads, 0, ctx->stream>>>(static_cast<const char*>(src), stage, (unsigned)bytes, is_wide(src, stage), flag, value);
+    EXHIP_LAUNCH_CHECK();
+    const auto start = std::chrono::steady_clock::now();
+    for (int i = 0; __atomic_load_n(flag, __ATOMIC_ACQUIRE) != value; ++i) {
+        __builtin_ia32_pause();
+        if (i % 256 == 255 && std::chrono::steady_clock::now() - start > std::chrono::milliseconds(2)) {
+            EXHIP_CHECK(hipStreamSynchronize(ctx->stream));  // a long queue in front (or an error): wait without spinning
+            break;
         }
-        memcpy(dst, stage, bytes);
-        return 0;
     }
-    return download(ctx, ctx->stream, dst, src, bytes);
+    memcpy(dst, stage, bytes);
+    return 0;
 }
 
 // A pinned host block for results of a megabyte and more: the copy engine writes it directly. Blocks are cached for reuse
@@ -474,10 +518,6 @@ extern "C" void exhip_host_free(void* p) {
 }
 
 void exhip_release_staging(exhip_ctx* ctx) {
-    for (exhip_staging* s : {&ctx->up, &ctx->down})
-        for (int i = 0; i < exhip_staging::kChunks; ++i) {
-            give_chunk(s->chunk[i]);
-            if (s->event[i]) (void)hipEventDestroy((hipEvent_t)s->event[i]);
-            s->chunk[i] = s->event[i] = nullptr;
-        }
+    for (exhip_staging_pool* pool : {&ctx->up, &ctx->down})
+        while (pool->n_idle > 0) release(pool->idle[--pool->n_idle]);
 }

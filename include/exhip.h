@@ -31,7 +31,9 @@ extern "C" {
 #define EXHIP_ERR_ARG 10001        /* invalid argument / unsupported geometry */
 #define EXHIP_ERR_UNSUPPORTED 10002
 
-typedef struct exhip_ctx exhip_ctx; /* one device + one stream; not thread-safe, like a reference pipeline */
+/* One device + one stream. Any thread may queue work on it (the stream orders what they queue) and copy through it at any
+ * time; recording a graph, destroying it and reading results another thread queues behind are the callers' to order. */
+typedef struct exhip_ctx exhip_ctx;
 
 /* ---- runtime: replaces syncedmem's cudaMalloc/cudaMemcpy use, src/Primitives/syncedmem.cpp:176-276 ---- */
 int exhip_init(int device, exhip_ctx** ctx);

@@ -8,7 +8,7 @@
 #include "host_device.h"
 
 namespace {
-constexpr int kThreads = 4;
+constexpr int kThreads = 7;  // more than a context keeps staging for
 #define OK(call)                                                             \
     do {                                                                     \
         const int rc_ = (call);                                              \
@@ -39,12 +39,47 @@ int scratch(exhip_ctx* ctx) {
     });
     return bad + (g_mallocs - before != 2);
 }
+
+// Every thread sends bytes of its own to a block of its own and reads them back, all on one context: the sizes take each way
+// through the staging memory.
+int shared(exhip_ctx* ctx) {
+    g_copy_us = 50;
+    return on_threads([&](int t) {
+        int bad = 0;
+        void* mark = nullptr;
+        for (int i = 0; i < 12; ++i) {
+            const size_t sizes[] = {300, 75 << 10, (size_t)900 << 10, (size_t)9 << 20};
+            const size_t bytes = sizes[(i + t) % 4] + t;
+            std::vector<char> want(bytes), got(bytes);
+            for (size_t k = 0; k < bytes; ++k) want[k] = (char)(k * 7 + t * 50 + i);
+            const std::vector<char> sent = want;
+            void* dev = nullptr;
+            OK(exhip_malloc(ctx, bytes, &dev));
+            if (i % 3 == 0) OK(exhip_memcpy_h2d(ctx, dev, want.data(), bytes));
+            else OK(exhip_upload(ctx, dev, want.data(), bytes));
+            std::memset(want.data(), 0x55, bytes);  // the source may change at once
+            if (i % 3 == 1) {
+                OK(exhip_mark(ctx, &mark));
+                OK(exhip_memcpy_d2h_from(ctx, mark, got.data(), dev, bytes));
+            } else {
+                OK(exhip_memcpy_d2h(ctx, got.data(), dev, bytes));
+            }
+            if (got != sent) {
+                std::printf("thread %d copy %d of %zu bytes differs\n", t, i, bytes);
+                ++bad;
+            }
+            OK(exhip_free(ctx, dev));
+        }
+        OK(exhip_mark_destroy(mark));
+        return bad;
+    });
+}
 }  // namespace
 
 int main(int, char** argv) {
     exhip_ctx* ctx = nullptr;
     OK(exhip_init(0, &ctx));
-    const int bad = !std::strcmp(argv[1], "scratch") ? scratch(ctx) : 1;
+    const int bad = !std::strcmp(argv[1], "scratch") ? scratch(ctx) : !std::strcmp(argv[1], "shared") ? shared(ctx) : 1;
     OK(exhip_destroy(ctx));
     std::printf("%s: %s\n", argv[1], bad ? "wrong" : "ok");
     return bad != 0;

@@ -127,3 +127,41 @@ def test_threads_with_a_slot_and_a_pipeline_each():
             xp.set_stream_slot(8)
     finally:
         os.unlink(path)
+
+
+def test_threads_with_a_default_pipeline_each_share_slot_0():
+    """Nobody sets a slot: both pipelines are on one context, and each thread gets the results of its own inputs. Inputs and
+    results of a kilobyte and of megabytes take every way through the staging memory."""
+    net = ResNet18Int8(seed=27, calib_hw=32)
+    path = _model_file(net)
+    try:
+        got, errors = {}, []
+        xs = {(k, i): np.random.default_rng(28 + 10 * k + i).uniform(-1, 1, (n, 3, hw, hw)).astype(np.float32)
+              for k in range(2) for i, (n, hw) in enumerate(((1, 32), (4, 320), (1, 96)))}
+        want = {}
+        for key, x in xs.items():
+            want[key], = _solo(net, path, "f32", [x])
+
+        def work(k):
+            try:
+                p = xp.Pipeline(net.topology(), path, 0, "f32", fusion=True)
+                for turn in range(12):
+                    key = (k, (turn + k) % 3)
+                    p.set_input(xs[key])
+                    p.run()
+                    got[key] = p.get(net.output).copy()
+                    if not np.array_equal(got[key], want[key]):
+                        errors.append((key, turn))
+                p.close()
+            except Exception as e:  # surfaced in the main thread below
+                errors.append(e)
+
+        threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not errors, errors
+        assert len(got) == len(xs)
+    finally:
+        os.unlink(path)

@@ -35,3 +35,7 @@ def check(tmp_path_factory):
 
 def test_threads_that_share_a_context_get_one_split_scratch(check):
     check("scratch")
+
+
+def test_threads_that_share_a_context_copy_at_once(check):
+    check("shared")
