@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "conv_f32.h"
+#include "pack.h"
 
 namespace {
 
@@ -533,22 +534,28 @@ int exhip_conv_f32_pack_weights(const exhip_conv_desc* d, const float* w, float*
     const bool pair = d->c_stride == 4;
     const int C = d->c, K = d->k, KH = d->kh, KW = d->kw, csteps = pair ? 1 : (C + 7) / 8;
     const int taps_w = pair ? (KW + 1) / 2 : KW;
-    const size_t tap_step = (size_t)csteps * 256;  // floats between a lane's vectors of neighbouring taps
-    for (int kb = 0; kb < (K + 31) / 32; ++kb, out += KH * taps_w * tap_step)
-        for (int j = 0; j < csteps; ++j)
-            for (int lane = 0; lane < 64; ++lane) {
-                const int rr = lane % 32, h = lane / 32;
-                const int k = kb * 32 + ((rr / 4) % 2) * 16 + (rr / 8) * 4 + rr % 4;
-                const int c = pair ? 0 : j * 8 + h * 4, n = k < K ? std::max(0, std::min(4, C - c)) : 0;
-                float* const o = out + (j * 64 + lane) * 4;
-                const float* const src = n ? w + ((size_t)k * C + c) * KH * KW : w;
-                for (int e = 0; e < 4; ++e)  // a channel's taps lie side by side in the OIHW weights
-                    for (int r = 0; r < KH; ++r)
-                        for (int q = 0; q < taps_w; ++q) {
-                            const int tap = pair ? 2 * q + h : q;
-                            o[(r * taps_w + q) * tap_step + e] = e < n && tap < KW ? src[(e * KH + r) * KW + tap] : 0.f;
+    const size_t tap_step = (size_t)csteps * 256;  // floats from a tap's vectors to the next one's
+    for (int kb = 0; kb < (K + 31) / 32; ++kb, out += KH * taps_w * tap_step) {
+        auto channel = [kb](int rr) { return kb * 32 + ((rr / 4) % 2) * 16 + (rr / 8) * 4 + rr % 4; };
+        if (pair) {
+            for (int lane = 0; lane < 64; ++lane)
+                for (int r = 0; r < KH; ++r)
+                    for (int q = 0; q < taps_w; ++q)
+                        for (int e = 0; e < 4; ++e) {
+                            const int k = channel(lane % 32), tap = 2 * q + lane / 32;
+                            out[(r * taps_w + q) * tap_step + lane * 4 + e] = k < K && e < C && tap < KW ? w[(((size_t)k * C + e) * KH + r) * KW + tap] : 0.f;
                         }
-            }
+            continue;
+        }
+        for (int j = 0; j < csteps; ++j)
+            exhip_pack_block<float>(
+                [&](int rr, int half, int* n) {
+                    const int k = channel(rr), c = j * 8 + half * 4;
+                    *n = k < K ? std::max(0, std::min(4, C - c)) : 0;
+                    return *n ? w + ((size_t)k * C + c) * KH * KW : w;
+                },
+                KH * KW, reinterpret_cast<char*>(out + j * 256), tap_step * 4);
+    }
     return 0;
 }
 

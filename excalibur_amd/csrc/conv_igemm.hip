@@ -30,6 +30,7 @@
 #include "conv_f32.h"
 #include "conv_i8_lean.h"
 #include "conv_pw.h"
+#include "pack.h"
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
@@ -1860,39 +1861,37 @@ int run_conv(exhip_ctx* ctx, const exhip_conv_desc* d, ConvParams p, const PoolS
     return launch_variant<DT, false, 0>(ctx, pl, p, (int)grid);
 }
 
-// A lane's 16 bytes are neighbouring channels of one tap (or, packed, neighbouring taps of few channels). The taps of these
-// channels lie side by side in the OIHW weights, so they are read once, in order, and dealt out to the taps' vectors.
+// A lane's 16 bytes are neighbouring channels of one tap (or, packed, neighbouring taps of few channels).
 template <typename T>
 void pack_weights_t(const exhip_conv_desc* d, int dt, const Plan& pl, const T* w, char* out) {
     const int es = esize_of(dt), cb = d->c_stride * es, per = 16 / es;
     const int mts = pl.TM / 32;
     const int C = d->c, K = d->k, KH = d->kh, KW = d->kw, taps = KH * KW;
-    const size_t tap_step = (size_t)pl.KS * mts * 64 * per;  // elements between a lane's vectors of neighbouring taps
+    const size_t tap_bytes = (size_t)pl.KS * mts * 1024;  // from a tap's vectors to the next one's
     for (int kt = 0; kt < pl.ktiles; ++kt)
-        for (int cc = 0; cc < pl.n_chunks; ++cc)
+        for (int cc = 0; cc < pl.n_chunks; ++cc, out += (size_t)KH * pl.KWe * tap_bytes)
             for (int j = 0; j < pl.KS; ++j)
-                for (int mt = 0; mt < mts; ++mt)
-                    for (int lane = 0; lane < 64; ++lane) {
-                        const int rr = lane % 32, h = lane / 32;
-                        const int chan = ((rr / 4) % 2) * 16 + (rr / 8) * 4 + (rr % 4);
-                        const int k = kt * pl.TM + mt * 32 + chan;
-                        T* const o = reinterpret_cast<T*>(out) + ((size_t)(kt * pl.n_chunks + cc) * KH * pl.KWe) * tap_step + ((size_t)(j * mts + mt) * 64 + lane) * per;
-                        if (pl.packed) {
+                for (int mt = 0; mt < mts; ++mt) {
+                    char* const block = out + (size_t)(j * mts + mt) * 1024;
+                    auto channel = [&](int rr) { return kt * pl.TM + mt * 32 + ((rr / 4) % 2) * 16 + (rr / 8) * 4 + (rr % 4); };
+                    if (pl.packed) {
+                        for (int lane = 0; lane < 64; ++lane)
                             for (int r = 0; r < KH; ++r)
                                 for (int e = 0; e < per; ++e) {
-                                    const int byte = h * 16 + e * es, slot = byte / cb, c = (byte % cb) / es;
-                                    o[r * tap_step + e] = k < K && slot < KW && c < C ? w[(((size_t)k * C + c) * KH + r) * KW + slot] : T(0);
+                                    const int byte = lane / 32 * 16 + e * es, slot = byte / cb, c = (byte % cb) / es, k = channel(lane % 32);
+                                    const T v = k < K && slot < KW && c < C ? w[(((size_t)k * C + c) * KH + r) * KW + slot] : T(0);
+                                    memcpy(block + r * tap_bytes + lane * 16 + e * es, &v, es);
                                 }
-                            continue;
-                        }
-                        const int c = (cc * pl.chunk_b + j * 32 + h * 16) / es;
-                        const int n = k < K ? std::max(0, std::min(per, C - c)) : 0;
-                        const T* src = n ? w + ((size_t)k * C + c) * taps : w;
-                        for (int e = 0; e < n; ++e)
-                            for (int t = 0; t < taps; ++t) o[t * tap_step + e] = *src++;
-                        for (int e = n; e < per; ++e)
-                            for (int t = 0; t < taps; ++t) o[t * tap_step + e] = T(0);
+                        continue;
                     }
+                    exhip_pack_block<T>(
+                        [&](int rr, int half, int* n) {
+                            const int k = channel(rr), c = (cc * pl.chunk_b + j * 32 + half * 16) / es;
+                            *n = k < K ? std::max(0, std::min(per, C - c)) : 0;
+                            return *n ? w + ((size_t)k * C + c) * taps : w;
+                        },
+                        taps, block, tap_bytes);
+                }
 }
 
 }  // namespace
