@@ -565,6 +565,7 @@ static int run_conv_f32(exhip_ctx* ctx, const exhip_conv_desc* d, const exhip_co
     EXHIP_REQUIRE(ctx, "conv: NULL ctx");
     const int rc = exhip_conv_f32_validate(d);
     if (rc) return rc;
+    if (!place && (d->post_bn_a || d->post_bn_b || d->exact_k)) return EXHIP_ERR_UNSUPPORTED;  // the placed entry's
     EXHIP_REQUIRE(x && wp, "conv: NULL input or weights");
     const int layout = place ? place->layout : EXHIP_PLACE_ROWS, group = place ? place->group : 0;
     EXHIP_REQUIRE(layout != EXHIP_PLACE_ROWS || d->k_stride >= d->k || (!y && !residual), "conv: k_stride %d < k %d", d->k_stride, d->k);

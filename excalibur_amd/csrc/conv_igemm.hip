@@ -1664,8 +1664,8 @@ int run_conv(exhip_ctx* ctx, const exhip_conv_desc* d, ConvParams p, const PoolS
              const exhip_pw_depthwise* dw = nullptr) {
     const bool joined = d->post_bn_a || d->post_bn_b || d->exact_k || group || dw;  // what only the pointwise kernel does
     EXHIP_REQUIRE(ctx, "conv: NULL ctx");
-    // a BatchNorm in the epilogue, writes limited to the layer's own channels and grouped results: pointwise layers only (below)
-    if (joined && (pool || proj)) return EXHIP_ERR_UNSUPPORTED;
+    // a BatchNorm in the epilogue, writes limited to the layer's own channels (both int8 only) and grouped results: pointwise layers (below)
+    if (joined && (pool || proj || (DT != EXHIP_I8 && (d->post_bn_a || d->post_bn_b || d->exact_k)))) return EXHIP_ERR_UNSUPPORTED;
     Plan pl;
     int rc = make_plan(d, DT, &pl, pool);
     if (rc) return rc;
@@ -1837,7 +1837,6 @@ int run_conv(exhip_ctx* ctx, const exhip_conv_desc* d, ConvParams p, const PoolS
             g.slab_blocks = pl.TM / 32; g.slabs = pl.ktiles;
             g.act = d->act; g.post_relu = d->post_relu; g.post_op = d->post_op; g.post_slope_shared = d->post_slope_shared;
             g.post_alpha = d->post_alpha; g.post_beta = d->post_beta; g.post_slope = d->post_slope; g.residual_last = d->residual_last;
-            g.post_bn_a = d->post_bn_a; g.post_bn_b = d->post_bn_b; g.exact_k = d->exact_k;
             g.group = group; g.map_h = d->h; g.map_w = d->w;
             rc = exhip_conv1x1_f16_pw(ctx, g, reinterpret_cast<const uint16_t*>(p.x), p.wp, p.bias, reinterpret_cast<const uint16_t*>(p.residual),
                                       reinterpret_cast<uint16_t*>(p.y_q), nullptr, dw);

@@ -14,8 +14,8 @@ struct exhip_pw_geom {
     float post_alpha, post_beta;
     const float* post_slope;
     float fs_out;               // int8 layers: the scale of the requantized int8 result
-    // A BatchNorm layer in front of post_op (device arrays of k floats, both or neither), whether only channels [0, k) are
-    // written (the results point into a wider tensor; k a multiple of 32), and a detection head's groups: results go to
+    // int8 layers: a BatchNorm layer in front of post_op (device arrays of k floats, both or neither) and whether only channels [0, k) are
+    // written (the results point into a wider tensor; k a multiple of 32); a detection head's groups: results go to
     // [image][k / group][pixel][group] (map_h x map_w pixels an image). Each makes the kernel take the layer whatever its size.
     const float* post_bn_a;
     const float* post_bn_b;

@@ -249,11 +249,10 @@ __device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[
             };
             if (ANY ? shortcut && !p.residual_last : EP::res == 1) add_shortcut();
             if (ANY ? p.post_relu != 0 : EP::post == kPostRelu) relu16<!I8>(v);
-            if (ANY ? p.post_bn_a != nullptr : EP::bn) {  // the BatchNorm layer between this layer (through a Concat) and its activation layer
+            if (I8 && (ANY ? p.post_bn_a != nullptr : EP::bn)) {  // the BatchNorm layer between this layer (through a Concat) and its activation layer
                 float a[16], b[16];
                 read16<MT>(lds, 2, m, half, a);
                 read16<MT>(lds, 3, m, half, b);
-                stored16<!I8>(v);
 #pragma unroll
                 for (int e = 0; e < 16; ++e) v[e] = __builtin_fmaf(b[e], v[e], a[e]);
             }
@@ -433,7 +432,7 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
         if constexpr (DT == EXHIP_I8) par[0] = load(p.scale, at, p.K);
         par[1] = load(p.bias, at, p.K);
         if (EP::any || EP::post == kPostPrelu) par[2] = load(p.post_slope, p.post_slope_shared ? 0 : at, p.post_slope_shared ? 1 : p.K);
-        if (EP::any ? p.post_bn_a != nullptr : EP::bn) {
+        if (DT == EXHIP_I8 && (EP::any ? p.post_bn_a != nullptr : EP::bn)) {
             par[2] = load(p.post_bn_a, at, p.K);
             par[3] = load(p.post_bn_b, at, p.K);
         }
@@ -560,7 +559,7 @@ __global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParam
         if constexpr (DT == EXHIP_I8) par[0] = load(p.scale, at, p.K);
         par[1] = load(p.bias, at, p.K);
         if (EP::any || EP::post == kPostPrelu) par[2] = load(p.post_slope, p.post_slope_shared ? 0 : at, p.post_slope_shared ? 1 : p.K);
-        if (EP::any ? p.post_bn_a != nullptr : EP::bn) {
+        if (DT == EXHIP_I8 && (EP::any ? p.post_bn_a != nullptr : EP::bn)) {
             par[2] = load(p.post_bn_a, at, p.K);
             par[3] = load(p.post_bn_b, at, p.K);
         }
@@ -822,8 +821,6 @@ int pick_epilogue(exhip_ctx* ctx, const PwParams& p) {
     if constexpr (DT == EXHIP_F16) {
         if (is(0, kPostPrelu, 0, false)) return go<DT, MT, NT, U, TAPS, Ep<0, kPostPrelu, 0>>(ctx, p);
         if (is(0, kPostNone, 1, false)) return go<DT, MT, NT, U, TAPS, Ep<0, kPostNone, 1>>(ctx, p);
-        if constexpr (!TAPS)
-            if (is(0, kPostLeaky, 0, true)) return go<DT, MT, NT, U, TAPS, Ep<0, kPostLeaky, 0, true>>(ctx, p);
     } else {
         if (is(0, kPostRelu, 2, false)) return go<DT, MT, NT, U, TAPS, Ep<0, kPostRelu, 2>>(ctx, p);
         if constexpr (!TAPS)

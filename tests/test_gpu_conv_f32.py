@@ -66,3 +66,34 @@ def test_conv_f32_tiles_and_splits(ctx, tile, args):
     assert cases.check_value(got[..., :k].transpose(0, 3, 1, 2), want, 1e-5) == 0
     assert not got[..., k:].any()
     assert np.array_equal(flat[:-guard].reshape(want.shape), got[..., :k].transpose(0, 3, 1, 2))
+
+
+def test_the_plain_entry_refuses_what_only_the_placed_one_does(ctx):
+    """A BatchNorm in the epilogue and writes limited to the layer's own channels: refused, nothing written."""
+    c, k, hw = 32, 32, 5
+    x, w = ctx.array(np.ones((1, hw, hw, c), np.float32)), np.ones((k, c, 1, 1), np.float32)
+    a, b = ctx.array(np.zeros(k, np.float32)), ctx.array(np.ones(k, np.float32))
+    y = ctx.array(np.full((1, hw, hw, k), 7.0, np.float32))
+    plain = ctx.conv_desc(1, c, hw, hw, k, 1)
+    wp = ctx.pack_conv_weights(plain, hip.F32, w)
+    for d in (ctx.conv_desc(1, c, hw, hw, k, 1, post_bn=(a, b)), ctx.conv_desc(1, c, hw, hw, k, 1, exact_k=1)):
+        with pytest.raises(hip.ExhipError, match="10002"):
+            ctx.conv2d_f32(d, x, wp, None, None, y)
+    ctx.sync()
+    assert (y.download() == 7.0).all()
+    ctx.conv2d_f32(plain, x, wp, None, None, y)
+    ctx.sync()
+    assert (y.download() == c).all()
+
+
+def test_the_fp16_entry_refuses_them_too(ctx):
+    c, k, hw = 32, 32, 5
+    x, w = ctx.array(np.ones((1, hw, hw, c), np.float16).view(np.uint16)), np.ones((k, c, 1, 1), np.float16).view(np.uint16)
+    a, b = ctx.array(np.zeros(k, np.float32)), ctx.array(np.ones(k, np.float32))
+    y = ctx.array(np.full((1, hw, hw, k), 0x4700, np.uint16))
+    wp = ctx.pack_conv_weights(ctx.conv_desc(1, c, hw, hw, k, 1), hip.F16, w)
+    for d in (ctx.conv_desc(1, c, hw, hw, k, 1, post_bn=(a, b)), ctx.conv_desc(1, c, hw, hw, k, 1, exact_k=1)):
+        with pytest.raises(hip.ExhipError, match="10002"):
+            ctx.conv2d_f16(d, x, wp, None, None, y)
+    ctx.sync()
+    assert (y.download() == 0x4700).all()
