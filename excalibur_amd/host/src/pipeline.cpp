@@ -1824,7 +1824,6 @@ bool pipeline<float>::impl::build_float_plan(const tensor_ptr& input, const std:
         int unary = -1, bn = -1, prelu = -1;  // layer numbers of absorbed layers
         bool post_relu = false, residual_last = false, bn_relu = false;
         int head_reshape = -1;                // convolution: the Reshape layer of a detection head (Reshape -> Transpose) it absorbs
-        int cascade = -1, cascade_k = 0;      // max pooling: the value of a smaller pool of the same input to pool again
         enum { launch, placed, joined } join = launch;  // Concat: how its result comes about
         int into = -1, into_offset = 0;       // convolution: the joined Concat's node and the first channel there
     };
