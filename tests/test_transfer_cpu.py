@@ -39,3 +39,7 @@ def test_threads_that_share_a_context_get_one_split_scratch(check):
 
 def test_threads_that_share_a_context_copy_at_once(check):
     check("shared")
+
+
+def test_helper_threads_sleep_while_the_link_works(check):
+    check("idle")
