@@ -76,7 +76,11 @@ private:
         helpers_ = cores >= 4 ? (int)(cores / 2 < 5 ? cores / 2 : 5) : 0;  // six threads in all reach the memory's rate
     }
     void start() {
-        for (; started_ < helpers_; ++started_) std::thread([this] { help(); }).detach();
+        try {
+            for (; started_ < helpers_; ++started_) std::thread([this] { help(); }).detach();
+        } catch (...) {  // the process may have no more threads: those there are will do
+            helpers_ = started_;
+        }
     }
     bool take_one() {
         unsigned long long n = next_.load(std::memory_order_acquire);
@@ -496,14 +500,19 @@ extern "C" void* exhip_host_alloc(size_t bytes) {
     {
         const unsigned cores = std::thread::hardware_concurrency();
         const int threads = cores >= 4 ? (cores / 2 < 8 ? (int)(cores / 2) : 8) : 1;
-        std::vector<std::thread> crew;
+        std::thread crew[8];
         auto touch = [p, rounded, threads](int t) {
             for (size_t o = rounded / threads * t; o < (t + 1 == threads ? rounded : rounded / threads * (t + 1)); o += 4096)
                 static_cast<volatile char*>(p)[o] = 0;
         };
-        for (int t = 1; t < threads; ++t) crew.emplace_back(touch, t);
+        int started = 1;
+        try {
+            for (; started < threads; ++started) crew[started] = std::thread(touch, started);
+        } catch (...) {  // the process may have no more threads
+        }
         touch(0);
-        for (auto& t : crew) t.join();
+        for (int t = started; t < threads; ++t) touch(t);
+        for (int t = 1; t < started; ++t) crew[t].join();
     }
     std::lock_guard<std::mutex> g(g_pinned_mu);
     g_blocks[static_cast<char*>(p)] = {rounded};

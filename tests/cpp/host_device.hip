@@ -11,11 +11,21 @@
 #include <string>
 #include <thread>
 
+#include <dlfcn.h>
+#include <errno.h>
+#include <pthread.h>
 #include <stdlib.h>
 #include <string.h>
 #include <unistd.h>
 
 std::atomic<int> g_copy_us{0}, g_mallocs{0}, g_malloc_us{0};
+std::atomic<bool> g_no_threads{false};
+
+// libstdc++'s threads come through here
+extern "C" int pthread_create(pthread_t* thread, const pthread_attr_t* attr, void* (*start)(void*), void* arg) {
+    static const auto real = reinterpret_cast<int (*)(pthread_t*, const pthread_attr_t*, void* (*)(void*), void*)>(dlsym(RTLD_NEXT, "pthread_create"));
+    return g_no_threads ? EAGAIN : real(thread, attr, start, arg);
+}
 
 struct ihipStream_t {
     std::mutex mu;

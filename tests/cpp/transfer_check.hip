@@ -98,12 +98,27 @@ int idle(exhip_ctx* ctx) {
     OK(exhip_free(ctx, dev));
     return got[bytes - 1] != 3 || cpu_s > wall_s / 2;
 }
+
+// A process that cannot have another thread copies without helpers.
+int limit(exhip_ctx* ctx) {
+    g_no_threads = true;
+    const size_t bytes = (size_t)9 << 20;
+    std::vector<char> sent(bytes, 5), got(bytes);
+    void *dev = nullptr, *block = exhip_host_alloc(bytes);
+    OK(exhip_malloc(ctx, bytes, &dev));
+    OK(exhip_memcpy_h2d(ctx, dev, sent.data(), bytes));
+    OK(exhip_memcpy_d2h(ctx, got.data(), dev, bytes));
+    OK(exhip_free(ctx, dev));
+    const bool zero = block && static_cast<char*>(block)[bytes - 1] == 0;
+    exhip_host_free(block);
+    return got != sent || !zero;
+}
 }  // namespace
 
 int main(int, char** argv) {
     exhip_ctx* ctx = nullptr;
     OK(exhip_init(0, &ctx));
-    const int bad = !std::strcmp(argv[1], "scratch") ? scratch(ctx) : !std::strcmp(argv[1], "shared") ? shared(ctx) : !std::strcmp(argv[1], "idle") ? idle(ctx) : 1;
+    const int bad = !std::strcmp(argv[1], "scratch") ? scratch(ctx) : !std::strcmp(argv[1], "shared") ? shared(ctx) : !std::strcmp(argv[1], "idle") ? idle(ctx) : !std::strcmp(argv[1], "limit") ? limit(ctx) : 1;
     OK(exhip_destroy(ctx));
     std::printf("%s: %s\n", argv[1], bad ? "wrong" : "ok");
     return bad != 0;

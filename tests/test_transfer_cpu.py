@@ -24,7 +24,7 @@ def check(tmp_path_factory):
     with ThreadPoolExecutor() as pool:
         list(pool.map(build, zip(sources, objects)))
     exe = str(tmp / "transfer_check")
-    subprocess.check_call(["g++", "-pthread", "-Wl,--allow-multiple-definition", "-o", exe] + objects)
+    subprocess.check_call(["g++", "-pthread", "-Wl,--allow-multiple-definition", "-rdynamic", "-o", exe] + objects + ["-ldl"])
 
     def run(name):
         out = subprocess.run([exe, name], capture_output=True, text=True, timeout=120)
@@ -43,3 +43,7 @@ def test_threads_that_share_a_context_copy_at_once(check):
 
 def test_helper_threads_sleep_while_the_link_works(check):
     check("idle")
+
+
+def test_a_process_at_its_thread_limit_copies_without_helpers(check):
+    check("limit")
