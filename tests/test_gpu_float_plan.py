@@ -114,3 +114,85 @@ def test_float_plan_equals_the_layers_bit_for_bit(focus):
         planned.close()
         plain.close()
         os.unlink(path)
+
+
+def pooled_slices():
+    """Two producers of a Concat whose slices have other readers too: pools of a slice, one of them inside another Concat. No layer
+    fixes the input size."""
+    r = np.random.default_rng(73)
+    lines, blobs = ["Input data 0 1 data 0=32 1=32 2=3 3=0,0,0 4=1"], []
+
+    def conv(bottom, top, cin, k, kernel=1, stride=1, act=0):
+        w = r.normal(0, np.sqrt(2.0 / (cin * kernel * kernel)), (k, cin, kernel, kernel)).astype(np.float32)
+        lines.append(mf.conv_line("Convolution", top + "_l", bottom, top, k, kernel, stride, kernel // 2, True, w.size, act=act))
+        blobs.append(mf.conv_blob_f32(w, r.normal(0, 0.5, (k,)).astype(np.float32)))
+
+    conv("data", "c0", 3, 16, 3, 2)
+    lines.append("Split c0_s 1 2 c0 c00 c01")
+    conv("c00", "y1", 16, 24, act=1)
+    conv("c01", "y2", 16, 40, 3)
+    lines.append("Split y1_s 1 3 y1 y10 y11 y12")
+    lines.append("Concat cat_l 2 1 y10 y2 cat 0=-1")
+    lines.append(mf.pool_line("mp", "y11", "mp", 0, 3, 1, 1))
+    lines.append(mf.pool_line("av", "y12", "av", 1, 3, 2, 1, count_include_pad=1))
+    conv("cat", "c1", 64, 24)
+    lines.append("Concat cat2_l 2 1 c1 mp cat2 0=-1")
+    conv("cat2", "c2", 48, 16, 3)
+    return lines, blobs, ["c2", "av"]
+
+
+@pytest.fixture
+def pair():
+    lines, blobs, outs = pooled_slices()
+    with tempfile.NamedTemporaryFile(suffix=".racy", delete=False) as f:
+        path = f.name
+    mf.write_model(path, blobs)
+    pipes = [xp.Pipeline(mf.topology(lines, "slices"), path, 0, fusion=on) for on in (True, False)]
+    os.unlink(path)
+    yield (*pipes, outs)
+    for p in pipes:
+        p.close()
+
+
+def inputs(shape, seed):
+    return np.random.default_rng(seed).uniform(-2, 2, shape).astype(np.float32)
+
+
+def test_float_plan_with_alternating_input_sizes(pair):
+    planned, plain, outs = pair
+    sizes = [(1, 3, 32, 32), (2, 3, 21, 46), (1, 3, 33, 17), (2, 3, 21, 46), (1, 3, 32, 32), (3, 3, 32, 32)]
+    for seed, shape in enumerate(sizes):
+        x = inputs(shape, seed)
+        planned.forward(x)
+        plain.forward(x)
+        assert not planned.stored("y2") and plain.stored("y2")
+        for o in outs:
+            got, want = planned.get(o), plain.get(o)
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32)) and np.ptp(want) > 0, (shape, o)
+
+
+def test_float_plan_replayed_as_a_graph(pair):
+    """Every replay against the eager layers, with their work between the replays; another size in the middle."""
+    planned, plain, outs = pair
+    planned.set_graphs(True)
+    for seed, shape in enumerate([(2, 3, 30, 28)] * 4 + [(1, 3, 32, 32)] * 3 + [(2, 3, 30, 28)] * 3):
+        x = inputs(shape, 20 + seed)
+        planned.forward(x)
+        plain.forward(x)
+        for o in outs:
+            assert np.array_equal(planned.get(o).view(np.uint32), plain.get(o).view(np.uint32)), (seed, o)
+
+
+def test_float_plan_results_held_across_forwards(pair):
+    planned, plain, outs = pair
+    shape, want = (2, 3, 40, 36), []
+    for seed in range(4):
+        x = inputs(shape, 40 + seed)
+        planned.set_input(x)
+        planned.run_keeping()
+        plain.forward(x)
+        want.append({o: plain.get(o).copy() for o in outs})
+    for o in outs:
+        assert np.array_equal(planned.get(o), want[3][o])
+        for back in (1, 2, 3):
+            assert np.array_equal(planned.get_kept(back, o), want[3 - back][o]), (back, o)

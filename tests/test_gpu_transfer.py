@@ -83,3 +83,31 @@ def test_results_in_pool_blocks_stay_their_holder_s(ctx):
     assert np.array_equal(view, np.arange(10, 20, dtype=np.float32))
     assert hip.lib().exhip_host_alloc((1 << 30) + 1) is None   # beyond the bound: the caller's own memory
     d.free()
+
+
+@pytest.mark.parametrize("size", [5, 64 * KB, 256 * KB + 1, 5 * MB + 3, 19 * MB])
+@pytest.mark.parametrize("pinned", [False, True])
+def test_a_marked_result_leaves_while_the_stream_goes_on(ctx, size, pinned):
+    """What was written before the mark arrives whatever is queued behind it; a mark is recorded anew for the next result."""
+    L = hip.lib()
+    xp.lib()
+    d, other = ctx.empty((size,), np.uint8), ctx.empty((64 * MB,), np.uint8)
+    mark = ctypes.c_void_p()
+    out = xp._host_array((max(size, MB),), np.uint8) if pinned else np.empty(size, np.uint8)
+    kept = None
+    for turn in range(3):
+        want = np.random.default_rng(size + turn).integers(0, 256, size, dtype=np.uint8)
+        hip._check(L.exhip_upload(ctx.h, d.ptr, want.ctypes.data_as(ctypes.c_void_p), ctypes.c_size_t(size)))
+        hip._check(L.exhip_mark(ctx.h, ctypes.byref(mark)))
+        assert kept is None or mark.value == kept
+        kept = mark.value
+        for value in range(40):
+            hip._check(L.exhip_memset(ctx.h, other.ptr, value, ctypes.c_size_t(other.nbytes)))
+        out[:] = 0
+        hip._check(L.exhip_memcpy_d2h_from(ctx.h, mark, out.ctypes.data_as(ctypes.c_void_p), d.ptr, ctypes.c_size_t(size)))
+        assert np.array_equal(out[:size], want) and not out[size:].any()
+        assert (other.download() == 39).all()
+    assert L.exhip_memcpy_d2h_from(ctx.h, None, out.ctypes.data_as(ctypes.c_void_p), d.ptr, ctypes.c_size_t(size)) == 10001
+    hip._check(L.exhip_mark_destroy(mark))
+    d.free()
+    other.free()
