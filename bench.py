@@ -102,9 +102,9 @@ def measured_traffic(n, hw):
 
 
 def network_table(iters=10, only=None):
-    """The generated topologies of the other configurations through pipeline<float> / pipeline<unsigned short> (float32 and
-    fp16: layer by layer with the executor's joins; int8: the int8 graph plan where it takes the network, which the row's
-    "executor" says), input resident on the device: wall time per forward over `iters` forwards, device drained before and
+    """The generated topologies of the other configurations through pipeline<float> / pipeline<unsigned short> (float32: the
+    float plan, int8: the int8 graph plan where they take the network, which the row's "executor" says; fp16: layer by layer with
+    the executor's joins), input resident on the device: wall time per forward over `iters` forwards, device drained before and
     after. Returns [{"network", "dtype", "executor", "ms", "images/s", ...}]."""
     import tempfile
     from excalibur_amd import pipeline as xp
@@ -130,9 +130,12 @@ def network_table(iters=10, only=None):
             p.run()
         p.sync()
         ms = (time.perf_counter() - t0) / iters * 1e3
-        executor = "int8 graph plan" if p.fused else "per-layer"
-        p.close()
         from excalibur_amd import topologies
+        from excalibur_amd.modelfile import parse_topology
+        layers = parse_topology(net.topology())   # a plan stores a blob or two between the layers, the per-layer executor most of them
+        inner = {t for l in layers for t in l.tops} & {b for l in layers for b in l.bottoms}
+        executor = "int8 graph plan" if p.fused else "per-layer" if 2 * sum(p.stored(b) for b in inner) > len(inner) else "float plan"
+        p.close()
         gop = topologies.algorithmic_gop(net.topology(), x.shape[1:]) * x.shape[0]   # of the whole batch
         peak = {"f32": PEAK_F32_TFLOPS, "f16": PEAK_F16_TFLOPS, "int8": PEAK_INT8_TOPS}[dtype]
         rows.append({"network": label, "dtype": dtype, "layers": len(net.lines), "executor": executor, "ms": round(ms, 3),

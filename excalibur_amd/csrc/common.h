@@ -103,7 +103,7 @@ struct exhip_options {
     int f32_tile = 0;        // the float32 convolution's wave tile and split: 0 by its rule, n = the n-th of its list
     int dw_pw = 1;           // depthwise + pointwise fp16 pairs in one kernel: 1 by its rule, 2 wherever it can run, 0 never
     int pw_split = 1;        // that kernel's split form (several waves to a tile): 1 by its rule, 2 wherever it can run, 0 never
-    int pw = 1;              // 1x1 stride-1 fp16 layers with an NHWC result: 1 the pointwise kernel where it measured faster, 2 wherever it can run, 0 never
+    int pw = 1;              // 1x1 stride-1 fp16 and int8 layers with NHWC results: 1 the pointwise kernel where it measured faster, 2 wherever it can run, 0 never
 };
 extern exhip_options g_exhip_options;
 extern unsigned g_exhip_options_version;  // counts exhip_set_option calls: what was planned under other options is planned again

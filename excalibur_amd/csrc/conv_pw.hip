@@ -1,17 +1,21 @@
-// conv1x1_f16_pw_kernel: the pointwise (1x1, stride 1, no padding) fp16 convolution, y[pixel][k] = sum_c x[pixel][c] * w[k][c].
+// conv1x1_pw_kernel: the pointwise (1x1, stride 1, no padding) convolution on half or int8 NHWC tensors, y[pixel][k] = sum_c x[pixel][c]
+// * w[k][c]; its tapped form (TAPS) for layers with a filter, a stride or padding; conv_pw_split_kernel, several waves to a tile; and
+// dw_pw_kernel, a depthwise 3x3 layer in front.
 //
 // A pointwise layer of a detection or mobile network moves a few tens of MB for a few GFLOP: what it costs is the
-// length of one group's chain from launch to last store, and the memory system's rate. So nothing is staged: a wave
+// length of one group's chain from launch to last store, and the memory system's rate. So no operand is staged: a wave
 // owns 32 * NT pixels x 32 * MT output channels and fetches its MFMA operands straight into registers, 16 bytes per
 // lane and k-step -- the weight fragments in the general kernel's packing (one contiguous KiB per 32-channel block and
 // k-step), the pixel fragments from the NHWC rows themselves (lane = pixel, the two half-waves the two 16-byte halves
-// of a 32-byte k-step). No LDS, no barrier, no tile geometry: the pixels of all images form one list. The four waves of
+// of a 32-byte k-step). No barrier, no tile geometry: the pixels of all images form one list. LDS holds what a wave keeps to
+// itself, its channels' parameters and its results on their way to whole rows. The four waves of
 // a group are neighbours in (pixel tile, channel group) order with the channel group running fastest, so the waves that
 // read the same pixels sit on one CU; the pixel rows come from HBM once and from the caches after that.
 //
 // Arithmetic and roundings are the general kernel's (conv_igemm.hip, general epilogue): float32 accumulation in
 // v_mfma_f32_32x32x16_f16, bias, activation, the optional shortcut added to the value rounded to half, ReLU / the
-// activation layer behind the convolution applied to the rounded half, one final rounding.
+// activation layer behind the convolution applied to the rounded half, one final rounding. (The split form adds its waves' sums
+// in an order of its own, the same every time.)
 //
 // The int8 layer (DT == EXHIP_I8) is the same kernel on the same byte geometry -- a 32-byte k-step is 32 int8 channels,
 // v_mfma_i32_32x32x32_i8 on the same 16-byte fragments -- with the int8 epilogue of the general kernel: dequantization
@@ -913,7 +917,7 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
     // kernel leaves (stride 2, 12 or 32 input channels, ragged output channels) are faster here as a whole (0.88 -> 0.85 ms
     // and 1.83 -> 1.81 ms per forward of the detection networks); of the int8 layers only a few deep ones are (3x3
     // stride 2 from 40 x 40: 29 -> 23 us) while the wide first layers lose (12 -> 32 channels at 320 x 320: 81 -> 94 us),
-    // so int8 layers stay with the staged kernels unless the option asks.
+    // so wide int8 layers stay with the staged kernels unless the option asks or the split form takes them.
     // A lone 32-channel block wins whatever its size (12 -> 32 at 16 x 320 x 320: int8 71 -> 46 us, fp16 66 -> 45; 32 -> 32 at
     // 160 x 160: one image 8.1 -> 5.3 us, sixteen 24.9 -> 15.8).
     const bool take = kblocks == 1 || DT == EXHIP_F16 || g.c_bytes == 32 || (g.pixels <= 32768 && kblocks <= 4) || g.pixels <= 6400;

@@ -1,4 +1,5 @@
-// exhip runtime: context, memory, events. Everything runs on one stream per context.
+// exhip runtime: context, memory, events. Everything runs on one stream per context (but for results that leave while it goes
+// on, transfer.hip).
 #include <stdarg.h>
 #include <string.h>
 
