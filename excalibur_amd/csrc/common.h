@@ -130,6 +130,20 @@ inline void exhip_host_divisor(unsigned d, unsigned* magic, int* shift) {
 }
 
 // ---- device helpers shared by the kernels ----
+// Reads one word of every 64 bytes of a kernel's argument struct, all of them before the first wait. The arguments of a launch
+// lie in memory that no cache has seen yet, and the compiler asks for them where they are used: one line, a wait of 500 to 800
+// cycles, some address arithmetic, the next line. Asked for together they arrive in the time of one (the address phase of a
+// small float32 convolution 3000 -> 1300 cycles of 14 100 in all, of an int8 one in four waves to a tile 1500 -> 900 of 7000).
+template <typename P>
+__device__ __forceinline__ void exhip_touch_args(const P& p) {
+#ifdef __HIP_DEVICE_COMPILE__
+    const int* const w = reinterpret_cast<const int*>(&p);
+    constexpr int kWords = sizeof(P) / 4;
+    constexpr auto at = [](int line) { return line * 16 < kWords ? line * 16 : kWords - 1; };
+    asm volatile("" ::"s"(w[at(0)]), "s"(w[at(1)]), "s"(w[at(2)]), "s"(w[at(3)]), "s"(w[at(4)]), "s"(w[at(5)]), "s"(w[at(6)]), "s"(w[at(7)]),
+                 "s"(w[at(8)]), "s"(w[at(9)]), "s"(w[at(10)]), "s"(w[at(11)]), "s"(w[at(12)]), "s"(w[at(13)]));
+#endif
+}
 typedef int exhip_v4i __attribute__((ext_vector_type(4)));
 // Stores reach full speed with runs of 64 contiguous bytes from neighbouring lanes (measured: 32-byte runs take twice as
 // long), so two pixels in neighbouring lanes trade halves: afterwards `a` holds, in the even lane, its own a and, in the

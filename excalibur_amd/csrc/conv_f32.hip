@@ -250,6 +250,7 @@ __device__ __forceinline__ void epilogue_block(const F32Params& p, const v16f& a
 // R: requested steps in flight.
 template <int MT, int NT, int WK, int R, int MODE, bool SLOW>
 __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256, 2) void conv_f32_kernel(const F32Params p) {
+    exhip_touch_args(p);
     constexpr int WAVES = WK > 4 ? WK : 4, ITEMS = WAVES / WK;  // tiles per group
     constexpr int RED = WK > 1 ? WAVES * MT * NT * 4096 : 0;    // the waves' partial sums
     constexpr int OWNERS = MT * NT < WK ? MT * NT : WK;         // waves of a tile that run the epilogue

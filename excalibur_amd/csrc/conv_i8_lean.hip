@@ -113,6 +113,7 @@ __device__ __forceinline__ void wait_vmcnt() { __asm__ volatile("s_waitcnt vmcnt
 // run as stages of one tap, into accumulators of their own.
 template <bool WRES, int NAB, int NWB, int EPI, bool PROJ = false>
 __global__ __launch_bounds__(kThreads, (WRES || NAB == 2 || NWB == 3 || PROJ) ? 2 : 3) void conv3x3_i8_lean_kernel(const LeanParams p) {
+    exhip_touch_args(p);
     static_assert(!(PROJ && WRES), "the projection's chunks run in the streamed form");
     constexpr int NWS = WRES ? 3 : NWB;
     constexpr int A0 = NWS * kWSlice;
@@ -855,6 +856,7 @@ __global__ __launch_bounds__(kThreads, (WRES || NAB == 2 || NWB == 3 || PROJ) ? 
 // slice buffers (or the resident filter), two activation tile buffers, 64 KiB for the accumulators.
 template <bool WRES, int EPI>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void conv3x3_i8_ws_kernel(const LeanParams p) {
+    exhip_touch_args(p);
     constexpr int A0 = 3 * kWSlice;
     constexpr int H0 = A0 + 2 * kActStride;          // accumulators on their way to the epilogue waves: 4 x 16 KiB
     constexpr int SB0 = H0 + 4 * 16384;

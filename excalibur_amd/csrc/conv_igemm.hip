@@ -261,6 +261,7 @@ __device__ __forceinline__ void post_activation4(v4f& v, int op, float alpha, fl
 // LOWREG: held to 128 registers (a few spills) so that two 512-thread groups can share a CU.
 template <int DT, int MT, int NT, int WM, int WN, bool PACKED, int EPI, int KWE, int KSC, bool LOWREG = false>
 __global__ __launch_bounds__(64 * WM * WN, (MT * NT > 4 ? 1 : (LOWREG ? 4 : 2))) void conv_igemm_kernel(const ConvParams p) {
+    exhip_touch_args(p);
     constexpr int THREADS = 64 * WM * WN;
     constexpr int TM = 32 * MT * WM;
     // staging limits scale with the group size so that a 512-thread group needs half the registers

@@ -326,6 +326,7 @@ __device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[
 // U: k-steps per request round; two rounds are in flight.
 template <int DT, int MT, int NT, int U, bool TAPS, typename EP>
 __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
+    exhip_touch_args(p);
     __shared__ __attribute__((aligned(16))) char lds_all[4 * wave_bytes(DT, MT)];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // workgroup ids are dealt round-robin to the 8 XCDs: give each XCD one contiguous run of items, so that the channel
@@ -472,6 +473,7 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
 // flight; those past a wave's run ask for operands it does not use.
 template <int DT, int MT, int WK, bool TAPS, typename EP>
 __global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParams p) {
+    exhip_touch_args(p);
     constexpr int R = 8;  // k-steps in flight
     constexpr int RED = WK * MT * 4096;
     static_assert(MT <= WK && WK <= kSplit, "a wave per block");
@@ -642,6 +644,7 @@ typedef int v2i __attribute__((ext_vector_type(2)));
 
 template <int S, int PX, typename EP>
 __global__ __launch_bounds__(256, 3) void dw_pw_kernel(const PwParams p) {
+    exhip_touch_args(p);
     constexpr int R = 4, NC = (PX - 1) * S + 3;
     constexpr unsigned kRowOutside = 0x80000000u, kColOutside = 0x40000000u;  // tensors of at most 2^30 bytes: beyond the view, alone or together
     extern __shared__ __attribute__((aligned(16))) char lds_dyn[];
