@@ -44,9 +44,10 @@ struct F32Params {
     const char* wp;
     const float *bias, *residual, *slope, *bn_a, *bn_b;
     float *y, *y_nchw;
-    unsigned pixels, x_bytes, w_bytes, tiles, items, ch_groups;
-    unsigned groups_magic, image_magic, width_magic;  // exhip_divide() by ch_groups, out_h * out_w, out_w
-    int groups_shift, image_shift, width_shift;
+    unsigned pixels, x_bytes, w_bytes, items;
+    unsigned fast;                 // the channel groups or (tiles_fast) the pixel tiles, whichever neighbouring items walk
+    unsigned fast_magic, image_magic, width_magic;  // exhip_divide() by fast, out_h * out_w, out_w
+    int fast_shift, image_shift, width_shift, tiles_fast;
     int in_h, in_w, out_h, out_w, stride, pad_t, pad_l, kh, kw;
     int xs_b, row_b;               // bytes per input pixel and input row
     int csteps, n_ksteps;          // steps per tap (kPair: 1) and in all
@@ -247,18 +248,124 @@ __device__ __forceinline__ void epilogue_block(const F32Params& p, const v16f& a
     }
 }
 
+// The epilogue of a tile that WK waves share: V channels from ch0 on of the lane's pixel. Each wave takes an equal part of the tile, so
+// that its chain is short, and stores from registers: a launch that splits its tiles is small, and the waves fill the same lines.
+// (One wave finished a whole block before, 2400 to 5300 cycles of a launch's 10 000 to 16 000: 512 -> 512 1x1 on three 13 x 13 maps
+// 6.9 -> 6.5 us, 32 -> 64 3x3 at stride 2 on three 104 x 104 maps 7.5 -> 7.1, 256 -> 128 1x1 on three 26 x 26 maps 5.8 -> 5.3.)
+template <int V>
+__device__ __forceinline__ void epilogue_part(const F32Params& p, float (&v)[V], const float (&par)[kParams][V], const float (&res)[V], unsigned pix, unsigned img,
+                                              unsigned in_image, int ch0) {
+    const unsigned per_image = (unsigned)(p.out_h * p.out_w);
+    auto relu = [&]() {
+#pragma unroll
+        for (int e = 0; e < V; ++e) v[e] = (0.f > v[e]) ? 0.f : v[e];
+    };
+    auto each = [&](auto op) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) v[e] = unary_value<decltype(op)::value>(v[e], p.alpha, p.beta);
+    };
+#pragma unroll
+    for (int e = 0; e < V; ++e) v[e] += par[0][e];
+    if (p.act == 1) relu();
+    if (p.act == 3) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) v[e] = exhip_act(v[e], 3);
+    }
+    if (p.residual && !p.residual_last) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) v[e] += res[e];
+    }
+    if (p.post_relu) relu();
+    if (p.bn_a) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) v[e] = __builtin_fmaf(par[3][e], v[e], par[2][e]);
+        if (p.bn_relu) relu();
+    }
+    switch (p.post_op) {
+    case 0: break;
+    case 1 + EXHIP_UNARY_HARDSWISH: each(std::integral_constant<int, 0>{}); break;
+    case 1 + EXHIP_UNARY_LEAKYRELU: each(std::integral_constant<int, 1>{}); break;
+    case 1 + EXHIP_UNARY_HARDSIGMOID: each(std::integral_constant<int, 3>{}); break;
+    case 1 + EXHIP_UNARY_CLIP: each(std::integral_constant<int, 4>{}); break;
+    default:
+#pragma unroll
+        for (int e = 0; e < V; ++e) v[e] = v[e] >= 0.f ? v[e] : par[1][e] * v[e];
+    }
+    if (p.residual && p.residual_last) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) v[e] += res[e];
+    }
+    if (pix >= p.pixels) return;
+    if (p.y) {
+#pragma unroll
+        for (int e = 0; e < V; ++e)
+            if (ch0 + e >= p.K) v[e] = 0.f;  // pad channels hold zeros
+        if (p.layout == EXHIP_PLACE_GROUPED) {
+            // y[img][group][pixel][member]
+            float* const to = p.y + (size_t)img * (unsigned)p.K * per_image + (size_t)in_image * (unsigned)p.group;
+            int g = ch0 / p.group, member = ch0 - g * p.group;
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+                if (ch0 + e < p.K) to[(size_t)g * per_image * (unsigned)p.group + member] = v[e];
+                if (++member == p.group) member = 0, ++g;
+            }
+        } else {
+            float* to = p.y + (size_t)pix * (unsigned)p.kstride + ch0;
+            int end = p.k_end, ch = ch0;
+            if (p.layout == EXHIP_PLACE_SHUFFLED && p.vector_rows) {
+                // channel pos * group + k of pixel (y, x) is channel k of pixel (2 y + pos / 2, 2 x + pos % 2) of a map twice as large
+                const unsigned oy = exhip_divide(in_image, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = in_image - oy * (unsigned)p.out_w;
+                const int pos = ch0 / p.group;
+                const unsigned at = (img * 2 * (unsigned)p.out_h + 2 * oy + (pos >> 1)) * 2 * (unsigned)p.out_w + 2 * ox + (pos & 1);
+                to = p.y + (size_t)at * (unsigned)p.kstride + (ch0 - pos * p.group);
+                end = p.K;
+            }
+            if (p.layout == EXHIP_PLACE_SHUFFLED && !p.vector_rows) {
+                const unsigned oy = exhip_divide(in_image, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = in_image - oy * (unsigned)p.out_w;
+                const unsigned corner = (img * 2 * (unsigned)p.out_h + 2 * oy) * 2 * (unsigned)p.out_w + 2 * ox;
+#pragma unroll
+                for (int e = 0; e < V; ++e) {
+                    const int pos = (ch0 + e) / p.group, k = ch0 + e - pos * p.group;
+                    if (ch0 + e < p.K) p.y[(size_t)(corner + (unsigned)(pos >> 1) * 2 * (unsigned)p.out_w + (pos & 1)) * (unsigned)p.kstride + k] = v[e];
+                }
+            } else if (p.vector_rows) {
+#pragma unroll
+                for (int e = 0; e < V; e += 4)
+                    if (ch + e < end) *reinterpret_cast<v4f*>(to + e) = v4f{v[e], v[e + 1], v[e + 2], v[e + 3]};
+            } else {
+#pragma unroll
+                for (int e = 0; e < V; ++e)
+                    if (ch + e < end) to[e] = v[e];
+            }
+        }
+    }
+    if (p.y_nchw) {  // 32 neighbouring pixels of a channel per store instruction and half-wave
+        float* const dst = p.y_nchw + ((size_t)img * p.K + ch0) * per_image + in_image;
+#pragma unroll
+        for (int e = 0; e < V; ++e)
+            if (ch0 + e < p.K) dst[(size_t)e * per_image] = v[e];
+    }
+}
+
 // R: requested steps in flight.
 template <int MT, int NT, int WK, int R, int MODE, bool SLOW>
 __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256, 2) void conv_f32_kernel(const F32Params p) {
     exhip_touch_args(p);
     constexpr int WAVES = WK > 4 ? WK : 4, ITEMS = WAVES / WK;  // tiles per group
-    constexpr int RED = WK > 1 ? WAVES * MT * NT * 4096 : 0;    // the waves' partial sums
-    constexpr int OWNERS = MT * NT < WK ? MT * NT : WK;         // waves of a tile that run the epilogue
-    __shared__ __attribute__((aligned(16))) char lds_all[RED + ITEMS * OWNERS * wave_lds(MT)];
+    constexpr int BLOCKS = MT * NT;
+    constexpr int QUADS = 4 * BLOCKS > WK ? 4 * BLOCKS / WK : 1;  // WK > 1: quarters of a block (four channels a lane) that a wave finishes
+    constexpr int V = 4 * QUADS;
+    // A wave that finishes a whole block stores its rows through LDS, one that finishes less from registers: a split launch of two
+    // waves to a tile is still a large one (32 -> 64 3x3 on a 320 x 320 map: 47 us, 52 with stores from registers).
+    constexpr bool ROWS = WK == 1 || QUADS == 4;
+    constexpr int RED = WK > 1 ? WAVES * BLOCKS * 4096 : 0;       // the waves' partial sums
+    static_assert(QUADS <= 4 || WK == 1, "a wave finishes at most one block");
+    __shared__ __attribute__((aligned(16))) char lds_all[RED + (ROWS ? WAVES * wave_lds(MT) : 0)];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int part = wave % WK;
-    // workgroup ids are dealt round-robin to the 8 XCDs: give each XCD one contiguous run of items, so that the channel
-    // groups of a pixel tile, neighbouring tiles and the weights' re-reads share that XCD's L2
+    // workgroup ids are dealt round-robin to the 8 XCDs: give each XCD one contiguous run of items. Either the channel groups of
+    // a pixel tile run fastest, and an XCD reads its share of the pixels and all weights, or the pixel tiles do (tiles_fast)
+    // and it reads its share of the weights and all pixels.
     unsigned bid = blockIdx.x;
     {
         const unsigned per = gridDim.x >> 3;
@@ -267,14 +374,15 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256, 2) void conv_f32_kernel(con
     const unsigned item = __builtin_amdgcn_readfirstlane(bid * ITEMS + wave / WK);
     if (WK == 1 && item >= p.items) return;  // wave-uniform; that form has no barrier
     const bool on = item < p.items;
-    const unsigned tile = __builtin_amdgcn_readfirstlane(exhip_divide(item, p.ch_groups, p.groups_magic, p.groups_shift));
-    const int kb0 = __builtin_amdgcn_readfirstlane((int)(item - tile * p.ch_groups) * MT);  // first 32-channel block
-    char* const lds = lds_all + RED + (wave / WK * OWNERS + (part < OWNERS ? part : 0)) * wave_lds(MT);
+    const unsigned slow = exhip_divide(item, p.fast, p.fast_magic, p.fast_shift), fast = item - slow * p.fast;
+    const unsigned tile = __builtin_amdgcn_readfirstlane(p.tiles_fast ? fast : slow);
+    const int kb0 = __builtin_amdgcn_readfirstlane((int)(p.tiles_fast ? slow : fast) * MT);  // first 32-channel block
 
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.x), 0, (int)p.x_bytes, kRsrcWord3);
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.wp), 0, (int)p.w_bytes, kRsrcWord3);
 
     // pixel fragments: lane = pixel (lane & 31), 16-byte half (lane >> 5) of each step
+    const unsigned per_image = (unsigned)(p.out_h * p.out_w);
     unsigned xoff[NT];
     int iy[NT], ix[NT];
 #pragma unroll
@@ -286,7 +394,6 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256, 2) void conv_f32_kernel(con
         } else {
             // the filter's top-left input pixel; its offset may lie in front of the tensor (padding), the taps inside the
             // image never do, and 32-bit wrap-around of the sum gives their offsets
-            const unsigned per_image = (unsigned)(p.out_h * p.out_w);
             const unsigned img = exhip_divide(pix, per_image, p.image_magic, p.image_shift), rem = pix - img * per_image;
             const int oy = (int)exhip_divide(rem, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = (int)(rem - (unsigned)oy * (unsigned)p.out_w);
             iy[n] = oy * p.stride - p.pad_t;
@@ -368,19 +475,28 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256, 2) void conv_f32_kernel(con
     };
 #pragma unroll
     for (int u = 0; u < R / 2; ++u) request(u);
-    // the channels' parameters: lane = channel of the wave's MT * 32, zeros beyond K and for an absent array
-    float par[kParams] = {};
-    {
-        auto load = [&](const float* src, unsigned offset, int count) {
+    // WK > 1: what a wave finishes of the tile -- channels ch0 .. ch0 + V - 1 of a pixel per lane -- and their parameters;
+    // ROWS: the parameters lane by lane, of the wave's MT * 32 channels
+    const int quad = part * QUADS, half = lane >> 5;
+    const bool owner = on && quad < 4 * BLOCKS;
+    const int own_ch = (kb0 + quad / 4 % MT) * 32 + half * 16 + quad % 4 * 4;
+    const unsigned own_pix = (tile * NT + quad / 4 / MT) * 32 + (lane & 31);
+    constexpr int PV = ROWS ? 1 : V;
+    float par[kParams][PV] = {};
+    auto load_parameters = [&]() {
+        const unsigned at = (unsigned)(ROWS ? kb0 * 32 + lane : own_ch) * 4;
+        auto load = [&](int i, const float* src, unsigned offset, int count, int step) {
+            if (!ROWS && !src) return;
             const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src), 0, src ? count * 4 : 0, kRsrcWord3);
-            return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)offset, 0, 0));
+#pragma unroll
+            for (int e = 0; e < PV; ++e) par[i][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)offset + e * step, 0, 0));
         };
-        const unsigned at = (unsigned)(kb0 * 32 + lane) * 4;
-        par[0] = load(p.bias, at, p.K);
-        par[1] = load(p.slope, p.slope_shared ? 0 : at, p.slope_shared ? 1 : p.K);
-        par[2] = load(p.bn_a, at, p.K);
-        par[3] = load(p.bn_b, at, p.K);
-    }
+        load(0, p.bias, at, p.K, 4);
+        load(1, p.slope, p.slope_shared ? 0 : at, p.slope_shared ? 1 : p.K, p.slope_shared ? 0 : 4);
+        load(2, p.bn_a, at, p.K, 4);
+        load(3, p.bn_b, at, p.K, 4);
+    };
+    if (ROWS) load_parameters();
 #pragma unroll
     for (int u = R / 2; u < R; ++u) request(u);
     int s = 0;
@@ -393,9 +509,11 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256, 2) void conv_f32_kernel(con
         }
     }
     // (the loop leaves with the last steps, at most R, requested)
-    if (part < OWNERS && (MT == 2 || lane < 32)) {
+    if (!ROWS && owner) load_parameters();
+    char* const lds = lds_all + RED + (ROWS ? wave * wave_lds(MT) : 0);
+    if (ROWS && (MT == 2 || lane < 32)) {
 #pragma unroll
-        for (int i = 0; i < kParams; ++i) *reinterpret_cast<float*>(lds + (i * MT * 32 + lane) * 4) = par[i];
+        for (int i = 0; i < kParams; ++i) *reinterpret_cast<float*>(lds + (i * MT * 32 + lane) * 4) = par[i][0];
     }
 #pragma unroll
     for (int u = 0; u < R; ++u)
@@ -409,36 +527,62 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256, 2) void conv_f32_kernel(con
                 __builtin_amdgcn_sched_barrier(0);
             }
     } else {
-        // wave `part` finishes the tile's blocks part, part + WK, ...: the others leave it their sums
-        constexpr int BLOCKS = MT * NT;
-        char* const red = lds_all + (wave - part) * BLOCKS * 4096;
-#pragma unroll
-        for (int blk = 0; blk < BLOCKS; ++blk) {
-            if (blk % WK == part) continue;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const v16f& c = acc[blk % MT][blk / MT];
-                const v4f o = {c[q * 4], c[q * 4 + 1], c[q * 4 + 2], c[q * 4 + 3]};
-                *reinterpret_cast<v4f*>(red + (part * BLOCKS + blk) * 4096 + q * 1024 + lane * 16) = o;
+        unsigned img = 0, in_image = 0;
+        float res[V] = {}, v[V];
+        if (!ROWS && owner) {
+            if (p.res_shift || p.y_nchw || p.layout != EXHIP_PLACE_ROWS) {
+                img = exhip_divide(own_pix, per_image, p.image_magic, p.image_shift);
+                in_image = own_pix - img * per_image;
             }
-        }
-        __syncthreads();
-        if (!on) return;
+            if (p.residual && own_pix < p.pixels) {
+                unsigned from = own_pix;
+                if (p.res_shift) {
+                    const unsigned oy = exhip_divide(in_image, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = in_image - oy * (unsigned)p.out_w;
+                    from = (img * ((unsigned)p.out_h >> p.res_shift) + (oy >> p.res_shift)) * ((unsigned)p.out_w >> p.res_shift) + (ox >> p.res_shift);
+                }
+                const float* const src = p.residual + (size_t)from * (unsigned)p.rstride + own_ch;
 #pragma unroll
-        for (int blk = 0; blk < BLOCKS; ++blk) {
-            if (blk % WK != part) continue;
-            v16f sum = acc[blk % MT][blk / MT];
+                for (int e = 0; e < V; e += 4) {
+                    if (p.vector_rows) {
+                        if (own_ch + e < p.K) {
+                            const v4f r = *reinterpret_cast<const v4f*>(src + e);
 #pragma unroll
-            for (int w = 0; w < WK; ++w) {
-                if (w == blk % WK) continue;
+                            for (int i = 0; i < 4; ++i) res[e + i] = r[i];
+                        }
+                    } else {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const v4f o = *reinterpret_cast<const v4f*>(red + (w * BLOCKS + blk) * 4096 + q * 1024 + lane * 16);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) sum[q * 4 + e] += o[e];
+                        for (int i = 0; i < 4; ++i) res[e + i] = own_ch + e + i < p.K ? src[e + i] : 0.f;
+                    }
                 }
             }
-            epilogue_block<MT, SLOW>(p, sum, (tile * NT + blk / MT) * 32, kb0 + blk % MT, blk % MT, lane, lds);
+        }
+        char* const red = lds_all + (wave - part) * BLOCKS * 4096 + lane * 16;
+#pragma unroll
+        for (int i = 0; i < 4 * BLOCKS; ++i) {
+            const v16f& c = acc[i / 4 % MT][i / 4 / MT];
+            *reinterpret_cast<v4f*>(red + (part * 4 * BLOCKS + i) * 1024) = v4f{c[i % 4 * 4], c[i % 4 * 4 + 1], c[i % 4 * 4 + 2], c[i % 4 * 4 + 3]};
+        }
+        __syncthreads();
+        if (!owner) return;
+#pragma unroll
+        for (int j = 0; j < QUADS; ++j) {
+            v4f sum = *reinterpret_cast<const v4f*>(red + (quad + j) * 1024);
+#pragma unroll
+            for (int w = 1; w < WK; ++w) {
+                const v4f o = *reinterpret_cast<const v4f*>(red + (w * 4 * BLOCKS + quad + j) * 1024);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sum[e] += o[e];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[j * 4 + e] = sum[e];
+        }
+        if constexpr (ROWS) {
+            v16f sum;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) sum[e] = v[e];
+            epilogue_block<MT, SLOW>(p, sum, (tile * NT + quad / 4 / MT) * 32, kb0 + quad / 4 % MT, quad / 4 % MT, lane, lds);
+        } else {
+            epilogue_part<V>(p, v, par, res, own_pix, img, in_image, own_ch);
         }
     }
 }
@@ -446,12 +590,14 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256, 2) void conv_f32_kernel(con
 template <int MT, int NT, int WK, int R, int MODE, bool SLOW>
 int go(exhip_ctx* ctx, F32Params& p, int kblocks) {
     const long long tiles = ((long long)p.pixels + 32 * NT - 1) / (32 * NT);
-    p.tiles = (unsigned)tiles;
-    p.ch_groups = (unsigned)((kblocks + MT - 1) / MT);
-    const long long items = tiles * p.ch_groups;
+    const long long groups = (kblocks + MT - 1) / MT, items = tiles * groups;
     EXHIP_REQUIRE(items < (1ll << 31) - 4, "conv: grid too large");
     p.items = (unsigned)items;
-    exhip_host_divisor(p.ch_groups, &p.groups_magic, &p.groups_shift);
+    // Weights that an XCD's 4 MiB of cache do not hold, and that are more than the pixels, are dealt out over the XCDs (512 -> 512
+    // 3x3 on one 20 x 20 map, 9.4 MB: 27.5 -> 24.9 us); smaller ones are as fast or faster the other way (2.4 MB: 22.5 against 22.7).
+    p.tiles_fast = p.w_bytes > (4u << 20) && p.w_bytes > p.x_bytes;
+    p.fast = (unsigned)(p.tiles_fast ? tiles : groups);
+    exhip_host_divisor(p.fast, &p.fast_magic, &p.fast_shift);
     const int taps_w = MODE == kPair ? (p.kw + 1) / 2 : p.kw;
     for (int i = 0; i <= WK; ++i) {
         const int s = (int)((long long)p.n_ksteps * i / WK), tap = s / p.csteps;

@@ -1,5 +1,7 @@
 """The float32 convolution kernel (conv_f32.hip): every wave tile and split of its list on ragged shapes, against the CPU
 oracle's layers; and what surrounds the products -- pad channels, odd channel strides, four-channel pixels, the shortcut."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -66,6 +68,66 @@ def test_conv_f32_tiles_and_splits(ctx, tile, args):
     assert cases.check_value(got[..., :k].transpose(0, 3, 1, 2), want, 1e-5) == 0
     assert not got[..., k:].any()
     assert np.array_equal(flat[:-guard].reshape(want.shape), got[..., :k].transpose(0, 3, 1, 2))
+
+
+class Place(ctypes.Structure):
+    _fields_ = [(name, ctypes.c_int) for name in ("layout", "group", "residual_stride", "residual_shift", "bn_relu")]
+
+
+ROWS, GROUPED, SHUFFLED = range(3)
+PLACES = [
+    # layout, group, n, c, h, w, k, kernel, shift of the shortcut's map (None: no shortcut), BatchNorm
+    (ROWS, 0, 2, 40, 6, 10, 44, 3, 1, True),        # written into 44 of 64 channels
+    (GROUPED, 85, 3, 72, 5, 7, 255, 1, None, False),  # a detection head, blocks that cross groups
+    (GROUPED, 3, 1, 256, 4, 4, 12, 1, None, True),
+    (SHUFFLED, 32, 2, 64, 5, 6, 128, 1, None, True),  # whole blocks per position
+    (SHUFFLED, 6, 1, 136, 3, 5, 24, 1, None, False),
+]
+
+
+@pytest.mark.parametrize("args", PLACES, ids=["rows", "head", "small-head", "shuffled", "shuffled-odd"])
+def test_placements_for_every_tile_and_split(ctx, tile, args):
+    """Results in their groups, as an upsampled map or inside a wider tensor, against the definition in 64 bits. The layers sum at most
+    360 float32 products of at most 1 each to results of order 1: 360 roundings of 2^-24 are 2.2e-5."""
+    layout, group, n, c, h, w, k, kernel, shift, bn = args
+    r = np.random.default_rng(k + c)
+    x, wt = r.uniform(-1, 1, (n, h, w, c)).astype(np.float32), r.normal(0, 0.1, (k, c, kernel, kernel)).astype(np.float32)
+    bias, slope = (r.normal(0, 0.5, k).astype(np.float32) for _ in range(2))
+    a, b = (r.normal(0, 1, k).astype(np.float32) for _ in range(2))
+    ks = 64 if layout == ROWS else group if layout == SHUFFLED else 256
+    pd = kernel // 2
+    d = ctx.conv_desc(n, c, h, w, k, kernel, 1, pd, 1, c, ks, residual_last=1, exact_k=int(layout == ROWS))
+    da, db, ds = ctx.array(a), ctx.array(b), ctx.array(slope)
+    if bn:
+        d.post_bn_a, d.post_bn_b = da.ptr, db.ptr
+    d.post_op, d.post_slope = 16, ds.ptr  # EXHIP_POST_PRELU
+    xp = np.pad(x.astype(np.float64), ((0, 0), (pd, pd), (pd, pd), (0, 0)))
+    want = sum(xp[:, i:i + h, j:j + w] @ wt[:, :, i, j].T.astype(np.float64) for i in range(kernel) for j in range(kernel)) + bias
+    want = np.maximum(want, 0)
+    if bn:
+        want = b * want + a.astype(np.float64)
+    want = np.where(want >= 0, want, slope * want)
+    res = None
+    if shift is not None:
+        small = r.uniform(-1, 1, (n, h >> shift, w >> shift, 48)).astype(np.float32)
+        res = ctx.array(small)
+        want = want + small[..., :k].repeat(1 << shift, 1).repeat(1 << shift, 2)
+    if layout == ROWS:
+        expect = np.full((n, h, w, ks), 7.0)
+        expect[..., :k] = want
+    elif layout == GROUPED:
+        expect = want.reshape(n, h * w, k // group, group).transpose(0, 2, 1, 3)
+    else:
+        expect = want.reshape(n, h, w, 2, 2, group).transpose(0, 1, 3, 2, 4, 5)
+    y = ctx.array(np.full(expect.size + 64, 7.0, np.float32))
+    place = Place(layout, group, 48, shift or 0, 0)
+    wp = ctx.pack_conv_weights(d, hip.F32, wt)
+    hip._check(hip.lib().exhip_conv2d_f32_placed(ctx.h, ctypes.byref(d), ctypes.byref(place), ctx.array(x).ptr, wp.ptr, ctx.array(bias).ptr,
+                                                 res.ptr if res else None, y.ptr, None))
+    ctx.sync()
+    got = y.download()
+    assert (got[-64:] == 7.0).all()
+    assert np.abs(got[:-64].reshape(expect.shape) - expect).max() < 2.2e-5 * max(1.0, np.abs(want).max())
 
 
 def test_the_plain_entry_refuses_what_only_the_placed_one_does(ctx):
