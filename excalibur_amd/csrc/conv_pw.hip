@@ -114,11 +114,12 @@ constexpr int param_bytes(int mt) { return kParams * mt * 32 * 4; }
 constexpr int tile_bytes(int dt, int mt) { return 32 * ((dt == EXHIP_I8 ? 128 : mt * 64) + 16); }  // int8 layers: one float32 block
 constexpr int wave_bytes(int dt, int mt) { return param_bytes(mt) + tile_bytes(dt, mt); }
 
-template <int MT>
-__device__ __forceinline__ void read16(const char* lds, int which, int m, int half, float (&v)[16]) {
-    const v4f* src = reinterpret_cast<const v4f*>(lds + (which * MT * 32 + m * 32 + half * 16) * 4);
+// N neighbouring channels' parameters from channel `at` of the wave's MT * 32 on.
+template <int MT, int N>
+__device__ __forceinline__ void read_parameters(const char* lds, int which, int at, float (&v)[N]) {
+    const v4f* src = reinterpret_cast<const v4f*>(lds + (which * MT * 32 + at) * 4);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < N / 4; ++q) {
         const v4f t = src[q];
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[q * 4 + e] = t[e];
@@ -134,11 +135,11 @@ __device__ __forceinline__ unsigned round_pair(float lo, float hi) {
 }
 
 // ROUND: the layer behind reads the halves that the layer in front of it stored.
-template <bool ROUND>
-__device__ __forceinline__ void stored16(float (&v)[16]) {
+template <bool ROUND, int N>
+__device__ __forceinline__ void stored(float (&v)[N]) {
     if constexpr (ROUND) {
 #pragma unroll
-        for (int e = 0; e < 16; e += 2) {
+        for (int e = 0; e < N; e += 2) {
             const unsigned d = round_pair(v[e], v[e + 1]);
             v[e] = exhip_h2f((uint16_t)(d & 0xffff));
             v[e + 1] = exhip_h2f((uint16_t)(d >> 16));
@@ -146,18 +147,18 @@ __device__ __forceinline__ void stored16(float (&v)[16]) {
     }
 }
 
-template <int OP, bool ROUND>
-__device__ __forceinline__ void unary16(float (&v)[16], float alpha, float beta) {
-    stored16<ROUND>(v);
+template <int OP, bool ROUND, int N>
+__device__ __forceinline__ void unary_values(float (&v)[N], float alpha, float beta) {
+    stored<ROUND>(v);
 #pragma unroll
-    for (int e = 0; e < 16; ++e) v[e] = unary_value<OP>(v[e], alpha, beta);
+    for (int e = 0; e < N; ++e) v[e] = unary_value<OP>(v[e], alpha, beta);
 }
 
-template <bool ROUND>
-__device__ __forceinline__ void relu16(float (&v)[16]) {
-    stored16<ROUND>(v);
+template <bool ROUND, int N>
+__device__ __forceinline__ void relu_values(float (&v)[N]) {
+    stored<ROUND>(v);
 #pragma unroll
-    for (int e = 0; e < 16; ++e) v[e] = (0.f > v[e]) ? 0.f : v[e];
+    for (int e = 0; e < N; ++e) v[e] = (0.f > v[e]) ? 0.f : v[e];
 }
 
 // Rows of a wave tile from its LDS slice to memory: CHUNKS 16-byte pieces per row of 32, neighbouring lanes on neighbouring
@@ -178,6 +179,44 @@ __device__ __forceinline__ void store_rows(const char* tile, int pitch, __amdgpu
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_view(const void* base, unsigned first, int row_bytes, int ch_bytes, int rows) {
     char* p = const_cast<char*>(static_cast<const char*>(base)) + (size_t)first * (unsigned)row_bytes + ch_bytes;
     return __builtin_amdgcn_make_buffer_rsrc(p, 0, pw_view_bytes(rows, row_bytes, ch_bytes), kRsrcWord3);
+}
+
+// The layers behind the products and the bias, of N neighbouring channels from channel `at` of the wave's MT * 32 on; residual(e): the
+// shortcut's value. (An activation that only EpAny has is evaluated value by value, so that its registers are needed once.)
+template <int DT, int MT, typename EP, int N, typename RES>
+__device__ __forceinline__ void layers_behind(const PwParams& p, float (&v)[N], const char* lds, int at, bool shortcut, RES residual) {
+    constexpr bool I8 = DT == EXHIP_I8, ANY = EP::any;
+    float t[N];
+    if (ANY ? p.act == 1 : EP::act == 1) relu_values<false>(v);
+    if (ANY && p.act > 1) {
+#pragma unroll 1
+        for (int e = 0; e < N; ++e) v[e] = slow_activation(v[e], p.act);
+    }
+    auto add_shortcut = [&]() {
+        stored<!I8>(v);
+#pragma unroll
+        for (int e = 0; e < N; ++e) v[e] += residual(e);
+    };
+    if (ANY ? shortcut && !p.residual_last : EP::res == 1) add_shortcut();
+    if (ANY ? p.post_relu != 0 : EP::post == kPostRelu) relu_values<!I8>(v);
+    if (I8 && (ANY ? p.post_bn_a != nullptr : EP::bn)) {  // the BatchNorm layer between this layer (through a Concat) and its activation layer
+        float a[N], b[N];
+        read_parameters<MT>(lds, 2, at, a);
+        read_parameters<MT>(lds, 3, at, b);
+#pragma unroll
+        for (int e = 0; e < N; ++e) v[e] = __builtin_fmaf(b[e], v[e], a[e]);
+    }
+    if (ANY ? p.post_op == 1 + EXHIP_UNARY_HARDSWISH : EP::post == kPostHardSwish) unary_values<0, !I8>(v, p.post_alpha, p.post_beta);
+    if (ANY ? p.post_op == 1 + EXHIP_UNARY_LEAKYRELU : EP::post == kPostLeaky) unary_values<1, !I8>(v, p.post_alpha, p.post_beta);
+    if (ANY && p.post_op == 1 + EXHIP_UNARY_HARDSIGMOID) unary_values<3, !I8>(v, p.post_alpha, p.post_beta);
+    if (ANY && p.post_op == 1 + EXHIP_UNARY_CLIP) unary_values<4, !I8>(v, p.post_alpha, p.post_beta);
+    if (ANY ? p.post_op == EXHIP_POST_PRELU : EP::post == kPostPrelu) {
+        read_parameters<MT>(lds, 2, at, t);
+        stored<!I8>(v);
+#pragma unroll
+        for (int e = 0; e < N; ++e) v[e] = v[e] >= 0.f ? v[e] : t[e] * v[e];
+    }
+    if (ANY ? shortcut && p.residual_last : EP::res == 2) add_shortcut();
 }
 
 template <int DT, int MT, int NT, typename EP, typename ACC>
@@ -228,49 +267,20 @@ __device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[
             float v[16], t[16];
             if constexpr (I8) {
                 float b[16];
-                read16<MT>(lds, 0, m, half, t);
-                read16<MT>(lds, 1, m, half, b);
+                read_parameters<MT>(lds, 0, m * 32 + half * 16, t);
+                read_parameters<MT>(lds, 1, m * 32 + half * 16, b);
 #pragma unroll
                 for (int e = 0; e < 16; ++e) v[e] = __builtin_fmaf((float)acc[m][n][e], t[e], b[e]);
             } else {
-                read16<MT>(lds, 1, m, half, t);
+                read_parameters<MT>(lds, 1, m * 32 + half * 16, t);
 #pragma unroll
                 for (int e = 0; e < 16; ++e) v[e] = acc[m][n][e] + t[e];
             }
-            if (ANY ? p.act == 1 : EP::act == 1) relu16<false>(v);
-            if (ANY && p.act > 1) {
-#pragma unroll 1
-                for (int e = 0; e < 16; ++e) v[e] = slow_activation(v[e], p.act);
-            }
-            auto add_shortcut = [&]() {
-                stored16<!I8>(v);
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    const int word = r[m][I8 ? e >> 2 : e >> 3][I8 ? e & 3 : (e >> 1) & 3];  // (a bit cast of the element itself takes the vector's first)
-                    if constexpr (I8) v[e] += __builtin_bit_cast(float, word);
-                    else v[e] += exhip_h2f((uint16_t)(((uint32_t)word >> ((e & 1) * 16)) & 0xffff));
-                }
-            };
-            if (ANY ? shortcut && !p.residual_last : EP::res == 1) add_shortcut();
-            if (ANY ? p.post_relu != 0 : EP::post == kPostRelu) relu16<!I8>(v);
-            if (I8 && (ANY ? p.post_bn_a != nullptr : EP::bn)) {  // the BatchNorm layer between this layer (through a Concat) and its activation layer
-                float a[16], b[16];
-                read16<MT>(lds, 2, m, half, a);
-                read16<MT>(lds, 3, m, half, b);
-#pragma unroll
-                for (int e = 0; e < 16; ++e) v[e] = __builtin_fmaf(b[e], v[e], a[e]);
-            }
-            if (ANY ? p.post_op == 1 + EXHIP_UNARY_HARDSWISH : EP::post == kPostHardSwish) unary16<0, !I8>(v, p.post_alpha, p.post_beta);
-            if (ANY ? p.post_op == 1 + EXHIP_UNARY_LEAKYRELU : EP::post == kPostLeaky) unary16<1, !I8>(v, p.post_alpha, p.post_beta);
-            if (ANY && p.post_op == 1 + EXHIP_UNARY_HARDSIGMOID) unary16<3, !I8>(v, p.post_alpha, p.post_beta);
-            if (ANY && p.post_op == 1 + EXHIP_UNARY_CLIP) unary16<4, !I8>(v, p.post_alpha, p.post_beta);
-            if (ANY ? p.post_op == EXHIP_POST_PRELU : EP::post == kPostPrelu) {
-                read16<MT>(lds, 2, m, half, t);
-                stored16<!I8>(v);
-#pragma unroll
-                for (int e = 0; e < 16; ++e) v[e] = v[e] >= 0.f ? v[e] : t[e] * v[e];
-            }
-            if (ANY ? shortcut && p.residual_last : EP::res == 2) add_shortcut();
+            layers_behind<DT, MT, EP>(p, v, lds, m * 32 + half * 16, shortcut, [&](int e) {
+                const int word = r[m][I8 ? e >> 2 : e >> 3][I8 ? e & 3 : (e >> 1) & 3];  // (a bit cast of the element itself takes the vector's first)
+                if constexpr (I8) return __builtin_bit_cast(float, word);
+                else return exhip_h2f((uint16_t)(((uint32_t)word >> ((e & 1) * 16)) & 0xffff));
+            });
             if (kb * 32 + 32 > p.K) {  // pad channels hold zeros (wave-uniform: only the block with the ragged end looks)
 #pragma unroll
                 for (int e = 0; e < 16; ++e)
@@ -469,15 +479,18 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
 // The split form, for launches of few tiles and many k-steps (one image, deep layers), where the kernel above is as long as one
 // wave's chain: 0.17 us a k-step, 16 us for 256 -> 256 3x3 int8 on a 20 x 20 map. WK waves share a tile of 32 pixels x 32 * MT
 // channels: each takes its run of the k-steps, the sums meet in LDS (exactly for int8; in a fixed order, so the same bits
-// every time, for fp16), wave m finishes block m. Every request in the loop is unconditional, so that the waits count what is in
+// every time, for fp16), and each wave finishes its quarter of the tile, eight channels of a pixel per lane (wave m the whole block m
+// where the layers behind are looked at at run time: a head's groups take 32 channels at a time). Every request in the loop is unconditional, so that the waits count what is in
 // flight; those past a wave's run ask for operands it does not use.
 template <int DT, int MT, int WK, bool TAPS, typename EP>
 __global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParams p) {
     exhip_touch_args(p);
     constexpr int R = 8;  // k-steps in flight
+    constexpr bool I8 = DT == EXHIP_I8;
     constexpr int RED = WK * MT * 4096;
-    static_assert(MT <= WK && WK <= kSplit, "a wave per block");
-    __shared__ __attribute__((aligned(16))) char lds_all[RED + MT * wave_bytes(DT, 1)];
+    constexpr int OWN = EP::any ? wave_bytes(DT, 1) : param_bytes(1);
+    static_assert(MT == 2 && WK == 4 && WK <= kSplit, "two waves finish a block");
+    __shared__ __attribute__((aligned(16))) char lds_all[RED + (EP::any ? MT : WK) * OWN];
     const int lane = threadIdx.x & 63, part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     unsigned item = blockIdx.x;
     {
@@ -486,7 +499,9 @@ __global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParam
     }
     const unsigned tile = __builtin_amdgcn_readfirstlane(exhip_divide(item, p.ch_groups, p.groups_magic, p.groups_shift));
     const int kb0 = __builtin_amdgcn_readfirstlane((int)(item - tile * p.ch_groups) * MT);
-    char* const lds = lds_all + RED + (part < MT ? part : 0) * wave_bytes(DT, 1);
+    const int own_block = EP::any ? part : part >> 1;   // the block the wave finishes, or half of it
+    const bool finishes = own_block < MT;
+    char* const lds = lds_all + RED + (finishes ? part : 0) * OWN;
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.x), 0, (int)p.x_bytes, kRsrcWord3);
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.wp), 0, (int)p.w_bytes, kRsrcWord3);
 
@@ -557,7 +572,7 @@ __global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParam
     };
     float par[kParams] = {};
     auto load_parameters = [&]() {  // of the block this wave will finish: lane = channel
-        const int at = lane < 32 ? ((kb0 + part) * 32 + lane) * 4 : kOutOfRange;
+        const int at = lane < 32 ? ((kb0 + own_block) * 32 + lane) * 4 : kOutOfRange;
         auto load = [&](const float* src, int offset, int count) {
             const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src), 0, src ? count * 4 : 0, kRsrcWord3);
             return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, offset, 0, 0));
@@ -582,7 +597,7 @@ __global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParam
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        if (part < MT) load_parameters();
+        if (finishes) load_parameters();
 #pragma unroll
         for (int u = 0; u < R; ++u)
             if (k + u < steps) step(u);
@@ -590,7 +605,7 @@ __global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParam
 #pragma unroll
         for (int u = 0; u < R; ++u)
             if (u < steps) request(u);
-        if (part < MT) load_parameters();
+        if (finishes) load_parameters();
 #pragma unroll
         for (int u = 0; u < R; ++u)
             if (u < steps) step(u);
@@ -600,36 +615,100 @@ __global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParam
         if constexpr (DT == EXHIP_I8) return v4i{c[q * 4], c[q * 4 + 1], c[q * 4 + 2], c[q * 4 + 3]};
         else return __builtin_bit_cast(v4i, v4f{c[q * 4], c[q * 4 + 1], c[q * 4 + 2], c[q * 4 + 3]});
     };
+    const int k_end = pw_channel_end(p.K, p.kstride, p.exact), half = lane >> 5, row = lane & 31, kb = kb0 + own_block;
+    const int rows = p.pixels - tile * 32 < 32 ? (int)(p.pixels - tile * 32) : 32;
+    constexpr int N = 8, RV = I8 ? 2 : 1;   // channels a lane, 16-byte pieces of their shortcut
+    const int ch = half * 16 + (part & 1) * N;   // of the block's
+    v4i res[RV];
+    if constexpr (!EP::any && EP::res != 0) {
+        const int row_b = p.kstride * (I8 ? 4 : 2), ch_b = I8 ? 4 : 2;
+        const __amdgpu_buffer_rsrc_t rr = tile_view(I8 ? (const void*)p.residual_f : (const void*)p.residual, tile * 32, row_b, kb * 32 * ch_b, rows);
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        if (m == part) continue;
+        for (int q = 0; q < RV; ++q)
+            res[q] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rr, pw_lane_offset(row, row_b, ch * ch_b + q * 16, (p.kstride - kb * 32) * ch_b), 0, 0));
+    }
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int q = 0; q < 4; ++q) *reinterpret_cast<v4i*>(lds_all + (part * MT + m) * 4096 + q * 1024 + lane * 16) = word4(acc[m], q);
-    }
     __syncthreads();
-    // the wave of a second block that does not exist (an odd number of blocks) is done too
-    if (part >= MT || !pw_block_exists(kb0 + part, pw_channel_end(p.K, p.kstride, p.exact))) return;
+    // what finishes a second block that does not exist (an odd number of blocks) is done too
+    if (!finishes || !pw_block_exists(kb, k_end)) return;
     if (lane < 32) {
 #pragma unroll
         for (int i = 0; i < kParams; ++i) *reinterpret_cast<float*>(lds + (i * 32 + lane) * 4) = par[i];
     }
-    acc_t sum[1][1];
+    auto sum4 = [&](int q, auto* to) {  // four channels' sums over the waves
+        v4i t = *reinterpret_cast<const v4i*>(lds_all + own_block * 4096 + q * 1024 + lane * 16);
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
-        if (m == part) sum[0][0] = acc[m];
-    for (int w = 0; w < WK; ++w) {
-        if (w == part) continue;
+        for (int e = 0; e < 4; ++e) {
+            if constexpr (I8) to[e] = t[e];
+            else to[e] = __builtin_bit_cast(v4f, t)[e];
+        }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const v4i t = *reinterpret_cast<const v4i*>(lds_all + (w * MT + part) * 4096 + q * 1024 + lane * 16);
+        for (int w = 1; w < WK; ++w) {
+            t = *reinterpret_cast<const v4i*>(lds_all + (w * MT + own_block) * 4096 + q * 1024 + lane * 16);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                if constexpr (DT == EXHIP_I8) sum[0][0][q * 4 + e] += t[e];
-                else sum[0][0][q * 4 + e] += __builtin_bit_cast(v4f, t)[e];
+                if constexpr (I8) to[e] += t[e];
+                else to[e] += __builtin_bit_cast(v4f, t)[e];
             }
         }
+    };
+    typename std::conditional<I8, int, float>::type total[EP::any ? 16 : N];
+#pragma unroll
+    for (int q = 0; q < (EP::any ? 4 : N / 4); ++q) sum4(EP::any ? q : (part & 1) * (N / 4) + q, total + q * 4);
+    if constexpr (EP::any) {
+        acc_t sum[1][1];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sum[0][0][e] = total[e];
+        pw_epilogue<DT, 1, 1, EP>(p, sum, tile * 32, kb, lane, lds);
+    } else {
+        float v[N], scale[N], bias[N];
+        if constexpr (I8) read_parameters<1>(lds, 0, ch, scale);
+        read_parameters<1>(lds, 1, ch, bias);
+#pragma unroll
+        for (int e = 0; e < N; ++e) {
+            if constexpr (I8) v[e] = __builtin_fmaf((float)total[e], scale[e], bias[e]);
+            else v[e] = total[e] + bias[e];
+        }
+        layers_behind<DT, 1, EP>(p, v, lds, ch, EP::res != 0, [&](int e) {
+            const int word = res[I8 ? e >> 2 : 0][I8 ? e & 3 : e >> 1];
+            if constexpr (I8) return __builtin_bit_cast(float, word);
+            else return exhip_h2f((uint16_t)(((uint32_t)word >> ((e & 1) * 16)) & 0xffff));
+        });
+        if (kb * 32 + 32 > p.K) {  // pad channels hold zeros
+#pragma unroll
+            for (int e = 0; e < N; ++e)
+                if (kb * 32 + ch + e >= p.K) v[e] = 0.f;
+        }
+        typedef unsigned v4u __attribute__((ext_vector_type(4)));
+        typedef unsigned v2u __attribute__((ext_vector_type(2)));
+        if constexpr (I8) {
+            if (p.y_f) {
+                const __amdgpu_buffer_rsrc_t y = tile_view(p.y_f, tile * 32, p.kstride * 4, kb * 128, rows);
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const v4f o = {v[q * 4], v[q * 4 + 1], v[q * 4 + 2], v[q * 4 + 3]};
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, o), y, pw_lane_offset(row, p.kstride * 4, ch * 4 + q * 16, (k_end - kb * 32) * 4), 0, 0);
+                }
+            }
+            if (p.y_q) {
+                v2u o;
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    uint32_t w = 0;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) w |= (uint32_t)(exhip_q8(v[q * 4 + e] * p.fs_out) & 0xff) << (8 * e);
+                    o[q] = w;
+                }
+                __builtin_amdgcn_raw_buffer_store_b64(o, tile_view(p.y_q, tile * 32, p.kstride, kb * 32, rows), pw_lane_offset(row, p.kstride, ch, k_end - kb * 32), 0, 0);
+            }
+        } else {
+            const v4u o = {round_pair(v[0], v[1]), round_pair(v[2], v[3]), round_pair(v[4], v[5]), round_pair(v[6], v[7])};
+            __builtin_amdgcn_raw_buffer_store_b128(o, tile_view(p.y, tile * 32, p.kstride * 2, kb * 64, rows), pw_lane_offset(row, p.kstride * 2, ch * 2, (k_end - kb * 32) * 2), 0, 0);
+        }
     }
-    pw_epilogue<DT, 1, 1, EP>(p, sum, tile * 32, kb0 + part, lane, lds);
 }
 
 // A depthwise 3x3 layer and the pointwise layer that alone reads it, the depthwise results staying in LDS. A group computes
