@@ -261,7 +261,6 @@ __device__ __forceinline__ void post_activation4(v4f& v, int op, float alpha, fl
 // LOWREG: held to 128 registers (a few spills) so that two 512-thread groups can share a CU.
 template <int DT, int MT, int NT, int WM, int WN, bool PACKED, int EPI, int KWE, int KSC, bool LOWREG = false>
 __global__ __launch_bounds__(64 * WM * WN, (MT * NT > 4 ? 1 : (LOWREG ? 4 : 2))) void conv_igemm_kernel(const ConvParams p) {
-    exhip_touch_args(p);
     constexpr int THREADS = 64 * WM * WN;
     constexpr int TM = 32 * MT * WM;
     // staging limits scale with the group size so that a 512-thread group needs half the registers
@@ -1725,7 +1724,8 @@ int run_conv(exhip_ctx* ctx, const exhip_conv_desc* d, ConvParams p, const PoolS
         // split keeps more CUs busy). EXHIP_ERR_UNSUPPORTED leaves the layer to this kernel.
         const int min_chunks_ = (3 + pl.n_rg - 1) / pl.n_rg;
         const bool would_split = g_exhip_options.force_splits != 1 && pl.n_chunks / min_chunks_ >= 2 && kCUs / tiles >= 2;
-        const bool deep = !pl.packed && exhip_pw_splits_f16((long long)d->n * pl.OH * pl.OW, d->k, d->k_stride, pl.n_chunks * d->kh * d->kw * (pl.chunk_b / 32));
+        const bool deep = !pl.packed && exhip_pw_splits_f16((long long)d->n * pl.OH * pl.OW, p.cstride_b, d->k, d->k_stride,
+                                                             pl.n_chunks * d->kh * d->kw * (pl.chunk_b / 32), d->sh, d->post_op);
         if ((tiles >= 16 || !would_split) && g_exhip_options.force_splits <= 1 && !deep) {
             if (!pl.packed && !pool && d->kh == 3 && d->kw == 3 && d->sh == 1 && d->sw == 1 && pl.variant == 0 && pl.chunk_b == 64 &&
                 pl.RS == 1 && p.cstride_b % 64 == 0 && d->k % 64 == 0 && d->k_stride == d->k && d->act <= 1 && p.y_q && !p.y_nchw_h && !p.y_nchw &&

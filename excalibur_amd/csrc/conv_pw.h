@@ -50,6 +50,6 @@ int exhip_conv1x1_f16_pw(exhip_ctx* ctx, const exhip_pw_geom& g, const uint16_t*
 // The int8 layer: semantics as exhip_conv2d_i8 with the NHWC results only (y_i8 and / or y_f32; k_stride a multiple of 16).
 int exhip_conv1x1_i8_pw(exhip_ctx* ctx, const exhip_pw_geom& g, const int8_t* x, const void* wp, const float* scale, const float* bias,
                         const float* residual, int8_t* y_i8, float* y_f32, const exhip_pw_taps* taps = nullptr);
-// Whether that kernel takes an fp16 layer with a filter of this many output pixels, channels and 32-byte k-steps in its split form
-// (several waves to a tile), which is then faster than any other kernel for it.
-bool exhip_pw_splits_f16(long long pixels, int k, int k_stride, int n_ksteps);
+// Whether that kernel takes an fp16 layer with a filter of this many output pixels, input bytes per pixel, channels and 32-byte k-steps
+// (and stride, activation layer behind it) in its split form (several waves to a tile), which is then faster than any other kernel for it.
+bool exhip_pw_splits_f16(long long pixels, int c_bytes, int k, int k_stride, int n_ksteps, int stride, int post_op);

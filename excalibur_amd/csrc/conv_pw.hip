@@ -75,11 +75,12 @@ struct PwParams {
     // for k-step s of tap r * kw + q, that many bytes behind its top-left input pixel
     int in_h, in_w, out_h, out_w, stride, pad_t, pad_l, kh, kw;
     int step[kMaxDirectSteps];   // offset | tap << kTapShift (not used by the split form)
-    // the split form: where each wave of a tile begins in that order -- its first k-step, bytes behind the top-left input pixel,
+    // the split form: where each wave of a tile begins -- its first k-step (and that of its weights), bytes behind the top-left input pixel,
     // filter row, tap and bytes left of the chunk -- and what leads from behind a row's last tap to the next row, and from
     // behind the last row to the next chunk
-    int start_s[kSplit + 1], start_b[kSplit + 1], start_r[kSplit + 1], start_q[kSplit + 1], start_left[kSplit + 1];
+    int start_s[kSplit + 1], start_w[kSplit + 1], start_b[kSplit + 1], start_r[kSplit + 1], start_q[kSplit + 1], start_left[kSplit + 1];
     int chunk_b, row_end_b, chunk_end_b;
+    int pair_w, next_w, chunk_w;  // pairs: k-steps of the weights from a pair's first to its second, to the next pair, and more behind the last tap
     // the depthwise 3x3 layer in front (dw_pw_kernel; geometry in in_h .. pad_l above, x is its input): weights, bias and PReLU slopes,
     // activation 0, 1 or 3; 32-pixel tiles of a group and output blocks of a group
     const float* dw_w;
@@ -482,7 +483,7 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
 // every time, for fp16), and each wave finishes its quarter of the tile, eight channels of a pixel per lane (wave m the whole block m
 // where the layers behind are looked at at run time: a head's groups take 32 channels at a time). Every request in the loop is unconditional, so that the waits count what is in
 // flight; those past a wave's run ask for operands it does not use.
-template <int DT, int MT, int WK, bool TAPS, typename EP>
+template <int DT, int MT, int WK, bool TAPS, bool PAIRS, typename EP>
 __global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParams p) {
     exhip_touch_args(p);
     constexpr int R = 8;  // k-steps in flight
@@ -505,28 +506,41 @@ __global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParam
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.x), 0, (int)p.x_bytes, kRsrcWord3);
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.wp), 0, (int)p.w_bytes, kRsrcWord3);
 
-    const unsigned pix = tile * 32 + (lane & 31);
-    int xoff, iy = 0, ix = 0;
-    if constexpr (TAPS) {
-        const unsigned per_image = (unsigned)(p.out_h * p.out_w);
-        const unsigned img = exhip_divide(pix, per_image, p.image_magic, p.image_shift), rem = pix - img * per_image;
-        const int oy = (int)exhip_divide(rem, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = (int)(rem - (unsigned)oy * (unsigned)p.out_w);
-        iy = oy * p.stride - p.pad_t;
-        ix = ox * p.stride - p.pad_l;
-        xoff = (((int)img * p.in_h + iy) * p.in_w + ix) * p.xs_b + (lane >> 5) * 16;
-        if (pix >= p.pixels) iy = -0x40000000;
-    } else {
-        xoff = pix < p.pixels ? (int)(pix * (unsigned)p.xs_b) + (lane >> 5) * 16 : kOutOfRange;
+    // What a lane requests of the pixels. PAIRS: two k-steps at a time, 64 bytes of every pixel; four lanes read a pixel's, sixteen
+    // pixels a load. Else a k-step at a time: the lane's pixel is lane & 31, its 16-byte half lane >> 5.
+    constexpr int XL = PAIRS ? 2 : 1;
+    int xoff[XL], iy[XL], ix[XL];
+#pragma unroll
+    for (int j = 0; j < XL; ++j) {
+        const unsigned pix = tile * 32 + (PAIRS ? j * 16 + (lane >> 2) : lane & 31);
+        const int byte = (PAIRS ? lane & 3 : lane >> 5) * 16;
+        if constexpr (TAPS) {
+            const unsigned per_image = (unsigned)(p.out_h * p.out_w);
+            const unsigned img = exhip_divide(pix, per_image, p.image_magic, p.image_shift), rem = pix - img * per_image;
+            const int oy = (int)exhip_divide(rem, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = (int)(rem - (unsigned)oy * (unsigned)p.out_w);
+            iy[j] = oy * p.stride - p.pad_t;
+            ix[j] = ox * p.stride - p.pad_l;
+            xoff[j] = (((int)img * p.in_h + iy[j]) * p.in_w + ix[j]) * p.xs_b + byte;
+            if (pix >= p.pixels) iy[j] = -0x40000000;
+        } else {
+            xoff[j] = pix < p.pixels ? (int)(pix * (unsigned)p.xs_b) + byte : kOutOfRange;
+        }
     }
-    const int s_first = p.start_s[part], steps = p.start_s[part + 1] - s_first, s_last = p.n_ksteps - 1;
+    const int s_first = PAIRS ? p.start_w[part] : p.start_s[part], steps = p.start_s[part + 1] - p.start_s[part];
+    const int pair_w = PAIRS ? p.pair_w : 0, s_last = p.n_ksteps - 1 - pair_w;
     const int w_step = p.mts * 1024, slab = kb0 >> (p.mts >> 1);
     const int w_base = (slab * p.n_ksteps * p.mts + (kb0 & (p.mts - 1))) * 1024;
     int s_at = s_first, b_at = p.start_b[part], r_at = p.start_r[part], q_at = p.start_q[part], left = p.start_left[part];
-    int xcur = xoff;
-    auto enter_tap = [&]() {  // the lane's offset at the tap, out of range outside the image
-        const bool in = (unsigned)(iy + r_at) < (unsigned)p.in_h && (unsigned)(ix + q_at) < (unsigned)p.in_w;
-        xcur = in ? xoff + b_at : kOutOfRange;
+    int xcur[XL];
+    auto enter_tap = [&]() {  // the lane's offsets at the tap, out of range outside the image
+#pragma unroll
+        for (int j = 0; j < XL; ++j) {
+            const bool in = (unsigned)(iy[j] + r_at) < (unsigned)p.in_h && (unsigned)(ix[j] + q_at) < (unsigned)p.in_w;
+            xcur[j] = in ? xoff[j] + b_at : kOutOfRange;
+        }
     };
+#pragma unroll
+    for (int j = 0; j < XL; ++j) xcur[j] = xoff[j];
     if constexpr (TAPS) enter_tap();
 
     typedef typename std::conditional<DT == EXHIP_I8, v16i, v16f>::type acc_t;
@@ -536,16 +550,19 @@ __global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParam
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[m][e] = 0;
     v4i a[R][MT], b[R];
-    auto request = [&](int u) {
+    auto request = [&](int u) {  // PAIRS: k-steps u and u + 1, u even
         const int s_in = s_at < s_last ? s_at : s_last;
 #pragma unroll
-        for (int m = 0; m < MT; ++m)
-            a[u][m] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, lane * 16 + m * 1024, w_base + s_in * w_step, 0));
-        b[u] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(xr, xcur, TAPS ? 0 : s_in * 32, 0));
-        ++s_at;
+        for (int j = 0; j < XL; ++j) {
+            b[u + j] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(xr, xcur[j], TAPS ? 0 : s_in * 32, 0));
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+                a[u + j][m] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, lane * 16 + m * 1024, w_base + (s_in + j * pair_w) * w_step, 0));
+        }
+        s_at += PAIRS ? p.next_w : 1;
         if constexpr (TAPS) {
-            b_at += 32;
-            left -= 32;
+            b_at += 32 * XL;
+            left -= 32 * XL;
             if (left == 0) {  // the next tap (no memory accesses under the branch)
                 left = p.chunk_b;
                 b_at += p.xs_b - p.chunk_b;
@@ -555,19 +572,35 @@ __global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParam
                     if (++r_at == p.kh) {
                         r_at = 0;
                         b_at += p.chunk_end_b;
+                        if (PAIRS) s_at += p.chunk_w;
                     }
                 }
                 enter_tap();
             } else {
-                xcur += xcur == kOutOfRange ? 0 : 32;
+#pragma unroll
+                for (int j = 0; j < XL; ++j) xcur[j] += xcur[j] == kOutOfRange ? 0 : 32 * XL;
             }
         }
     };
-    auto step = [&](int u) {
+    // PAIRS: through the wave's own LDS from four lanes a pixel to one. A CU takes 16 cycles for a load whose neighbouring lanes read
+    // 64 bytes of a pixel, up to 64 for one whose lanes read pixels a power of two apart, and a short launch spends its time on
+    // the requests (256 -> 256 3x3 int8 on one 20 x 20 map: 3400 cycles of 12 500 until the last of the first eight k-steps' is out).
+    // A pixel's 16-byte columns are dealt out by its number, so that neither side meets bank conflicts.
+    char* const stage = lds_all + part * MT * 4096;
+    char* const stage_in = stage + (lane >> 2) * 64 + ((lane & 3) ^ (lane >> 3 & 3)) * 16;   // (pixel >> 1) & 3, for either load
+    const char* const stage_out = stage + (lane & 31) * 64;
+    v4i x[2][2];
+    auto arrange = [&](int u, int to) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) *reinterpret_cast<v4i*>(stage_in + j * 1024) = b[u + j];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) x[to][j] = *reinterpret_cast<const v4i*>(stage_out + (((2 * j + (lane >> 5)) ^ (lane >> 1 & 3)) * 16));
+    };
+    auto product = [&](int u, const v4i& xb) {
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-            if constexpr (DT == EXHIP_I8) acc[m] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[u][m], b[u], acc[m], 0, 0, 0);
-            else acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a[u][m]), __builtin_bit_cast(v8h, b[u]), acc[m], 0, 0, 0);
+            if constexpr (DT == EXHIP_I8) acc[m] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[u][m], xb, acc[m], 0, 0, 0);
+            else acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a[u][m]), __builtin_bit_cast(v8h, xb), acc[m], 0, 0, 0);
         }
     };
     float par[kParams] = {};
@@ -585,13 +618,23 @@ __global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParam
             par[3] = load(p.post_bn_b, at, p.K);
         }
     };
+    auto step = [&](int u) {  // k-step u; PAIRS: the pair, whose pixels have been arranged
+        if constexpr (PAIRS) {
+            product(u, x[u / 2 & 1][0]);
+            product(u + 1, x[u / 2 & 1][1]);
+        } else {
+            product(u, b[u]);
+        }
+    };
     if (steps > R) {
 #pragma unroll
-        for (int u = 0; u < R; ++u) request(u);
+        for (int u = 0; u < R; u += XL) request(u);
+        if constexpr (PAIRS) arrange(0, 0);
         int k = 0;
         for (; k + R < steps; k += R) {
 #pragma unroll
-            for (int u = 0; u < R; ++u) {
+            for (int u = 0; u < R; u += XL) {
+                if constexpr (PAIRS) arrange((u + 2) % R, (u / 2 + 1) & 1);
                 step(u);
                 request(u);
                 __builtin_amdgcn_sched_barrier(0);
@@ -599,16 +642,23 @@ __global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParam
         }
         if (finishes) load_parameters();
 #pragma unroll
-        for (int u = 0; u < R; ++u)
-            if (k + u < steps) step(u);
+        for (int u = 0; u < R; u += XL)
+            if (k + u < steps) {
+                if constexpr (PAIRS)
+                    if (u + 2 < R) arrange(u + 2, (u / 2 + 1) & 1);
+                step(u);
+            }
     } else {
 #pragma unroll
-        for (int u = 0; u < R; ++u)
+        for (int u = 0; u < R; u += XL)
             if (u < steps) request(u);
         if (finishes) load_parameters();
 #pragma unroll
-        for (int u = 0; u < R; ++u)
-            if (u < steps) step(u);
+        for (int u = 0; u < R; u += XL)
+            if (u < steps) {
+                if constexpr (PAIRS) arrange(u, u / 2 & 1);
+                step(u);
+            }
     }
     // the waves' sums: 16 words a lane and block, 16 bytes side by side per lane
     auto word4 = [](const acc_t& c, int q) {
@@ -874,10 +924,10 @@ int go_dw(exhip_ctx* ctx, const PwParams& p) {
     return run(dw_pw_kernel<S, PX, EpAny>);
 }
 
-// U < 0: the split form with -U waves to a tile
+// U < 0: the split form, -kSplit a k-step at a time, -2 * kSplit in pairs
 template <int DT, int MT, int NT, int U, bool TAPS, typename EP>
 int go(exhip_ctx* ctx, const PwParams& p) {
-    if constexpr (U < 0) hipLaunchKernelGGL((conv_pw_split_kernel<DT, MT, -U, TAPS, EP>), dim3(p.items), dim3(64 * -U), 0, ctx->stream, p);
+    if constexpr (U < 0) hipLaunchKernelGGL((conv_pw_split_kernel<DT, MT, kSplit, TAPS, U == -2 * kSplit, EP>), dim3(p.items), dim3(64 * kSplit), 0, ctx->stream, p);
     else hipLaunchKernelGGL((conv1x1_pw_kernel<DT, MT, NT, U, TAPS, EP>), dim3((p.items + 3) / 4), dim3(256), 0, ctx->stream, p);
     EXHIP_LAUNCH_CHECK();
     return 0;
@@ -915,17 +965,35 @@ int pick_epilogue(exhip_ctx* ctx, const PwParams& p) {
     return go<DT, MT, NT, U == 8 ? 4 : U, TAPS, EpAny>(ctx, p);
 }
 
-// Whether a launch takes the split form: few enough wave tiles that their chains, not their sum, set the time, and k-steps enough
-// to share. Measured on the layers of yolov5s_simp at 1, 2, 4, 8 and 16 images (us, unsplit -> split): int8 256 -> 512 3x3 stride 2
-// from 40 x 40 at one image 24.5 -> 6.8, 128 -> 128 3x3 at 40 x 40 9.5 -> 5.5, 1024 -> 512 at 20 x 20 8.4 -> 4.6, fp16 13.1 -> 5.5. The
-// lines: up to 800 blocks of 32 pixels x 32 channels from 8 k-steps on (128 -> 128 3x3 int8 at 800 blocks 9.7 -> 8.3, at 1600
-// 10.0 -> 13.2; four k-steps gain nothing); int8 layers with a filter and 64 k-steps, which otherwise run the staged kernel, up to
-// 1600 (26.7 -> 18.6; 3200: 30.4 -> 29.7). A lone 32-channel block would leave half of every tile unused.
-bool split_wins(int dt, bool taps, long long pixels, int kblocks, int n_ksteps) {
+// Whether a launch takes the split form: long enough reductions, few enough blocks of 32 pixels x 32 channels. Its waves request their
+// pixels in 64-byte pieces (`pairs`), which the other kernels for these layers do not, so it also wins where every SIMD has several
+// waves. Measured over 64 to 1024 channels on maps of 20, 40 and 80 at 1 to 32 images, us without -> with it; a line lies between
+// the largest launch that wins throughout and the next one measured:
+//  * 1x1, from 16 k-steps on: fp16 800 blocks 5.7 -> 4.2, 1600 6.1 -> 5.8, 6400 15.5 -> 14.0 (64 k-steps 13.6 -> 6.7, 14.3 -> 10.6,
+//    48 -> 31); int8 32 k-steps 3200 blocks 15.1 -> 11.5 (6400 20.5
+//    against 20.9), 16 k-steps 800 blocks 6.1 -> 4.6 (1600 6.30 against 6.40).
+//    8 k-steps: fp16 800 blocks 4.19 -> 4.05, 1600 4.5 against 5.1; int8 800 blocks 4.55 against 4.9.
+//  * a filter at stride 1, against the lean kernel: 1200 blocks fp16 9.2 -> 7.3 (36 k-steps), 12.8 -> 10.6 (72), 19.7 -> 18.0
+//    (144), int8 6.05 -> 4.95 (18), 9.7 -> 7.4 (36); 1600 blocks fp16 12.5 against 13.3 (72), int8 10.0 -> 9.0 (36), 11.5 against 13.4
+//    (72, but 20.3 -> 13.3 with an activation layer behind, 2400 blocks 21.1 -> 16.9, 3200 21.5 against 22.3).
+//  * a filter at stride 2, where the staged kernel and the tapped form compete: 3200 blocks fp16 16.8 -> 14.1 (36), 24.9 -> 24.1 (72),
+//    int8 10.6 -> 10.2 (18), 17.1 -> 14.3 (36); 64 k-steps and more: 1600 blocks 23.6 -> 14.0 (fp16, 72), 17.1 -> 12.2 (int8, 72 at
+//    1440 blocks; at 2160 16.9 against 17.4), 30.7 -> 23.7 (fp16, 144), 28.6 -> 23.8 (int8, 144).
+// Layers without pairs (32-byte pixels, an odd number of chunks): 800 blocks. A lone 32-channel block would leave half of every tile
+// unused.
+bool split_wins(int dt, const exhip_pw_geom& g, int kblocks, int n_ksteps, bool taps, int stride) {
     if (g_exhip_options.force_splits == 1 || g_exhip_options.pw_split == 0 || kblocks < 2) return false;
     if (g_exhip_options.pw_split == 2) return true;
-    const long long blocks = (pixels + 31) / 32 * kblocks;
-    return n_ksteps >= 8 && blocks <= (dt == EXHIP_I8 && taps && n_ksteps >= 64 ? 1664 : 832);
+    if (n_ksteps < 8) return false;
+    const long long blocks = (g.pixels + 31) / 32 * kblocks;
+    if (g.c_bytes % 64 != 0) return blocks <= 832;
+    if (!taps) {
+        if (dt == EXHIP_I8) return blocks <= (n_ksteps < 16 ? 640 : n_ksteps < 32 ? 832 : 3328);
+        return blocks <= (n_ksteps < 16 ? 832 : 6656);
+    }
+    if (stride != 1) return blocks <= (n_ksteps < 16 ? 832 : n_ksteps < 64 ? 3328 : blocks * n_ksteps <= 240000 ? 1920 : 832);
+    if (dt == EXHIP_I8 && n_ksteps >= 32) return blocks <= (n_ksteps < 64 ? 1664 : g.post_op ? 2560 : 1280);
+    return blocks <= 1280;
 }
 
 template <int DT, int MT, int NT, bool TAPS = false>
@@ -943,6 +1011,11 @@ int launch(exhip_ctx* ctx, PwParams& p, int kblocks) {
     else return pick_epilogue<DT, MT, NT, 4, TAPS>(ctx, p);
 }
 
+// The k-step where wave i of a split tile begins.
+int split_start(int n_ksteps, bool pairs, int i) {
+    return pairs ? (int)((long long)(n_ksteps / 2) * i / kSplit) * 2 : (int)((long long)n_ksteps * i / kSplit);
+}
+
 template <int DT, bool TAPS>
 int launch_split(exhip_ctx* ctx, PwParams& p, int kblocks) {
     p.ch_groups = (unsigned)((kblocks + 1) / 2);
@@ -950,19 +1023,33 @@ int launch_split(exhip_ctx* ctx, PwParams& p, int kblocks) {
     if (items >= (1ll << 31) - 4) return EXHIP_ERR_UNSUPPORTED;
     p.items = (unsigned)items;
     exhip_host_divisor(p.ch_groups, &p.groups_magic, &p.groups_shift);
+    // Where a pixel's bytes of a tap (of all channels for a 1x1 layer) come in whole 64-byte pieces: pairs of k-steps, none of them
+    // shared. A packing in chunks of 32 bytes gives them too if the chunks are even in number: the pair's second k-step then
+    // is the next chunk's.
+    const bool pairs = TAPS ? p.chunk_b % 64 == 0 || p.n_ksteps / (p.kh * p.kw) % 2 == 0 : p.n_ksteps % 2 == 0, two_chunks = TAPS && pairs && p.chunk_b == 32;
+    const int taps = TAPS ? p.kh * p.kw : 1;
+    if (two_chunks) {
+        p.chunk_end_b += 32;
+        p.chunk_b = 64;
+    }
+    p.pair_w = two_chunks ? taps : 1;
+    p.next_w = two_chunks ? 1 : 2;
+    p.chunk_w = two_chunks ? taps : 0;
     for (int i = 0; i <= kSplit; ++i) {
-        const int s = (int)((long long)p.n_ksteps * i / kSplit);
+        const int s = split_start(p.n_ksteps, pairs, i);
         p.start_s[i] = s;
+        p.start_w[i] = s;
         if (TAPS) {
             const int per_tap = p.chunk_b / 32, per_row = p.kw * per_tap, per_chunk = p.kh * per_row;
-            const int chunk = s / per_chunk, in_chunk = s % per_chunk, row = in_chunk / per_row, tap = in_chunk % per_row / per_tap, j = in_chunk % per_tap;
+            const int chunk = s / per_chunk, in_chunk = s % per_chunk, row = in_chunk / per_row, tap = in_chunk % per_row / per_tap, k = in_chunk % per_tap;
+            if (two_chunks) p.start_w[i] = chunk * per_chunk + in_chunk / 2;
             p.start_r[i] = row;
             p.start_q[i] = tap;
-            p.start_b[i] = (row * p.in_w + tap) * p.xs_b + chunk * p.chunk_b + j * 32;
-            p.start_left[i] = p.chunk_b - j * 32;
+            p.start_b[i] = (row * p.in_w + tap) * p.xs_b + chunk * p.chunk_b + k * 32;
+            p.start_left[i] = p.chunk_b - k * 32;
         }
     }
-    return pick_epilogue<DT, 2, 1, -kSplit, TAPS>(ctx, p);
+    return pairs ? pick_epilogue<DT, 2, 1, -2 * kSplit, TAPS>(ctx, p) : pick_epilogue<DT, 2, 1, -kSplit, TAPS>(ctx, p);
 }
 
 }  // namespace
@@ -984,7 +1071,7 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
     if (g.post_bn_a || g.post_bn_b || g.exact_k || g.group) return EXHIP_ERR_UNSUPPORTED;
     const long long n_ksteps = (long long)t.n_chunks * t.kh * t.kw * (t.chunk_b / 32);
     if (g.pixels <= 0 || g.c_bytes <= 0 || g.c_bytes % 32 != 0 || t.chunk_b % 32 != 0 || t.n_chunks * t.chunk_b != g.c_bytes ||
-        (g.slab_blocks != 2 && g.slab_blocks != 4) || g.k_stride % 8 != 0 || !pw_row_fits(4ll * g.k_stride) || (n_ksteps > kMaxDirectSteps && !split_wins(DT, true, g.pixels, (std::max(g.k, g.k_stride) + 31) / 32, (int)n_ksteps)) || t.kh * t.kw > (1 << (32 - kTapShift)) || t.stride < 1 || t.pad_t < 0 || t.pad_l < 0)
+        (g.slab_blocks != 2 && g.slab_blocks != 4) || g.k_stride % 8 != 0 || !pw_row_fits(4ll * g.k_stride) || (n_ksteps > kMaxDirectSteps && !split_wins(DT, g, (std::max(g.k, g.k_stride) + 31) / 32, (int)n_ksteps, true, t.stride)) || t.kh * t.kw > (1 << (32 - kTapShift)) || t.stride < 1 || t.pad_t < 0 || t.pad_l < 0)
         return EXHIP_ERR_UNSUPPORTED;
     const long long x_bytes = (long long)t.n * t.in_h * t.in_w * g.c_bytes;
     const long long w_bytes = (long long)g.slabs * n_ksteps * g.slab_blocks * 1024;
@@ -1003,7 +1090,7 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
     // A lone 32-channel block wins whatever its size (12 -> 32 at 16 x 320 x 320: int8 71 -> 46 us, fp16 66 -> 45; 32 -> 32 at
     // 160 x 160: one image 8.1 -> 5.3 us, sixteen 24.9 -> 15.8).
     const bool take = kblocks == 1 || DT == EXHIP_F16 || g.c_bytes == 32 || (g.pixels <= 32768 && kblocks <= 4) || g.pixels <= 6400;
-    const bool split = split_wins(DT, true, g.pixels, kblocks, (int)n_ksteps);
+    const bool split = split_wins(DT, g, kblocks, (int)n_ksteps, true, t.stride);
     if (g_exhip_options.direct != 2 && !take && !split) return EXHIP_ERR_UNSUPPORTED;
     p.post_slope = g.post_slope;
     p.pixels = (unsigned)g.pixels; p.x_bytes = (unsigned)x_bytes; p.w_bytes = (unsigned)w_bytes;
@@ -1063,7 +1150,7 @@ int run_depthwise(exhip_ctx* ctx, const exhip_pw_depthwise& dw, PwParams& p, int
     p.items = (unsigned)(tiles * p.ch_groups);
     exhip_host_divisor(p.ch_groups, &p.groups_magic, &p.groups_shift);
     p.dw_split = split;
-    for (int i = 0; i <= kSplit; ++i) p.start_s[i] = (int)((long long)p.n_ksteps * i / kSplit);
+    for (int i = 0; i <= kSplit; ++i) p.start_s[i] = split_start(p.n_ksteps, p.n_ksteps % 2 == 0, i);
     if (dw.stride == 2) return pixels == 2 ? go_dw<2, 2>(ctx, p) : go_dw<2, 1>(ctx, p);
     return pixels == 4 ? go_dw<1, 4>(ctx, p) : pixels == 2 ? go_dw<1, 2>(ctx, p) : go_dw<1, 1>(ctx, p);
 }
@@ -1126,10 +1213,10 @@ int run_pw(exhip_ctx* ctx, const exhip_pw_geom& g, PwParams& p, int es, bool has
     // (exact_k: only the blocks of the k channels themselves)
     const int kblocks = std::min(g.slabs * g.slab_blocks, (out_channels + 31) / 32);
     if constexpr (DT == EXHIP_F16)
-        if (dw) return run_depthwise(ctx, *dw, p, kblocks, split_wins(DT, false, g.pixels, kblocks, (int)n_ksteps));
+        if (dw) return run_depthwise(ctx, *dw, p, kblocks, split_wins(DT, g, kblocks, (int)n_ksteps, false, 1));
     // 64 x 64 per wave unless that leaves SIMDs without a wave: then 64 channels x 32 pixels; a lone 32-channel block
     // takes 128 pixels per wave
-    if (split_wins(DT, false, g.pixels, kblocks, (int)n_ksteps)) return launch_split<DT, false>(ctx, p, kblocks);
+    if (split_wins(DT, g, kblocks, (int)n_ksteps, false, 1)) return launch_split<DT, false>(ctx, p, kblocks);
     if (kblocks == 1) return launch<DT, 1, 2>(ctx, p, kblocks);
     const long long waves64 = ((g.pixels + 63) / 64) * ((kblocks + 1) / 2);
     if (waves64 < 2048 || small_tile<DT>()) return launch<DT, 2, 1>(ctx, p, kblocks);
@@ -1154,6 +1241,8 @@ int exhip_conv1x1_i8_pw(exhip_ctx* ctx, const exhip_pw_geom& g, const int8_t* x,
     return run_pw<EXHIP_I8>(ctx, g, p, 1, residual != nullptr, taps);
 }
 
-bool exhip_pw_splits_f16(long long pixels, int k, int k_stride, int n_ksteps) {
-    return g_exhip_options.pw != 0 && g_exhip_options.direct != 0 && split_wins(EXHIP_F16, true, pixels, (std::max(k, k_stride) + 31) / 32, n_ksteps);
+bool exhip_pw_splits_f16(long long pixels, int c_bytes, int k, int k_stride, int n_ksteps, int stride, int post_op) {
+    exhip_pw_geom g = {};
+    g.pixels = pixels; g.c_bytes = c_bytes; g.post_op = post_op;
+    return g_exhip_options.pw != 0 && g_exhip_options.direct != 0 && split_wins(EXHIP_F16, g, (std::max(k, k_stride) + 31) / 32, n_ksteps, true, stride);
 }

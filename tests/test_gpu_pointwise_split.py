@@ -158,3 +158,28 @@ def test_int8_split_of_an_odd_number_of_blocks(ctx, options, args, split, shortc
     assert np.array_equal(read_f().astype(np.int64), want)
     t = want * 0.25
     assert np.array_equal(read_q().astype(np.int64), np.clip(np.trunc(t + np.copysign(0.5, t)), -128, 127).astype(np.int64))
+
+
+# Pairs of k-steps: 64 bytes of a pixel's tap at a time, of one packed chunk or (32-byte chunks, even in number) of two.
+PAIRS = [
+    # seed, n, c, h, w, k, kernel, stride, pad
+    (970, 2, 64, 9, 11, 64, 3, 2, 1),              # int8: two chunks, nine pairs
+    (971, 1, 128, 14, 9, 96, 3, 2, (0, 1, 1, 0)),  # uneven padding, three blocks
+    (972, 1, 192, 8, 8, 64, (2, 3), 2, 1),         # six chunks: waves that begin in the middle of one
+    (973, 3, 128, 7, 5, 160, 1, 2, 0),             # one tap, every other pixel
+    (974, 1, 64, 1, 3, 64, 1, 1, 0),               # a single pair for four waves (int8)
+    (975, 1, 64, 33, 1, 64, 3, 1, 1),              # a column: the outer taps of every row outside; 33 pixels
+    (976, 1, 320, 6, 7, 64, 3, 1, 1),              # 90 steps: waves of 22 and 24
+]
+
+
+@pytest.mark.parametrize("shortcut", [0, 1])
+@pytest.mark.parametrize("args", PAIRS, ids=[f"s{a[0]}" for a in PAIRS])
+def test_int8_pairs_of_steps(ctx, options, args, shortcut):
+    options("direct", 2)
+    test_int8_split_equals_unsplit(ctx, options, args, shortcut)
+
+
+@pytest.mark.parametrize("args", PAIRS, ids=[f"s{a[0]}" for a in PAIRS])
+def test_fp16_pairs_of_steps(ctx, options, args):
+    test_fp16_split_against_the_oracle(ctx, options, args)
