@@ -7,6 +7,11 @@
 // copied by several threads (70 GB/s with six) while the previous chunk is on the link, and small ones are one kernel that
 // reads or writes the pinned memory itself (no copy engine, no hand-over between queues: 15 instead of 19 us for 75 KB with
 // the kernel behind it; 6 instead of 11 us for a result the host polls for instead of waiting on the stream).
+//
+// Uploads of every size are kernels that read the pinned memory: the copy engine leaves the link idle for some 15 us between two
+// copies, a kernel for 3, so an upload can begin with a small piece and needs no hand-over to the kernels behind it (16 groups: 54
+// GB/s in launches of 4 MiB, 48 in 1 MiB; the engine 50 and 38; 64 groups 53 and 41). Until everything is there: 4.9 MB 147 -> 130
+// us, 19 MB 480 -> 416, 79 MB 1755 -> 1562.
 #include <string.h>
 
 #include <atomic>
@@ -22,9 +27,11 @@
 
 namespace {
 
-constexpr size_t kChunk = (size_t)4 << 20;       // staging chunk: 50 GB/s on the link with one copy each (38 at 1 MiB), short enough to start early
-constexpr size_t kPiece = (size_t)512 << 10;     // what one thread copies at a time
-constexpr size_t kUploadKernel = (size_t)256 << 10;   // up to here a kernel reads the staging memory; the copy engine is as fast from 1 MiB on
+constexpr size_t kChunk = (size_t)4 << 20;       // staging chunk, the longest piece on the link
+constexpr size_t kPiece = (size_t)128 << 10;     // what one thread copies at a time
+constexpr size_t kStep = (size_t)512 << 10;      // what the first launch of an upload takes
+constexpr unsigned kUploadGroups = 16;
+constexpr size_t kUploadKernel = (size_t)256 << 10;   // small uploads; results up to here leave without staging
 constexpr size_t kSmallRing = (size_t)512 << 10;      // small uploads turn in this much of each chunk, so that the GPU's translations of it stay
                                                       // cached (75 KB from pages not seen lately take the kernel 31 us)
 constexpr size_t kDownloadKernel = (size_t)64 << 10;  // up to here one group writes the host's memory and a flag
@@ -194,8 +201,18 @@ __global__ void __launch_bounds__(256) upload_kernel(const char* __restrict__ sr
     unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
     if (wide) {
         const unsigned n = bytes / 16;
-        for (unsigned k = i; k < n; k += stride) reinterpret_cast<uint4*>(dst)[k] = reinterpret_cast<const uint4*>(src)[k];
-        for (unsigned k = n * 16 + i; k < bytes; k += stride) dst[k] = src[k];
+        const uint4* const from = reinterpret_cast<const uint4*>(src);
+        uint4* const to = reinterpret_cast<uint4*>(dst);
+        unsigned k = i;
+        for (; k + 3 * stride < n; k += 4 * stride) {
+            const uint4 a = from[k], b = from[k + stride], c = from[k + 2 * stride], d = from[k + 3 * stride];
+            to[k] = a;
+            to[k + stride] = b;
+            to[k + 2 * stride] = c;
+            to[k + 3 * stride] = d;
+        }
+        for (; k < n; k += stride) to[k] = from[k];
+        for (unsigned b = n * 16 + i; b < bytes; b += stride) dst[b] = src[b];
     } else {
         for (; i < bytes; i += stride) dst[i] = src[i];
     }
@@ -294,10 +311,12 @@ extern "C" int exhip_upload(exhip_ctx* ctx, void* dst, const void* src, size_t b
     staging_loan loan(ctx->up, ctx->stream);
     EXHIP_REQUIRE(loan.staging, "exhip_upload: no host memory");
     exhip_staging& s = *loan.staging;
-    copy_crew::session crew(bytes >= 4 * kPiece);
-    while (bytes) {
-        const size_t now = bytes < kChunk ? bytes : kChunk;
-        if (s.at < 0 || s.used + now > (now <= kUploadKernel ? kSmallRing : kChunk)) {
+    const bool small = bytes <= kUploadKernel;
+    copy_crew::session crew(bytes >= 2 * kStep);
+    for (size_t done = 0; bytes;) {
+        // as much again as is on its way: the link starts early and later launches are long
+        const size_t step = done < kStep ? kStep : done < kChunk ? done : kChunk, now = bytes < step ? bytes : step;
+        if (s.at < 0 || s.used + now > (small ? kSmallRing : kChunk)) {
             const int rc = next_chunk(ctx, s);
             if (rc == EXHIP_ERR_UNSUPPORTED) {  // no pinned memory left: the runtime's own way
                 EXHIP_CHECK(hipMemcpyAsync(to, from, bytes, hipMemcpyHostToDevice, ctx->stream));
@@ -310,16 +329,17 @@ extern "C" int exhip_upload(exhip_ctx* ctx, void* dst, const void* src, size_t b
         }
         char* stage = static_cast<char*>(s.chunk[s.at]) + s.used;
         crew.copy(stage, from, now);
-        if (now <= kUploadKernel) {
-            const unsigned groups = (unsigned)((now + 4095) / 4096);
-            upload_kernel<<<groups < 64 ? groups : 64, 256, 0, ctx->stream>>>(stage, to, (unsigned)now, is_wide(stage, to));
+        if (small || is_wide(stage, to)) {
+            const unsigned groups = (unsigned)((now + 4095) / 4096), most = small ? 64 : kUploadGroups;
+            upload_kernel<<<groups < most ? groups : most, 256, 0, ctx->stream>>>(stage, to, (unsigned)now, is_wide(stage, to));
             EXHIP_LAUNCH_CHECK();
-        } else {
+        } else {  // a destination off 16 bytes would be written byte by byte
             EXHIP_CHECK(hipMemcpyAsync(to, stage, now, hipMemcpyHostToDevice, ctx->stream));
         }
         s.used += (now + 255) / 256 * 256;
         from += now;
         to += now;
+        done += now;
         bytes -= now;
     }
     return 0;
@@ -369,7 +389,7 @@ static int download_through(exhip_staging& s, hipStream_t stream, void* dst, con
             EXHIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
             s.event[i] = e;
         }
-    copy_crew::session crew(bytes >= 4 * kPiece);
+    copy_crew::session crew(bytes >= 4 * kStep);
     const size_t total = (bytes + kChunk - 1) / kChunk;
     auto request = [&](size_t i) -> int {
         const size_t o = i * kChunk, n = bytes - o < kChunk ? bytes - o : kChunk;

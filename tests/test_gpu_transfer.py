@@ -35,6 +35,13 @@ def test_bytes_arrive_in_both_directions(ctx, size, offset):
     d.free()
 
 
+@pytest.mark.parametrize("size", [512 * KB, 512 * KB + 16, MB + 1, 2 * MB - 1, 4 * MB + 16, 8 * MB + 512 * KB + 7, 12 * MB])
+@pytest.mark.parametrize("offset", [0, 16, 8])
+def test_uploads_in_steps(ctx, size, offset):
+    """An upload's pieces: half a megabyte twice, then as much again as is on its way up to a chunk; by kernel or (8) by the engine."""
+    test_bytes_arrive_in_both_directions(ctx, size, offset)
+
+
 def test_uploads_do_not_wait_and_the_source_may_change_at_once(ctx):
     """More uploads than the staging ring holds, queued behind each other from one reused host buffer."""
     L, n, size = hip.lib(), 40, 900 * KB + 8
