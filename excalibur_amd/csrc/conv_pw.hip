@@ -40,7 +40,7 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 constexpr unsigned kRsrcWord3 = 0x00020000u;  // raw buffer: out-of-range loads return 0
 constexpr int kOutOfRange = kPwOutOfRange;    // a lane offset beyond every view
-constexpr int kMaxDirectSteps = 40;           // k-steps of a layer with a filter (taps x 32-byte steps per pixel)
+constexpr int kMaxDirectSteps = 40;           // table entries of a layer with a filter, a k-step (taps x 32-byte steps per pixel) or a pair each
 constexpr int kSplit = 4;                     // waves that share a tile's k-steps in the split form
 constexpr int kTapShift = 27;                 // a step's table entry: byte offset below, tap number above
 
@@ -74,7 +74,8 @@ struct PwParams {
     // the form with a filter (TAPS): output pixel (img, oy, ox) reads input pixel (oy * stride - pt + r, ox * stride - pl + q)
     // for k-step s of tap r * kw + q, that many bytes behind its top-left input pixel
     int in_h, in_w, out_h, out_w, stride, pad_t, pad_l, kh, kw;
-    int step[kMaxDirectSteps];   // offset | tap << kTapShift (not used by the split form)
+    int step[kMaxDirectSteps];   // of a k-step or pair: offset | tap << kTapShift (not used by the split form)
+    int pair_first[kMaxDirectSteps];  // the weights' k-step of a pair's first
     // the split form: where each wave of a tile begins -- its first k-step (and that of its weights), bytes behind the top-left input pixel,
     // filter row, tap and bytes left of the chunk -- and what leads from behind a row's last tap to the next row, and from
     // behind the last row to the next chunk
@@ -334,11 +335,12 @@ __device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[
     }
 }
 
-// U: k-steps per request round; two rounds are in flight.
-template <int DT, int MT, int NT, int U, bool TAPS, typename EP>
+// U: k-steps per request round; two rounds are in flight. PAIRS: the pixels in 64-byte pieces, as in the split form below.
+template <int DT, int MT, int NT, int U, bool TAPS, bool PAIRS, typename EP>
 __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
     exhip_touch_args(p);
-    __shared__ __attribute__((aligned(16))) char lds_all[4 * wave_bytes(DT, MT)];
+    constexpr int OWN = param_bytes(MT) + (PAIRS && NT * 4096 > tile_bytes(DT, MT) ? NT * 4096 : tile_bytes(DT, MT));
+    __shared__ __attribute__((aligned(16))) char lds_all[4 * OWN];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // workgroup ids are dealt round-robin to the 8 XCDs: give each XCD one contiguous run of items, so that the channel
     // groups of a pixel tile (and the weights' re-reads) share that XCD's L2
@@ -351,36 +353,40 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
     if (item >= p.items) return;  // wave-uniform; the kernel has no barrier
     const unsigned tile = __builtin_amdgcn_readfirstlane(exhip_divide(item, p.ch_groups, p.groups_magic, p.groups_shift));
     const int kb0 = __builtin_amdgcn_readfirstlane((int)(item - tile * p.ch_groups) * MT);  // first 32-channel block
-    char* const lds = lds_all + wave * wave_bytes(DT, MT);
+    char* const lds = lds_all + wave * OWN;
 
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.x), 0, (int)p.x_bytes, kRsrcWord3);
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.wp), 0, (int)p.w_bytes, kRsrcWord3);
 
-    // pixel fragments: lane = pixel (lane & 31), 16-byte half (lane >> 5) of each 32-byte k-step
-    int xoff[NT];
-    unsigned taps_in[NT];  // TAPS: bit r * kw + q set where that tap of the pixel lies inside the image
+    // What a lane requests of the pixels. PAIRS: two k-steps at a time, 64 bytes of every pixel; four lanes read a pixel's, sixteen
+    // pixels a load. Else a k-step at a time: the lane's pixel is lane & 31, its 16-byte half lane >> 5.
+    constexpr int XL = PAIRS ? 2 : 1;
+    int xoff[NT][XL];
+    unsigned taps_in[NT][XL];  // TAPS: bit r * kw + q set where that tap of the pixel lies inside the image
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-        const unsigned pix = (tile * NT + nt) * 32 + (lane & 31);
-        if constexpr (TAPS) {
-            // the filter's top-left input pixel; its offset may lie in front of the tensor (padding), the taps inside the
-            // image never do, and 32-bit wrap-around of the sum gives their offsets
-            const unsigned per_image = (unsigned)(p.out_h * p.out_w);
-            const unsigned img = exhip_divide(pix, per_image, p.image_magic, p.image_shift), rem = pix - img * per_image;
-            const int oy = (int)exhip_divide(rem, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = (int)(rem - (unsigned)oy * (unsigned)p.out_w);
-            const int iy = oy * p.stride - p.pad_t, ix = ox * p.stride - p.pad_l;
-            xoff[nt] = (((int)img * p.in_h + iy) * p.in_w + ix) * p.xs_b + (lane >> 5) * 16;
-            unsigned m = 0;
-            if (pix < p.pixels) {
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int l = 0; l < XL; ++l) {
+            const unsigned pix = (tile * NT + nt) * 32 + (PAIRS ? l * 16 + (lane >> 2) : lane & 31);
+            const int byte = (PAIRS ? lane & 3 : lane >> 5) * 16;
+            if constexpr (TAPS) {
+                // the filter's top-left input pixel; its offset may lie in front of the tensor (padding), the taps inside the
+                // image never do, and 32-bit wrap-around of the sum gives their offsets
+                const unsigned per_image = (unsigned)(p.out_h * p.out_w);
+                const unsigned img = exhip_divide(pix, per_image, p.image_magic, p.image_shift), rem = pix - img * per_image;
+                const int oy = (int)exhip_divide(rem, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = (int)(rem - (unsigned)oy * (unsigned)p.out_w);
+                const int iy = oy * p.stride - p.pad_t, ix = ox * p.stride - p.pad_l;
+                xoff[nt][l] = (((int)img * p.in_h + iy) * p.in_w + ix) * p.xs_b + byte;
+                unsigned row = 0, m = 0;
+                for (int q = 0; q < p.kw; ++q)
+                    if ((unsigned)(ix + q) < (unsigned)p.in_w) row |= 1u << q;
                 for (int r = 0; r < p.kh; ++r)
-                    for (int q = 0; q < p.kw; ++q)
-                        if ((unsigned)(iy + r) < (unsigned)p.in_h && (unsigned)(ix + q) < (unsigned)p.in_w) m |= 1u << (r * p.kw + q);
+                    if ((unsigned)(iy + r) < (unsigned)p.in_h) m |= row << (r * p.kw);
+                taps_in[nt][l] = pix < p.pixels ? m : 0;
+            } else {
+                xoff[nt][l] = pix < p.pixels ? (int)(pix * (unsigned)p.xs_b) + byte : kOutOfRange;
             }
-            taps_in[nt] = m;
-        } else {
-            xoff[nt] = pix < p.pixels ? (int)(pix * (unsigned)p.xs_b) + (lane >> 5) * 16 : kOutOfRange;
         }
-    }
     // weight fragments: block kb of slab kb / mts lies at ((slab * n_ksteps + ks) * mts + kb % mts) KiB; the MT blocks
     // of a wave are neighbours in one slab (mts, 2 or 4, is a multiple of MT)
     const int w_step = p.mts * 1024, slab = kb0 >> (p.mts >> 1);
@@ -402,37 +408,70 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
     auto request = [&](auto buf_c, int ks0) {
         constexpr int buf = decltype(buf_c)::value;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
+        for (int u = 0; u < U; u += XL) {
             if (ks0 + (u & ~1) >= nks) continue;
+            const int at = (ks0 + u) / XL < kMaxDirectSteps ? (ks0 + u) / XL : 0, entry = TAPS ? p.step[at] : 0;
+            const int ws = TAPS && PAIRS ? p.pair_first[at] : ks0 + u;
 #pragma unroll
-            for (int m = 0; m < MT; ++m)
-                a[buf][u][m] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, woff + m * 1024, w_base + (ks0 + u) * w_step, 0));
-            if constexpr (TAPS) {
-                const int entry = p.step[ks0 + u < kMaxDirectSteps ? ks0 + u : 0];
-                const int off = entry & ((1 << kTapShift) - 1);
-                const unsigned bit = 1u << ((unsigned)entry >> kTapShift);
+            for (int l = 0; l < XL; ++l)
 #pragma unroll
-                for (int n = 0; n < NT; ++n)
-                    b[buf][u][n] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(xr, (taps_in[n] & bit) ? xoff[n] + off : kOutOfRange, 0, 0));
-            } else {
+                for (int m = 0; m < MT; ++m)
+                    a[buf][u + l][m] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, woff + m * 1024, w_base + (ws + l * (PAIRS ? p.pair_w : 0)) * w_step, 0));
+            const int off = entry & ((1 << kTapShift) - 1);
+            const unsigned bit = 1u << ((unsigned)entry >> kTapShift);
 #pragma unroll
-                for (int n = 0; n < NT; ++n)
-                    b[buf][u][n] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(xr, xoff[n], (ks0 + u) * 32, 0));
-            }
+            for (int l = 0; l < XL; ++l)
+#pragma unroll
+                for (int n = 0; n < NT; ++n) {
+                    if constexpr (TAPS)
+                        b[buf][u + l][n] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(xr, (taps_in[n][l] & bit) ? xoff[n][l] + off : kOutOfRange, 0, 0));
+                    else
+                        b[buf][u + l][n] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(xr, xoff[n][l], (ks0 + u) * 32, 0));
+                }
         }
     };
-    auto step = [&](auto buf_c, int u) {
+    auto step = [&](auto buf_c, int u, const v4i (&xb)[NT]) {
         constexpr int buf = decltype(buf_c)::value;
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
             for (int n = 0; n < NT; ++n) {
                 if constexpr (DT == EXHIP_I8)
-                    acc[m][n] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[buf][u][m], b[buf][u][n], acc[m][n], 0, 0, 0);
+                    acc[m][n] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[buf][u][m], xb[n], acc[m][n], 0, 0, 0);
                 else
-                    acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a[buf][u][m]), __builtin_bit_cast(v8h, b[buf][u][n]),
+                    acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a[buf][u][m]), __builtin_bit_cast(v8h, xb[n]),
                                                                        acc[m][n], 0, 0, 0);
             }
+    };
+    // PAIRS: four k-steps at a time through the wave's own LDS, from four lanes a pixel to one
+    char* const stage_in = lds + param_bytes(MT) + (lane >> 2) * 64 + ((lane & 3) ^ (lane >> 3 & 3)) * 16;
+    const char* const stage_out = lds + param_bytes(MT) + (lane & 31) * 64;
+    // one round's products, of its k-steps below `left`
+    auto products = [&](auto buf_c, int left) {
+        constexpr int buf = decltype(buf_c)::value;
+        if constexpr (PAIRS) {
+#pragma unroll
+            for (int u0 = 0; u0 < U; u0 += 4) {
+                if (u0 >= left) continue;
+                v4i x[4][NT];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) *reinterpret_cast<v4i*>(stage_in + ((u >> 1) * NT + n) * 2048 + (u & 1) * 1024) = b[buf][u0 + u][n];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int n = 0; n < NT; ++n)
+                        x[u][n] = *reinterpret_cast<const v4i*>(stage_out + ((u >> 1) * NT + n) * 2048 + (((2 * (u & 1) + (lane >> 5)) ^ (lane >> 1 & 3)) * 16));
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (u < 2 || u0 + 2 < left) step(buf_c, u0 + u, x[u]);
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (u < left) step(buf_c, u, b[buf][u]);
+        }
     };
     using B0 = std::integral_constant<int, 0>;
     using B1 = std::integral_constant<int, 1>;
@@ -456,11 +495,9 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
     request(B1{}, U);
     int ks0 = 0;
     for (; ks0 + 2 * U < nks; ks0 += 2 * U) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) step(B0{}, u);
+        products(B0{}, U);
         request(B0{}, ks0 + 2 * U);
-#pragma unroll
-        for (int u = 0; u < U; ++u) step(B1{}, u);
+        products(B1{}, U);
         request(B1{}, ks0 + 3 * U);
     }
     // (the loop leaves with both rounds of the last 2 * U k-steps requested)
@@ -468,12 +505,8 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
 #pragma unroll
         for (int i = 0; i < kParams; ++i) *reinterpret_cast<float*>(lds + (i * MT * 32 + lane) * 4) = par[i];
     }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-        if (ks0 + u < nks) step(B0{}, u);
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-        if (ks0 + U + u < nks) step(B1{}, u);
+    products(B0{}, nks - ks0);
+    products(B1{}, nks - ks0 - U);
     pw_epilogue<DT, MT, NT, EP>(p, acc, tile * NT * 32, kb0, lane, lds);
 }
 
@@ -924,11 +957,11 @@ int go_dw(exhip_ctx* ctx, const PwParams& p) {
     return run(dw_pw_kernel<S, PX, EpAny>);
 }
 
-// U < 0: the split form, -kSplit a k-step at a time, -2 * kSplit in pairs
+// U > 0: the kernel with U k-steps a request round, 100 + U in pairs; U < 0: the split form, -kSplit a k-step at a time, -2 * kSplit in pairs
 template <int DT, int MT, int NT, int U, bool TAPS, typename EP>
 int go(exhip_ctx* ctx, const PwParams& p) {
     if constexpr (U < 0) hipLaunchKernelGGL((conv_pw_split_kernel<DT, MT, kSplit, TAPS, U == -2 * kSplit, EP>), dim3(p.items), dim3(64 * kSplit), 0, ctx->stream, p);
-    else hipLaunchKernelGGL((conv1x1_pw_kernel<DT, MT, NT, U, TAPS, EP>), dim3((p.items + 3) / 4), dim3(256), 0, ctx->stream, p);
+    else hipLaunchKernelGGL((conv1x1_pw_kernel<DT, MT, NT, U % 100, TAPS, (U > 100), EP>), dim3((p.items + 3) / 4), dim3(256), 0, ctx->stream, p);
     EXHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -974,11 +1007,11 @@ int pick_epilogue(exhip_ctx* ctx, const PwParams& p) {
 //    against 20.9), 16 k-steps 800 blocks 6.1 -> 4.6 (1600 6.30 against 6.40).
 //    8 k-steps: fp16 800 blocks 4.19 -> 4.05, 1600 4.5 against 5.1; int8 800 blocks 4.55 against 4.9.
 //  * a filter at stride 1, against the lean kernel: 1200 blocks fp16 9.2 -> 7.3 (36 k-steps), 12.8 -> 10.6 (72), 19.7 -> 18.0
-//    (144), int8 6.05 -> 4.95 (18), 9.7 -> 7.4 (36); 1600 blocks fp16 12.5 against 13.3 (72), int8 10.0 -> 9.0 (36), 11.5 against 13.4
-//    (72, but 20.3 -> 13.3 with an activation layer behind, 2400 blocks 21.1 -> 16.9, 3200 21.5 against 22.3).
-//  * a filter at stride 2, where the staged kernel and the tapped form compete: 3200 blocks fp16 16.8 -> 14.1 (36), 24.9 -> 24.1 (72),
-//    int8 10.6 -> 10.2 (18), 17.1 -> 14.3 (36); 64 k-steps and more: 1600 blocks 23.6 -> 14.0 (fp16, 72), 17.1 -> 12.2 (int8, 72 at
-//    1440 blocks; at 2160 16.9 against 17.4), 30.7 -> 23.7 (fp16, 144), 28.6 -> 23.8 (int8, 144).
+//    (144), int8 6.05 -> 4.95 (18), 9.7 -> 7.4 (36); 1600 blocks fp16 12.5 against 13.3 (72), int8 6.2 against 6.7 (18), 11.5 against
+//    13.4 (72, but 20.3 -> 13.3 with an activation layer behind, 2400 blocks 21.1 -> 16.9, 3200 21.5 against 22.3).
+//  * a filter at stride 2, against the tapped form: int8 1600 blocks 6.3 against 6.9 (18), 8.6 against 9.4 (36), fp16 3200 blocks 12.3
+//    against 14.1 (36), 20.0 against 24.5 (72); beyond the tapped form's k-steps against the staged kernel: 1600 blocks 30.7 -> 23.7
+//    (fp16, 144) and 28.6 -> 23.8 (int8, 144), 3200 blocks 38 and 35 against 42.
 // Layers without pairs (32-byte pixels, an odd number of chunks): 800 blocks. A lone 32-channel block would leave half of every tile
 // unused.
 bool split_wins(int dt, const exhip_pw_geom& g, int kblocks, int n_ksteps, bool taps, int stride) {
@@ -991,13 +1024,42 @@ bool split_wins(int dt, const exhip_pw_geom& g, int kblocks, int n_ksteps, bool 
         if (dt == EXHIP_I8) return blocks <= (n_ksteps < 16 ? 640 : n_ksteps < 32 ? 832 : 3328);
         return blocks <= (n_ksteps < 16 ? 832 : 6656);
     }
-    if (stride != 1) return blocks <= (n_ksteps < 16 ? 832 : n_ksteps < 64 ? 3328 : blocks * n_ksteps <= 240000 ? 1920 : 832);
-    if (dt == EXHIP_I8 && n_ksteps >= 32) return blocks <= (n_ksteps < 64 ? 1664 : g.post_op ? 2560 : 1280);
-    return blocks <= 1280;
+    if (stride != 1) return blocks <= (n_ksteps < 16 ? 832 : n_ksteps < 64 ? (dt == EXHIP_I8 ? 1280 : 1920) : blocks * n_ksteps <= 240000 ? 1920 : 832);
+    return blocks <= (dt == EXHIP_I8 && n_ksteps >= 64 && g.post_op ? 2560 : 1280);
+}
+
+// Where a pixel's bytes of a tap (of all channels for a 1x1 layer) come in whole 64-byte pieces, the k-steps are taken in pairs. A
+// packing in chunks of 32 bytes gives them too if the chunks are even in number: a pair's second k-step is the next chunk's then
+// (`any_order`: unsplit fp16 sums keep the order of the general kernel's, and so its bits).
+template <bool TAPS>
+bool plan_pairs(PwParams& p, bool any_order) {
+    const int taps = TAPS ? p.kh * p.kw : 1;
+    const bool two_chunks = TAPS && p.chunk_b == 32 && any_order && p.n_ksteps / taps % 2 == 0;
+    const bool pairs = two_chunks || (TAPS ? p.chunk_b : p.n_ksteps * 32) % 64 == 0;
+    if (two_chunks) {
+        p.chunk_end_b += 32;
+        p.chunk_b = 64;
+    }
+    p.pair_w = two_chunks ? taps : 1;
+    p.next_w = two_chunks ? 1 : 2;
+    p.chunk_w = two_chunks ? taps : 0;
+    return pairs;
 }
 
 template <int DT, int MT, int NT, bool TAPS = false>
 int launch(exhip_ctx* ctx, PwParams& p, int kblocks) {
+    // (two k-steps and no filter: pixels of 64 bytes, which lie side by side in the tensor: 64 -> 32 at 16 x 160 x 160 int8 9.6, in pairs 9.8)
+    const bool pairs = MT + NT <= 3 && (TAPS || p.n_ksteps >= 4) && plan_pairs<TAPS>(p, DT == EXHIP_I8);
+    if (TAPS) {
+        const int taps = p.kh * p.kw, per_tap = p.chunk_b / 32;
+        const int each = pairs ? 2 : 1;
+        if (p.n_ksteps > each * kMaxDirectSteps) return EXHIP_ERR_UNSUPPORTED;
+        for (int i = 0; i * each < p.n_ksteps; ++i) {
+            const int s = i * each, chunk = s / (taps * per_tap), tap = s / per_tap % taps, r = tap / p.kw, q = tap % p.kw;
+            p.step[i] = ((r * p.in_w + q) * p.xs_b + chunk * p.chunk_b + s % per_tap * 32) | (int)((unsigned)tap << kTapShift);
+            p.pair_first[i] = pairs && p.next_w == 1 ? chunk * 2 * taps + tap : s;
+        }
+    }
     const long long tiles = ((long long)p.pixels + 32 * NT - 1) / (32 * NT);
     p.ch_groups = (unsigned)((kblocks + MT - 1) / MT);
     const long long items = tiles * p.ch_groups;
@@ -1005,6 +1067,7 @@ int launch(exhip_ctx* ctx, PwParams& p, int kblocks) {
     p.items = (unsigned)items;
     exhip_host_divisor(p.ch_groups, &p.groups_magic, &p.groups_shift);
     if constexpr (MT + NT > 3) return go<DT, MT, NT, 2, TAPS, EpAny>(ctx, p);
+    else if (pairs) return pick_epilogue<DT, MT, NT, 104, TAPS>(ctx, p);
     // A launch of at most two waves per SIMD is as long as one wave's chain of load round trips: sixteen k-steps in flight
     // where there are more than eight. Larger ones hide each other's round trips and want the registers for more waves.
     else if (MT == 2 && items <= 2048 && p.n_ksteps > 8) return pick_epilogue<DT, MT, NT, 8, TAPS>(ctx, p);
@@ -1023,18 +1086,7 @@ int launch_split(exhip_ctx* ctx, PwParams& p, int kblocks) {
     if (items >= (1ll << 31) - 4) return EXHIP_ERR_UNSUPPORTED;
     p.items = (unsigned)items;
     exhip_host_divisor(p.ch_groups, &p.groups_magic, &p.groups_shift);
-    // Where a pixel's bytes of a tap (of all channels for a 1x1 layer) come in whole 64-byte pieces: pairs of k-steps, none of them
-    // shared. A packing in chunks of 32 bytes gives them too if the chunks are even in number: the pair's second k-step then
-    // is the next chunk's.
-    const bool pairs = TAPS ? p.chunk_b % 64 == 0 || p.n_ksteps / (p.kh * p.kw) % 2 == 0 : p.n_ksteps % 2 == 0, two_chunks = TAPS && pairs && p.chunk_b == 32;
-    const int taps = TAPS ? p.kh * p.kw : 1;
-    if (two_chunks) {
-        p.chunk_end_b += 32;
-        p.chunk_b = 64;
-    }
-    p.pair_w = two_chunks ? taps : 1;
-    p.next_w = two_chunks ? 1 : 2;
-    p.chunk_w = two_chunks ? taps : 0;
+    const bool pairs = plan_pairs<TAPS>(p, true), two_chunks = pairs && p.next_w == 1;
     for (int i = 0; i <= kSplit; ++i) {
         const int s = split_start(p.n_ksteps, pairs, i);
         p.start_s[i] = s;
@@ -1071,7 +1123,7 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
     if (g.post_bn_a || g.post_bn_b || g.exact_k || g.group) return EXHIP_ERR_UNSUPPORTED;
     const long long n_ksteps = (long long)t.n_chunks * t.kh * t.kw * (t.chunk_b / 32);
     if (g.pixels <= 0 || g.c_bytes <= 0 || g.c_bytes % 32 != 0 || t.chunk_b % 32 != 0 || t.n_chunks * t.chunk_b != g.c_bytes ||
-        (g.slab_blocks != 2 && g.slab_blocks != 4) || g.k_stride % 8 != 0 || !pw_row_fits(4ll * g.k_stride) || (n_ksteps > kMaxDirectSteps && !split_wins(DT, g, (std::max(g.k, g.k_stride) + 31) / 32, (int)n_ksteps, true, t.stride)) || t.kh * t.kw > (1 << (32 - kTapShift)) || t.stride < 1 || t.pad_t < 0 || t.pad_l < 0)
+        (g.slab_blocks != 2 && g.slab_blocks != 4) || g.k_stride % 8 != 0 || !pw_row_fits(4ll * g.k_stride) || (n_ksteps > (g.c_bytes % 64 ? 1 : 2) * kMaxDirectSteps && !split_wins(DT, g, (std::max(g.k, g.k_stride) + 31) / 32, (int)n_ksteps, true, t.stride)) || t.kh * t.kw > (1 << (32 - kTapShift)) || t.stride < 1 || t.pad_t < 0 || t.pad_l < 0)
         return EXHIP_ERR_UNSUPPORTED;
     const long long x_bytes = (long long)t.n * t.in_h * t.in_w * g.c_bytes;
     const long long w_bytes = (long long)g.slabs * n_ksteps * g.slab_blocks * 1024;
@@ -1082,14 +1134,18 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
     if (g.post_op && g.post_op != EXHIP_POST_PRELU && (g.post_op < 1 || g.post_op > 1 + EXHIP_UNARY_CLIP || g.post_op == 1 + EXHIP_UNARY_SIGMOID))
         return EXHIP_ERR_UNSUPPORTED;
     const int kblocks = std::min(g.slabs * g.slab_blocks, (std::max(g.k, g.k_stride) + 31) / 32);
-    // Measured inside two detection networks at 16 x 3 x 640 x 640 and two mobile networks: the fp16 layers the lean
-    // kernel leaves (stride 2, 12 or 32 input channels, ragged output channels) are faster here as a whole (0.88 -> 0.85 ms
-    // and 1.83 -> 1.81 ms per forward of the detection networks); of the int8 layers only a few deep ones are (3x3
-    // stride 2 from 40 x 40: 29 -> 23 us) while the wide first layers lose (12 -> 32 channels at 320 x 320: 81 -> 94 us),
-    // so wide int8 layers stay with the staged kernels unless the option asks or the split form takes them.
-    // A lone 32-channel block wins whatever its size (12 -> 32 at 16 x 320 x 320: int8 71 -> 46 us, fp16 66 -> 45; 32 -> 32 at
-    // 160 x 160: one image 8.1 -> 5.3 us, sixteen 24.9 -> 15.8).
-    const bool take = kblocks == 1 || DT == EXHIP_F16 || g.c_bytes == 32 || (g.pixels <= 32768 && kblocks <= 4) || g.pixels <= 6400;
+    // Every fp16 layer that the lean kernel leaves (stride 2, 12 or 32 input channels, ragged output channels): 128 -> 256 3x3 at stride
+    // 2 from 16 x 80 x 80 48.6 us on the staged kernel, 36.9 here; 64 -> 128 from 16 x 160 x 160 71.9 and 35.8. A lone 32-channel block and
+    // 32-byte pixels win whatever their size (12 -> 32 at 16 x 320 x 320 int8 71 -> 46 us, 32 -> 32 at 16 x 160 x 160 24.9 -> 15.8).
+    // Other int8 layers up to 3328 blocks of 32 x 32: at stride 2 and 3200 blocks 14.5 -> 12.2 us (36 k-steps), 27.6 -> 20.2 (72), 18.9
+    // -> 8.2 (18); at 6400 blocks 17.1 against 21.5. At stride 1 the lean kernel's forms differ: with a plain ReLU it takes 8.7 us for
+    // 128 -> 128 at 16 x 40 x 40 where this one takes 12.2, with the ReLU behind 13.7, with a sum 17.2 (15.0 here), with an
+    // activation layer 17.8; up to 64 input channels also the ReLU behind and sums are faster there (64 x 30 x 30: 6.3 against 8.5,
+    // 10.4 against 11.4).
+    const long long blocks = (g.pixels + 31) / 32 * kblocks;
+    const bool lean_wins = t.kh == 3 && t.kw == 3 && t.stride == 1 && t.chunk_b == 64 && g.k % 64 == 0 && !g.post_op &&
+                           (n_ksteps <= 18 || (!g.post_relu && !has_residual));
+    const bool take = kblocks == 1 || DT == EXHIP_F16 || g.c_bytes == 32 || (blocks <= 3328 && !lean_wins);
     const bool split = split_wins(DT, g, kblocks, (int)n_ksteps, true, t.stride);
     if (g_exhip_options.direct != 2 && !take && !split) return EXHIP_ERR_UNSUPPORTED;
     p.post_slope = g.post_slope;
@@ -1107,12 +1163,6 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
     p.row_end_b = (t.in_w - t.kw) * g.c_bytes;
     p.chunk_end_b = t.chunk_b - t.kh * t.in_w * g.c_bytes;
     if (split) return launch_split<DT, true>(ctx, p, kblocks);
-    int s = 0;
-    for (int cc = 0; cc < t.n_chunks; ++cc)
-        for (int r = 0; r < t.kh; ++r)
-            for (int q = 0; q < t.kw; ++q)
-                for (int j = 0; j < t.chunk_b / 32; ++j)
-                    p.step[s++] = ((r * t.in_w + q) * g.c_bytes + cc * t.chunk_b + j * 32) | (int)((unsigned)(r * t.kw + q) << kTapShift);
     if (kblocks == 1) return launch<DT, 1, 2, true>(ctx, p, kblocks);
     const long long waves64 = ((g.pixels + 63) / 64) * ((kblocks + 1) / 2);
     if (waves64 < 2048 || small_tile<DT>()) return launch<DT, 2, 1, true>(ctx, p, kblocks);
