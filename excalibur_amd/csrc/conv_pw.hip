@@ -1137,15 +1137,26 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
     // Every fp16 layer that the lean kernel leaves (stride 2, 12 or 32 input channels, ragged output channels): 128 -> 256 3x3 at stride
     // 2 from 16 x 80 x 80 48.6 us on the staged kernel, 36.9 here; 64 -> 128 from 16 x 160 x 160 71.9 and 35.8. A lone 32-channel block and
     // 32-byte pixels win whatever their size (12 -> 32 at 16 x 320 x 320 int8 71 -> 46 us, 32 -> 32 at 16 x 160 x 160 24.9 -> 15.8).
-    // Other int8 layers up to 3328 blocks of 32 x 32: at stride 2 and 3200 blocks 14.5 -> 12.2 us (36 k-steps), 27.6 -> 20.2 (72), 18.9
-    // -> 8.2 (18); at 6400 blocks 17.1 against 21.5. At stride 1 the lean kernel's forms differ: with a plain ReLU it takes 8.7 us for
-    // 128 -> 128 at 16 x 40 x 40 where this one takes 12.2, with the ReLU behind 13.7, with a sum 17.2 (15.0 here), with an
-    // activation layer 17.8; up to 64 input channels also the ReLU behind and sums are faster there (64 x 30 x 30: 6.3 against 8.5,
-    // 10.4 against 11.4).
+    // Other int8 layers by what stands behind the products, us on the staged or lean kernel -> here, over some 60 maps from 16 to 111 wide:
+    //  * stride 2: everything, 27.5 -> 21.9 (256 -> 256 at 48 x 37 x 34), 17.4 -> 11.1 with a float32 result (64 -> 128 at 48 x 50 x 47) --
+    //    but with an int8 result alone large maps in powers of two stay (128 -> 256 at 16 x 80 x 80 17.1 against 21.5): up to 4800
+    //    blocks of 32 x 32 (17.9 -> 16.8).
+    //  * stride 1, where the lean kernel takes a plain ReLU in 8.7 us for 128 -> 128 at 16 x 40 x 40 and this one in 12.2: an activation
+    //    layer (17.8 -> 12.0; 64 -> 64 at 8 x 80 x 80 9.9 -> 8.1, at 16 x 80 x 80 12.2 against 13.4), a float32 result beside the
+    //    int8 one (20.9 -> 14.6 at 4 x 80 x 80, 40.5 -> 40.2 at 11 856 blocks; 72 k-steps 27.9 -> 23.6 at 4096, 37.1 against 40.4 at
+    //    6400), a sum (17.6 -> 15.3 at 3200, 20.8 against 21.4 at 4376; 18 k-steps 8.8 -> 8.4 at 1944, 9.2 against 10.8 at 2376; 72 never),
+    //    the ReLU behind (13.7 -> 12.2; 18 k-steps never).
     const long long blocks = (g.pixels + 31) / 32 * kblocks;
-    const bool lean_wins = t.kh == 3 && t.kw == 3 && t.stride == 1 && t.chunk_b == 64 && g.k % 64 == 0 && !g.post_op &&
-                           (n_ksteps <= 18 || (!g.post_relu && !has_residual));
-    const bool take = kblocks == 1 || DT == EXHIP_F16 || g.c_bytes == 32 || (blocks <= 3328 && !lean_wins);
+    auto int8_most = [&]() -> long long {
+        const long long all = 1ll << 40;
+        if (t.stride != 1) return g.post_op || has_residual || p.y_f ? all : 4800;
+        if (t.kh != 3 || t.kw != 3 || t.chunk_b != 64 || g.k % 64 != 0) return 3328;  // the staged kernel's
+        if (g.post_op) return n_ksteps <= 40 ? 4096 : 3328;
+        if (has_residual) return n_ksteps <= 18 ? 2048 : n_ksteps <= 40 ? 3328 : 0;
+        if (p.y_f) return n_ksteps <= 40 ? 12000 : 4096;
+        return g.post_relu && n_ksteps > 18 ? 3328 : 0;
+    };
+    const bool take = kblocks == 1 || DT == EXHIP_F16 || g.c_bytes == 32 || blocks <= int8_most();
     const bool split = split_wins(DT, g, kblocks, (int)n_ksteps, true, t.stride);
     if (g_exhip_options.direct != 2 && !take && !split) return EXHIP_ERR_UNSUPPORTED;
     p.post_slope = g.post_slope;
