@@ -130,6 +130,19 @@ def test_placements_for_every_tile_and_split(ctx, tile, args):
     assert np.abs(got[:-64].reshape(expect.shape) - expect).max() < 2.2e-5 * max(1.0, np.abs(want).max())
 
 
+PAIRS = [  # 1x1 layers that take the pixels two steps at a time
+    (910, 1, 16, 9, 5, 40, 1, 1, 0, 16, 64, False),      # a single pair for all waves
+    (911, 3, 48, 13, 13, 96, 1, 1, 0, 48, 96, True),     # three pairs
+    (912, 2, 80, 11, 7, 33, 1, 2, 0, 96, 33, False),     # every other pixel, five pairs of a wider pixel, unaligned rows
+    (913, 1, 272, 7, 7, 64, 1, 1, 0, 272, 64, True),     # 34 steps: runs of eight and ten
+]
+
+
+@pytest.mark.parametrize("args", PAIRS, ids=[f"s{a[0]}" for a in PAIRS])
+def test_conv_f32_pairs_of_steps(ctx, tile, args):
+    test_conv_f32_tiles_and_splits(ctx, tile, args)
+
+
 def test_the_plain_entry_refuses_what_only_the_placed_one_does(ctx):
     """A BatchNorm in the epilogue and writes limited to the layer's own channels: refused, nothing written."""
     c, k, hw = 32, 32, 5
