@@ -87,7 +87,7 @@ struct PwParams {
     const float* dw_w;
     const float* dw_bias;
     const float* dw_slope;
-    int dw_act, dw_slope_shared, dw_tiles, dw_kblocks, dw_split, kblocks;
+    int dw_act, dw_slope_shared, dw_pixels, dw_tiles, dw_kblocks, dw_split, dw_mid, kblocks;  // dw_mid: where its results begin in LDS
 };
 
 __device__ __noinline__ float slow_activation(float v, int act) { return exhip_act(v, act); }
@@ -222,7 +222,7 @@ __device__ __forceinline__ void layers_behind(const PwParams& p, float (&v)[N], 
 }
 
 template <int DT, int MT, int NT, typename EP, typename ACC>
-__device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[MT][NT], unsigned pix0, int kb0, int lane, char* lds) {
+__device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[MT][NT], unsigned pix0, unsigned end, int kb0, int lane, char* lds) {
     constexpr bool I8 = DT == EXHIP_I8, ANY = EP::any;
     constexpr int ES = I8 ? 4 : 2;  // bytes per value of the shortcut tensor
     const int half = lane >> 5, row = lane & 31;
@@ -246,8 +246,8 @@ __device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
         const unsigned first = pix0 + n * 32;
-        if (n > 0 && first >= p.pixels) continue;
-        const int rows = p.pixels - first < 32 ? (int)(p.pixels - first) : 32;
+        if (n > 0 && first >= end) continue;
+        const int rows = end - first < 32 ? (int)(end - first) : 32;
         v4i r[MT][ES];
         if (shortcut) {
             // a channel group beyond the tensor's stride reads zeros; pad channels inside it read what lies there and are
@@ -507,7 +507,7 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
     }
     products(B0{}, nks - ks0);
     products(B1{}, nks - ks0 - U);
-    pw_epilogue<DT, MT, NT, EP>(p, acc, tile * NT * 32, kb0, lane, lds);
+    pw_epilogue<DT, MT, NT, EP>(p, acc, tile * NT * 32, p.pixels, kb0, lane, lds);
 }
 
 // The split form, for launches of few tiles and many k-steps (one image, deep layers), where the kernel above is as long as one
@@ -745,7 +745,7 @@ __global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParam
         acc_t sum[1][1];
 #pragma unroll
         for (int e = 0; e < 16; ++e) sum[0][0][e] = total[e];
-        pw_epilogue<DT, 1, 1, EP>(p, sum, tile * 32, kb, lane, lds);
+        pw_epilogue<DT, 1, 1, EP>(p, sum, tile * 32, p.pixels, kb, lane, lds);
     } else {
         float v[N], scale[N], bias[N];
         if constexpr (I8) read_parameters<1>(lds, 0, ch, scale);
@@ -795,16 +795,18 @@ __global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParam
 }
 
 // A depthwise 3x3 layer and the pointwise layer that alone reads it, the depthwise results staying in LDS. A group computes
-// all C channels of 32 * dw_tiles output pixels -- a thread owns four channels of strips of PX pixels, the arithmetic and roundings
-// of dwconv3x3_nhwc_strip_kernel -- and its four waves then take the tile's 32 x 32 output blocks, pixel fragments from LDS, weight
-// fragments from L2 with R k-steps in flight. A small launch deals the output channels over several groups, each with depthwise
-// results of its own. A layer that the split form above would take (dw_split) adds its four runs of k-steps in that form's order.
-// Bound by a launch's fixed cost where it is small, by the depthwise loads where it is large: 64 x 128 x 56 x 56 takes 43 us (61 as two
-// launches), 1 x 64 x 56 x 56 takes 4.6 us (9.0).
+// all C channels of dw_pixels output pixels -- a thread owns four channels of strips of PX pixels, the arithmetic and roundings
+// of dwconv3x3_nhwc_strip_kernel -- and its four waves then take the pixels' 32 x 32 output blocks (of fewer than 32 pixels the
+// block's other columns repeat them and are not stored), pixel fragments from LDS, weight fragments from L2 with R k-steps in flight;
+// SMALL, a launch of few groups, asks for the first of them before the depthwise half. A small launch deals the output channels over
+// several groups, each with depthwise results of its own. A layer that the split form above would take (dw_split) adds its four
+// runs of k-steps in that form's order. Bound by the chain of one group where it is small (1 x 64 x 56 x 56 takes 3.9 us, 7.7 as two launches;
+// 256 -> 128 at 1 x 14 x 14 5.2 and 8.2), by the depthwise loads where it is large (64 x 128 x 56 x 56 -> 64: 33.8 us and 47.5; 40.3 when
+// every thread read its 36 weights by itself and 64 pixels a group were the most).
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
 
-template <int S, int PX, typename EP>
+template <int S, int PX, bool SMALL, typename EP>
 __global__ __launch_bounds__(256, 3) void dw_pw_kernel(const PwParams p) {
     exhip_touch_args(p);
     constexpr int R = 4, NC = (PX - 1) * S + 3;
@@ -818,44 +820,87 @@ __global__ __launch_bounds__(256, 3) void dw_pw_kernel(const PwParams p) {
     }
     const unsigned tile = __builtin_amdgcn_readfirstlane(exhip_divide(item0, p.ch_groups, p.groups_magic, p.groups_shift));
     const int kb_first = __builtin_amdgcn_readfirstlane((int)(item0 - tile * p.ch_groups) * p.dw_kblocks);
-    const unsigned pix0 = tile * 32 * p.dw_tiles;
+    const unsigned pix0 = tile * p.dw_pixels, pix_end = min(p.pixels, pix0 + p.dw_pixels);
     char* const lds = lds_dyn + wave * wave_bytes(EXHIP_F16, 1);
-    char* const mid = lds_dyn + 4 * wave_bytes(EXHIP_F16, 1);
+    char* const mid = lds_dyn + p.dw_mid;
     const int mid_pitch = p.xs_b + 16;
+    const int nks = p.n_ksteps, w_step = p.mts * 1024;
+    const int blocks = p.kblocks - kb_first < p.dw_kblocks ? p.kblocks - kb_first : p.dw_kblocks;
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.wp), 0, (int)p.w_bytes, kRsrcWord3);
+    v4i a[R];
+    float par[kParams] = {};
+    auto weights_at = [&](int kb) { return ((kb >> (p.mts >> 1)) * nks * p.mts + (kb & (p.mts - 1))) * 1024; };
+    auto request = [&](int w_base, int u, int s) {
+        a[u] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, lane * 16, w_base + (s < nks ? s : nks - 1) * w_step, 0));
+    };
+    auto load_parameters = [&](int kb) {
+        const int at = lane < 32 ? (kb * 32 + lane) * 4 : kOutOfRange;
+        auto load = [&](const float* src, int offset, int count) {
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src), 0, src ? count * 4 : 0, kRsrcWord3);
+            return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, offset, 0, 0));
+        };
+        par[1] = load(p.bias, at, p.K);
+        if (EP::any || EP::post == kPostPrelu) par[2] = load(p.post_slope, p.post_slope_shared ? 0 : at, p.post_slope_shared ? 1 : p.K);
+    };
     {
         const int groups = p.xs_b >> 3, g = threadIdx.x % groups, lanes = 256 / groups, first = threadIdx.x / groups;
-        const int strips = first < lanes ? 32 * p.dw_tiles / PX : 0;
+        const int strips = first < lanes ? p.dw_pixels / PX : 0;
         const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.x), 0, (int)p.x_bytes, kRsrcWord3);
-        float k[36], b[4] = {0.f, 0.f, 0.f, 0.f}, sl[4] = {0.f, 0.f, 0.f, 0.f};
+        const unsigned per_image = (unsigned)(p.out_h * p.out_w);
+        const int row_b = p.in_w * p.xs_b;
+        // The 36 weights of a thread's four channels lie 144 bytes from the next thread's: read so, each load is 64 lines and takes
+        // its CU 64 cycles. The group's threads read them side by side instead and take their own from LDS.
+        v4f* const wk = reinterpret_cast<v4f*>(lds_dyn);
+        constexpr int kAhead = 2;   // 16-byte pieces a thread has in flight
+        const int pieces = groups * 9;
+        v4f piece[kAhead];
 #pragma unroll
-        for (int q = 0; q < 9; ++q) {
-            const v4f t = reinterpret_cast<const v4f*>(p.dw_w + g * 36)[q];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) k[q * 4 + e] = t[e];
-        }
+        for (int q = 0; q < kAhead; ++q) piece[q] = reinterpret_cast<const v4f*>(p.dw_w)[min((int)threadIdx.x + q * 256, pieces - 1)];
+        float b[4] = {0.f, 0.f, 0.f, 0.f}, sl[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             if (p.dw_bias) b[e] = p.dw_bias[g * 4 + e];
             if (p.dw_slope) sl[e] = p.dw_slope[p.dw_slope_shared ? 0 : g * 4 + e];
         }
-        const unsigned per_image = (unsigned)(p.out_h * p.out_w);
-        const int row_b = p.in_w * p.xs_b;
-        for (int st = first; st < strips; st += lanes) {
+        auto load = [&](int st, v4h (&r)[3][NC]) {
             const unsigned pix = pix0 + st * PX;
             const unsigned img = exhip_divide(pix, per_image, p.image_magic, p.image_shift), rem = pix - img * per_image;
             const int oy = (int)exhip_divide(rem, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = (int)(rem - (unsigned)oy * (unsigned)p.out_w);
-            const int iy = pix < p.pixels ? oy * S - p.pad_t : -4, ix = ox * S - p.pad_l;
+            const int iy = pix < p.pixels && st < strips ? oy * S - p.pad_t : -4, ix = ox * S - p.pad_l;
             const unsigned at = img * (unsigned)(p.in_h * row_b) + g * 8;
             unsigned row_off[3], col_off[NC];
 #pragma unroll
             for (int a = 0; a < 3; ++a) row_off[a] = (unsigned)(iy + a) < (unsigned)p.in_h ? at + (unsigned)((iy + a) * row_b) : kRowOutside;
 #pragma unroll
             for (int c = 0; c < NC; ++c) col_off[c] = (unsigned)(ix + c) < (unsigned)p.in_w ? (unsigned)((ix + c) * p.xs_b) : kColOutside;
-            v4h r[3][NC];
 #pragma unroll
             for (int a = 0; a < 3; ++a)
 #pragma unroll
                 for (int c = 0; c < NC; ++c) r[a][c] = __builtin_bit_cast(v4h, __builtin_amdgcn_raw_buffer_load_b64(xr, (int)(row_off[a] + col_off[c]), 0, 0));
+        };
+        v4h r[3][NC];
+        load(first, r);
+        if constexpr (SMALL) {  // the pointwise layer's first weights are on their way while the depthwise results are made
+            if (wave < blocks) {
+#pragma unroll
+                for (int u = 0; u < R; ++u) request(weights_at(kb_first + wave), u, u);
+                load_parameters(kb_first + wave);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < kAhead; ++q)
+            if ((int)threadIdx.x + q * 256 < pieces) wk[threadIdx.x + q * 256] = piece[q];
+        for (int i = threadIdx.x + kAhead * 256; i < pieces; i += 256) wk[i] = reinterpret_cast<const v4f*>(p.dw_w)[i];
+        __syncthreads();
+        float k[36];
+#pragma unroll
+        for (int q = 0; q < 9; ++q) {
+            const v4f t = wk[g * 9 + q];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) k[q * 4 + e] = t[e];
+        }
+        auto compute = [&](int st, const v4h (&r)[3][NC]) {
 #pragma unroll
             for (int px = 0; px < PX; ++px) {
                 v4f res;
@@ -887,37 +932,27 @@ __global__ __launch_bounds__(256, 3) void dw_pw_kernel(const PwParams p) {
                 const v2i o = {(int)round_pair(res[0], res[1]), (int)round_pair(res[2], res[3])};
                 *reinterpret_cast<v2i*>(mid + (st * PX + px) * mid_pitch + g * 8) = o;
             }
+        };
+        for (int st = first; st < strips; st += lanes) {
+            compute(st, r);
+            if (st + lanes < strips) load(st + lanes, r);
         }
     }
     __syncthreads();
-    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.wp), 0, (int)p.w_bytes, kRsrcWord3);
-    const int blocks = p.kblocks - kb_first < p.dw_kblocks ? p.kblocks - kb_first : p.dw_kblocks;
-    const int nks = p.n_ksteps, w_step = p.mts * 1024;
     for (int item = wave; item < blocks * p.dw_tiles; item += 4) {
-        const int sub = item & (p.dw_tiles - 1), kb = kb_first + (item >> (p.dw_tiles - 1));
+        const int sub = item & (p.dw_tiles - 1), kb = kb_first + (item >> __builtin_ctz(p.dw_tiles));
         const unsigned first = pix0 + sub * 32;
         if (first >= p.pixels) continue;  // wave-uniform; no barrier follows
-        const int w_base = ((kb >> (p.mts >> 1)) * nks * p.mts + (kb & (p.mts - 1))) * 1024;
-        v4i a[R];
-        auto request = [&](int u, int s) {
-            a[u] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, lane * 16, w_base + (s < nks ? s : nks - 1) * w_step, 0));
-        };
+        const int w_base = weights_at(kb);
+        if (!SMALL || item != wave) {
 #pragma unroll
-        for (int u = 0; u < R; ++u) request(u, u);
-        float par[kParams] = {};
-        {
-            const int at = lane < 32 ? (kb * 32 + lane) * 4 : kOutOfRange;
-            auto load = [&](const float* src, int offset, int count) {
-                const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src), 0, src ? count * 4 : 0, kRsrcWord3);
-                return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, offset, 0, 0));
-            };
-            par[1] = load(p.bias, at, p.K);
-            if (EP::any || EP::post == kPostPrelu) par[2] = load(p.post_slope, p.post_slope_shared ? 0 : at, p.post_slope_shared ? 1 : p.K);
+            for (int u = 0; u < R; ++u) request(w_base, u, u);
+            load_parameters(kb);
         }
         v16f acc, sum[1][1];
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[e] = sum[0][0][e] = 0.f;
-        const char* src = mid + (sub * 32 + (lane & 31)) * mid_pitch + (lane >> 5) * 16;
+        const char* src = mid + (sub * 32 + (lane & 31 & (p.dw_pixels - 1))) * mid_pitch + (lane >> 5) * 16;
         int run = 1, end = p.dw_split ? p.start_s[1] : nks;
         for (int s = 0; s < nks; s += R) {
 #pragma unroll
@@ -930,7 +965,7 @@ __global__ __launch_bounds__(256, 3) void dw_pw_kernel(const PwParams p) {
                     }
                     acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a[u]), *reinterpret_cast<const v8h*>(src + (s + u) * 32), acc, 0, 0, 0);
                 }
-                request(u, s + R + u);
+                request(w_base, u, s + R + u);
             }
         }
 #pragma unroll
@@ -939,22 +974,25 @@ __global__ __launch_bounds__(256, 3) void dw_pw_kernel(const PwParams p) {
 #pragma unroll
             for (int i = 0; i < kParams; ++i) *reinterpret_cast<float*>(lds + (i * 32 + lane) * 4) = par[i];
         }
-        pw_epilogue<EXHIP_F16, 1, 1, EP>(p, sum, first, kb, lane, lds);
+        pw_epilogue<EXHIP_F16, 1, 1, EP>(p, sum, first, pix_end, kb, lane, lds);
     }
 }
 
-template <int S, int PX>
-int go_dw(exhip_ctx* ctx, const PwParams& p) {
-    const int lds = 4 * wave_bytes(EXHIP_F16, 1) + 32 * p.dw_tiles * (p.xs_b + 16);
+template <int S, int PX, bool SMALL>
+int go_dw(exhip_ctx* ctx, PwParams& p) {
+    // the depthwise weights, later the waves' epilogue slices; behind them the depthwise results
+    p.dw_mid = std::max(4 * wave_bytes(EXHIP_F16, 1), p.xs_b / 8 * 144);
+    const int lds = p.dw_mid + p.dw_pixels * (p.xs_b + 16);
     auto run = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(p.items), dim3(256), lds, ctx->stream, p);
         EXHIP_LAUNCH_CHECK();
         return 0;
     };
     const int res = !p.residual ? 0 : p.residual_last ? 2 : 1;
-    if (!p.post_relu && !p.post_op && p.act == 0 && res < 2) return res ? run(dw_pw_kernel<S, PX, Ep<0, kPostNone, 1>>) : run(dw_pw_kernel<S, PX, Ep<0, kPostNone, 0>>);
-    if (!p.post_relu && p.act == 0 && p.post_op == EXHIP_POST_PRELU && res == 0) return run(dw_pw_kernel<S, PX, Ep<0, kPostPrelu, 0>>);
-    return run(dw_pw_kernel<S, PX, EpAny>);
+    if (!p.post_relu && !p.post_op && p.act == 0 && res < 2)
+        return res ? run(dw_pw_kernel<S, PX, SMALL, Ep<0, kPostNone, 1>>) : run(dw_pw_kernel<S, PX, SMALL, Ep<0, kPostNone, 0>>);
+    if (!p.post_relu && p.act == 0 && p.post_op == EXHIP_POST_PRELU && res == 0) return run(dw_pw_kernel<S, PX, SMALL, Ep<0, kPostPrelu, 0>>);
+    return run(dw_pw_kernel<S, PX, SMALL, EpAny>);
 }
 
 // U > 0: the kernel with U k-steps a request round, 100 + U in pairs; U < 0: the split form, -kSplit a k-step at a time, -2 * kSplit in pairs
@@ -1193,27 +1231,44 @@ int run_depthwise(exhip_ctx* ctx, const exhip_pw_depthwise& dw, PwParams& p, int
     exhip_host_divisor((unsigned)(dw.out_h * dw.out_w), &p.image_magic, &p.image_shift);
     exhip_host_divisor((unsigned)dw.out_w, &p.width_magic, &p.width_shift);
     const long long tiles32 = ((long long)p.pixels + 31) / 32;
-    // A thread that computes more than four strips of a tile one behind the other makes the depthwise half the longer one (1 x 512 x 22 x 22
-    // at stride 2: 15.6 against 9.5 us for two launches; 1 x 256 x 22 x 22: 10.3 against 11.0; 64 x 512 x 14 x 14 at stride 2: 20.6
-    // against 16.6). Beyond 128 tiles, where a launch's fixed 4 us no longer count, a widening layer loses as well: its depthwise half
-    // waits behind the stores of the wider result (64 x 32 x 112 x 112 -> 64: 81 against 67 us). The others win (64 x 128 x 56 x 56: 43
-    // against 61 us).
-    const int pixels = dw.stride == 2 ? 2 - dw.out_w % 2 : dw.out_w % 4 == 0 ? 4 : 2 - dw.out_w % 2;
-    const bool long_strips = 32 / pixels * (p.xs_b >> 3) > 4 * 256;
-    if (g_exhip_options.dw_pw != 2 && (long_strips || (tiles32 > 128 && kblocks * 64 > p.xs_b))) return EXHIP_ERR_UNSUPPORTED;
-    p.dw_tiles = p.xs_b <= 512 && tiles32 >= 1024 ? 2 : 1;
-    const long long tiles = (tiles32 + p.dw_tiles - 1) / p.dw_tiles;
+    const int widest = dw.stride == 2 ? 2 - dw.out_w % 2 : dw.out_w % 4 == 0 ? 4 : 2 - dw.out_w % 2, channels4 = p.xs_b >> 3;
+    p.kblocks = kblocks;
+    p.dw_split = split;
+    for (int i = 0; i <= kSplit; ++i) p.start_s[i] = split_start(p.n_ksteps, p.n_ksteps % 2 == 0, i);
+    // Pixels of a group. A small launch is as long as one group's chain, a strip of four channels that a thread computes behind another
+    // 0.8 us of it: while the chip has room, groups of half the pixels (256 -> 128 at 1 x 14 x 14: 8.0 us with 32 pixels, 6.5 with
+    // 16, 5.5 with 8, 5.2 with 4; 512 -> 128 at 1 x 7 x 7: 14.6, 10.1, 8.2, 7.1), but a second round of groups costs what
+    // it saves (256 -> 128 at 16 x 14 x 14: 8.3 with 32, 6.6 with 16 in 196 groups, 6.8 with 8 in 392) unless the strips are many (512 ->
+    // 128 at 64 x 7 x 7: 10.5 with 16, 9.8 with 8 in 392). A large launch wants a strip for every thread and no more: 16 -> 32 at
+    // 64 x 112 x 112 24.5 us with 256 pixels, 33.6 with 128, 55.5 with 64; 32 -> 64 43.7 with 128, 61.8 with 64; 128 -> 64 at 64 x 56 x 56
+    // 33.8 with 64, 39.3 with 32; 256 -> 128 at 64 x 28 x 28 27.7 with 64, 22.7 with 32.
+    p.dw_pixels = 32;
+    if (tiles32 >= 1024)
+        while (p.dw_pixels < 256 && p.dw_pixels * channels4 < (channels4 < 24 ? 1024 : 2048)) p.dw_pixels *= 2;
+    auto more = [&]() { return ((long long)p.pixels * 2 + p.dw_pixels - 1) / p.dw_pixels * ((kblocks + 3) / 4); };  // groups with half the pixels each
+    while (p.dw_pixels > 4 && p.dw_pixels * channels4 > 256 && more() <= (p.dw_pixels * channels4 > 1024 ? 512 : 256)) p.dw_pixels /= 2;
+    if (const int forced = g_exhip_options.dw_pw; forced >= 4 && forced <= 256 && (forced & (forced - 1)) == 0 && forced * (p.xs_b + 16) <= 40960) p.dw_pixels = forced;
+    const bool small = p.dw_pixels < 32;
+    // One launch is the faster one but for wide layers of a middling size, whose groups are few and long: 512 -> 512 at 20 x 14 x 14 16.6 us,
+    // 15.8 as two launches, 384 -> 384 at 8 x 14 x 14 10.8 and 9.9, 256 -> 512 at stride 2 from 8 x 28 x 28 8.2 and 7.8; on the other
+    // sides 512 -> 512 at 1 x 14 x 14 6.8 and 8.9, at 64 x 14 x 14 27.0 and 31.0, 512 -> 128 at 64 x 7 x 7 10.1 and 10.5.
+    if (g_exhip_options.dw_pw == 1 && tiles32 > 40 && tiles32 <= 256 && kblocks > (p.xs_b > 512 ? 4 : 8)) return EXHIP_ERR_UNSUPPORTED;
+    p.dw_tiles = std::max(p.dw_pixels / 32, 1);
+    const long long tiles = ((long long)p.pixels + p.dw_pixels - 1) / p.dw_pixels;
     int groups = 1;
     while (groups * 4 < kblocks * p.dw_tiles && tiles * groups * 2 <= 512) groups *= 2;
-    p.kblocks = kblocks;
     p.dw_kblocks = (kblocks + groups - 1) / groups;
     p.ch_groups = (unsigned)((kblocks + p.dw_kblocks - 1) / p.dw_kblocks);
     p.items = (unsigned)(tiles * p.ch_groups);
     exhip_host_divisor(p.ch_groups, &p.groups_magic, &p.groups_shift);
-    p.dw_split = split;
-    for (int i = 0; i <= kSplit; ++i) p.start_s[i] = split_start(p.n_ksteps, p.n_ksteps % 2 == 0, i);
-    if (dw.stride == 2) return pixels == 2 ? go_dw<2, 2>(ctx, p) : go_dw<2, 1>(ctx, p);
-    return pixels == 4 ? go_dw<1, 4>(ctx, p) : pixels == 2 ? go_dw<1, 2>(ctx, p) : go_dw<1, 1>(ctx, p);
+    if (small) {
+        int px = 1;
+        while (px < widest && p.dw_pixels * channels4 / px > 256) px *= 2;
+        if (dw.stride == 2) return px == 2 ? go_dw<2, 2, true>(ctx, p) : go_dw<2, 1, true>(ctx, p);
+        return px == 4 ? go_dw<1, 4, true>(ctx, p) : px == 2 ? go_dw<1, 2, true>(ctx, p) : go_dw<1, 1, true>(ctx, p);
+    }
+    if (dw.stride == 2) return widest == 2 ? go_dw<2, 2, false>(ctx, p) : go_dw<2, 1, false>(ctx, p);
+    return widest == 4 ? go_dw<1, 4, false>(ctx, p) : widest == 2 ? go_dw<1, 2, false>(ctx, p) : go_dw<1, 1, false>(ctx, p);
 }
 
 // Geometry checks and the wave tile, shared by the two data types. `es`: bytes per input element.

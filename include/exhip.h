@@ -71,7 +71,7 @@ const char* exhip_last_error(void);
  * tile (0 = 32 pixels x 64 channels, 2 = 64 x 64 for large launches), "stem" the one-kernel stem: every form computes
  * the same values. "pw_split" chooses that kernel's split form (1 by its rule, 2 wherever it can run, 0 never; fp16 sums then run
  * in another order). "dw_pw" chooses the depthwise + pointwise fp16 pairs that exhip_dw_pw_f16 takes (1 by its rule, 2 wherever it can
- * run, 0 never; the same values). "f32_tile" pins the float32 convolution's wave tile and split (0 = its rule, n = the n-th of its list;
+ * run, a power of two from 4 to 256 so with that many pixels a group, 0 never; the same values). "f32_tile" pins the float32 convolution's wave tile and split (0 = its rule, n = the n-th of its list;
  * sums then run in another order).
  * Process-wide; packed weights depend on the first three, so set them before packing. */
 int exhip_set_option(const char* name, int value);

@@ -117,3 +117,12 @@ def test_every_option_of_the_two_layers(ctx, pairs, stride, pad, hw, act, with_b
     assert (got[-guard:] == 0x7e00).all()
     assert np.array_equal(got[:-guard].reshape(want.shape), want)
     assert np.isfinite(want.view(np.float16)).all() and np.ptp(want.view(np.float16).astype(np.float32)) > .5
+
+
+# pixels of a group: fewer than a strip's round and than a block, several blocks, more than the map has
+@pytest.mark.parametrize("pixels", [4, 8, 16, 32, 64, 128, 256])
+@pytest.mark.parametrize("front", [0, 2, 4, 5, 6])
+@pytest.mark.parametrize("c,behind", [(16, 0), (96, 4), (512, 1)])
+def test_pixels_of_a_group(ctx, pairs, front, behind, c, pixels):
+    forced = lambda value: pairs(pixels)
+    test_every_option_of_the_two_layers(ctx, forced, *FRONT[front], *BEHIND[behind], c)
