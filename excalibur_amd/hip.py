@@ -577,3 +577,11 @@ class Ctx:
         y = self.empty((m, n_out, 1, 1), np.float32)
         _check(lib().exhip_innerproduct_f32(self.h, x.ptr, w.ptr, _ptr(bias), y.ptr, m, n_out, k_in))
         return y
+
+    def innerproduct_f16(self, x, w, bias=None):
+        m = x.shape[0]
+        k_in = x.size // m
+        n_out = w.size // k_in
+        y = self.empty((m, n_out, 1, 1), np.uint16)
+        _check(lib().exhip_innerproduct_f16(self.h, x.ptr, w.ptr, _ptr(bias), y.ptr, m, n_out, k_in))
+        return y

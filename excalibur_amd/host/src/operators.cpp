@@ -1116,13 +1116,24 @@ void operation_innerproduct<Dtype>::forward_gpu_f16(const tensor_list<unsigned s
     CHECK_EQ(bottoms.size(), 1);
     CHECK_EQ(tops.size(), 1);
     const int dev = this->params_.device_;
-    tensor_list<float> fb(1), ft(1);
-    const half_ptr in = as_nchw(this->ctx(), bottoms[0], dev);  // the flattening order is NCHW's
-    fb[0] = std::make_shared<tensor<float>>(in->data_shape(), dev, in->order());
-    EXHIP_FATAL(exhip_f16_to_f32(this->ctx(), in->gpu_data(), fb[0]->mutable_gpu_data(), fb[0]->count()));
-    forward_gpu_f32(fb, ft);
-    tops[0] = std::make_shared<tensor<unsigned short>>(ft[0]->data_shape(), dev, ft[0]->order());
-    EXHIP_FATAL(exhip_f32_to_f16(this->ctx(), ft[0]->gpu_data(), tops[0]->mutable_gpu_data(), ft[0]->count()));
+    if (this->weights_f32_.empty()) NOT_IMPLEMENTED << " (int8 InnerProduct has no CPU counterpart in the reference)";
+    // the flattening order is NCHW's, which one pixel an image has in either layout
+    const half_ptr in = bottoms[0]->height() * bottoms[0]->width() == 1 ? bottoms[0] : as_nchw(this->ctx(), bottoms[0], dev);
+    const int m = in->num(), n = num_output_, c = in->channels(), h = in->height(), w = in->width();
+    const float* weights = this->weights_f32_[0]->gpu_data();
+    const int dims = (w == 1 ? 0 : 1) + (h == 1 ? 0 : 1) + (c == 1 ? 0 : 1);
+    if (dims == 2) {
+        tops[0] = new_tensor<unsigned short>({m, 1, h, n}, dev);
+        for (int i = 0; i < m; ++i)
+            EXHIP_FATAL(exhip_innerproduct_f16(this->ctx(), in->gpu_data() + in->offset(i), weights, nullptr,
+                                               tops[0]->mutable_gpu_data() + tops[0]->offset(i), h, n, w));
+        return;
+    }
+    const int k = in->count(1, 4);
+    CHECK_EQ(k * n, weight_data_size_);
+    tops[0] = new_tensor<unsigned short>({m, n, 1, 1}, dev);
+    EXHIP_FATAL(exhip_innerproduct_f16(this->ctx(), in->gpu_data(), weights, bias_term_ ? this->weights_f32_[1]->gpu_data() : nullptr,
+                                       tops[0]->mutable_gpu_data(), m, n, k));
 }
 
 // ------------------------------------------------------------------ default fp16 layer

@@ -451,6 +451,8 @@ int exhip_deconv2d_f32(exhip_ctx* ctx, const float* x, const float* w, const flo
  * y[m,n] = sum_k x[m,k]*w[n,k] + bias[n]; x [m][k_in], w [n_out][k_in] row-major f32. */
 int exhip_innerproduct_f32(exhip_ctx* ctx, const float* x, const float* w, const float* bias, float* y, int m,
                            int n_out, int k_in);
+/* the same on half rows, as the fp16 wrapper runs it (include/Excalibur/operation.hpp:204-266): sums in float32, results rounded once */
+int exhip_innerproduct_f16(exhip_ctx* ctx, const uint16_t* x, const float* w, const float* bias, uint16_t* y, int m, int n_out, int k_in);
 
 #ifdef __cplusplus
 }

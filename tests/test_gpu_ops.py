@@ -528,6 +528,21 @@ def test_innerproduct_within_1e4(ctx):
         assert cases.check_value(gpueval.gpu_eval(ctx, case), cases.oracle_eval(case), 1e-4) == 0
 
 
+@pytest.mark.parametrize("m,n_out,k_in,bias", [(1, 128, 512, True), (64, 128, 512, False), (9, 7, 1028, True), (3, 5, 130, True), (8, 1, 4, False)])
+def test_innerproduct_half_is_the_float_one_rounded(ctx, m, n_out, k_in, bias):
+    r = np.random.default_rng(k_in)
+    x = r.normal(0, 1, (m, k_in)).astype(np.float16)
+    w = r.normal(0, .1, (n_out, k_in)).astype(np.float32)
+    b = r.normal(0, 1, n_out).astype(np.float32) if bias else None
+    dev = lambda a: ctx.array(a) if a is not None else None
+    got = ctx.innerproduct_f16(ctx.array(x.view(np.uint16)), dev(w), dev(b)).download()
+    as_float = ctx.innerproduct_f32(ctx.array(x.astype(np.float32)), dev(w), dev(b)).download()
+    assert np.array_equal(got, as_float.astype(np.float16).view(np.uint16))
+    want = x.astype(np.float64) @ w.astype(np.float64).T + (b.astype(np.float64) if bias else 0)
+    # k_in roundings of a sum whose parts stay below its absolute sum
+    assert np.all(np.abs(as_float.reshape(want.shape) - want) <= (k_in + 2) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T + 4))
+
+
 def test_error_paths_return_codes_not_crashes(ctx):
     from excalibur_amd import hip
     d = ctx.conv_desc(1, 20, 8, 8, 8, 3, 1, 1, c_stride=20)  # 20-byte pixels: not a multiple of 32
