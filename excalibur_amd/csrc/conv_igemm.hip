@@ -2047,3 +2047,22 @@ extern "C" int exhip_dw_pw_f16(exhip_ctx* ctx, const exhip_depthwise_desc* dw, c
     p.x = (const char*)dw->x; p.wp = (const char*)wp; p.bias = bias; p.residual = (const char*)residual; p.y_q = y;
     return run_conv<EXHIP_F16>(ctx, d, p, nullptr, nullptr, 0, &g);
 }
+
+extern "C" int exhip_stem_f16(exhip_ctx* ctx, const exhip_conv_desc* d, const uint16_t* x_nchw, const float* mean, const float* factor, const void* wp,
+                              const float* bias, uint16_t* y) {
+    EXHIP_REQUIRE(ctx && d && x_nchw && wp && y && !mean == !factor, "exhip_stem_f16: bad argument");
+    Plan pl;
+    if (d->c_stride != 4 || d->c > 4 || d->sh != d->sw) return EXHIP_ERR_UNSUPPORTED;
+    const int rc = make_plan(d, EXHIP_F16, &pl);
+    if (rc) return rc;
+    EXHIP_REQUIRE((d->post_op >= 0 && d->post_op <= 1 + EXHIP_UNARY_CLIP && d->post_op != 1 + EXHIP_UNARY_SIGMOID) ||
+                      (d->post_op == EXHIP_POST_PRELU && d->post_slope),
+                  "conv: post_op %d is not an activation the epilogue applies", d->post_op);
+    exhip_pw_geom g = {};
+    g.pixels = (long long)d->n * pl.OH * pl.OW; g.k = d->k; g.k_stride = d->k_stride; g.slab_blocks = pl.TM / 32; g.slabs = pl.ktiles;
+    g.act = d->act; g.post_relu = d->post_relu; g.post_op = d->post_op; g.post_alpha = d->post_alpha; g.post_beta = d->post_beta;
+    g.post_slope = d->post_slope; g.post_slope_shared = d->post_slope_shared;
+    exhip_pw_taps t = {};
+    t.n = d->n; t.in_h = d->h; t.in_w = d->w; t.out_h = pl.OH; t.out_w = pl.OW; t.kh = d->kh; t.kw = d->kw; t.stride = d->sh; t.pad_t = d->pt; t.pad_l = d->pl;
+    return exhip_conv_f16_stem(ctx, g, t, d->c, x_nchw, mean, factor, wp, bias, y);
+}

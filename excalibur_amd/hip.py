@@ -54,6 +54,9 @@ def set_option(name, value):
     _check(lib().exhip_set_option(name.encode(), int(value)))
 
 
+ERR_UNSUPPORTED = 10002  # a form that an entry point leaves to others
+
+
 def _check(rc):
     if rc != 0:
         raise ExhipError(f"exhip error {rc}: {lib().exhip_last_error().decode()}")
@@ -585,3 +588,8 @@ class Ctx:
         y = self.empty((m, n_out, 1, 1), np.uint16)
         _check(lib().exhip_innerproduct_f16(self.h, x.ptr, w.ptr, _ptr(bias), y.ptr, m, n_out, k_in))
         return y
+
+    def stem_f16(self, d, x, mean, factor, wp, bias, y):
+        """The status: 0, or EXHIP_ERR_UNSUPPORTED where the layers run by themselves."""
+        rc = lib().exhip_stem_f16(self.h, ctypes.byref(d), x.ptr, _ptr(mean), _ptr(factor), wp.ptr, _ptr(bias), y.ptr)
+        return rc if rc == ERR_UNSUPPORTED else _check(rc) or 0

@@ -36,6 +36,8 @@ public:
 
 template <typename Dtype>
 class operation_convolutiondepthwise;
+template <typename Dtype>
+class operation_input;
 
 template <typename Dtype>
 class operation_convolution : public operation_general_conv<Dtype> {
@@ -81,6 +83,9 @@ public:
     // fp16: this layer, a pointwise one, with the 3x3 depthwise layer that it alone reads in front of it in one kernel, each with
     // the layers set behind it; `bottoms` are the depthwise layer's. False, with nothing done, where the pair runs as two layers.
     bool forward_behind_depthwise(operation_convolutiondepthwise<Dtype>& dw, const tensor_list<unsigned short>& bottoms, tensor_list<unsigned short>& tops);
+    // fp16: this layer, of at most four input channels, straight on its NCHW input, with the Input layer that it alone reads in front of it
+    // (or NULL) and the layers set behind it; `bottoms` are the first one's. False, with nothing done, where the layers run by themselves.
+    bool forward_stem(operation_input<Dtype>* input, const tensor_list<unsigned short>& bottoms, tensor_list<unsigned short>& tops);
     // int8 layers on the MFMA kernel. The next forward calls also write the int8 NHWC form of the output that a reader
     // quantizing with `fs` into `stride` channels per pixel would make of it (attached to the top blob as its
     // `quantized` copy), and with `only` leave the float data unwritten; fs = 0 switches it off. False where this
@@ -340,6 +345,7 @@ public:
     int w_ = 0, h_ = 0, c_ = 0;
     std::vector<float> means_, vars_;
     std::shared_ptr<memory::tensor<float>> means_dev_, vars_dev_;
+    void upload_tables(int ch);
 
 protected:
     void forward_gpu_f32(const tensor_list<float>& bottoms, tensor_list<float>& tops) override;

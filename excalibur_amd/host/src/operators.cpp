@@ -544,6 +544,7 @@ void operation_convolution<Dtype>::forward_gpu_f16(const tensor_list<unsigned sh
     if (bottoms[0]->order() == memory::NHWC && d.c_stride == c) {
         x = bottoms[0];
     } else {
+        if (forward_stem(nullptr, bottoms, tops)) return;
         const half_ptr in = as_nchw(this->ctx(), bottoms[0], dev);
         x = new_tensor<unsigned short>({n, h, w, d.c_stride}, dev);
         EXHIP_FATAL(exhip_nchw_f16_to_nhwc_f16(this->ctx(), in->gpu_data(), n, c, h, w, d.c_stride, x->mutable_gpu_data()));
@@ -566,6 +567,27 @@ const unsigned short* operation_convolution<Dtype>::sum_operand(const tensor_lis
     d->residual_last = post_sum_last_ ? 1 : 0;
     post_sum_used_ = true;
     return post_sum_->gpu_data();
+}
+
+template <typename Dtype>
+bool operation_convolution<Dtype>::forward_stem(operation_input<Dtype>* input, const tensor_list<unsigned short>& bottoms, tensor_list<unsigned short>& tops) {
+    const int dev = this->params_.device_, c = this->input_channels();
+    if (bottoms[0]->order() != memory::NCHW || bottoms[0]->channels() != c || !mfma_path_ok() || this->output_channel_ % 16 != 0 || !nhwc_allowed() ||
+        post_sum_ || conv_in_stride(c, EXHIP_F16, this->kernel_size_w_) != 4)
+        return false;
+    const int n = bottoms[0]->num(), h = bottoms[0]->height(), w = bottoms[0]->width();
+    exhip_conv_desc d = describe(n, h, w, c, this->output_channel_);
+    d.c_stride = 4;
+    int oh, ow;
+    EXHIP_FATAL(exhip_conv_out_hw(&d, &oh, &ow));
+    if (input) input->upload_tables(c);
+    auto y = new_tensor<unsigned short>({n, oh, ow, this->output_channel_}, dev, memory::NHWC);
+    const int rc = exhip_stem_f16(this->ctx(), &d, bottoms[0]->gpu_data(), input ? input->means_dev_->gpu_data() : nullptr,
+                                  input ? input->vars_dev_->gpu_data() : nullptr, packed_weights(EXHIP_F16, d), bias_gpu(), y->mutable_gpu_data());
+    if (rc == EXHIP_ERR_UNSUPPORTED) return false;
+    EXHIP_FATAL(rc);
+    tops[0] = y;
+    return true;
 }
 
 template <typename Dtype>
@@ -1367,6 +1389,21 @@ operation_input<Dtype>::operation_input(const operation_param& param) : operatio
     }
 }
 
+// The means and factors on the device; stops where the layer does not take `ch` channels.
+template <typename Dtype>
+void operation_input<Dtype>::upload_tables(int ch) {
+    if (ch != 1 && ch != 3) LOG(FATAL) << "Un-supprted channel num: " << ch;
+    CHECK_EQ(static_cast<size_t>(ch), means_.size());
+    CHECK_GE(vars_.size(), static_cast<size_t>(ch));
+    if (means_dev_) return;
+    means_dev_ = vec_tensor<float>(ch, this->params_.device_);
+    vars_dev_ = vec_tensor<float>(ch, this->params_.device_);
+    for (int c = 0; c < ch; ++c) {
+        means_dev_->mutable_cpu_data()[c] = means_[c];
+        vars_dev_->mutable_cpu_data()[c] = vars_[c];
+    }
+}
+
 template <typename Dtype>
 void operation_input<Dtype>::forward_gpu_f32(const tensor_list<float>& bottoms, tensor_list<float>& tops) {
     CHECK_EQ(bottoms.size(), tops.size());
@@ -1375,16 +1412,7 @@ void operation_input<Dtype>::forward_gpu_f32(const tensor_list<float>& bottoms, 
         const int ch = b->channels();
         if (ch != 1 && ch != 3) LOG(FATAL) << "Un-supprted channel num: " << ch;
         if (b->order() != memory::NCHW) NOT_IMPLEMENTED;
-        CHECK_EQ(static_cast<size_t>(ch), means_.size());
-        CHECK_GE(vars_.size(), static_cast<size_t>(ch));
-        if (!means_dev_) {
-            means_dev_ = vec_tensor<float>(ch, this->params_.device_);
-            vars_dev_ = vec_tensor<float>(ch, this->params_.device_);
-            for (int c = 0; c < ch; ++c) {
-                means_dev_->mutable_cpu_data()[c] = means_[c];
-                vars_dev_->mutable_cpu_data()[c] = vars_[c];
-            }
-        }
+        upload_tables(ch);
         tops[i] = std::make_shared<tensor<float>>(b->data_shape(), this->params_.device_, b->order());
         EXHIP_FATAL(exhip_channelwise_f32(this->ctx(), EXHIP_CHANNEL_INPUT, b->gpu_data(), tops[i]->mutable_gpu_data(), b->num(), ch,
                                           b->height() * b->width(), means_dev_->gpu_data(), vars_dev_->gpu_data(), 0));
@@ -1397,17 +1425,7 @@ void operation_input<Dtype>::forward_gpu_f16(const tensor_list<unsigned short>& 
     for (size_t i = 0; i < bottoms.size(); ++i) {
         const half_ptr b = as_nchw(this->ctx(), bottoms[i], this->params_.device_);
         const int ch = b->channels();
-        if (ch != 1 && ch != 3) LOG(FATAL) << "Un-supprted channel num: " << ch;
-        CHECK_EQ(static_cast<size_t>(ch), means_.size());
-        CHECK_GE(vars_.size(), static_cast<size_t>(ch));
-        if (!means_dev_) {
-            means_dev_ = vec_tensor<float>(ch, this->params_.device_);
-            vars_dev_ = vec_tensor<float>(ch, this->params_.device_);
-            for (int c = 0; c < ch; ++c) {
-                means_dev_->mutable_cpu_data()[c] = means_[c];
-                vars_dev_->mutable_cpu_data()[c] = vars_[c];
-            }
-        }
+        upload_tables(ch);
         tops[i] = std::make_shared<tensor<unsigned short>>(b->data_shape(), this->params_.device_, b->order());
         EXHIP_FATAL(exhip_channelwise_f16(this->ctx(), EXHIP_CHANNEL_INPUT, b->gpu_data(), tops[i]->mutable_gpu_data(), b->num(), ch,
                                           b->height() * b->width(), means_dev_->gpu_data(), vars_dev_->gpu_data(), 0));

@@ -235,7 +235,27 @@ public:
         find_quantized_links();
         find_sum_pairs();
         find_depthwise_pairs();
+        find_stem();
         find_glue_chains();
+    }
+
+    // fp16 pipeline: an Input layer whose only reader is the convolution on the next line: one kernel runs both where it takes the
+    // convolution, and the blob between them is never stored.
+    void find_stem() {
+        behind_input_.assign(operations_.size(), false);
+        if constexpr (std::is_same_v<Dtype, unsigned short>) {
+            for (size_t i = 0; i + 1 < operations_.size(); ++i) {
+                if (!dynamic_cast<operation_input<Dtype>*>(operations_[i].get()) || op_inputs_[i].size() != 1 || op_outputs_[i].size() != 1) continue;
+                const int mid = op_outputs_[i][0];
+                auto* conv = dynamic_cast<operation_convolution<Dtype>*>(operations_[i + 1].get());
+                if (!conv || dynamic_cast<operation_convolutiondepthwise<Dtype>*>(conv) || op_inputs_[i + 1] != std::vector<int>{mid} ||
+                    op_outputs_[i + 1].size() != 1 || op_outputs_[i + 1][0] == mid || sum_other_[i + 1] >= 0)
+                    continue;
+                int readers = 0;
+                for (const auto& in : op_inputs_) readers += static_cast<int>(std::count(in.begin(), in.end(), mid));
+                behind_input_[i] = readers == 1 && std::find(output_names_.begin(), output_names_.end(), blob_names_[mid]) == output_names_.end();
+            }
+        }
     }
 
     // fp16 pipeline: a depthwise layer (with its PReLU layer) whose only reader is the convolution behind it: where that is a
@@ -499,6 +519,20 @@ private:
                 return conv;
             };
             if constexpr (std::is_same_v<Dtype, unsigned short>) {
+                if (fusion_ && behind_input_[i]) {
+                    auto* conv = set_paired_activation(i + 1);
+                    const bool ran = conv->forward_stem(static_cast<operation_input<Dtype>*>(operations_[i].get()), in, out);
+                    conv->clear_post();
+                    if (ran) {
+                        const size_t done = i + 1 + (pair_[i + 1].on ? 1 : 0);  // the last layer whose work the launch did
+                        for (size_t k = i; k < done; ++k) featmaps_[op_outputs_[k][0]] = nullptr;
+                        featmaps_[op_outputs_[done][0]] = out[0];
+                        i = done;
+                        continue;
+                    }
+                }
+            }
+            if constexpr (std::is_same_v<Dtype, unsigned short>) {
                 if (fusion_ && behind_depthwise_[i] >= 0) {
                     const size_t j = behind_depthwise_[i];
                     auto* dw = static_cast<operation_convolutiondepthwise<Dtype>*>(set_paired_activation(i));
@@ -631,6 +665,7 @@ private:
     };
     std::vector<int> sum_other_;         // per layer: the other operand's blob of the sum layer this convolution absorbs, or -1
     std::vector<int> behind_depthwise_;  // per layer: the pointwise layer that runs in this depthwise layer's kernel, or -1
+    std::vector<char> behind_input_;     // per layer: the convolution on the next line runs in this Input layer's kernel
     struct glue_chain {
         int bn = -1, unary = -1, last = -1;  // layer numbers of the absorbed BatchNorm / activation, and of the last absorbed layer
     };

@@ -68,7 +68,8 @@ const char* exhip_last_error(void);
  * "lean" / "lean_cfg" / "lean_wres" / "lean_groups" / "lean_f16" choose the form of the lean 3x3 kernel for int8 / fp16
  * layers (0 = the general kernel), "pw" the fp16 / int8 kernel without staging for pointwise layers and "direct" its
  * form for layers with a filter (1 where it measured faster, 2 wherever it can run, 0 never), "pw_tile" that kernel's wave
- * tile (0 = 32 pixels x 64 channels, 2 = 64 x 64 for large launches), "stem" the one-kernel stem: every form computes
+ * tile (0 = 32 pixels x 64 channels, 2 = 64 x 64 for large launches), "stem" the one-kernel stems (2 upwards:
+ * that many output rows a group of the fp16 one): every form computes
  * the same values. "pw_split" chooses that kernel's split form (1 by its rule, 2 wherever it can run, 0 never; fp16 sums then run
  * in another order). "dw_pw" chooses the depthwise + pointwise fp16 pairs that exhip_dw_pw_f16 takes (1 by its rule, 2 wherever it can
  * run, a power of two from 4 to 256 so with that many pixels a group, 0 never; the same values). "f32_tile" pins the float32 convolution's wave tile and split (0 = its rule, n = the n-th of its list;
@@ -223,6 +224,12 @@ typedef struct exhip_depthwise_desc {
 } exhip_depthwise_desc;
 int exhip_dw_pw_f16(exhip_ctx* ctx, const exhip_depthwise_desc* dw, const exhip_conv_desc* d, const void* w_packed, const float* bias,
                     const uint16_t* residual_nhwc, uint16_t* y_nhwc);
+
+/* The first layer of an fp16 network on its half NCHW input: exhip_conv2d_f16 of at most four channels (c_stride 4, its packed weights) with the NHWC
+ * result, without the conversion in front; with the Input layer (operation_input.cpp, (x - mean[c]) * factor[c] rounded to half) where mean and factor
+ * are given, both or neither. EXHIP_ERR_UNSUPPORTED, with nothing launched, where the layers run by themselves. */
+int exhip_stem_f16(exhip_ctx* ctx, const exhip_conv_desc* d, const uint16_t* x_nchw, const float* mean, const float* factor, const void* w_packed,
+                   const float* bias, uint16_t* y_nhwc);
 
 /* A detection head: the 1x1 convolution, the Reshape of its channels into groups and the Transpose of the last two axes
  * (operation_reshape.cpp, operation_transpose.cpp) as one launch, y[n][k / group][pixel][group] (float32 of an int8 layer, halves).
