@@ -93,8 +93,8 @@ struct exhip_options {
     int lean_cfg = 0;        // its staging buffers for layers of more than 64 input channels: 0 one tile + two slices, 1 two + two, 2 one + three
     int lean_wres = 1;       // 64 input channels: keep the slab's whole filter in LDS (0: stream it like the deeper layers)
     int lean_stagger = 0;    // experiment: start delay per hardware wave slot, in units of 64 cycles
-    int stem = 1;            // the stems (int8: quantizer + first convolution + max pooling; fp16: Input layer + first convolution) as one kernel where the entry point offers it;
-                             // the fp16 one 2 upwards with that many output rows a group
+    int stem = 1;            // the stems (int8: quantizer + first convolution + max pooling; others: Input layer, quantizer + first 3x3 convolution) as one kernel where the entry point offers it;
+                             // the latter 2 upwards with that many output rows a group
     int lean_groups = 0;     // at most this many groups per 64-channel slab (tests: a few groups that walk many patches each)
     int lean_f16 = 1;        // 3x3 stride-1 fp16 layers with an NHWC result on the lean kernel: 0 never, 1 the form per layer class, 2 one group per
                              // patch, 3 persistent groups with three slice buffers, 4 persistent groups with two

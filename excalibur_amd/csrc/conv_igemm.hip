@@ -2048,21 +2048,38 @@ extern "C" int exhip_dw_pw_f16(exhip_ctx* ctx, const exhip_depthwise_desc* dw, c
     return run_conv<EXHIP_F16>(ctx, d, p, nullptr, nullptr, 0, &g);
 }
 
-extern "C" int exhip_stem_f16(exhip_ctx* ctx, const exhip_conv_desc* d, const uint16_t* x_nchw, const float* mean, const float* factor, const void* wp,
-                              const float* bias, uint16_t* y) {
-    EXHIP_REQUIRE(ctx && d && x_nchw && wp && y && !mean == !factor, "exhip_stem_f16: bad argument");
-    Plan pl;
+// The geometry of a first layer that the kernel on NCHW planes may take.
+static int stem_geometry(const exhip_conv_desc* d, int dt, exhip_pw_geom* g, exhip_pw_taps* t) {
     if (d->c_stride != 4 || d->c > 4 || d->sh != d->sw) return EXHIP_ERR_UNSUPPORTED;
-    const int rc = make_plan(d, EXHIP_F16, &pl);
+    Plan pl;
+    const int rc = make_plan(d, dt, &pl);
     if (rc) return rc;
     EXHIP_REQUIRE((d->post_op >= 0 && d->post_op <= 1 + EXHIP_UNARY_CLIP && d->post_op != 1 + EXHIP_UNARY_SIGMOID) ||
                       (d->post_op == EXHIP_POST_PRELU && d->post_slope),
                   "conv: post_op %d is not an activation the epilogue applies", d->post_op);
-    exhip_pw_geom g = {};
-    g.pixels = (long long)d->n * pl.OH * pl.OW; g.k = d->k; g.k_stride = d->k_stride; g.slab_blocks = pl.TM / 32; g.slabs = pl.ktiles;
-    g.act = d->act; g.post_relu = d->post_relu; g.post_op = d->post_op; g.post_alpha = d->post_alpha; g.post_beta = d->post_beta;
-    g.post_slope = d->post_slope; g.post_slope_shared = d->post_slope_shared;
-    exhip_pw_taps t = {};
-    t.n = d->n; t.in_h = d->h; t.in_w = d->w; t.out_h = pl.OH; t.out_w = pl.OW; t.kh = d->kh; t.kw = d->kw; t.stride = d->sh; t.pad_t = d->pt; t.pad_l = d->pl;
-    return exhip_conv_f16_stem(ctx, g, t, d->c, x_nchw, mean, factor, wp, bias, y);
+    *g = {};
+    g->pixels = (long long)d->n * pl.OH * pl.OW; g->k = d->k; g->k_stride = d->k_stride; g->slab_blocks = pl.TM / 32; g->slabs = pl.ktiles;
+    g->act = d->act; g->post_relu = d->post_relu; g->post_op = d->post_op; g->post_alpha = d->post_alpha; g->post_beta = d->post_beta;
+    g->post_slope = d->post_slope; g->post_slope_shared = d->post_slope_shared; g->fs_out = d->fs_out;
+    *t = {};
+    t->n = d->n; t->in_h = d->h; t->in_w = d->w; t->out_h = pl.OH; t->out_w = pl.OW; t->kh = d->kh; t->kw = d->kw; t->stride = d->sh; t->pad_t = d->pt; t->pad_l = d->pl;
+    return 0;
+}
+
+extern "C" int exhip_stem_f16(exhip_ctx* ctx, const exhip_conv_desc* d, const uint16_t* x_nchw, const float* mean, const float* factor, const void* wp,
+                              const float* bias, uint16_t* y) {
+    EXHIP_REQUIRE(ctx && d && x_nchw && wp && y && !mean == !factor, "exhip_stem_f16: bad argument");
+    exhip_pw_geom g;
+    exhip_pw_taps t;
+    const int rc = stem_geometry(d, EXHIP_F16, &g, &t);
+    return rc ? rc : exhip_conv_f16_stem(ctx, g, t, d->c, x_nchw, mean, factor, wp, bias, y);
+}
+
+extern "C" int exhip_stem_i8(exhip_ctx* ctx, const exhip_conv_desc* d, const float* x_nchw, const float* mean, const float* factor, float fs_in, const void* wp,
+                             const float* scale, const float* bias, int8_t* y_i8, float* y_f32) {
+    EXHIP_REQUIRE(ctx && d && x_nchw && wp && scale && (y_i8 || y_f32) && !mean == !factor, "exhip_stem_i8: bad argument");
+    exhip_pw_geom g;
+    exhip_pw_taps t;
+    const int rc = stem_geometry(d, EXHIP_I8, &g, &t);
+    return rc ? rc : exhip_conv_i8_stem(ctx, g, t, d->c, x_nchw, mean, factor, fs_in, wp, scale, bias, y_i8, y_f32);
 }

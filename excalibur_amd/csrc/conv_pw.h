@@ -47,10 +47,12 @@ struct exhip_pw_depthwise {
 // runs the general kernel), another code on failure. Semantics as exhip_conv2d_f16 with only the NHWC half output.
 int exhip_conv1x1_f16_pw(exhip_ctx* ctx, const exhip_pw_geom& g, const uint16_t* x, const void* wp, const float* bias,
                          const uint16_t* residual, uint16_t* y, const exhip_pw_taps* taps = nullptr, const exhip_pw_depthwise* dw = nullptr);
-// The first layer of an fp16 network on its half NCHW planes (g.c_bytes unused; t: one packed k-step a filter row), (x - mean[c]) * factor[c]
-// rounded to half in front of it where `mean` is given.
+// The first layer of a network on its NCHW planes (g.c_bytes unused; t: one packed k-step a filter row), (x - mean[c]) * factor[c] in front of it
+// where `mean` is given: half planes, that rounded to half; float32 planes, that quantized with fs_in.
 int exhip_conv_f16_stem(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, int channels, const uint16_t* x, const float* mean, const float* factor,
                         const void* wp, const float* bias, uint16_t* y);
+int exhip_conv_i8_stem(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, int channels, const float* x, const float* mean, const float* factor,
+                       float fs_in, const void* wp, const float* scale, const float* bias, int8_t* y_i8, float* y_f32);
 // The int8 layer: semantics as exhip_conv2d_i8 with the NHWC results only (y_i8 and / or y_f32; k_stride a multiple of 16).
 int exhip_conv1x1_i8_pw(exhip_ctx* ctx, const exhip_pw_geom& g, const int8_t* x, const void* wp, const float* scale, const float* bias,
                         const float* residual, int8_t* y_i8, float* y_f32, const exhip_pw_taps* taps = nullptr);

@@ -88,10 +88,11 @@ struct PwParams {
     const float* dw_bias;
     const float* dw_slope;
     int dw_act, dw_slope_shared, dw_pixels, dw_tiles, dw_kblocks, dw_split, dw_mid, kblocks;  // dw_mid: where its results begin in LDS
-    // the first layer on half planes (stem_f16_kernel; geometry in in_h .. pad_l above, x is its input): channels, the Input layer's means and
+    // the first layer on NCHW planes (stem_planes_kernel; geometry in in_h .. pad_l above, x is its input): channels, the Input layer's means and
     // factors (or NULL), output rows of a group, groups an image (ch_groups), pixels of a row in LDS, 16-byte pieces of an input row
     const float* mean;
     const float* factor;
+    float fs_in;  // the quantizer's
     int in_c, tile_rows, row_pixels, pieces, pieces_shift;
     unsigned pieces_magic;
 };
@@ -984,17 +985,21 @@ __global__ __launch_bounds__(256, 3) void dw_pw_kernel(const PwParams p) {
     }
 }
 
-// ---- the first layer of an fp16 network: 3x3 on the half planes of at most four channels, with the Input layer in front ----
-// A group takes tile_rows whole output rows of an image, which are neighbouring pixels of the NHWC result. It reads the input rows they need
-// from the planes (VEC: eight pixels a load), applies (x - mean) * factor, rounds to half as the Input layer does and leaves
-// pixels of four halves in LDS, padding as zeros; a filter row is then one k-step, a lane's 16 bytes two neighbouring taps. The weights are the general
-// kernel's packed first-layer form, the order of the sums is its as well. Bound by the stores of the result in a large launch (3 -> 64 at stride 2
+// ---- the first layer of a network: 3x3 on the planes of at most four channels, with the Input layer in front ----
+// Halves for an fp16 network, float32 for an int8 one, whose quantizer is in here as well. A group takes tile_rows whole output rows of an image, which are
+// neighbouring pixels of the NHWC result. It reads the input rows they need from the planes (VEC: eight pixels at a time), applies (x - mean) * factor, rounds
+// to half as the Input layer does or quantizes, and leaves pixels of four halves or bytes in LDS, padding as zeros; a filter row is then one
+// k-step, a lane's 16 bytes two or four neighbouring taps. The weights are the general kernel's packed first-layer form, the order of the sums is its as well. Bound by the stores of the result in a large launch (3 -> 64 at stride 2
 // with the Input layer, 64 x 224 x 224: 26 us, 103 MB; 81 as Input layer, conversion and convolution, 61 the convolution alone), by the
-// launch in a small one (1 x 112 x 112: 4.0, 16.0 and 11.4). Rows of a width that is no multiple of eight cost two-byte loads (64 x 223 x 223: 34 us, 142).
-template <int MT, bool VEC, typename EP>
-__global__ __launch_bounds__(256, EP::any ? 2 : 4) void stem_f16_kernel(const PwParams p) {
+// launch in a small one (1 x 112 x 112: 4.0, 16.0 and 11.4); the int8 form 3 -> 16 at 64 x 128 x 128 takes 24.6 us, 70 as Input layer, quantizer (11.3) and convolution.
+// Rows of a width that is no multiple of eight cost two-byte loads (64 x 223 x 223: 34 us, 142).
+template <int DT, int MT, bool VEC, typename EP>
+__global__ __launch_bounds__(256, EP::any ? 2 : 4) void stem_planes_kernel(const PwParams p) {
     exhip_touch_args(p);
+    constexpr bool I8 = DT == EXHIP_I8;
     constexpr int KH = 3;
+    typedef typename std::conditional<I8, int, v2i>::type pixel_t;
+    typedef typename std::conditional<I8, float, uint16_t>::type plane_t;
     extern __shared__ __attribute__((aligned(16))) char lds_dyn[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     unsigned item0 = blockIdx.x;
@@ -1005,8 +1010,8 @@ __global__ __launch_bounds__(256, EP::any ? 2 : 4) void stem_f16_kernel(const Pw
     const unsigned img = __builtin_amdgcn_readfirstlane(exhip_divide(item0, p.ch_groups, p.groups_magic, p.groups_shift));
     const int oy0 = __builtin_amdgcn_readfirstlane((int)(item0 - img * p.ch_groups) * p.tile_rows);
     const int rows = min(p.tile_rows, p.out_h - oy0), in_rows = (rows - 1) * p.stride + KH, iy0 = oy0 * p.stride - p.pad_t;
-    char* const lds = lds_dyn + wave * wave_bytes(EXHIP_F16, MT);
-    v2i* const px = reinterpret_cast<v2i*>(lds_dyn + 4 * wave_bytes(EXHIP_F16, MT));
+    char* const lds = lds_dyn + wave * wave_bytes(DT, MT);
+    pixel_t* const px = reinterpret_cast<pixel_t*>(lds_dyn + 4 * wave_bytes(DT, MT));
 
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.wp), 0, (int)p.w_bytes, kRsrcWord3);
     v4i a[KH][MT];
@@ -1023,61 +1028,89 @@ __global__ __launch_bounds__(256, EP::any ? 2 : 4) void stem_f16_kernel(const Pw
             const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src), 0, src ? count * 4 : 0, kRsrcWord3);
             return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, offset, 0, 0));
         };
+        if constexpr (I8) par[0] = load(p.scale, at, p.K);
         par[1] = load(p.bias, at, p.K);
         if (EP::any || EP::post == kPostPrelu) par[2] = load(p.post_slope, p.post_slope_shared ? 0 : at, p.post_slope_shared ? 1 : p.K);
     };
 
     const int plane = p.in_h * p.in_w;
-    const uint16_t* const image = reinterpret_cast<const uint16_t*>(p.x) + (size_t)img * p.in_c * plane;
+    const plane_t* const image = reinterpret_cast<const plane_t*>(p.x) + (size_t)img * p.in_c * plane;
     auto scaled = [&](float v, int c) { return p.mean ? (v - p.mean[c]) * p.factor[c] : v; };
     if constexpr (VEC) {
         typedef float v8f __attribute__((ext_vector_type(8)));
         for (int i = threadIdx.x; i < in_rows * p.pieces; i += 256) {
             const int r = (int)exhip_divide((unsigned)i, (unsigned)p.pieces, p.pieces_magic, p.pieces_shift), x8 = i - r * p.pieces, iy = iy0 + r;
             const bool inside = (unsigned)iy < (unsigned)p.in_h;
-            v4i v[4] = {};
-            if (inside) {
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
-                    if (c < p.in_c) v[c] = *reinterpret_cast<const v4i*>(image + (size_t)c * plane + iy * p.in_w + x8 * 8);
-                if (p.mean) {
+            pixel_t* const to = px + r * p.row_pixels + p.pad_l + x8 * 8;
+            if constexpr (I8) {
+                v4f v[4][2] = {};
+                if (inside) {
 #pragma unroll
                     for (int c = 0; c < 4; ++c)
                         if (c < p.in_c) {
-                            v8f f = __builtin_convertvector(__builtin_bit_cast(v8h, v[c]), v8f);
-#pragma unroll
-                            for (int e = 0; e < 8; ++e) f[e] = (f[e] - p.mean[c]) * p.factor[c];
-                            v[c] = __builtin_bit_cast(v4i, __builtin_convertvector(f, v8h));
+                            const v4f* const from = reinterpret_cast<const v4f*>(image + (size_t)c * plane + iy * p.in_w + x8 * 8);
+                            v[c][0] = from[0];
+                            v[c][1] = from[1];
                         }
                 }
-            }
-            v2i* const to = px + r * p.row_pixels + p.pad_l + x8 * 8;
+                int word[8] = {};
+                if (inside) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                auto half_of = [&](const v4i& q) { return ((unsigned)q[e >> 1] >> ((e & 1) * 16)) & 0xffffu; };
-                to[e] = v2i{(int)(half_of(v[0]) | half_of(v[1]) << 16), (int)(half_of(v[2]) | half_of(v[3]) << 16)};
+                    for (int c = 0; c < 4; ++c)
+                        if (c < p.in_c) {
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) word[e] |= (int)((unsigned)(exhip_q8(scaled(v[c][e >> 2][e & 3], c) * p.fs_in) & 0xff) << (8 * c));
+                        }
+                }
+#pragma unroll
+                for (int e = 0; e < 8; ++e) to[e] = word[e];
+            } else {
+                v4i v[4] = {};
+                if (inside) {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        if (c < p.in_c) v[c] = *reinterpret_cast<const v4i*>(image + (size_t)c * plane + iy * p.in_w + x8 * 8);
+                    if (p.mean) {
+#pragma unroll
+                        for (int c = 0; c < 4; ++c)
+                            if (c < p.in_c) {
+                                v8f f = __builtin_convertvector(__builtin_bit_cast(v8h, v[c]), v8f);
+#pragma unroll
+                                for (int e = 0; e < 8; ++e) f[e] = (f[e] - p.mean[c]) * p.factor[c];
+                                v[c] = __builtin_bit_cast(v4i, __builtin_convertvector(f, v8h));
+                            }
+                    }
+                }
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    auto half_of = [&](const v4i& q) { return ((unsigned)q[e >> 1] >> ((e & 1) * 16)) & 0xffffu; };
+                    to[e] = v2i{(int)(half_of(v[0]) | half_of(v[1]) << 16), (int)(half_of(v[2]) | half_of(v[3]) << 16)};
+                }
             }
         }
     } else {
         for (int i = threadIdx.x; i < in_rows * p.in_w; i += 256) {
             const int r = (int)exhip_divide((unsigned)i, (unsigned)p.in_w, p.pieces_magic, p.pieces_shift), x = i - r * p.in_w, iy = iy0 + r;
-            unsigned h[4] = {};
+            plane_t v[4] = {};
+            unsigned word[4] = {};
             if ((unsigned)iy < (unsigned)p.in_h) {
 #pragma unroll
                 for (int c = 0; c < 4; ++c)
-                    if (c < p.in_c) h[c] = image[(size_t)c * plane + iy * p.in_w + x];
-                if (p.mean) {
+                    if (c < p.in_c) v[c] = image[(size_t)c * plane + iy * p.in_w + x];
 #pragma unroll
-                    for (int c = 0; c < 4; ++c)
-                        if (c < p.in_c) h[c] = exhip_f2h(scaled(exhip_h2f((uint16_t)h[c]), c));
-                }
+                for (int c = 0; c < 4; ++c)
+                    if (c < p.in_c) {
+                        if constexpr (I8) word[c] = (unsigned)exhip_q8(scaled(v[c], c) * p.fs_in) & 0xff;
+                        else word[c] = p.mean ? exhip_f2h(scaled(exhip_h2f(v[c]), c)) : v[c];
+                    }
             }
-            px[r * p.row_pixels + p.pad_l + x] = v2i{(int)(h[0] | h[1] << 16), (int)(h[2] | h[3] << 16)};
+            if constexpr (I8) px[r * p.row_pixels + p.pad_l + x] = (int)(word[0] | word[1] << 8 | word[2] << 16 | word[3] << 24);
+            else px[r * p.row_pixels + p.pad_l + x] = v2i{(int)(word[0] | word[1] << 16), (int)(word[2] | word[3] << 16)};
         }
     }
     const int beside = p.row_pixels - p.in_w;  // padding: left of a row's pixels and behind them
     for (int r = wave; r < in_rows; r += 4)
-        for (int x = lane; x < beside; x += 64) px[r * p.row_pixels + (x < p.pad_l ? x : x + p.in_w)] = v2i{0, 0};
+        for (int x = lane; x < beside; x += 64) px[r * p.row_pixels + (x < p.pad_l ? x : x + p.in_w)] = pixel_t{};
     const int count = rows * p.out_w, blocks = (count + 31) / 32, items = blocks * ((p.kblocks + MT - 1) / MT);
     int b = wave, kb = 0;
     while (b >= blocks) b -= blocks, kb += MT;
@@ -1091,20 +1124,23 @@ __global__ __launch_bounds__(256, EP::any ? 2 : 4) void stem_f16_kernel(const Pw
         }
         const int at = min(b * 32 + (lane & 31), count - 1);
         const int row = (int)exhip_divide((unsigned)at, (unsigned)p.out_w, p.width_magic, p.width_shift), col = at - row * p.out_w;
-        const v2i* src = px + row * p.stride * p.row_pixels + col * p.stride + (lane >> 5) * 2;
-        v16f acc[MT][1];
+        const pixel_t* src = px + row * p.stride * p.row_pixels + col * p.stride + (lane >> 5) * (I8 ? 4 : 2);
+        typedef typename std::conditional<I8, v16i, v16f>::type acc_t;
+        acc_t acc[MT][1];
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[m][0][e] = 0.f;
+            for (int e = 0; e < 16; ++e) acc[m][0][e] = 0;
 #pragma unroll
         for (int r = 0; r < KH; ++r) {
-            const v2i lo = src[r * p.row_pixels], hi = src[r * p.row_pixels + 1];
-            const v8h taps = __builtin_bit_cast(v8h, v4i{lo[0], lo[1], hi[0], hi[1]});
+            const pixel_t* const t = src + r * p.row_pixels;
 #pragma unroll
-            for (int m = 0; m < MT; ++m) acc[m][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a[r][m]), taps, acc[m][0], 0, 0, 0);
+            for (int m = 0; m < MT; ++m) {
+                if constexpr (I8) acc[m][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[r][m], v4i{t[0], t[1], t[2], t[3]}, acc[m][0], 0, 0, 0);
+                else acc[m][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a[r][m]), __builtin_bit_cast(v8h, v4i{t[0][0], t[0][1], t[1][0], t[1][1]}), acc[m][0], 0, 0, 0);
+            }
         }
-        pw_epilogue<EXHIP_F16, MT, 1, EP>(p, acc, first + b * 32, end, kb, lane, lds);
+        pw_epilogue<DT, MT, 1, EP>(p, acc, first + b * 32, end, kb, lane, lds);
         b += 4;
         if (b >= blocks && item + 4 < items) {
             while (b >= blocks) b -= blocks, kb += MT;
@@ -1130,16 +1166,60 @@ int go_dw(exhip_ctx* ctx, PwParams& p) {
     return run(dw_pw_kernel<S, PX, SMALL, EpAny>);
 }
 
-template <int MT, bool VEC>
+template <int DT, int MT, bool VEC>
 int go_stem(exhip_ctx* ctx, const PwParams& p, int lds) {
     auto run = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(p.items), dim3(256), lds, ctx->stream, p);
         EXHIP_LAUNCH_CHECK();
         return 0;
     };
-    if (!p.post_relu && !p.post_op && p.act <= 1) return p.act ? run(stem_f16_kernel<MT, VEC, Ep<1, kPostNone, 0>>) : run(stem_f16_kernel<MT, VEC, Ep<0, kPostNone, 0>>);
-    if (!p.post_relu && p.act == 0 && p.post_op == EXHIP_POST_PRELU) return run(stem_f16_kernel<MT, VEC, Ep<0, kPostPrelu, 0>>);
-    return run(stem_f16_kernel<MT, VEC, EpAny>);
+    if (!p.post_op && !p.post_relu && p.act == 0) return run(stem_planes_kernel<DT, MT, VEC, Ep<0, kPostNone, 0>>);
+    if (!p.post_op && !p.post_relu && p.act == 1) return run(stem_planes_kernel<DT, MT, VEC, Ep<1, kPostNone, 0>>);
+    if (!p.post_op && p.post_relu && p.act == 0) return run(stem_planes_kernel<DT, MT, VEC, Ep<0, kPostRelu, 0>>);
+    if constexpr (DT == EXHIP_F16)
+        if (!p.post_relu && p.act == 0 && p.post_op == EXHIP_POST_PRELU) return run(stem_planes_kernel<DT, MT, VEC, Ep<0, kPostPrelu, 0>>);
+    return run(stem_planes_kernel<DT, MT, VEC, EpAny>);
+}
+
+// Geometry checks and the rows of a group, shared by the two data types.
+template <int DT>
+int run_stem(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, int channels, PwParams& p) {
+    constexpr int kSlots = DT == EXHIP_I8 ? 8 : 4, kPixelBytes = DT == EXHIP_I8 ? 4 : 8;   // a k-step's taps, a pixel in LDS
+    if (g_exhip_options.stem == 0 || t.kh != 3 || t.kw > kSlots || t.stride < 1 || channels > 4 || g.k_stride % (DT == EXHIP_I8 ? 16 : 8) != 0 ||
+        !pw_row_fits(4ll * g.k_stride) || g.pixels != (long long)t.n * t.out_h * t.out_w || g.pixels >= (1ll << 31) ||
+        g.pixels * 4 * g.k_stride >= (1ll << 40) || (long long)t.in_h * t.in_w >= (1ll << 28))
+        return EXHIP_ERR_UNSUPPORTED;
+    p.in_c = channels;
+    p.pixels = (unsigned)g.pixels; p.w_bytes = (unsigned)(g.slabs * t.kh * g.slab_blocks * 1024);
+    p.mts = g.slab_blocks; p.K = g.k; p.kstride = g.k_stride;
+    p.act = g.act; p.post_relu = g.post_relu; p.post_op = g.post_op; p.post_alpha = g.post_alpha; p.post_beta = g.post_beta;
+    p.post_slope = g.post_slope; p.post_slope_shared = g.post_slope_shared;
+    p.in_h = t.in_h; p.in_w = t.in_w; p.out_h = t.out_h; p.out_w = t.out_w; p.stride = t.stride; p.pad_t = t.pad_t; p.pad_l = t.pad_l;
+    p.kblocks = std::min(g.slabs * g.slab_blocks, (std::max(g.k, g.k_stride) + 31) / 32);
+    p.row_pixels = std::max((t.out_w - 1) * t.stride + kSlots, t.pad_l + t.in_w);
+    p.row_pixels += p.row_pixels & 1;
+    const int mt = p.kblocks == 1 ? 1 : 2, slices = 4 * wave_bytes(DT, mt);
+    auto bytes = [&](int rows) { return slices + ((rows - 1) * t.stride + t.kh) * p.row_pixels * kPixelBytes; };
+    if (bytes(1) > 65536) return EXHIP_ERR_UNSUPPORTED;
+    p.tile_rows = 1;
+    auto groups = [&](int rows) { return (long long)t.n * ((t.out_h + rows - 1) / rows); };
+    // Rows of a group: as many as leave four groups for every CU (16 x 112 x 112 -> 64: 5.1 us with one, 5.8 with four, 7.9 with eight), up to 512
+    // pixels and 32 KiB of LDS, five groups on a CU (64 x 112 x 112: 13.0 with one, 10.6 with two, 9.5 with four; 64 x 224 x 224: 29.9, 26.2, 25.9 and with
+    // eight 28.7).
+    if (g_exhip_options.stem > 1) p.tile_rows = std::min(g_exhip_options.stem, t.out_h);
+    else while (p.tile_rows < 8 && groups(p.tile_rows * 2) >= 1024 && p.tile_rows * 2 * t.out_w <= 512 && bytes(p.tile_rows * 2) <= 32768) p.tile_rows *= 2;
+    while (p.tile_rows > 1 && bytes(p.tile_rows) > 65536) --p.tile_rows;
+    if (groups(p.tile_rows) >= (1ll << 31)) return EXHIP_ERR_UNSUPPORTED;
+    p.items = (unsigned)groups(p.tile_rows);
+    p.ch_groups = (unsigned)((t.out_h + p.tile_rows - 1) / p.tile_rows);
+    exhip_host_divisor(p.ch_groups, &p.groups_magic, &p.groups_shift);
+    exhip_host_divisor((unsigned)t.out_w, &p.width_magic, &p.width_shift);
+    const bool vec = t.in_w % 8 == 0 && (uintptr_t)p.x % 16 == 0;
+    p.pieces = t.in_w / 8;
+    exhip_host_divisor((unsigned)(vec ? p.pieces : t.in_w), &p.pieces_magic, &p.pieces_shift);
+    const int lds = bytes(p.tile_rows);
+    if (mt == 1) return vec ? go_stem<DT, 1, true>(ctx, p, lds) : go_stem<DT, 1, false>(ctx, p, lds);
+    return vec ? go_stem<DT, 2, true>(ctx, p, lds) : go_stem<DT, 2, false>(ctx, p, lds);
 }
 
 // U > 0: the kernel with U k-steps a request round, 100 + U in pairs; U < 0: the split form, -kSplit a k-step at a time, -2 * kSplit in pairs
@@ -1506,42 +1586,18 @@ int exhip_conv1x1_i8_pw(exhip_ctx* ctx, const exhip_pw_geom& g, const int8_t* x,
 
 int exhip_conv_f16_stem(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, int channels, const uint16_t* x, const float* mean, const float* factor,
                         const void* wp, const float* bias, uint16_t* y) {
-    if (g_exhip_options.stem == 0 || t.kh != 3 || t.kw > 4 || t.stride < 1 || channels > 4 || g.k_stride % 8 != 0 || !pw_row_fits(4ll * g.k_stride) ||
-        g.pixels != (long long)t.n * t.out_h * t.out_w || g.pixels >= (1ll << 31) || g.pixels * 4 * g.k_stride >= (1ll << 40) || (long long)t.in_h * t.in_w >= (1ll << 28))
-        return EXHIP_ERR_UNSUPPORTED;
     PwParams p = {};
     p.x = reinterpret_cast<const char*>(x); p.wp = reinterpret_cast<const char*>(wp); p.bias = bias; p.y = y;
-    p.mean = mean; p.factor = factor; p.in_c = channels;
-    p.pixels = (unsigned)g.pixels; p.w_bytes = (unsigned)(g.slabs * t.kh * g.slab_blocks * 1024);
-    p.mts = g.slab_blocks; p.K = g.k; p.kstride = g.k_stride;
-    p.act = g.act; p.post_relu = g.post_relu; p.post_op = g.post_op; p.post_alpha = g.post_alpha; p.post_beta = g.post_beta;
-    p.post_slope = g.post_slope; p.post_slope_shared = g.post_slope_shared;
-    p.in_h = t.in_h; p.in_w = t.in_w; p.out_h = t.out_h; p.out_w = t.out_w; p.stride = t.stride; p.pad_t = t.pad_t; p.pad_l = t.pad_l;
-    p.kblocks = std::min(g.slabs * g.slab_blocks, (std::max(g.k, g.k_stride) + 31) / 32);
-    p.row_pixels = std::max((t.out_w - 1) * t.stride + 4, t.pad_l + t.in_w);
-    p.row_pixels += p.row_pixels & 1;
-    const int mt = p.kblocks == 1 ? 1 : 2, slices = 4 * wave_bytes(EXHIP_F16, mt);
-    auto bytes = [&](int rows) { return slices + ((rows - 1) * t.stride + t.kh) * p.row_pixels * 8; };
-    if (bytes(1) > 65536) return EXHIP_ERR_UNSUPPORTED;
-    p.tile_rows = 1;
-    auto groups = [&](int rows) { return (long long)t.n * ((t.out_h + rows - 1) / rows); };
-    // Rows of a group: as many as leave four groups for every CU (16 x 112 x 112 -> 64: 5.1 us with one, 5.8 with four, 7.9 with eight), up to 512
-    // pixels and 32 KiB of LDS, five groups on a CU (64 x 112 x 112: 13.0 with one, 10.6 with two, 9.5 with four; 64 x 224 x 224: 29.9, 26.2, 25.9 and with
-    // eight 28.7).
-    if (g_exhip_options.stem > 1) p.tile_rows = std::min(g_exhip_options.stem, t.out_h);
-    else while (p.tile_rows < 8 && groups(p.tile_rows * 2) >= 1024 && p.tile_rows * 2 * t.out_w <= 512 && bytes(p.tile_rows * 2) <= 32768) p.tile_rows *= 2;
-    while (p.tile_rows > 1 && bytes(p.tile_rows) > 65536) --p.tile_rows;
-    if (groups(p.tile_rows) >= (1ll << 31)) return EXHIP_ERR_UNSUPPORTED;
-    p.items = (unsigned)groups(p.tile_rows);
-    p.ch_groups = (unsigned)((t.out_h + p.tile_rows - 1) / p.tile_rows);
-    exhip_host_divisor(p.ch_groups, &p.groups_magic, &p.groups_shift);
-    exhip_host_divisor((unsigned)t.out_w, &p.width_magic, &p.width_shift);
-    const bool vec = t.in_w % 8 == 0 && (uintptr_t)x % 16 == 0;
-    p.pieces = t.in_w / 8;
-    exhip_host_divisor((unsigned)(vec ? p.pieces : t.in_w), &p.pieces_magic, &p.pieces_shift);
-    const int lds = bytes(p.tile_rows);
-    if (mt == 1) return vec ? go_stem<1, true>(ctx, p, lds) : go_stem<1, false>(ctx, p, lds);
-    return vec ? go_stem<2, true>(ctx, p, lds) : go_stem<2, false>(ctx, p, lds);
+    p.mean = mean; p.factor = factor;
+    return run_stem<EXHIP_F16>(ctx, g, t, channels, p);
+}
+
+int exhip_conv_i8_stem(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, int channels, const float* x, const float* mean, const float* factor,
+                       float fs_in, const void* wp, const float* scale, const float* bias, int8_t* y_i8, float* y_f32) {
+    PwParams p = {};
+    p.x = reinterpret_cast<const char*>(x); p.wp = reinterpret_cast<const char*>(wp); p.scale = scale; p.bias = bias; p.y_q = y_i8; p.y_f = y_f32;
+    p.mean = mean; p.factor = factor; p.fs_in = fs_in; p.fs_out = g.fs_out;
+    return run_stem<EXHIP_I8>(ctx, g, t, channels, p);
 }
 
 bool exhip_pw_splits_f16(long long pixels, int c_bytes, int k, int k_stride, int n_ksteps, int stride, int post_op) {

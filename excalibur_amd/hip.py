@@ -593,3 +593,9 @@ class Ctx:
         """The status: 0, or EXHIP_ERR_UNSUPPORTED where the layers run by themselves."""
         rc = lib().exhip_stem_f16(self.h, ctypes.byref(d), x.ptr, _ptr(mean), _ptr(factor), wp.ptr, _ptr(bias), y.ptr)
         return rc if rc == ERR_UNSUPPORTED else _check(rc) or 0
+
+    def stem_i8(self, d, x, mean, factor, fs_in, wp, scale, bias, y_i8, y_f32=None):
+        """As stem_f16."""
+        rc = lib().exhip_stem_i8(self.h, ctypes.byref(d), x.ptr, _ptr(mean), _ptr(factor), ctypes.c_float(fs_in), wp.ptr, scale.ptr, _ptr(bias),
+                                 _ptr(y_i8), _ptr(y_f32))
+        return rc if rc == ERR_UNSUPPORTED else _check(rc) or 0

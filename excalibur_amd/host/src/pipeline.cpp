@@ -698,7 +698,7 @@ struct pipeline<Dtype>::impl::fused_plan {
     std::vector<int> front_ops, tail_ops;
     std::shared_ptr<tensor<float>> front_blob;
     const float* input_ptr = nullptr;
-    int first_conv_launch = 1;  // 1: launch 0 is the input quantizer; 0: the stem kernel quantizes its own input
+    int first_conv_launch = 1;  // 1: launch 0 is the input quantizer; 0: a stem kernel quantizes its own input
     // Launches 1 .. end (everything behind the input quantizer, which alone reads the caller's input pointer) recorded as
     // one HIP graph: made on the plan's second forward (the first runs eagerly, which also sets the kernels' attributes),
     // replayed afterwards, made again when a result tensor was replaced.
@@ -1433,6 +1433,7 @@ bool pipeline<float>::impl::build_graph_plan(const tensor_ptr& input, const std:
         plan->outputs.back().blobs = blobs_of(value);
         return v.nchw;
     };
+    bool one_kernel = false;  // the front layers and the quantizer
     {
         value_info& v = vals[front_value];
         if (!v.need_i8 || v.need_f32 || v.need_nchw) return refuse(__LINE__);
@@ -1445,7 +1446,6 @@ bool pipeline<float>::impl::build_graph_plan(const tensor_ptr& input, const std:
         const value_info vi = v;
         fused_plan* pl = plan.get();
         // Input -> YoloV5Focus -> quantizer as one kernel where the library has it; else the two layers run as layers
-        bool one_kernel = false;
         if (plan->front_ops.size() == 2 && kind[plan->front_ops[0]] == 'n' && kind[plan->front_ops[1]] == 'f') {
             auto* in_op = static_cast<operation_input<float>*>(operations_[plan->front_ops[0]].get());
             const int ch = shape[1];
@@ -1599,6 +1599,29 @@ bool pipeline<float>::impl::build_graph_plan(const tensor_ptr& input, const std:
             const float *scale = c->scale_gpu(), *bias = c->bias_gpu();
             int8_t* yq = static_cast<int8_t*>(out.i8);
             float* yf = static_cast<float*>(out.f32);
+            // the first convolution alone reads the quantized input: Input layer, quantizer and convolution in one kernel where it takes the layer
+            if (nd.in[0] == front_value && consumers[front_value].size() == 1 && plan->launches.size() == 1 && !one_kernel && !res && !nchw &&
+                (plan->front_ops.empty() || (plan->front_ops.size() == 1 && kind[plan->front_ops[0]] == 'n'))) {
+                const float *mean = nullptr, *factor = nullptr;
+                if (!plan->front_ops.empty()) {
+                    auto* in_op = static_cast<operation_input<float>*>(operations_[plan->front_ops[0]].get());
+                    in_op->upload_tables(in.c);
+                    mean = in_op->means_dev_->gpu_data();
+                    factor = in_op->vars_dev_->gpu_data();
+                }
+                const float fs_in = in.fs;
+                const int rc = exhip_stem_i8(ctx, &d, input->gpu_data(), mean, factor, fs_in, wp, scale, bias, yq, yf);  // trial launch
+                if (rc == 0) {
+                    fused_plan* pl = plan.get();
+                    plan->launches[0] = [=]() { EXHIP_FATAL(exhip_stem_i8(ctx, &d, pl->input_ptr, mean, factor, fs_in, wp, scale, bias, yq, yf)); };
+                    plan->front_ops.clear();
+                    plan->first_conv_launch = 0;
+                    plan->buffers.erase(std::find_if(plan->buffers.begin(), plan->buffers.end(), [&](const dev_buffer& b) { return b.ptr == in.i8; }));
+                    vals[front_value].i8 = nullptr;
+                    continue;
+                }
+                if (rc != EXHIP_ERR_UNSUPPORTED) EXHIP_FATAL(rc);
+            }
             plan->launches.push_back(
                 [=]() { EXHIP_FATAL(exhip_conv2d_i8(ctx, &d, x, wp, scale, bias, res, yq, yf, nchw ? *nchw : nullptr, nullptr)); });
         } else if (nd.kind == 'g' && nd.joined) {

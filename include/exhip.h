@@ -69,7 +69,7 @@ const char* exhip_last_error(void);
  * layers (0 = the general kernel), "pw" the fp16 / int8 kernel without staging for pointwise layers and "direct" its
  * form for layers with a filter (1 where it measured faster, 2 wherever it can run, 0 never), "pw_tile" that kernel's wave
  * tile (0 = 32 pixels x 64 channels, 2 = 64 x 64 for large launches), "stem" the one-kernel stems (2 upwards:
- * that many output rows a group of the fp16 one): every form computes
+ * that many output rows a group of the ones without pooling): every form computes
  * the same values. "pw_split" chooses that kernel's split form (1 by its rule, 2 wherever it can run, 0 never; fp16 sums then run
  * in another order). "dw_pw" chooses the depthwise + pointwise fp16 pairs that exhip_dw_pw_f16 takes (1 by its rule, 2 wherever it can
  * run, a power of two from 4 to 256 so with that many pixels a group, 0 never; the same values). "f32_tile" pins the float32 convolution's wave tile and split (0 = its rule, n = the n-th of its list;
@@ -230,6 +230,10 @@ int exhip_dw_pw_f16(exhip_ctx* ctx, const exhip_depthwise_desc* dw, const exhip_
  * are given, both or neither. EXHIP_ERR_UNSUPPORTED, with nothing launched, where the layers run by themselves. */
 int exhip_stem_f16(exhip_ctx* ctx, const exhip_conv_desc* d, const uint16_t* x_nchw, const float* mean, const float* factor, const void* w_packed,
                    const float* bias, uint16_t* y_nhwc);
+/* The same of an int8 network on its float32 NCHW input: Input layer (or NULLs), quantizer with fs_in (src/Excalibur/operation_general_conv.cpp:584-720) and
+ * exhip_conv2d_i8 with the NHWC results only (y_i8 and / or y_f32). */
+int exhip_stem_i8(exhip_ctx* ctx, const exhip_conv_desc* d, const float* x_nchw, const float* mean, const float* factor, float fs_in, const void* w_packed,
+                  const float* scale, const float* bias, int8_t* y_i8, float* y_f32);
 
 /* A detection head: the 1x1 convolution, the Reshape of its channels into groups and the Transpose of the last two axes
  * (operation_reshape.cpp, operation_transpose.cpp) as one launch, y[n][k / group][pixel][group] (float32 of an int8 layer, halves).

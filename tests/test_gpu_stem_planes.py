@@ -1,5 +1,5 @@
-"""The first layer of an fp16 network on half planes, with the Input layer in front (conv_pw.hip, stem_f16_kernel): the results are those of the
-Input layer, the layout conversion and the convolution run one after the other, bit for bit."""
+"""The first layer of a network on its planes, with the Input layer in front (conv_pw.hip, stem_planes_kernel): the results are those of the
+Input layer, the layout conversion or quantizer and the convolution run one after the other, bit for bit."""
 import numpy as np
 import pytest
 
@@ -64,6 +64,42 @@ def test_stem_equals_the_layers(ctx, n, c, h, w, k, kw, stride, pad, post, scale
         assert np.array_equal(got[:-guard].reshape(want.shape), want.download())
     values = want.download().view(np.float16)[..., :k].astype(np.float32)
     assert np.isfinite(values).all() and np.ptp(values) > .5
+
+
+@pytest.mark.parametrize("scaled", [False, True], ids=["plain", "input"])
+@pytest.mark.parametrize("results", ["int8", "float", "both"])
+@pytest.mark.parametrize("n,c,h,w,k,kw,stride,pad,post", SHAPES[1:] + [(3, 3, 26, 24, 64, 7, 2, (3, 3, 3, 3), dict(act=1))],
+                         ids=[f"s{i}" for i in range(1, len(SHAPES) + 1)])
+def test_int8_stem_equals_the_layers(ctx, n, c, h, w, k, kw, stride, pad, post, results, scaled):
+    r = np.random.default_rng(h * w + k)
+    x = ctx.array((r.integers(0, 256, (n, c, h, w)) if scaled else r.normal(0, 1, (n, c, h, w))).astype(np.float32))
+    mean = ctx.array(r.uniform(100, 150, c).astype(np.float32)) if scaled else None
+    factor = ctx.array(r.uniform(.005, .02, c).astype(np.float32)) if scaled else None
+    ks, fs_in = hip.pad_to(k, 32), 60.0
+    d = ctx.conv_desc(n, c, h, w, k, (3, kw), stride, pad, c_stride=4, k_stride=ks, fs_out=40.0 if results != "float" else 0.0, **post)
+    oh, ow = ctx.conv_out_hw(d)
+    wp = ctx.pack_conv_weights(d, hip.I8, r.integers(-127, 128, (k, c, 3, kw), dtype=np.int8))
+    scale = ctx.array((r.uniform(.5, 1.5, k) / (fs_in * 73 * np.sqrt(9 * c))).astype(np.float32))
+    bias = ctx.array(r.normal(0, .3, k).astype(np.float32))
+    seen = ctx.channelwise_f32("input", x, mean, factor) if scaled else x
+    pixels = ctx.quantize_nchw_to_nhwc_i8(seen, fs_in, 4)
+    shape = (n, oh, ow, ks)
+    forms = [np.int8] * (results != "float") + [np.float32] * (results != "int8")
+    want = {t: ctx.empty(shape, t) for t in forms}
+    ctx.conv2d_i8(d, pixels, wp, scale, bias, None, want.get(np.int8), want.get(np.float32))
+    for rows in (1, 2, 4):
+        got = {t: ctx.array(np.full(want[t].size + 64 * ks, 77, t)) for t in forms}
+        hip.set_option("stem", rows)
+        try:
+            assert ctx.stem_i8(d, x, mean, factor, fs_in, wp, scale, bias, got.get(np.int8), got.get(np.float32)) == 0
+            ctx.sync()
+        finally:
+            hip.set_option("stem", 1)
+        for t in forms:
+            y = got[t].download()
+            assert (y[-64 * ks:] == 77).all()
+            assert np.array_equal(y[:-64 * ks].reshape(shape), want[t].download())
+    assert all(np.ptp(want[t].download()[..., :k].astype(np.float32)) > .5 for t in forms)
 
 
 def test_what_the_stem_leaves_to_the_layers(ctx):
