@@ -2048,6 +2048,24 @@ extern "C" int exhip_dw_pw_f16(exhip_ctx* ctx, const exhip_depthwise_desc* dw, c
     return run_conv<EXHIP_F16>(ctx, d, p, nullptr, nullptr, 0, &g);
 }
 
+extern "C" int exhip_conv2d_i8_maxpool2x2(exhip_ctx* ctx, const exhip_conv_desc* d, int pool_oh, int pool_ow, const int8_t* x, const void* wp,
+                                          const float* scale, const float* bias, int8_t* y_i8, float* y_f32) {
+    EXHIP_REQUIRE(ctx && d && x && wp && scale && (y_i8 || y_f32), "exhip_conv2d_i8_maxpool2x2: bad argument");
+    if (d->sh != d->sw || d->post_op || d->post_bn_a || d->exact_k || d->act > 1) return EXHIP_ERR_UNSUPPORTED;
+    Plan pl;
+    const int rc = make_plan(d, EXHIP_I8, &pl);
+    if (rc) return rc;
+    EXHIP_REQUIRE(pool_oh > 0 && pool_ow > 0 && 2 * pool_oh <= pl.OH && 2 * pool_ow <= pl.OW, "conv+pool: pooled size %dx%d does not fit a %dx%d convolution output",
+                  pool_oh, pool_ow, pl.OH, pl.OW);
+    if (pl.packed || pl.KWe != d->kw) return EXHIP_ERR_UNSUPPORTED;
+    exhip_pw_geom g = {};
+    g.pixels = 4ll * d->n * pool_oh * pool_ow; g.c_bytes = d->c_stride; g.k = d->k; g.k_stride = d->k_stride;
+    g.slab_blocks = pl.TM / 32; g.slabs = pl.ktiles;
+    g.act = d->act; g.post_relu = d->post_relu; g.fs_out = d->fs_out; g.pool = 1;
+    const exhip_pw_taps t = {d->n, d->h, d->w, 2 * pool_oh, 2 * pool_ow, d->kh, d->kw, d->sh, d->pt, d->pl, pl.n_chunks, pl.chunk_b};
+    return exhip_conv1x1_i8_pw(ctx, g, x, wp, scale, bias, nullptr, y_i8, y_f32, &t);
+}
+
 // The geometry of a first layer that the kernel on NCHW planes may take.
 static int stem_geometry(const exhip_conv_desc* d, int dt, exhip_pw_geom* g, exhip_pw_taps* t) {
     if (d->c_stride != 4 || d->c > 4 || d->sh != d->sw) return EXHIP_ERR_UNSUPPORTED;

@@ -21,6 +21,7 @@ struct exhip_pw_geom {
     const float* post_bn_b;
     int exact_k;
     int group, map_h, map_w;
+    int pool;                   // int8 layers with a filter: 1 with a 2x2 stride-2 max pooling behind it all, the results those of the pooled map
 };
 
 // A layer with a filter, a stride or padding on the same kernel (`taps` below; NULL: the pointwise layer). The wave's

@@ -24,6 +24,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cfloat>
 #include <cstdint>
 #include <type_traits>
 
@@ -80,7 +81,7 @@ struct PwParams {
     // filter row, tap and bytes left of the chunk -- and what leads from behind a row's last tap to the next row, and from
     // behind the last row to the next chunk
     int start_s[kSplit + 1], start_w[kSplit + 1], start_b[kSplit + 1], start_r[kSplit + 1], start_q[kSplit + 1], start_left[kSplit + 1];
-    int chunk_b, row_end_b, chunk_end_b;
+    int chunk_b, row_end_b, chunk_end_b, pool;
     int pair_w, next_w, chunk_w;  // pairs: k-steps of the weights from a pair's first to its second, to the next pair, and more behind the last tap
     // the depthwise 3x3 layer in front (dw_pw_kernel; geometry in in_h .. pad_l above, x is its input): weights, bias and PReLU slopes,
     // activation 0, 1 or 3; 32-pixel tiles of a group and output blocks of a group
@@ -112,7 +113,13 @@ enum { kPostNone, kPostRelu, kPostHardSwish, kPostLeaky, kPostPrelu, kPostHardSi
 template <int ACT, int POST, int RES, bool BN, bool ANY>
 struct EpT {
     static constexpr int act = ACT, post = POST, res = RES;  // res: 0 no shortcut, 1 added in front of the layers behind, 2 behind them
-    static constexpr bool bn = BN, any = ANY;
+    static constexpr bool bn = BN, any = ANY, pool = false;
+};
+// ... and a 2x2 stride-2 max pooling of whole windows behind them all: four neighbouring lanes have a window's pixels (p.out_h, p.out_w: the pooled map).
+// Spares a large layer the float32 map, which is most of its bytes: 32 -> 32 at 64 x 126 x 126 39.6 us and 28.1 for the pooling -> 32.3.
+template <typename E>
+struct Pooled : E {
+    static constexpr bool pool = true;
 };
 template <int ACT, int POST, int RES, bool BN = false>
 using Ep = EpT<ACT, POST, RES, BN, false>;
@@ -295,7 +302,32 @@ __device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[
                 for (int e = 0; e < 16; ++e)
                     if (ch0 + e >= p.K) v[e] = 0.f;
             }
-            if constexpr (I8) {
+            if constexpr (EP::pool) {
+                // the maximum over the quad's lanes, as the pooling kernel takes it (a NaN never is the larger one); each of them then stores
+                // four of the channels
+                const int member = lane & 3, ch = half * 16 + member * 4, pixel = row >> 2, quads = rows >> 2;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    v[e] = -FLT_MAX < v[e] ? v[e] : -FLT_MAX;
+                    const float beside = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v[e]), 0xB1, 0xF, 0xF, true));
+                    v[e] = v[e] < beside ? beside : v[e];
+                    const float below = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v[e]), 0x4E, 0xF, 0xF, true));
+                    v[e] = v[e] < below ? below : v[e];
+                }
+                v4f o;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = member == 0 ? v[e] : member == 1 ? v[4 + e] : member == 2 ? v[8 + e] : v[12 + e];
+                typedef unsigned v4u __attribute__((ext_vector_type(4)));
+                if (p.y_f)
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, o), tile_view(p.y_f, first >> 2, p.kstride * 4, kb * 128, quads),
+                                                           pw_lane_offset(pixel, p.kstride * 4, ch * 4, (k_end - kb * 32) * 4), 0, 0);
+                if (p.y_q) {
+                    uint32_t w = 0;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) w |= (uint32_t)(exhip_q8(o[e] * p.fs_out) & 0xff) << (8 * e);
+                    __builtin_amdgcn_raw_buffer_store_b32(w, tile_view(p.y_q, first >> 2, p.kstride, kb * 32, quads), pw_lane_offset(pixel, p.kstride, ch, k_end - kb * 32), 0, 0);
+                }
+            } else if constexpr (I8) {
                 if (p.y_f) {  // one block at a time: 128 bytes per pixel
                     constexpr int pitch = 128 + 16;
 #pragma unroll
@@ -380,8 +412,13 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
                 // the filter's top-left input pixel; its offset may lie in front of the tensor (padding), the taps inside the
                 // image never do, and 32-bit wrap-around of the sum gives their offsets
                 const unsigned per_image = (unsigned)(p.out_h * p.out_w);
-                const unsigned img = exhip_divide(pix, per_image, p.image_magic, p.image_shift), rem = pix - img * per_image;
-                const int oy = (int)exhip_divide(rem, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = (int)(rem - (unsigned)oy * (unsigned)p.out_w);
+                const unsigned place = EP::pool ? pix >> 2 : pix;
+                const unsigned img = exhip_divide(place, per_image, p.image_magic, p.image_shift), rem = place - img * per_image;
+                int oy = (int)exhip_divide(rem, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = (int)(rem - (unsigned)oy * (unsigned)p.out_w);
+                if constexpr (EP::pool) {
+                    oy = 2 * oy + (int)(pix >> 1 & 1);
+                    ox = 2 * ox + (int)(pix & 1);
+                }
                 const int iy = oy * p.stride - p.pad_t, ix = ox * p.stride - p.pad_l;
                 xoff[nt][l] = (((int)img * p.in_h + iy) * p.in_w + ix) * p.xs_b + byte;
                 unsigned row = 0, m = 0;
@@ -1244,6 +1281,14 @@ int pick_epilogue(exhip_ctx* ctx, const PwParams& p) {
         post = post == kPostNone ? op : -1;
     }
     const bool bn = p.post_bn_a != nullptr;
+    if (p.pool) {
+        if constexpr (DT == EXHIP_I8 && TAPS && U > 0) {
+            if (p.act == 0 && post == kPostNone) return go<DT, MT, NT, U, TAPS, Pooled<Ep<0, kPostNone, 0>>>(ctx, p);
+            if (p.act == 0 && post == kPostRelu) return go<DT, MT, NT, U, TAPS, Pooled<Ep<0, kPostRelu, 0>>>(ctx, p);
+            if (p.act == 1 && post == kPostNone) return go<DT, MT, NT, U, TAPS, Pooled<Ep<1, kPostNone, 0>>>(ctx, p);
+        }
+        return EXHIP_ERR_UNSUPPORTED;
+    }
     if (p.group) return go<DT, MT, NT, U == 8 ? 4 : U, TAPS, EpAny>(ctx, p);
     auto is = [&](int a, int q, int r, bool b) { return p.act == a && post == q && res == r && bn == b; };
     if (is(0, kPostNone, 0, false)) return go<DT, MT, NT, U, TAPS, Ep<0, kPostNone, 0>>(ctx, p);
@@ -1386,6 +1431,7 @@ template <int DT>
 int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwParams& p, bool has_residual) {
     if (g_exhip_options.direct == 0) return EXHIP_ERR_UNSUPPORTED;
     if (g.post_bn_a || g.post_bn_b || g.exact_k || g.group) return EXHIP_ERR_UNSUPPORTED;
+    if (g.pool && (DT != EXHIP_I8 || has_residual || t.out_h % 2 || t.out_w % 2)) return EXHIP_ERR_UNSUPPORTED;
     const long long n_ksteps = (long long)t.n_chunks * t.kh * t.kw * (t.chunk_b / 32);
     if (g.pixels <= 0 || g.c_bytes <= 0 || g.c_bytes % 32 != 0 || t.chunk_b % 32 != 0 || t.n_chunks * t.chunk_b != g.c_bytes ||
         (g.slab_blocks != 2 && g.slab_blocks != 4) || g.k_stride % 8 != 0 || !pw_row_fits(4ll * g.k_stride) || (n_ksteps > (g.c_bytes % 64 ? 1 : 2) * kMaxDirectSteps && !split_wins(DT, g, (std::max(g.k, g.k_stride) + 31) / 32, (int)n_ksteps, true, t.stride)) || t.kh * t.kw > (1 << (32 - kTapShift)) || t.stride < 1 || t.pad_t < 0 || t.pad_l < 0)
@@ -1421,8 +1467,13 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
         if (p.y_f) return n_ksteps <= 40 ? 12000 : 4096;
         return g.post_relu && n_ksteps > 18 ? 3328 : 0;
     };
-    const bool take = kblocks == 1 || DT == EXHIP_F16 || g.c_bytes == 32 || blocks <= int8_most();
-    const bool split = split_wins(DT, g, kblocks, (int)n_ksteps, true, t.stride);
+    const bool take = g.pool || kblocks == 1 || DT == EXHIP_F16 || g.c_bytes == 32 || blocks <= int8_most();
+    // With the pooling layer behind it: where the layer by itself would run in the split form, on few blocks, that and a launch for the pooling are
+    // the faster two, us as two launches -> as one: 64 -> 128 at 1 x 30 x 30 7.4 -> 6.4, 128 -> 128 at 1 x 14 x 14 (36 k-steps) 8.0 against 8.4, at 16
+    // x 14 x 14 (288 blocks) 8.7 and 8.6, 256 -> 256 at 4 x 16 x 16 (72 k-steps) 9.5 against 13.2, at 16 x 16 x 16 (1024) 14.2 -> 13.5. Beyond, the float32
+    // map that is neither stored nor read decides: 32 -> 64 at 64 x 62 x 62 31.6 -> 17.2, 64 -> 64 at 64 x 112 x 112 112.9 -> 64.2.
+    if (g.pool && g_exhip_options.direct != 2 && blocks <= (n_ksteps <= 18 ? 0 : n_ksteps <= 40 ? 300 : 960)) return EXHIP_ERR_UNSUPPORTED;
+    const bool split = !g.pool && split_wins(DT, g, kblocks, (int)n_ksteps, true, t.stride);
     if (g_exhip_options.direct != 2 && !take && !split) return EXHIP_ERR_UNSUPPORTED;
     p.post_slope = g.post_slope;
     p.pixels = (unsigned)g.pixels; p.x_bytes = (unsigned)x_bytes; p.w_bytes = (unsigned)w_bytes;
@@ -1431,10 +1482,11 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
     p.act = g.act; p.post_relu = g.post_relu; p.post_op = g.post_op; p.post_slope_shared = g.post_slope_shared;
     p.residual_last = g.residual_last && has_residual;
     p.post_alpha = g.post_alpha; p.post_beta = g.post_beta;
-    p.in_h = t.in_h; p.in_w = t.in_w; p.out_h = t.out_h; p.out_w = t.out_w; p.stride = t.stride; p.pad_t = t.pad_t; p.pad_l = t.pad_l;
+    p.pool = g.pool;
+    p.in_h = t.in_h; p.in_w = t.in_w; p.out_h = t.out_h >> g.pool; p.out_w = t.out_w >> g.pool; p.stride = t.stride; p.pad_t = t.pad_t; p.pad_l = t.pad_l;
     p.kh = t.kh; p.kw = t.kw;
-    exhip_host_divisor((unsigned)(t.out_h * t.out_w), &p.image_magic, &p.image_shift);
-    exhip_host_divisor((unsigned)t.out_w, &p.width_magic, &p.width_shift);
+    exhip_host_divisor((unsigned)(p.out_h * p.out_w), &p.image_magic, &p.image_shift);
+    exhip_host_divisor((unsigned)p.out_w, &p.width_magic, &p.width_shift);
     p.chunk_b = t.chunk_b;
     p.row_end_b = (t.in_w - t.kw) * g.c_bytes;
     p.chunk_end_b = t.chunk_b - t.kh * t.in_w * g.c_bytes;

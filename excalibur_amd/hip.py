@@ -599,3 +599,8 @@ class Ctx:
         rc = lib().exhip_stem_i8(self.h, ctypes.byref(d), x.ptr, _ptr(mean), _ptr(factor), ctypes.c_float(fs_in), wp.ptr, scale.ptr, _ptr(bias),
                                  _ptr(y_i8), _ptr(y_f32))
         return rc if rc == ERR_UNSUPPORTED else _check(rc) or 0
+
+    def conv2d_i8_maxpool2x2(self, d, pool_oh, pool_ow, x, wp, scale, bias=None, y_i8=None, y_f32=None):
+        """As stem_f16."""
+        rc = lib().exhip_conv2d_i8_maxpool2x2(self.h, ctypes.byref(d), pool_oh, pool_ow, x.ptr, wp.ptr, scale.ptr, _ptr(bias), _ptr(y_i8), _ptr(y_f32))
+        return rc if rc == ERR_UNSUPPORTED else _check(rc) or 0

@@ -1502,6 +1502,7 @@ bool pipeline<float>::impl::build_graph_plan(const tensor_ptr& input, const std:
         for (auto& r : plan->outputs)
             if (r.launch < 0) r.launch = static_cast<int>(plan->launches.size()) - 1;
     };
+    int pooled_already = -1;  // a pooling layer's value that the convolution in front has written
     for (const node& nd : nodes) {
         results_complete();
         const value_info in = vals[nd.in[0]];
@@ -1622,6 +1623,38 @@ bool pipeline<float>::impl::build_graph_plan(const tensor_ptr& input, const std:
                 }
                 if (rc != EXHIP_ERR_UNSUPPORTED) EXHIP_FATAL(rc);
             }
+            // a 2x2 max pooling layer that alone reads the float32 result: in the convolution's epilogue where that takes the layer
+            const size_t next = static_cast<size_t>(&nd - nodes.data()) + 1;
+            if (yf && !yq && !nchw && !res && next < nodes.size() && nodes[next].kind == 'p' && nodes[next].as_f32 && nodes[next].cascade < 0 &&
+                nodes[next].in[0] == nd.out) {
+                int readers = 0;
+                for (const node& m : nodes) readers += static_cast<int>(std::count(m.in.begin(), m.in.end(), nd.out)) + (m.res == nd.out ? 1 : 0);
+                auto* p = static_cast<operation_pooling<float>*>(operations_[nodes[next].op].get());
+                int kh, kw, sh, sw, pt, pb, pl, pr, ph, pw;
+                p->geometry(oh, ow, &kh, &kw, &sh, &sw, &pt, &pb, &pl, &pr, &ph, &pw);
+                if (readers == 1 && kh == 2 && kw == 2 && sh == 2 && sw == 2 && pt == 0 && pl == 0 && 2 * ph <= oh && 2 * pw <= ow) {
+                    value_info& to = vals[nodes[next].out];
+                    const size_t pooled = static_cast<size_t>(out.n) * ph * pw * ks;
+                    exhip_conv_desc dp = d;
+                    dp.fs_out = to.need_i8 ? to.fs : 0.f;
+                    void* q = to.need_i8 ? alloc(pooled) : nullptr;
+                    void* f = to.need_f32 || to.need_nchw || !q ? alloc(pooled * sizeof(float)) : nullptr;
+                    int8_t* pq = static_cast<int8_t*>(q);
+                    float* pf = static_cast<float*>(f);
+                    const int rc = exhip_conv2d_i8_maxpool2x2(ctx, &dp, ph, pw, x, wp, scale, bias, pq, pf);  // trial launch
+                    if (rc == 0) {
+                        plan->launches.push_back([=]() { EXHIP_FATAL(exhip_conv2d_i8_maxpool2x2(ctx, &dp, ph, pw, x, wp, scale, bias, pq, pf)); });
+                        plan->buffers.erase(std::find_if(plan->buffers.begin(), plan->buffers.end(), [&](const dev_buffer& b) { return b.ptr == yf; }));
+                        out.f32 = nullptr;
+                        to.i8 = q; to.f32 = f;
+                        pooled_already = nodes[next].out;
+                        continue;
+                    }
+                    if (rc != EXHIP_ERR_UNSUPPORTED) EXHIP_FATAL(rc);
+                    for (void* unused : {q, f})
+                        if (unused) plan->buffers.erase(std::find_if(plan->buffers.begin(), plan->buffers.end(), [&](const dev_buffer& b) { return b.ptr == unused; }));
+                }
+            }
             plan->launches.push_back(
                 [=]() { EXHIP_FATAL(exhip_conv2d_i8(ctx, &d, x, wp, scale, bias, res, yq, yf, nchw ? *nchw : nullptr, nullptr)); });
         } else if (nd.kind == 'g' && nd.joined) {
@@ -1706,6 +1739,12 @@ bool pipeline<float>::impl::build_graph_plan(const tensor_ptr& input, const std:
             auto* p = static_cast<operation_pooling<float>*>(operations_[nd.op].get());
             int kh, kw, sh, sw, pt, pb, pl, pr, oh, ow;
             p->geometry(in.h, in.w, &kh, &kw, &sh, &sw, &pt, &pb, &pl, &pr, &oh, &ow);
+            if (nd.out == pooled_already) {  // in the launch of the convolution in front
+                out.n = in.n; out.c = in.c; out.h = oh; out.w = ow; out.cs = in.cs;
+                if (out.need_nchw) nchw_from_f32(out, nd.out);
+                if (!more_forms(out)) return refuse(__LINE__);
+                continue;
+            }
             const void* source = nd.as_f32 ? in.f32 : in.int8_at(out.fs);
             if (nd.cascade >= 0) {  // the smaller pool's result, pooled again (same size as the input: stride 1, "same" padding)
                 const value_info& q = vals[nd.cascade];

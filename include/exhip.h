@@ -225,6 +225,11 @@ typedef struct exhip_depthwise_desc {
 int exhip_dw_pw_f16(exhip_ctx* ctx, const exhip_depthwise_desc* dw, const exhip_conv_desc* d, const void* w_packed, const float* bias,
                     const uint16_t* residual_nhwc, uint16_t* y_nhwc);
 
+/* exhip_conv2d_i8 and the 2x2 stride-2 max pooling behind it (operation_pooling.cpp:145-159, windows inside the map: 2 * pool_oh <= output rows) as one launch;
+ * y_i8 and / or y_f32 are the pooled NHWC results. EXHIP_ERR_UNSUPPORTED, with nothing launched, where the two run by themselves. */
+int exhip_conv2d_i8_maxpool2x2(exhip_ctx* ctx, const exhip_conv_desc* d, int pool_oh, int pool_ow, const int8_t* x_nhwc, const void* w_packed,
+                               const float* scale, const float* bias, int8_t* y_i8, float* y_f32);
+
 /* The first layer of an fp16 network on its half NCHW input: exhip_conv2d_f16 of at most four channels (c_stride 4, its packed weights) with the NHWC
  * result, without the conversion in front; with the Input layer (operation_input.cpp, (x - mean[c]) * factor[c] rounded to half) where mean and factor
  * are given, both or neither. EXHIP_ERR_UNSUPPORTED, with nothing launched, where the layers run by themselves. */
