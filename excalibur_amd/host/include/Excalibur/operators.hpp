@@ -38,6 +38,8 @@ template <typename Dtype>
 class operation_convolutiondepthwise;
 template <typename Dtype>
 class operation_input;
+template <typename Dtype>
+class operation_reshape;
 
 template <typename Dtype>
 class operation_convolution : public operation_general_conv<Dtype> {
@@ -86,6 +88,11 @@ public:
     // fp16: this layer, of at most four input channels, straight on its NCHW input, with the Input layer that it alone reads in front of it
     // (or NULL) and the layers set behind it; `bottoms` are the first one's. False, with nothing done, where the layers run by themselves.
     bool forward_stem(operation_input<Dtype>* input, const tensor_list<unsigned short>& bottoms, tensor_list<unsigned short>& tops);
+    // fp16: this layer, a pointwise one, with the Reshape of its channels into groups and the Transpose of the last two axes behind it (a detection
+    // head) as one launch; `tops` are the Transpose layer's. False, with nothing done, where the three run by themselves.
+    bool forward_head(const operation_reshape<Dtype>& reshape, const tensor_list<unsigned short>& bottoms, tensor_list<unsigned short>& tops);
+    // fp16: an NCHW result of NHWC pixels is made from NHWC rows, so that a head's layers by themselves run the kernel, and add in the order, of the one launch
+    void set_through_rows() { through_rows_ = true; }
     // int8 layers on the MFMA kernel. The next forward calls also write the int8 NHWC form of the output that a reader
     // quantizing with `fs` into `stride` channels per pixel would make of it (attached to the top blob as its
     // `quantized` copy), and with `only` leave the float data unwritten; fs = 0 switches it off. False where this
@@ -99,6 +106,7 @@ protected:
     void forward_gpu_i8(const tensor_list<float>& bottoms, tensor_list<float>& tops) override;
     void forward_gpu_f16(const tensor_list<unsigned short>& bottoms, tensor_list<unsigned short>& tops) override;
     bool mfma_path_ok() const;
+    bool through_rows_ = false;
     const unsigned short* sum_operand(const tensor_list<unsigned short>& tops, exhip_conv_desc* d);
     int post_op_ = 0;
     float post_alpha_ = 0.f, post_beta_ = 0.f;

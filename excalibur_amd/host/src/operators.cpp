@@ -552,6 +552,13 @@ void operation_convolution<Dtype>::forward_gpu_f16(const tensor_list<unsigned sh
     const bool out_nhwc = this->output_channel_ % 16 == 0 && nhwc_allowed();
     tops[0] = out_nhwc ? new_tensor<unsigned short>({n, oh, ow, this->output_channel_}, dev, memory::NHWC)
                        : new_tensor<unsigned short>({n, this->output_channel_, oh, ow}, dev);
+    if (through_rows_ && !out_nhwc && x == bottoms[0]) {
+        d.k_stride = (this->output_channel_ + 31) / 32 * 32;
+        auto rows = new_tensor<unsigned short>({n, oh, ow, d.k_stride}, dev);
+        EXHIP_FATAL(exhip_conv2d_f16(this->ctx(), &d, x->gpu_data(), packed_weights(EXHIP_F16, d), bias_gpu(), nullptr, rows->mutable_gpu_data(), nullptr, nullptr));
+        EXHIP_FATAL(exhip_nhwc_f16_to_nchw_f16(this->ctx(), rows->gpu_data(), n, this->output_channel_, oh, ow, d.k_stride, tops[0]->mutable_gpu_data()));
+        return;
+    }
     unsigned short* y = tops[0]->mutable_gpu_data();
     const unsigned short* residual = out_nhwc ? sum_operand(tops, &d) : nullptr;
     EXHIP_FATAL(exhip_conv2d_f16(this->ctx(), &d, x->gpu_data(), packed_weights(EXHIP_F16, d), bias_gpu(), residual,
@@ -584,6 +591,25 @@ bool operation_convolution<Dtype>::forward_stem(operation_input<Dtype>* input, c
     auto y = new_tensor<unsigned short>({n, oh, ow, this->output_channel_}, dev, memory::NHWC);
     const int rc = exhip_stem_f16(this->ctx(), &d, bottoms[0]->gpu_data(), input ? input->means_dev_->gpu_data() : nullptr,
                                   input ? input->vars_dev_->gpu_data() : nullptr, packed_weights(EXHIP_F16, d), bias_gpu(), y->mutable_gpu_data());
+    if (rc == EXHIP_ERR_UNSUPPORTED) return false;
+    EXHIP_FATAL(rc);
+    tops[0] = y;
+    return true;
+}
+
+template <typename Dtype>
+bool operation_convolution<Dtype>::forward_head(const operation_reshape<Dtype>& reshape, const tensor_list<unsigned short>& bottoms,
+                                                tensor_list<unsigned short>& tops) {
+    const int dev = this->params_.device_, c = this->input_channels();
+    if (bottoms[0]->order() != memory::NHWC || bottoms[0]->channels() != c || !mfma_path_ok() || !nhwc_allowed()) return false;
+    const int n = bottoms[0]->num(), h = bottoms[0]->height(), w = bottoms[0]->width();
+    exhip_conv_desc d = describe(n, h, w, c, (this->output_channel_ + 31) / 32 * 32);
+    if (d.kh != 1 || d.kw != 1 || d.sh != 1 || d.sw != 1 || d.pt || d.pb || d.pl || d.pr || conv_in_stride(c, EXHIP_F16, 1) != c) return false;
+    d.c_stride = c;
+    const std::vector<int> to = reshape.new_shape({n, this->output_channel_, h, w}, static_cast<int>(static_cast<size_t>(n) * this->output_channel_ * h * w));
+    if (to.size() != 4 || to[0] != n || to[1] < 1 || to[2] < 1 || to[1] * to[2] != this->output_channel_ || to[3] != h * w) return false;
+    auto y = new_tensor<unsigned short>({n, to[1], to[3], to[2]}, dev);
+    const int rc = exhip_conv2d_f16_grouped(this->ctx(), &d, to[2], bottoms[0]->gpu_data(), packed_weights(EXHIP_F16, d), bias_gpu(), y->mutable_gpu_data());
     if (rc == EXHIP_ERR_UNSUPPORTED) return false;
     EXHIP_FATAL(rc);
     tops[0] = y;
