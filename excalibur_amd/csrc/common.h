@@ -100,7 +100,7 @@ struct exhip_options {
                              // patch, 3 persistent groups with three slice buffers, 4 persistent groups with two
     int direct = 1;          // layers with a filter, a stride or padding and NHWC results on the pointwise kernel's tapped form: 1 where it measured
                              // faster, 2 wherever it can run, 0 never
-    int pw_tile = 0;         // that kernel's wave tile for more than 32 output channels: 0 = 32 pixels x 64 channels, 2 = 64 x 64 from 2048 waves on
+    int pw_tile = 0;         // that kernel's wave tile for more than 32 output channels: 0 = 32 pixels x 64 channels, 2 = 64 x 64 from 2048 waves on, without a pooling layer in the launch
     int f32_tile = 0;        // the float32 convolution's wave tile and split: 0 by its rule, n = the n-th of its list
     int dw_pw = 1;           // depthwise + pointwise fp16 pairs in one kernel: 1 by its rule, 2 wherever it can run, 4, 8 .. 256 so with that many pixels a group, 0 never
     int pw_split = 1;        // that kernel's split form (several waves to a tile): 1 by its rule, 2 wherever it can run, 0 never

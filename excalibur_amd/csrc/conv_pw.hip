@@ -1492,8 +1492,9 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
     p.chunk_end_b = t.chunk_b - t.kh * t.in_w * g.c_bytes;
     if (split) return launch_split<DT, true>(ctx, p, kblocks);
     if (kblocks == 1) return launch<DT, 1, 2, true>(ctx, p, kblocks);
+    // (the 64 x 64 tile has the epilogue without pooling only: it would number the pooled map's pixels as the convolution's, four times too many)
     const long long waves64 = ((g.pixels + 63) / 64) * ((kblocks + 1) / 2);
-    if (waves64 < 2048 || small_tile<DT>()) return launch<DT, 2, 1, true>(ctx, p, kblocks);
+    if (g.pool || waves64 < 2048 || small_tile<DT>()) return launch<DT, 2, 1, true>(ctx, p, kblocks);
     return launch<DT, 2, 2, true>(ctx, p, kblocks);
 }
 

@@ -68,7 +68,7 @@ const char* exhip_last_error(void);
  * "lean" / "lean_cfg" / "lean_wres" / "lean_groups" / "lean_f16" choose the form of the lean 3x3 kernel for int8 / fp16
  * layers (0 = the general kernel), "pw" the fp16 / int8 kernel without staging for pointwise layers and "direct" its
  * form for layers with a filter (1 where it measured faster, 2 wherever it can run, 0 never), "pw_tile" that kernel's wave
- * tile (0 = 32 pixels x 64 channels, 2 = 64 x 64 for large launches), "stem" the one-kernel stems (2 upwards:
+ * tile (0 = 32 pixels x 64 channels, 2 = 64 x 64 for large launches without a pooling layer), "stem" the one-kernel stems (2 upwards:
  * that many output rows a group of the ones without pooling): every form computes
  * the same values. "pw_split" chooses that kernel's split form (1 by its rule, 2 wherever it can run, 0 never; fp16 sums then run
  * in another order). "dw_pw" chooses the depthwise + pointwise fp16 pairs that exhip_dw_pw_f16 takes (1 by its rule, 2 wherever it can

@@ -30,10 +30,8 @@ SHAPES = [
 ]
 
 
-@pytest.mark.parametrize("act,post_relu", [(0, 0), (1, 0), (0, 1)], ids=["none", "relu", "relu_layer"])
-@pytest.mark.parametrize("results", ["int8", "float", "both"])
-@pytest.mark.parametrize("n,c,h,w,k,kernel,stride,pad", SHAPES, ids=[f"s{i}" for i in range(len(SHAPES))])
-def test_pooled_equals_the_two_layers(ctx, n, c, h, w, k, kernel, stride, pad, results, act, post_relu):
+def pooled_and_the_two_layers(ctx, n, c, h, w, k, kernel, stride, pad, results, act=0, post_relu=0, **options):
+    """Asserts that the one launch gives the bytes of the two layers and writes nothing behind its results; its status."""
     r = np.random.default_rng(h * w + k)
     cs, ks = hip.pad_to(c, 32), hip.pad_to(k, 32)
     d = ctx.conv_desc(n, c, h, w, k, kernel, stride, pad, act, cs, ks, post_relu, 40.0 if results != "float" else 0.0)
@@ -54,21 +52,39 @@ def test_pooled_equals_the_two_layers(ctx, n, c, h, w, k, kernel, stride, pad, r
     hip._check(hip.lib().exhip_maxpool2d_nhwc_f32(ctx.h, mid.ptr, ptr(want.get(np.float32)), ptr(want.get(np.int8)), ctypes.c_float(40.0), n, ks, oh, ow, ks, ph, pw,
                                                   2, 2, 2, 2, 0, 0))
     got = {t: ctx.array(np.full(want[t].size + 64 * ks, 77, t)) for t in forms}
-    hip.set_option("direct", 2)
+    defaults = dict(direct=1, pw_tile=0)
+    for name in options:
+        hip.set_option(name, options[name])
     try:
         rc = ctx.conv2d_i8_maxpool2x2(d, ph, pw, x, wp, scale, bias, got.get(np.int8), got.get(np.float32))
     finally:
-        hip.set_option("direct", 1)
-    if kernel == 1:   # pointwise layers have no taps to place: the two layers run by themselves, or the same values
-        assert rc in (0, hip.ERR_UNSUPPORTED)
-        if rc:
-            return
-    assert rc == 0
+        for name in options:
+            hip.set_option(name, defaults[name])
+    if rc:
+        return rc
     for t in forms:
         y = got[t].download()
         assert (y[-64 * ks:] == 77).all()
         assert np.array_equal(y[:-64 * ks].reshape(shape), want[t].download())
     assert all(np.ptp(want[t].download()[..., :k].astype(np.float32)) > .5 for t in forms)
+    return 0
+
+
+@pytest.mark.parametrize("act,post_relu", [(0, 0), (1, 0), (0, 1)], ids=["none", "relu", "relu_layer"])
+@pytest.mark.parametrize("results", ["int8", "float", "both"])
+@pytest.mark.parametrize("n,c,h,w,k,kernel,stride,pad", SHAPES, ids=[f"s{i}" for i in range(len(SHAPES))])
+def test_pooled_equals_the_two_layers(ctx, n, c, h, w, k, kernel, stride, pad, results, act, post_relu):
+    rc = pooled_and_the_two_layers(ctx, n, c, h, w, k, kernel, stride, pad, results, act, post_relu, direct=2)
+    assert rc in ((0, hip.ERR_UNSUPPORTED) if kernel == 1 else (0,))   # pointwise layers have no taps to place: the two layers may run by themselves
+
+
+# waves of 64 pixels x 64 channels (2048 and more take the larger wave tile where option pw_tile asks for it): 2048 exactly, one less, a layer with an
+# odd number of channel blocks, one with single k-steps
+@pytest.mark.parametrize("results", ["int8", "float", "both"])
+@pytest.mark.parametrize("n,c,h,w,k", [(32, 64, 64, 64, 64), (89, 32, 46, 32, 48), (21, 64, 65, 67, 96), (32, 96, 64, 64, 64)], ids=["most", "fewer", "odd", "single"])
+def test_pooled_equals_the_two_layers_whatever_the_tile_option(ctx, n, c, h, w, k, results):
+    for tile in (0, 2):
+        assert pooled_and_the_two_layers(ctx, n, c, h, w, k, 3, 1, 1, results, direct=2, pw_tile=tile) == 0
 
 
 def test_what_the_pooled_form_leaves_to_the_layers(ctx):
