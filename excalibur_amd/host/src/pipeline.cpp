@@ -1663,6 +1663,7 @@ bool pipeline<float>::impl::build_graph_plan(const tensor_ptr& input, const std:
                     plan->first_conv_launch = 0;
                     plan->buffers.erase(std::find_if(plan->buffers.begin(), plan->buffers.end(), [&](const dev_buffer& b) { return b.ptr == in.i8; }));
                     vals[front_value].i8 = nullptr;
+                    if (!more_forms(out)) return refuse(__LINE__);
                     continue;
                 }
                 if (rc != EXHIP_ERR_UNSUPPORTED) EXHIP_FATAL(rc);

@@ -109,3 +109,53 @@ def test_what_the_stem_leaves_to_the_layers(ctx):
         assert ctx.stem_f16(d, x, None, None, w, None, y) == hip.ERR_UNSUPPORTED
     with pytest.raises(hip.ExhipError):
         ctx.stem_f16(ctx.conv_desc(1, 3, 16, 16, 64, 3, 1, 1, c_stride=4, k_stride=64), x, ctx.empty((3,), np.float32).zero(), None, w, None, y)
+
+
+@pytest.mark.parametrize("scales", [(40.0, 30.0), (40.0, 30.0, 40.0, 20.0)], ids=["two", "three"])
+@pytest.mark.parametrize("channels", [32, 24])
+@pytest.mark.parametrize("front", ["Input", "none"])
+def test_int8_plan_whose_first_layer_is_read_at_several_scales(tmp_path, front, channels, scales):
+    """The first layer's float32 result is quantized again for the readers with other feature-map scales, as any layer's is: the plan takes the
+    network, with the first layer as one launch or as a quantizer and a convolution, and gives the separate layers' bytes."""
+    from excalibur_amd import modelfile as mf
+    from excalibur_amd import pipeline as xp
+    r = np.random.default_rng(7)
+    lines, blobs = ["Input data 0 1 data 0=40 1=24 2=3 3=104,117,123 4=0.017,0.018,0.017"] if front == "Input" else [], []
+
+    def conv(bottom, top, cin, k, kernel, stride, fs):
+        w = r.normal(0, np.sqrt(2.0 / (cin * kernel * kernel)), (k, cin, kernel, kernel)).astype(np.float32)
+        ws = (np.float32(127.0) / np.abs(w).reshape(k, -1).max(axis=1)).astype(np.float32)
+        wq = np.clip(np.rint(w * ws[:, None, None, None]), -127, 127).astype(np.int8)
+        lines.append(mf.conv_line("Convolution", top + "_l", bottom, top, k, kernel, stride, kernel // 2, True, w.size, 1, int8=True))
+        blobs.append(mf.conv_blob_i8(wq, r.normal(0, .3, k).astype(np.float32), ws, np.float32(fs)))
+
+    conv("data", "c0", 3, channels, 3, 2, 50.0)
+    lines.append("HardSwish hs0 1 1 c0 a0 0=1.666667e-01 1=5.000000e-01")
+    readers = [f"a0_{i}" for i in range(len(scales))]
+    lines.append(f"Split sp0 1 {len(scales)} a0 " + " ".join(readers))
+    outputs = [f"c{i + 1}" for i in range(len(scales))]
+    for reader, top, fs in zip(readers, outputs, scales):
+        conv(reader, top, channels, 16, 1, 1, fs)
+    path = str(tmp_path / "net.racy")
+    mf.write_model(path, blobs)
+    x = np.random.default_rng(8).uniform(0, 255, (3, 3, 24, 40)).astype(np.float32)
+    if front != "Input":
+        x = (x - 128) / 64
+    got, launches = {}, {}
+    for way, fusion, stem in (("layers", False, 1), ("quantizer", True, 0), ("stem", True, 1)):
+        hip.set_option("stem", stem)
+        try:
+            p = xp.Pipeline(mf.topology(lines, "scales"), path, 0, fusion=fusion)
+            p.time_fused_span(0)
+            p.forward(x)
+            assert p.fused == fusion, way
+            launches[way] = p.last_span()[1]
+            got[way] = {b: p.get(b) for b in outputs}
+            p.close()
+        finally:
+            hip.set_option("stem", 1)
+    assert launches["stem"] == launches["quantizer"] - 1
+    for b in outputs:
+        assert np.ptp(got["layers"][b]) > .5
+        for way in ("quantizer", "stem"):
+            assert np.array_equal(got[way][b].view(np.uint32), got["layers"][b].view(np.uint32)), (way, b)
