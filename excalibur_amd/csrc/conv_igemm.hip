@@ -1659,6 +1659,15 @@ inline bool fused_epilogue_ok(const exhip_conv_desc* d, const ConvParams& p, lon
            out_elems < (long long)kEpiInvalid;
 }
 
+// What every kernel asks of its operands: rows of the NHWC tensors that do not overlap, and the alignment of its loads. A stem's planes have
+// none and come as NULL here.
+int check_operands(const exhip_conv_desc* d, bool rows, const void* x, const void* wp, const float* scale, const float* bias) {
+    EXHIP_REQUIRE(d->k_stride >= d->k || !rows, "conv: k_stride %d < k %d", d->k_stride, d->k);
+    EXHIP_REQUIRE((uintptr_t)scale % 16 == 0 && (uintptr_t)bias % 16 == 0, "conv: scale and bias arrays must be 16-byte aligned");
+    EXHIP_REQUIRE((uintptr_t)x % 16 == 0 && (uintptr_t)wp % 16 == 0, "conv: input and weights must be 16-byte aligned");
+    return 0;
+}
+
 template <int DT>
 int run_conv(exhip_ctx* ctx, const exhip_conv_desc* d, ConvParams p, const PoolSpec* pool = nullptr, const exhip_lean_proj* proj = nullptr, int group = 0,
              const exhip_pw_depthwise* dw = nullptr) {
@@ -1678,11 +1687,9 @@ int run_conv(exhip_ctx* ctx, const exhip_conv_desc* d, ConvParams p, const PoolS
         }
     }
     EXHIP_REQUIRE(p.x && p.wp, "conv: NULL input or weights");
-    EXHIP_REQUIRE(d->k_stride >= d->k || (!p.y_q && !p.y_nhwc && !p.residual), "conv: k_stride %d < k %d", d->k_stride, d->k);
     EXHIP_REQUIRE(!(p.y_q) || d->k_stride % 16 == 0, "conv: NHWC int8/half output needs k_stride %% 16 == 0");
-    EXHIP_REQUIRE((!p.scale || (uintptr_t)p.scale % 16 == 0) && (!p.bias || (uintptr_t)p.bias % 16 == 0),
-                  "conv: scale and bias arrays must be 16-byte aligned");
-    EXHIP_REQUIRE((uintptr_t)p.x % 16 == 0 && (uintptr_t)p.wp % 16 == 0, "conv: input and weights must be 16-byte aligned");
+    rc = check_operands(d, p.y_q || p.y_nhwc || p.residual, p.x, p.wp, p.scale, p.bias);
+    if (rc) return rc;
     p.N = d->n; p.H = d->h; p.W = d->w; p.K = d->k; p.OH = pl.OH; p.OW = pl.OW;
     p.KH = d->kh; p.KWe = pl.KWe; p.KS = pl.KS; p.S = pl.S; p.tile_step = pl.tile_step;
     p.PT = d->pt; p.PL = d->pl;
@@ -2051,11 +2058,12 @@ extern "C" int exhip_dw_pw_f16(exhip_ctx* ctx, const exhip_depthwise_desc* dw, c
 extern "C" int exhip_conv2d_i8_maxpool2x2(exhip_ctx* ctx, const exhip_conv_desc* d, int pool_oh, int pool_ow, const int8_t* x, const void* wp,
                                           const float* scale, const float* bias, int8_t* y_i8, float* y_f32) {
     EXHIP_REQUIRE(ctx && d && x && wp && scale && (y_i8 || y_f32), "exhip_conv2d_i8_maxpool2x2: bad argument");
-    if (d->sh != d->sw || d->post_op || d->post_bn_a || d->exact_k || d->act > 1) return EXHIP_ERR_UNSUPPORTED;
+    if (d->sh != d->sw || d->post_op || d->post_bn_a || d->post_bn_b || d->exact_k || d->act > 1) return EXHIP_ERR_UNSUPPORTED;
     Plan pl;
-    const int rc = make_plan(d, EXHIP_I8, &pl);
+    int rc = make_plan(d, EXHIP_I8, &pl);
+    if (!rc) rc = check_operands(d, true, x, wp, scale, bias);
     if (rc) return rc;
-    EXHIP_REQUIRE(pool_oh > 0 && pool_ow > 0 && 2 * pool_oh <= pl.OH && 2 * pool_ow <= pl.OW, "conv+pool: pooled size %dx%d does not fit a %dx%d convolution output",
+    EXHIP_REQUIRE(pool_oh > 0 && pool_ow > 0 && pool_oh <= pl.OH / 2 && pool_ow <= pl.OW / 2, "conv+pool: pooled size %dx%d does not fit a %dx%d convolution output",
                   pool_oh, pool_ow, pl.OH, pl.OW);
     if (pl.packed || pl.KWe != d->kw) return EXHIP_ERR_UNSUPPORTED;
     exhip_pw_geom g = {};
@@ -2066,11 +2074,12 @@ extern "C" int exhip_conv2d_i8_maxpool2x2(exhip_ctx* ctx, const exhip_conv_desc*
     return exhip_conv1x1_i8_pw(ctx, g, x, wp, scale, bias, nullptr, y_i8, y_f32, &t);
 }
 
-// The geometry of a first layer that the kernel on NCHW planes may take.
-static int stem_geometry(const exhip_conv_desc* d, int dt, exhip_pw_geom* g, exhip_pw_taps* t) {
-    if (d->c_stride != 4 || d->c > 4 || d->sh != d->sw) return EXHIP_ERR_UNSUPPORTED;
+// The geometry of a first layer that the kernel on NCHW planes may take, its operands checked.
+static int stem_geometry(const exhip_conv_desc* d, int dt, const void* wp, const float* scale, const float* bias, exhip_pw_geom* g, exhip_pw_taps* t) {
+    if (d->c_stride != 4 || d->c > 4 || d->sh != d->sw || d->post_bn_a || d->post_bn_b || d->exact_k) return EXHIP_ERR_UNSUPPORTED;
     Plan pl;
-    const int rc = make_plan(d, dt, &pl);
+    int rc = make_plan(d, dt, &pl);
+    if (!rc) rc = check_operands(d, true, nullptr, wp, scale, bias);
     if (rc) return rc;
     EXHIP_REQUIRE((d->post_op >= 0 && d->post_op <= 1 + EXHIP_UNARY_CLIP && d->post_op != 1 + EXHIP_UNARY_SIGMOID) ||
                       (d->post_op == EXHIP_POST_PRELU && d->post_slope),
@@ -2089,7 +2098,7 @@ extern "C" int exhip_stem_f16(exhip_ctx* ctx, const exhip_conv_desc* d, const ui
     EXHIP_REQUIRE(ctx && d && x_nchw && wp && y && !mean == !factor, "exhip_stem_f16: bad argument");
     exhip_pw_geom g;
     exhip_pw_taps t;
-    const int rc = stem_geometry(d, EXHIP_F16, &g, &t);
+    const int rc = stem_geometry(d, EXHIP_F16, wp, nullptr, bias, &g, &t);
     return rc ? rc : exhip_conv_f16_stem(ctx, g, t, d->c, x_nchw, mean, factor, wp, bias, y);
 }
 
@@ -2098,6 +2107,6 @@ extern "C" int exhip_stem_i8(exhip_ctx* ctx, const exhip_conv_desc* d, const flo
     EXHIP_REQUIRE(ctx && d && x_nchw && wp && scale && (y_i8 || y_f32) && !mean == !factor, "exhip_stem_i8: bad argument");
     exhip_pw_geom g;
     exhip_pw_taps t;
-    const int rc = stem_geometry(d, EXHIP_I8, &g, &t);
+    const int rc = stem_geometry(d, EXHIP_I8, wp, scale, bias, &g, &t);
     return rc ? rc : exhip_conv_i8_stem(ctx, g, t, d->c, x_nchw, mean, factor, fs_in, wp, scale, bias, y_i8, y_f32);
 }

@@ -232,7 +232,8 @@ int exhip_conv2d_i8_maxpool2x2(exhip_ctx* ctx, const exhip_conv_desc* d, int poo
 
 /* The first layer of an fp16 network on its half NCHW input: exhip_conv2d_f16 of at most four channels (c_stride 4, its packed weights) with the NHWC
  * result, without the conversion in front; with the Input layer (operation_input.cpp, (x - mean[c]) * factor[c] rounded to half) where mean and factor
- * are given, both or neither. EXHIP_ERR_UNSUPPORTED, with nothing launched, where the layers run by themselves. */
+ * are given, both or neither. The planes may begin anywhere; the other operands as for exhip_conv2d_f16. EXHIP_ERR_UNSUPPORTED, with nothing
+ * launched, where the layers run by themselves. */
 int exhip_stem_f16(exhip_ctx* ctx, const exhip_conv_desc* d, const uint16_t* x_nchw, const float* mean, const float* factor, const void* w_packed,
                    const float* bias, uint16_t* y_nhwc);
 /* The same of an int8 network on its float32 NCHW input: Input layer (or NULLs), quantizer with fs_in (src/Excalibur/operation_general_conv.cpp:584-720) and

@@ -78,3 +78,69 @@ def test_stream_slots_and_options_need_no_gpu():
     with pytest.raises(ValueError):
         pipeline.set_option("no_such_option", 1)
     pipeline.set_option("share_gpu", 0)
+
+
+ERR_ARG = 10001
+
+
+def _fused_entry(name, change):
+    """The status of a fused entry point for operands that are addresses only, in a process without a GPU: a call that its checks let through ends
+    in the runtime's own error."""
+    from excalibur_amd import hip
+    L = hip.lib()
+    ctx = ctypes.create_string_buffer(4096)
+    at = {n: 0x10000 * (i + 1) for i, n in enumerate(("x", "wp", "scale", "bias", "mean", "factor", "y", "y_f32"))}
+    shape = dict(c=3, c_stride=4, h=16, w=16, k=64, k_stride=64, pool=(4, 4)) if name != "exhip_conv2d_i8_maxpool2x2" else \
+        dict(c=64, c_stride=64, h=64, w=64, k=64, k_stride=64, pool=(32, 32))
+    fields = {}
+    for key, value in change.items():
+        if key in at: at[key] = at[key] + value if value else 0
+        elif key in shape: shape[key] = value
+        else: fields[key] = value
+    d = hip.Ctx.conv_desc(1, shape["c"], shape["h"], shape["w"], shape["k"], 3, 1, 1, c_stride=shape["c_stride"], k_stride=shape["k_stride"], fs_out=1.0)
+    for key, value in fields.items():
+        setattr(d, key, value)
+    p = {n: ctypes.c_void_p(v) for n, v in at.items()}
+    c, d = ctypes.cast(ctx, ctypes.c_void_p), ctypes.byref(d)
+    if name == "exhip_stem_f16":
+        return L.exhip_stem_f16(c, d, p["x"], p["mean"], p["factor"], p["wp"], p["bias"], p["y"])
+    if name == "exhip_stem_i8":
+        return L.exhip_stem_i8(c, d, p["x"], p["mean"], p["factor"], ctypes.c_float(1.0), p["wp"], p["scale"], p["bias"], p["y"], p["y_f32"])
+    return L.exhip_conv2d_i8_maxpool2x2(c, d, *shape["pool"], p["x"], p["wp"], p["scale"], p["bias"], p["y"], p["y_f32"])
+
+
+@pytest.mark.parametrize("name,change,says", [
+    ("exhip_stem_f16", dict(k_stride=32), b"k_stride 32 < k 64"),
+    ("exhip_stem_f16", dict(wp=4), b"16-byte aligned"),
+    ("exhip_stem_f16", dict(bias=4), b"16-byte aligned"),
+    ("exhip_stem_i8", dict(k_stride=32), b"k_stride 32 < k 64"),
+    ("exhip_stem_i8", dict(wp=8), b"16-byte aligned"),
+    ("exhip_stem_i8", dict(scale=4), b"16-byte aligned"),
+    ("exhip_stem_i8", dict(bias=12), b"16-byte aligned"),
+    ("exhip_conv2d_i8_maxpool2x2", dict(k_stride=32), b"k_stride 32 < k 64"),
+    ("exhip_conv2d_i8_maxpool2x2", dict(x=8), b"16-byte aligned"),
+    ("exhip_conv2d_i8_maxpool2x2", dict(wp=4), b"16-byte aligned"),
+    ("exhip_conv2d_i8_maxpool2x2", dict(scale=4), b"16-byte aligned"),
+    ("exhip_conv2d_i8_maxpool2x2", dict(bias=4), b"16-byte aligned"),
+    ("exhip_conv2d_i8_maxpool2x2", dict(pool=(1 << 30, 32)), b"does not fit"),
+])
+def test_fused_first_layers_and_pooling_check_their_operands(name, change, says):
+    """What exhip_conv2d_* refuses, the entry points that run the same layers in one launch refuse with the same error, before any launch."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("the operands are no memory of a GPU")
+    assert _fused_entry(name, {}) not in (0, ERR_ARG)   # past the checks: no GPU to launch on
+    assert _fused_entry(name, change) == ERR_ARG
+    from excalibur_amd import hip
+    assert says in hip.lib().exhip_last_error()
+
+
+@pytest.mark.parametrize("name", ["exhip_stem_f16", "exhip_stem_i8", "exhip_conv2d_i8_maxpool2x2"])
+@pytest.mark.parametrize("change", [dict(exact_k=1), dict(post_bn_a=0x900000, post_bn_b=0xa00000), dict(post_bn_b=0xa00000)], ids=["exact", "bn", "half_bn"])
+def test_fused_first_layers_and_pooling_leave_joined_layers_alone(name, change):
+    """A BatchNorm in the epilogue and writes limited to the layer's channels are the pointwise layers'."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("the operands are no memory of a GPU")
+    from excalibur_amd import hip
+    assert _fused_entry(name, change) == hip.ERR_UNSUPPORTED

@@ -102,6 +102,29 @@ def test_int8_stem_equals_the_layers(ctx, n, c, h, w, k, kw, stride, pad, post, 
     assert all(np.ptp(want[t].download()[..., :k].astype(np.float32)) > .5 for t in forms)
 
 
+@pytest.mark.parametrize("width", [48, 41])
+def test_planes_that_begin_anywhere(ctx, width):
+    """Planes off 16 bytes are read value by value, whatever their width: the results of the aligned ones."""
+    r = np.random.default_rng(width)
+    for values in (r.normal(0, 1, (2, 3, 21, width)).astype(np.float16).view(np.uint16), r.normal(0, 1, (2, 3, 21, width)).astype(np.float32)):
+        half = values.dtype == np.uint16
+        d = ctx.conv_desc(2, 3, 21, width, 64, 3, 2, 1, 1, c_stride=4, k_stride=64, fs_out=0.0 if half else 40.0)
+        shape = (2,) + ctx.conv_out_hw(d) + (64,)
+        w = r.integers(-127, 128, (64, 3, 3, 3), dtype=np.int8)
+        wp = ctx.pack_conv_weights(d, hip.F16 if half else hip.I8, (w / np.float16(400)).astype(np.float16).view(np.uint16) if half else w)
+        scale, bias = ctx.array(r.uniform(.5, 1.5, 64).astype(np.float32) / 24000), ctx.array(r.normal(0, .3, 64).astype(np.float32))
+        got = []
+        for shift in (0, 1, 3):
+            x = ctx.array(np.concatenate([np.zeros(shift, values.dtype), values.reshape(-1)]))
+            x = x.at(shift * values.itemsize)
+            y = ctx.empty(shape, np.uint16 if half else np.int8).zero()
+            rc = ctx.stem_f16(d, x, None, None, wp, bias, y) if half else ctx.stem_i8(d, x, None, None, 60.0, wp, scale, bias, y)
+            assert rc == 0
+            got.append(y.download())
+        assert np.count_nonzero(got[0]) > got[0].size // 4
+        assert all(np.array_equal(g, got[0]) for g in got)
+
+
 def test_what_the_stem_leaves_to_the_layers(ctx):
     x, w, y = ctx.empty((1, 3, 16, 16), np.uint16).zero(), ctx.empty((64 * 1024,), np.uint8).zero(), ctx.empty((1, 16, 16, 64), np.uint16)
     for c, kernel, c_stride in ((3, 1, 4), (5, 3, 16)):
