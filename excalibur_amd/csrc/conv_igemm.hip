@@ -1732,7 +1732,7 @@ int run_conv(exhip_ctx* ctx, const exhip_conv_desc* d, ConvParams p, const PoolS
         const int min_chunks_ = (3 + pl.n_rg - 1) / pl.n_rg;
         const bool would_split = g_exhip_options.force_splits != 1 && pl.n_chunks / min_chunks_ >= 2 && kCUs / tiles >= 2;
         const bool deep = !pl.packed && exhip_pw_splits_f16((long long)d->n * pl.OH * pl.OW, p.cstride_b, d->k, d->k_stride,
-                                                             pl.n_chunks * d->kh * d->kw * (pl.chunk_b / 32), d->sh, d->post_op);
+                                                             pl.n_chunks * d->kh * d->kw * (pl.chunk_b / 32), d->sh);
         if ((tiles >= 16 || !would_split) && g_exhip_options.force_splits <= 1 && !deep) {
             if (!pl.packed && !pool && d->kh == 3 && d->kw == 3 && d->sh == 1 && d->sw == 1 && pl.variant == 0 && pl.chunk_b == 64 &&
                 pl.RS == 1 && p.cstride_b % 64 == 0 && d->k % 64 == 0 && d->k_stride == d->k && d->act <= 1 && p.y_q && !p.y_nchw_h && !p.y_nchw &&

@@ -58,5 +58,5 @@ int exhip_conv_i8_stem(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_ta
 int exhip_conv1x1_i8_pw(exhip_ctx* ctx, const exhip_pw_geom& g, const int8_t* x, const void* wp, const float* scale, const float* bias,
                         const float* residual, int8_t* y_i8, float* y_f32, const exhip_pw_taps* taps = nullptr);
 // Whether that kernel takes an fp16 layer with a filter of this many output pixels, input bytes per pixel, channels and 32-byte k-steps
-// (and stride, activation layer behind it) in its split form (several waves to a tile), which is then faster than any other kernel for it.
-bool exhip_pw_splits_f16(long long pixels, int c_bytes, int k, int k_stride, int n_ksteps, int stride, int post_op);
+// (and stride) in its split form (several waves to a tile), which is then faster than any other kernel for it.
+bool exhip_pw_splits_f16(long long pixels, int c_bytes, int k, int k_stride, int n_ksteps, int stride);

@@ -1376,12 +1376,16 @@ int launch(exhip_ctx* ctx, PwParams& p, int kblocks) {
     if (items >= (1ll << 31) - 4) return EXHIP_ERR_UNSUPPORTED;
     p.items = (unsigned)items;
     exhip_host_divisor(p.ch_groups, &p.groups_magic, &p.groups_shift);
-    if constexpr (MT + NT > 3) return go<DT, MT, NT, 2, TAPS, EpAny>(ctx, p);
-    else if (pairs) return pick_epilogue<DT, MT, NT, 104, TAPS>(ctx, p);
-    // A launch of at most two waves per SIMD is as long as one wave's chain of load round trips: sixteen k-steps in flight
-    // where there are more than eight. Larger ones hide each other's round trips and want the registers for more waves.
-    else if (MT == 2 && items <= 2048 && p.n_ksteps > 8) return pick_epilogue<DT, MT, NT, 8, TAPS>(ctx, p);
-    else return pick_epilogue<DT, MT, NT, 4, TAPS>(ctx, p);
+    if constexpr (MT + NT > 3) {
+        return go<DT, MT, NT, 2, TAPS, EpAny>(ctx, p);
+    } else {
+        if (pairs) return pick_epilogue<DT, MT, NT, 104, TAPS>(ctx, p);
+        // A launch of at most two waves per SIMD is as long as one wave's chain of load round trips: sixteen k-steps in flight
+        // where there are more than eight. Larger ones hide each other's round trips and want the registers for more waves.
+        if constexpr (MT == 2)
+            if (items <= 2048 && p.n_ksteps > 8) return pick_epilogue<DT, MT, NT, 8, TAPS>(ctx, p);
+        return pick_epilogue<DT, MT, NT, 4, TAPS>(ctx, p);
+    }
 }
 
 // The k-step where wave i of a split tile begins.
@@ -1653,8 +1657,8 @@ int exhip_conv_i8_stem(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_ta
     return run_stem<EXHIP_I8>(ctx, g, t, channels, p);
 }
 
-bool exhip_pw_splits_f16(long long pixels, int c_bytes, int k, int k_stride, int n_ksteps, int stride, int post_op) {
+bool exhip_pw_splits_f16(long long pixels, int c_bytes, int k, int k_stride, int n_ksteps, int stride) {
     exhip_pw_geom g = {};
-    g.pixels = pixels; g.c_bytes = c_bytes; g.post_op = post_op;
+    g.pixels = pixels; g.c_bytes = c_bytes;
     return g_exhip_options.pw != 0 && g_exhip_options.direct != 0 && split_wins(EXHIP_F16, g, (std::max(k, k_stride) + 31) / 32, n_ksteps, true, stride);
 }
