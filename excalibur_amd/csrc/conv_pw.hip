@@ -1,6 +1,6 @@
 // conv1x1_pw_kernel: the pointwise (1x1, stride 1, no padding) convolution on half or int8 NHWC tensors, y[pixel][k] = sum_c x[pixel][c]
-// * w[k][c]; its tapped form (TAPS) for layers with a filter, a stride or padding; conv_pw_split_kernel, several waves to a tile; and
-// dw_pw_kernel, a depthwise 3x3 layer in front.
+// * w[k][c]; its tapped form (TAPS) for layers with a filter, a stride or padding; conv_pw_split_kernel, several waves to a tile;
+// dw_pw_kernel, a depthwise 3x3 layer in front; and stem_planes_kernel, a network's first layer from its planes.
 //
 // A pointwise layer of a detection or mobile network moves a few tens of MB for a few GFLOP: what it costs is the
 // length of one group's chain from launch to last store, and the memory system's rate. So no operand is staged: a wave
@@ -1496,7 +1496,7 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
     p.chunk_end_b = t.chunk_b - t.kh * t.in_w * g.c_bytes;
     if (split) return launch_split<DT, true>(ctx, p, kblocks);
     if (kblocks == 1) return launch<DT, 1, 2, true>(ctx, p, kblocks);
-    // (the 64 x 64 tile has the epilogue without pooling only: it would number the pooled map's pixels as the convolution's, four times too many)
+    // (the 64 x 64 tile has no pooled epilogue: its kernel would take the convolution's pixels, four times as many, for the pooled map's)
     const long long waves64 = ((g.pixels + 63) / 64) * ((kblocks + 1) / 2);
     if (g.pool || waves64 < 2048 || small_tile<DT>()) return launch<DT, 2, 1, true>(ctx, p, kblocks);
     return launch<DT, 2, 2, true>(ctx, p, kblocks);
@@ -1614,8 +1614,8 @@ int run_pw(exhip_ctx* ctx, const exhip_pw_geom& g, PwParams& p, int es, bool has
     const int kblocks = std::min(g.slabs * g.slab_blocks, (out_channels + 31) / 32);
     if constexpr (DT == EXHIP_F16)
         if (dw) return run_depthwise(ctx, *dw, p, kblocks, split_wins(DT, g, kblocks, (int)n_ksteps, false, 1));
-    // 64 x 64 per wave unless that leaves SIMDs without a wave: then 64 channels x 32 pixels; a lone 32-channel block
-    // takes 128 pixels per wave
+    // 32 pixels x 64 channels a wave, 64 x 64 only where the option asks for it and no SIMD is left without a wave; a lone 32-channel
+    // block takes 64 pixels
     if (split_wins(DT, g, kblocks, (int)n_ksteps, false, 1)) return launch_split<DT, false>(ctx, p, kblocks);
     if (kblocks == 1) return launch<DT, 1, 2>(ctx, p, kblocks);
     const long long waves64 = ((g.pixels + 63) / 64) * ((kblocks + 1) / 2);
