@@ -132,9 +132,11 @@ def network_table(iters=10, only=None):
         ms = (time.perf_counter() - t0) / iters * 1e3
         from excalibur_amd import topologies
         from excalibur_amd.modelfile import parse_topology
-        layers = parse_topology(net.topology())   # a plan stores a blob or two between the layers, the per-layer executor most of them
+        # fp16 has no plan; a float plan stores a blob or two between the layers, the per-layer executor most of them
+        layers = parse_topology(net.topology())
         inner = {t for l in layers for t in l.tops} & {b for l in layers for b in l.bottoms}
-        executor = "int8 graph plan" if p.fused else "per-layer" if 2 * sum(p.stored(b) for b in inner) > len(inner) else "float plan"
+        planned = pipe_dtype == "f32" and 2 * sum(p.stored(b) for b in inner) <= len(inner)
+        executor = "int8 graph plan" if p.fused else "float plan" if planned else "per-layer"
         p.close()
         gop = topologies.algorithmic_gop(net.topology(), x.shape[1:]) * x.shape[0]   # of the whole batch
         peak = {"f32": PEAK_F32_TFLOPS, "f16": PEAK_F16_TFLOPS, "int8": PEAK_INT8_TOPS}[dtype]
