@@ -202,7 +202,7 @@ __global__ __launch_bounds__(kBlock) void nhwc_to_nchw_tiled_kernel(const Tin* _
         for (int v = tid; v < 64 * VPP; v += kBlock) {
             const int pp = v / VPP, part = v % VPP;
             const int cb = c0 + part * VE;
-            if (p0 + pp < HW && cb < c_stride) {
+            if (p0 + pp < HW && cb < C) {  // (x may be a slice of a wider tensor: behind its last pixel's channels the tensor may end)
                 const v4i raw = *reinterpret_cast<const v4i*>(x + ((size_t)n * HW + p0 + pp) * c_stride + cb);
                 if constexpr (sizeof(Tin) == 4) {
                     const v4f f = __builtin_bit_cast(v4f, raw);
