@@ -125,7 +125,8 @@ typedef struct exhip_conv_desc {
     int pt, pb, pl, pr;         /* zero padding top/bottom/left/right */
     int act;                    /* fused activation applied to conv + bias */
     int c_stride;               /* channel stride of the NHWC input, in elements */
-    int k_stride;               /* channel stride of the NHWC outputs, in elements (>= k) */
+    int k_stride;               /* channel stride of the NHWC outputs, in elements (>= k). Pad channels are written as zeros: all of them by
+                                 * float32 layers, by int8 and half ones those below the next multiple of 64 at least */
     int post_relu;              /* ReLU applied after the residual add (0/1) */
     float fs_out;               /* scale of the optional int8 output: q = sat8(trunc(v*fs_out +- 0.5)) */
     int post_op;                /* 0, or 1 + EXHIP_UNARY_*: the activation layer behind the convolution, applied to the
