@@ -1858,7 +1858,7 @@ bool pipeline<float>::impl::build_graph_plan(const tensor_ptr& input, const std:
 //   * Convolution [-> activation layer / ReLU / PReLU] [-> add] [-> ReLU / activation layer] is one launch, a depthwise 3x3
 //     layer with its PReLU or ReLU too; a nearest Interp in front of the add (a feature pyramid's top-down path) is read through;
 //   * Concat costs nothing: its inputs' producers write their channels of the joined tensor. BatchNorm and the activation
-//     layer behind it run in the producers' epilogues where those are plain convolutions, else as one launch over the result;
+//     layer behind it run in the producers' epilogues where those are plain convolutions, else as one launch from there to another tensor;
 //   * a 2x2 stride-2 Deconvolution [-> BatchNorm] [-> ReLU] is four 1x1 layers in one launch;
 //   * Input and YoloV5Focus make the NHWC tensor the first convolution reads; a detection head's Reshape -> Transpose is how its
 //     convolution stores; anything behind the last planned layer runs as a layer on the NCHW results (the tail).
@@ -2397,10 +2397,12 @@ bool pipeline<float>::impl::build_float_plan(const tensor_ptr& input, const std:
                 if (out.parent >= 0 || total % 4 != 0) return refuse(__LINE__);
                 for (int ch : channels)
                     if (ch % 4 != 0) return refuse(__LINE__);
-                if (nd.join == node::placed) {  // the joined tensor is there: one pass over it
+                const size_t pixels = static_cast<size_t>(out.n) * out.h * out.w;
+                if (nd.join == node::placed) {  // the joined tensor is there: one pass over it, into another, for its slices may have more readers
                     ptrs = {out.p};
                     channels = {total};
                     strides = {out.cs};
+                    out.p = alloc(pixels * out.cs);
                 }
                 const float *bn_a = nullptr, *bn_b = nullptr;
                 if (nd.bn >= 0) {
@@ -2415,7 +2417,6 @@ bool pipeline<float>::impl::build_float_plan(const tensor_ptr& input, const std:
                     auto* u = static_cast<operation_unary<float>*>(operations_[nd.unary].get());
                     uop = u->op_; alpha = u->alpha_; beta = u->beta_;
                 }
-                const size_t pixels = static_cast<size_t>(out.n) * out.h * out.w;
                 float* y = out.p;
                 const int cs = out.cs, n_in = static_cast<int>(ptrs.size());
                 plan->launches.push_back([=]() {

@@ -196,3 +196,55 @@ def test_float_plan_results_held_across_forwards(pair):
         assert np.array_equal(planned.get(o), want[3][o])
         for back in (1, 2, 3):
             assert np.array_equal(planned.get_kept(back, o), want[3 - back][o]), (back, o)
+
+
+@pytest.mark.parametrize("activation", [True, False], ids=["activation", "batchnorm"])
+@pytest.mark.parametrize("reader", ["convolution", "interp", "concat", "larger pool", "result"])
+def test_a_concats_inputs_keep_their_values_behind_its_batchnorm(tmp_path, reader, activation):
+    """The producers of a Concat that is no plain convolutions' write into the joined tensor; the BatchNorm and activation behind it leave
+    those values to their other readers, which run later."""
+    r = np.random.default_rng(91)
+    lines, blobs = [], []
+
+    def conv(bottom, top, cin, k, kernel=1):
+        w = r.normal(0, np.sqrt(2.0 / (cin * kernel * kernel)), (k, cin, kernel, kernel)).astype(np.float32)
+        lines.append(mf.conv_line("Convolution", top + "_l", bottom, top, k, kernel, 1, kernel // 2, True, w.size, 1))
+        blobs.append(mf.conv_blob_f32(w, r.normal(0, 0.5, (k,)).astype(np.float32)))
+
+    def joined(bottoms, top, c):
+        lines.append(f"Concat {top}_l 2 1 {' '.join(bottoms)} {top}k 0=-1")
+        lines.append(f"BatchNorm {top}_bn 1 1 {top}k {top if not activation else top + 'b'} 0={c}")
+        blobs.append(mf.floats_blob(r.uniform(.5, 1.5, c), r.normal(0, .5, c), r.uniform(.5, 2, c), r.normal(0, .5, c)))
+        if activation:
+            lines.append(f"LeakyRelu {top}_a 1 1 {top}b {top} 0=1.000000e-01")
+
+    conv("data", "c0", 3, 16, 3)
+    lines.append("HardSwish hs 1 1 c0 a0 0=1.666667e-01 1=5.000000e-01")
+    lines.append("Split sp0 1 3 a0 a0x a0y a0z")
+    lines.append(mf.pool_line("p1_l", "a0x", "p1", 0, 3, 1, 1))
+    lines.append("Split sp1 1 2 p1 p1x p1y")
+    joined(["p1x", "a0y"], "s2", 32)
+    if reader == "larger pool":   # reads the smaller pool's result in place of its own input
+        lines.append(mf.pool_line("p5_l", "a0z", "late", 0, 5, 1, 2))
+    elif reader == "convolution":
+        conv("p1y", "late", 16, 24, 3)
+    elif reader == "interp":
+        lines.append("Interp up 1 1 p1y late 0=1 1=2.000000e+00 2=2.000000e+00")
+    elif reader == "concat":
+        joined(["a0z", "p1y"], "late", 32)
+    conv("s2", "c3", 32, 16)
+    outputs = ["c3", "p1y" if reader == "result" else "late"]
+    path = str(tmp_path / "net.racy")
+    mf.write_model(path, blobs)
+    planned, plain = (xp.Pipeline(mf.topology(lines, "joined"), path, 0, fusion=on) for on in (True, False))
+    for seed in (1, 2):
+        x = np.random.default_rng(seed).normal(0, 1, (2, 3, 12, 20)).astype(np.float32)
+        planned.forward(x)
+        plain.forward(x)
+        assert not planned.stored("c0") and plain.stored("c0")
+        for o in outputs:
+            got, want = planned.get(o), plain.get(o)
+            assert np.ptp(want) > .5
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), o
+    planned.close()
+    plain.close()
