@@ -21,6 +21,8 @@ extern "C" const char* exhip_last_error(void) { return g_err; }
 exhip_options g_exhip_options;
 unsigned g_exhip_options_version = 0;
 
+extern "C" unsigned exhip_options_version(void) { return g_exhip_options_version; }
+
 extern "C" int exhip_set_option(const char* name, int value) {
     EXHIP_REQUIRE(name, "exhip_set_option: NULL name");
     exhip_options& o = g_exhip_options;

@@ -681,6 +681,7 @@ private:
     struct fused_plan;
     std::shared_ptr<fused_plan> plan_;
     bool fused_unsupported_ = false;
+    unsigned options_version_ = 0;  // of the library's options that plan_ was built, or refused, under
 
     std::string name_ = "Unknown Pipeleine Name";
     int device_ = -1;
@@ -2523,7 +2524,13 @@ bool pipeline<float>::impl::build_float_plan(const tensor_ptr& input, const std:
 
 template <>
 bool pipeline<float>::impl::try_fused(const tensor_ptr& input, blob_map* results) {
-    if (!fusion_ || fused_unsupported_) return false;
+    if (!fusion_) return false;
+    if (const unsigned version = exhip_options_version(); version != options_version_) {
+        options_version_ = version;  // other options: the launches that were tried under the old ones may not take their layers any more
+        plan_.reset();
+        fused_unsupported_ = false;
+    }
+    if (fused_unsupported_) return false;
     const std::vector<int> shape = input->data_shape();
     if (!plan_ || plan_->in_shape != shape) {
         plan_.reset();

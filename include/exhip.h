@@ -76,6 +76,7 @@ const char* exhip_last_error(void);
  * sums then run in another order).
  * Process-wide; packed weights depend on the first three, so set them before packing. */
 int exhip_set_option(const char* name, int value);
+unsigned exhip_options_version(void); /* counts the calls above: plans made under other options are made again */
 int exhip_device_name(exhip_ctx* ctx, char* buf, size_t len);
 
 /* HIP events on the context's stream, for timing kernels where they are launched
