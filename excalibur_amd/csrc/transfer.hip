@@ -8,10 +8,11 @@
 // reads or writes the pinned memory itself (no copy engine, no hand-over between queues: 15 instead of 19 us for 75 KB with
 // the kernel behind it; 6 instead of 11 us for a result the host polls for instead of waiting on the stream).
 //
-// Uploads of every size are kernels that read the pinned memory: the copy engine leaves the link idle for some 15 us between two
+// Uploads of every size from pageable memory to a destination on 16 bytes are kernels that read the pinned memory: the copy engine leaves the link idle for some 15 us between two
 // copies, a kernel for 3, so an upload can begin with a small piece and needs no hand-over to the kernels behind it (16 groups: 54
 // GB/s in launches of 4 MiB, 48 in 1 MiB; the engine 50 and 38; 64 groups 53 and 41). Until everything is there: 4.9 MB 147 -> 130
-// us, 19 MB 480 -> 416, 79 MB 1755 -> 1562.
+// us, 19 MB 480 -> 416, 79 MB 1755 -> 1562. Two kinds stay with the engine, in whole chunks: sources in the pinned pool of results, and above
+// 256 KiB destinations off 16 bytes, which a kernel would write byte by byte (4.9 MB 138 us, 148 in pieces that grow; 20 MB 465 and 480; 83 MB 1814 and 1800).
 #include <string.h>
 
 #include <atomic>
@@ -311,11 +312,11 @@ extern "C" int exhip_upload(exhip_ctx* ctx, void* dst, const void* src, size_t b
     staging_loan loan(ctx->up, ctx->stream);
     EXHIP_REQUIRE(loan.staging, "exhip_upload: no host memory");
     exhip_staging& s = *loan.staging;
-    const bool small = bytes <= kUploadKernel;
+    const bool small = bytes <= kUploadKernel, kernels = small || is_wide(to, to);
     copy_crew::session crew(bytes >= 2 * kStep);
     for (size_t done = 0; bytes;) {
-        // as much again as is on its way: the link starts early and later launches are long
-        const size_t step = done < kStep ? kStep : done < kChunk ? done : kChunk, now = bytes < step ? bytes : step;
+        // kernels: as much again as is on its way, so that the link starts early and later launches are long
+        const size_t step = !kernels ? kChunk : done < kStep ? kStep : done < kChunk ? done : kChunk, now = bytes < step ? bytes : step;
         if (s.at < 0 || s.used + now > (small ? kSmallRing : kChunk)) {
             const int rc = next_chunk(ctx, s);
             if (rc == EXHIP_ERR_UNSUPPORTED) {  // no pinned memory left: the runtime's own way
@@ -329,7 +330,7 @@ extern "C" int exhip_upload(exhip_ctx* ctx, void* dst, const void* src, size_t b
         }
         char* stage = static_cast<char*>(s.chunk[s.at]) + s.used;
         crew.copy(stage, from, now);
-        if (small || is_wide(stage, to)) {
+        if (kernels) {
             const unsigned groups = (unsigned)((now + 4095) / 4096), most = small ? 64 : kUploadGroups;
             upload_kernel<<<groups < most ? groups : most, 256, 0, ctx->stream>>>(stage, to, (unsigned)now, is_wide(stage, to));
             EXHIP_LAUNCH_CHECK();

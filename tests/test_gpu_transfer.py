@@ -38,7 +38,7 @@ def test_bytes_arrive_in_both_directions(ctx, size, offset):
 @pytest.mark.parametrize("size", [512 * KB, 512 * KB + 16, MB + 1, 2 * MB - 1, 4 * MB + 16, 8 * MB + 512 * KB + 7, 12 * MB])
 @pytest.mark.parametrize("offset", [0, 16, 8])
 def test_uploads_in_steps(ctx, size, offset):
-    """An upload's pieces: half a megabyte twice, then as much again as is on its way up to a chunk; by kernel or (8) by the engine."""
+    """An upload's pieces: half a megabyte twice, then as much again as is on its way up to a chunk, by kernel; or (8) whole chunks by the engine."""
     test_bytes_arrive_in_both_directions(ctx, size, offset)
 
 
