@@ -72,7 +72,8 @@ const char* exhip_last_error(void);
  * that many output rows a group of the ones without pooling): every form computes
  * the same values. "pw_split" chooses that kernel's split form (1 by its rule, 2 wherever it can run, 0 never; fp16 sums then run
  * in another order). "dw_pw" chooses the depthwise + pointwise fp16 pairs that exhip_dw_pw_f16 takes (1 by its rule, 2 wherever it can
- * run, a power of two from 4 to 256 so with that many pixels a group, 0 never; the same values). "f32_tile" pins the float32 convolution's wave tile and split (0 = its rule, n = the n-th of its list;
+ * run, a power of two from 4 to 256 so with that many pixels a group where 40 KiB hold their depthwise results, 2 c + 16 bytes each, 0 never; the same
+ * values). "f32_tile" pins the float32 convolution's wave tile and split (0 = its rule, n = the n-th of its list;
  * sums then run in another order).
  * Process-wide; packed weights depend on the first three, so set them before packing. */
 int exhip_set_option(const char* name, int value);

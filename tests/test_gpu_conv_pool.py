@@ -74,8 +74,7 @@ def pooled_and_the_two_layers(ctx, n, c, h, w, k, kernel, stride, pad, results, 
 @pytest.mark.parametrize("results", ["int8", "float", "both"])
 @pytest.mark.parametrize("n,c,h,w,k,kernel,stride,pad", SHAPES, ids=[f"s{i}" for i in range(len(SHAPES))])
 def test_pooled_equals_the_two_layers(ctx, n, c, h, w, k, kernel, stride, pad, results, act, post_relu):
-    rc = pooled_and_the_two_layers(ctx, n, c, h, w, k, kernel, stride, pad, results, act, post_relu, direct=2)
-    assert rc in ((0, hip.ERR_UNSUPPORTED) if kernel == 1 else (0,))   # pointwise layers have no taps to place: the two layers may run by themselves
+    assert pooled_and_the_two_layers(ctx, n, c, h, w, k, kernel, stride, pad, results, act, post_relu, direct=2) == 0
 
 
 # waves of 64 pixels x 64 channels (2048 and more take the larger wave tile where option pw_tile asks for it): 2048 exactly, one less, a layer with an

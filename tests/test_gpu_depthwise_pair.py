@@ -119,7 +119,8 @@ def test_every_option_of_the_two_layers(ctx, pairs, stride, pad, hw, act, with_b
     assert np.isfinite(want.view(np.float16)).all() and np.ptp(want.view(np.float16).astype(np.float32)) > .5
 
 
-# pixels of a group: fewer than a strip's round and than a block, several blocks, more than the map has
+# pixels of a group: fewer than a strip's round and than a block, several blocks, more than the map has. Up to 32 for 512 channels and 128 for 96: beyond
+# the 40 KiB that a group's depthwise results may take, the option leaves the number to the rule, whose launch must then come out
 @pytest.mark.parametrize("pixels", [4, 8, 16, 32, 64, 128, 256])
 @pytest.mark.parametrize("front", [0, 2, 4, 5, 6])
 @pytest.mark.parametrize("c,behind", [(16, 0), (96, 4), (512, 1)])
