@@ -91,8 +91,10 @@ public:
     // fp16: this layer, a pointwise one, with the Reshape of its channels into groups and the Transpose of the last two axes behind it (a detection
     // head) as one launch; `tops` are the Transpose layer's. False, with nothing done, where the three run by themselves.
     bool forward_head(const operation_reshape<Dtype>& reshape, const tensor_list<unsigned short>& bottoms, tensor_list<unsigned short>& tops);
-    // fp16: an NCHW result of NHWC pixels is made from NHWC rows, so that a head's layers by themselves run the kernel, and add in the order, of the one launch
-    void set_through_rows() { through_rows_ = true; }
+    // Whether that launch is for these layers and pixels; the layers by themselves then make the NCHW result from NHWC rows, so that they run the
+    // kernel, and add in the order, of the one launch. (Others do not: 128 -> 255 3x3 at 16 x 80 x 80 takes 80 us straight to NCHW, 123 through rows.)
+    bool head_form(const operation_reshape<Dtype>& reshape, const tensor_list<unsigned short>& bottoms, exhip_conv_desc* d, std::vector<int>* to) const;
+    void set_through_rows(bool on) { through_rows_ = on; }
     // int8 layers on the MFMA kernel. The next forward calls also write the int8 NHWC form of the output that a reader
     // quantizing with `fs` into `stride` channels per pixel would make of it (attached to the top blob as its
     // `quantized` copy), and with `only` leave the float data unwritten; fs = 0 switches it off. False where this

@@ -598,17 +598,25 @@ bool operation_convolution<Dtype>::forward_stem(operation_input<Dtype>* input, c
 }
 
 template <typename Dtype>
-bool operation_convolution<Dtype>::forward_head(const operation_reshape<Dtype>& reshape, const tensor_list<unsigned short>& bottoms,
-                                                tensor_list<unsigned short>& tops) {
-    const int dev = this->params_.device_, c = this->input_channels();
+bool operation_convolution<Dtype>::head_form(const operation_reshape<Dtype>& reshape, const tensor_list<unsigned short>& bottoms, exhip_conv_desc* d,
+                                             std::vector<int>* to) const {
+    const int c = this->input_channels();
     if (bottoms[0]->order() != memory::NHWC || bottoms[0]->channels() != c || !mfma_path_ok() || !nhwc_allowed()) return false;
     const int n = bottoms[0]->num(), h = bottoms[0]->height(), w = bottoms[0]->width();
-    exhip_conv_desc d = describe(n, h, w, c, (this->output_channel_ + 31) / 32 * 32);
-    if (d.kh != 1 || d.kw != 1 || d.sh != 1 || d.sw != 1 || d.pt || d.pb || d.pl || d.pr || conv_in_stride(c, EXHIP_F16, 1) != c) return false;
-    d.c_stride = c;
-    const std::vector<int> to = reshape.new_shape({n, this->output_channel_, h, w}, static_cast<int>(static_cast<size_t>(n) * this->output_channel_ * h * w));
-    if (to.size() != 4 || to[0] != n || to[1] < 1 || to[2] < 1 || to[1] * to[2] != this->output_channel_ || to[3] != h * w) return false;
-    auto y = new_tensor<unsigned short>({n, to[1], to[3], to[2]}, dev);
+    *d = describe(n, h, w, c, (this->output_channel_ + 31) / 32 * 32);
+    if (d->kh != 1 || d->kw != 1 || d->sh != 1 || d->sw != 1 || d->pt || d->pb || d->pl || d->pr || conv_in_stride(c, EXHIP_F16, 1) != c) return false;
+    d->c_stride = c;
+    *to = reshape.new_shape({n, this->output_channel_, h, w}, static_cast<int>(static_cast<size_t>(n) * this->output_channel_ * h * w));
+    return to->size() == 4 && (*to)[0] == n && (*to)[1] >= 1 && (*to)[2] >= 1 && (*to)[1] * (*to)[2] == this->output_channel_ && (*to)[3] == h * w;
+}
+
+template <typename Dtype>
+bool operation_convolution<Dtype>::forward_head(const operation_reshape<Dtype>& reshape, const tensor_list<unsigned short>& bottoms,
+                                                tensor_list<unsigned short>& tops) {
+    exhip_conv_desc d;
+    std::vector<int> to;
+    if (!head_form(reshape, bottoms, &d, &to)) return false;
+    auto y = new_tensor<unsigned short>({d.n, to[1], to[3], to[2]}, this->params_.device_);
     const int rc = exhip_conv2d_f16_grouped(this->ctx(), &d, to[2], bottoms[0]->gpu_data(), packed_weights(EXHIP_F16, d), bias_gpu(), y->mutable_gpu_data());
     if (rc == EXHIP_ERR_UNSUPPORTED) return false;
     EXHIP_FATAL(rc);

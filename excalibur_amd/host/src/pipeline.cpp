@@ -281,7 +281,6 @@ public:
                     return readers == 1 && std::find(output_names_.begin(), output_names_.end(), blob_names_[mid]) == output_names_.end();
                 };
                 in_groups_[i] = op_inputs_[i].size() == 1 && passes(i) && passes(i + 1) && op_outputs_[i + 2] != op_outputs_[i];
-                if (in_groups_[i]) conv->set_through_rows();
             }
         }
     }
@@ -567,9 +566,13 @@ private:
                 }
             }
             if constexpr (std::is_same_v<Dtype, unsigned short>) {
-                if (fusion_ && in_groups_[i]) {
+                if (in_groups_[i]) {
                     auto* conv = static_cast<operation_convolution<Dtype>*>(operations_[i].get());
-                    if (conv->forward_head(*static_cast<operation_reshape<Dtype>*>(operations_[i + 1].get()), in, out)) {
+                    auto* reshape = static_cast<operation_reshape<Dtype>*>(operations_[i + 1].get());
+                    exhip_conv_desc d;
+                    std::vector<int> to;
+                    conv->set_through_rows(conv->head_form(*reshape, in, &d, &to));
+                    if (fusion_ && conv->forward_head(*reshape, in, out)) {
                         featmaps_[op_outputs_[i][0]] = featmaps_[op_outputs_[i + 1][0]] = nullptr;
                         i += 2;  // the Reshape and Transpose layers have run
                         featmaps_[op_outputs_[i][0]] = out[0];

@@ -57,3 +57,31 @@ def test_heads_in_one_launch_equal_their_layers(name):
         p.close()
     finally:
         os.unlink(path)
+
+
+@pytest.mark.parametrize("kernel,dims", [(3, (400, 85, 3)), (1, (1200, 85, 1))], ids=["3x3", "other groups"])
+def test_a_head_that_one_launch_cannot_do_runs_as_layers_that_are_none(kernel, dims):
+    """With a filter, or a Reshape that is not one of channels into groups: the convolution makes its NCHW result as it does in front of any other layer."""
+    c, k = 256, 255
+    r = np.random.default_rng(kernel)
+    wy, wh = np.eye(c, dtype=np.float32).reshape(c, c, 1, 1), r.normal(0, .05, (k, c, kernel, kernel)).astype(np.float32)
+    x = r.normal(0, 1, (1, c, 20, 20)).astype(np.float16).view(np.uint16)
+    lines = [mf.conv_line("Convolution", "y_l", "data", "y", c, 1, 1, 0, True, c * c), "ReLU x_l 1 1 y x",
+             mf.conv_line("Convolution", "h_l", "x", "h", k, kernel, 1, kernel // 2, True, wh.size, 1), "Reshape r_l 1 1 h r 0=%d 1=%d 2=%d" % dims]
+    with tempfile.NamedTemporaryFile(suffix=".racy", delete=False) as f:
+        f.write(mf.conv_blob_f32(wy, np.zeros(c, np.float32)) + mf.conv_blob_f32(wh, r.normal(0, 1, k).astype(np.float32)))
+        path = f.name
+    got = []
+    try:
+        for perms in ("1,0,2", "0,1,2"):
+            for fusion in (True, False):
+                p = xp.Pipeline(mf.topology(lines + [f"Transpose t_l 1 1 r out 0={perms}"], "head"), path, 0, "f16", fusion=fusion)
+                p.forward(x)
+                out = p.get("out").view(np.float16)
+                got.append(out if perms == "0,1,2" else out.transpose(0, 1, 3, 2))
+                p.close()
+    finally:
+        os.unlink(path)
+    assert np.isfinite(got[0]).all() and np.ptp(got[0].astype(np.float32)) > 1
+    for other in got[1:]:
+        assert np.array_equal(got[0], other)
