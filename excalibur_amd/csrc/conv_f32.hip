@@ -248,10 +248,10 @@ __device__ __forceinline__ void epilogue_block(const F32Params& p, const v16f& a
     }
 }
 
-// The epilogue of a tile that WK waves share: V channels from ch0 on of the lane's pixel. Each wave takes an equal part of the tile, so
-// that its chain is short, and stores from registers: a launch that splits its tiles is small, and the waves fill the same lines.
-// (One wave finished a whole block before, 2400 to 5300 cycles of a launch's 10 000 to 16 000: 512 -> 512 1x1 on three 13 x 13 maps
-// 6.9 -> 6.5 us, 32 -> 64 3x3 at stride 2 on three 104 x 104 maps 7.5 -> 7.1, 256 -> 128 1x1 on three 26 x 26 maps 5.8 -> 5.3.)
+// The epilogue of a tile whose blocks four waves or more share: V channels from ch0 on of the lane's pixel. Each wave takes an equal part of
+// the tile, so that its chain is short, and stores from registers: a launch that splits its tiles so far is small, and the waves fill the same
+// lines. (One wave finished a whole block before, 2400 to 5300 cycles of a launch's 10 000 to 16 000: 512 -> 512 1x1 on three 13 x 13 maps
+// 6.9 -> 6.5 us, 256 -> 128 1x1 on three 26 x 26 maps 5.8 -> 5.3.)
 template <int V>
 __device__ __forceinline__ void epilogue_part(const F32Params& p, float (&v)[V], const float (&par)[kParams][V], const float (&res)[V], unsigned pix, unsigned img,
                                               unsigned in_image, int ch0) {
@@ -353,14 +353,16 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256, 2) void conv_f32_kernel(con
     exhip_touch_args(p);
     constexpr int WAVES = WK > 4 ? WK : 4, ITEMS = WAVES / WK;  // tiles per group
     constexpr int BLOCKS = MT * NT;
-    constexpr int QUADS = 4 * BLOCKS > WK ? 4 * BLOCKS / WK : 1;  // WK > 1: quarters of a block (four channels a lane) that a wave finishes
-    constexpr int V = 4 * QUADS;
-    // A wave that finishes a whole block stores its rows through LDS, one that finishes less from registers: a split launch of two
-    // waves to a tile is still a large one (32 -> 64 3x3 on a 320 x 320 map: 47 us, 52 with stores from registers).
-    constexpr bool ROWS = WK == 1 || QUADS == 4;
+    // A wave of a split tile finishes a block, and stores its rows through LDS, or where that leaves every block to four waves or more a
+    // quarter of one (four channels a lane), and stores from registers. Halves from registers fill lines in pieces of 32 bytes, and launches
+    // of two waves a block are still large: 64 -> 64 3x3 at 24 x 40 x 40 33.8 us in halves, 28.9 in blocks, 128 -> 128 at 4 x 80 x 80 73.7 and
+    // 64.3, 1x1 64 -> 64 at 8 x 80 x 80 12.9 and 11.1.
+    constexpr bool ROWS = WK == 1 || WK < 4 * BLOCKS;
+    constexpr int QUADS = ROWS ? 4 : 1, V = 4 * QUADS;            // WK > 1: quarters of a block that a wave finishes
+    constexpr int OWNERS = WK > 1 ? BLOCKS : 1;                   // ROWS: waves of a tile that finish a block
     constexpr int RED = WK > 1 ? WAVES * BLOCKS * 4096 : 0;       // the waves' partial sums
-    static_assert(QUADS <= 4 || WK == 1, "a wave finishes at most one block");
-    __shared__ __attribute__((aligned(16))) char lds_all[RED + (ROWS ? WAVES * wave_lds(MT) : 0)];
+    static_assert(WK == 1 || OWNERS <= WK, "a wave finishes at most one block");
+    __shared__ __attribute__((aligned(16))) char lds_all[RED + (ROWS ? ITEMS * OWNERS * wave_lds(MT) : 0)];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int part = wave % WK;
     // workgroup ids are dealt round-robin to the 8 XCDs: give each XCD one contiguous run of items. Either the channel groups of
@@ -550,8 +552,8 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256, 2) void conv_f32_kernel(con
     }
     // (the loop leaves with the last steps, at most R, requested)
     if (!ROWS && owner) load_parameters();
-    char* const lds = lds_all + RED + (ROWS ? wave * wave_lds(MT) : 0);
-    if (ROWS && (MT == 2 || lane < 32)) {
+    char* const lds = lds_all + RED + (ROWS && part < OWNERS ? (wave / WK * OWNERS + part) * wave_lds(MT) : 0);
+    if (ROWS && part < OWNERS && (MT == 2 || lane < 32)) {
 #pragma unroll
         for (int i = 0; i < kParams; ++i) *reinterpret_cast<float*>(lds + (i * MT * 32 + lane) * 4) = par[i][0];
     }
