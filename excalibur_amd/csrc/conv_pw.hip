@@ -1471,7 +1471,14 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
         if (p.y_f) return n_ksteps <= 40 ? 12000 : 4096;
         return g.post_relu && n_ksteps > 18 ? 3328 : 0;
     };
-    const bool take = g.pool || kblocks == 1 || DT == EXHIP_F16 || g.c_bytes == 32 || blocks <= int8_most();
+    // Layers at stride 1 of more than 40 k-steps and ragged output channels once more go to the staged kernel from the second round of waves on
+    // (two a SIMD): fp16 96 -> 96 at 5 x 80 x 80 (2000 waves) 16.7 -> 14.9, at 8 x 80 x 80 (3200) 19.9 against 24.7, 128 -> 205 at 3 x 102 x 101
+    // 25.1 against 34.1. A lone block's waves have 64 pixels: fp16 96 -> 32 at 16 x 80 x 80 (1600) 17.6 -> 17.1, at 29 x 69 x 69 (2158) 23.2 against
+    // 26.6; int8 192 -> 32 at 23 x 52 x 52 (972) 16.5 -> 12.2, at 17 x 71 x 71 (1340) 15.9 against 16.6, 256 -> 32 at 24 x 83 x 82 29.2 against 34.9.
+    // The figures are us on the staged kernel -> here.
+    const long long waves = kblocks == 1 ? (g.pixels + 63) / 64 : (g.pixels + 31) / 32 * ((kblocks + 1) / 2);
+    const bool late = t.stride == 1 && n_ksteps > 40 && g.k % 64 != 0 && waves > (kblocks > 1 ? 2048 : DT == EXHIP_F16 ? 1664 : 1024);
+    const bool take = g.pool || g.c_bytes == 32 || (!late && (kblocks == 1 || DT == EXHIP_F16 || blocks <= int8_most()));
     // With the pooling layer behind it: where the layer by itself would run in the split form, on few blocks, that and a launch for the pooling are
     // the faster two, us as two launches -> as one: 64 -> 128 at 1 x 30 x 30 7.4 -> 6.4, 128 -> 128 at 1 x 14 x 14 (36 k-steps) 8.0 against 8.4, at 16
     // x 14 x 14 (288 blocks) 8.7 and 8.6, 256 -> 256 at 4 x 16 x 16 (72 k-steps) 9.5 against 13.2, at 16 x 16 x 16 (1024) 14.2 -> 13.5. Beyond, the float32
