@@ -1455,16 +1455,19 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
     // Other int8 layers by what stands behind the products, us on the staged or lean kernel -> here, over some 60 maps from 16 to 111 wide:
     //  * stride 2: everything, 27.5 -> 21.9 (256 -> 256 at 48 x 37 x 34), 17.4 -> 11.1 with a float32 result (64 -> 128 at 48 x 50 x 47) --
     //    but with an int8 result alone large maps in powers of two stay (128 -> 256 at 16 x 80 x 80 17.1 against 21.5): up to 4800
-    //    blocks of 32 x 32 (17.9 -> 16.8).
+    //    blocks of 32 x 32 (17.9 -> 16.8) and three waves a SIMD (192 -> 96 at 8 x 80 x 80, 3200 waves, 24.9 against 28.9). A ReLU alone behind
+    //    whole blocks makes the staged kernel faster (192 -> 96 at stride 1, 2 x 106 x 109, 13.1 with it, 16.2 without): two waves a SIMD there beyond 40
+    //    k-steps or without pairs (256 -> 96 at 5 x 80 x 80, 2000 waves, 24.4 -> 20.9, at 7 x 75 x 75, 2462 waves, 26.0 against 28.9).
     //  * stride 1, where the lean kernel takes a plain ReLU in 8.7 us for 128 -> 128 at 16 x 40 x 40 and this one in 12.2: an activation
     //    layer (17.8 -> 12.0; 64 -> 64 at 8 x 80 x 80 9.9 -> 8.1, at 16 x 80 x 80 12.2 against 13.4), a float32 result beside the
     //    int8 one (20.9 -> 14.6 at 4 x 80 x 80, 40.5 -> 40.2 at 11 856 blocks; 72 k-steps 27.9 -> 23.6 at 4096, 37.1 against 40.4 at
     //    6400), a sum (17.6 -> 15.3 at 3200, 20.8 against 21.4 at 4376; 18 k-steps 8.8 -> 8.4 at 1944, 9.2 against 10.8 at 2376; 72 never),
     //    the ReLU behind (13.7 -> 12.2; 18 k-steps never).
-    const long long blocks = (g.pixels + 31) / 32 * kblocks;
+    const long long blocks = (g.pixels + 31) / 32 * kblocks, waves = kblocks == 1 ? (g.pixels + 63) / 64 : (g.pixels + 31) / 32 * ((kblocks + 1) / 2);
+    const bool relu_alone = DT == EXHIP_I8 && (g.act == 1 || g.post_relu) && g.k % 32 == 0 && !g.post_op && !has_residual && !p.y_f;
     auto int8_most = [&]() -> long long {
         const long long all = 1ll << 40;
-        if (t.stride != 1) return g.post_op || has_residual || p.y_f ? all : 4800;
+        if (t.stride != 1) return g.post_op || has_residual || p.y_f ? all : waves <= (relu_alone && (n_ksteps > 40 || g.c_bytes % 64 != 0) ? 2048 : 3072) ? 4800 : 0;
         if (t.kh != 3 || t.kw != 3 || t.chunk_b != 64 || g.k % 64 != 0) return 3328;  // the staged kernel's
         if (g.post_op) return n_ksteps <= 40 ? 4096 : 3328;
         if (has_residual) return n_ksteps <= 18 ? 2048 : n_ksteps <= 40 ? 3328 : 0;
@@ -1475,9 +1478,11 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
     // (two a SIMD): fp16 96 -> 96 at 5 x 80 x 80 (2000 waves) 16.7 -> 14.9, at 8 x 80 x 80 (3200) 19.9 against 24.7, 128 -> 205 at 3 x 102 x 101
     // 25.1 against 34.1. A lone block's waves have 64 pixels: fp16 96 -> 32 at 16 x 80 x 80 (1600) 17.6 -> 17.1, at 29 x 69 x 69 (2158) 23.2 against
     // 26.6; int8 192 -> 32 at 23 x 52 x 52 (972) 16.5 -> 12.2, at 17 x 71 x 71 (1340) 15.9 against 16.6, 256 -> 32 at 24 x 83 x 82 29.2 against 34.9.
-    // The figures are us on the staged kernel -> here.
-    const long long waves = kblocks == 1 ? (g.pixels + 63) / 64 : (g.pixels + 31) / 32 * ((kblocks + 1) / 2);
-    const bool late = t.stride == 1 && n_ksteps > 40 && g.k % 64 != 0 && waves > (kblocks > 1 ? 2048 : DT == EXHIP_F16 ? 1664 : 1024);
+    // The figures are us on the staged kernel -> here. int8 layers with a ReLU alone (above): from the second wave a SIMD on (192 -> 96 at 2 x 80 x 80, 800
+    // waves, 14.5 -> 10.9, at 3 x 75 x 75, 1056 waves, 13.3 against 14.3), and a lone block of 72 k-steps on fewer than one SIMD in four, which the staged
+    // kernel splits (256 -> 32 at 1 x 80 x 80 12.6 against 14.0, at 28 x 26 x 26, 296 waves, 14.8 -> 14.3).
+    const bool late = t.stride == 1 && n_ksteps > 40 && g.k % 64 != 0 &&
+                      (waves > (relu_alone ? 1024 : kblocks > 1 ? 2048 : DT == EXHIP_F16 ? 1664 : 1024) || (relu_alone && kblocks == 1 && n_ksteps >= 64 && waves <= 256));
     const bool take = g.pool || g.c_bytes == 32 || (!late && (kblocks == 1 || DT == EXHIP_F16 || blocks <= int8_most()));
     // With the pooling layer behind it: where the layer by itself would run in the split form, on few blocks, that and a launch for the pooling are
     // the faster two, us as two launches -> as one: 64 -> 128 at 1 x 30 x 30 7.4 -> 6.4, 128 -> 128 at 1 x 14 x 14 (36 k-steps) 8.0 against 8.4, at 16
