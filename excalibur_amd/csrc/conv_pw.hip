@@ -1335,6 +1335,8 @@ bool split_wins(int dt, const exhip_pw_geom& g, int kblocks, int n_ksteps, bool 
         return blocks <= (n_ksteps < 16 ? 832 : 6656);
     }
     if (stride != 1) return blocks <= (n_ksteps < 16 ? 832 : n_ksteps < 64 ? (dt == EXHIP_I8 ? 1280 : 1920) : blocks * n_ksteps <= 240000 ? 1920 : 832);
+    // (parts of blocks, and more k-steps than the tapped form takes, leave the staged kernel: int8 384 -> 48 at 1600 blocks 23.5 -> 18.6)
+    if (dt == EXHIP_I8 && n_ksteps > 2 * kMaxDirectSteps && g.k % 32 != 0 && !g.post_op) return blocks <= 1664;
     return blocks <= (dt == EXHIP_I8 && n_ksteps >= 64 && g.post_op ? 2560 : 1280);
 }
 
