@@ -1337,7 +1337,13 @@ bool split_wins(int dt, const exhip_pw_geom& g, int kblocks, int n_ksteps, bool 
     if (stride != 1) return blocks <= (n_ksteps < 16 ? 832 : n_ksteps < 64 ? (dt == EXHIP_I8 ? 1280 : 1920) : blocks * n_ksteps <= 240000 ? 1920 : 832);
     // (parts of blocks, and more k-steps than the tapped form takes, leave the staged kernel: int8 384 -> 48 at 1600 blocks 23.5 -> 18.6)
     if (dt == EXHIP_I8 && n_ksteps > 2 * kMaxDirectSteps && g.k % 32 != 0 && !g.post_op) return blocks <= 1664;
-    return blocks <= (dt == EXHIP_I8 && n_ksteps >= 64 && g.post_op ? 2560 : 1280);
+    if (dt == EXHIP_I8 && n_ksteps >= 64 && g.post_op) {
+        // beyond 100 k-steps, of whole blocks, the products decide: up to 1216 tiles (384 -> 64 at 1000 tiles 19.9 and 19.7, at 1231 20.0 against 23.2, 384 -> 96 at
+        // 1184 24.2 -> 22.4, at 1432 24.0 against 26.8)
+        const long long tiles = (g.pixels + 31) / 32 * ((kblocks + 1) / 2);
+        return blocks <= 2560 && (n_ksteps <= 100 || g.k % 32 != 0 || tiles <= 1216);
+    }
+    return blocks <= 1280;
 }
 
 // Where a pixel's bytes of a tap (of all channels for a 1x1 layer) come in whole 64-byte pieces, the k-steps are taken in pairs. A
