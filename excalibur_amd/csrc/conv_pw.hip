@@ -1543,20 +1543,31 @@ int run_depthwise(exhip_ctx* ctx, const exhip_pw_depthwise& dw, PwParams& p, int
     // 0.8 us of it: while the chip has room, groups of half the pixels (256 -> 128 at 1 x 14 x 14: 8.0 us with 32 pixels, 6.5 with
     // 16, 5.5 with 8, 5.2 with 4; 512 -> 128 at 1 x 7 x 7: 14.6, 10.1, 8.2, 7.1), but a second round of groups costs what
     // it saves (256 -> 128 at 16 x 14 x 14: 8.3 with 32, 6.6 with 16 in 196 groups, 6.8 with 8 in 392) unless the strips are many (512 ->
-    // 128 at 64 x 7 x 7: 10.5 with 16, 9.8 with 8 in 392). A large launch wants a strip for every thread and no more: 16 -> 32 at
+    // 128 at 64 x 7 x 7: 10.5 with 16, 9.8 with 8 in 392; 384 -> 128 at stride 2 to 305 x 32 pixels 19.1 with 32, 15.1 with 16 in 610). A large
+    // launch wants a strip for every thread and no more, and two groups for every CU or so, more where many output channels follow (16 -> 256 at
+    // 1182 x 32 pixels 13.8 with 256, 9.8 with 64, 9.5 with 32; 96 -> 512 at 1425 x 32 31.9 with 128, 22.5 with 64): 16 -> 32 at
     // 64 x 112 x 112 24.5 us with 256 pixels, 33.6 with 128, 55.5 with 64; 32 -> 64 43.7 with 128, 61.8 with 64; 128 -> 64 at 64 x 56 x 56
     // 33.8 with 64, 39.3 with 32; 256 -> 128 at 64 x 28 x 28 27.7 with 64, 22.7 with 32.
     p.dw_pixels = 32;
     if (tiles32 >= 1024)
-        while (p.dw_pixels < 256 && p.dw_pixels * channels4 < (channels4 < 24 ? 1024 : 2048)) p.dw_pixels *= 2;
+        while (p.dw_pixels < 256 && p.dw_pixels * channels4 < (channels4 < 24 ? 1024 : 2048) && p.pixels / (2 * p.dw_pixels) >= (kblocks < 4 ? 448u : 640u)) p.dw_pixels *= 2;
     auto more = [&]() { return ((long long)p.pixels * 2 + p.dw_pixels - 1) / p.dw_pixels * ((kblocks + 3) / 4); };  // groups with half the pixels each
-    while (p.dw_pixels > 4 && p.dw_pixels * channels4 > 256 && more() <= (p.dw_pixels * channels4 > 1024 ? 512 : 256)) p.dw_pixels /= 2;
+    while (p.dw_pixels > 4 && p.dw_pixels * channels4 > 256 && more() <= (p.dw_pixels * channels4 > 1024 ? 704 : 256)) p.dw_pixels /= 2;
     if (const int forced = g_exhip_options.dw_pw; forced >= 4 && forced <= 256 && (forced & (forced - 1)) == 0 && forced * (p.xs_b + 16) <= 40960) p.dw_pixels = forced;
     const bool small = p.dw_pixels < 32;
     // One launch is the faster one but for wide layers of a middling size, whose groups are few and long: 512 -> 512 at 20 x 14 x 14 16.6 us,
     // 15.8 as two launches, 384 -> 384 at 8 x 14 x 14 10.8 and 9.9, 256 -> 512 at stride 2 from 8 x 28 x 28 8.2 and 7.8; on the other
     // sides 512 -> 512 at 1 x 14 x 14 6.8 and 8.9, at 64 x 14 x 14 27.0 and 31.0, 512 -> 128 at 64 x 7 x 7 10.1 and 10.5.
-    if (g_exhip_options.dw_pw == 1 && tiles32 > 40 && tiles32 <= 256 && kblocks > (p.xs_b > 512 ? 4 : 8)) return EXHIP_ERR_UNSUPPORTED;
+    // The depthwise half reads a strip's neighbours once for all its pixels; strips of one pixel (an odd width) or two make it the longer one where a
+    // launch has many: us for the pair and for the two, 384 -> 256 at 302 x 32 pixels 20.2 and 14.6, 512 -> 64 at 24 x 39 x 39 38.5 and 30.7, 192 -> 32 at 17 x 125 x 125
+    // 74.4 and 57.0, 96 -> 128 at 10747 x 32 65.8 and 52.3; in strips of two 384 -> 64 at 3 x 111 x 114 28.1 and 24.8. (384 -> 96 at 885 x 32 23.3 and 27.0.)
+    if (g_exhip_options.dw_pw == 1) {
+        if (tiles32 > 40 && tiles32 <= 256 && kblocks > (p.xs_b > 512 ? 4 : 8)) return EXHIP_ERR_UNSUPPORTED;
+        if (tiles32 > 20 && tiles32 <= 40 && kblocks > 8 && p.xs_b >= 768) return EXHIP_ERR_UNSUPPORTED;  // 384 -> 512 at 34 x 32 11.3 and 8.3
+        if (widest == 1 && p.xs_b >= 768 && ((tiles32 > 256 && tiles32 <= 640) || tiles32 > (p.xs_b < 1024 ? 1024 : 768))) return EXHIP_ERR_UNSUPPORTED;
+        if (widest == 1 && ((p.xs_b >= 384 && tiles32 > 2048) || (p.xs_b >= 128 && tiles32 > 6144))) return EXHIP_ERR_UNSUPPORTED;
+        if (widest == 2 && p.xs_b >= 768 && tiles32 > 1024) return EXHIP_ERR_UNSUPPORTED;
+    }
     p.dw_tiles = std::max(p.dw_pixels / 32, 1);
     const long long tiles = ((long long)p.pixels + p.dw_pixels - 1) / p.dw_pixels;
     int groups = 1;
