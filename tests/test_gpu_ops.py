@@ -528,7 +528,7 @@ def test_innerproduct_within_1e4(ctx):
         assert cases.check_value(gpueval.gpu_eval(ctx, case), cases.oracle_eval(case), 1e-4) == 0
 
 
-@pytest.mark.parametrize("m,n_out,k_in,bias", [(1, 128, 512, True), (64, 128, 512, False), (9, 7, 1028, True), (3, 5, 130, True), (8, 1, 4, False)])
+@pytest.mark.parametrize("m,n_out,k_in,bias", [(1, 128, 512, True), (64, 128, 512, False), (9, 7, 1028, True), (3, 5, 130, True), (8, 1, 4, False), (2, 6, 516, True), (2, 9, 70, False)])
 def test_innerproduct_half_is_the_float_one_rounded(ctx, m, n_out, k_in, bias):
     r = np.random.default_rng(k_in)
     x = r.normal(0, 1, (m, k_in)).astype(np.float16)
