@@ -1469,7 +1469,9 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
     //  * stride 1, where the lean kernel takes a plain ReLU in 8.7 us for 128 -> 128 at 16 x 40 x 40 and this one in 12.2: an activation
     //    layer (17.8 -> 12.0; 64 -> 64 at 8 x 80 x 80 9.9 -> 8.1, at 16 x 80 x 80 12.2 against 13.4), a float32 result beside the
     //    int8 one (20.9 -> 14.6 at 4 x 80 x 80, 40.5 -> 40.2 at 11 856 blocks; 72 k-steps 27.9 -> 23.6 at 4096, 37.1 against 40.4 at
-    //    6400), a sum (17.6 -> 15.3 at 3200, 20.8 against 21.4 at 4376; 18 k-steps 8.8 -> 8.4 at 1944, 9.2 against 10.8 at 2376; 72 never),
+    //    6400; 18 k-steps but for 5632 to 8192 blocks, one full round of the lean kernel, 14.4 against 15.7 at 6400), no activation at all, which the
+    //    lean kernel has no form for (18 k-steps 9.7 -> 6.4 at 1600, 11.1 -> 9.8 at 4800, 11.5 against 12.5 at 6400; 36 16.0 -> 8.5 and 22.7 -> 19.1 at 6400,
+    //    17.3 against 19.2 at 7504; 72 20.5 -> 18.7 at 3200, 18.3 against 18.8 at 3752), a sum (17.6 -> 15.3 at 3200, 20.8 against 21.4 at 4376; 18 k-steps 8.8 -> 8.4 at 1944, 9.2 against 10.8 at 2376; 72 never),
     //    the ReLU behind (13.7 -> 12.2; 18 k-steps never).
     const long long blocks = (g.pixels + 31) / 32 * kblocks, waves = kblocks == 1 ? (g.pixels + 63) / 64 : (g.pixels + 31) / 32 * ((kblocks + 1) / 2);
     const bool relu_alone = DT == EXHIP_I8 && (g.act == 1 || g.post_relu) && g.k % 32 == 0 && !g.post_op && !has_residual && !p.y_f;
@@ -1479,7 +1481,8 @@ int run_taps(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, PwP
         if (t.kh != 3 || t.kw != 3 || t.chunk_b != 64 || g.k % 64 != 0) return 3328;  // the staged kernel's
         if (g.post_op) return n_ksteps <= 40 ? 4096 : 3328;
         if (has_residual) return n_ksteps <= 18 ? 2048 : n_ksteps <= 40 ? 3328 : 0;
-        if (p.y_f) return n_ksteps <= 40 ? 12000 : 4096;
+        if (p.y_f) return n_ksteps <= 18 && blocks > 5632 && blocks <= 8192 ? 0 : n_ksteps <= 40 ? 12000 : 4096;
+        if (!g.act && !g.post_relu) return n_ksteps <= 18 ? 4800 : n_ksteps <= 40 ? 6400 : 3328;
         return g.post_relu && n_ksteps > 18 ? 3328 : 0;
     };
     // Layers at stride 1 of more than 40 k-steps and ragged output channels once more go to the staged kernel from the second round of waves on
