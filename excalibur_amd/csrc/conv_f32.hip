@@ -1,4 +1,5 @@
-// conv_f32_kernel: the float32 convolution, any filter, stride and padding, on NHWC input with v_mfma_f32_32x32x2_f32.
+// conv_f32_kernel: the float32 convolution, any filter, stride and padding, on NHWC input with v_mfma_f32_32x32x2_f32. (3x3 layers at stride 1
+// of whole 16-channel steps run in conv_f32_thirds.hip.)
 //
 // float32 products run at a sixteenth of the half-precision rate (157 TFLOP/s), so operands are cheap next to the
 // arithmetic: one 32-byte step of a 64-channel x 32-pixel wave tile fetches 3 KiB for 512 matrix cycles. Nothing is staged
@@ -22,47 +23,10 @@
 #include <type_traits>
 
 #include "conv_f32.h"
+#include "conv_f32_epilogue.h"
 #include "pack.h"
 
 namespace {
-
-typedef exhip_v4i v4i;
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef unsigned v4u __attribute__((ext_vector_type(4)));
-
-constexpr unsigned kRsrcWord3 = 0x00020000u;      // raw buffer: out-of-range loads return 0, such stores are dropped
-constexpr unsigned kOutOfRange = 0xfffff000u;     // a lane offset beyond every view
-constexpr int kMaxSplit = 8;
-
-// How a step's 32 bytes lie in the input: kPoint one tap, always inside the image (1x1 filters without padding); kTaps 8
-// channels of one tap; kPair two neighbouring taps of 16-byte pixels (layers of at most four channels).
-enum { kPoint, kTaps, kPair };
-
-struct F32Params {
-    const char* x;
-    const char* wp;
-    const float *bias, *residual, *slope, *bn_a, *bn_b;
-    float *y, *y_nchw;
-    unsigned pixels, x_bytes, w_bytes, items;
-    unsigned fast;                 // the channel groups or (tiles_fast) the pixel tiles, whichever neighbouring items walk
-    unsigned fast_magic, image_magic, width_magic;  // exhip_divide() by fast, out_h * out_w, out_w
-    int fast_shift, image_shift, width_shift, tiles_fast;
-    int in_h, in_w, out_h, out_w, stride, pad_t, pad_l, kh, kw;
-    int xs_b, row_b;               // bytes per input pixel and input row
-    int csteps, n_ksteps;          // steps per tap (kPair: 1) and in all
-    int start_r[kMaxSplit + 1], start_q[kMaxSplit + 1], start_c[kMaxSplit + 1], start_s[kMaxSplit + 1];  // where each wave of a tile begins
-    int K, kstride, k_end;         // channels from k_end on are not written
-    int act, post_relu, bn_relu, post_op, slope_shared, residual_last;
-    float alpha, beta;
-    int vector_rows;               // output (and shortcut) rows take 16-byte accesses
-    int rstride, res_shift;        // the shortcut's channel stride; log2 of how many output pixels per axis share one of its pixels
-    int layout, group;             // EXHIP_PLACE_*; grouped: channels per group, shuffled: channels of an upsampled pixel
-};
-
-__device__ __forceinline__ v4f load4(__amdgpu_buffer_rsrc_t r, unsigned voff, int soff) {
-    return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, soff, 0));
-}
 
 // A view of a pixel-major float tensor from pixel `first` and channel ch0 on, `rows` pixels long.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_view(const float* base, unsigned first, int stride, int ch0, int rows) {
@@ -91,7 +55,6 @@ __device__ __forceinline__ void relu16(float (&v)[16]) {
     for (int e = 0; e < 16; ++e) v[e] = (0.f > v[e]) ? 0.f : v[e];
 }
 
-constexpr int kParams = 4;                // bias / PReLU slope / BatchNorm a / b
 constexpr int kTilePitch = 128 + 16;      // one pixel's 32 channels and padding
 constexpr int wave_lds(int mt) { return kParams * mt * 32 * 4 + 32 * kTilePitch; }
 
@@ -244,105 +207,6 @@ __device__ __forceinline__ void epilogue_block(const F32Params& p, const v16f& a
         float* const dst = p.y_nchw + ((size_t)img * p.K + ch0) * per_image + in_image;
 #pragma unroll
         for (int e = 0; e < 16; ++e)
-            if (ch0 + e < p.K) dst[(size_t)e * per_image] = v[e];
-    }
-}
-
-// The epilogue of a tile whose blocks four waves or more share: V channels from ch0 on of the lane's pixel. Each wave takes an equal part of
-// the tile, so that its chain is short, and stores from registers: a launch that splits its tiles so far is small, and the waves fill the same
-// lines. (One wave finished a whole block before, 2400 to 5300 cycles of a launch's 10 000 to 16 000: 512 -> 512 1x1 on three 13 x 13 maps
-// 6.9 -> 6.5 us, 256 -> 128 1x1 on three 26 x 26 maps 5.8 -> 5.3.)
-template <int V>
-__device__ __forceinline__ void epilogue_part(const F32Params& p, float (&v)[V], const float (&par)[kParams][V], const float (&res)[V], unsigned pix, unsigned img,
-                                              unsigned in_image, int ch0) {
-    const unsigned per_image = (unsigned)(p.out_h * p.out_w);
-    auto relu = [&]() {
-#pragma unroll
-        for (int e = 0; e < V; ++e) v[e] = (0.f > v[e]) ? 0.f : v[e];
-    };
-    auto each = [&](auto op) {
-#pragma unroll
-        for (int e = 0; e < V; ++e) v[e] = unary_value<decltype(op)::value>(v[e], p.alpha, p.beta);
-    };
-#pragma unroll
-    for (int e = 0; e < V; ++e) v[e] += par[0][e];
-    if (p.act == 1) relu();
-    if (p.act == 3) {
-#pragma unroll
-        for (int e = 0; e < V; ++e) v[e] = exhip_act(v[e], 3);
-    }
-    if (p.residual && !p.residual_last) {
-#pragma unroll
-        for (int e = 0; e < V; ++e) v[e] += res[e];
-    }
-    if (p.post_relu) relu();
-    if (p.bn_a) {
-#pragma unroll
-        for (int e = 0; e < V; ++e) v[e] = __builtin_fmaf(par[3][e], v[e], par[2][e]);
-        if (p.bn_relu) relu();
-    }
-    switch (p.post_op) {
-    case 0: break;
-    case 1 + EXHIP_UNARY_HARDSWISH: each(std::integral_constant<int, 0>{}); break;
-    case 1 + EXHIP_UNARY_LEAKYRELU: each(std::integral_constant<int, 1>{}); break;
-    case 1 + EXHIP_UNARY_HARDSIGMOID: each(std::integral_constant<int, 3>{}); break;
-    case 1 + EXHIP_UNARY_CLIP: each(std::integral_constant<int, 4>{}); break;
-    default:
-#pragma unroll
-        for (int e = 0; e < V; ++e) v[e] = v[e] >= 0.f ? v[e] : par[1][e] * v[e];
-    }
-    if (p.residual && p.residual_last) {
-#pragma unroll
-        for (int e = 0; e < V; ++e) v[e] += res[e];
-    }
-    if (pix >= p.pixels) return;
-    if (p.y) {
-#pragma unroll
-        for (int e = 0; e < V; ++e)
-            if (ch0 + e >= p.K) v[e] = 0.f;  // pad channels hold zeros
-        if (p.layout == EXHIP_PLACE_GROUPED) {
-            // y[img][group][pixel][member]
-            float* const to = p.y + (size_t)img * (unsigned)p.K * per_image + (size_t)in_image * (unsigned)p.group;
-            int g = ch0 / p.group, member = ch0 - g * p.group;
-#pragma unroll
-            for (int e = 0; e < V; ++e) {
-                if (ch0 + e < p.K) to[(size_t)g * per_image * (unsigned)p.group + member] = v[e];
-                if (++member == p.group) member = 0, ++g;
-            }
-        } else {
-            float* to = p.y + (size_t)pix * (unsigned)p.kstride + ch0;
-            int end = p.k_end, ch = ch0;
-            if (p.layout == EXHIP_PLACE_SHUFFLED && p.vector_rows) {
-                // channel pos * group + k of pixel (y, x) is channel k of pixel (2 y + pos / 2, 2 x + pos % 2) of a map twice as large
-                const unsigned oy = exhip_divide(in_image, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = in_image - oy * (unsigned)p.out_w;
-                const int pos = ch0 / p.group;
-                const unsigned at = (img * 2 * (unsigned)p.out_h + 2 * oy + (pos >> 1)) * 2 * (unsigned)p.out_w + 2 * ox + (pos & 1);
-                to = p.y + (size_t)at * (unsigned)p.kstride + (ch0 - pos * p.group);
-                end = p.K;
-            }
-            if (p.layout == EXHIP_PLACE_SHUFFLED && !p.vector_rows) {
-                const unsigned oy = exhip_divide(in_image, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = in_image - oy * (unsigned)p.out_w;
-                const unsigned corner = (img * 2 * (unsigned)p.out_h + 2 * oy) * 2 * (unsigned)p.out_w + 2 * ox;
-#pragma unroll
-                for (int e = 0; e < V; ++e) {
-                    const int pos = (ch0 + e) / p.group, k = ch0 + e - pos * p.group;
-                    if (ch0 + e < p.K) p.y[(size_t)(corner + (unsigned)(pos >> 1) * 2 * (unsigned)p.out_w + (pos & 1)) * (unsigned)p.kstride + k] = v[e];
-                }
-            } else if (p.vector_rows) {
-#pragma unroll
-                for (int e = 0; e < V; e += 4)
-                    if (ch + e < end) *reinterpret_cast<v4f*>(to + e) = v4f{v[e], v[e + 1], v[e + 2], v[e + 3]};
-            } else {
-#pragma unroll
-                for (int e = 0; e < V; ++e)
-                    if (ch + e < end) to[e] = v[e];
-            }
-        }
-    }
-    if (p.y_nchw) {  // 32 neighbouring pixels of a channel per store instruction and half-wave
-        float* const dst = p.y_nchw + ((size_t)img * p.K + ch0) * per_image + in_image;
-#pragma unroll
-        for (int e = 0; e < V; ++e)
             if (ch0 + e < p.K) dst[(size_t)e * per_image] = v[e];
     }
 }
@@ -716,6 +580,7 @@ int exhip_conv_f32_validate(const exhip_conv_desc* d) {
 
 size_t exhip_conv_f32_packed_bytes(const exhip_conv_desc* d) {
     if (exhip_conv_f32_validate(d)) return 0;
+    if (exhip_conv_f32_thirds(d)) return exhip_conv_f32_thirds_bytes(d);
     return (size_t)((d->k + 31) / 32) * taps_steps(d) * 1024;
 }
 
@@ -724,6 +589,10 @@ size_t exhip_conv_f32_packed_bytes(const exhip_conv_desc* d) {
 int exhip_conv_f32_pack_weights(const exhip_conv_desc* d, const float* w, float* out) {
     const int rc = exhip_conv_f32_validate(d);
     if (rc) return rc;
+    if (exhip_conv_f32_thirds(d)) {
+        exhip_conv_f32_thirds_pack(d, w, out);
+        return 0;
+    }
     const bool pair = d->c_stride == 4;
     const int C = d->c, K = d->k, KH = d->kh, KW = d->kw, csteps = pair ? 1 : (C + 7) / 8;
     const int taps_w = pair ? (KW + 1) / 2 : KW;
@@ -792,9 +661,10 @@ static int run_conv_f32(exhip_ctx* ctx, const exhip_conv_desc* d, const exhip_co
     p.xs_b = d->c_stride * 4;
     p.row_b = d->w * p.xs_b;
     const bool pair = d->c_stride == 4;
-    p.csteps = pair ? 1 : (d->c + 7) / 8;
+    const bool thirds = exhip_conv_f32_thirds(d);
+    p.csteps = thirds ? d->c / 16 : pair ? 1 : (d->c + 7) / 8;
     p.n_ksteps = taps_steps(d);
-    p.w_bytes = (unsigned)((size_t)((d->k + 31) / 32) * p.n_ksteps * 1024);
+    p.w_bytes = (unsigned)(thirds ? exhip_conv_f32_thirds_bytes(d) : (size_t)((d->k + 31) / 32) * p.n_ksteps * 1024);
     p.K = d->k;
     p.kstride = d->k_stride;
     p.k_end = d->exact_k || !y || layout != EXHIP_PLACE_ROWS ? d->k : std::max(d->k, d->k_stride);
@@ -811,7 +681,7 @@ static int run_conv_f32(exhip_ctx* ctx, const exhip_conv_desc* d, const exhip_co
     const long long img_bytes = (long long)d->h * p.row_b, per_image = (long long)oh * ow;
     EXHIP_REQUIRE(per_image < (1ll << 29) && (layout != EXHIP_PLACE_GROUPED || per_image * d->k < (1ll << 31)), "conv: too many output pixels in an image");
     // input offsets are 32-bit, pixel numbers 31-bit, offsets of grouped results 32-bit: as many images per launch as fit
-    long long most = std::min(0x7fff0000ll / img_bytes, ((1ll << (layout == EXHIP_PLACE_SHUFFLED ? 29 : 31)) - 256) / per_image);
+    long long most = std::min(0x7fff0000ll / img_bytes, ((1ll << (thirds || layout == EXHIP_PLACE_SHUFFLED ? 29 : 31)) - 256) / per_image);
     if (layout == EXHIP_PLACE_GROUPED) most = std::min(most, (1ll << 32) / (per_image * d->k) - 1);
     most = std::max(1ll, most);
     const long long y_image = layout == EXHIP_PLACE_SHUFFLED ? per_image * 4 * d->k_stride : layout == EXHIP_PLACE_GROUPED ? per_image * d->k : per_image * d->k_stride;
@@ -825,9 +695,10 @@ static int run_conv_f32(exhip_ctx* ctx, const exhip_conv_desc* d, const exhip_co
         p.y_nchw = y_nchw ? y_nchw + n0 * per_image * d->k : nullptr;
         // 1x1 layers of whole 64-byte pieces take the pixels in pairs of steps: 512 -> 256 on one 20 x 20 map 6.05 -> 5.44 us, 1024 -> 512 on
         // three 13 x 13 maps 9.1 -> 8.3. With a filter the products bound the chain, and the detour through LDS only lengthens it
-        // (64 -> 64 3x3 on one 160 x 160 map 23.6 us, 25.2 in pairs).
+        // (64 -> 64 3x3 on one 160 x 160 map 23.6 us, 25.2 in pairs, 15.4 in thirds).
         const bool point = d->kh == 1 && d->kw == 1 && !d->pt && !d->pb && !d->pl && !d->pr;
-        const int go_rc = pair                  ? pick<kPair, false>(ctx, p, write_blocks)
+        const int go_rc = thirds                ? exhip_conv_f32_thirds_run(ctx, {&p, n, write_blocks})
+                          : pair                  ? pick<kPair, false>(ctx, p, write_blocks)
                           : !point              ? pick<kTaps, false>(ctx, p, write_blocks)
                           : p.csteps % 2 == 0   ? pick<kPoint, true>(ctx, p, write_blocks)
                                                 : pick<kPoint, false>(ctx, p, write_blocks);

@@ -1,0 +1,698 @@
+// conv3x3_thirds_kernel: float32 convolution with 3x3 filters of whole 16-channel steps at stride 1 on the bfloat16 matrix units.
+//
+// float32 products run at a sixteenth of the bfloat16 rate (157 against 2500 TFLOP/s), and a float32 is exactly the sum of three bfloat16
+// values, its thirds: h = round(x), m = round(x - h), l = x - h - m. Six of the nine products of two numbers' thirds hold everything down
+// to 2^-24 of the result (h h; h m, m h; m m, h l, l h: the other three lie below half a float32 ulp of it), so that a step of 16 channels
+// costs six v_mfma_f32_32x32x16_bf16 (192 cycles) instead of eight v_mfma_f32_32x32x2_f32 (512). The unit adds 16 products at a
+// time and rounds once; it rounds small addends toward minus infinity, though, so h h has accumulators of its own, and the five
+// others, 2^-8 of it, theirs. Against sums in 64 bits the results are off by a third to a half of what the float32 products leave
+// (2-norm over K = 576 random values 1.4e-7 and 4.3e-7, over 4608 4.2e-7 and 12.2e-7, all positive 1.3e-7 and 3.7e-7).
+//
+// The weights are packed as thirds. The pixels are split once, on their way into LDS: a group of four or eight waves stages the input
+// under a run of pixels, 16 * CS channels at a time, and takes the nine taps from there; a split in registers would cost every wave 44
+// vector instructions per 32 pixels, tap and step. Weight fragments come straight from memory, three taps ahead.
+//
+// A group's pixels are neighbours in a list of the output's vertical strips, row by row (a strip of a 13 x 13 map is the map). So ragged maps
+// waste no lanes, small maps of several images share groups, and what a run needs of the input are whole rows of a strip, one after
+// another, whatever the run begins with. WK waves share a run's steps, their sums meet in LDS in a fixed order.
+//
+// Infinities and NaN: a third of an infinity is NaN, as is one times the zero third of a finite weight. A result that is not finite is
+// therefore computed again with float32 products (exact_products), whose result it gets.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+#include <cstdint>
+#include <cstring>
+#include <mutex>
+#include <thread>
+
+#include "conv_f32.h"
+#include "conv_f32_epilogue.h"
+
+namespace {
+
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef unsigned v2u __attribute__((ext_vector_type(2)));
+
+constexpr int kTapBytes = 3 * 1024;          // a 32-channel block's weights of one tap and step: three thirds
+constexpr int kStepBytes = 9 * kTapBytes;
+constexpr int kLdsLimit = 160 * 1024;
+
+// Division by a launch constant without a branch (exhip_divide() tests for 1; a taken branch is a line of code that no cache has seen yet).
+struct Divisor {
+    unsigned magic, one;  // one: all ones for a divisor of 1, whose magic is 0
+    int shift;
+    __device__ __forceinline__ unsigned operator()(unsigned n) const { return (__umulhi(n, magic) >> shift) | (n & one); }
+    void set(unsigned d) {
+        exhip_host_divisor(d, &magic, &shift);
+        one = d == 1 ? ~0u : 0u;
+    }
+};
+
+struct ThirdsParams {
+    F32Params f;
+    unsigned total;                // pixels of the list (strips of a ragged width count their missing columns)
+    unsigned strip_w, strips;
+    Divisor by_fast, by_strip_w, by_height, by_strips, by_rows, by_cols;
+    int staged_rows, staged_cols;  // input rows of a map and columns of a strip with their border
+    int chunks;                    // 16 * CS channels each
+    int table_b, buffer_b;         // bytes of the tables in front of the staged pixels, and of a buffer of those
+    float floor, post_floor;       // `plain`: what the activation and the ReLU behind the shortcut cut off at, -inf: nothing
+    int plain;                     // results are rows that take 16-byte accesses, and nothing but ReLUs and a shortcut lie behind the products
+};
+
+// Two values' thirds, as pairs of bfloat16.
+__device__ __forceinline__ unsigned bf16_pair(float a, float b) { return __builtin_bit_cast(unsigned, __builtin_convertvector(v2f{a, b}, v2bf)); }
+__device__ __forceinline__ void split_thirds(v4f x, v2u& h, v2u& m, v2u& l) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        float a = x[2 * i], b = x[2 * i + 1];
+        h[i] = bf16_pair(a, b);
+        a -= __uint_as_float(h[i] << 16);
+        b -= __uint_as_float(h[i] & 0xffff0000u);
+        m[i] = bf16_pair(a, b);
+        a -= __uint_as_float(m[i] << 16);
+        b -= __uint_as_float(m[i] & 0xffff0000u);
+        l[i] = bf16_pair(a, b);
+    }
+}
+
+// The pixel at a place of the list: its number in the output (p.pixels or more: none), its row of all staged ones and its column of the strip.
+struct Where {
+    unsigned pix;
+    int row, x;
+};
+__device__ __forceinline__ Where where(const ThirdsParams& p, unsigned at) {
+    const unsigned in = at < p.total ? at : p.total - 1, row = p.by_strip_w(in), map = p.by_height(row), img = p.by_strips(map);
+    const unsigned col = in - row * p.strip_w, y = row - map * (unsigned)p.f.out_h, x = (map - img * p.strips) * p.strip_w + col;
+    Where w;
+    w.row = (int)(map * (unsigned)p.staged_rows + y);
+    w.x = (int)col;
+    w.pix = at < p.total && x < (unsigned)p.f.out_w ? (img * (unsigned)p.f.out_h + y) * (unsigned)p.f.out_w + x : 0xffffffffu;
+    return w;
+}
+
+// Four channels from ch0 on of one pixel with float32 products: for results whose thirds met an infinity or a NaN. Slow.
+__device__ __forceinline__ v4f exact_products(const F32Params& p, unsigned pix, int ch0) {
+    const unsigned per_image = (unsigned)(p.out_h * p.out_w);
+    const bool in = pix < p.pixels;
+    const unsigned img = in ? exhip_divide(pix, per_image, p.image_magic, p.image_shift) : 0, rem = in ? pix - img * per_image : 0;
+    const int oy = (int)exhip_divide(rem, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = (int)rem - oy * p.out_w;
+    v4f v = {0.f, 0.f, 0.f, 0.f};
+    const __bf16* const w = reinterpret_cast<const __bf16*>(p.wp);
+#pragma unroll 1
+    for (int tap = 0; tap < 9; ++tap) {
+        const int iy = oy - p.pad_t + tap / 3, ix = ox - p.pad_l + tap % 3;
+        const bool inside = in && (unsigned)iy < (unsigned)p.in_h && (unsigned)ix < (unsigned)p.in_w;
+        const float* const src = reinterpret_cast<const float*>(p.x) + (size_t)((img * (unsigned)p.in_h + iy) * (unsigned)p.in_w + ix) * (unsigned)(p.xs_b / 4);
+#pragma unroll 1
+        for (int c = 0; c < p.csteps * 16; ++c) {
+            const float xv = inside ? src[c] : 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int ch = ch0 + e;
+                if (ch < p.K) {
+                    const int rr = (ch % 16 / 4) * 8 + (ch / 16 % 2) * 4 + ch % 4;
+                    const __bf16* const at = w + (size_t)(unsigned)(ch / 32 * p.csteps + c / 16) * (kStepBytes / 2) + tap * (kTapBytes / 2) +
+                                             ((c / 8 % 2) * 32 + rr) * 8 + c % 8;
+                    v[e] = __builtin_fmaf((float)at[0] + ((float)at[512] + (float)at[1024]), xv, v[e]);
+                }
+            }
+        }
+    }
+    return v;
+}
+
+// A wave's tile is 32 * MT channels x 32 * NT pixels; WP waves side by side make a group's run of pixels, WK share the steps of 16 channels,
+// of which CS are staged at a time.
+template <int MT, int NT, int WK, int WP, int CS, int OCC, bool SLOW>
+__global__ __launch_bounds__(64 * WK * WP, OCC) void conv3x3_thirds_kernel(const ThirdsParams q) {
+    exhip_touch_args(q);
+    const F32Params& p = q.f;
+    constexpr int WAVES = WK * WP, THREADS = 64 * WAVES, BLOCKS = MT * NT, RUN = 32 * NT * WP;
+    constexpr int PIECES = CS * 4, PASS = THREADS / PIECES;       // 16-byte pieces of a staged pixel; pixels that a pass of the group stages
+    constexpr int PITCH = CS * 96 + 16;                           // bytes of a staged pixel: [step][third][16 channels], an odd number of 16s
+    constexpr int BATCH = (RUN * 7 / 4 * WK / CS + PASS - 1) / PASS;  // passes whose pixels are on the way at a time
+    constexpr int PER_TAP = (BATCH + 5) / 6;                      // of them are put in place under the products of a tap
+    static_assert(CS % WK == 0, "every wave has its steps of a chunk");
+    extern __shared__ __attribute__((aligned(16))) char lds_all[];
+    unsigned* const pixels = reinterpret_cast<unsigned*>(lds_all);   // the run's pixels in the output
+    float* const params = reinterpret_cast<float*>(pixels + RUN);    // kParams of the tile's channels
+    unsigned* const table = pixels + RUN + kParams * MT * 32;        // where the staged pixels lie in the input
+    char* const stage = lds_all + q.table_b;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = lane >> 5;
+    const int part = wave % WK, side = wave / WK;
+    unsigned bid = blockIdx.x;
+    {
+        const unsigned per = gridDim.x >> 3;  // one contiguous run of items per XCD (conv_f32_kernel)
+        if (bid < (per << 3)) bid = (bid & 7) * per + (bid >> 3);
+    }
+    const unsigned slow = q.by_fast(bid), fast = bid - slow * p.fast;
+    const unsigned tile = __builtin_amdgcn_readfirstlane(p.tiles_fast ? fast : slow);
+    const int kb0 = __builtin_amdgcn_readfirstlane((int)(p.tiles_fast ? slow : fast) * MT);
+
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.x), 0, (int)p.x_bytes, kRsrcWord3);
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.wp), 0, (int)p.w_bytes, kRsrcWord3);
+
+    // weights: the wave's steps part, part + WK ..., nine taps each
+    unsigned woff[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) woff[m] = (kb0 + m) * 32 < p.K && part < p.csteps ? (unsigned)(m * p.csteps * kStepBytes + lane * 16) : kOutOfRange;
+    v8bf a[3][MT][3];
+    int w_at = (kb0 * p.csteps + part) * kStepBytes;
+    auto request = [&](int u, int at) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int t = 0; t < 3; ++t) a[u][m][t] = __builtin_bit_cast(v8bf, load4(wr, woff[m], at + t * 1024));
+    };
+
+    // the staged rows: those under the run's first pixel to those under its last
+    const unsigned run0 = tile * RUN;
+    const int first_row = __builtin_amdgcn_readfirstlane(where(q, run0).row), last_row = __builtin_amdgcn_readfirstlane(where(q, run0 + RUN - 1).row) + 2;
+    const int staged = (last_row - first_row + 1) * q.staged_cols;
+    for (int i = threadIdx.x; i < staged; i += THREADS) {
+        const unsigned r = q.by_cols((unsigned)i), row = (unsigned)first_row + r, map = q.by_rows(row), img = q.by_strips(map);
+        const int c = i - (int)r * q.staged_cols;
+        const int y = (int)(row - map * (unsigned)q.staged_rows) - p.pad_t, x = (int)((map - img * q.strips) * q.strip_w) + c - p.pad_l;
+        const bool in = (unsigned)y < (unsigned)p.in_h && (unsigned)x < (unsigned)p.in_w;
+        table[i] = in ? ((img * (unsigned)p.in_h + (unsigned)y) * (unsigned)p.in_w + (unsigned)x) * (unsigned)p.xs_b : kOutOfRange;
+    }
+    __syncthreads();
+    v4f x[BATCH];
+    const int my_piece = threadIdx.x % PIECES, my_pixel = threadIdx.x / PIECES;
+    auto load_batch = [&](int first, int chunk) {
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) {
+            const int at = first + i * PASS + my_pixel;
+            x[i] = load4(xr, at < staged ? table[at] + my_piece * 16 : kOutOfRange, chunk * CS * 64);
+        }
+    };
+    char* const my_stage = stage + (my_piece / 4) * 96 + (my_piece % 4) * 8;
+    auto store_pass = [&](const v4f& from, int first, int buffer) {  // without a branch: what is no pixel goes behind the last one
+        v2u h, m, l;
+        split_thirds(from, h, m, l);
+        const int at = first + my_pixel;
+        char* const to = my_stage + buffer + (at < staged ? at : staged) * PITCH;
+        *reinterpret_cast<v2u*>(to) = h;
+        *reinterpret_cast<v2u*>(to + 32) = m;
+        *reinterpret_cast<v2u*>(to + 64) = l;
+    };
+    load_batch(0, 0);
+#pragma unroll
+    for (int u = 0; u < 3; ++u) request(u, w_at + u * kTapBytes);
+    float par[kParams] = {};
+    {
+        const unsigned ch = (unsigned)(kb0 * 32 + lane);
+        const float* const from[kParams] = {p.bias, p.slope, p.bn_a, p.bn_b};
+#pragma unroll
+        for (int i = 0; i < kParams; ++i)
+            if (from[i]) {
+                const bool shared = i == 1 && p.slope_shared;
+                const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(from[i]), 0, shared ? 4 : p.K * 4, kRsrcWord3);
+                par[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, shared ? 0 : (int)ch * 4, 0, 0));
+            }
+    }
+    // the wave's pixels: their place in the staged rows, and in the output
+    const char* b_at[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        const int at = (side * NT + n) * 32 + (lane & 31);
+        const Where w = where(q, run0 + at);
+        if (part == 0) pixels[at] = w.pix;
+        b_at[n] = stage + ((w.row - first_row) * q.staged_cols + w.x) * PITCH + half * 16;
+    }
+    const int tap_row = q.staged_cols * PITCH;
+    v16f acc[MT][NT], low[MT][NT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[m][n][e] = low[m][n][e] = 0.f;
+    auto product = [&](int u, const v8bf (&b)[NT][3], int ta, int tb, v16f (&to)[MT][NT]) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int n = 0; n < NT; ++n) to[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[u][m][ta], b[n][tb], to[m][n], 0, 0, 0);
+    };
+    for (int first = 0;;) {
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i)
+            if (first + i * PASS < staged) store_pass(x[i], first + i * PASS, 0);
+        first += BATCH * PASS;
+        if (first >= staged) break;
+        load_batch(first, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < kParams; ++i)
+        if (lane < MT * 32) params[i * MT * 32 + lane] = par[i];  // (every wave the same)
+    __syncthreads();
+
+    // A chunk's products; NEXT: and under those of each of its steps a batch of the next chunk's pixels on their way into the other buffer.
+    int step = part, here = 0;
+    auto products = [&](int chunk, auto next) {
+        constexpr bool NEXT = decltype(next)::value;
+#pragma unroll 1
+        for (int s = part; s < CS && (NEXT || step < p.csteps); s += WK, step += WK) {
+            const bool more = NEXT || step + WK < p.csteps;
+            const int first = s / WK * (BATCH * PASS);
+            if constexpr (NEXT) load_batch(first, chunk + 1);
+            v8bf b[3][NT][3];
+            auto fetch = [&](v8bf (&to)[NT][3], int at) {
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+#pragma unroll
+                    for (int t = 0; t < 3; ++t) to[n][t] = *reinterpret_cast<const v8bf*>(b_at[n] + at + t * 32);
+            };
+            auto tap = [&](int u, const v8bf (&now)[NT][3], int w_next) {
+                product(u, now, 2, 0, low);
+                product(u, now, 0, 2, low);
+                product(u, now, 1, 1, low);
+                product(u, now, 1, 0, low);
+                product(u, now, 0, 1, low);
+                product(u, now, 0, 0, acc);
+                request(u, w_next);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            auto next_step = [&]() {  // what is requested from here on belongs to the next step
+                w_at += WK * kStepBytes;
+#pragma unroll
+                for (int m = 0; m < MT; ++m) woff[m] = more ? woff[m] : kOutOfRange;
+            };
+            int row_at = here + s * 96;
+            fetch(b[0], row_at);
+            if constexpr (NEXT) {
+#pragma unroll
+                for (int i = 0; i < 9; ++i) {
+                    if (i < 8) fetch(b[(i + 1) % 3], row_at + (i + 1) / 3 * tap_row + (i + 1) % 3 * PITCH);
+                    __builtin_amdgcn_sched_barrier(0);  // (the reads would sink to the next tap's first product)
+                    if (i == 6) next_step();
+                    if (i >= 3) {
+#pragma unroll
+                        for (int k = (i - 3) * PER_TAP; k < (i - 2) * PER_TAP && k < BATCH; ++k) store_pass(x[k], first + k * PASS, q.buffer_b - here);
+                    }
+                    tap(i % 3, b[i % 3], w_at + (i < 6 ? i + 3 : i - 6) * kTapBytes);
+                }
+            } else {  // the last chunk, often the only one: a filter row at a time, since no cache has seen a launch's code yet
+#pragma unroll 1
+                for (int r = 0; r < 3; ++r) {
+                    int w_next = w_at + (r + 1) * (3 * kTapBytes), row_next = row_at + tap_row;
+                    if (r == 2) {
+                        next_step();
+                        w_next = w_at;
+                        row_next = row_at;  // (what is read there is not used)
+                    }
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+                        fetch(b[(c + 1) % 3], c == 2 ? row_next : row_at + (c + 1) * PITCH);
+                        __builtin_amdgcn_sched_barrier(0);
+                        tap(c, b[c], w_next + c * kTapBytes);
+                    }
+                    row_at = row_next;
+                }
+            }
+        }
+    };
+#pragma unroll 1
+    for (int chunk = 0; chunk + 1 < q.chunks; ++chunk) {
+        products(chunk, std::true_type{});
+        for (int first = CS / WK * (BATCH * PASS); first < staged; first += BATCH * PASS) {
+            load_batch(first, chunk + 1);
+#pragma unroll
+            for (int i = 0; i < BATCH; ++i)
+                if (first + i * PASS < staged) store_pass(x[i], first + i * PASS, q.buffer_b - here);
+        }
+        here = q.buffer_b - here;
+        __syncthreads();
+    }
+    products(q.chunks - 1, std::false_type{});
+
+    // The waves' sums meet where the pixels were staged, [part][block][four channels][pixel]; a thread finishes four channels of one pixel
+    // at a time. Eight neighbouring lanes have a pixel's 32 channels, whose 128 bytes they store together, or for a planar result 32
+    // neighbouring lanes the pixels of a channel. Pixels are dealt out by their channels' number, so that neither side meets bank conflicts.
+    constexpr int UNITS = BLOCKS * 4 >= WK ? BLOCKS * 4 / WK : 1;
+    const bool owner = BLOCKS * 4 >= WK || part < BLOCKS * 4;
+    auto place = [&](int u, int& block, int& quad, int& row) {
+        const int at = (part * 64 + lane + u * WK * 64) % (BLOCKS * 256);
+        quad = p.y_nchw ? at >> 5 & 7 : at & 7;
+        row = p.y_nchw ? at & 31 : at >> 3 & 31;
+        block = at >> 8;
+    };
+    v4f res[UNITS];
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) res[u] = v4f{0.f, 0.f, 0.f, 0.f};
+    if (p.residual) {
+#pragma unroll
+        for (int u = 0; u < UNITS; ++u) {
+            int block, quad, row;
+            place(u, block, quad, row);
+            const int ch = (kb0 + block % MT) * 32 + quad * 4;
+            unsigned from = pixels[(side * NT + block / MT) * 32 + row];
+            if (from >= p.pixels || ch >= p.K) continue;
+            if (p.res_shift) {
+                const unsigned per_image = (unsigned)(p.out_h * p.out_w), img = exhip_divide(from, per_image, p.image_magic, p.image_shift);
+                const unsigned in_image = from - img * per_image, oy = exhip_divide(in_image, (unsigned)p.out_w, p.width_magic, p.width_shift);
+                from = (img * ((unsigned)p.out_h >> p.res_shift) + (oy >> p.res_shift)) * ((unsigned)p.out_w >> p.res_shift) +
+                       ((in_image - oy * (unsigned)p.out_w) >> p.res_shift);
+            }
+            const float* const src = p.residual + (size_t)from * (unsigned)p.rstride + ch;
+            if (p.vector_rows) {
+                res[u] = *reinterpret_cast<const v4f*>(src);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) res[u][e] = ch + e < p.K ? src[e] : 0.f;
+            }
+        }
+    }
+    __syncthreads();  // the staged pixels are no longer read
+    char* const red = stage + side * (WK * BLOCKS * 4096);
+#pragma unroll
+    for (int i = 0; i < 4 * BLOCKS; ++i) {
+        const v16f &c = acc[i / 4 % MT][i / 4 / MT], &d = low[i / 4 % MT][i / 4 / MT];
+        const int quad = half * 4 + i % 4;
+        v4f sum;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[e] = c[i % 4 * 4 + e] + d[i % 4 * 4 + e];
+        *reinterpret_cast<v4f*>(red + part * BLOCKS * 4096 + (i / 4 * 8 + quad) * 512 + ((lane & 31) ^ quad) * 16) = sum;
+    }
+    // The loads are waited for here. In the loop below the wait would take its own stores along: one counter counts both, and a unit would
+    // last 1000 cycles.
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) asm volatile("" : "+v"(res[u]));
+    __syncthreads();
+    if (!owner) return;
+#pragma unroll 1
+    for (int u = 0; u < UNITS; ++u) {
+        struct {
+            unsigned pix;
+            int block, quad, row;
+            v4f res;
+        } now;
+        place(u, now.block, now.quad, now.row);
+        now.pix = pixels[(side * NT + now.block / MT) * 32 + now.row];
+        now.res = res[0];
+        if (p.residual) {
+#pragma unroll
+            for (int i = 1; i < UNITS; ++i) now.res = u == i ? res[i] : now.res;
+        }
+        const char* const from = red + (now.block * 8 + now.quad) * 512 + (now.row ^ now.quad) * 16;
+        const float* const my_params = params + now.block % MT * 32 + now.quad * 4;
+        const int ch = (kb0 + now.block % MT) * 32 + now.quad * 4;
+        v4f sum = *reinterpret_cast<const v4f*>(from);
+#pragma unroll
+        for (int w = 1; w < WK; ++w) sum += *reinterpret_cast<const v4f*>(from + w * BLOCKS * 4096);
+        const float t = __builtin_fmaf(sum[3], 0.f, __builtin_fmaf(sum[2], 0.f, __builtin_fmaf(sum[1], 0.f, sum[0] * 0.f)));
+        if (__builtin_expect(__any(!(t == 0.f)), 0)) {  // (0 unless a value is infinite or NaN)
+            const v4f exact = exact_products(p, now.pix, ch);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum[e] = sum[e] * 0.f == 0.f ? sum[e] : exact[e];
+        }
+        if (q.plain) {
+            const v4f bias = *reinterpret_cast<const v4f*>(my_params);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float v = sum[e] + bias[e];
+                v = q.floor > v ? q.floor : v;
+                if (p.residual) v += now.res[e];
+                v = q.post_floor > v ? q.post_floor : v;
+                sum[e] = ch + e < p.K ? v : 0.f;  // pad channels hold zeros
+            }
+            if (now.pix < p.pixels && ch < p.k_end) *reinterpret_cast<v4f*>(p.y + (size_t)now.pix * (unsigned)p.kstride + ch) = sum;
+        } else {
+            float v[4], par[kParams][4], res[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[e] = sum[e];
+                res[e] = now.res[e];
+#pragma unroll
+                for (int i = 0; i < kParams; ++i) par[i][e] = my_params[i * MT * 32 + e];
+            }
+            const unsigned per_image = (unsigned)(p.out_h * p.out_w);
+            unsigned img = 0, in_image = 0;
+            if (p.y_nchw || p.layout != EXHIP_PLACE_ROWS) {
+                img = exhip_divide(now.pix, per_image, p.image_magic, p.image_shift);
+                in_image = now.pix - img * per_image;
+            }
+            epilogue_part<4, SLOW>(p, v, par, res, now.pix, img, in_image, ch);
+        }
+    }
+}
+
+std::mutex g_attr_mutex;
+
+// A launch's strips and form.
+struct Plan {
+    int form = -1;
+    unsigned width = 0, strips = 0;
+    int staged = 0;  // pixels that a group stages at most
+    long long tiles = 0;
+};
+
+// The strips for runs of `run` pixels: of all widths that split the map evenly the one whose groups, weighed with what they stage, are least,
+// among those of at most `most` staged pixels where there are any.
+void choose_strips(const F32Params& p, long long images, int run, int most, Plan* plan) {
+    double best_cost = 0;
+    for (int width = p.out_w;;) {
+        const int count = (p.out_w + width - 1) / width;
+        width = (p.out_w + count - 1) / count;  // the narrowest of that many
+        const long long tiles = ((long long)count * width * p.out_h * images + run - 1) / run;
+        // rows that a run touches beside its first, maps that it enters beside its first, and their rows and columns with the border
+        const int rows = run % width == 0 ? run / width - 1 : (run + width - 2) / width;
+        const int crossed = (int)std::min<long long>((rows + p.out_h - 1) / p.out_h, images * count - 1);
+        const int staged = (rows + 2 * crossed + 3) * (width + 2);
+        const double cost = (staged > most ? 1e18 * staged : 0.) + (double)tiles * (run + 0.2 * staged);
+        if (plan->width == 0 || cost < best_cost) {
+            plan->width = (unsigned)width;
+            plan->strips = (unsigned)count;
+            plan->staged = staged;
+            plan->tiles = tiles;
+            best_cost = cost;
+        }
+        if (width <= 4 && (width == 1 || plan->staged <= most)) break;
+        --width;
+    }
+}
+
+constexpr int kForms = 5;
+struct Shape {
+    int mt, nt, wk, wp, cs, occ;  // conv3x3_thirds_kernel's template arguments
+};
+constexpr Shape kForm[kForms] = {{1, 1, 4, 1, 4, 3}, {1, 1, 8, 1, 8, 2}, {1, 1, 2, 2, 2, 3}, {1, 1, 1, 4, 1, 3}, {2, 1, 2, 2, 2, 2}};
+
+struct Sizes {
+    int run, pitch, waves;
+    explicit Sizes(const Shape& f) : run(32 * f.nt * f.wp), pitch(f.cs * 96 + 16), waves(f.wk * f.wp), f_(f) {}
+    int table_bytes(int staged) const { return ((run + kParams * f_.mt * 32 + staged) * 4 + 15) / 16 * 16; }
+    int lds(int staged, int buffers) const { return table_bytes(staged) + std::max((staged + 1) * pitch * buffers, waves * f_.mt * f_.nt * 4096); }
+    // staged pixels with which as many groups share a CU as its registers allow
+    int most(int buffers) const { return (kLdsLimit / std::max(f_.occ * 4 / waves, 1) - table_bytes(0) - 16 - pitch * buffers) / (pitch * buffers + 4); }
+
+private:
+    const Shape f_;
+};
+
+// The form that a model of the launch says is shortest, in microseconds: 2.5 for the launch; per round of groups on 256 CUs 1.5 for a group's
+// start, 0.2 for every four channels of a pixel that a thread finishes and 0.09 for every chunk; the products at 0.021 each, all of a SIMD's or
+// a group's where it is alone; or the weights at 14.6 TB/s where that is longer. Its constants are fitted to 83 layers from 1 x 11 x 11 to 37
+// GFLOP in these forms (11 % off on average); its choice is 2 % slower than the fastest on average, and 1.49 times as fast as the float32
+// products (conv_f32_kernel), which no more than noise beats anywhere. Wave tiles of 64 x 64, 32 x 64 and eight waves to 64 x 32 or 64 x 64 are
+// within 3 % of these or slower on all of the layers but four.
+int choose_form(const F32Params& p, long long pixels, int kblocks) {
+    int best = 0;
+    double best_cost = 0;
+    for (int i = 0; i < kForms; ++i) {
+        const Shape& f = kForm[i];
+        const int waves = f.wk * f.wp, blocks = f.mt * f.nt, steps = (p.csteps + f.wk - 1) / f.wk, units = std::max(1, blocks * 4 / f.wk);
+        const int resident = std::max(1, f.occ * 4 / waves), slots = waves > 4 ? 240 : 256;  // (256 groups of eight waves took a second round)
+        const long long items = (pixels + 32 * f.nt * f.wp - 1) / (32 * f.nt * f.wp) * ((kblocks + f.mt - 1) / f.mt), each = (items + slots - 1) / slots;
+        const double products = steps * 9 * blocks * 6 * 0.0212, rounds = (double)((each + resident - 1) / resident);
+        const double time = rounds * (1.5 + 0.2 * units + 0.09 * ((p.csteps + f.cs - 1) / f.cs - 1)) + std::max(each * (waves / 4) * products, rounds * products);
+        const double cost = std::max(time, (double)items * f.mt * p.csteps * kStepBytes / 14.6e6);
+        if (i == 0 || cost < best_cost) {
+            best_cost = cost;
+            best = i;
+        }
+    }
+    return best;
+}
+
+// A thread keeps the plans of its last layers: the search is 1 to 2 us, half of what a launch costs the host.
+const Plan& plan_of(const F32Params& p, long long images, int kblocks, int tile) {
+    struct Entry {
+        long long images = -1;
+        int h, w, csteps, kblocks, tile;
+        Plan plan;
+    };
+    static thread_local Entry cache[64];
+    Entry& e = cache[(unsigned)(p.out_h * 31 + p.out_w * 7 + p.csteps * 5 + kblocks * 3 + (int)images) % 64];
+    if (e.images != images || e.h != p.out_h || e.w != p.out_w || e.csteps != p.csteps || e.kblocks != kblocks || e.tile != tile) {
+        e = Entry();
+        e.h = p.out_h; e.w = p.out_w; e.csteps = p.csteps; e.kblocks = kblocks; e.tile = tile;
+        for (int form = tile > 0 ? std::min(tile, kForms) - 1 : choose_form(p, (long long)p.out_h * p.out_w * images, kblocks);; form = 0) {
+            const Sizes s(kForm[form]);
+            const int buffers = p.csteps > kForm[form].cs ? 2 : 1;
+            e.plan = Plan();
+            e.plan.form = form;
+            choose_strips(p, images, s.run, s.most(buffers), &e.plan);
+            // maps of a few pixels stage up to nine for each; the first form has room for nine times its 32 pixels
+            if (form == 0 || s.lds(e.plan.staged, buffers) <= kLdsLimit) break;
+        }
+        e.images = images;
+    }
+    return e.plan;
+}
+
+template <int FORM, bool SLOW>
+int go(exhip_ctx* ctx, ThirdsParams& q, const Plan& plan, long long images, int kblocks) {
+    constexpr Shape f = kForm[FORM];
+    const Sizes s(f);
+    F32Params& p = q.f;
+    q.chunks = (p.csteps + f.cs - 1) / f.cs;
+    const int lds = s.lds(plan.staged, q.chunks > 1 ? 2 : 1);
+    EXHIP_REQUIRE(lds <= kLdsLimit, "conv: %d pixels to stage", plan.staged);
+    q.strip_w = plan.width;
+    q.strips = plan.strips;
+    q.total = (unsigned)((long long)plan.width * plan.strips * p.out_h * images);
+    q.staged_rows = p.out_h + 2;
+    q.staged_cols = (int)plan.width + 2;
+    q.by_strip_w.set(plan.width);
+    q.by_strips.set(plan.strips);
+    q.by_height.set((unsigned)p.out_h);
+    q.by_rows.set((unsigned)q.staged_rows);
+    q.by_cols.set((unsigned)q.staged_cols);
+    q.table_b = s.table_bytes(plan.staged);
+    q.buffer_b = (plan.staged + 1) * s.pitch;
+    const long long groups = (kblocks + f.mt - 1) / f.mt, items = plan.tiles * groups;
+    EXHIP_REQUIRE(items < (1ll << 31) - 4, "conv: grid too large");
+    p.items = (unsigned)items;
+    p.tiles_fast = p.w_bytes > (4u << 20) && p.w_bytes > p.x_bytes;  // (conv_f32_kernel)
+    p.fast = (unsigned)(p.tiles_fast ? plan.tiles : groups);
+    q.by_fast.set(p.fast);
+    auto kernel = conv3x3_thirds_kernel<f.mt, f.nt, f.wk, f.wp, f.cs, f.occ, SLOW>;
+    {
+        static unsigned long long attr_set = 0;
+        std::lock_guard<std::mutex> lock(g_attr_mutex);
+        const unsigned long long bit = 1ull << (ctx->device & 63);
+        if (!(attr_set & bit)) {
+            EXHIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsLimit));
+            attr_set |= bit;
+        }
+    }
+    hipLaunchKernelGGL(kernel, dim3(p.items), dim3(64 * f.wk * f.wp), lds, ctx->stream, q);
+    EXHIP_LAUNCH_CHECK();
+    return 0;
+}
+
+// The thirds of 72 weights, eight channels' nine taps: [third][tap][channel]. Whole vectors where all of them are finite and none rounds up to an infinity.
+__attribute__((always_inline)) inline bool split_finite(const float* src, uint16_t (*out)[72]) {
+    float v[72];
+    unsigned u[72];
+    for (int i = 0; i < 8; ++i)
+        for (int tap = 0; tap < 9; ++tap) v[tap * 8 + i] = src[i * 9 + tap];
+    memcpy(u, v, sizeof(u));
+    unsigned high = 0;
+    for (int i = 0; i < 72; ++i) high |= (u[i] & 0x7fffffffu) + 0x808000u;  // the sign bit from 0x7f7f8000 on
+    if (high & 0x80000000u) return false;
+    for (int t = 0; t < 3; ++t) {
+        for (int i = 0; i < 72; ++i) {
+            unsigned b;
+            float f;
+            memcpy(&b, v + i, 4);
+            b = (b + 0x7fffu + (b >> 16 & 1)) & 0xffff0000u;  // to the nearest, ties to even
+            memcpy(&f, &b, 4);
+            out[t][i] = (uint16_t)(b >> 16);
+            v[i] -= f;
+        }
+    }
+    return true;
+}
+
+void split_weights(const float* src, uint16_t (*out)[72]) {
+    for (int tap = 0; tap < 9; ++tap)
+        for (int c = 0; c < 8; ++c) {  // an infinity or NaN is its own first third; what would round up to an infinity is cut off
+            float x = src[c * 9 + tap];
+            for (int t = 0; t < 3; ++t) {
+                unsigned b;
+                memcpy(&b, &x, 4);
+                const bool finite = (b & 0x7f800000u) != 0x7f800000u;
+                const unsigned r = b + 0x7fffu + (b >> 16 & 1);
+                const unsigned third = finite && (r & 0x7f800000u) != 0x7f800000u ? r >> 16 : b >> 16 | (!finite && (b & 0x7fffffu) ? 0x40u : 0u);
+                out[t][tap * 8 + c] = (uint16_t)third;
+                const unsigned back = third << 16;
+                float f;
+                memcpy(&f, &back, 4);
+                x = finite ? x - f : 0.f;
+            }
+        }
+}
+
+// One step's weights of a 32-channel block.
+__attribute__((always_inline)) inline void pack_step(const float* w, int C, int K, int kb, int j, char* to) {
+    for (int lane = 0; lane < 64; ++lane) {
+        const int rr = lane % 32, k = kb * 32 + (rr / 4 % 2) * 16 + rr / 8 * 4 + rr % 4;
+        uint16_t thirds[3][72];
+        if (k >= K) memset(thirds, 0, sizeof(thirds));
+        else if (const float* const src = w + ((size_t)k * C + j * 16 + lane / 32 * 8) * 9; !split_finite(src, thirds)) split_weights(src, thirds);
+        for (int tap = 0; tap < 9; ++tap)
+            for (int t = 0; t < 3; ++t) memcpy(to + (tap * 3 + t) * 1024 + lane * 16, thirds[t] + tap * 8, 16);
+    }
+}
+#ifndef __HIP_DEVICE_COMPILE__
+__attribute__((target("avx2"))) void pack_step_avx2(const float* w, int C, int K, int kb, int j, char* to) { pack_step(w, C, K, kb, j, to); }
+#endif
+void pack_step_any(const float* w, int C, int K, int kb, int j, char* to) { pack_step(w, C, K, kb, j, to); }
+
+}  // namespace
+
+bool exhip_conv_f32_thirds(const exhip_conv_desc* d) {
+    return d->kh == 3 && d->kw == 3 && d->sh == 1 && d->c % 16 == 0 && (long long)((d->k + 31) / 32) * (d->c / 16) * kStepBytes < (1ll << 31);
+}
+
+size_t exhip_conv_f32_thirds_bytes(const exhip_conv_desc* d) { return (size_t)((d->k + 31) / 32) * (d->c / 16) * kStepBytes; }
+
+// [32-channel block][16 channels][tap][third][lane][8 bfloat16]: lane rr of either half has the output channel that conv_f32.hip's packing gives
+// it, and eight neighbouring input channels. Large layers are dealt out to a few threads: 512 -> 512 takes one of them 2.4 ms, four 1.1 (whole floats, one: 1.5).
+void exhip_conv_f32_thirds_pack(const exhip_conv_desc* d, const float* w, void* out) {
+    const int C = d->c, K = d->k, steps = C / 16, blocks = (K + 31) / 32;
+    auto step = pack_step_any;
+#ifndef __HIP_DEVICE_COMPILE__
+    if (__builtin_cpu_supports("avx2")) step = pack_step_avx2;
+#endif
+    auto pack = [=](int first, int last) {
+        for (int kb = first; kb < last; ++kb)
+            for (int j = 0; j < steps; ++j) step(w, C, K, kb, j, static_cast<char*>(out) + (size_t)(kb * steps + j) * kStepBytes);
+    };
+    const unsigned cores = std::thread::hardware_concurrency();
+    const int most = (int)std::min<unsigned>(8, std::max(1u, cores / 2)), threads = std::min({most, blocks, (int)((long long)C * K / 65536) + 1});
+    std::thread crew[8];
+    int started = 1;
+    try {
+        for (; started < threads; ++started) crew[started] = std::thread(pack, blocks * started / threads, blocks * (started + 1) / threads);
+    } catch (...) {  // the process may have no more threads: this one does the rest
+    }
+    pack(0, blocks / threads);
+    if (started < threads) pack(blocks * started / threads, blocks);
+    for (int t = 1; t < started; ++t) crew[t].join();
+}
+
+int exhip_conv_f32_thirds_run(exhip_ctx* ctx, const F32Launch& launch) {
+    ThirdsParams q = {};
+    q.f = *static_cast<const F32Params*>(launch.params);
+    F32Params& p = q.f;
+    q.plain = p.y && !p.y_nchw && p.layout == EXHIP_PLACE_ROWS && p.vector_rows && p.act <= 1 && !p.bn_a && !p.post_op && !(p.residual && p.residual_last);
+    q.floor = p.act == 1 ? 0.f : -INFINITY;
+    q.post_floor = p.post_relu ? 0.f : -INFINITY;
+    const bool slow = p.act == 4 || p.act == 5;
+    const Plan plan = plan_of(p, launch.images, launch.blocks, slow ? 1 : g_exhip_options.f32_tile);
+    switch (plan.form) {
+    case 0: return slow ? go<0, true>(ctx, q, plan, launch.images, launch.blocks) : go<0, false>(ctx, q, plan, launch.images, launch.blocks);
+    case 1: return go<1, false>(ctx, q, plan, launch.images, launch.blocks);
+    case 2: return go<2, false>(ctx, q, plan, launch.images, launch.blocks);
+    case 3: return go<3, false>(ctx, q, plan, launch.images, launch.blocks);
+    default: return go<4, false>(ctx, q, plan, launch.images, launch.blocks);
+    }
+}

@@ -399,7 +399,8 @@ const void* operation_convolution<Dtype>::packed_weights(int dtype, const exhip_
     }
     const size_t bytes = exhip_conv_packed_bytes(&d, dtype);
     if (bytes == 0) LOG(FATAL) << "layer " << this->params_.name_ << ": " << exhip_last_error();
-    std::vector<char> host(bytes);
+    // (not a vector, which would be filled with zeros first: the packing writes every byte)
+    const std::unique_ptr<char[]> host(new char[bytes]);
     std::vector<unsigned short> half_w;
     const void* src = nullptr;
     if (dtype == EXHIP_I8) {
@@ -413,9 +414,9 @@ const void* operation_convolution<Dtype>::packed_weights(int dtype, const exhip_
         for (int i = 0; i < this->weight_data_size_; ++i) half_w[i] = half_bits_rne(w[i]);
         src = half_w.data();
     }
-    EXHIP_FATAL(exhip_conv_pack_weights(&d, dtype, src, host.data()));
+    EXHIP_FATAL(exhip_conv_pack_weights(&d, dtype, src, host.get()));
     void* dev = memory::device_alloc(this->params_.device_, bytes);
-    EXHIP_FATAL(exhip_memcpy_h2d(this->ctx(), dev, host.data(), bytes));
+    EXHIP_FATAL(exhip_memcpy_h2d(this->ctx(), dev, host.get(), bytes));
     packed_[key] = {dev, bytes, ++packed_clock_, 0};
     return dev;
 }
