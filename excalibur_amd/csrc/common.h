@@ -103,6 +103,7 @@ struct exhip_options {
     int pw_tile = 0;         // that kernel's wave tile for more than 32 output channels: 0 = 32 pixels x 64 channels, 2 = 64 x 64 from 2048 waves on, without a pooling layer in the launch
     int f32_tile = 0;        // the float32 convolution's wave tile and split: 0 by its rule, n = the n-th of its list
     int dw_pw = 1;           // depthwise + pointwise fp16 pairs in one kernel: 1 by its rule, 2 wherever it can run, 4, 8 .. 256 so with that many pixels a group (where 40 KiB hold them), 0 never
+    int bottleneck = 1;      // pointwise + depthwise + pointwise fp16 blocks in one kernel: 1 by its rule, 16 * rows + columns of a tile (up to 15 each) wherever it can run, + 256 with eight waves a group, 0 never
     int pw_split = 1;        // that kernel's split form (several waves to a tile): 1 by its rule, 2 wherever it can run, 0 never
     int pw = 1;              // 1x1 stride-1 fp16 and int8 layers with NHWC results: 1 the pointwise kernel where it measured faster, 2 wherever it can run, 0 never
 };
@@ -129,6 +130,17 @@ inline void exhip_host_divisor(unsigned d, unsigned* magic, int* shift) {
     *magic = (unsigned)(((1ull << (31 + s)) + d - 1) / d);
     *shift = s - 1;
 }
+
+// The same without a branch (exhip_divide() tests for 1; where the code runs once, a taken branch is a line of it that no cache has seen yet).
+struct exhip_divisor {
+    unsigned magic, one;  // one: all ones for a divisor of 1, whose magic is 0
+    int shift;
+    __device__ __forceinline__ unsigned operator()(unsigned n) const { return (__umulhi(n, magic) >> shift) | (n & one); }
+    void set(unsigned d) {
+        exhip_host_divisor(d, &magic, &shift);
+        one = d == 1 ? ~0u : 0u;
+    }
+};
 
 // ---- device helpers shared by the kernels ----
 // Reads one word of every 64 bytes of a kernel's argument struct, all of them before the first wait. The arguments of a launch

@@ -41,22 +41,11 @@ constexpr int kTapBytes = 3 * 1024;          // a 32-channel block's weights of 
 constexpr int kStepBytes = 9 * kTapBytes;
 constexpr int kLdsLimit = 160 * 1024;
 
-// Division by a launch constant without a branch (exhip_divide() tests for 1; a taken branch is a line of code that no cache has seen yet).
-struct Divisor {
-    unsigned magic, one;  // one: all ones for a divisor of 1, whose magic is 0
-    int shift;
-    __device__ __forceinline__ unsigned operator()(unsigned n) const { return (__umulhi(n, magic) >> shift) | (n & one); }
-    void set(unsigned d) {
-        exhip_host_divisor(d, &magic, &shift);
-        one = d == 1 ? ~0u : 0u;
-    }
-};
-
 struct ThirdsParams {
     F32Params f;
     unsigned total;                // pixels of the list (strips of a ragged width count their missing columns)
     unsigned strip_w, strips;
-    Divisor by_fast, by_strip_w, by_height, by_strips, by_rows, by_cols;
+    exhip_divisor by_fast, by_strip_w, by_height, by_strips, by_rows, by_cols;
     int staged_rows, staged_cols;  // input rows of a map and columns of a strip with their border
     int chunks;                    // 16 * CS channels each
     int table_b, buffer_b;         // bytes of the tables in front of the staged pixels, and of a buffer of those

@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "common.h"
+#include "bottleneck.h"
 #include "conv_f32.h"
 #include "conv_i8_lean.h"
 #include "conv_pw.h"
@@ -2053,6 +2054,49 @@ extern "C" int exhip_dw_pw_f16(exhip_ctx* ctx, const exhip_depthwise_desc* dw, c
     ConvParams p = {};
     p.x = (const char*)dw->x; p.wp = (const char*)wp; p.bias = bias; p.residual = (const char*)residual; p.y_q = y;
     return run_conv<EXHIP_F16>(ctx, d, p, nullptr, nullptr, 0, &g);
+}
+
+// A pointwise layer of a block, its operands checked.
+static int bottleneck_layer(const exhip_conv_desc* d, const void* wp, const float* bias, exhip_bottleneck_layer* l) {
+    Plan pl;
+    int rc = make_plan(d, EXHIP_F16, &pl);
+    if (!rc) rc = check_operands(d, true, nullptr, wp, nullptr, bias);
+    if (rc) return rc;
+    if (d->kh != 1 || d->kw != 1 || d->sh != 1 || d->sw != 1 || d->pt || d->pb || d->pl || d->pr || d->c_stride != d->c || d->k_stride != d->k || pl.packed)
+        return EXHIP_ERR_UNSUPPORTED;
+    exhip_pw_geom g = {};
+    g.pixels = (long long)d->n * d->h * d->w; g.c_bytes = d->c * 2; g.k = d->k; g.k_stride = d->k_stride;
+    g.slab_blocks = pl.TM / 32; g.slabs = pl.ktiles;
+    g.act = d->act; g.post_relu = d->post_relu; g.post_op = d->post_op;
+    *l = {};
+    l->wp = wp; l->bias = bias; l->steps = g.c_bytes / 32; l->slab_blocks = g.slab_blocks; l->channels = d->k;
+    l->w_bytes = (long long)g.slabs * l->steps * g.slab_blocks * 1024;
+    l->runs = exhip_pw_runs_f16(g, l->start);
+    return 0;
+}
+
+extern "C" int exhip_bottleneck_f16(exhip_ctx* ctx, const exhip_conv_desc* first, const void* w_first, const float* bias_first, const exhip_depthwise_desc* dw,
+                                    const exhip_conv_desc* last, const void* w_last, const float* bias_last, const uint16_t* residual, uint16_t* y) {
+    EXHIP_REQUIRE(ctx && first && w_first && dw && dw->x && dw->w9 && last && w_last && y, "exhip_bottleneck_f16: NULL argument");
+    EXHIP_REQUIRE(first->n == dw->n && first->h == dw->h && first->w == dw->w && dw->n == last->n && dw->h > 0 && dw->w > 0 && dw->stride > 0 && dw->pt >= 0 && dw->pl >= 0 &&
+                      dw->pb >= 0 && dw->pr >= 0 && dw->h + dw->pt + dw->pb >= 3 && dw->w + dw->pl + dw->pr >= 3 && (dw->h + dw->pt + dw->pb - 3) / dw->stride + 1 == last->h &&
+                      (dw->w + dw->pl + dw->pr - 3) / dw->stride + 1 == last->w && first->k == last->c,
+                  "exhip_bottleneck_f16: the layers' maps do not fit");
+    EXHIP_REQUIRE((uintptr_t)dw->x % 16 == 0 && (uintptr_t)y % 16 == 0 && (uintptr_t)residual % 16 == 0 && (uintptr_t)dw->w9 % 16 == 0,
+                  "exhip_bottleneck_f16: tensors must be 16-byte aligned");
+    const bool prelu = first->post_op == EXHIP_POST_PRELU;
+    if (first->act > 1 || (first->post_op && !prelu) || (prelu && (first->act || first->post_relu || !first->post_slope)) || last->act || last->post_relu || last->post_op || last->residual_last || dw->pt > 2 || dw->pl > 2)
+        return EXHIP_ERR_UNSUPPORTED;
+    exhip_bottleneck b = {};
+    int rc = bottleneck_layer(first, w_first, bias_first, &b.first);
+    if (!rc) rc = bottleneck_layer(last, w_last, bias_last, &b.last);
+    if (rc) return rc;
+    b.x = dw->x; b.slope = prelu ? first->post_slope : nullptr; b.slope_shared = first->post_slope_shared; b.relu = first->act == 1 || first->post_relu;
+    b.dw_w = dw->w9; b.dw_bias = dw->bias; b.dw_slope = dw->slope; b.dw_slope_shared = dw->slope_shared; b.dw_act = dw->act;
+    b.residual = residual; b.y = y;
+    b.n = dw->n; b.in_h = dw->h; b.in_w = dw->w; b.out_h = last->h; b.out_w = last->w; b.stride = dw->stride; b.pad_t = dw->pt; b.pad_l = dw->pl;
+    b.pixel_b = first->c * 2;
+    return exhip_bottleneck_run(ctx, b);
 }
 
 extern "C" int exhip_conv2d_i8_maxpool2x2(exhip_ctx* ctx, const exhip_conv_desc* d, int pool_oh, int pool_ow, const int8_t* x, const void* wp,

@@ -60,3 +60,5 @@ int exhip_conv1x1_i8_pw(exhip_ctx* ctx, const exhip_pw_geom& g, const int8_t* x,
 // Whether that kernel takes an fp16 layer with a filter of this many output pixels, input bytes per pixel, channels and 32-byte k-steps
 // (and stride) in its split form (several waves to a tile), which is then faster than any other kernel for it.
 bool exhip_pw_splits_f16(long long pixels, int c_bytes, int k, int k_stride, int n_ksteps, int stride);
+// The runs of 32-byte k-steps that an fp16 pointwise layer's sums are made of (1: all in one), and where they begin.
+int exhip_pw_runs_f16(const exhip_pw_geom& g, int start[5]);

@@ -1691,6 +1691,13 @@ int exhip_conv_i8_stem(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_ta
     return run_stem<EXHIP_I8>(ctx, g, t, channels, p);
 }
 
+int exhip_pw_runs_f16(const exhip_pw_geom& g, int start[5]) {
+    const int n_ksteps = g.c_bytes / 32, kblocks = std::min(g.slabs * g.slab_blocks, (std::max(g.k, g.k_stride) + 31) / 32);
+    if (!split_wins(EXHIP_F16, g, kblocks, n_ksteps, false, 1)) return 1;
+    for (int i = 0; i <= kSplit; ++i) start[i] = split_start(n_ksteps, n_ksteps % 2 == 0, i);
+    return kSplit;
+}
+
 bool exhip_pw_splits_f16(long long pixels, int c_bytes, int k, int k_stride, int n_ksteps, int stride) {
     exhip_pw_geom g = {};
     g.pixels = pixels; g.c_bytes = c_bytes;

@@ -85,6 +85,9 @@ public:
     // fp16: this layer, a pointwise one, with the 3x3 depthwise layer that it alone reads in front of it in one kernel, each with
     // the layers set behind it; `bottoms` are the depthwise layer's. False, with nothing done, where the pair runs as two layers.
     bool forward_behind_depthwise(operation_convolutiondepthwise<Dtype>& dw, const tensor_list<unsigned short>& bottoms, tensor_list<unsigned short>& tops);
+    // the same with the pointwise layer `first` that the depthwise layer alone reads: a mobile network's block; `bottoms` are that layer's
+    bool forward_block(operation_convolution<Dtype>& first, operation_convolutiondepthwise<Dtype>& dw, const tensor_list<unsigned short>& bottoms,
+                       tensor_list<unsigned short>& tops);
     // fp16: this layer, of at most four input channels, straight on its NCHW input, with the Input layer that it alone reads in front of it
     // (or NULL) and the layers set behind it; `bottoms` are the first one's. False, with nothing done, where the layers run by themselves.
     bool forward_stem(operation_input<Dtype>* input, const tensor_list<unsigned short>& bottoms, tensor_list<unsigned short>& tops);

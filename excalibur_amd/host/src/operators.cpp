@@ -649,6 +649,35 @@ bool operation_convolution<Dtype>::forward_behind_depthwise(operation_convolutio
     return true;
 }
 
+template <typename Dtype>
+bool operation_convolution<Dtype>::forward_block(operation_convolution<Dtype>& first, operation_convolutiondepthwise<Dtype>& dw,
+                                                 const tensor_list<unsigned short>& bottoms, tensor_list<unsigned short>& tops) {
+    const int dev = this->params_.device_, c = first.input_channels(), wide = this->input_channels();
+    if (bottoms[0]->order() != memory::NHWC || bottoms[0]->channels() != c || first.output_channel_ != wide || dw.output_channel_ != wide || dw.group_ != wide ||
+        !dw.fast3x3() || !first.mfma_path_ok() || !mfma_path_ok() || !nhwc_allowed() || wide % 16 != 0 || this->output_channel_ % 16 != 0 || first.post_sum_ ||
+        conv_in_stride(c, EXHIP_F16, 1) != c || conv_in_stride(wide, EXHIP_F16, 1) != wide)
+        return false;
+    const int n = bottoms[0]->num(), h = bottoms[0]->height(), w = bottoms[0]->width();
+    exhip_conv_desc a = first.describe(n, h, w, c, wide);
+    if (a.kh != 1 || a.kw != 1 || a.sh != 1 || a.sw != 1 || a.pt || a.pb || a.pl || a.pr) return false;
+    const int oh = (h + dw.pad_top_ + dw.pad_bottom_ - 3) / dw.stride_h_ + 1, ow = (w + dw.pad_left_ + dw.pad_right_ - 3) / dw.stride_w_ + 1;
+    if (h + dw.pad_top_ + dw.pad_bottom_ < 3 || w + dw.pad_left_ + dw.pad_right_ < 3) return false;
+    exhip_conv_desc d = describe(n, oh, ow, wide, this->output_channel_);
+    if (d.kh != 1 || d.kw != 1 || d.sh != 1 || d.sw != 1 || d.pt || d.pb || d.pl || d.pr) return false;
+    const exhip_depthwise_desc q = {bottoms[0]->gpu_data(), dw.weights_f32_[0]->gpu_data(), dw.bias_gpu(), dw.post_slope_, dw.post_slope_shared_,
+                                    dw.activation_type_, n, h, w, dw.stride_h_, dw.pad_top_, dw.pad_bottom_, dw.pad_left_, dw.pad_right_};
+    tops[0] = new_tensor<unsigned short>({n, oh, ow, this->output_channel_}, dev, memory::NHWC);
+    const unsigned short* residual = sum_operand(tops, &d);
+    const int rc = exhip_bottleneck_f16(this->ctx(), &a, first.packed_weights(EXHIP_F16, a), first.bias_gpu(), &q, &d, packed_weights(EXHIP_F16, d), bias_gpu(),
+                                        residual, tops[0]->mutable_gpu_data());
+    if (rc == EXHIP_ERR_UNSUPPORTED) {
+        post_sum_used_ = false;
+        return false;
+    }
+    EXHIP_FATAL(rc);
+    return true;
+}
+
 // ------------------------------------------------------------------ depthwise convolution
 template <typename Dtype>
 bool operation_convolutiondepthwise<Dtype>::fast3x3() const {

@@ -235,6 +235,7 @@ public:
         find_quantized_links();
         find_sum_pairs();
         find_depthwise_pairs();
+        find_blocks();
         find_stem();
         find_heads();
         find_glue_chains();
@@ -305,6 +306,27 @@ public:
                 if (readers[mid] != own_readers || op_outputs_[last + 1].size() != 1 || op_outputs_[last + 1][0] == mid) continue;
                 if (std::find(output_names_.begin(), output_names_.end(), blob_names_[mid]) != output_names_.end()) continue;
                 behind_depthwise_[i] = static_cast<int>(last + 1);
+            }
+        }
+    }
+
+    // fp16 pipeline: a convolution (with its activation layer) whose only reader is a depthwise layer that leads such a pair: where it is a
+    // pointwise layer one kernel runs all three, and neither blob between them is stored.
+    void find_blocks() {
+        opens_block_.assign(operations_.size(), -1);
+        if constexpr (std::is_same_v<Dtype, unsigned short>) {
+            for (size_t i = 0; i + 1 < operations_.size(); ++i) {
+                auto* conv = dynamic_cast<operation_convolution<Dtype>*>(operations_[i].get());
+                if (!conv || dynamic_cast<operation_convolutiondepthwise<Dtype>*>(conv) || sum_other_[i] >= 0 || op_inputs_[i].size() != 1) continue;
+                const size_t last = pair_[i].on ? i + 1 : i;
+                if (last + 1 >= operations_.size() || behind_depthwise_[last + 1] < 0 || op_outputs_[last].size() != 1) continue;
+                const int mid = op_outputs_[last][0];
+                if (op_inputs_[last + 1] != std::vector<int>{mid} || op_outputs_[last + 1] == op_outputs_[last]) continue;
+                int readers = 0;
+                for (const auto& in : op_inputs_) readers += static_cast<int>(std::count(in.begin(), in.end(), mid));
+                if (readers != (pair_[i].on && op_outputs_[i][0] == mid ? 2 : 1) || op_inputs_[i][0] == mid) continue;  // (an activation over its input reads the blob as well)
+                if (std::find(output_names_.begin(), output_names_.end(), blob_names_[mid]) != output_names_.end()) continue;
+                opens_block_[i] = static_cast<int>(last + 1);
             }
         }
     }
@@ -582,12 +604,15 @@ private:
                 }
             }
             if constexpr (std::is_same_v<Dtype, unsigned short>) {
-                if (fusion_ && behind_depthwise_[i] >= 0) {
-                    const size_t j = behind_depthwise_[i];
-                    auto* dw = static_cast<operation_convolutiondepthwise<Dtype>*>(set_paired_activation(i));
+                const bool block = opens_block_[i] >= 0;
+                if (fusion_ && (block || behind_depthwise_[i] >= 0)) {
+                    const size_t dw_at = block ? opens_block_[i] : i, j = behind_depthwise_[dw_at];
+                    auto* first = block ? set_paired_activation(i) : nullptr;
+                    auto* dw = static_cast<operation_convolutiondepthwise<Dtype>*>(set_paired_activation(dw_at));
                     auto* conv = set_paired_activation(j);
                     if (sum_other_[j] >= 0 && featmaps_[sum_other_[j]]) conv->set_post_sum(featmaps_[sum_other_[j]], pair_[j].on);
-                    const bool ran = conv->forward_behind_depthwise(*dw, in, out), summed = conv->post_sum_used();
+                    const bool ran = block ? conv->forward_block(*first, *dw, in, out) : conv->forward_behind_depthwise(*dw, in, out), summed = conv->post_sum_used();
+                    if (first) first->clear_post();
                     dw->clear_post();
                     conv->clear_post();
                     if (ran) {
@@ -711,6 +736,7 @@ private:
         int stride = 0;
     };
     std::vector<int> sum_other_;         // per layer: the other operand's blob of the sum layer this convolution absorbs, or -1
+    std::vector<int> opens_block_;       // per layer: the depthwise layer of the block that this pointwise layer begins, or -1
     std::vector<int> behind_depthwise_;  // per layer: the pointwise layer that runs in this depthwise layer's kernel, or -1
     std::vector<char> behind_input_;     // per layer: the convolution on the next line runs in this Input layer's kernel
     std::vector<char> in_groups_;        // per layer: this convolution stores its results as the Reshape and Transpose behind it leave them

@@ -73,7 +73,8 @@ const char* exhip_last_error(void);
  * the same values. "pw_split" chooses that kernel's split form (1 by its rule, 2 wherever it can run, 0 never; fp16 sums then run
  * in another order). "dw_pw" chooses the depthwise + pointwise fp16 pairs that exhip_dw_pw_f16 takes (1 by its rule, 2 wherever it can
  * run, a power of two from 4 to 256 so with that many pixels a group where 40 KiB hold their depthwise results, 2 c + 16 bytes each, 0 never; the same
- * values). "f32_tile" pins the float32 convolution's wave tile and split (0 = its rule, n = the n-th of its list;
+ * values). "bottleneck" chooses the fp16 blocks that exhip_bottleneck_f16 takes (1 by its rule, 16 rows + columns, up to 15 each, with that tile, + 256 with
+ * eight waves a group, wherever it fits into LDS, 0 never; the same values). "f32_tile" pins the float32 convolution's wave tile and split (0 = its rule, n = the n-th of its list;
  * sums then run in another order).
  * Process-wide; packed weights depend on the first three, so set them before packing. */
 int exhip_set_option(const char* name, int value);
@@ -227,6 +228,13 @@ typedef struct exhip_depthwise_desc {
 } exhip_depthwise_desc;
 int exhip_dw_pw_f16(exhip_ctx* ctx, const exhip_depthwise_desc* dw, const exhip_conv_desc* d, const void* w_packed, const float* bias,
                     const uint16_t* residual_nhwc, uint16_t* y_nhwc);
+
+/* A mobile network's block as one launch on NHWC halves: the pointwise layer `first` (ReLU or a PReLU layer behind it, or nothing), the depthwise layer
+ * (dw->x is first's input), the pointwise layer `last` (nothing behind it) and, where `residual_nhwc` is given, the sum behind that. c_stride == c and
+ * k_stride == k of both; tensors on 16 bytes. Values are those of the layers run one after the other, bit for bit.
+ * EXHIP_ERR_UNSUPPORTED, with nothing launched, where they run by themselves. */
+int exhip_bottleneck_f16(exhip_ctx* ctx, const exhip_conv_desc* first, const void* w_first, const float* bias_first, const exhip_depthwise_desc* dw,
+                         const exhip_conv_desc* last, const void* w_last, const float* bias_last, const uint16_t* residual_nhwc, uint16_t* y_nhwc);
 
 /* exhip_conv2d_i8 and the 2x2 stride-2 max pooling behind it (operation_pooling.cpp:145-159, windows inside the map: 2 * pool_oh <= output rows) as one launch;
  * y_i8 and / or y_f32 are the pooled NHWC results. EXHIP_ERR_UNSUPPORTED, with nothing launched, where the two run by themselves. */
