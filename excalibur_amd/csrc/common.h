@@ -103,6 +103,7 @@ struct exhip_options {
     int pw_tile = 0;         // that kernel's wave tile for more than 32 output channels: 0 = 32 pixels x 64 channels, 2 = 64 x 64 from 2048 waves on, without a pooling layer in the launch
     int f32_tile = 0;        // the float32 convolution's wave tile and split: 0 by its rule, n = the n-th of its list
     int dw_pw = 1;           // depthwise + pointwise fp16 pairs in one kernel: 1 by its rule, 2 wherever it can run, 4, 8 .. 256 so with that many pixels a group (where 40 KiB hold them), 0 never
+    int staged = 1;          // 3x3 fp16 / int8 layers with their input staged in LDS: 1 by its rule, 2 to 4 wherever it can run, in the first to third of its forms, 0 never
     int bottleneck = 1;      // pointwise + depthwise + pointwise fp16 blocks in one kernel: 1 by its rule, 16 * rows + columns of a tile (up to 15 each) wherever it can run, + 256 with eight waves a group, 0 never
     int pw_split = 1;        // that kernel's split form (several waves to a tile): 1 by its rule, 2 wherever it can run, 0 never
     int pw = 1;              // 1x1 stride-1 fp16 and int8 layers with NHWC results: 1 the pointwise kernel where it measured faster, 2 wherever it can run, 0 never

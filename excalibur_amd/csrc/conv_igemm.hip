@@ -31,6 +31,7 @@
 #include "conv_f32.h"
 #include "conv_i8_lean.h"
 #include "conv_pw.h"
+#include "conv_staged.h"
 #include "pack.h"
 
 typedef int v4i __attribute__((ext_vector_type(4)));
@@ -1726,6 +1727,36 @@ int run_conv(exhip_ctx* ctx, const exhip_conv_desc* d, ConvParams p, const PoolS
     EXHIP_REQUIRE((long long)d->n * pl.OH * pl.OW < (1ll << 31), "conv: more than 2^31 output pixels");
     const long long tiles = (long long)d->n * pl.tiles_y * pl.tiles_x * pl.ktiles;
     EXHIP_REQUIRE(tiles > 0 && tiles < (1ll << 31), "conv: grid too large");
+    // a layer with a filter as the kernels without a plan of tiles see it
+    auto with_taps = [&](exhip_pw_geom* g, exhip_pw_taps* t) {
+        *g = {};
+        g->pixels = (long long)d->n * pl.OH * pl.OW; g->c_bytes = p.cstride_b; g->k = d->k; g->k_stride = d->k_stride;
+        g->slab_blocks = pl.TM / 32; g->slabs = pl.ktiles;
+        g->act = d->act; g->post_relu = d->post_relu; g->post_op = d->post_op; g->post_slope_shared = d->post_slope_shared;
+        g->post_alpha = d->post_alpha; g->post_beta = d->post_beta; g->post_slope = d->post_slope; g->residual_last = d->residual_last;
+        g->fs_out = d->fs_out;
+        *t = {d->n, d->h, d->w, pl.OH, pl.OW, d->kh, d->kw, d->sh, d->pt, d->pl, pl.n_chunks, pl.chunk_b, false, 0};
+    };
+    const bool lean_shape = !pl.packed && !pool && d->kh == 3 && d->kw == 3 && d->sh == 1 && d->sw == 1 && pl.variant == 0 && pl.chunk_b == 64 && pl.RS == 1 &&
+                            p.cstride_b % 64 == 0;
+    if (!pl.packed && !pool && !proj && !joined && pl.KWe == 3 && d->kw == 3 && d->kh == 3 && d->sh == d->sw && !p.acc_nchw && !p.y_nchw && !p.y_nchw_h &&
+        (p.y_q || (DT == EXHIP_I8 && p.y_nhwc))) {
+        // 3x3 layers whose input under a run of pixels LDS holds, where that is the fastest way
+        exhip_pw_geom g;
+        exhip_pw_taps t;
+        with_taps(&g, &t);
+        t.staged = true;
+        if (DT == EXHIP_F16 && lean_shape && d->k % 64 == 0 && d->k_stride == d->k && d->act <= 1 && d->post_op != EXHIP_POST_PRELU) t.lean_tiles = (int)tiles;
+        if (exhip_staged_wins(DT, g, d->sh, pl.n_chunks * 9 * (pl.chunk_b / 32), p.residual, p.y_nhwc)) {
+            if constexpr (DT == EXHIP_I8)
+                rc = exhip_conv1x1_i8_pw(ctx, g, reinterpret_cast<const int8_t*>(p.x), p.wp, p.scale, p.bias, reinterpret_cast<const float*>(p.residual),
+                                         reinterpret_cast<int8_t*>(p.y_q), reinterpret_cast<float*>(p.y_nhwc), &t);
+            else
+                rc = exhip_conv1x1_f16_pw(ctx, g, reinterpret_cast<const uint16_t*>(p.x), p.wp, p.bias, reinterpret_cast<const uint16_t*>(p.residual),
+                                          reinterpret_cast<uint16_t*>(p.y_q), &t);
+            if (rc != EXHIP_ERR_UNSUPPORTED) return rc;
+        }
+    }
     if constexpr (DT == EXHIP_F16) {
         // 3x3 stride-1 layers with only the NHWC result: the lean kernel takes them with the same packed weights, also where
         // this kernel would split the reduction of a small launch (measured faster down to 25 tiles; below 16 tiles the
@@ -1735,8 +1766,7 @@ int run_conv(exhip_ctx* ctx, const exhip_conv_desc* d, ConvParams p, const PoolS
         const bool deep = !pl.packed && exhip_pw_splits_f16((long long)d->n * pl.OH * pl.OW, p.cstride_b, d->k, d->k_stride,
                                                              pl.n_chunks * d->kh * d->kw * (pl.chunk_b / 32), d->sh);
         if ((tiles >= 16 || !would_split) && g_exhip_options.force_splits <= 1 && !deep) {
-            if (!pl.packed && !pool && d->kh == 3 && d->kw == 3 && d->sh == 1 && d->sw == 1 && pl.variant == 0 && pl.chunk_b == 64 &&
-                pl.RS == 1 && p.cstride_b % 64 == 0 && d->k % 64 == 0 && d->k_stride == d->k && d->act <= 1 && p.y_q && !p.y_nchw_h && !p.y_nchw &&
+            if (lean_shape && d->k % 64 == 0 && d->k_stride == d->k && d->act <= 1 && p.y_q && !p.y_nchw_h && !p.y_nchw &&
                 d->post_op != EXHIP_POST_PRELU) {
                 exhip_lean_geom g = {};
                 g.n = d->n; g.h = d->h; g.w = d->w; g.c_bytes = p.cstride_b; g.k = d->k; g.oh = pl.OH; g.ow = pl.OW;
@@ -1798,13 +1828,9 @@ int run_conv(exhip_ctx* ctx, const exhip_conv_desc* d, ConvParams p, const PoolS
         if (joined) return EXHIP_ERR_UNSUPPORTED;
         if (!pl.packed && !proj && !p.acc_nchw && !p.y_nchw && (p.y_q || p.y_nhwc) && pl.KWe == d->kw) {
             // a layer with a filter on that kernel's tapped form, where it takes the layer
-            exhip_pw_geom g = {};
-            g.pixels = (long long)d->n * pl.OH * pl.OW; g.c_bytes = p.cstride_b; g.k = d->k; g.k_stride = d->k_stride;
-            g.slab_blocks = pl.TM / 32; g.slabs = pl.ktiles;
-            g.act = d->act; g.post_relu = d->post_relu; g.post_op = d->post_op; g.post_slope_shared = d->post_slope_shared;
-            g.post_alpha = d->post_alpha; g.post_beta = d->post_beta; g.post_slope = d->post_slope; g.residual_last = d->residual_last;
-            g.fs_out = d->fs_out;
-            const exhip_pw_taps t = {d->n, d->h, d->w, pl.OH, pl.OW, d->kh, d->kw, d->sh, d->pt, d->pl, pl.n_chunks, pl.chunk_b};
+            exhip_pw_geom g;
+            exhip_pw_taps t;
+            with_taps(&g, &t);
             rc = exhip_conv1x1_i8_pw(ctx, g, reinterpret_cast<const int8_t*>(p.x), p.wp, p.scale, p.bias, reinterpret_cast<const float*>(p.residual),
                                      reinterpret_cast<int8_t*>(p.y_q), reinterpret_cast<float*>(p.y_nhwc), &t);
             if (rc != EXHIP_ERR_UNSUPPORTED) return rc;
@@ -1854,12 +1880,9 @@ int run_conv(exhip_ctx* ctx, const exhip_conv_desc* d, ConvParams p, const PoolS
             return EXHIP_ERR_UNSUPPORTED;
         } else if (!pl.packed && !pool && p.y_q && !p.y_nchw_h && !p.y_nchw && pl.KWe == d->kw) {
             // a layer with a filter on that kernel's tapped form, where it takes the layer
-            exhip_pw_geom g = {};
-            g.pixels = (long long)d->n * pl.OH * pl.OW; g.c_bytes = p.cstride_b; g.k = d->k; g.k_stride = d->k_stride;
-            g.slab_blocks = pl.TM / 32; g.slabs = pl.ktiles;
-            g.act = d->act; g.post_relu = d->post_relu; g.post_op = d->post_op; g.post_slope_shared = d->post_slope_shared;
-            g.post_alpha = d->post_alpha; g.post_beta = d->post_beta; g.post_slope = d->post_slope; g.residual_last = d->residual_last;
-            const exhip_pw_taps t = {d->n, d->h, d->w, pl.OH, pl.OW, d->kh, d->kw, d->sh, d->pt, d->pl, pl.n_chunks, pl.chunk_b};
+            exhip_pw_geom g;
+            exhip_pw_taps t;
+            with_taps(&g, &t);
             rc = exhip_conv1x1_f16_pw(ctx, g, reinterpret_cast<const uint16_t*>(p.x), p.wp, p.bias, reinterpret_cast<const uint16_t*>(p.residual),
                                       reinterpret_cast<uint16_t*>(p.y_q), &t);
             if (rc != EXHIP_ERR_UNSUPPORTED) return rc;

@@ -31,6 +31,8 @@ struct exhip_pw_taps {
     int n, in_h, in_w, out_h, out_w;   // images, input and output maps
     int kh, kw, stride, pad_t, pad_l;  // at most 32 taps
     int n_chunks, chunk_b;             // the packing: channel chunks of chunk_b bytes (a multiple of 32), n_chunks * chunk_b bytes per pixel
+    bool staged;                       // only where conv_staged.hip takes the layer; lean_tiles: that one's
+    int lean_tiles;
 };
 
 // The depthwise 3x3 layer in front of a pointwise layer, in the same kernel: its NHWC input, weights [channel][9], bias or NULL,

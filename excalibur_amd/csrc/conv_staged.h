@@ -1,0 +1,10 @@
+// The 3x3 fp16 / int8 convolution with its input staged in LDS (conv_staged.hip): conv_pw.hip fills the launch's parameters (a PwParams of a layer with a
+// filter) and hands it over. lean_tiles: groups of conv_i8_lean.hip's fp16 form for the
+// layer, 0 where it cannot take it. EXHIP_ERR_UNSUPPORTED, with nothing launched, where another kernel runs the layer.
+#pragma once
+#include "common.h"
+#include "conv_pw.h"
+
+int exhip_conv3x3_staged(exhip_ctx* ctx, int dt, const void* pw_params, long long images, int kblocks, int lean_tiles);
+// What can be said of that beforehand, by the layer's kind and size: false where another kernel is faster. y_f: a float32 result is asked for.
+bool exhip_staged_wins(int dt, const exhip_pw_geom& g, int stride, int n_ksteps, bool shortcut, bool y_f);

@@ -42,6 +42,7 @@ extern "C" int exhip_set_option(const char* name, int value) {
     else if (!strcmp(name, "pw_tile")) o.pw_tile = value;
     else if (!strcmp(name, "pw_split")) o.pw_split = value;
     else if (!strcmp(name, "dw_pw")) o.dw_pw = value;
+    else if (!strcmp(name, "staged")) o.staged = value;
     else if (!strcmp(name, "bottleneck")) o.bottleneck = value;
     else if (!strcmp(name, "f32_tile")) o.f32_tile = value;
     else if (!strcmp(name, "lean_f16")) o.lean_f16 = value;

@@ -74,7 +74,9 @@ const char* exhip_last_error(void);
  * in another order). "dw_pw" chooses the depthwise + pointwise fp16 pairs that exhip_dw_pw_f16 takes (1 by its rule, 2 wherever it can
  * run, a power of two from 4 to 256 so with that many pixels a group where 40 KiB hold their depthwise results, 2 c + 16 bytes each, 0 never; the same
  * values). "bottleneck" chooses the fp16 blocks that exhip_bottleneck_f16 takes (1 by its rule, 16 rows + columns, up to 15 each, with that tile, + 256 with
- * eight waves a group, wherever it fits into LDS, 0 never; the same values). "f32_tile" pins the float32 convolution's wave tile and split (0 = its rule, n = the n-th of its list;
+ * eight waves a group, wherever it fits into LDS, 0 never; the same values). "staged" chooses the kernel
+ * that stages the input of 3x3 fp16 / int8 layers in LDS (1 by its rule, 2 to 4 its first to third form wherever it can run, 0 never; fp16 sums then run in another
+ * order). "f32_tile" pins the float32 convolution's wave tile and split (0 = its rule, n = the n-th of its list;
  * sums then run in another order).
  * Process-wide; packed weights depend on the first three, so set them before packing. */
 int exhip_set_option(const char* name, int value);
