@@ -865,15 +865,41 @@ __global__ __launch_bounds__(kBlock) void maxpool_nhwc_i8_kernel(const int8_t* _
 // (windows k, 2k - 1, 3k - 2 over x: 5 / 9 / 13). One group per image and 16-channel slab keeps the slab's map in LDS as
 // int16 pairs (v_pk_max_i16 takes two channels per instruction) and pools it separably, rows then columns, level after
 // level; taps outside the image count in no maximum. kPyrPixels bounds the map (two buffers of 32 bytes per pixel).
-constexpr int kPyrPixels = 960;
+// RADIUS > 0: its taps are read at clamped places, a border pixel more than once, all of them before the first maximum: with bounds for the loop each tap is an LDS
+// round trip (256 channels of one 20 x 20 map 8.6 us, of sixteen 11.9, in 256 threads; 5.4 and 9.1).
+constexpr int kPyrPixels = 960, kPyrThreads = 512;
 typedef short v2s __attribute__((ext_vector_type(2)));
 struct PyrPixel { v2s c[8]; };  // 16 channels
-__global__ __launch_bounds__(kBlock) void maxpool_pyramid_nhwc_i8_kernel(const int8_t* __restrict__ x, int8_t* __restrict__ y1, int8_t* __restrict__ y2,
+template <int RADIUS>
+__device__ __forceinline__ PyrPixel pyramid_max(const PyrPixel* line, int stride, int at, int count, int r) {
+    PyrPixel m;
+    if constexpr (RADIUS > 0) {
+        PyrPixel t[2 * RADIUS + 1];
+#pragma unroll
+        for (int d = -RADIUS; d <= RADIUS; ++d) t[d + RADIUS] = line[min(max(at + d, 0), count - 1) * stride];
+        m = t[0];
+#pragma unroll
+        for (int d = 1; d <= 2 * RADIUS; ++d)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) m.c[e] = __builtin_elementwise_max(m.c[e], t[d].c[e]);
+    } else {
+        const int lo = max(at - r, 0), hi = min(at + r, count - 1);
+        m = line[lo * stride];
+        for (int b = lo + 1; b <= hi; ++b) {
+            const PyrPixel t = line[b * stride];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) m.c[e] = __builtin_elementwise_max(m.c[e], t.c[e]);
+        }
+    }
+    return m;
+}
+template <int RADIUS>
+__global__ __launch_bounds__(kPyrThreads) void maxpool_pyramid_nhwc_i8_kernel(const int8_t* __restrict__ x, int8_t* __restrict__ y1, int8_t* __restrict__ y2,
                                                                         int8_t* __restrict__ y3, int H, int W, int cs, int k) {
     __shared__ PyrPixel buf[2][kPyrPixels];
     const int slab = blockIdx.x, n = blockIdx.y, px = H * W, r = k / 2;
     const size_t base = (size_t)n * px * cs + (size_t)slab * 16;
-    for (int i = threadIdx.x; i < px; i += kBlock) {
+    for (int i = threadIdx.x; i < px; i += kPyrThreads) {
         const v4i t = *reinterpret_cast<const v4i*>(x + base + (size_t)i * cs);
         PyrPixel o;
 #pragma unroll
@@ -890,28 +916,15 @@ __global__ __launch_bounds__(kBlock) void maxpool_pyramid_nhwc_i8_kernel(const i
         int8_t* const y = outs[level];
         if (!y) break;  // uniform
         // rows: buf[0] -> buf[1]
-        for (int i = threadIdx.x; i < px; i += kBlock) {
+        for (int i = threadIdx.x; i < px; i += kPyrThreads) {
             const int yy = i / W, xx = i - yy * W;
-            const int lo = xx - r < 0 ? 0 : xx - r, hi = xx + r >= W ? W - 1 : xx + r;
-            PyrPixel m = buf[0][yy * W + lo];
-            for (int b = lo + 1; b <= hi; ++b) {
-                const PyrPixel t = buf[0][yy * W + b];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) m.c[e] = __builtin_elementwise_max(m.c[e], t.c[e]);
-            }
-            buf[1][i] = m;
+            buf[1][i] = pyramid_max<RADIUS>(buf[0] + yy * W, 1, xx, W, r);
         }
         __syncthreads();
         // columns: buf[1] -> buf[0] (the level's result, the next level's input) and out
-        for (int i = threadIdx.x; i < px; i += kBlock) {
+        for (int i = threadIdx.x; i < px; i += kPyrThreads) {
             const int yy = i / W, xx = i - yy * W;
-            const int lo = yy - r < 0 ? 0 : yy - r, hi = yy + r >= H ? H - 1 : yy + r;
-            PyrPixel m = buf[1][lo * W + xx];
-            for (int a = lo + 1; a <= hi; ++a) {
-                const PyrPixel t = buf[1][a * W + xx];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) m.c[e] = __builtin_elementwise_max(m.c[e], t.c[e]);
-            }
+            const PyrPixel m = pyramid_max<RADIUS>(buf[1] + xx, W, yy, H, r);
             buf[0][i] = m;
             v4i o;
 #pragma unroll
@@ -1698,6 +1711,51 @@ __global__ __launch_bounds__(kBlock) void maxpool_same_1d_nhwc_f16_kernel(const 
             best = __builtin_elementwise_max(best, __builtin_bit_cast(v8h, reinterpret_cast<const v4i*>(x)[((n * H + iy) * W + ix) * C8 + v]));
     }
     reinterpret_cast<v4i*>(y)[i] = __builtin_bit_cast(v4i, best);
+}
+
+// The pyramid of stride-1 "same" max pools with windows 5, 9 and 13 and the Concat of the tensor with its three results in one launch: maxima over 5 of
+// maxima over 5 are maxima over 9. A group keeps 8 * L channels of a map in LDS, two buffers that rows and columns are taken between.
+// As layers it was six passes over the maps and a seventh for the Concat: 256 channels of sixteen 20 x 20 maps 48 us, of one 21.
+template <int L>
+__global__ __launch_bounds__(512) void maxpool_pyramid_concat_nhwc_f16_kernel(const uint16_t* __restrict__ x, uint16_t* __restrict__ y, int H, int W, int C,
+                                                                             exhip_divisor by_w) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    const int px = H * W, items = px * L;
+    v8h* const map = reinterpret_cast<v8h*>(lds);
+    v8h* const rows = map + items;
+    const size_t image = (size_t)blockIdx.y * px;
+    const int ch = blockIdx.x * 8 * L;
+    auto store = [&](int i, int level, v8h v) { *reinterpret_cast<v8h*>(y + (image + i / L) * (4 * C) + level * C + ch + i % L * 8) = v; };
+    for (int i = threadIdx.x; i < items; i += 512) {
+        const v8h v = *reinterpret_cast<const v8h*>(x + (image + i / L) * C + ch + i % L * 8);
+        map[i] = v;
+        store(i, 0, v);
+    }
+    __syncthreads();
+    auto maximum = [&](const v8h* line, int stride, int at, int count) {  // at clamped places: a border pixel more than once
+        const _Float16 ninf = -__builtin_inff16();
+        v8h t[5], m = {ninf, ninf, ninf, ninf, ninf, ninf, ninf, ninf};
+#pragma unroll
+        for (int d = 0; d < 5; ++d) t[d] = line[min(max(at + d - 2, 0), count - 1) * stride];
+#pragma unroll
+        for (int d = 0; d < 5; ++d) m = __builtin_elementwise_max(m, t[d]);
+        return m;
+    };
+#pragma unroll 1
+    for (int level = 1; level <= 3; ++level) {
+        for (int i = threadIdx.x; i < items; i += 512) {
+            const int p = i / L, row = (int)by_w((unsigned)p);
+            rows[i] = maximum(map + row * W * L + i % L, L, p - row * W, W);
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < items; i += 512) {
+            const int p = i / L, row = (int)by_w((unsigned)p);
+            const v8h m = maximum(rows + (p - row * W) * L + i % L, W * L, row, H);
+            map[i] = m;
+            store(i, level, m);
+        }
+        __syncthreads();
+    }
 }
 
 // Nearest-neighbour resize: in = min((int)(out * scale), size - 1), scale = size / (float)out_size.
@@ -2572,7 +2630,8 @@ extern "C" int exhip_maxpool_same_pyramid_nhwc_i8(exhip_ctx* ctx, const int8_t* 
     EXHIP_REQUIRE(((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y1) | reinterpret_cast<uintptr_t>(y2) | reinterpret_cast<uintptr_t>(y3)) & 15) == 0,
                   "exhip_maxpool_same_pyramid_nhwc_i8: tensors must be 16-byte aligned");
     if ((long long)h * w <= kPyrPixels && n <= 65535) {
-        hipLaunchKernelGGL(maxpool_pyramid_nhwc_i8_kernel, dim3((unsigned)(cs / 16), (unsigned)n), dim3(kBlock), 0, ctx->stream, x, y1, y2, y3, h, w, cs, k);
+        if (k == 5) hipLaunchKernelGGL(maxpool_pyramid_nhwc_i8_kernel<2>, dim3((unsigned)(cs / 16), (unsigned)n), dim3(kPyrThreads), 0, ctx->stream, x, y1, y2, y3, h, w, cs, k);
+        else hipLaunchKernelGGL(maxpool_pyramid_nhwc_i8_kernel<0>, dim3((unsigned)(cs / 16), (unsigned)n), dim3(kPyrThreads), 0, ctx->stream, x, y1, y2, y3, h, w, cs, k);
         EXHIP_LAUNCH_CHECK();
         return 0;
     }
@@ -2584,6 +2643,24 @@ extern "C" int exhip_maxpool_same_pyramid_nhwc_i8(exhip_ctx* ctx, const int8_t* 
         if (rc) return rc;
         src = outs[level];
     }
+    return 0;
+}
+
+extern "C" int exhip_maxpool_pyramid_concat_nhwc_f16(exhip_ctx* ctx, const uint16_t* x, uint16_t* y, int n, int c, int h, int w) {
+    REQ_CTX("exhip_maxpool_pyramid_concat_nhwc_f16");
+    EXHIP_REQUIRE(x && y && n > 0 && c > 0 && h > 0 && w > 0, "exhip_maxpool_pyramid_concat_nhwc_f16: bad argument");
+    EXHIP_REQUIRE(((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15) == 0, "exhip_maxpool_pyramid_concat_nhwc_f16: tensors must be 16-byte aligned");
+    // (64 KiB hold the two buffers of 16 channels of 1024 pixels, or of 8 of 2048)
+    const long long px = (long long)h * w;
+    if (c % 8 != 0 || c > (1 << 20) || n > 65535 || px > 2048) return EXHIP_ERR_UNSUPPORTED;
+    exhip_divisor by_w;
+    by_w.set((unsigned)w);
+    // 32 bytes of a pixel at a time where that still gives every CU a group
+    if (c % 16 == 0 && px <= 1024 && (long long)n * (c / 16) >= 256)
+        hipLaunchKernelGGL(maxpool_pyramid_concat_nhwc_f16_kernel<2>, dim3((unsigned)(c / 16), (unsigned)n), dim3(512), (size_t)px * 64, ctx->stream, x, y, h, w, c, by_w);
+    else
+        hipLaunchKernelGGL(maxpool_pyramid_concat_nhwc_f16_kernel<1>, dim3((unsigned)(c / 8), (unsigned)n), dim3(512), (size_t)px * 32, ctx->stream, x, y, h, w, c, by_w);
+    EXHIP_LAUNCH_CHECK();
     return 0;
 }
 

@@ -381,6 +381,9 @@ public:
     }
     void clear_post() { post_set_ = false; post_used_ = false; post_bn_a_ = post_bn_b_ = nullptr; post_unary_ = -1; }
     bool post_used() const { return post_used_; }
+    // fp16: this layer and the max pools with windows 5, 9 and 13 of x in front of it, whose results stand behind x in it, as one launch. False, with nothing done,
+    // where the four run by themselves.
+    bool forward_pyramid(const std::shared_ptr<memory::tensor<unsigned short>>& x, tensor_list<unsigned short>& tops);
 
 protected:
     const float *post_bn_a_ = nullptr, *post_bn_b_ = nullptr;

@@ -1568,6 +1568,18 @@ void operation_concat<Dtype>::forward_gpu_f16(const tensor_list<unsigned short>&
 }
 
 template <typename Dtype>
+bool operation_concat<Dtype>::forward_pyramid(const half_ptr& x, tensor_list<unsigned short>& tops) {
+    const int n = x->num(), c = x->channels(), h = x->height(), w = x->width();
+    if (x->order() != memory::NHWC || !nhwc_channels_ok(c)) return false;
+    auto y = new_tensor<unsigned short>({n, h, w, 4 * c}, this->params_.device_, memory::NHWC);
+    const int rc = exhip_maxpool_pyramid_concat_nhwc_f16(this->ctx(), x->gpu_data(), y->mutable_gpu_data(), n, c, h, w);
+    if (rc == EXHIP_ERR_UNSUPPORTED) return false;
+    EXHIP_FATAL(rc);
+    tops[0] = y;
+    return true;
+}
+
+template <typename Dtype>
 operation_interp<Dtype>::operation_interp(const operation_param& param) : operation<Dtype>(param) {
     for (const layer_attr& a : parse_attrs(param.specific_params_)) {
         switch (std::atoi(a.key.c_str())) {

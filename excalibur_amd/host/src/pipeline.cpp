@@ -236,6 +236,7 @@ public:
         find_sum_pairs();
         find_depthwise_pairs();
         find_blocks();
+        find_pyramids();
         find_stem();
         find_heads();
         find_glue_chains();
@@ -306,6 +307,34 @@ public:
                 if (readers[mid] != own_readers || op_outputs_[last + 1].size() != 1 || op_outputs_[last + 1][0] == mid) continue;
                 if (std::find(output_names_.begin(), output_names_.end(), blob_names_[mid]) != output_names_.end()) continue;
                 behind_depthwise_[i] = static_cast<int>(last + 1);
+            }
+        }
+    }
+
+    // fp16 pipeline: three stride-1 "same" max pools of one tensor (through a Split), windows 5, 9 and 13, whose only reader is the Concat behind them of that tensor
+    // and their results: one kernel runs the four where the map fits, and the three blobs are never stored. That the inputs are one tensor is
+    // known when the blobs are there.
+    void find_pyramids() {
+        opens_pyramid_.assign(operations_.size(), false);
+        if constexpr (std::is_same_v<Dtype, unsigned short>) {
+            for (size_t i = 0; i + 3 < operations_.size(); ++i) {
+                auto* cat = dynamic_cast<operation_concat<Dtype>*>(operations_[i + 3].get());
+                if (!cat || cat->axis_ + 2 != 1 || op_inputs_[i + 3].size() != 4 || op_outputs_[i + 3].size() != 1) continue;
+                bool ok = true;
+                for (size_t j = 0; ok && j < 3; ++j) {
+                    auto* pool = dynamic_cast<operation_pooling<Dtype>*>(operations_[i + j].get());
+                    const int k = 5 + 4 * static_cast<int>(j);
+                    ok = pool && pool->type_ == 0 && !pool->global_pooling_ && pool->kernel_size_h_ == k && pool->kernel_size_w_ == k && pool->stride_h_ == 1 &&
+                         pool->stride_w_ == 1 && pool->pad_top_ == k / 2 && pool->pad_bottom_ == k / 2 && pool->pad_left_ == k / 2 && pool->pad_right_ == k / 2 &&
+                         op_inputs_[i + j].size() == 1 && op_outputs_[i + j].size() == 1 && op_inputs_[i + 3][j + 1] == op_outputs_[i + j][0];
+                    if (!ok) break;
+                    const int mid = op_outputs_[i + j][0];
+                    int readers = 0, writers = 0;
+                    for (const auto& in : op_inputs_) readers += static_cast<int>(std::count(in.begin(), in.end(), mid));
+                    for (size_t q = i; q < i + 4; ++q) writers += static_cast<int>(std::count(op_outputs_[q].begin(), op_outputs_[q].end(), mid));
+                    ok = readers == 1 && writers == 1 && std::find(output_names_.begin(), output_names_.end(), blob_names_[mid]) == output_names_.end();
+                }
+                opens_pyramid_[i] = ok;
             }
         }
     }
@@ -604,6 +633,19 @@ private:
                 }
             }
             if constexpr (std::is_same_v<Dtype, unsigned short>) {
+                if (fusion_ && opens_pyramid_[i] && chain_[i + 3].last <= static_cast<int>(i + 3)) {
+                    const auto& x = in[0];
+                    bool one = true;
+                    for (int b : {op_inputs_[i + 1][0], op_inputs_[i + 2][0], op_inputs_[i + 3][0]}) one = one && featmaps_[b] == x;
+                    if (one && static_cast<operation_concat<Dtype>*>(operations_[i + 3].get())->forward_pyramid(x, out)) {
+                        for (size_t k = i; k < i + 3; ++k) featmaps_[op_outputs_[k][0]] = nullptr;
+                        i += 3;
+                        featmaps_[op_outputs_[i][0]] = out[0];
+                        continue;
+                    }
+                }
+            }
+            if constexpr (std::is_same_v<Dtype, unsigned short>) {
                 const bool block = opens_block_[i] >= 0;
                 if (fusion_ && (block || behind_depthwise_[i] >= 0)) {
                     const size_t dw_at = block ? opens_block_[i] : i, j = behind_depthwise_[dw_at];
@@ -738,6 +780,7 @@ private:
     std::vector<int> sum_other_;         // per layer: the other operand's blob of the sum layer this convolution absorbs, or -1
     std::vector<int> opens_block_;       // per layer: the depthwise layer of the block that this pointwise layer begins, or -1
     std::vector<int> behind_depthwise_;  // per layer: the pointwise layer that runs in this depthwise layer's kernel, or -1
+    std::vector<char> opens_pyramid_;    // per layer: the first pooling layer of a pyramid whose Concat is three lines on
     std::vector<char> behind_input_;     // per layer: the convolution on the next line runs in this Input layer's kernel
     std::vector<char> in_groups_;        // per layer: this convolution stores its results as the Reshape and Transpose behind it leave them
     struct glue_chain {

@@ -355,6 +355,9 @@ int exhip_maxpool2d_nhwc_i8(exhip_ctx* ctx, const int8_t* x, int8_t* y, int n, i
  * the image count in no maximum). y3, or y2 and y3, may be NULL. k odd; tensors [n][h][w][cs], cs a multiple of 16. */
 int exhip_maxpool_same_pyramid_nhwc_i8(exhip_ctx* ctx, const int8_t* x, int8_t* y1, int8_t* y2, int8_t* y3, int n, int c, int h, int w,
                                        int cs, int k);
+/* The same pyramid on halves, windows 5, 9 and 13, with the Concat of the tensor and its three results behind it: y [n][h][w][4 c]. Tensors on 16 bytes;
+ * EXHIP_ERR_UNSUPPORTED, with nothing launched, for c not a multiple of 8 and maps of more than 2048 pixels. */
+int exhip_maxpool_pyramid_concat_nhwc_f16(exhip_ctx* ctx, const uint16_t* x, uint16_t* y, int n, int c, int h, int w);
 int exhip_pool2d_nhwc_f16(exhip_ctx* ctx, const uint16_t* x, uint16_t* y, int n, int c, int h, int w, int c_stride,
                           int oh, int ow, int type, int kh, int kw, int sh, int sw, int pt, int pb, int pl, int pr,
                           int count_include_pad);
