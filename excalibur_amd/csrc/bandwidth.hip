@@ -1719,10 +1719,8 @@ __global__ __launch_bounds__(kBlock) void maxpool_same_1d_nhwc_f16_kernel(const 
 template <int L>
 __global__ __launch_bounds__(512) void maxpool_pyramid_concat_nhwc_f16_kernel(const uint16_t* __restrict__ x, uint16_t* __restrict__ y, int H, int W, int C,
                                                                              exhip_divisor by_w) {
-    extern __shared__ __attribute__((aligned(16))) char lds[];
+    __shared__ v8h map[2048], rows[2048];
     const int px = H * W, items = px * L;
-    v8h* const map = reinterpret_cast<v8h*>(lds);
-    v8h* const rows = map + items;
     const size_t image = (size_t)blockIdx.y * px;
     const int ch = blockIdx.x * 8 * L;
     auto store = [&](int i, int level, v8h v) { *reinterpret_cast<v8h*>(y + (image + i / L) * (4 * C) + level * C + ch + i % L * 8) = v; };
@@ -2657,9 +2655,9 @@ extern "C" int exhip_maxpool_pyramid_concat_nhwc_f16(exhip_ctx* ctx, const uint1
     by_w.set((unsigned)w);
     // 32 bytes of a pixel at a time where that still gives every CU a group
     if (c % 16 == 0 && px <= 1024 && (long long)n * (c / 16) >= 256)
-        hipLaunchKernelGGL(maxpool_pyramid_concat_nhwc_f16_kernel<2>, dim3((unsigned)(c / 16), (unsigned)n), dim3(512), (size_t)px * 64, ctx->stream, x, y, h, w, c, by_w);
+        hipLaunchKernelGGL(maxpool_pyramid_concat_nhwc_f16_kernel<2>, dim3((unsigned)(c / 16), (unsigned)n), dim3(512), 0, ctx->stream, x, y, h, w, c, by_w);
     else
-        hipLaunchKernelGGL(maxpool_pyramid_concat_nhwc_f16_kernel<1>, dim3((unsigned)(c / 8), (unsigned)n), dim3(512), (size_t)px * 32, ctx->stream, x, y, h, w, c, by_w);
+        hipLaunchKernelGGL(maxpool_pyramid_concat_nhwc_f16_kernel<1>, dim3((unsigned)(c / 8), (unsigned)n), dim3(512), 0, ctx->stream, x, y, h, w, c, by_w);
     EXHIP_LAUNCH_CHECK();
     return 0;
 }
