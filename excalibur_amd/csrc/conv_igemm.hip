@@ -2122,6 +2122,24 @@ extern "C" int exhip_bottleneck_f16(exhip_ctx* ctx, const exhip_conv_desc* first
     return exhip_bottleneck_run(ctx, b);
 }
 
+extern "C" int exhip_conv2d_i8_pair(exhip_ctx* ctx, const exhip_conv_i8_call* a, const exhip_conv_i8_call* b) {
+    EXHIP_REQUIRE(ctx && a && b && a->d && b->d, "exhip_conv2d_i8_pair: NULL argument");
+    auto layer = [](exhip_ctx* on, const void* call) {
+        const auto* c = static_cast<const exhip_conv_i8_call*>(call);
+        return exhip_conv2d_i8(on, c->d, c->x, c->w_packed, c->scale, c->bias, nullptr, c->y_i8, c->y_f32, nullptr, nullptr);
+    };
+    return exhip_pw_pair(ctx, layer, a, b);
+}
+
+extern "C" int exhip_conv2d_f16_pair(exhip_ctx* ctx, const exhip_conv_f16_call* a, const exhip_conv_f16_call* b) {
+    EXHIP_REQUIRE(ctx && a && b && a->d && b->d, "exhip_conv2d_f16_pair: NULL argument");
+    auto layer = [](exhip_ctx* on, const void* call) {
+        const auto* c = static_cast<const exhip_conv_f16_call*>(call);
+        return exhip_conv2d_f16(on, c->d, c->x, c->w_packed, c->bias, nullptr, c->y, nullptr, nullptr);
+    };
+    return exhip_pw_pair(ctx, layer, a, b);
+}
+
 extern "C" int exhip_conv2d_i8_maxpool2x2(exhip_ctx* ctx, const exhip_conv_desc* d, int pool_oh, int pool_ow, const int8_t* x, const void* wp,
                                           const float* scale, const float* bias, int8_t* y_i8, float* y_f32) {
     EXHIP_REQUIRE(ctx && d && x && wp && scale && (y_i8 || y_f32), "exhip_conv2d_i8_maxpool2x2: bad argument");

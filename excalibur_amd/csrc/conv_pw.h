@@ -64,3 +64,5 @@ int exhip_conv1x1_i8_pw(exhip_ctx* ctx, const exhip_pw_geom& g, const int8_t* x,
 bool exhip_pw_splits_f16(long long pixels, int c_bytes, int k, int k_stride, int n_ksteps, int stride);
 // The runs of 32-byte k-steps that an fp16 pointwise layer's sums are made of (1: all in one), and where they begin.
 int exhip_pw_runs_f16(const exhip_pw_geom& g, int start[5]);
+// Runs two layers of which neither reads what the other writes, in one launch where both are pointwise layers that kernel takes.
+int exhip_pw_pair(exhip_ctx* ctx, int (*layer)(exhip_ctx*, const void*), const void* first, const void* second);

@@ -33,17 +33,16 @@
 namespace {
 
 // U: k-steps per request round; two rounds are in flight. PAIRS: the pixels in 64-byte pieces, as in the split form below.
+constexpr int pw_wave_lds(int dt, int mt, int nt, bool pairs) { return param_bytes(mt) + (pairs && nt * 4096 > tile_bytes(dt, mt) ? nt * 4096 : tile_bytes(dt, mt)); }
+// (the kernel's group `bid` of `groups`)
 template <int DT, int MT, int NT, int U, bool TAPS, bool PAIRS, typename EP>
-__global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
-    exhip_touch_args(p);
-    constexpr int OWN = param_bytes(MT) + (PAIRS && NT * 4096 > tile_bytes(DT, MT) ? NT * 4096 : tile_bytes(DT, MT));
-    __shared__ __attribute__((aligned(16))) char lds_all[4 * OWN];
+__device__ __forceinline__ void pw_group(const PwParams& p, char* lds_all, unsigned bid, unsigned groups) {
+    constexpr int OWN = pw_wave_lds(DT, MT, NT, PAIRS);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // workgroup ids are dealt round-robin to the 8 XCDs: give each XCD one contiguous run of items, so that the channel
     // groups of a pixel tile (and the weights' re-reads) share that XCD's L2
-    unsigned bid = blockIdx.x;
     {
-        const unsigned per = gridDim.x >> 3;
+        const unsigned per = groups >> 3;
         if (bid < (per << 3)) bid = (bid & 7) * per + (bid >> 3);
     }
     const unsigned item = __builtin_amdgcn_readfirstlane(bid * 4 + wave);
@@ -212,25 +211,31 @@ __global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
     pw_epilogue<DT, MT, NT, EP>(p, acc, tile * NT * 32, p.pixels, kb0, lane, lds);
 }
 
+template <int DT, int MT, int NT, int U, bool TAPS, bool PAIRS, typename EP>
+__global__ __launch_bounds__(256, 2) void conv1x1_pw_kernel(const PwParams p) {
+    exhip_touch_args(p);
+    __shared__ __attribute__((aligned(16))) char lds_all[4 * pw_wave_lds(DT, MT, NT, PAIRS)];
+    pw_group<DT, MT, NT, U, TAPS, PAIRS, EP>(p, lds_all, blockIdx.x, gridDim.x);
+}
+
 // The split form, for launches of few tiles and many k-steps (one image, deep layers), where the kernel above is as long as one
 // wave's chain: 0.17 us a k-step, 16 us for 256 -> 256 3x3 int8 on a 20 x 20 map. WK waves share a tile of 32 pixels x 32 * MT
 // channels: each takes its run of the k-steps, the sums meet in LDS (exactly for int8; in a fixed order, so the same bits
 // every time, for fp16), and each wave finishes its quarter of the tile, eight channels of a pixel per lane (wave m the whole block m
 // where the layers behind are looked at at run time: a head's groups take 32 channels at a time). Every request in the loop is unconditional, so that the waits count what is in
 // flight; those past a wave's run ask for operands it does not use.
+template <int DT, int MT, int WK, typename EP>
+constexpr int split_lds() { return WK * MT * 4096 + (EP::any ? MT * wave_bytes(DT, 1) : WK * param_bytes(1)); }
 template <int DT, int MT, int WK, bool TAPS, bool PAIRS, typename EP>
-__global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParams p) {
-    exhip_touch_args(p);
+__device__ __forceinline__ void split_group(const PwParams& p, char* lds_all, unsigned item, unsigned groups) {
     constexpr int R = 8;  // k-steps in flight
     constexpr bool I8 = DT == EXHIP_I8;
     constexpr int RED = WK * MT * 4096;
     constexpr int OWN = EP::any ? wave_bytes(DT, 1) : param_bytes(1);
     static_assert(MT == 2 && WK == 4 && WK <= kSplit, "two waves finish a block");
-    __shared__ __attribute__((aligned(16))) char lds_all[RED + (EP::any ? MT : WK) * OWN];
     const int lane = threadIdx.x & 63, part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    unsigned item = blockIdx.x;
     {
-        const unsigned per = gridDim.x >> 3;
+        const unsigned per = groups >> 3;
         if (item < (per << 3)) item = (item & 7) * per + (item >> 3);
     }
     const unsigned tile = __builtin_amdgcn_readfirstlane(exhip_divide(item, p.ch_groups, p.groups_magic, p.groups_shift));
@@ -494,6 +499,49 @@ __global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParam
             __builtin_amdgcn_raw_buffer_store_b128(o, tile_view(p.y, tile * 32, p.kstride * 2, kb * 64, rows), pw_lane_offset(row, p.kstride * 2, ch * 2, (k_end - kb * 32) * 2), 0, 0);
         }
     }
+}
+
+template <int DT, int MT, int WK, bool TAPS, bool PAIRS, typename EP>
+__global__ __launch_bounds__(64 * WK, 2) void conv_pw_split_kernel(const PwParams p) {
+    exhip_touch_args(p);
+    __shared__ __attribute__((aligned(16))) char lds_all[split_lds<DT, MT, WK, EP>()];
+    split_group<DT, MT, WK, TAPS, PAIRS, EP>(p, lds_all, blockIdx.x, gridDim.x);
+}
+
+// Two pointwise layers that do not read each other's results in one launch, each in its own form: a bottleneck's last layer and the one beside it, on the
+// two inputs of a Concat. Launched one after the other each waits for the other's last group, and at one image each is 4 us whatever it computes:
+// 64 -> 64 and 128 -> 64 at 1 x 80 x 80 int8 7.7 us, here 4.2, at 16 x 80 x 80 15.0 and 12.1; fp16 7.1 and 3.5, 16.2 and 13.2. No pair of eight sizes took longer.
+struct PwTwo {
+    PwParams p[2];
+    int kind[2];
+    unsigned groups[2];
+};
+constexpr int kTwoLds = 34816;
+template <int DT>  // what stands behind them in the networks: int8 a BatchNorm and a LeakyReLU layer (through the Concat), fp16 nothing
+using TwoEp = typename std::conditional<DT == EXHIP_I8, Ep<0, kPostLeaky, 0, true>, Ep<0, kPostNone, 0>>::type;
+// the forms by number, -1 for all others
+template <int DT, int MT, int NT, int U, bool TAPS, typename EP>
+constexpr int two_kind() {
+    if (TAPS || !std::is_same<EP, TwoEp<DT>>::value) return -1;
+    if (MT == 1 && NT == 2) return U == 4 ? 0 : U == 104 ? 1 : -1;
+    return MT != 2 || NT != 1 ? -1 : U == 4 ? 2 : U == 104 ? 3 : U == -2 * kSplit ? 4 : -1;
+}
+template <int DT>
+__device__ __forceinline__ void two_group(const PwParams& p, int kind, char* lds, unsigned bid, unsigned groups) {
+    exhip_touch_args(p);
+    if (kind == 0) pw_group<DT, 1, 2, 4, false, false, TwoEp<DT>>(p, lds, bid, groups);
+    else if (kind == 1) pw_group<DT, 1, 2, 4, false, true, TwoEp<DT>>(p, lds, bid, groups);
+    else if (kind == 2) pw_group<DT, 2, 1, 4, false, false, TwoEp<DT>>(p, lds, bid, groups);
+    else if (kind == 3) pw_group<DT, 2, 1, 4, false, true, TwoEp<DT>>(p, lds, bid, groups);
+    else split_group<DT, 2, kSplit, false, true, TwoEp<DT>>(p, lds, bid, groups);
+}
+template <int DT>
+__global__ __launch_bounds__(256, 2) void conv_pw_two_kernel(const PwTwo q) {
+    static_assert(4 * pw_wave_lds(DT, 1, 2, true) <= kTwoLds && 4 * pw_wave_lds(DT, 2, 1, true) <= kTwoLds && split_lds<DT, 2, kSplit, TwoEp<DT>>() <= kTwoLds, "one LDS for all");
+    __shared__ __attribute__((aligned(16))) char lds[kTwoLds];
+    const unsigned first = q.groups[0];
+    if (blockIdx.x < first) two_group<DT>(q.p[0], q.kind[0], lds, blockIdx.x, first);
+    else two_group<DT>(q.p[1], q.kind[1], lds, blockIdx.x - first, q.groups[1]);
 }
 
 // A depthwise 3x3 layer and the pointwise layer that alone reads it, the depthwise results staying in LDS. A group computes
@@ -917,9 +965,30 @@ int run_stem(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, int
     return vec ? go_stem<DT, 2, true>(ctx, p, lds) : go_stem<DT, 2, false>(ctx, p, lds);
 }
 
+// A launch that waits for another one to share it with (exhip_pw_pair).
+struct Waiting {
+    int kind = -1, dt = 0;
+    unsigned groups = 0;
+    const void* kernel = nullptr;
+    PwParams p;
+};
+thread_local Waiting* t_collect = nullptr;  // while the pair's layers are run: the place for the next launch
+
 // U > 0: the kernel with U k-steps a request round, 100 + U in pairs; U < 0: the split form, -kSplit a k-step at a time, -2 * kSplit in pairs
 template <int DT, int MT, int NT, int U, bool TAPS, typename EP>
 int go(exhip_ctx* ctx, const PwParams& p) {
+    if constexpr (two_kind<DT, MT, NT, U, TAPS, EP>() >= 0) {
+        if (t_collect) {
+            t_collect->kind = two_kind<DT, MT, NT, U, TAPS, EP>();
+            t_collect->dt = DT;
+            t_collect->groups = U < 0 ? p.items : (p.items + 3) / 4;
+            if constexpr (U < 0) t_collect->kernel = reinterpret_cast<const void*>(conv_pw_split_kernel<DT, MT, kSplit, TAPS, U == -2 * kSplit, EP>);
+            else t_collect->kernel = reinterpret_cast<const void*>(conv1x1_pw_kernel<DT, MT, NT, U % 100, TAPS, (U > 100), EP>);
+            t_collect->p = p;
+            t_collect = nullptr;
+            return 0;
+        }
+    }
     if constexpr (U < 0) hipLaunchKernelGGL((conv_pw_split_kernel<DT, MT, kSplit, TAPS, U == -2 * kSplit, EP>), dim3(p.items), dim3(64 * kSplit), 0, ctx->stream, p);
     else hipLaunchKernelGGL((conv1x1_pw_kernel<DT, MT, NT, U % 100, TAPS, (U > 100), EP>), dim3((p.items + 3) / 4), dim3(256), 0, ctx->stream, p);
     EXHIP_LAUNCH_CHECK();
@@ -1362,4 +1431,32 @@ bool exhip_pw_splits_f16(long long pixels, int c_bytes, int k, int k_stride, int
     exhip_pw_geom g = {};
     g.pixels = pixels; g.c_bytes = c_bytes;
     return g_exhip_options.pw != 0 && g_exhip_options.direct != 0 && split_wins(EXHIP_F16, g, (std::max(k, k_stride) + 31) / 32, n_ksteps, true, stride);
+}
+
+int exhip_pw_pair(exhip_ctx* ctx, int (*layer)(exhip_ctx*, const void*), const void* first, const void* second) {
+    Waiting w[2];
+    int rc = 0;
+    for (int i = 0; i < 2 && !rc; ++i) {
+        t_collect = &w[i];
+        rc = layer(ctx, i ? second : first);
+        t_collect = nullptr;
+    }
+    // (a layer that ran by itself is done; it reads nothing of the other's)
+    const bool fits = (long long)w[0].groups + w[1].groups < (1ll << 31);
+    if (!rc && w[0].kind >= 0 && w[1].kind >= 0 && w[0].dt == w[1].dt && fits) {
+        PwTwo q;
+        for (int i = 0; i < 2; ++i) q.p[i] = w[i].p, q.kind[i] = w[i].kind, q.groups[i] = w[i].groups;
+        const dim3 grid(w[0].groups + w[1].groups);
+        if (w[0].dt == EXHIP_I8) hipLaunchKernelGGL(conv_pw_two_kernel<EXHIP_I8>, grid, dim3(256), 0, ctx->stream, q);
+        else hipLaunchKernelGGL(conv_pw_two_kernel<EXHIP_F16>, grid, dim3(256), 0, ctx->stream, q);
+        EXHIP_LAUNCH_CHECK();
+        return 0;
+    }
+    for (Waiting& one : w) {
+        if (one.kind < 0) continue;
+        void* args[] = {&one.p};
+        EXHIP_CHECK(hipLaunchKernel(one.kernel, dim3(one.groups), dim3(256), args, 0, ctx->stream));
+        EXHIP_LAUNCH_CHECK();
+    }
+    return rc;
 }

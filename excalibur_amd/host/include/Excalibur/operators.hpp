@@ -88,6 +88,11 @@ public:
     // the same with the pointwise layer `first` that the depthwise layer alone reads: a mobile network's block; `bottoms` are that layer's
     bool forward_block(operation_convolution<Dtype>& first, operation_convolutiondepthwise<Dtype>& dw, const tensor_list<unsigned short>& bottoms,
                        tensor_list<unsigned short>& tops);
+    // fp16: this layer and `next`, pointwise ones of which neither reads the other, in one launch where their forms allow it. False, with nothing done, where a layer's
+    // tensors are not for it.
+    bool forward_beside(operation_convolution<Dtype>& next, const tensor_list<unsigned short>& bottoms, tensor_list<unsigned short>& tops,
+                        const tensor_list<unsigned short>& next_bottoms, tensor_list<unsigned short>& next_tops);
+    bool beside_form(const tensor_list<unsigned short>& bottoms, exhip_conv_desc* d) const;
     // fp16: this layer, of at most four input channels, straight on its NCHW input, with the Input layer that it alone reads in front of it
     // (or NULL) and the layers set behind it; `bottoms` are the first one's. False, with nothing done, where the layers run by themselves.
     bool forward_stem(operation_input<Dtype>* input, const tensor_list<unsigned short>& bottoms, tensor_list<unsigned short>& tops);

@@ -650,6 +650,29 @@ bool operation_convolution<Dtype>::forward_behind_depthwise(operation_convolutio
 }
 
 template <typename Dtype>
+bool operation_convolution<Dtype>::beside_form(const tensor_list<unsigned short>& bottoms, exhip_conv_desc* d) const {
+    const int c = this->input_channels();
+    if (bottoms[0]->order() != memory::NHWC || bottoms[0]->channels() != c || !mfma_path_ok() || !nhwc_allowed() || this->output_channel_ % 16 != 0 || through_rows_ ||
+        conv_in_stride(c, EXHIP_F16, 1) != c)
+        return false;
+    *d = describe(bottoms[0]->num(), bottoms[0]->height(), bottoms[0]->width(), c, this->output_channel_);
+    return d->kh == 1 && d->kw == 1 && d->sh == 1 && d->sw == 1 && !d->pt && !d->pb && !d->pl && !d->pr;
+}
+
+template <typename Dtype>
+bool operation_convolution<Dtype>::forward_beside(operation_convolution<Dtype>& next, const tensor_list<unsigned short>& bottoms, tensor_list<unsigned short>& tops,
+                                                  const tensor_list<unsigned short>& next_bottoms, tensor_list<unsigned short>& next_tops) {
+    exhip_conv_desc d, e;
+    if (!beside_form(bottoms, &d) || !next.beside_form(next_bottoms, &e)) return false;
+    tops[0] = new_tensor<unsigned short>({d.n, d.h, d.w, this->output_channel_}, this->params_.device_, memory::NHWC);
+    next_tops[0] = new_tensor<unsigned short>({e.n, e.h, e.w, next.output_channel_}, this->params_.device_, memory::NHWC);
+    const exhip_conv_f16_call a = {&d, bottoms[0]->gpu_data(), packed_weights(EXHIP_F16, d), bias_gpu(), tops[0]->mutable_gpu_data()};
+    const exhip_conv_f16_call b = {&e, next_bottoms[0]->gpu_data(), next.packed_weights(EXHIP_F16, e), next.bias_gpu(), next_tops[0]->mutable_gpu_data()};
+    EXHIP_FATAL(exhip_conv2d_f16_pair(this->ctx(), &a, &b));
+    return true;
+}
+
+template <typename Dtype>
 bool operation_convolution<Dtype>::forward_block(operation_convolution<Dtype>& first, operation_convolutiondepthwise<Dtype>& dw,
                                                  const tensor_list<unsigned short>& bottoms, tensor_list<unsigned short>& tops) {
     const int dev = this->params_.device_, c = first.input_channels(), wide = this->input_channels();

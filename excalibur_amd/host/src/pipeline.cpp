@@ -239,6 +239,7 @@ public:
         find_pyramids();
         find_stem();
         find_heads();
+        find_neighbours();
         find_glue_chains();
     }
 
@@ -307,6 +308,23 @@ public:
                 if (readers[mid] != own_readers || op_outputs_[last + 1].size() != 1 || op_outputs_[last + 1][0] == mid) continue;
                 if (std::find(output_names_.begin(), output_names_.end(), blob_names_[mid]) != output_names_.end()) continue;
                 behind_depthwise_[i] = static_cast<int>(last + 1);
+            }
+        }
+    }
+
+    // fp16 pipeline: a convolution without layers of its own behind it in front of another such that does not read it (a bottleneck's last layer and the one beside it,
+    // on a Concat's two inputs): where both are pointwise one launch runs both.
+    void find_neighbours() {
+        beside_next_.assign(operations_.size(), false);
+        if constexpr (std::is_same_v<Dtype, unsigned short>) {
+            auto plain = [&](size_t i) {
+                auto* conv = dynamic_cast<operation_convolution<Dtype>*>(operations_[i].get());
+                return conv && !dynamic_cast<operation_convolutiondepthwise<Dtype>*>(conv) && conv->kernel_size_h_ == 1 && conv->kernel_size_w_ == 1 && !pair_[i].on &&
+                       sum_other_[i] < 0 && !in_groups_[i] && opens_block_[i] < 0 && op_inputs_[i].size() == 1 && op_outputs_[i].size() == 1;
+            };
+            for (size_t i = 0; i + 1 < operations_.size(); ++i) {
+                beside_next_[i] = !(i > 0 && beside_next_[i - 1]) && plain(i) && plain(i + 1) && op_inputs_[i + 1] != op_outputs_[i] && op_outputs_[i + 1] != op_outputs_[i] &&
+                                  op_outputs_[i] != op_inputs_[i] && op_outputs_[i + 1] != op_inputs_[i];
             }
         }
     }
@@ -633,6 +651,21 @@ private:
                 }
             }
             if constexpr (std::is_same_v<Dtype, unsigned short>) {
+                if (fusion_ && beside_next_[i] && featmaps_[op_inputs_[i + 1][0]]) {
+                    auto* conv = static_cast<operation_convolution<Dtype>*>(operations_[i].get());
+                    auto* next = static_cast<operation_convolution<Dtype>*>(operations_[i + 1].get());
+                    std::vector<tensor_ptr> next_in = {featmaps_[op_inputs_[i + 1][0]]}, next_out(1);
+                    if (conv->forward_beside(*next, in, out, next_in, next_out)) {
+                        featmaps_[op_outputs_[i][0]] = out[0];
+                        mark_result(i, out);
+                        ++i;
+                        featmaps_[op_outputs_[i][0]] = next_out[0];
+                        mark_result(i, next_out);
+                        continue;
+                    }
+                }
+            }
+            if constexpr (std::is_same_v<Dtype, unsigned short>) {
                 if (fusion_ && opens_pyramid_[i] && chain_[i + 3].last <= static_cast<int>(i + 3)) {
                     const auto& x = in[0];
                     bool one = true;
@@ -780,6 +813,7 @@ private:
     std::vector<int> sum_other_;         // per layer: the other operand's blob of the sum layer this convolution absorbs, or -1
     std::vector<int> opens_block_;       // per layer: the depthwise layer of the block that this pointwise layer begins, or -1
     std::vector<int> behind_depthwise_;  // per layer: the pointwise layer that runs in this depthwise layer's kernel, or -1
+    std::vector<char> beside_next_;      // per layer: this pointwise convolution and the one on the next line, which does not read it, run in one launch
     std::vector<char> opens_pyramid_;    // per layer: the first pooling layer of a pyramid whose Concat is three lines on
     std::vector<char> behind_input_;     // per layer: the convolution on the next line runs in this Input layer's kernel
     std::vector<char> in_groups_;        // per layer: this convolution stores its results as the Reshape and Transpose behind it leave them
@@ -1620,6 +1654,14 @@ bool pipeline<float>::impl::build_graph_plan(const tensor_ptr& input, const std:
             if (r.launch < 0) r.launch = static_cast<int>(plan->launches.size()) - 1;
     };
     int pooled_already = -1;  // a pooling layer's value that the convolution in front has written
+    struct joined_layer {  // a convolution that writes its part of a joined Concat
+        exhip_conv_desc d;
+        const int8_t* x;
+        const void* wp;
+        const float *scale, *bias;
+        int8_t* yq;
+        size_t launch;
+    } beside = {};
     for (const node& nd : nodes) {
         results_complete();
         const value_info in = vals[nd.in[0]];
@@ -1674,7 +1716,18 @@ bool pipeline<float>::impl::build_graph_plan(const tensor_ptr& input, const std:
                 const int rc = exhip_conv2d_i8(ctx, &d, x, wp, scale, bias, nullptr, yq, nullptr, nullptr, nullptr);  // trial launch
                 if (rc == EXHIP_ERR_UNSUPPORTED) return refuse(__LINE__);
                 EXHIP_FATAL(rc);
+                const joined_layer own = {d, x, wp, scale, bias, yq, plan->launches.size()};
+                if (beside.wp && beside.launch + 1 == own.launch && x != beside.yq) {  // the layer in front writes its part of a joined Concat too: both in one launch
+                    const joined_layer other = beside;
+                    plan->launches.back() = [=]() {
+                        const exhip_conv_i8_call a = {&other.d, other.x, other.wp, other.scale, other.bias, other.yq, nullptr}, b = {&own.d, own.x, own.wp, own.scale, own.bias, own.yq, nullptr};
+                        EXHIP_FATAL(exhip_conv2d_i8_pair(ctx, &a, &b));
+                    };
+                    beside = {};
+                    continue;
+                }
                 plan->launches.push_back([=]() { EXHIP_FATAL(exhip_conv2d_i8(ctx, &d, x, wp, scale, bias, nullptr, yq, nullptr, nullptr, nullptr)); });
+                beside = own;
                 continue;
             }
             if (nd.head_reshape >= 0) {

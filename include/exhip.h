@@ -238,6 +238,26 @@ int exhip_dw_pw_f16(exhip_ctx* ctx, const exhip_depthwise_desc* dw, const exhip_
 int exhip_bottleneck_f16(exhip_ctx* ctx, const exhip_conv_desc* first, const void* w_first, const float* bias_first, const exhip_depthwise_desc* dw,
                          const exhip_conv_desc* last, const void* w_last, const float* bias_last, const uint16_t* residual_nhwc, uint16_t* y_nhwc);
 
+/* Two layers of which neither reads what the other writes: the values of exhip_conv2d_i8 / exhip_conv2d_f16 for each, pointwise ones with the same kind of
+ * layers behind them in one launch. An error is that of the first layer that has one; the other may have run. */
+typedef struct exhip_conv_i8_call {
+    const exhip_conv_desc* d;
+    const int8_t* x;
+    const void* w_packed;
+    const float *scale, *bias;
+    int8_t* y_i8;
+    float* y_f32;
+} exhip_conv_i8_call;
+int exhip_conv2d_i8_pair(exhip_ctx* ctx, const exhip_conv_i8_call* a, const exhip_conv_i8_call* b);
+typedef struct exhip_conv_f16_call {
+    const exhip_conv_desc* d;
+    const uint16_t* x;
+    const void* w_packed;
+    const float* bias;
+    uint16_t* y;
+} exhip_conv_f16_call;
+int exhip_conv2d_f16_pair(exhip_ctx* ctx, const exhip_conv_f16_call* a, const exhip_conv_f16_call* b);
+
 /* exhip_conv2d_i8 and the 2x2 stride-2 max pooling behind it (operation_pooling.cpp:145-159, windows inside the map: 2 * pool_oh <= output rows) as one launch;
  * y_i8 and / or y_f32 are the pooled NHWC results. EXHIP_ERR_UNSUPPORTED, with nothing launched, where the two run by themselves. */
 int exhip_conv2d_i8_maxpool2x2(exhip_ctx* ctx, const exhip_conv_desc* d, int pool_oh, int pool_ow, const int8_t* x_nhwc, const void* w_packed,

@@ -1,0 +1,120 @@
+"""Two pointwise layers that do not read each other's results in one launch (exhip_conv2d_i8_pair, exhip_conv2d_f16_pair): the bytes of the layers
+run by themselves, whichever forms the two have, and also where they do run by themselves."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from excalibur_amd import hip, modelfile, topologies
+from excalibur_amd import pipeline as xp
+
+pytestmark = pytest.mark.gpu
+
+
+class CallI8(ctypes.Structure):
+    _fields_ = [(name, ctypes.c_void_p) for name in ("d", "x", "w", "scale", "bias", "y_i8", "y_f32")]
+
+
+class CallF16(ctypes.Structure):
+    _fields_ = [(name, ctypes.c_void_p) for name in ("d", "x", "w", "bias", "y")]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = hip.Ctx(0)
+    yield c
+    c.close()
+
+
+LAYERS = {
+    # n, h, w, channels, output channels, kernel: forms of one wave to 64 pixels or to 64 channels, with and without pairs of k-steps, and four waves to a tile
+    "narrow": (2, 9, 13, 32, 32, 1),
+    "narrow pairs": (1, 24, 11, 128, 32, 1),
+    "wide": (1, 7, 5, 64, 96, 1),
+    "wide pairs": (3, 30, 31, 256, 64, 1),
+    "split": (1, 10, 10, 512, 128, 1),
+    "split ragged": (1, 6, 7, 320, 160, 1),
+    "filter": (1, 8, 8, 64, 64, 3),
+}
+
+
+def layer(ctx, spec, int8, seed, plain):
+    n, h, w, c, k, kernel = spec
+    r = np.random.default_rng(seed)
+    arrays = [r.normal(0, 1, k).astype(np.float32) for _ in range(3)]
+    post = {} if plain else dict(post_op="leakyrelu" if int8 else "hardswish", post_alpha=.1 if int8 else 1 / 6, post_beta=.5)
+    bias, a, b = (ctx.array(v) for v in arrays)
+    if int8:
+        post.update(fs_out=15.0, exact_k=int(kernel == 1 and not plain))
+        if kernel == 1 and not plain:
+            post.update(post_bn=(a, b))
+    d = ctx.conv_desc(n, c, h, w, k, kernel, 1, kernel // 2, c_stride=c, k_stride=k, **post)
+    if int8:
+        x, wt = r.integers(-127, 128, (n, h, w, c), dtype=np.int8), r.integers(-127, 128, (k, c, kernel, kernel), dtype=np.int8)
+        scale = ctx.array(np.full(k, 1 / (127 * 73 * np.sqrt(c * kernel * kernel)), np.float32))
+    else:
+        x, wt = (v.astype(np.float16).view(np.uint16) for v in (r.normal(0, 1, (n, h, w, c)), r.normal(0, c ** -.5, (k, c, kernel, kernel))))
+    xd, wp = ctx.array(x), ctx.pack_conv_weights(d, hip.I8 if int8 else hip.F16, wt)
+
+    def call():
+        y = ctx.array(np.full(n * h * w * k + 64, 0x55, np.int8 if int8 else np.uint16))
+        if int8:
+            return y, CallI8(ctypes.addressof(d), xd.ptr, wp.ptr, scale.ptr, bias.ptr, y.ptr, None)
+        return y, CallF16(ctypes.addressof(d), xd.ptr, wp.ptr, bias.ptr, y.ptr)
+
+    def alone():
+        y, _ = call()
+        if int8:
+            ctx.conv2d_i8(d, xd, wp, scale, bias, None, y)
+        else:
+            ctx.conv2d_f16(d, xd, wp, bias, None, y)
+        return y.download()
+    call.keep = (d, xd, wp, bias, a, b) + ((scale,) if int8 else ())
+    return call, alone
+
+
+@pytest.mark.parametrize("int8", [True, False], ids=["int8", "fp16"])
+@pytest.mark.parametrize("second", LAYERS)
+@pytest.mark.parametrize("first", LAYERS)
+def test_two_layers(ctx, first, second, int8):
+    # int8: both with the BatchNorm and LeakyReLU of a joined Concat behind them, fp16: nothing; then a layer that has something else behind it
+    for plain in ((False, False), (False, True)) if int8 else ((True, True), (True, False)):
+        made = [layer(ctx, LAYERS[name], int8, seed, p) for name, seed, p in zip((first, second), (1, 2), plain)]
+        want = [alone() for _, alone in made]
+        (ya, a), (yb, b) = made[0][0](), made[1][0]()
+        run = hip.lib().exhip_conv2d_i8_pair if int8 else hip.lib().exhip_conv2d_f16_pair
+        hip._check(run(ctx.h, ctypes.byref(a), ctypes.byref(b)))
+        ctx.sync()
+        for got, expected in zip((ya, yb), want):
+            assert np.array_equal(got.download(), expected) and np.unique(expected).size > 10
+
+
+def test_an_error_of_either_layer_is_reported(ctx):
+    call, alone = layer(ctx, LAYERS["wide"], False, 1, True)
+    want = alone()
+    for bad_first in (True, False):
+        (y, good), (_, bad) = call(), call()
+        bad.y = None
+        pair = (bad, good) if bad_first else (good, bad)
+        assert hip.lib().exhip_conv2d_f16_pair(ctx.h, ctypes.byref(pair[0]), ctypes.byref(pair[1])) != 0
+        ctx.sync()
+        if not bad_first:
+            assert np.array_equal(y.download(), want)
+
+
+@pytest.mark.parametrize("int8", [True, False], ids=["int8", "fp16"])
+def test_a_detection_network(tmp_path, int8):
+    text, outs = topologies.yolov5s_simp(128, int8=int8)
+    path = str(tmp_path / "net.racy")
+    modelfile.write_model(path, modelfile.SeededModel(modelfile.parse_topology(text), 5, default_fs=16.0, gain=2.0).blobs)
+    x = np.random.default_rng(3).integers(0, 256, (3, 3, 128, 128))
+    x = x.astype(np.float32) if int8 else x.astype(np.float16).view(np.uint16)
+    got = []
+    for fusion in (True, False):
+        pipe = xp.Pipeline(text, path, 0, "f32" if int8 else "f16", fusion=fusion)
+        for _ in range(2):
+            pipe.set_input(x)
+            pipe.run()
+        got.append([pipe.get(name) for name in outs])
+    for a, b in zip(*got):
+        assert a.tobytes() == b.tobytes() if int8 else np.array_equal(a.view(np.float16), b.view(np.float16))
