@@ -209,7 +209,7 @@ __global__ __launch_bounds__(64 * WK * WP, 3) void conv3x3_staged_kernel(const S
 #pragma unroll
         for (int i = 0; i < BATCH; ++i) {
             const int at = first + i * PASS + my_pixel;
-            x[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(xr, at < staged ? table[at] + my_piece * 16 : kOutOfRange, chunk * BYTES, 0));
+            x[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(xr, at < staged && chunk * BYTES + my_piece * 16 < p.xs_b ? table[at] + my_piece * 16 : kOutOfRange, chunk * BYTES, 0));
         }
     };
     auto store_batch = [&](int first) {
@@ -582,6 +582,9 @@ Plan plan_of(int dt, const PwParams& p, long long images, int subs, int kblocks)
 //    float32 results 1.02 to 1.6, with them from 80 K of work on (1.03 to 1.4, below 0.96 to 1.0). A shortcut with ReLU: 1.0 to 1.3 up to 128 K of work,
 //    beyond only what the lean kernel cannot take (64 -> 64 0.8, 192 -> 64 at 7 x 92 x 92 0.85). A ReLU alone, which the lean kernel has forms for: from 72 k-steps on
 //    1.06 to 1.19 up to 128 K, 0.74 to 0.98 beyond and below; ragged channels, which it cannot take, 0.98 to 1.17.
+//    Channels in odd thirty-twos, of which half a piece of products is for nothing and which the lean kernel has no form for: from 160 on 1.1 to 2.0
+//    (160 -> 96 at 2 x 80 x 80 with HardSwish 16.5 -> 8.9, with a ReLU 12.3 -> 9.1; 760 blocks 0.94, 784 1.12), 96 where the launch is large (96 -> 160 at
+//    8 x 66 x 66 18.0 -> 14.1, with a ReLU 0.95; 1800 blocks 0.9), 32 never (0.7 to 0.9).
 //  * int8 at stride 2: 0.7 to 1.3 without a line between them; left alone.
 bool exhip_staged_wins(int dt, const exhip_pw_geom& g, int stride, int n_ksteps, bool shortcut, bool y_f) {
     const exhip_options& o = g_exhip_options;  // (an option that pins another kernel's form is for that kernel)
@@ -594,6 +597,7 @@ bool exhip_staged_wins(int dt, const exhip_pw_geom& g, int stride, int n_ksteps,
     if (blocks <= (dt == EXHIP_F16 && ks < 72 ? 1024 : 512)) return false;
     if (dt == EXHIP_F16) return stride == 1 || (ks >= 72 ? blocks > 1280 : (kblocks <= 3 && blocks >= 1536) || blocks >= 12288);
     if (stride == 2 || work < 41 * 1024) return false;
+    if (g.c_bytes % 64 != 0) return ks >= 45 ? blocks > 768 : ks >= 27 && blocks > 4096 && (g.post_op || shortcut || y_f || !(g.act || g.post_relu));
     const bool mid = work <= 128 * 1024 || g.k % 64 != 0;
     if (g.post_op) return ks >= 36 || (!shortcut && !y_f) || work >= 80 * 1024;
     if (shortcut) return ks >= 36 && mid;
@@ -604,10 +608,10 @@ bool exhip_staged_wins(int dt, const exhip_pw_geom& g, int stride, int n_ksteps,
 
 int exhip_conv3x3_staged(exhip_ctx* ctx, int dt, const void* pw_params, long long images, int kblocks, int lean_tiles) {
     const PwParams& p = *static_cast<const PwParams*>(pw_params);
-    const int option = g_exhip_options.staged, subs = p.xs_b / 64;
+    const int option = g_exhip_options.staged, subs = (p.xs_b + 63) / 64;
     const int widest = dt == EXHIP_F16 ? 2 : p.y_f || p.residual_f ? 4 : 1;  // bytes of an output (or shortcut) value
     if ((long long)p.pixels * p.kstride * widest >= kOutOfRange || p.kh != 3 || p.kw != 3 || (p.stride != 1 && (p.stride != 2 || dt != EXHIP_F16)) ||
-        p.xs_b % 64 != 0 || p.pool || p.group || p.exact || kblocks < 2)
+        (p.xs_b % 64 != 0 && dt != EXHIP_I8) || p.pool || p.group || p.exact || kblocks < 2)
         return EXHIP_ERR_UNSUPPORTED;
     Plan plan;
     if (option > 1) {
@@ -624,6 +628,7 @@ int exhip_conv3x3_staged(exhip_ctx* ctx, int dt, const void* pw_params, long lon
     }
     StagedParams q = {};
     q.f = p;
+    // (int8 pixels that end with half a piece: the other half is staged as zeros, whatever weights its products read)
     q.subs = subs;
     q.tap_w = p.mts * (p.chunk_b == 64 ? 2048 : 1024);
     q.half_w = p.mts * (p.chunk_b == 64 ? 1024 : 9 * 1024);

@@ -33,6 +33,9 @@ SHAPES = [
     (1, 128, 24, 50, 96, 2, (0, 1, 0, 1)),
     (7, 96, 5, 4, 64, 2, (1, 1, 1, 1)),       # fp16: the packing's chunks are half a piece
     (1, 32, 33, 70, 72, 2, (1, 1, 1, 1)),
+    (2, 160, 11, 9, 96, 1, (1, 1, 1, 1)),     # int8: the last piece of 64 bytes half full
+    (1, 32, 20, 31, 64, 1, (1, 1, 1, 1)),
+    (1, 288, 5, 23, 64, 1, (2, 0, 1, 1)),
 ]
 KINDS = {
     "none": {}, "act": dict(act=1), "relu": dict(post_relu=1), "hardswish": dict(post_op="hardswish", post_alpha=1 / 6, post_beta=.5),
@@ -92,7 +95,7 @@ def results(ctx, shape, kind, int8, wider, floats, values):
 
 
 @pytest.mark.parametrize("kind", KINDS)
-@pytest.mark.parametrize("shape", [s for s in SHAPES if s[5] == 1 and s[1] % 64 == 0], ids=lambda s: "x".join(map(str, s[:6])))
+@pytest.mark.parametrize("shape", [s for s in SHAPES if s[5] == 1], ids=lambda s: "x".join(map(str, s[:6])))
 def test_int8_equals_the_other_kernels(ctx, staged, shape, kind):
     for wider, floats in ((0, False), (1, True)):
         run, _ = results(ctx, shape, kind, True, wider, floats, "")
