@@ -1739,7 +1739,9 @@ int run_conv(exhip_ctx* ctx, const exhip_conv_desc* d, ConvParams p, const PoolS
     };
     const bool lean_shape = !pl.packed && !pool && d->kh == 3 && d->kw == 3 && d->sh == 1 && d->sw == 1 && pl.variant == 0 && pl.chunk_b == 64 && pl.RS == 1 &&
                             p.cstride_b % 64 == 0;
-    if (!pl.packed && !pool && !proj && !joined && pl.KWe == 3 && d->kw == 3 && d->kh == 3 && d->sh == d->sw && !p.acc_nchw && !p.y_nchw && !p.y_nchw_h &&
+    // (a small launch is known by its blocks alone: it pays for nothing else here)
+    const bool large = d->kh == 3 && (((long long)d->n * pl.OH * pl.OW + 31) / 32 * ((std::max(d->k, d->k_stride) + 31) / 32) > kStagedBlocks || g_exhip_options.staged > 1);
+    if (large && !pl.packed && !pool && !proj && !joined && pl.KWe == 3 && d->kw == 3 && d->kh == 3 && d->sh == d->sw && !p.acc_nchw && !p.y_nchw && !p.y_nchw_h &&
         (p.y_q || (DT == EXHIP_I8 && p.y_nhwc))) {
         // 3x3 layers whose input under a run of pixels LDS holds, where that is the fastest way
         exhip_pw_geom g;

@@ -594,7 +594,7 @@ bool exhip_staged_wins(int dt, const exhip_pw_geom& g, int stride, int n_ksteps,
         return false;
     const int kblocks = std::min(g.slabs * g.slab_blocks, (std::max(g.k, g.k_stride) + 31) / 32), ks = n_ksteps;
     const long long blocks = (g.pixels + 31) / 32 * kblocks, work = blocks * ks;
-    if (blocks <= (dt == EXHIP_F16 && ks < 72 ? 1024 : 512)) return false;
+    if (blocks <= (dt == EXHIP_F16 && ks < 72 ? 1024 : kStagedBlocks)) return false;
     if (dt == EXHIP_F16) return stride == 1 || (ks >= 72 ? blocks > 1280 : (kblocks <= 3 && blocks >= 1536) || blocks >= 12288);
     if (stride == 2 || work < 41 * 1024) return false;
     if (g.c_bytes % 64 != 0) return ks >= 45 ? blocks > 768 : ks >= 27 && blocks > 4096 && (g.post_op || shortcut || y_f || !(g.act || g.post_relu));
