@@ -1661,6 +1661,7 @@ bool pipeline<float>::impl::build_graph_plan(const tensor_ptr& input, const std:
         const float *scale, *bias;
         int8_t* yq;
         size_t launch;
+        const int8_t *joined, *joined_end;  // the whole Concat
     } beside = {};
     for (const node& nd : nodes) {
         results_complete();
@@ -1716,8 +1717,10 @@ bool pipeline<float>::impl::build_graph_plan(const tensor_ptr& input, const std:
                 const int rc = exhip_conv2d_i8(ctx, &d, x, wp, scale, bias, nullptr, yq, nullptr, nullptr, nullptr);  // trial launch
                 if (rc == EXHIP_ERR_UNSUPPORTED) return refuse(__LINE__);
                 EXHIP_FATAL(rc);
-                const joined_layer own = {d, x, wp, scale, bias, yq, plan->launches.size()};
-                if (beside.wp && beside.launch + 1 == own.launch && x != beside.yq) {  // the layer in front writes its part of a joined Concat too: both in one launch
+                const int8_t* const joined = static_cast<const int8_t*>(jo.i8);
+                const joined_layer own = {d, x, wp, scale, bias, yq, plan->launches.size(), joined, joined + static_cast<size_t>(jo.n) * oh * ow * total};
+                // the layer in front writes its part of a joined Concat too, which this one does not read: both in one launch
+                if (beside.wp && beside.launch + 1 == own.launch && (x < beside.joined || x >= beside.joined_end)) {
                     const joined_layer other = beside;
                     plan->launches.back() = [=]() {
                         const exhip_conv_i8_call a = {&other.d, other.x, other.wp, other.scale, other.bias, other.yq, nullptr}, b = {&own.d, own.x, own.wp, own.scale, own.bias, own.yq, nullptr};

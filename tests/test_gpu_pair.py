@@ -118,3 +118,24 @@ def test_a_detection_network(tmp_path, int8):
         got.append([pipe.get(name) for name in outs])
     for a, b in zip(*got):
         assert a.tobytes() == b.tobytes() if int8 else np.array_equal(a.view(np.float16), b.view(np.float16))
+
+
+def test_a_layer_that_reads_the_concat_in_front_is_not_paired_with_its_last_writer(tmp_path):
+    conv = lambda name, src, dst, c, k, kernel=1: f"Convolution {name} 1 1 {src} {dst} 0={k} 1={kernel} 11={kernel} 2=1 12=1 3=1 13=1 4={kernel // 2} 14={kernel // 2} 15={kernel // 2} 16={kernel // 2} 5=1 6={c * k * kernel * kernel} 8=2"
+    lines = ["Input in 0 1 in 0=24 1=24 2=3 3=0,0,0 4=0.0039215", conv("first", "in", "f", 3, 32, 3), "Split s 1 3 f f0 f1 f2", conv("a", "f0", "a", 32, 32), conv("x", "f1", "x0", 32, 64),
+             "HardSwish hx 1 1 x0 x 0=1.666667e-01 1=5.000000e-01", conv("b", "x", "b", 64, 32), "Concat p 2 1 a b p 0=-1", conv("c", "p", "c", 64, 32), conv("d", "f2", "d", 32, 32),
+             "Concat q 2 1 c d q 0=-1", conv("e", "q", "e", 64, 32)]
+    blobs = sum(int(line.split()[3]) for line in lines)
+    text = "glsv1\n%d %d\n%s\n" % (len(lines), blobs, "\n".join(lines))
+    path = str(tmp_path / "net.racy")
+    modelfile.write_model(path, modelfile.SeededModel(modelfile.parse_topology(text), 5, default_fs=16.0, gain=2.0).blobs)
+    x = np.random.default_rng(3).integers(0, 256, (4, 3, 24, 24)).astype(np.float32)
+    got = []
+    for fusion in (True, False):
+        pipe = xp.Pipeline(text, path, 0, "f32", fusion=fusion)
+        for _ in range(2):
+            pipe.set_input(x)
+            pipe.run()
+        got.append(pipe.get("e"))
+        assert pipe.fused == fusion
+    assert np.array_equal(*got) and np.ptp(got[0]) > 0
