@@ -212,29 +212,34 @@ __device__ __forceinline__ void epilogue_block(const F32Params& p, const v16f& a
 }
 
 // R: requested steps in flight. PAIRS: the pixels in 64-byte pieces, two steps at a time.
-template <int MT, int NT, int WK, int R, int MODE, bool PAIRS, bool SLOW>
-__global__ __launch_bounds__(WK > 4 ? 64 * WK : 256, 2) void conv_f32_kernel(const F32Params p) {
-    exhip_touch_args(p);
-    constexpr int WAVES = WK > 4 ? WK : 4, ITEMS = WAVES / WK;  // tiles per group
-    constexpr int BLOCKS = MT * NT;
+template <int MT, int NT, int WK>
+struct F32Shape {
+    static constexpr int WAVES = WK > 4 ? WK : 4, ITEMS = WAVES / WK;  // tiles per group
+    static constexpr int BLOCKS = MT * NT;
     // A wave of a split tile finishes a block, and stores its rows through LDS, or where that leaves every block to four waves or more a
     // quarter of one (four channels a lane), and stores from registers. Halves from registers fill lines in pieces of 32 bytes, and launches
     // of two waves a block are still large: 64 -> 64 3x3 at 24 x 40 x 40 33.8 us in halves, 28.9 in blocks, 128 -> 128 at 4 x 80 x 80 73.7 and
     // 64.3, 1x1 64 -> 64 at 8 x 80 x 80 12.9 and 11.1.
-    constexpr bool ROWS = WK == 1 || WK < 4 * BLOCKS;
-    constexpr int QUADS = ROWS ? 4 : 1, V = 4 * QUADS;            // WK > 1: quarters of a block that a wave finishes
-    constexpr int OWNERS = WK > 1 ? BLOCKS : 1;                   // ROWS: waves of a tile that finish a block
-    constexpr int RED = WK > 1 ? WAVES * BLOCKS * 4096 : 0;       // the waves' partial sums
+    static constexpr bool ROWS = WK == 1 || WK < 4 * BLOCKS;
+    static constexpr int OWNERS = WK > 1 ? BLOCKS : 1;              // ROWS: waves of a tile that finish a block
+    static constexpr int RED = WK > 1 ? WAVES * BLOCKS * 4096 : 0;  // the waves' partial sums
+    static constexpr int LDS = RED + (ROWS ? ITEMS * OWNERS * wave_lds(MT) : 0);
     static_assert(WK == 1 || OWNERS <= WK, "a wave finishes at most one block");
-    __shared__ __attribute__((aligned(16))) char lds_all[RED + (ROWS ? ITEMS * OWNERS * wave_lds(MT) : 0)];
+};
+// (the kernel's group `bid` of `groups`)
+template <int MT, int NT, int WK, int R, int MODE, bool PAIRS, bool SLOW>
+__device__ __forceinline__ void f32_group(const F32Params& p, char* lds_all, unsigned bid, unsigned groups) {
+    typedef F32Shape<MT, NT, WK> Shape;
+    constexpr int ITEMS = Shape::ITEMS, BLOCKS = Shape::BLOCKS, OWNERS = Shape::OWNERS, RED = Shape::RED;
+    constexpr bool ROWS = Shape::ROWS;
+    constexpr int QUADS = ROWS ? 4 : 1, V = 4 * QUADS;            // WK > 1: quarters of a block that a wave finishes
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int part = wave % WK;
     // workgroup ids are dealt round-robin to the 8 XCDs: give each XCD one contiguous run of items. Either the channel groups of
     // a pixel tile run fastest, and an XCD reads its share of the pixels and all weights, or the pixel tiles do (tiles_fast)
     // and it reads its share of the weights and all pixels.
-    unsigned bid = blockIdx.x;
     {
-        const unsigned per = gridDim.x >> 3;
+        const unsigned per = groups >> 3;
         if (bid < (per << 3)) bid = (bid & 7) * per + (bid >> 3);
     }
     const unsigned item = __builtin_amdgcn_readfirstlane(bid * ITEMS + wave / WK);
@@ -498,6 +503,55 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256, 2) void conv_f32_kernel(con
 }
 
 template <int MT, int NT, int WK, int R, int MODE, bool PAIRS, bool SLOW>
+__global__ __launch_bounds__(WK > 4 ? 64 * WK : 256, 2) void conv_f32_kernel(const F32Params p) {
+    exhip_touch_args(p);
+    __shared__ __attribute__((aligned(16))) char lds_all[F32Shape<MT, NT, WK>::LDS];
+    f32_group<MT, NT, WK, R, MODE, PAIRS, SLOW>(p, lds_all, blockIdx.x, gridDim.x);
+}
+
+// Two pointwise layers that do not read each other's results in one launch, each in its own form, as conv_pw_two_kernel (conv_pw.hip): a layer
+// of a few hundred groups is bounded by its chain of loads and by the gap to the next launch, and two of them fill each other's. The forms are
+// those that a detector's neighbours take; any other runs by itself. The layers' parameters are arguments of their own: chosen from an array
+// by number they were copied to scratch (792 bytes per lane, 28 - 50 us a launch). Two launches and one, us: 64 and 128 -> 64 channels at
+// 1 x 80 x 80 9.7 -> 6.4, at 3 x 80 x 80 14.6 -> 12.2, at 8 x 80 x 80 28.0 -> 27.1; 256 and 512 -> 256 at 1 x 20 x 20 10.1 -> 6.0, at 3
+// 13.9 -> 10.6, at 8 21.1 -> 17.4.
+struct F32Two {
+    int kind[2];
+    unsigned groups[2];
+};
+// the forms by number, -1 for all others
+template <int MT, int NT, int WK, int R, int MODE, bool PAIRS, bool SLOW>
+constexpr int two_kind() {
+    if (MODE != 0 || !PAIRS || SLOW || NT != 1 || R != 8) return -1;
+    return MT == 2 ? (WK == 1 ? 0 : WK == 2 ? 1 : WK == 4 ? 2 : -1) : WK == 2 ? 3 : WK == 4 ? 4 : -1;
+}
+constexpr int kTwoLds = F32Shape<2, 1, 2>::LDS;
+__device__ __forceinline__ void two_group(const F32Params& p, int kind, char* lds, unsigned bid, unsigned groups) {
+    exhip_touch_args(p);
+    if (kind == 0) f32_group<2, 1, 1, 8, 0, true, false>(p, lds, bid, groups);
+    else if (kind == 1) f32_group<2, 1, 2, 8, 0, true, false>(p, lds, bid, groups);
+    else if (kind == 2) f32_group<2, 1, 4, 8, 0, true, false>(p, lds, bid, groups);
+    else if (kind == 3) f32_group<1, 1, 2, 8, 0, true, false>(p, lds, bid, groups);
+    else f32_group<1, 1, 4, 8, 0, true, false>(p, lds, bid, groups);
+}
+__global__ __launch_bounds__(256, 2) void conv_f32_two_kernel(const F32Params a, const F32Params b, const F32Two q) {
+    static_assert(F32Shape<2, 1, 1>::LDS <= kTwoLds && F32Shape<2, 1, 4>::LDS <= kTwoLds && F32Shape<1, 1, 2>::LDS <= kTwoLds && F32Shape<1, 1, 4>::LDS <= kTwoLds, "one LDS for all");
+    __shared__ __attribute__((aligned(16))) char lds[kTwoLds];
+    const unsigned first = q.groups[0];
+    if (blockIdx.x < first) two_group(a, q.kind[0], lds, blockIdx.x, first);
+    else two_group(b, q.kind[1], lds, blockIdx.x - first, q.groups[1]);
+}
+
+// A launch that waits for another one to share it with (exhip_conv2d_f32_pair).
+struct Waiting {
+    int kind = -1;
+    unsigned groups = 0;
+    const void* kernel = nullptr;
+    F32Params p;
+};
+thread_local Waiting* t_collect = nullptr;  // while the pair's layers are run: the place for the next launch
+
+template <int MT, int NT, int WK, int R, int MODE, bool PAIRS, bool SLOW>
 int go(exhip_ctx* ctx, F32Params& p, int kblocks) {
     const long long tiles = ((long long)p.pixels + 32 * NT - 1) / (32 * NT);
     const long long groups = (kblocks + MT - 1) / MT, items = tiles * groups;
@@ -516,7 +570,17 @@ int go(exhip_ctx* ctx, F32Params& p, int kblocks) {
         p.start_r[i] = tap / taps_w;
         p.start_q[i] = tap % taps_w * (MODE == kPair ? 2 : 1);
     }
-    constexpr int WAVES = WK > 4 ? WK : 4, ITEMS = WAVES / WK;
+    constexpr int WAVES = F32Shape<MT, NT, WK>::WAVES, ITEMS = F32Shape<MT, NT, WK>::ITEMS;
+    if constexpr (two_kind<MT, NT, WK, R, MODE, PAIRS, SLOW>() >= 0) {
+        if (t_collect) {
+            t_collect->kind = two_kind<MT, NT, WK, R, MODE, PAIRS, SLOW>();
+            t_collect->groups = (p.items + ITEMS - 1) / ITEMS;
+            t_collect->kernel = reinterpret_cast<const void*>(conv_f32_kernel<MT, NT, WK, R, MODE, PAIRS, SLOW>);
+            t_collect->p = p;
+            t_collect = nullptr;
+            return 0;
+        }
+    }
     hipLaunchKernelGGL((conv_f32_kernel<MT, NT, WK, R, MODE, PAIRS, SLOW>), dim3((p.items + ITEMS - 1) / ITEMS), dim3(64 * WAVES), 0, ctx->stream, p);
     EXHIP_LAUNCH_CHECK();
     return 0;
@@ -716,4 +780,37 @@ extern "C" int exhip_conv2d_f32_placed(exhip_ctx* ctx, const exhip_conv_desc* d,
                                        const float* bias, const float* residual, float* y, float* y_f32_nchw) {
     EXHIP_REQUIRE(place, "exhip_conv2d_f32_placed: NULL placement");
     return run_conv_f32(ctx, d, place, x, wp, bias, residual, y, y_f32_nchw);
+}
+
+static int run_pair(exhip_ctx* ctx, int (*layer)(exhip_ctx*, const void*), const void* first, const void* second) {
+    Waiting w[2];
+    int rc = 0;
+    for (int i = 0; i < 2 && !rc; ++i) {
+        t_collect = &w[i];
+        rc = layer(ctx, i ? second : first);
+        t_collect = nullptr;
+    }
+    // (a layer that ran by itself is done; it reads nothing of the other's)
+    if (!rc && w[0].kind >= 0 && w[1].kind >= 0 && (long long)w[0].groups + w[1].groups < (1ll << 31)) {
+        const F32Two q = {{w[0].kind, w[1].kind}, {w[0].groups, w[1].groups}};
+        hipLaunchKernelGGL(conv_f32_two_kernel, dim3(w[0].groups + w[1].groups), dim3(256), 0, ctx->stream, w[0].p, w[1].p, q);
+        EXHIP_LAUNCH_CHECK();
+        return 0;
+    }
+    for (Waiting& one : w) {
+        if (one.kind < 0) continue;
+        void* args[] = {&one.p};
+        EXHIP_CHECK(hipLaunchKernel(one.kernel, dim3(one.groups), dim3(256), args, 0, ctx->stream));
+        EXHIP_LAUNCH_CHECK();
+    }
+    return rc;
+}
+
+extern "C" int exhip_conv2d_f32_pair(exhip_ctx* ctx, const exhip_conv_f32_call* a, const exhip_conv_f32_call* b) {
+    EXHIP_REQUIRE(ctx && a && b && a->d && a->place && b->d && b->place, "exhip_conv2d_f32_pair: NULL argument");
+    auto layer = [](exhip_ctx* on, const void* call) {
+        const auto* c = static_cast<const exhip_conv_f32_call*>(call);
+        return exhip_conv2d_f32_placed(on, c->d, c->place, c->x, c->w_packed, c->bias, c->residual, c->y, c->y_nchw);
+    };
+    return run_pair(ctx, layer, a, b);
 }

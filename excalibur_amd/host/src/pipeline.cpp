@@ -2365,6 +2365,18 @@ bool pipeline<float>::impl::build_float_plan(const tensor_ptr& input, const std:
         for (auto& r : plan->outputs)
             if (r.launch < 0) r.launch = static_cast<int>(plan->launches.size()) - 1;
     };
+    struct placed_layer {  // a convolution's launch, and the value it writes or, of a Concat's part, the Concat
+        exhip_conv_desc d;
+        exhip_conv_place how;
+        const float* x;
+        const void* wp;
+        const float *bias, *res;
+        float *y, **slot;
+        bool slot_is_rows;
+        size_t launch;
+        int value;
+        exhip_conv_f32_call call() const { return {&d, &how, x, wp, bias, res, slot_is_rows ? *slot : y, slot && !slot_is_rows ? *slot : nullptr}; }
+    } beside = {};
     for (const node& nd : nodes) {
         results_complete();
         const value_info in = vals[nd.in[0]];
@@ -2438,6 +2450,24 @@ bool pipeline<float>::impl::build_float_plan(const tensor_ptr& input, const std:
             const void* wp = c->pin_packed_weights(EXHIP_F32, d);  // the launch keeps this pointer
             plan->pinned.emplace_back([c, wp]() { c->unpin_packed_weights(wp); });
             const float *bias = c->bias_gpu(), *x = in.p;
+            // the layer in front and this one in one launch where both are pointwise and this one reads nothing of that one's: not its result, and not the Concat it is part of
+            auto whole = [&](int value) {
+                while (value >= 0 && vals[value].parent >= 0) value = vals[value].parent;
+                return value;
+            };
+            const int sum = nd.res >= 0 && vals[nd.res].through >= 0 ? vals[nd.res].through : nd.res;
+            const placed_layer own = {d, how, x, wp, bias, res, y, slot, slot_is_rows, plan->launches.size(), whole(nd.out)};
+            const bool pointwise = d.kh == 1 && d.kw == 1 && d.sh == 1 && !d.pt && !d.pb && !d.pl && !d.pr;
+            if (pointwise && beside.wp && beside.launch + 1 == own.launch && whole(nd.in[0]) != beside.value && (sum < 0 || whole(sum) != beside.value)) {
+                const placed_layer other = beside;
+                plan->launches.back() = [=]() {
+                    const exhip_conv_f32_call a = other.call(), b = own.call();
+                    EXHIP_FATAL(exhip_conv2d_f32_pair(ctx, &a, &b));
+                };
+                beside = {};
+                continue;
+            }
+            beside = pointwise ? own : placed_layer{};
             plan->launches.push_back([=]() {
                 EXHIP_FATAL(exhip_conv2d_f32_placed(ctx, &d, &how, x, wp, bias, res, slot_is_rows ? *slot : y, slot && !slot_is_rows ? *slot : nullptr));
             });

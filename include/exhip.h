@@ -310,6 +310,16 @@ typedef struct exhip_conv_place {
 } exhip_conv_place;
 int exhip_conv2d_f32_placed(exhip_ctx* ctx, const exhip_conv_desc* d, const exhip_conv_place* place, const float* x_nhwc, const void* w_packed,
                             const float* bias, const float* residual_nhwc, float* y, float* y_f32_nchw);
+/* Two layers of which neither reads what the other writes: the values of exhip_conv2d_f32_placed for each, pointwise ones in one launch. */
+typedef struct exhip_conv_f32_call {
+    const exhip_conv_desc* d;
+    const exhip_conv_place* place;
+    const float* x;
+    const void* w_packed;
+    const float *bias, *residual;
+    float *y, *y_nchw;
+} exhip_conv_f32_call;
+int exhip_conv2d_f32_pair(exhip_ctx* ctx, const exhip_conv_f32_call* a, const exhip_conv_f32_call* b);
 
 /* Any geometry incl. groups, straight from the definition on NCHW f32 (slow; used for shapes the
  * MFMA path does not take). int8 mode when w_i8 != NULL: quantizes x with fs on the fly and applies

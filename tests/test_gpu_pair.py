@@ -1,4 +1,4 @@
-"""Two pointwise layers that do not read each other's results in one launch (exhip_conv2d_i8_pair, exhip_conv2d_f16_pair): the bytes of the layers
+"""Two pointwise layers that do not read each other's results in one launch (exhip_conv2d_i8_pair, exhip_conv2d_f16_pair, exhip_conv2d_f32_pair): the bytes of the layers
 run by themselves, whichever forms the two have, and also where they do run by themselves."""
 import ctypes
 
@@ -100,6 +100,46 @@ def test_an_error_of_either_layer_is_reported(ctx):
         ctx.sync()
         if not bad_first:
             assert np.array_equal(y.download(), want)
+
+
+class Place(ctypes.Structure):
+    _fields_ = [(name, ctypes.c_int) for name in ("layout", "group", "residual_stride", "residual_shift", "bn_relu")]
+
+
+class CallF32(ctypes.Structure):
+    _fields_ = [(name, ctypes.c_void_p) for name in ("d", "place", "x", "w", "bias", "residual", "y", "y_nchw")]
+
+
+def layer_f32(ctx, spec, seed, shortcut):
+    n, h, w, c, k, kernel = spec
+    r = np.random.default_rng(seed)
+    d = ctx.conv_desc(n, c, h, w, k, kernel, 1, kernel // 2, c_stride=c, k_stride=k, act=seed % 2)
+    place = Place(0, 0, k, 0, 0)
+    x, bias = (ctx.array(r.normal(0, 1, size).astype(np.float32)) for size in ((n, h, w, c), k))
+    res = ctx.array(r.normal(0, 1, (n, h, w, k)).astype(np.float32)) if shortcut else None
+    wp = ctx.pack_conv_weights(d, hip.F32, r.normal(0, c ** -.5, (k, c, kernel, kernel)).astype(np.float32))
+
+    def call():
+        y = ctx.array(np.full(n * h * w * k + 64, -77, np.float32))
+        return y, CallF32(ctypes.addressof(d), ctypes.addressof(place), x.ptr, wp.ptr, bias.ptr, res.ptr if shortcut else None, y.ptr, None)
+    call.keep = d, place, x, bias, res, wp
+    return call
+
+
+@pytest.mark.parametrize("second", LAYERS)
+@pytest.mark.parametrize("first", LAYERS)
+def test_two_float32_layers(ctx, first, second):
+    made = [layer_f32(ctx, LAYERS[name], seed, shortcut) for name, seed, shortcut in ((first, 1, False), (second, 2, True))]
+    want = []
+    for call in made:
+        y, c = call()
+        hip._check(hip.lib().exhip_conv2d_f32_placed(ctx.h, *(ctypes.c_void_p(getattr(c, name)) for name, _ in c._fields_)))
+        want.append(y.download())
+    (ya, a), (yb, b) = made[0](), made[1]()
+    hip._check(hip.lib().exhip_conv2d_f32_pair(ctx.h, ctypes.byref(a), ctypes.byref(b)))
+    ctx.sync()
+    for got, expected in zip((ya, yb), want):
+        assert np.array_equal(got.download(), expected) and np.ptp(expected[:-64]) > 1
 
 
 @pytest.mark.parametrize("int8", [True, False], ids=["int8", "fp16"])
