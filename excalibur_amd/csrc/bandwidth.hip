@@ -1196,6 +1196,51 @@ __global__ __launch_bounds__(kBlock) void pool2d_nhwc_f32_kernel(const float* __
     *reinterpret_cast<v4f*>(y + (size_t)pix * ys + c) = v;
 }
 
+// Two or three levels of stride-1 "same" 5 x 5 max pools, each of the one before: the windows 5, 9 and 13 of the input. A group keeps 4 * L
+// channels of a map in LDS, two buffers that rows and columns are taken between. The comparisons are pool2d_nhwc_f32_kernel's, from -FLT_MAX and
+// the first of equals, row by row: the same bits, and a NaN is taken by neither.
+// As three launches, each bound by the loads of its windows and by the gap to the next, and as one, us: 256 channels of three 13 x 13 maps 19.1 -> 5.0,
+// of sixteen 20 x 20 maps 36.9 -> 11.6, of four 40 x 40 maps 38.8 -> 24.4.
+struct PyramidF32 {
+    float* y[3];
+    int ys[3];
+};
+template <int L>
+__global__ __launch_bounds__(512) void maxpool_pyramid_nhwc_f32_kernel(const float* __restrict__ x, int xs, const PyramidF32 out, int levels, int H, int W, exhip_divisor by_w) {
+    __shared__ v4f map[2048], rows[2048];
+    const int px = H * W, items = px * L, ch = blockIdx.x * 4 * L;
+    const size_t image = (size_t)blockIdx.y * px;
+    for (int i = threadIdx.x; i < items; i += 512) map[i] = *reinterpret_cast<const v4f*>(x + (image + i / L) * xs + ch + i % L * 4);
+    __syncthreads();
+    auto maximum = [&](const v4f* line, int stride, int at, int count) {  // at clamped places: a border pixel more than once
+        v4f t[5], m = {-FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX};
+#pragma unroll
+        for (int d = 0; d < 5; ++d) t[d] = line[min(max(at + d - 2, 0), count - 1) * stride];
+#pragma unroll
+        for (int d = 0; d < 5; ++d)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) m[e] = m[e] < t[d][e] ? t[d][e] : m[e];
+        return m;
+    };
+    auto level = [&](float* y, int ys) {
+        for (int i = threadIdx.x; i < items; i += 512) {
+            const int p = i / L, row = (int)by_w((unsigned)p);
+            rows[i] = maximum(map + row * W * L + i % L, L, p - row * W, W);
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < items; i += 512) {
+            const int p = i / L, row = (int)by_w((unsigned)p);
+            const v4f m = maximum(rows + (p - row * W) * L + i % L, W * L, row, H);
+            map[i] = m;
+            *reinterpret_cast<v4f*>(y + (image + p) * ys + ch + i % L * 4) = m;
+        }
+        __syncthreads();
+    };
+    level(out.y[0], out.ys[0]);
+    level(out.y[1], out.ys[1]);
+    if (levels == 3) level(out.y[2], out.ys[2]);
+}
+
 // Global average pooling on NHWC float storage: a group per image and 16 channels. The sums are those of the NCHW kernel below:
 // pixels l, l + 64, ... for l = 0 .. 63, then a tree over the 64 partial sums.
 __global__ __launch_bounds__(kBlock) void global_avgpool_nhwc_f32_kernel(const float* __restrict__ x, float* __restrict__ y, int C, int xs, int ys, int HW) {
@@ -2658,6 +2703,31 @@ extern "C" int exhip_maxpool_pyramid_concat_nhwc_f16(exhip_ctx* ctx, const uint1
         hipLaunchKernelGGL(maxpool_pyramid_concat_nhwc_f16_kernel<2>, dim3((unsigned)(c / 16), (unsigned)n), dim3(512), 0, ctx->stream, x, y, h, w, c, by_w);
     else
         hipLaunchKernelGGL(maxpool_pyramid_concat_nhwc_f16_kernel<1>, dim3((unsigned)(c / 8), (unsigned)n), dim3(512), 0, ctx->stream, x, y, h, w, c, by_w);
+    EXHIP_LAUNCH_CHECK();
+    return 0;
+}
+
+extern "C" int exhip_maxpool_pyramid_nhwc_f32(exhip_ctx* ctx, const float* x, int x_stride, float* y1, int y1_stride, float* y2, int y2_stride, float* y3, int y3_stride,
+                                              int n, int c, int h, int w) {
+    REQ_CTX("exhip_maxpool_pyramid_nhwc_f32");
+    EXHIP_REQUIRE(x && y1 && y2 && n > 0 && c > 0 && h > 0 && w > 0 && x_stride >= c && y1_stride >= c && y2_stride >= c && (!y3 || y3_stride >= c),
+                  "exhip_maxpool_pyramid_nhwc_f32: bad argument");
+    const uintptr_t all = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y1) | reinterpret_cast<uintptr_t>(y2) | reinterpret_cast<uintptr_t>(y3);
+    EXHIP_REQUIRE((all & 15) == 0 && ((x_stride | y1_stride | y2_stride | (y3 ? y3_stride : 0)) & 3) == 0, "exhip_maxpool_pyramid_nhwc_f32: pixels must be 16-byte aligned");
+    // (64 KiB hold the two buffers of 4 channels of 2048 pixels)
+    const long long px = (long long)h * w;
+    if (c % 4 != 0 || c > (1 << 20) || n > 65535 || px > 2048) return EXHIP_ERR_UNSUPPORTED;
+    exhip_divisor by_w;
+    by_w.set((unsigned)w);
+    const PyramidF32 out = {{y1, y2, y3}, {y1_stride, y2_stride, y3_stride}};
+    const int levels = y3 ? 3 : 2;
+    const long long quads = (long long)n * (c / 4);
+    // 64 bytes of a pixel at a time where that still gives every CU a group (256 channels of sixteen 20 x 20 maps 11.6 us, 32 bytes 13.8, 16 bytes 23.3), 32
+    // where it is every second one (of eight 9.5, the others 10.0 and 12.5); fewer groups are bounded by their own passes (of one 5.4, 32 bytes 6.8, 64 9.0)
+    auto run = [&](auto kernel, int l) { hipLaunchKernelGGL(kernel, dim3((unsigned)(c / 4 / l), (unsigned)n), dim3(512), 0, ctx->stream, x, x_stride, out, levels, h, w, by_w); };
+    if (c % 16 == 0 && px <= 512 && quads >= 4 * 256) run(maxpool_pyramid_nhwc_f32_kernel<4>, 4);
+    else if (c % 8 == 0 && px <= 1024 && quads >= 2 * 128) run(maxpool_pyramid_nhwc_f32_kernel<2>, 2);
+    else run(maxpool_pyramid_nhwc_f32_kernel<1>, 1);
     EXHIP_LAUNCH_CHECK();
     return 0;
 }

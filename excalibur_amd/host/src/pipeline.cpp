@@ -2365,6 +2365,11 @@ bool pipeline<float>::impl::build_float_plan(const tensor_ptr& input, const std:
         for (auto& r : plan->outputs)
             if (r.launch < 0) r.launch = static_cast<int>(plan->launches.size()) - 1;
     };
+    struct {  // the 5 x 5 max pools, each of the one before, whose launch is the plan's last one
+        value_info x, y[3];
+        int levels = 0;
+        size_t launch = 0;
+    } pyramid;
     struct placed_layer {  // a convolution's launch, and the value it writes or, of a Concat's part, the Concat
         exhip_conv_desc d;
         exhip_conv_place how;
@@ -2662,6 +2667,29 @@ bool pipeline<float>::impl::build_float_plan(const tensor_ptr& input, const std:
             const int rc = exhip_pool2d_nhwc_f32(ctx, src.p, src.cs, o.p, o.cs, in.n, ch, in.h, in.w, oh, ow, type, kh, kw, sh, sw, pt, pb, pl, pr, include_pad);
             if (rc == EXHIP_ERR_UNSUPPORTED) return refuse(__LINE__);
             EXHIP_FATAL(rc);
+            // 5 x 5 "same" maxima of the launch in front, which is such a level itself, join it: the map stays in LDS for all levels
+            const bool five = type == 0 && kh == 5 && kw == 5 && sh == 1 && sw == 1 && pt == 2 && pb == 2 && pl == 2 && pr == 2;
+            const bool joins = five && pyramid.levels > 0 && pyramid.levels < 3 && pyramid.launch + 1 == plan->launches.size() && src.p == pyramid.y[pyramid.levels - 1].p;
+            if (joins) {
+                auto py = pyramid;
+                py.y[py.levels++] = o;
+                auto run = [=]() {
+                    return exhip_maxpool_pyramid_nhwc_f32(ctx, py.x.p, py.x.cs, py.y[0].p, py.y[0].cs, py.y[1].p, py.y[1].cs, py.levels == 3 ? py.y[2].p : nullptr, py.y[2].cs,
+                                                          in.n, ch, in.h, in.w);
+                };
+                const int one = run();  // trial
+                if (one == 0) {
+                    plan->launches.back() = [=]() { EXHIP_FATAL(run()); };
+                    pyramid = py;
+                    nchw_from_rows(nd.out);
+                    continue;
+                }
+                if (one != EXHIP_ERR_UNSUPPORTED) EXHIP_FATAL(one);
+            }
+            pyramid.levels = 0;
+            if (five) {
+                pyramid.x = src; pyramid.y[0] = o; pyramid.levels = 1; pyramid.launch = plan->launches.size();
+            }
             plan->launches.push_back([=]() {
                 EXHIP_FATAL(exhip_pool2d_nhwc_f32(ctx, src.p, src.cs, o.p, o.cs, in.n, ch, in.h, in.w, oh, ow, type, kh, kw, sh, sw, pt, pb, pl, pr, include_pad));
             });

@@ -388,6 +388,11 @@ int exhip_maxpool_same_pyramid_nhwc_i8(exhip_ctx* ctx, const int8_t* x, int8_t* 
 /* The same pyramid on halves, windows 5, 9 and 13, with the Concat of the tensor and its three results behind it: y [n][h][w][4 c]. Tensors on 16 bytes;
  * EXHIP_ERR_UNSUPPORTED, with nothing launched, for c not a multiple of 8 and maps of more than 2048 pixels. */
 int exhip_maxpool_pyramid_concat_nhwc_f16(exhip_ctx* ctx, const uint16_t* x, uint16_t* y, int n, int c, int h, int w);
+/* Two or three (y3 != NULL) levels of stride-1 "same" 5 x 5 max pools on floats in one launch, each of the one before: y1, y2, y3 hold the maxima over
+ * windows 5, 9 and 13 of x. Strides in floats, multiples of 4, tensors on 16 bytes; EXHIP_ERR_UNSUPPORTED, with nothing launched, for c not a multiple
+ * of 4 and maps of more than 2048 pixels. */
+int exhip_maxpool_pyramid_nhwc_f32(exhip_ctx* ctx, const float* x, int x_stride, float* y1, int y1_stride, float* y2, int y2_stride, float* y3, int y3_stride,
+                                   int n, int c, int h, int w);
 int exhip_pool2d_nhwc_f16(exhip_ctx* ctx, const uint16_t* x, uint16_t* y, int n, int c, int h, int w, int c_stride,
                           int oh, int ow, int type, int kh, int kw, int sh, int sw, int pt, int pb, int pl, int pr,
                           int count_include_pad);

@@ -1,4 +1,5 @@
-"""The fp16 pooling pyramid and the Concat behind it as one launch: the values of the layers run one after the other."""
+"""The fp16 pooling pyramid and the Concat behind it as one launch, and the float32 one: the values of the layers run one after the other."""
+import ctypes
 import os
 import tempfile
 
@@ -46,6 +47,39 @@ def test_the_launch_equals_its_layers(ctx, n, c, h, w, values):
     layers = [x] + [ctx.maxpool_same_nhwc_f16(xd, k).download().reshape(x.shape).view(np.float16) for k in (5, 9, 13)]
     for level, want in enumerate(layers):
         assert np.array_equal(got[..., level * c:(level + 1) * c].view(np.float16), want, equal_nan=True), level
+
+
+@pytest.mark.parametrize("n,c,h,w,levels", [(1, 8, 1, 1, 3), (2, 24, 3, 5, 2), (1, 4, 1, 40, 3), (5, 16, 13, 7, 3), (1, 8, 45, 45, 2), (17, 256, 20, 20, 3), (2, 2048, 32, 32, 3), (4, 256, 20, 20, 3), (3, 352, 24, 24, 3)])
+@pytest.mark.parametrize("values", ["finite", "any"])
+def test_the_float32_launch_equals_its_layers(ctx, n, c, h, w, levels, values):
+    r = np.random.default_rng(h * w + c)
+    x = r.normal(0, 2, (n, h, w, c)).astype(np.float32)
+    if values == "any":
+        at = r.random(x.shape)
+        x[at < .2], x[at > .7] = -np.inf, np.nan
+        x[(at > .2) & (at < .25)] = np.inf
+        x[(at > .25) & (at < .5)] = r.choice([-0., 0.], np.count_nonzero((at > .25) & (at < .5)))
+    # the input with wider pixels than its own channels, the results side by side
+    xd, y = ctx.array(np.pad(x, ((0, 0),) * 3 + ((0, 8),))), ctx.array(np.full(n * h * w * 3 * c + 512, -77, np.float32))
+    at = lambda level: ctypes.c_void_p(y.ptr.value + level * c * 4)
+    hip._check(hip.lib().exhip_maxpool_pyramid_nhwc_f32(ctx.h, xd.ptr, c + 8, at(0), 3 * c, at(1), 3 * c, at(2) if levels == 3 else None, 3 * c, n, c, h, w))
+    ctx.sync()
+    got, src, stride = y.download(), xd, c + 8
+    assert (got[-512:] == -77).all()
+    got = got[:-512].reshape(n, h, w, 3 * c)
+    for level in range(levels):
+        want = ctx.array(np.zeros(x.shape, np.float32))
+        hip._check(hip.lib().exhip_pool2d_nhwc_f32(ctx.h, src.ptr, stride, want.ptr, c, n, c, h, w, h, w, 0, 5, 5, 1, 1, 2, 2, 2, 2, 0))
+        ctx.sync()
+        src, stride = want, c
+        assert got[..., level * c:(level + 1) * c].tobytes() == want.download().reshape(x.shape).tobytes(), level
+    assert levels == 3 or (got[..., 2 * c:] == -77).all()
+
+
+def test_what_the_float32_launch_leaves_to_the_layers(ctx):
+    x = ctx.array(np.zeros(43 * 48 * 8, np.float32))
+    assert hip.lib().exhip_maxpool_pyramid_nhwc_f32(ctx.h, x.ptr, 8, x.ptr, 8, x.ptr, 8, None, 0, 1, 8, 43, 48) == 10002
+    assert hip.lib().exhip_maxpool_pyramid_nhwc_f32(ctx.h, x.ptr, 8, x.ptr, 8, x.ptr, 8, None, 0, 1, 6, 4, 4) == 10002
 
 
 def test_what_it_leaves_to_the_layers(ctx):
