@@ -582,6 +582,11 @@ Plan plan_of(int dt, const PwParams& p, long long images, int subs, int kblocks)
 //    float32 results 1.02 to 1.6, with them from 80 K of work on (1.03 to 1.4, below 0.96 to 1.0). A shortcut with ReLU: 1.0 to 1.3 up to 128 K of work,
 //    beyond only what the lean kernel cannot take (64 -> 64 0.8, 192 -> 64 at 7 x 92 x 92 0.85). A ReLU alone, which the lean kernel has forms for: from 72 k-steps on
 //    1.06 to 1.19 up to 128 K, 0.74 to 0.98 beyond and below; ragged channels, which it cannot take, 0.98 to 1.17.
+//    Below 126 k-steps the split form, whose waves share a tile's steps, as long as its groups of two blocks are one round of 512 (384 -> 368 at 4 x 26 x 26
+//    10.6 there and 12.3 here, 192 -> 352 at 12 x 14 x 14 6.5 and 7.4, 320 -> 128 at 3 x 41 x 41 8.8 and 9.2; even at 72 k-steps; from 126 on 1.03 to 1.2 here,
+//    512 -> 64 at 12 x 30 x 30 12.0 and 10.1), 54 and 90 k-steps, which its waves divide better, to 704 (320 -> 128 at 1 x 93 x 93 11.2
+//    and 11.8, 192 -> 128 at 50 x 14 x 14 8.0 and 8.5). 18 and 36 k-steps from 46 K of work on
+//    (64 -> 352 at 35 x 14 x 14, 42 K, 0.96).
 //    Channels in odd thirty-twos, of which half a piece of products is for nothing and which the lean kernel has no form for: from 160 on 1.1 to 2.0
 //    (160 -> 96 at 2 x 80 x 80 with HardSwish 16.5 -> 8.9, with a ReLU 12.3 -> 9.1; 760 blocks 0.94, 784 1.12), 96 where the launch is large (96 -> 160 at
 //    8 x 66 x 66 18.0 -> 14.1, with a ReLU 0.95; 1800 blocks 0.9), 32 never (0.7 to 0.9).
@@ -596,8 +601,9 @@ bool exhip_staged_wins(int dt, const exhip_pw_geom& g, int stride, int n_ksteps,
     const long long blocks = (g.pixels + 31) / 32 * kblocks, work = blocks * ks;
     if (blocks <= (dt == EXHIP_F16 && ks < 72 ? 1024 : kStagedBlocks)) return false;
     if (dt == EXHIP_F16) return stride == 1 || (ks >= 72 ? blocks > 1280 : (kblocks <= 3 && blocks >= 1536) || blocks >= 12288);
-    if (stride == 2 || work < 41 * 1024) return false;
+    if (stride == 2 || work < (ks <= 36 ? 46 : 41) * 1024) return false;
     if (g.c_bytes % 64 != 0) return ks >= 45 ? blocks > 768 : ks >= 27 && blocks > 4096 && (g.post_op || shortcut || y_f || !(g.act || g.post_relu));
+    if (ks < 126 && (g.pixels + 31) / 32 * ((kblocks + 1) / 2) <= (ks == 54 || ks == 90 ? 704 : 512)) return false;
     const bool mid = work <= 128 * 1024 || g.k % 64 != 0;
     if (g.post_op) return ks >= 36 || (!shortcut && !y_f) || work >= 80 * 1024;
     if (shortcut) return ks >= 36 && mid;
