@@ -571,6 +571,8 @@ Plan plan_of(int dt, const PwParams& p, long long images, int subs, int kblocks)
 // channels times k-steps.
 //  * Few blocks: the split form (conv_pw.hip), whose tiles of 32 pixels share a CU by twos and fours (fp16 72 k-steps 502 blocks 0.78, 588 1.06; 36 k-steps 926
 //    blocks 0.85, 1263 1.22).
+//  * 54 and 90 k-steps at stride 1 to 704 of the split form's groups of two blocks, in either type: its waves divide them better (fp16 160 -> 320 at 10 x 13 x 13 8.0 there and 9.1
+//    here, 96 -> 128 at 50 x 14 x 14 8.9 and 9.3, 96 -> 96 at 18 x 25 x 25, 704 groups, equal; int8 320 -> 128 at 1 x 93 x 93 11.2 and 11.8, 192 -> 128 at 50 x 14 x 14 8.0 and 8.5).
 //  * fp16 at stride 1: everything else that the lean kernel cannot take, 1.04 to 1.6; what it can where its rounds of 256 patches of 256 pixels x 64 channels
 //    take longer: 128 -> 128 at 8 x 40 x 40 13.6 -> 10.4 us, 256 -> 256 at 16 x 20 x 20 20.7 -> 14.8, 64 -> 128 at 11 x 151 x 151 77 -> 47;
 //    its full rounds are 1 to 8 % shorter (64 -> 64 at 64 x 56 x 56, 128 -> 128 at 8 x 80 x 80).
@@ -584,9 +586,7 @@ Plan plan_of(int dt, const PwParams& p, long long images, int subs, int kblocks)
 //    1.06 to 1.19 up to 128 K, 0.74 to 0.98 beyond and below; ragged channels, which it cannot take, 0.98 to 1.17.
 //    Below 126 k-steps the split form, whose waves share a tile's steps, as long as its groups of two blocks are one round of 512 (384 -> 368 at 4 x 26 x 26
 //    10.6 there and 12.3 here, 192 -> 352 at 12 x 14 x 14 6.5 and 7.4, 320 -> 128 at 3 x 41 x 41 8.8 and 9.2; even at 72 k-steps; from 126 on 1.03 to 1.2 here,
-//    512 -> 64 at 12 x 30 x 30 12.0 and 10.1), 54 and 90 k-steps, which its waves divide better, to 704 (320 -> 128 at 1 x 93 x 93 11.2
-//    and 11.8, 192 -> 128 at 50 x 14 x 14 8.0 and 8.5). 18 and 36 k-steps from 46 K of work on
-//    (64 -> 352 at 35 x 14 x 14, 42 K, 0.96).
+//    512 -> 64 at 12 x 30 x 30 12.0 and 10.1), 18 and 36 k-steps from 46 K of work on (64 -> 352 at 35 x 14 x 14, 42 K, 0.96).
 //    Channels in odd thirty-twos, of which half a piece of products is for nothing and which the lean kernel has no form for: from 160 on 1.1 to 2.0
 //    (160 -> 96 at 2 x 80 x 80 with HardSwish 16.5 -> 8.9, with a ReLU 12.3 -> 9.1; 760 blocks 0.94, 784 1.12), 96 where the launch is large (96 -> 160 at
 //    8 x 66 x 66 18.0 -> 14.1, with a ReLU 0.95; 1800 blocks 0.9), 32 never (0.7 to 0.9).
@@ -600,10 +600,13 @@ bool exhip_staged_wins(int dt, const exhip_pw_geom& g, int stride, int n_ksteps,
     const int kblocks = std::min(g.slabs * g.slab_blocks, (std::max(g.k, g.k_stride) + 31) / 32), ks = n_ksteps;
     const long long blocks = (g.pixels + 31) / 32 * kblocks, work = blocks * ks;
     if (blocks <= (dt == EXHIP_F16 && ks < 72 ? 1024 : kStagedBlocks)) return false;
+    const bool odd = ks == 54 || ks == 90;  // k-steps that the split form's waves divide better
+    const long long pairs = (g.pixels + 31) / 32 * ((kblocks + 1) / 2);
+    if (odd && stride == 1 && g.c_bytes % 64 == 0 && pairs <= 704) return false;
     if (dt == EXHIP_F16) return stride == 1 || (ks >= 72 ? blocks > 1280 : (kblocks <= 3 && blocks >= 1536) || blocks >= 12288);
     if (stride == 2 || work < (ks <= 36 ? 46 : 41) * 1024) return false;
     if (g.c_bytes % 64 != 0) return ks >= 45 ? blocks > 768 : ks >= 27 && blocks > 4096 && (g.post_op || shortcut || y_f || !(g.act || g.post_relu));
-    if (ks < 126 && (g.pixels + 31) / 32 * ((kblocks + 1) / 2) <= (ks == 54 || ks == 90 ? 704 : 512)) return false;
+    if (ks < 126 && pairs <= 512) return false;
     const bool mid = work <= 128 * 1024 || g.k % 64 != 0;
     if (g.post_op) return ks >= 36 || (!shortcut && !y_f) || work >= 80 * 1024;
     if (shortcut) return ks >= 36 && mid;
