@@ -648,7 +648,8 @@ bool exhip_conv_f32_thirds(const exhip_conv_desc* d) {
 size_t exhip_conv_f32_thirds_bytes(const exhip_conv_desc* d) { return (size_t)((d->k + 31) / 32) * (d->c / 16) * kStepBytes; }
 
 // [32-channel block][16 channels][tap][third][lane][8 bfloat16]: lane rr of either half has the output channel that conv_f32.hip's packing gives
-// it, and eight neighbouring input channels. Large layers are dealt out to a few threads: 512 -> 512 takes one of them 2.4 ms, four 1.1 (whole floats, one: 1.5).
+// it, and eight neighbouring input channels. Layers are dealt out to
+// a few threads, one for each 8192 pairs of channels: 512 -> 512 takes one of them 2.4 ms, eight 0.8 (whole floats, one: 1.4), 256 -> 256 0.6 and 0.27 (0.31).
 void exhip_conv_f32_thirds_pack(const exhip_conv_desc* d, const float* w, void* out) {
     const int C = d->c, K = d->k, steps = C / 16, blocks = (K + 31) / 32;
     auto step = pack_step_any;
@@ -660,7 +661,7 @@ void exhip_conv_f32_thirds_pack(const exhip_conv_desc* d, const float* w, void* 
             for (int j = 0; j < steps; ++j) step(w, C, K, kb, j, static_cast<char*>(out) + (size_t)(kb * steps + j) * kStepBytes);
     };
     const unsigned cores = std::thread::hardware_concurrency();
-    const int most = (int)std::min<unsigned>(8, std::max(1u, cores / 2)), threads = std::min({most, blocks, (int)((long long)C * K / 65536) + 1});
+    const int most = (int)std::min<unsigned>(8, std::max(1u, cores / 2)), threads = std::min({most, blocks, (int)((long long)C * K / 8192) + 1});
     std::thread crew[8];
     int started = 1;
     try {
