@@ -2369,6 +2369,7 @@ bool pipeline<float>::impl::build_float_plan(const tensor_ptr& input, const std:
         value_info x, y[3];
         int levels = 0;
         size_t launch = 0;
+        int value = -1;  // the last level's. (Its address is that of a Concat as well that it is the first part of.)
     } pyramid;
     struct placed_layer {  // a convolution's launch, and the value it writes or, of a Concat's part, the Concat
         exhip_conv_desc d;
@@ -2642,6 +2643,7 @@ bool pipeline<float>::impl::build_float_plan(const tensor_ptr& input, const std:
             // A pyramid of stride-1 "same" max pools over one tensor: the maximum over a window of k is the maximum over a window
             // of k - k' + 1 of the maxima over windows of k' (taps outside the image count in neither)
             value_info src = in;
+            int from = nd.in[0];
             auto same_window = [&](const operation_pooling<float>* q) {
                 const int k = q->kernel_size_w_;
                 const bool same = q->type_ == 0 && !q->global_pooling_ && k == q->kernel_size_h_ && (k & 1) && q->stride_w_ == 1 && q->stride_h_ == 1 &&
@@ -2658,6 +2660,7 @@ bool pipeline<float>::impl::build_float_plan(const tensor_ptr& input, const std:
                     if (kq > best && kq < k && qv.p && qv.h == in.h && qv.w == in.w) {
                         best = kq;
                         src = qv;
+                        from = q.out;
                         kh = kw = k - kq + 1;
                         pt = pb = pl = pr = (k - kq + 1) / 2;
                     }
@@ -2669,10 +2672,11 @@ bool pipeline<float>::impl::build_float_plan(const tensor_ptr& input, const std:
             EXHIP_FATAL(rc);
             // 5 x 5 "same" maxima of the launch in front, which is such a level itself, join it: the map stays in LDS for all levels
             const bool five = type == 0 && kh == 5 && kw == 5 && sh == 1 && sw == 1 && pt == 2 && pb == 2 && pl == 2 && pr == 2;
-            const bool joins = five && pyramid.levels > 0 && pyramid.levels < 3 && pyramid.launch + 1 == plan->launches.size() && src.p == pyramid.y[pyramid.levels - 1].p;
+            const bool joins = five && pyramid.levels > 0 && pyramid.levels < 3 && pyramid.launch + 1 == plan->launches.size() && from == pyramid.value;
             if (joins) {
                 auto py = pyramid;
                 py.y[py.levels++] = o;
+                py.value = nd.out;
                 auto run = [=]() {
                     return exhip_maxpool_pyramid_nhwc_f32(ctx, py.x.p, py.x.cs, py.y[0].p, py.y[0].cs, py.y[1].p, py.y[1].cs, py.levels == 3 ? py.y[2].p : nullptr, py.y[2].cs,
                                                           in.n, ch, in.h, in.w);
@@ -2688,7 +2692,7 @@ bool pipeline<float>::impl::build_float_plan(const tensor_ptr& input, const std:
             }
             pyramid.levels = 0;
             if (five) {
-                pyramid.x = src; pyramid.y[0] = o; pyramid.levels = 1; pyramid.launch = plan->launches.size();
+                pyramid.x = src; pyramid.y[0] = o; pyramid.levels = 1; pyramid.launch = plan->launches.size(); pyramid.value = nd.out;
             }
             plan->launches.push_back([=]() {
                 EXHIP_FATAL(exhip_pool2d_nhwc_f32(ctx, src.p, src.cs, o.p, o.cs, in.n, ch, in.h, in.w, oh, ow, type, kh, kw, sh, sw, pt, pb, pl, pr, include_pad));

@@ -248,3 +248,46 @@ def test_a_concats_inputs_keep_their_values_behind_its_batchnorm(tmp_path, reade
             assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), o
     planned.close()
     plain.close()
+
+
+@pytest.mark.parametrize("wider", [False, True])
+def test_a_pool_of_a_concat_is_no_level_over_the_pool_it_begins_with(tmp_path, wider):
+    """p = pool(a), q = Concat(p, b), r = pool(q): q lies where p does and has no launch of its own, but r has to pool all of q's channels. `wider`: a
+    itself is a slice of a tensor with room for that many channels behind it."""
+    r = np.random.default_rng(93)
+    lines, blobs = [], []
+
+    def conv(bottom, top, cin, k, kernel=1):
+        w = r.normal(0, np.sqrt(2.0 / (cin * kernel * kernel)), (k, cin, kernel, kernel)).astype(np.float32)
+        lines.append(mf.conv_line("Convolution", top + "_l", bottom, top, k, kernel, 1, kernel // 2, True, w.size, 1))
+        blobs.append(mf.conv_blob_f32(w, r.normal(0, 0.5, (k,)).astype(np.float32)))
+
+    conv("data", "c0", 3, 16, 3)
+    lines.append("Split sp0 1 2 c0 c00 c01")
+    conv("c00", "a", 16, 16)
+    conv("c01", "z", 16, 48)
+    lines.append("Split sp1 1 " + ("3 a a0 a1 a2" if wider else "2 a a0 a2"))
+    conv("a0", "b", 16, 16)
+    if wider:
+        lines.append("Concat wide_l 2 1 a1 z wide 0=-1")
+    lines.append(mf.pool_line("p_l", "a2", "p", 0, 5, 1, 2))
+    lines.append("Concat q_l 2 1 p b q 0=-1")
+    lines.append("Split sp2 1 2 q q0 q1")
+    lines.append(mf.pool_line("r_l", "q0", "r", 0, 5, 1, 2))
+    conv("r", "late", 32, 16)
+    conv("q1", "early", 32, 16)
+    conv("wide" if wider else "z", "rest", 64 if wider else 48, 16)
+    path = str(tmp_path / "net.racy")
+    mf.write_model(path, blobs)
+    planned, plain = (xp.Pipeline(mf.topology(lines, "pools"), path, 0, fusion=on) for on in (True, False))
+    for seed in (1, 2, 3):
+        x = np.random.default_rng(seed).normal(0, 1, (2, 3, 12, 20)).astype(np.float32)
+        planned.forward(x)
+        plain.forward(x)
+        assert not planned.stored("c0") and plain.stored("c0")
+        for o in ("late", "early", "rest"):
+            got, want = planned.get(o), plain.get(o)
+            assert np.ptp(want) > .5
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (seed, o)
+    planned.close()
+    plain.close()
