@@ -470,11 +470,12 @@ void choose_strips(const F32Params& p, long long images, int run, int most, Plan
     }
 }
 
-constexpr int kForms = 5;
+// The last form is for maps of one pixel, each of which stages nine of its own: 32 of them fit twice with two steps at a time (120 KiB), with the first form's four not.
+constexpr int kForms = 5, kSmallest = kForms;
 struct Shape {
     int mt, nt, wk, wp, cs, occ;  // conv3x3_thirds_kernel's template arguments
 };
-constexpr Shape kForm[kForms] = {{1, 1, 4, 1, 4, 3}, {1, 1, 8, 1, 8, 2}, {1, 1, 2, 2, 2, 3}, {1, 1, 1, 4, 1, 3}, {2, 1, 2, 2, 2, 2}};
+constexpr Shape kForm[kForms + 1] = {{1, 1, 4, 1, 4, 3}, {1, 1, 8, 1, 8, 2}, {1, 1, 2, 2, 2, 3}, {1, 1, 1, 4, 1, 3}, {2, 1, 2, 2, 2, 2}, {1, 1, 2, 1, 2, 3}};
 
 struct Sizes {
     int run, pitch, waves;
@@ -525,14 +526,14 @@ const Plan& plan_of(const F32Params& p, long long images, int kblocks, int tile)
     if (e.images != images || e.h != p.out_h || e.w != p.out_w || e.csteps != p.csteps || e.kblocks != kblocks || e.tile != tile) {
         e = Entry();
         e.h = p.out_h; e.w = p.out_w; e.csteps = p.csteps; e.kblocks = kblocks; e.tile = tile;
-        for (int form = tile > 0 ? std::min(tile, kForms) - 1 : choose_form(p, (long long)p.out_h * p.out_w * images, kblocks);; form = 0) {
+        const int chosen = tile > 0 ? std::min(tile, kForms + 1) - 1 : choose_form(p, (long long)p.out_h * p.out_w * images, kblocks);
+        for (int form : {chosen, 0, kSmallest}) {  // maps of a few pixels stage up to nine for each
             const Sizes s(kForm[form]);
             const int buffers = p.csteps > kForm[form].cs ? 2 : 1;
             e.plan = Plan();
             e.plan.form = form;
             choose_strips(p, images, s.run, s.most(buffers), &e.plan);
-            // maps of a few pixels stage up to nine for each; the first form has room for nine times its 32 pixels
-            if (form == 0 || s.lds(e.plan.staged, buffers) <= kLdsLimit) break;
+            if (s.lds(e.plan.staged, buffers) <= kLdsLimit) break;
         }
         e.images = images;
     }
@@ -687,6 +688,7 @@ int exhip_conv_f32_thirds_run(exhip_ctx* ctx, const F32Launch& launch) {
     case 1: return go<1, false>(ctx, q, plan, launch.images, launch.blocks);
     case 2: return go<2, false>(ctx, q, plan, launch.images, launch.blocks);
     case 3: return go<3, false>(ctx, q, plan, launch.images, launch.blocks);
-    default: return go<4, false>(ctx, q, plan, launch.images, launch.blocks);
+    case 4: return go<4, false>(ctx, q, plan, launch.images, launch.blocks);
+    default: return slow ? go<kSmallest, true>(ctx, q, plan, launch.images, launch.blocks) : go<kSmallest, false>(ctx, q, plan, launch.images, launch.blocks);
     }
 }

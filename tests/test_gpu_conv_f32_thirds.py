@@ -17,7 +17,7 @@ def ctx():
     c.close()
 
 
-@pytest.fixture(params=range(6))
+@pytest.fixture(params=range(7))
 def tile(request):
     hip.set_option("f32_tile", request.param)
     yield request.param
@@ -66,6 +66,9 @@ SHAPES = [
     (2, 9, 31, 48, 40, (0, 0, 0, 0)),      # no padding, strips of a ragged width
     (1, 40, 7, 144, 70, (2, 0, 1, 2)),     # uneven padding, a third chunk of one step
     (2, 17, 19, 272, 32, (1, 1, 1, 1)),
+    (18, 1, 1, 80, 33, (1, 1, 1, 1)),      # maps of a pixel and more channels than are staged at a time: two buffers
+    (70, 1, 1, 272, 40, (1, 1, 1, 1)),
+    (32, 3, 3, 96, 64, (0, 0, 0, 0)),
 ]
 
 
