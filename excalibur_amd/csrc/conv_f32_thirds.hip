@@ -178,10 +178,11 @@ __global__ __launch_bounds__(64 * WK * WP, OCC) void conv3x3_thirds_kernel(const
     v4f x[BATCH];
     const int my_piece = threadIdx.x % PIECES, my_pixel = threadIdx.x / PIECES;
     auto load_batch = [&](int first, int chunk) {
+        const int end = chunk * CS * 64 + my_piece * 16 < p.csteps * 64 ? staged : 0;  // (the last chunk may reach beyond the channels)
 #pragma unroll
         for (int i = 0; i < BATCH; ++i) {
             const int at = first + i * PASS + my_pixel;
-            x[i] = load4(xr, at < staged ? table[at] + my_piece * 16 : kOutOfRange, chunk * CS * 64);
+            x[i] = load4(xr, at < end ? table[at] + my_piece * 16 : kOutOfRange, chunk * CS * 64);
         }
     };
     char* const my_stage = stage + (my_piece / 4) * 96 + (my_piece % 4) * 8;
@@ -251,7 +252,7 @@ __global__ __launch_bounds__(64 * WK * WP, OCC) void conv3x3_thirds_kernel(const
         constexpr bool NEXT = decltype(next)::value;
 #pragma unroll 1
         for (int s = part; s < CS && (NEXT || step < p.csteps); s += WK, step += WK) {
-            const bool more = NEXT || step + WK < p.csteps;
+            const bool more = step + WK < p.csteps;  // (a next chunk need not have a step for every wave)
             const int first = s / WK * (BATCH * PASS);
             if constexpr (NEXT) load_batch(first, chunk + 1);
             v8bf b[3][NT][3];
