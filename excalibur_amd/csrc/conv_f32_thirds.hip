@@ -1,12 +1,14 @@
 // conv3x3_thirds_kernel: float32 convolution with 3x3 filters of whole 16-channel steps at stride 1 on the bfloat16 matrix units.
 //
 // float32 products run at a sixteenth of the bfloat16 rate (157 against 2500 TFLOP/s), and a float32 is exactly the sum of three bfloat16
-// values, its thirds: h = round(x), m = round(x - h), l = x - h - m. Six of the nine products of two numbers' thirds hold everything down
-// to 2^-24 of the result (h h; h m, m h; m m, h l, l h: the other three lie below half a float32 ulp of it), so that a step of 16 channels
-// costs six v_mfma_f32_32x32x16_bf16 (192 cycles) instead of eight v_mfma_f32_32x32x2_f32 (512). The unit adds 16 products at a
-// time and rounds once; it rounds small addends toward minus infinity, though, so h h has accumulators of its own, and the five
+// values, its thirds: h = round(x), m = round(x - h), l = x - h - m. Eight of the nine products of two numbers' thirds are taken (all but l l,
+// 2^-34 of the result), so that a step of 16 channels costs eight v_mfma_f32_32x32x16_bf16 (256 cycles) instead of eight
+// v_mfma_f32_32x32x2_f32 (512). m l and l m, 2^-25 each, are nothing to the sum of many products, whose rounding is larger; a sum of one would be off by up
+// to .95 ulp without them. The unit adds 16 products at a
+// time and rounds once; it rounds small addends toward minus infinity, though, so h h has accumulators of its own, and the seven
 // others, 2^-8 of it, theirs. Against sums in 64 bits the results are off by a third to a half of what the float32 products leave
-// (2-norm over K = 576 random values 1.4e-7 and 4.3e-7, over 4608 4.2e-7 and 12.2e-7, all positive 1.3e-7 and 3.7e-7).
+// (2-norm over K = 576 random values 1.4e-7 and 4.3e-7, over 4608 4.2e-7 and 12.2e-7, all positive 1.3e-7 and 3.7e-7), where only some of the weights are not
+// zero by as much for one product, .60 to .98 of it for four.
 //
 // The weights are packed as thirds. The pixels are split once, on their way into LDS: a group of four or eight waves stages the input
 // under a run of pixels, 16 * CS channels at a time, and takes the nine taps from there; a split in registers would cost every wave 44
@@ -16,9 +18,9 @@
 // waste no lanes, small maps of several images share groups, and what a run needs of the input are whole rows of a strip, one after
 // another, whatever the run begins with. WK waves share a run's steps, their sums meet in LDS in a fixed order.
 //
-// Bounded by the matrix unit on large maps (128 -> 128 at 16 x 80 x 80 158 us, 191 TFLOP/s of float32 work, conv_f32_kernel 226) and by a group's chain of
-// loads, split and products on small ones: us, conv_f32_kernel and this one, 64 -> 64 on one 56 x 56 map 6.6, 4.9, at 160 x 160 22.6, 15.4, 128 -> 128 at
-// 80 x 80 21.7, 14.6, 512 -> 512 at 20 x 20 23.4, 15.7; over 83 layers 1.49 times as fast on average, 0.97 to 1.9.
+// Bounded by the matrix unit on large maps (128 -> 128 at 16 x 80 x 80 183 us, 165 TFLOP/s of float32 work, conv_f32_kernel 223) and by a group's chain of
+// loads, split and products on small ones: us, conv_f32_kernel and this one, launches queued from Python, 64 -> 64 on one 56 x 56 map 6.7, 5.5, at 160 x 160 23.5, 18.6,
+// 128 -> 128 at 80 x 80 22.5, 17.7, 512 -> 512 at 20 x 20 24.8, 21.4; over 62 layers 1.08 times as fast on average (with six products 1.20).
 //
 // Infinities and NaN: a third of an infinity is NaN, as is one times the zero third of a finite weight. A result that is not finite is
 // therefore computed again with float32 products (exact_products), whose result it gets.
@@ -263,6 +265,8 @@ __global__ __launch_bounds__(64 * WK * WP, OCC) void conv3x3_thirds_kernel(const
                     for (int t = 0; t < 3; ++t) to[n][t] = *reinterpret_cast<const v8bf*>(b_at[n] + at + t * 32);
             };
             auto tap = [&](int u, const v8bf (&now)[NT][3], int w_next) {
+                product(u, now, 2, 1, low);
+                product(u, now, 1, 2, low);
                 product(u, now, 2, 0, low);
                 product(u, now, 0, 2, low);
                 product(u, now, 1, 1, low);
@@ -491,7 +495,7 @@ private:
 };
 
 // The form that a model of the launch says is shortest, in microseconds: 2.5 for the launch; per round of groups on 256 CUs 1.5 for a group's
-// start, 0.2 for every four channels of a pixel that a thread finishes and 0.09 for every chunk; the products at 0.021 each, all of a SIMD's or
+// start, 0.2 for every four channels of a pixel that a thread finishes and 0.09 for every chunk; the products at 0.019 each, all of a SIMD's or
 // a group's where it is alone; or the weights at 14.6 TB/s where that is longer. Its constants are fitted to 83 layers from 1 x 11 x 11 to 37
 // GFLOP in these forms (11 % off on average); its choice is 2 % slower than the fastest on average, and 1.49 times as fast as the float32
 // products (conv_f32_kernel), which no more than noise beats anywhere. Wave tiles of 64 x 64, 32 x 64 and eight waves to 64 x 32 or 64 x 64 are
@@ -504,7 +508,7 @@ int choose_form(const F32Params& p, long long pixels, int kblocks) {
         const int waves = f.wk * f.wp, blocks = f.mt * f.nt, steps = (p.csteps + f.wk - 1) / f.wk, units = std::max(1, blocks * 4 / f.wk);
         const int resident = std::max(1, f.occ * 4 / waves), slots = waves > 4 ? 240 : 256;  // (256 groups of eight waves took a second round)
         const long long items = (pixels + 32 * f.nt * f.wp - 1) / (32 * f.nt * f.wp) * ((kblocks + f.mt - 1) / f.mt), each = (items + slots - 1) / slots;
-        const double products = steps * 9 * blocks * 6 * 0.0212, rounds = (double)((each + resident - 1) / resident);
+        const double products = steps * 9 * blocks * 8 * 0.0191, rounds = (double)((each + resident - 1) / resident);
         const double time = rounds * (1.5 + 0.2 * units + 0.09 * ((p.csteps + f.cs - 1) / f.cs - 1)) + std::max(each * (waves / 4) * products, rounds * products);
         const double cost = std::max(time, (double)items * f.mt * p.csteps * kStepBytes / 14.6e6);
         if (i == 0 || cost < best_cost) {

@@ -101,6 +101,28 @@ def test_errors_are_no_larger_than_those_of_float32_products(ctx):
             assert np.linalg.norm(run(ctx, x, wt, (1, 1, 1, 1)) - want) <= np.linalg.norm(y.download().reshape(want.shape) - want)
 
 
+@pytest.mark.parametrize("products", [1, 2, 4])
+def test_errors_of_few_products_are_no_larger_than_those_of_float32_products(ctx, tile, products):
+    """Pruned filters: `products` weights of each output channel are not zero. One product is rounded once by either, except that a sum of thirds that lies
+    within 2^-8 of the middle between two floats may be rounded the other way, by 2^-9 more: less than 1e-3 of the 2-norm. (16 channels: one wave has all of a tile's
+    products, so that none of the difference is that of sums in parts.)"""
+    r = np.random.default_rng(products)
+    mine = theirs = 0
+    for _ in range(3):
+        x, wt = r.standard_normal((1, 12, 20, 16)).astype(np.float32), np.zeros((64, 144), np.float32)
+        for row in wt:
+            row[r.permutation(144)[:products]] = r.standard_normal(products)
+        wt = wt.reshape(64, 16, 3, 3)
+        want, _ = conv64(x, wt, (1, 1, 1, 1))
+        d = ctx.conv_desc(1, 16, 12, 20, 64, (3, 4), 1, (1, 1, 1, 2), 0, 16, 64)
+        y = ctx.empty((1, 12, 20, 64), np.float32)
+        ctx.conv2d_f32(d, ctx.array(x), ctx.pack_conv_weights(d, hip.F32, np.pad(wt, ((0, 0), (0, 0), (0, 0), (0, 1)))), None, None, y)
+        ctx.sync()
+        mine += np.sum((run(ctx, x, wt, (1, 1, 1, 1)) - want) ** 2)
+        theirs += np.sum((y.download().reshape(want.shape) - want) ** 2)
+    assert np.sqrt(mine) <= 1.001 * np.sqrt(theirs)
+
+
 def test_infinities_nan_and_the_largest_floats(ctx, tile):
     r = np.random.default_rng(3)
     x, wt = r.standard_normal((2, 9, 11, 32)).astype(np.float32), (r.integers(1, 9, (40, 32, 3, 3)) / 8).astype(np.float32)
