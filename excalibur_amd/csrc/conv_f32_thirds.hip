@@ -452,11 +452,12 @@ struct Plan {
 
 // The strips for runs of `run` pixels: of all widths that split the map evenly the one whose groups, weighed with what they stage, are least,
 // among those of at most `most` staged pixels where there are any.
-void choose_strips(const F32Params& p, long long images, int run, int most, Plan* plan) {
+// `wide`: strips of a column that does not exist beside the map's only one.
+void choose_strips(const F32Params& p, long long images, int run, int most, bool wide, Plan* plan) {
     double best_cost = 0;
-    for (int width = p.out_w;;) {
+    for (int width = wide ? 2 : p.out_w;;) {
         const int count = (p.out_w + width - 1) / width;
-        width = (p.out_w + count - 1) / count;  // the narrowest of that many
+        if (!wide) width = (p.out_w + count - 1) / count;  // the narrowest of that many
         const long long tiles = ((long long)count * width * p.out_h * images + run - 1) / run;
         // rows that a run touches beside its first, maps that it enters beside its first, and their rows and columns with the border
         const int rows = run % width == 0 ? run / width - 1 : (run + width - 2) / width;
@@ -470,17 +471,16 @@ void choose_strips(const F32Params& p, long long images, int run, int most, Plan
             plan->tiles = tiles;
             best_cost = cost;
         }
-        if (width <= 4 && (width == 1 || plan->staged <= most)) break;
+        if (wide || (width <= 4 && (width == 1 || plan->staged <= most))) break;
         --width;
     }
 }
 
-// The last form is for maps of one pixel, each of which stages nine of its own: 32 of them fit twice with two steps at a time (120 KiB), with the first form's four not.
-constexpr int kForms = 5, kSmallest = kForms;
+constexpr int kForms = 5;
 struct Shape {
     int mt, nt, wk, wp, cs, occ;  // conv3x3_thirds_kernel's template arguments
 };
-constexpr Shape kForm[kForms + 1] = {{1, 1, 4, 1, 4, 3}, {1, 1, 8, 1, 8, 2}, {1, 1, 2, 2, 2, 3}, {1, 1, 1, 4, 1, 3}, {2, 1, 2, 2, 2, 2}, {1, 1, 2, 1, 2, 3}};
+constexpr Shape kForm[kForms] = {{1, 1, 4, 1, 4, 3}, {1, 1, 8, 1, 8, 2}, {1, 1, 2, 2, 2, 3}, {1, 1, 1, 4, 1, 3}, {2, 1, 2, 2, 2, 2}};
 
 struct Sizes {
     int run, pitch, waves;
@@ -531,13 +531,15 @@ const Plan& plan_of(const F32Params& p, long long images, int kblocks, int tile)
     if (e.images != images || e.h != p.out_h || e.w != p.out_w || e.csteps != p.csteps || e.kblocks != kblocks || e.tile != tile) {
         e = Entry();
         e.h = p.out_h; e.w = p.out_w; e.csteps = p.csteps; e.kblocks = kblocks; e.tile = tile;
-        const int chosen = tile > 0 ? std::min(tile, kForms + 1) - 1 : choose_form(p, (long long)p.out_h * p.out_w * images, kblocks);
-        for (int form : {chosen, 0, kSmallest}) {  // maps of a few pixels stage up to nine for each
+        const int chosen = tile > 0 ? std::min(tile, kForms) - 1 : choose_form(p, (long long)p.out_h * p.out_w * images, kblocks);
+        // Maps of a few pixels stage up to nine for each. LDS holds nine times the first form's 32 pixels once, but not twice: of maps of one pixel every second
+        // lane has one then (16 images stage 192 pixels).
+        for (int tries = 0; tries < 3; ++tries) {
+            const int form = tries ? 0 : chosen, buffers = p.csteps > kForm[form].cs ? 2 : 1;
             const Sizes s(kForm[form]);
-            const int buffers = p.csteps > kForm[form].cs ? 2 : 1;
             e.plan = Plan();
             e.plan.form = form;
-            choose_strips(p, images, s.run, s.most(buffers), &e.plan);
+            choose_strips(p, images, s.run, s.most(buffers), tries == 2, &e.plan);
             if (s.lds(e.plan.staged, buffers) <= kLdsLimit) break;
         }
         e.images = images;
@@ -693,7 +695,6 @@ int exhip_conv_f32_thirds_run(exhip_ctx* ctx, const F32Launch& launch) {
     case 1: return go<1, false>(ctx, q, plan, launch.images, launch.blocks);
     case 2: return go<2, false>(ctx, q, plan, launch.images, launch.blocks);
     case 3: return go<3, false>(ctx, q, plan, launch.images, launch.blocks);
-    case 4: return go<4, false>(ctx, q, plan, launch.images, launch.blocks);
-    default: return slow ? go<kSmallest, true>(ctx, q, plan, launch.images, launch.blocks) : go<kSmallest, false>(ctx, q, plan, launch.images, launch.blocks);
+    default: return go<4, false>(ctx, q, plan, launch.images, launch.blocks);
     }
 }

@@ -17,7 +17,7 @@ def ctx():
     c.close()
 
 
-@pytest.fixture(params=range(7))
+@pytest.fixture(params=range(6))
 def tile(request):
     hip.set_option("f32_tile", request.param)
     yield request.param
