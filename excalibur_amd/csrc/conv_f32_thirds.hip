@@ -22,8 +22,10 @@
 // loads, split and products on small ones: us, conv_f32_kernel and this one, launches queued from Python, 64 -> 64 on one 56 x 56 map 6.7, 5.5, at 160 x 160 23.5, 18.6,
 // 128 -> 128 at 80 x 80 22.5, 17.7, 512 -> 512 at 20 x 20 24.8, 21.4; over 62 layers 1.08 times as fast on average (with six products 1.20).
 //
-// Infinities and NaN: a third of an infinity is NaN, as is one times the zero third of a finite weight. A result that is not finite is
-// therefore computed again with float32 products (exact_products), whose result it gets.
+// What thirds do not hold: a third of an infinity is NaN, as is one times the zero third of a finite weight; below 2^-103 a last third is no normal number, below
+// 2^-110 it is cut off, and products below 2^-112 lose their smaller parts. A group that stages a value or finds a sum of that kind computes its
+// tile again with float32 products (float32_sums), whose results it gets, all of them; a weight of that kind is packed as a NaN that calls for them (split_weights).
+// Such a group takes 2.5 to 4 times as long.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -56,6 +58,7 @@ struct ThirdsParams {
     int chunks;                    // 16 * CS channels each
     int table_b, buffer_b;         // bytes of the tables in front of the staged pixels, and of a buffer of those
     float floor, post_floor;       // `plain`: what the activation and the ReLU behind the shortcut cut off at, -inf: nothing
+    int in_place;                  // the results take the shortcut's place
     int plain;                     // results are rows that take 16-byte accesses, and nothing but ReLUs and a shortcut lie behind the products
 };
 
@@ -90,35 +93,233 @@ __device__ __forceinline__ Where where(const ThirdsParams& p, unsigned at) {
     return w;
 }
 
-// Four channels from ch0 on of one pixel with float32 products: for results whose thirds met an infinity or a NaN. Slow.
-__device__ __forceinline__ v4f exact_products(const F32Params& p, unsigned pix, int ch0) {
+constexpr unsigned kLeast = 0x0c000000;  // 2^-103: every third of a larger float32 is a normal number
+constexpr int kNoSum = 0x297;  // v_cmp_class: NaN, infinite or below 2^-126 (and not zero)
+__device__ __forceinline__ bool no_sum(float v) { return __builtin_amdgcn_classf(v * 0x1p-14f, kNoSum); }  // nor below 2^-112
+constexpr unsigned kWhole = 0x7fff;  // the first third of a weight that thirds do not hold; the others are the halves of its bits
+
+// A weight from its thirds, the even or the odd one of two words of pairs.
+__device__ __forceinline__ float whole_weight(unsigned h, unsigned m, unsigned l, bool odd) {
+    const unsigned top = odd ? h & 0xffff0000u : h << 16, mid = odd ? m & 0xffff0000u : m << 16, low = odd ? l & 0xffff0000u : l << 16;
+    const float sum = __uint_as_float(top) + (__uint_as_float(mid) + __uint_as_float(low));
+    return top == kWhole << 16 ? __uint_as_float(mid | low >> 16) : sum;
+}
+
+// A wave's sums of the taps [first, last) of all 9 * csteps with float32 products, straight from memory: pix, the lane's pixels in the output. Steps of eight
+// v_mfma_f32_32x32x2_f32, the next two taps' operands on their way under a tap's products.
+template <int MT, int NT>
+__device__ __forceinline__ void float32_sums(const F32Params& p, __amdgpu_buffer_rsrc_t xr, __amdgpu_buffer_rsrc_t wr, int kb0, int first, int last, const unsigned (&pix)[NT], int lane,
+                                             v16f (&acc)[MT][NT]) {
+    constexpr int R = 2;
     const unsigned per_image = (unsigned)(p.out_h * p.out_w);
-    const bool in = pix < p.pixels;
-    const unsigned img = in ? exhip_divide(pix, per_image, p.image_magic, p.image_shift) : 0, rem = in ? pix - img * per_image : 0;
-    const int oy = (int)exhip_divide(rem, (unsigned)p.out_w, p.width_magic, p.width_shift), ox = (int)rem - oy * p.out_w;
-    v4f v = {0.f, 0.f, 0.f, 0.f};
-    const __bf16* const w = reinterpret_cast<const __bf16*>(p.wp);
-#pragma unroll 1
-    for (int tap = 0; tap < 9; ++tap) {
-        const int iy = oy - p.pad_t + tap / 3, ix = ox - p.pad_l + tap % 3;
-        const bool inside = in && (unsigned)iy < (unsigned)p.in_h && (unsigned)ix < (unsigned)p.in_w;
-        const float* const src = reinterpret_cast<const float*>(p.x) + (size_t)((img * (unsigned)p.in_h + iy) * (unsigned)p.in_w + ix) * (unsigned)(p.xs_b / 4);
-#pragma unroll 1
-        for (int c = 0; c < p.csteps * 16; ++c) {
-            const float xv = inside ? src[c] : 0.f;
+    unsigned corner[NT], inside[NT];  // the pixel's top-left input pixel (32-bit wrap-around where it lies in front of the tensor), and which of its taps lie in the image
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int ch = ch0 + e;
-                if (ch < p.K) {
-                    const int rr = (ch % 16 / 4) * 8 + (ch / 16 % 2) * 4 + ch % 4;
-                    const __bf16* const at = w + (size_t)(unsigned)(ch / 32 * p.csteps + c / 16) * (kStepBytes / 2) + tap * (kTapBytes / 2) +
-                                             ((c / 8 % 2) * 32 + rr) * 8 + c % 8;
-                    v[e] = __builtin_fmaf((float)at[0] + ((float)at[512] + (float)at[1024]), xv, v[e]);
+    for (int n = 0; n < NT; ++n) {
+        const bool in = pix[n] < p.pixels;
+        const unsigned img = exhip_divide(in ? pix[n] : 0, per_image, p.image_magic, p.image_shift), rem = in ? pix[n] - img * per_image : 0;
+        const int oy = (int)exhip_divide(rem, (unsigned)p.out_w, p.width_magic, p.width_shift), iy = oy - p.pad_t, ix = (int)rem - oy * p.out_w - p.pad_l;
+        corner[n] = (unsigned)((((int)img * p.in_h + iy) * p.in_w + ix) * p.xs_b + (lane >> 5) * 32);
+        inside[n] = 0;
+#pragma unroll
+        for (int tap = 0; tap < 9; ++tap)
+            inside[n] |= in && (unsigned)(iy + tap / 3) < (unsigned)p.in_h && (unsigned)(ix + tap % 3) < (unsigned)p.in_w ? 1u << tap : 0u;
+    }
+    unsigned woff[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) woff[m] = (kb0 + m) * 32 < p.K ? (unsigned)(m * p.csteps * kStepBytes + lane * 16) : kOutOfRange;
+    const int w_base = kb0 * p.csteps * kStepBytes;
+    v4u a[R][MT][3];
+    v4f b[R][NT][2];
+    auto request = [&](int u, int at) {  // always: behind a branch the products would wait for all that is on its way. Past the last tap zeros.
+        const bool on = at < last;
+        const int t = on ? at : last - 1, step = t / 9, tap = t - step * 9, off = tap / 3 * p.row_b + tap % 3 * p.xs_b;
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int i = 0; i < 3; ++i) a[u][m][i] = __builtin_bit_cast(v4u, load4(wr, on ? woff[m] : kOutOfRange, w_base + t * kTapBytes + i * 1024));
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            const unsigned from = on && (inside[n] >> tap & 1) ? corner[n] + (unsigned)off : kOutOfRange;
+            b[u][n][0] = load4(xr, from, step * 64);
+            b[u][n][1] = load4(xr, from + 16, step * 64);
+        }
+    };
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[m][n][e] = 0.f;
+    if (first >= last) return;
+#pragma unroll
+    for (int u = 0; u < R; ++u) request(u, first + u);
+#pragma unroll 1
+    for (int t = first; t < last; t += R) {
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+#pragma unroll
+                for (int m = 0; m < MT; ++m) {
+                    const float w = whole_weight(a[u][m][0][i / 2], a[u][m][1][i / 2], a[u][m][2][i / 2], i % 2 != 0);
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(w, b[u][n][i / 4][i % 4], acc[m][n], 0, 0, 0);
                 }
+            }
+            request(u, t + u + R);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+}
+
+// A channel's parameters, zeros for an absent array and beyond the channels.
+__device__ __forceinline__ void load_parameters(const F32Params& p, int ch, float (&par)[kParams]) {
+    const float* const from[kParams] = {p.bias, p.slope, p.bn_a, p.bn_b};
+#pragma unroll
+    for (int i = 0; i < kParams; ++i) {
+        par[i] = 0.f;
+        if (from[i]) {
+            const bool shared = i == 1 && p.slope_shared;
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(from[i]), 0, shared ? 4 : p.K * 4, kRsrcWord3);
+            par[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, shared ? 0 : ch * 4, 0, 0));
+        }
+    }
+}
+
+// How a tile is finished. The waves' sums meet where the pixels were staged, [part][block][four channels][pixel]; a thread finishes four channels of one pixel
+// at a time. Eight neighbouring lanes have a pixel's 32 channels, whose 128 bytes they store together, or for a planar result 32
+// neighbouring lanes the pixels of a channel. Pixels are dealt out by their channels' number, so that neither side meets bank conflicts.
+template <int MT, int NT, int WK>
+struct Tail {
+    static constexpr int BLOCKS = MT * NT, UNITS = BLOCKS * 4 >= WK ? BLOCKS * 4 / WK : 1;
+    static __device__ __forceinline__ bool owner(int part) { return BLOCKS * 4 >= WK || part < BLOCKS * 4; }
+    static __device__ __forceinline__ void place(bool planar, int part, int lane, int u, int& block, int& quad, int& row) {
+        const int at = (part * 64 + lane + u * WK * 64) % (BLOCKS * 256);
+        quad = planar ? at >> 5 & 7 : at & 7;
+        row = planar ? at & 31 : at >> 3 & 31;
+        block = at >> 8;
+    }
+};
+template <int MT, int NT, int WK>
+__device__ __forceinline__ void load_shortcut(const F32Params& p, const unsigned* pixels, int kb0, int part, int side, int lane, v4f (&res)[Tail<MT, NT, WK>::UNITS]) {
+    constexpr int UNITS = Tail<MT, NT, WK>::UNITS;
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) res[u] = v4f{0.f, 0.f, 0.f, 0.f};
+    if (p.residual) {
+#pragma unroll
+        for (int u = 0; u < UNITS; ++u) {
+            int block, quad, row;
+            Tail<MT, NT, WK>::place(p.y_nchw != nullptr, part, lane, u, block, quad, row);
+            const int ch = (kb0 + block % MT) * 32 + quad * 4;
+            unsigned from = pixels[(side * NT + block / MT) * 32 + row];
+            if (from >= p.pixels || ch >= p.K) continue;
+            if (p.res_shift) {
+                const unsigned per_image = (unsigned)(p.out_h * p.out_w), img = exhip_divide(from, per_image, p.image_magic, p.image_shift);
+                const unsigned in_image = from - img * per_image, oy = exhip_divide(in_image, (unsigned)p.out_w, p.width_magic, p.width_shift);
+                from = (img * ((unsigned)p.out_h >> p.res_shift) + (oy >> p.res_shift)) * ((unsigned)p.out_w >> p.res_shift) +
+                       ((in_image - oy * (unsigned)p.out_w) >> p.res_shift);
+            }
+            const float* const src = p.residual + (size_t)from * (unsigned)p.rstride + ch;
+            if (p.vector_rows) {
+                res[u] = *reinterpret_cast<const v4f*>(src);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) res[u][e] = ch + e < p.K ? src[e] : 0.f;
             }
         }
     }
-    return v;
+}
+template <int MT, int NT>
+__device__ __forceinline__ void put_sums(const v16f (&acc)[MT][NT], char* red, int part, int lane) {
+    constexpr int BLOCKS = MT * NT;
+#pragma unroll
+    for (int i = 0; i < 4 * BLOCKS; ++i) {
+        const v16f& c = acc[i / 4 % MT][i / 4 / MT];
+        const int quad = (lane >> 5) * 4 + i % 4;
+        *reinterpret_cast<v4f*>(red + part * BLOCKS * 4096 + (i / 4 * 8 + quad) * 512 + ((lane & 31) ^ quad) * 16) =
+            v4f{c[i % 4 * 4], c[i % 4 * 4 + 1], c[i % 4 * 4 + 2], c[i % 4 * 4 + 3]};
+    }
+}
+// (whether one of the sums is of a kind that thirds do not hold)
+template <int MT, int NT, int WK, bool SLOW>
+__device__ __forceinline__ bool finish_tile(const ThirdsParams& q, const unsigned* pixels, const float* params, const char* red, int kb0, int part, int side, int lane,
+                                            const v4f (&res)[Tail<MT, NT, WK>::UNITS]) {
+    const F32Params& p = q.f;
+    constexpr int BLOCKS = MT * NT, UNITS = Tail<MT, NT, WK>::UNITS;
+    bool missing = false;
+#pragma unroll 1
+    for (int u = 0; u < UNITS; ++u) {
+        struct {
+            unsigned pix;
+            int block, quad, row;
+            v4f res;
+        } now;
+        Tail<MT, NT, WK>::place(p.y_nchw != nullptr, part, lane, u, now.block, now.quad, now.row);
+        now.pix = pixels[(side * NT + now.block / MT) * 32 + now.row];
+        now.res = res[0];
+        if (p.residual) {
+#pragma unroll
+            for (int i = 1; i < UNITS; ++i) now.res = u == i ? res[i] : now.res;
+        }
+        const char* const from = red + (now.block * 8 + now.quad) * 512 + (now.row ^ now.quad) * 16;
+        const float* const my_params = params + now.block % MT * 32 + now.quad * 4;
+        const int ch = (kb0 + now.block % MT) * 32 + now.quad * 4;
+        v4f sum = *reinterpret_cast<const v4f*>(from);
+#pragma unroll
+        for (int w = 1; w < WK; ++w) sum += *reinterpret_cast<const v4f*>(from + w * BLOCKS * 4096);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) missing |= no_sum(sum[e]);
+        if (q.plain) {
+            const v4f bias = *reinterpret_cast<const v4f*>(my_params);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float v = sum[e] + bias[e];
+                v = q.floor > v ? q.floor : v;
+                if (p.residual) v += now.res[e];
+                v = q.post_floor > v ? q.post_floor : v;
+                sum[e] = ch + e < p.K ? v : 0.f;  // pad channels hold zeros
+            }
+            if (now.pix < p.pixels && ch < p.k_end) *reinterpret_cast<v4f*>(p.y + (size_t)now.pix * (unsigned)p.kstride + ch) = sum;
+        } else {
+            float v[4], par[kParams][4], res[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[e] = sum[e];
+                res[e] = now.res[e];
+#pragma unroll
+                for (int i = 0; i < kParams; ++i) par[i][e] = my_params[i * MT * 32 + e];
+            }
+            const unsigned per_image = (unsigned)(p.out_h * p.out_w);
+            unsigned img = 0, in_image = 0;
+            if (p.y_nchw || p.layout != EXHIP_PLACE_ROWS) {
+                img = exhip_divide(now.pix, per_image, p.image_magic, p.image_shift);
+                in_image = now.pix - img * per_image;
+            }
+            epilogue_part<4, SLOW>(p, v, par, res, now.pix, img, in_image, ch);
+        }
+    }
+    return missing;
+}
+
+// A tile's results with float32 products, for one that thirds did not do for. A call, so that none of it stands in the way of the others (inlined, scalar registers
+// spilled: .1 to .5 us of a small launch). args: where the kernel's arguments are (by reference the parameter would be copied to scratch first).
+template <int MT, int NT, int WK, bool SLOW>
+__device__ __noinline__ void again_with_floats(const ThirdsParams* args, const unsigned* pixels, const float* params, char* red, int kb0, int part, int side, int lane) {
+    const F32Params& p = args->f;
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.x), 0, (int)p.x_bytes, kRsrcWord3);
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.wp), 0, (int)p.w_bytes, kRsrcWord3);
+    unsigned pix[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) pix[n] = pixels[(side * NT + n) * 32 + (lane & 31)];
+    v16f acc[MT][NT];
+    float32_sums<MT, NT>(p, xr, wr, kb0, 9 * p.csteps * part / WK, 9 * p.csteps * (part + 1) / WK, pix, lane, acc);
+    v4f res[Tail<MT, NT, WK>::UNITS];
+    load_shortcut<MT, NT, WK>(p, pixels, kb0, part, side, lane, res);
+    put_sums<MT, NT>(acc, red, part, lane);
+#pragma unroll
+    for (int u = 0; u < Tail<MT, NT, WK>::UNITS; ++u) asm volatile("" : "+v"(res[u]));
+    __syncthreads();
+    if (Tail<MT, NT, WK>::owner(part)) finish_tile<MT, NT, WK, SLOW>(*args, pixels, params, red, kb0, part, side, lane, res);
 }
 
 // A wave's tile is 32 * MT channels x 32 * NT pixels; WP waves side by side make a group's run of pixels, WK share the steps of 16 channels,
@@ -136,7 +337,8 @@ __global__ __launch_bounds__(64 * WK * WP, OCC) void conv3x3_thirds_kernel(const
     extern __shared__ __attribute__((aligned(16))) char lds_all[];
     unsigned* const pixels = reinterpret_cast<unsigned*>(lds_all);   // the run's pixels in the output
     float* const params = reinterpret_cast<float*>(pixels + RUN);    // kParams of the tile's channels
-    unsigned* const table = pixels + RUN + kParams * MT * 32;        // where the staged pixels lie in the input
+    unsigned* const again = pixels + RUN + kParams * MT * 32;        // whether the tile is computed again
+    unsigned* const table = again + 4;                               // where the staged pixels lie in the input
     char* const stage = lds_all + q.table_b;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = lane >> 5;
     const int part = wave % WK, side = wave / WK;
@@ -169,6 +371,7 @@ __global__ __launch_bounds__(64 * WK * WP, OCC) void conv3x3_thirds_kernel(const
     const unsigned run0 = tile * RUN;
     const int first_row = __builtin_amdgcn_readfirstlane(where(q, run0).row), last_row = __builtin_amdgcn_readfirstlane(where(q, run0 + RUN - 1).row) + 2;
     const int staged = (last_row - first_row + 1) * q.staged_cols;
+    if (threadIdx.x == 0) *again = 0;
     for (int i = threadIdx.x; i < staged; i += THREADS) {
         const unsigned r = q.by_cols((unsigned)i), row = (unsigned)first_row + r, map = q.by_rows(row), img = q.by_strips(map);
         const int c = i - (int)r * q.staged_cols;
@@ -187,10 +390,13 @@ __global__ __launch_bounds__(64 * WK * WP, OCC) void conv3x3_thirds_kernel(const
             x[i] = load4(xr, at < end ? table[at] + my_piece * 16 : kOutOfRange, chunk * CS * 64);
         }
     };
+    unsigned least = ~0u;  // of twice the bits of what this thread stages, less one: zeros are the largest
     char* const my_stage = stage + (my_piece / 4) * 96 + (my_piece % 4) * 8;
     auto store_pass = [&](const v4f& from, int first, int buffer) {  // without a branch: what is no pixel goes behind the last one
         v2u h, m, l;
         split_thirds(from, h, m, l);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) least = min(least, (__float_as_uint(from[e]) << 1) - 1);
         const int at = first + my_pixel;
         char* const to = my_stage + buffer + (at < staged ? at : staged) * PITCH;
         *reinterpret_cast<v2u*>(to) = h;
@@ -200,18 +406,8 @@ __global__ __launch_bounds__(64 * WK * WP, OCC) void conv3x3_thirds_kernel(const
     load_batch(0, 0);
 #pragma unroll
     for (int u = 0; u < 3; ++u) request(u, w_at + u * kTapBytes);
-    float par[kParams] = {};
-    {
-        const unsigned ch = (unsigned)(kb0 * 32 + lane);
-        const float* const from[kParams] = {p.bias, p.slope, p.bn_a, p.bn_b};
-#pragma unroll
-        for (int i = 0; i < kParams; ++i)
-            if (from[i]) {
-                const bool shared = i == 1 && p.slope_shared;
-                const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(from[i]), 0, shared ? 4 : p.K * 4, kRsrcWord3);
-                par[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, shared ? 0 : (int)ch * 4, 0, 0));
-            }
-    }
+    float par[kParams];
+    load_parameters(p, kb0 * 32 + lane, par);
     // the wave's pixels: their place in the staged rows, and in the output
     const char* b_at[NT];
 #pragma unroll
@@ -329,114 +525,46 @@ __global__ __launch_bounds__(64 * WK * WP, OCC) void conv3x3_thirds_kernel(const
     }
     products(q.chunks - 1, std::false_type{});
 
-    // The waves' sums meet where the pixels were staged, [part][block][four channels][pixel]; a thread finishes four channels of one pixel
-    // at a time. Eight neighbouring lanes have a pixel's 32 channels, whose 128 bytes they store together, or for a planar result 32
-    // neighbouring lanes the pixels of a channel. Pixels are dealt out by their channels' number, so that neither side meets bank conflicts.
-    constexpr int UNITS = BLOCKS * 4 >= WK ? BLOCKS * 4 / WK : 1;
-    const bool owner = BLOCKS * 4 >= WK || part < BLOCKS * 4;
-    auto place = [&](int u, int& block, int& quad, int& row) {
-        const int at = (part * 64 + lane + u * WK * 64) % (BLOCKS * 256);
-        quad = p.y_nchw ? at >> 5 & 7 : at & 7;
-        row = p.y_nchw ? at & 31 : at >> 3 & 31;
-        block = at >> 8;
-    };
-    v4f res[UNITS];
-#pragma unroll
-    for (int u = 0; u < UNITS; ++u) res[u] = v4f{0.f, 0.f, 0.f, 0.f};
-    if (p.residual) {
-#pragma unroll
-        for (int u = 0; u < UNITS; ++u) {
-            int block, quad, row;
-            place(u, block, quad, row);
-            const int ch = (kb0 + block % MT) * 32 + quad * 4;
-            unsigned from = pixels[(side * NT + block / MT) * 32 + row];
-            if (from >= p.pixels || ch >= p.K) continue;
-            if (p.res_shift) {
-                const unsigned per_image = (unsigned)(p.out_h * p.out_w), img = exhip_divide(from, per_image, p.image_magic, p.image_shift);
-                const unsigned in_image = from - img * per_image, oy = exhip_divide(in_image, (unsigned)p.out_w, p.width_magic, p.width_shift);
-                from = (img * ((unsigned)p.out_h >> p.res_shift) + (oy >> p.res_shift)) * ((unsigned)p.out_w >> p.res_shift) +
-                       ((in_image - oy * (unsigned)p.out_w) >> p.res_shift);
-            }
-            const float* const src = p.residual + (size_t)from * (unsigned)p.rstride + ch;
-            if (p.vector_rows) {
-                res[u] = *reinterpret_cast<const v4f*>(src);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) res[u][e] = ch + e < p.K ? src[e] : 0.f;
-            }
-        }
-    }
+    v4f res[Tail<MT, NT, WK>::UNITS];
+    load_shortcut<MT, NT, WK>(p, pixels, kb0, part, side, lane, res);
     __syncthreads();  // the staged pixels are no longer read
     char* const red = stage + side * (WK * BLOCKS * 4096);
 #pragma unroll
-    for (int i = 0; i < 4 * BLOCKS; ++i) {
-        const v16f &c = acc[i / 4 % MT][i / 4 / MT], &d = low[i / 4 % MT][i / 4 / MT];
-        const int quad = half * 4 + i % 4;
-        v4f sum;
+    for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) sum[e] = c[i % 4 * 4 + e] + d[i % 4 * 4 + e];
-        *reinterpret_cast<v4f*>(red + part * BLOCKS * 4096 + (i / 4 * 8 + quad) * 512 + ((lane & 31) ^ quad) * 16) = sum;
-    }
-    // The loads are waited for here. In the loop below the wait would take its own stores along: one counter counts both, and a unit would
+        for (int n = 0; n < NT; ++n) acc[m][n] += low[m][n];
+    put_sums<MT, NT>(acc, red, part, lane);
+    // The loads are waited for here. In finish_tile's loop the wait would take its own stores along: one counter counts both, and a unit would
     // last 1000 cycles.
 #pragma unroll
-    for (int u = 0; u < UNITS; ++u) asm volatile("" : "+v"(res[u]));
+    for (int u = 0; u < Tail<MT, NT, WK>::UNITS; ++u) asm volatile("" : "+v"(res[u]));
     __syncthreads();
-    if (!owner) return;
-#pragma unroll 1
-    for (int u = 0; u < UNITS; ++u) {
-        struct {
-            unsigned pix;
-            int block, quad, row;
-            v4f res;
-        } now;
-        place(u, now.block, now.quad, now.row);
-        now.pix = pixels[(side * NT + now.block / MT) * 32 + now.row];
-        now.res = res[0];
-        if (p.residual) {
+    bool missing = least < (kLeast << 1) - 1;  // what thirds do not hold: what this thread staged, or a sum it finishes
+    auto any_missing = [&]() {
+        if (missing) *again = 1;
+        __syncthreads();
+        return *again != 0;
+    };
+    bool found = false;
+    if (q.in_place) {  // nothing may be stored before it is known, then: a second time reads the shortcut again
+        for (int i = threadIdx.x * 16; i < WAVES * BLOCKS * 4096; i += THREADS * 16) {
+            const v4f t = *reinterpret_cast<const v4f*>(stage + i);
 #pragma unroll
-            for (int i = 1; i < UNITS; ++i) now.res = u == i ? res[i] : now.res;
+            for (int e = 0; e < 4; ++e) missing |= no_sum(t[e]);
         }
-        const char* const from = red + (now.block * 8 + now.quad) * 512 + (now.row ^ now.quad) * 16;
-        const float* const my_params = params + now.block % MT * 32 + now.quad * 4;
-        const int ch = (kb0 + now.block % MT) * 32 + now.quad * 4;
-        v4f sum = *reinterpret_cast<const v4f*>(from);
-#pragma unroll
-        for (int w = 1; w < WK; ++w) sum += *reinterpret_cast<const v4f*>(from + w * BLOCKS * 4096);
-        const float t = __builtin_fmaf(sum[3], 0.f, __builtin_fmaf(sum[2], 0.f, __builtin_fmaf(sum[1], 0.f, sum[0] * 0.f)));
-        if (__builtin_expect(__any(!(t == 0.f)), 0)) {  // (0 unless a value is infinite or NaN)
-            const v4f exact = exact_products(p, now.pix, ch);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) sum[e] = sum[e] * 0.f == 0.f ? sum[e] : exact[e];
-        }
-        if (q.plain) {
-            const v4f bias = *reinterpret_cast<const v4f*>(my_params);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                float v = sum[e] + bias[e];
-                v = q.floor > v ? q.floor : v;
-                if (p.residual) v += now.res[e];
-                v = q.post_floor > v ? q.post_floor : v;
-                sum[e] = ch + e < p.K ? v : 0.f;  // pad channels hold zeros
-            }
-            if (now.pix < p.pixels && ch < p.k_end) *reinterpret_cast<v4f*>(p.y + (size_t)now.pix * (unsigned)p.kstride + ch) = sum;
-        } else {
-            float v[4], par[kParams][4], res[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                v[e] = sum[e];
-                res[e] = now.res[e];
-#pragma unroll
-                for (int i = 0; i < kParams; ++i) par[i][e] = my_params[i * MT * 32 + e];
-            }
-            const unsigned per_image = (unsigned)(p.out_h * p.out_w);
-            unsigned img = 0, in_image = 0;
-            if (p.y_nchw || p.layout != EXHIP_PLACE_ROWS) {
-                img = exhip_divide(now.pix, per_image, p.image_magic, p.image_shift);
-                in_image = now.pix - img * per_image;
-            }
-            epilogue_part<4, SLOW>(p, v, par, res, now.pix, img, in_image, ch);
-        }
+        found = any_missing();
+    }
+    if (!found) {
+        if (Tail<MT, NT, WK>::owner(part)) missing |= finish_tile<MT, NT, WK, SLOW>(q, pixels, params, red, kb0, part, side, lane, res);
+        if (!q.in_place) found = any_missing();
+    }
+    if (__builtin_expect(found, 0)) {
+#ifdef __HIP_DEVICE_COMPILE__
+        const auto* const args = (const ThirdsParams*)__builtin_amdgcn_kernarg_segment_ptr();
+#else
+        const auto* const args = &q;
+#endif
+        again_with_floats<MT, NT, WK, SLOW>(args, pixels, params, red, kb0, part, side, lane);
     }
 }
 
@@ -485,7 +613,7 @@ constexpr Shape kForm[kForms] = {{1, 1, 4, 1, 4, 3}, {1, 1, 8, 1, 8, 2}, {1, 1, 
 struct Sizes {
     int run, pitch, waves;
     explicit Sizes(const Shape& f) : run(32 * f.nt * f.wp), pitch(f.cs * 96 + 16), waves(f.wk * f.wp), f_(f) {}
-    int table_bytes(int staged) const { return ((run + kParams * f_.mt * 32 + staged) * 4 + 15) / 16 * 16; }
+    int table_bytes(int staged) const { return ((run + kParams * f_.mt * 32 + 4 + staged) * 4 + 15) / 16 * 16; }
     int lds(int staged, int buffers) const { return table_bytes(staged) + std::max((staged + 1) * pitch * buffers, waves * f_.mt * f_.nt * 4096); }
     // staged pixels with which as many groups share a CU as its registers allow
     int most(int buffers) const { return (kLdsLimit / std::max(f_.occ * 4 / waves, 1) - table_bytes(0) - 16 - pitch * buffers) / (pitch * buffers + 4); }
@@ -588,16 +716,19 @@ int go(exhip_ctx* ctx, ThirdsParams& q, const Plan& plan, long long images, int 
     return 0;
 }
 
-// The thirds of 72 weights, eight channels' nine taps: [third][tap][channel]. Whole vectors where all of them are finite and none rounds up to an infinity.
+// The thirds of 72 weights, eight channels' nine taps: [third][tap][channel]. Whole vectors where all of them are zeros or between 2^-103 and what rounds up to an infinity.
 __attribute__((always_inline)) inline bool split_finite(const float* src, uint16_t (*out)[72]) {
     float v[72];
     unsigned u[72];
     for (int i = 0; i < 8; ++i)
         for (int tap = 0; tap < 9; ++tap) v[tap * 8 + i] = src[i * 9 + tap];
     memcpy(u, v, sizeof(u));
-    unsigned high = 0;
-    for (int i = 0; i < 72; ++i) high |= (u[i] & 0x7fffffffu) + 0x808000u;  // the sign bit from 0x7f7f8000 on
-    if (high & 0x80000000u) return false;
+    unsigned high = 0, least = ~0u;
+    for (int i = 0; i < 72; ++i) {
+        high |= (u[i] & 0x7fffffffu) + 0x808000u;  // the sign bit from 0x7f7f8000 on
+        least = std::min(least, (u[i] << 1) - 1);
+    }
+    if (high & 0x80000000u || least < (kLeast << 1) - 1) return false;
     for (int t = 0; t < 3; ++t) {
         for (int i = 0; i < 72; ++i) {
             unsigned b;
@@ -616,6 +747,12 @@ void split_weights(const float* src, uint16_t (*out)[72]) {
     for (int tap = 0; tap < 9; ++tap)
         for (int c = 0; c < 8; ++c) {  // an infinity or NaN is its own first third; what would round up to an infinity is cut off
             float x = src[c * 9 + tap];
+            unsigned whole;
+            memcpy(&whole, &x, 4);
+            if (const unsigned size = whole & 0x7fffffffu; (size > 0 && size < kLeast) || size > 0x7f800000u) {
+                for (int t = 0; t < 3; ++t) out[t][tap * 8 + c] = (uint16_t)(t == 0 ? kWhole : t == 1 ? whole >> 16 : whole);
+                continue;
+            }
             for (int t = 0; t < 3; ++t) {
                 unsigned b;
                 memcpy(&b, &x, 4);
@@ -689,6 +826,8 @@ int exhip_conv_f32_thirds_run(exhip_ctx* ctx, const F32Launch& launch) {
     q.floor = p.act == 1 ? 0.f : -INFINITY;
     q.post_floor = p.post_relu ? 0.f : -INFINITY;
     const bool slow = p.act == 4 || p.act == 5;
+    const size_t res_pixels = (size_t)(p.pixels >> 2 * p.res_shift), y_pixels = (size_t)p.pixels * (p.layout == EXHIP_PLACE_SHUFFLED ? 4 : 1);
+    q.in_place = p.residual && p.y && p.residual < p.y + y_pixels * (unsigned)p.kstride && p.y < p.residual + res_pixels * (unsigned)p.rstride;
     const Plan plan = plan_of(p, launch.images, launch.blocks, slow ? 1 : g_exhip_options.f32_tile);
     switch (plan.form) {
     case 0: return slow ? go<0, true>(ctx, q, plan, launch.images, launch.blocks) : go<0, false>(ctx, q, plan, launch.images, launch.blocks);

@@ -136,6 +136,51 @@ def test_infinities_nan_and_the_largest_floats(ctx, tile):
     assert (np.abs(got[ok] - want[ok]) <= 288 * 2.0 ** -24 * scale[ok]).all()
 
 
+def tiny(r, shape, e):
+    return np.ldexp(r.choice([-1., 1.], shape) * r.uniform(1, 2, shape), e).astype(np.float32)
+
+
+@pytest.mark.parametrize("kind", ["pixels", "one pixel", "weights", "one weight", "products"])
+def test_values_that_thirds_do_not_hold(ctx, tile, kind):
+    """Operands below 2^-103, the smallest ones no normal numbers, and products of that size: float32 sums, as many as products, in any order."""
+    r = np.random.default_rng(11)
+    n, h, w, c, k = 2, 9, 11, 80, 40
+    x, wt = r.standard_normal((n, h, w, c)), r.standard_normal((k, c, 3, 3))
+    if kind == "pixels":
+        x, wt = tiny(r, x.shape, r.integers(-146, -100, x.shape)), np.ldexp(wt, 60)
+    elif kind == "one pixel":
+        x, wt = np.zeros_like(x), np.ldexp(wt, 60)
+        x[1, 4, 5, 33] = np.ldexp(1 + 2. ** -12 + 2. ** -23, -118)
+    elif kind == "weights":
+        x, wt = np.ldexp(x, 60), tiny(r, wt.shape, r.integers(-146, -100, wt.shape))
+    elif kind == "one weight":
+        x, wt = np.ldexp(x, 60), np.zeros_like(wt)
+        wt[7, 70, 1, 2] = np.ldexp(1 + 2. ** -12 + 2. ** -23, -118)
+    else:
+        x, wt = np.ldexp(x, -58), np.ldexp(wt, -62)
+    x, wt = x.astype(np.float32), wt.astype(np.float32)
+    want, scale = conv64(x, wt, (1, 1, 1, 1))
+    products = 1 if kind in ("one pixel", "one weight") else 9 * c
+    assert np.count_nonzero(want)
+    assert (np.abs(run(ctx, x, wt, (1, 1, 1, 1)) - want) <= products * (2. ** -24 * scale + 2. ** -150)).all()
+
+
+@pytest.mark.parametrize("tiny", [False, True])
+def test_results_in_the_place_of_the_shortcut(ctx, tile, tiny):
+    r = np.random.default_rng(13)
+    n, h, w, c, k = 2, 7, 12, 48, 64
+    x, wt = (r.standard_normal(s).astype(np.float32) for s in ((n, h, w, c), (k, c, 3, 3)))
+    res = r.standard_normal((n, h, w, k)).astype(np.float32)
+    if tiny:  # (a tile that is computed again)
+        x[:, 3, 4], wt[5, 6] = 2.0 ** -120, 2.0 ** -115
+    want, scale = conv64(x, wt, (1, 1, 1, 1))
+    d = ctx.conv_desc(n, c, h, w, k, 3, 1, (1, 1, 1, 1), 0, c, k)
+    y = ctx.array(res)
+    ctx.conv2d_f32(d, ctx.array(x), ctx.pack_conv_weights(d, hip.F32, wt), None, y, y, None)
+    ctx.sync()
+    assert (np.abs(y.download().reshape(want.shape) - (want + res)) <= (9 * c + 1) * 2.0 ** -24 * (scale + np.abs(res))).all()
+
+
 PLACES = [
     (plain.ROWS, 0, 2, 32, 6, 10, 44, 3, 1, True),
     (plain.GROUPED, 85, 3, 32, 5, 7, 255, 3, None, False),

@@ -30,6 +30,22 @@ def test_thirds_add_up_to_the_weight_and_lie_in_fragment_order(c, k):
                 assert (np.abs(m[ok]) <= np.abs(want[ok]) / 128).all() and (np.abs(l[ok]) <= np.abs(want[ok]) / 32768).all()
 
 
+def test_weights_that_thirds_do_not_hold_are_kept_whole():
+    r = np.random.default_rng(3)
+    w = r.standard_normal((32, 16, 3, 3)).astype(np.float32)
+    at = r.random(w.shape) < .1
+    w[at] = np.ldexp(r.uniform(-2, 2, at.sum()), r.integers(-150, -103, at.sum())).astype(np.float32)
+    w[1, 1, 1, 1] = np.uint32(0xffffffff).view(np.float32)
+    got = pack(hip.Ctx.conv_desc(1, 16, 20, 20, 32, 3, 1, 1, 0, 16, 32), hip.F32, w).view(np.uint16).reshape(9, 3, 64, 8)
+    for tap in range(9):
+        h, m, l = got[tap]
+        want = lanes(w[:, :, tap // 3, tap % 3]).view(np.uint32)
+        size = want & 0x7fffffff
+        whole = (size > 0) & (size < 0x0c000000) | (size > 0x7f800000)
+        assert whole.any() and np.array_equal(h == 0x7fff, whole)
+        assert np.array_equal(m[whole].astype(np.uint32) << 16 | l[whole], want[whole])
+
+
 @pytest.mark.parametrize("kernel,stride,c", [(3, 2, 64), (3, 1, 24), (1, 1, 64), ((1, 3), 1, 64)])
 def test_other_layers_keep_whole_floats(kernel, stride, c):
     kh, kw = (kernel, kernel) if np.isscalar(kernel) else kernel
