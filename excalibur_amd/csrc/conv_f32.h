@@ -16,4 +16,5 @@ struct F32Launch {
 bool exhip_conv_f32_thirds(const exhip_conv_desc* d);
 size_t exhip_conv_f32_thirds_bytes(const exhip_conv_desc* d);
 void exhip_conv_f32_thirds_pack(const exhip_conv_desc* d, const float* w_oihw, void* packed);
+int exhip_conv_f32_thirds_pack_device(exhip_ctx* ctx, const exhip_conv_desc* d, const float* w_oihw, void* packed);  // both on the device
 int exhip_conv_f32_thirds_run(exhip_ctx* ctx, const F32Launch& launch);

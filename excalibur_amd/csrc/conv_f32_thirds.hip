@@ -24,7 +24,7 @@
 //
 // What thirds do not hold: a third of an infinity is NaN, as is one times the zero third of a finite weight; below 2^-103 a last third is no normal number, below
 // 2^-110 it is cut off, and products below 2^-112 lose their smaller parts. A group that stages a value or finds a sum of that kind computes its
-// tile again with float32 products (float32_sums), whose results it gets, all of them; a weight of that kind is packed as a NaN that calls for them (split_weights).
+// tile again with float32 products (float32_sums), whose results it gets, all of them; a weight of that kind is packed as a NaN that calls for them (split_weight).
 // Such a group takes 2.5 to 4 times as long.
 #include <hip/hip_runtime.h>
 
@@ -33,7 +33,6 @@
 #include <cstdint>
 #include <cstring>
 #include <mutex>
-#include <thread>
 
 #include "conv_f32.h"
 #include "conv_f32_epilogue.h"
@@ -716,67 +715,86 @@ int go(exhip_ctx* ctx, ThirdsParams& q, const Plan& plan, long long images, int 
     return 0;
 }
 
-// The thirds of 72 weights, eight channels' nine taps: [third][tap][channel]. Whole vectors where all of them are zeros or between 2^-103 and what rounds up to an infinity.
-__attribute__((always_inline)) inline bool split_finite(const float* src, uint16_t (*out)[72]) {
-    float v[72];
-    unsigned u[72];
-    for (int i = 0; i < 8; ++i)
-        for (int tap = 0; tap < 9; ++tap) v[tap * 8 + i] = src[i * 9 + tap];
-    memcpy(u, v, sizeof(u));
-    unsigned high = 0, least = ~0u;
-    for (int i = 0; i < 72; ++i) {
-        high |= (u[i] & 0x7fffffffu) + 0x808000u;  // the sign bit from 0x7f7f8000 on
-        least = std::min(least, (u[i] << 1) - 1);
+// A weight's thirds. An infinity is its own first third; what would round up to an infinity is cut off; what thirds do not hold is kept whole.
+__host__ __device__ inline void split_weight(float x, uint16_t (&out)[3]) {
+    const unsigned whole = __builtin_bit_cast(unsigned, x), size = whole & 0x7fffffffu;
+    if ((size > 0 && size < kLeast) || size > 0x7f800000u) {
+        out[0] = kWhole;
+        out[1] = (uint16_t)(whole >> 16);
+        out[2] = (uint16_t)whole;
+        return;
     }
-    if (high & 0x80000000u || least < (kLeast << 1) - 1) return false;
     for (int t = 0; t < 3; ++t) {
-        for (int i = 0; i < 72; ++i) {
-            unsigned b;
-            float f;
-            memcpy(&b, v + i, 4);
+        const unsigned b = __builtin_bit_cast(unsigned, x), r = b + 0x7fffu + (b >> 16 & 1);
+        const bool finite = (b & 0x7f800000u) != 0x7f800000u;
+        const unsigned third = finite && (r & 0x7f800000u) != 0x7f800000u ? r >> 16 : b >> 16;
+        out[t] = (uint16_t)third;
+        x = finite ? x - __builtin_bit_cast(float, third << 16) : 0.f;
+    }
+}
+
+typedef unsigned v8w __attribute__((ext_vector_type(8)));
+typedef float v8f __attribute__((ext_vector_type(8)));
+typedef uint16_t v8s __attribute__((ext_vector_type(8)));
+
+// Eight channels' nine taps to where a lane has them, [tap][third] 1 KiB each: eight channels at a time where all weights are zeros or between 2^-103 and what rounds
+// up to an infinity.
+__attribute__((always_inline)) inline bool split_finite(const float* src, char* to) {
+    v8w w[9], t[8];  // [tap]: the rows of eight taps turned over, and the ninth
+    for (int i = 0; i < 8; ++i) {
+        memcpy(&w[i], src + i * 9, 32);
+        memcpy(reinterpret_cast<char*>(&w[8]) + i * 4, src + i * 9 + 8, 4);
+    }
+    for (int i = 0; i < 8; i += 2) {
+        t[i] = __builtin_shufflevector(w[i], w[i + 1], 0, 8, 2, 10, 4, 12, 6, 14);
+        t[i + 1] = __builtin_shufflevector(w[i], w[i + 1], 1, 9, 3, 11, 5, 13, 7, 15);
+    }
+    for (int i = 0; i < 8; i += i % 4 == 1 ? 3 : 1) {
+        w[i] = __builtin_shufflevector(t[i], t[i + 2], 0, 1, 8, 9, 4, 5, 12, 13);
+        w[i + 2] = __builtin_shufflevector(t[i], t[i + 2], 2, 3, 10, 11, 6, 7, 14, 15);
+    }
+    for (int i = 0; i < 4; ++i) {
+        t[i] = __builtin_shufflevector(w[i], w[i + 4], 0, 1, 2, 3, 8, 9, 10, 11);
+        t[i + 4] = __builtin_shufflevector(w[i], w[i + 4], 4, 5, 6, 7, 12, 13, 14, 15);
+    }
+    v8w high = 0, least = ~0u;
+    for (int tap = 0; tap < 9; ++tap) {
+        if (tap < 8) w[tap] = t[tap];
+        high |= (w[tap] & 0x7fffffffu) + 0x808000u;  // the sign bit from 0x7f7f8000 on
+        least = __builtin_elementwise_min(least, (w[tap] << 1) - 1);
+    }
+    for (int i = 0; i < 8; ++i)
+        if (high[i] & 0x80000000u || least[i] < (kLeast << 1) - 1) return false;
+    for (int tap = 0; tap < 9; ++tap) {
+        v8f x = __builtin_bit_cast(v8f, w[tap]);
+        for (int third = 0; third < 3; ++third) {
+            v8w b = __builtin_bit_cast(v8w, x);
             b = (b + 0x7fffu + (b >> 16 & 1)) & 0xffff0000u;  // to the nearest, ties to even
-            memcpy(&f, &b, 4);
-            out[t][i] = (uint16_t)(b >> 16);
-            v[i] -= f;
+            x -= __builtin_bit_cast(v8f, b);
+            const v8s out = __builtin_convertvector(b >> 16, v8s);
+            memcpy(to + (tap * 3 + third) * 1024, &out, 16);
         }
     }
     return true;
 }
 
-void split_weights(const float* src, uint16_t (*out)[72]) {
-    for (int tap = 0; tap < 9; ++tap)
-        for (int c = 0; c < 8; ++c) {  // an infinity or NaN is its own first third; what would round up to an infinity is cut off
-            float x = src[c * 9 + tap];
-            unsigned whole;
-            memcpy(&whole, &x, 4);
-            if (const unsigned size = whole & 0x7fffffffu; (size > 0 && size < kLeast) || size > 0x7f800000u) {
-                for (int t = 0; t < 3; ++t) out[t][tap * 8 + c] = (uint16_t)(t == 0 ? kWhole : t == 1 ? whole >> 16 : whole);
-                continue;
-            }
-            for (int t = 0; t < 3; ++t) {
-                unsigned b;
-                memcpy(&b, &x, 4);
-                const bool finite = (b & 0x7f800000u) != 0x7f800000u;
-                const unsigned r = b + 0x7fffu + (b >> 16 & 1);
-                const unsigned third = finite && (r & 0x7f800000u) != 0x7f800000u ? r >> 16 : b >> 16 | (!finite && (b & 0x7fffffu) ? 0x40u : 0u);
-                out[t][tap * 8 + c] = (uint16_t)third;
-                const unsigned back = third << 16;
-                float f;
-                memcpy(&f, &back, 4);
-                x = finite ? x - f : 0.f;
-            }
-        }
+// The output channel that lane rr of either half has in a block.
+__host__ __device__ inline int lane_channel(int kb, int lane) {
+    const int rr = lane % 32;
+    return kb * 32 + (rr / 4 % 2) * 16 + rr / 8 * 4 + rr % 4;
 }
 
 // One step's weights of a 32-channel block.
 __attribute__((always_inline)) inline void pack_step(const float* w, int C, int K, int kb, int j, char* to) {
     for (int lane = 0; lane < 64; ++lane) {
-        const int rr = lane % 32, k = kb * 32 + (rr / 4 % 2) * 16 + rr / 8 * 4 + rr % 4;
-        uint16_t thirds[3][72];
-        if (k >= K) memset(thirds, 0, sizeof(thirds));
-        else if (const float* const src = w + ((size_t)k * C + j * 16 + lane / 32 * 8) * 9; !split_finite(src, thirds)) split_weights(src, thirds);
-        for (int tap = 0; tap < 9; ++tap)
-            for (int t = 0; t < 3; ++t) memcpy(to + (tap * 3 + t) * 1024 + lane * 16, thirds[t] + tap * 8, 16);
+        const int k = lane_channel(kb, lane);
+        const float* const src = w + ((size_t)k * C + j * 16 + lane / 32 * 8) * 9;
+        if (k < K && split_finite(src, to + lane * 16)) continue;
+        for (int i = 0; i < 72; ++i) {
+            uint16_t thirds[3] = {};
+            if (k < K) split_weight(src[i], thirds);
+            for (int t = 0; t < 3; ++t) memcpy(to + (i % 9 * 3 + t) * 1024 + lane * 16 + i / 9 * 2, &thirds[t], 2);
+        }
     }
 }
 #ifndef __HIP_DEVICE_COMPILE__
@@ -793,29 +811,45 @@ bool exhip_conv_f32_thirds(const exhip_conv_desc* d) {
 size_t exhip_conv_f32_thirds_bytes(const exhip_conv_desc* d) { return (size_t)((d->k + 31) / 32) * (d->c / 16) * kStepBytes; }
 
 // [32-channel block][16 channels][tap][third][lane][8 bfloat16]: lane rr of either half has the output channel that conv_f32.hip's packing gives
-// it, and eight neighbouring input channels. Layers are dealt out to
-// a few threads, one for each 8192 pairs of channels: 512 -> 512 takes one of them 2.4 ms, eight 0.8 (whole floats, one: 1.4), 256 -> 256 0.6 and 0.27 (0.31).
+// it, and eight neighbouring input channels. .8 ns a weight (whole floats 1.0).
 void exhip_conv_f32_thirds_pack(const exhip_conv_desc* d, const float* w, void* out) {
     const int C = d->c, K = d->k, steps = C / 16, blocks = (K + 31) / 32;
     auto step = pack_step_any;
 #ifndef __HIP_DEVICE_COMPILE__
     if (__builtin_cpu_supports("avx2")) step = pack_step_avx2;
 #endif
-    auto pack = [=](int first, int last) {
-        for (int kb = first; kb < last; ++kb)
-            for (int j = 0; j < steps; ++j) step(w, C, K, kb, j, static_cast<char*>(out) + (size_t)(kb * steps + j) * kStepBytes);
-    };
-    const unsigned cores = std::thread::hardware_concurrency();
-    const int most = (int)std::min<unsigned>(8, std::max(1u, cores / 2)), threads = std::min({most, blocks, (int)((long long)C * K / 8192) + 1});
-    std::thread crew[8];
-    int started = 1;
-    try {
-        for (; started < threads; ++started) crew[started] = std::thread(pack, blocks * started / threads, blocks * (started + 1) / threads);
-    } catch (...) {  // the process may have no more threads: this one does the rest
+    for (int kb = 0; kb < blocks; ++kb)
+        for (int j = 0; j < steps; ++j) step(w, C, K, kb, j, static_cast<char*>(out) + (size_t)(kb * steps + j) * kStepBytes);
+}
+
+// The same on the device: a wave a step and block, a lane its eight channels' taps. A network's first call uploads two thirds of the bytes then, and the host, which takes .5
+// to 2 ms for a layer of 512 -> 512 whose weights no cache holds, has nothing to pack (first call of the text detector 9.2 -> 5.1 ms, of the float32 detector 9.7 -> 8.8).
+__global__ __launch_bounds__(64) void pack_thirds_kernel(const float* __restrict__ w, char* __restrict__ out, int C, int K, int steps) {
+    const int lane = threadIdx.x, kb = (int)blockIdx.x / steps, j = (int)blockIdx.x - kb * steps, k = lane_channel(kb, lane);
+    const float* const src = w + ((size_t)k * C + j * 16 + lane / 32 * 8) * 9;
+    char* const to = out + (size_t)blockIdx.x * kStepBytes + lane * 16;
+#pragma unroll
+    for (int tap = 0; tap < 9; ++tap) {
+        v4u words[3] = {};
+        if (k < K) {
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                uint16_t thirds[3];
+                split_weight(src[c * 9 + tap], thirds);
+#pragma unroll
+                for (int t = 0; t < 3; ++t) words[t][c / 2] |= (unsigned)thirds[t] << (c % 2 * 16);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 3; ++t) *reinterpret_cast<v4u*>(to + (tap * 3 + t) * 1024) = words[t];
     }
-    pack(0, blocks / threads);
-    if (started < threads) pack(blocks * started / threads, blocks);
-    for (int t = 1; t < started; ++t) crew[t].join();
+}
+
+int exhip_conv_f32_thirds_pack_device(exhip_ctx* ctx, const exhip_conv_desc* d, const float* w, void* out) {
+    const int steps = d->c / 16, blocks = (d->k + 31) / 32;
+    hipLaunchKernelGGL(pack_thirds_kernel, dim3((unsigned)(blocks * steps)), dim3(64), 0, ctx->stream, w, static_cast<char*>(out), d->c, d->k, steps);
+    EXHIP_LAUNCH_CHECK();
+    return 0;
 }
 
 int exhip_conv_f32_thirds_run(exhip_ctx* ctx, const F32Launch& launch) {

@@ -1965,6 +1965,17 @@ extern "C" int exhip_conv_pack_weights(const exhip_conv_desc* d, int dtype, cons
     return 0;
 }
 
+extern "C" int exhip_conv_packs_on_device(const exhip_conv_desc* d, int dtype) {
+    return dtype == EXHIP_F32 && exhip_conv_f32_validate(d) == 0 && exhip_conv_f32_thirds(d);
+}
+
+extern "C" int exhip_conv_pack_weights_device(exhip_ctx* ctx, const exhip_conv_desc* d, int dtype, const void* w, void* packed) {
+    EXHIP_REQUIRE(ctx && d && w && packed, "exhip_conv_pack_weights_device: NULL argument");
+    EXHIP_REQUIRE(reinterpret_cast<uintptr_t>(w) % 4 == 0 && reinterpret_cast<uintptr_t>(packed) % 16 == 0, "exhip_conv_pack_weights_device: misaligned operand");
+    if (!exhip_conv_packs_on_device(d, dtype)) return EXHIP_ERR_UNSUPPORTED;
+    return exhip_conv_f32_thirds_pack_device(ctx, d, static_cast<const float*>(w), packed);
+}
+
 extern "C" int exhip_conv2d_i8(exhip_ctx* ctx, const exhip_conv_desc* d, const int8_t* x, const void* wp,
                                const float* scale, const float* bias, const float* residual, int8_t* y_i8,
                                float* y_f32_nhwc, float* y_f32_nchw, int32_t* acc_nchw) {

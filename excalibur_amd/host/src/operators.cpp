@@ -399,6 +399,17 @@ const void* operation_convolution<Dtype>::packed_weights(int dtype, const exhip_
     }
     const size_t bytes = exhip_conv_packed_bytes(&d, dtype);
     if (bytes == 0) LOG(FATAL) << "layer " << this->params_.name_ << ": " << exhip_last_error();
+    if (exhip_conv_packs_on_device(&d, dtype)) {
+        const int device = this->params_.device_;
+        const size_t plain = static_cast<size_t>(this->weight_data_size_) * sizeof(float);
+        void* const w = memory::device_alloc(device, plain);
+        void* const dev = memory::device_alloc(device, bytes);
+        EXHIP_FATAL(exhip_memcpy_h2d(this->ctx(), w, this->weights_f32_[0]->cpu_data(), plain));
+        EXHIP_FATAL(exhip_conv_pack_weights_device(this->ctx(), &d, dtype, w, dev));
+        memory::device_release(device, w, plain);  // (what takes the block next is queued behind)
+        packed_[key] = {dev, bytes, ++packed_clock_, 0};
+        return dev;
+    }
     // (not a vector, which would be filled with zeros first: the packing writes every byte)
     const std::unique_ptr<char[]> host(new char[bytes]);
     std::vector<unsigned short> half_w;

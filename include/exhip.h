@@ -165,6 +165,10 @@ int exhip_conv_out_hw(const exhip_conv_desc* d, int* oh, int* ow);
  * exhip_conv_packed_bytes() bytes that the caller then uploads. */
 size_t exhip_conv_packed_bytes(const exhip_conv_desc* d, int dtype);
 int exhip_conv_pack_weights(const exhip_conv_desc* d, int dtype, const void* w_oihw, void* packed);
+/* The same bytes made on the device, both operands in its memory, queued on the context's stream: for layers of which exhip_conv_packs_on_device() says 1
+ * (float32, 3x3 at stride 1 on whole 16-channel steps), EXHIP_ERR_UNSUPPORTED with nothing launched for others. */
+int exhip_conv_packs_on_device(const exhip_conv_desc* d, int dtype);
+int exhip_conv_pack_weights_device(exhip_ctx* ctx, const exhip_conv_desc* d, int dtype, const void* w_oihw, void* packed);
 
 /* operation_convolution::forward_cpu_i8 after quantization (src/Excalibur/operation_convolution.cpp:373-408):
  * acc = int8 x int8 -> int32 convolution; v = fmaf((float)acc, scale[k], bias[k]) (bias NULL = 0);

@@ -1,5 +1,7 @@
 """The float32 convolution with bfloat16 thirds (conv_f32_thirds.hip): every form on ragged shapes, against sums in 64 bits; infinities, NaN and
 values whose thirds would leave the range; and the placements of its results."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -121,6 +123,22 @@ def test_errors_of_few_products_are_no_larger_than_those_of_float32_products(ctx
         mine += np.sum((run(ctx, x, wt, (1, 1, 1, 1)) - want) ** 2)
         theirs += np.sum((y.download().reshape(want.shape) - want) ** 2)
     assert np.sqrt(mine) <= 1.001 * np.sqrt(theirs)
+
+
+@pytest.mark.parametrize("c,k", [(16, 1), (48, 40), (64, 64), (512, 130)])
+def test_weights_packed_on_the_device_are_the_hosts(ctx, c, k):
+    r = np.random.default_rng(c + k)
+    w = (r.standard_normal((k, c, 3, 3)) * np.exp2(r.integers(-150, 120, (k, c, 3, 3)))).astype(np.float32)
+    at = r.random(w.shape)
+    w[at < .02], w[(at > .02) & (at < .04)], w[(at > .04) & (at < .06)], w[(at > .06) & (at < .08)] = np.inf, -np.nan, 0., np.float32(-3.4028235e38)
+    d = ctx.conv_desc(1, c, 20, 20, k, 3, 1, 1, 0, c, hip.pad_to(k, 32))
+    want = ctx.pack_conv_weights(d, hip.F32, w).download().view(np.uint8)
+    got = ctx.array(np.full(want.size + 64, 0xa5, np.uint8))
+    assert hip.lib().exhip_conv_packs_on_device(ctypes.byref(d), hip.F32) == 1
+    hip._check(hip.lib().exhip_conv_pack_weights_device(ctx.h, ctypes.byref(d), hip.F32, ctx.array(w).ptr, got.ptr))
+    ctx.sync()
+    got = got.download()
+    assert (got[-64:] == 0xa5).all() and np.array_equal(got[:-64], want)
 
 
 def test_infinities_nan_and_the_largest_floats(ctx, tile):
