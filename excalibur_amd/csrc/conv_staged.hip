@@ -573,8 +573,11 @@ Plan plan_of(int dt, const PwParams& p, long long images, int subs, int kblocks)
 // channels times k-steps.
 //  * Few blocks: the split form (conv_pw.hip), whose tiles of 32 pixels share a CU by twos and fours (fp16 72 k-steps 502 blocks 0.78, 588 1.06; 36 k-steps 926
 //    blocks 0.85, 1263 1.22).
-//  * 54 and 90 k-steps at stride 1 to 704 of the split form's groups of two blocks, in either type: its waves divide them better (fp16 160 -> 320 at 10 x 13 x 13 8.0 there and 9.1
-//    here, 96 -> 128 at 50 x 14 x 14 8.9 and 9.3, 96 -> 96 at 18 x 25 x 25, 704 groups, equal; int8 320 -> 128 at 1 x 93 x 93 11.2 and 11.8, 192 -> 128 at 50 x 14 x 14 8.0 and 8.5).
+//  * An odd number of pieces at stride 1 leaves the last stage of the forms for small launches, two or four pieces, partly empty. Below 126 k-steps (from there on the split form's own
+//    waves are the longer ones: seven pieces 1.05 to 1.2) such layers stay with the split form up to 704 of its groups of two blocks, in either type: three pieces fp16 160 -> 320 at
+//    10 x 13 x 13 8.0 there and 9.1 here, 96 -> 128 at 50 x 14 x 14 8.9 and 9.3, 96 -> 96 at 18 x 25 x 25, 704 groups, equal; five int8 320 -> 128 at 1 x 93 x 93 11.2 and 11.8, at
+//    49 x 13 x 13 11.0 and 12.3. (Two and four pieces 0.95 to 1.2 between 512 and 704.) One piece is all staging: up to two rounds of 512 groups (fp16 32 -> 160 at
+//    50 x 12 x 11 4.8 there and 6.6 here, 32 -> 352 at 2 x 52 x 52 5.8 and 7.5; equal from there on).
 //  * fp16 at stride 1: everything else that the lean kernel cannot take, 1.04 to 1.6; what it can where its rounds of 256 patches of 256 pixels x 64 channels
 //    take longer: 128 -> 128 at 8 x 40 x 40 13.6 -> 10.4 us, 256 -> 256 at 16 x 20 x 20 20.7 -> 14.8, 64 -> 128 at 11 x 151 x 151 77 -> 47;
 //    its full rounds are 1 to 8 % shorter (64 -> 64 at 64 x 56 x 56, 128 -> 128 at 8 x 80 x 80).
@@ -602,9 +605,9 @@ bool exhip_staged_wins(int dt, const exhip_pw_geom& g, int stride, int n_ksteps,
     const int kblocks = std::min(g.slabs * g.slab_blocks, (std::max(g.k, g.k_stride) + 31) / 32), ks = n_ksteps;
     const long long blocks = (g.pixels + 31) / 32 * kblocks, work = blocks * ks;
     if (blocks <= (dt == EXHIP_F16 && ks < 72 ? 1024 : kStagedBlocks)) return false;
-    const bool odd = ks == 54 || ks == 90;  // k-steps that the split form's waves divide better
+    const bool ragged = g.c_bytes % 128 == 64 && ks < 126;  // an odd number of pieces: the last stage of two or four is not full
     const long long pairs = (g.pixels + 31) / 32 * ((kblocks + 1) / 2);
-    if (odd && stride == 1 && g.c_bytes % 64 == 0 && pairs <= 704) return false;
+    if (ragged && stride == 1 && pairs <= (ks <= 18 ? 1024 : 704)) return false;
     if (dt == EXHIP_F16) return stride == 1 || (ks >= 72 ? blocks > 1280 : (kblocks <= 3 && blocks >= 1536) || blocks >= 12288);
     if (stride == 2 || work < (ks <= 36 ? 46 : 41) * 1024) return false;
     if (g.c_bytes % 64 != 0) return ks >= 45 ? blocks > 768 : ks >= 27 && blocks > 4096 && (g.post_op || shortcut || y_f || !(g.act || g.post_relu));
