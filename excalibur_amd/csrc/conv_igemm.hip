@@ -1927,6 +1927,11 @@ void pack_weights_t(const exhip_conv_desc* d, int dt, const Plan& pl, const T* w
                 }
 }
 
+// Zeros behind the packed weights that the kernel with its input in LDS reads (conv_staged.h).
+size_t packed_pad(const exhip_conv_desc* d, int dtype, const Plan& pl) {
+    return dtype == EXHIP_I8 && !pl.packed && d->kh == 3 && d->kw == 3 && d->sh == 1 && d->c_stride % 64 != 0 ? exhip_staged_pad(pl.TM / 32) : 0;
+}
+
 }  // namespace
 
 int exhip_conv_packed_layout(const exhip_conv_desc* d, int dtype, int* slab_channels, int* packed_form) {
@@ -1950,7 +1955,7 @@ extern "C" size_t exhip_conv_packed_bytes(const exhip_conv_desc* d, int dtype) {
     if (dtype == EXHIP_F32) return exhip_conv_f32_packed_bytes(d);
     Plan pl;
     if (dtype < 0 || dtype > 2 || make_plan(d, dtype, &pl)) return 0;
-    return (size_t)pl.ktiles * pl.n_chunks * d->kh * pl.KWe * pl.KS * (pl.TM / 32) * 1024;
+    return (size_t)pl.ktiles * pl.n_chunks * d->kh * pl.KWe * pl.KS * (pl.TM / 32) * 1024 + packed_pad(d, dtype, pl);
 }
 
 extern "C" int exhip_conv_pack_weights(const exhip_conv_desc* d, int dtype, const void* w, void* packed) {
@@ -1962,6 +1967,8 @@ extern "C" int exhip_conv_pack_weights(const exhip_conv_desc* d, int dtype, cons
     if (rc) return rc;
     if (dtype == EXHIP_I8) pack_weights_t<int8_t>(d, dtype, pl, (const int8_t*)w, (char*)packed);
     else pack_weights_t<uint16_t>(d, dtype, pl, (const uint16_t*)w, (char*)packed);
+    const size_t pad = packed_pad(d, dtype, pl);
+    memset((char*)packed + exhip_conv_packed_bytes(d, dtype) - pad, 0, pad);
     return 0;
 }
 

@@ -26,7 +26,8 @@ bool layer(int dt, int n, int h, int w, int c, int k, int mts, int stride, int f
     p.pixels = n * oh * ow; p.x_bytes = n * h * w * xs_b; p.w_bytes = (kblocks + mts - 1) / mts * steps * mts * 1024;
     p.xs_b = xs_b; p.n_ksteps = steps; p.mts = mts; p.K = k; p.kstride = ks; p.act = 0;
     p.in_h = h; p.in_w = w; p.out_h = oh; p.out_w = ow; p.stride = stride; p.pad_t = p.pad_l = 1; p.kh = p.kw = 3; p.chunk_b = chunk_b; p.fs_out = 1;
-    p.x = ending_at_a_page(p.x_bytes); p.wp = ending_at_a_page(p.w_bytes); p.bias = (float*)ending_at_a_page(k * 4); p.scale = (float*)ending_at_a_page(k * 4);
+    p.x = ending_at_a_page(p.x_bytes); p.wp = ending_at_a_page(p.w_bytes + (xs_b % 64 && dt == EXHIP_I8 ? 9 * mts * 1024 : 0));  // (the packing's zeros behind the weights)
+    p.bias = (float*)ending_at_a_page(k * 4); p.scale = (float*)ending_at_a_page(k * 4);
     char* const y = ending_at_a_page((size_t)p.pixels * ks * es);
     if (dt == EXHIP_I8) p.y_q = (int8_t*)y;
     else p.y = (uint16_t*)y;

@@ -69,6 +69,17 @@ def test_packed_layout(dtype, c, k, kernel):
     raise AssertionError("no slab and chunk give these bytes")
 
 
+@pytest.mark.parametrize("c,k", [(32, 64), (96, 70), (160, 300)])
+def test_int8_pixels_that_end_with_half_a_piece_have_zeros_behind_their_weights(c, k):
+    w = np.random.default_rng(c).integers(1, 120, (k, c, 3, 3)).astype(np.int8)
+    got = pack(hip.Ctx.conv_desc(1, c, 20, 20, k, 3, 1, 1, 0, c, hip.pad_to(k, 32)), hip.I8, w)
+    for slab_blocks in (2, 4):
+        pad = 9 * slab_blocks * 1024
+        if got.size - pad == -(-k // (32 * slab_blocks)) * slab_blocks * 9 * c // 32 * 1024 and not got[-pad:].any() and got[:-pad].any():
+            return
+    raise AssertionError("no slab gives this size")
+
+
 def test_a_pointwise_layer_packs_no_slower_than_its_share_of_a_3x3_layer():
     """The same loop packs both: a weight of a 1x1 layer, whose vectors are plain copies, takes at most twice a 3x3 layer's."""
     def best(kernel):
