@@ -1680,6 +1680,15 @@ int run_conv(exhip_ctx* ctx, const exhip_conv_desc* d, ConvParams p, const PoolS
     Plan pl;
     int rc = make_plan(d, DT, &pl, pool);
     if (rc) return rc;
+    // An int8 layer with a ReLU layer alone behind it is one with that activation: nothing is rounded between the two. The lean kernel has a form for it
+    // (128 -> 128 at 16 x 80 x 80 36.5 -> 21 us, 192 -> 128 at 26 x 26 x 26 14.9 -> 10.2; 60 layers of other kinds the same).
+    exhip_conv_desc as_act;
+    if (DT == EXHIP_I8 && d->post_relu && d->act == 0 && !p.residual && !d->post_op && !d->post_bn_a && !proj) {
+        as_act = *d;
+        as_act.act = 1;
+        as_act.post_relu = 0;
+        d = &as_act;
+    }
     if constexpr (DT == EXHIP_I8) {
         if (!pool) {
             const long long elems = (long long)d->n * pl.OH * pl.OW * d->k;

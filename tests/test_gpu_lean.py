@@ -109,3 +109,21 @@ def test_lean_and_general_kernel_agree_on_a_stage_sized_launch(ctx, options):
         got = gpueval.conv_i8(ctx, case, fs_out=fs_out, residual=res, post_relu=1, want=("nhwc",))
         assert np.array_equal(got["nhwc"], want["nhwc"])
         assert np.array_equal(got["i8"], want["i8"])
+
+
+@pytest.mark.parametrize("floats", [False, True])
+@pytest.mark.parametrize("n,c,hw,k,kernel,stride", [(16, 128, 40, 128, 3, 1), (26, 192, 26, 128, 3, 1), (2, 64, 9, 96, 3, 2), (3, 96, 14, 64, 1, 1), (1, 32, 5, 32, 3, 1)])
+def test_a_relu_behind_the_layer_is_its_activation(ctx, n, c, hw, k, kernel, stride, floats):
+    r = np.random.default_rng(c + k)
+    x, wt = ctx.array(r.integers(-127, 128, (n, hw, hw, c), dtype=np.int8)), r.integers(-127, 128, (k, c, kernel, kernel), dtype=np.int8)
+    scale, bias = (ctx.array(v.astype(np.float32)) for v in (r.uniform(.5, 1.5, k) / (73 * 127 * np.sqrt(c) * kernel), r.normal(0, .3, k)))
+    got = []
+    for act, post in ((1, 0), (0, 1)):
+        d = ctx.conv_desc(n, c, hw, hw, k, kernel, stride, kernel // 2, act, c_stride=c, k_stride=k, fs_out=30.0, post_relu=post)
+        oh, ow = ctx.conv_out_hw(d)
+        y, yf = ctx.empty((n, oh, ow, k), np.int8), ctx.empty((n, oh, ow, k), np.float32) if floats else None
+        ctx.conv2d_i8(d, x, ctx.pack_conv_weights(d, hip.I8, wt), scale, bias, None, y, yf)
+        ctx.sync()
+        got.append((y.download(), yf.download() if floats else None))
+    assert np.array_equal(got[0][0], got[1][0]) and np.unique(got[0][0]).size > 20 and (got[0][0] >= 0).all()
+    assert not floats or got[0][1].tobytes() == got[1][1].tobytes()
