@@ -142,6 +142,71 @@ def test_two_float32_layers(ctx, first, second):
         assert np.array_equal(got.download(), expected) and np.ptp(expected[:-64]) > 1
 
 
+@pytest.mark.parametrize("hw,n", [(128, 3), (96, 1)])
+def test_a_float32_detection_network(tmp_path, hw, n):
+    text, outs = topologies.yolov5s_simp(hw, int8=False)
+    path = str(tmp_path / "net.racy")
+    modelfile.write_model(path, modelfile.SeededModel(modelfile.parse_topology(text), 5, default_fs=16.0, gain=2.0).blobs)
+    x = np.random.default_rng(4).integers(0, 256, (n, 3, hw, hw)).astype(np.float32)
+    got = []
+    for fusion in (True, False):
+        pipe = xp.Pipeline(text, path, 0, "f32", fusion=fusion)
+        for _ in range(2):
+            pipe.set_input(x)
+            pipe.run()
+        assert pipe.stored("465") != fusion  # (a blob that the plan makes in no layout of its own)
+        got.append([pipe.get(name) for name in outs])
+    for a, b in zip(*got):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32)) and np.ptp(a) > 0
+
+
+def test_float32_layers_that_read_what_the_layer_in_front_writes(tmp_path):
+    """Pointwise layers on neighbouring lines: one reads the other's result, the Concat the other is part of, adds the other's result as its shortcut, or adds it through an
+    upsampling: none of them shares a launch with what it reads. The same with nothing read in between."""
+    r = np.random.default_rng(17)
+    lines, blobs = [], []
+
+    def conv(bottom, top, c, k, kernel=1, stride=1, act=0):
+        w = r.normal(0, (c * kernel * kernel) ** -.5, (k, c, kernel, kernel)).astype(np.float32)
+        lines.append(modelfile.conv_line("Convolution", top + "_l", bottom, top, k, kernel, stride, kernel // 2, True, w.size, act=act))
+        blobs.append(modelfile.conv_blob_f32(w, r.normal(0, .5, k).astype(np.float32)))
+
+    def add(*line):
+        lines.append(" ".join(line))
+
+    conv("data", "c0", 3, 32, 3)
+    add("Split s0 1 5 c0 c00 c01 c02 c03 c04")
+    conv("c00", "a", 32, 64)                        # a and b share a launch
+    conv("c01", "b", 32, 32)
+    add("Split s1 1 2 b b0 b1")
+    add("Concat ab 2 1 a b0 ab 0=-1")
+    conv("ab", "d", 96, 32)                         # reads the Concat that b is part of
+    add("Split s2 1 2 d d0 d1")
+    conv("d0", "e", 32, 32)                         # reads d
+    add("Eltwise f_l 2 1 e b1 f 0=1")
+    conv("c02", "g", 32, 32, 3, 2)
+    add("Interp up 1 1 g gu 0=1 1=2.000000e+00 2=2.000000e+00")
+    conv("d1", "h", 32, 32)                         # adds g through the upsampling
+    add("BinaryOp i_l 2 1 gu h i 0=0")
+    conv("c03", "j", 32, 32)
+    conv("c04", "k", 32, 32)
+    add("Eltwise l_l 2 1 k j l 0=1")                # adds the layer in front's result
+    add("Concat out_l 3 1 f i l out 0=-1")
+    conv("out", "m", 96, 48)
+    path = str(tmp_path / "net.racy")
+    modelfile.write_model(path, blobs)
+    pipes = [xp.Pipeline(modelfile.topology(lines, "reads"), path, 0, "f32", fusion=on) for on in (True, False)]
+    for seed, n, hw in ((1, 1, 16), (2, 3, 24), (3, 3, 24)):
+        x = np.random.default_rng(seed).normal(0, 1, (n, 3, hw, hw)).astype(np.float32)
+        got = []
+        for pipe in pipes:
+            pipe.set_input(x)
+            pipe.run()
+            got.append(pipe.get("m"))
+        assert [pipe.stored("c0") for pipe in pipes] == [False, True]
+        assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32)) and np.ptp(got[0]) > .5
+
+
 @pytest.mark.parametrize("int8", [True, False], ids=["int8", "fp16"])
 def test_a_detection_network(tmp_path, int8):
     text, outs = topologies.yolov5s_simp(128, int8=int8)
