@@ -62,15 +62,10 @@ struct BottleneckParams {
     int params_at, wide_at, narrow_at, mid_at;  // LDS: the first layer's parameters; its results; the input's pixels, later depthwise weights and results
 };
 
-__device__ __forceinline__ unsigned round_pair(float lo, float hi) {  // (written out: left to itself the compiler may round a product to half in one step)
-    unsigned d;
-    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(d) : "v"(lo), "v"(hi));
-    return d;
-}
 __device__ __forceinline__ void round_halves(float (&v)[16]) {
 #pragma unroll
     for (int e = 0; e < 16; e += 2) {
-        const unsigned d = round_pair(v[e], v[e + 1]);
+        const unsigned d = exhip_round_pair(v[e], v[e + 1]);
         v[e] = exhip_h2f((uint16_t)(d & 0xffff));
         v[e + 1] = exhip_h2f((uint16_t)(d >> 16));
     }
@@ -80,9 +75,9 @@ __device__ __forceinline__ void round_halves(float (&v)[16]) {
 // zero here; the sums behind begin with one, so nothing follows from that.)
 // Sixteen bits of a sign by one packed shift and the selection by one v_bfi: left to itself the compiler takes the pair apart (14 instructions for 6).
 __device__ __forceinline__ unsigned prelu_pair(float lo, float hi, float slope_lo, float slope_hi) {
-    const unsigned h = round_pair(lo, hi);
+    const unsigned h = exhip_round_pair(lo, hi);
     const v2h v = __builtin_bit_cast(v2h, h);
-    const unsigned below = round_pair(__builtin_fmaf((float)v[0], slope_lo, 0.f), __builtin_fmaf((float)v[1], slope_hi, 0.f));
+    const unsigned below = exhip_round_pair(__builtin_fmaf((float)v[0], slope_lo, 0.f), __builtin_fmaf((float)v[1], slope_hi, 0.f));
     unsigned negative;
     asm("v_pk_ashrrev_i16 %0, %1, %2" : "=v"(negative) : "v"(0x000f000f), "v"(h));
     return (below & negative) | (h & ~negative);
@@ -253,7 +248,7 @@ __global__ __launch_bounds__(64 * WAVES, RUNS == 2 ? 3 : 4) void bottleneck_kern
                         for (int e = 0; e < 16; ++e) v[e] = (0.f > v[e]) ? 0.f : v[e];
                     }
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) o[e] = round_pair(v[2 * e], v[2 * e + 1]);
+                    for (int e = 0; e < 8; ++e) o[e] = exhip_round_pair(v[2 * e], v[2 * e + 1]);
                 }
 #pragma unroll
                 for (int e = 0; e < 8; ++e) o[e] = in[n] ? o[e] : 0;  // the depthwise layer's padding
@@ -324,7 +319,7 @@ __global__ __launch_bounds__(64 * WAVES, RUNS == 2 ? 3 : 4) void bottleneck_kern
                             if (p.dw_act == 3) res[e] = res[e] <= 6.f ? res[e] : 0.f;
                         }
                     }
-                    o = v2i{(int)round_pair(res[0], res[1]), (int)round_pair(res[2], res[3])};
+                    o = v2i{(int)exhip_round_pair(res[0], res[1]), (int)exhip_round_pair(res[2], res[3])};
                 }
                 *reinterpret_cast<v2i*>(mid + (oy * p.tw + ox + px) * wide_pitch + g * 8) = o;
             }
@@ -365,7 +360,7 @@ __global__ __launch_bounds__(64 * WAVES, RUNS == 2 ? 3 : 4) void bottleneck_kern
         }
         v4i o[2];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) o[e >> 2][e & 3] = (int)round_pair(v[2 * e], v[2 * e + 1]);
+        for (int e = 0; e < 8; ++e) o[e >> 2][e & 3] = (int)exhip_round_pair(v[2 * e], v[2 * e + 1]);
         *reinterpret_cast<v4i*>(slice + (lane & 31) * kSlicePitch + half * 32) = o[0];
         *reinterpret_cast<v4i*>(slice + (lane & 31) * kSlicePitch + half * 32 + 16) = o[1];
         // four neighbouring lanes store a pixel's 64 bytes

@@ -214,6 +214,14 @@ __device__ __forceinline__ float exhip_act(float v, int act) {
 __device__ __forceinline__ float exhip_h2f(uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
 __device__ __forceinline__ uint16_t exhip_f2h(float f) { return __builtin_bit_cast(uint16_t, (_Float16)f); }
 
+// Two float32 values rounded to nearest-even halves, one instruction. (Written out: left to itself the compiler may round a
+// product to half in one step, which is another value than the float32 product rounded.)
+__device__ __forceinline__ unsigned exhip_round_pair(float lo, float hi) {
+    unsigned d;
+    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(d) : "v"(lo), "v"(hi));
+    return d;
+}
+
 // One value of an elementwise activation. OP 0 HardSwish, 1 LeakyReLU, 2 sigmoid, 3 HardSigmoid, 4 Clip; the multiply-adds
 // are fused where the CPU path's are (vector fmadd, and scalar expressions contracted by its compiler flags).
 template <int OP>

@@ -25,6 +25,7 @@
 #include "conv_f32.h"
 #include "conv_f32_epilogue.h"
 #include "pack.h"
+#include "pair.h"
 
 namespace {
 
@@ -542,14 +543,7 @@ __global__ __launch_bounds__(256, 2) void conv_f32_two_kernel(const F32Params a,
     else two_group(b, q.kind[1], lds, blockIdx.x - first, q.groups[1]);
 }
 
-// A launch that waits for another one to share it with (exhip_conv2d_f32_pair).
-struct Waiting {
-    int kind = -1;
-    unsigned groups = 0;
-    const void* kernel = nullptr;
-    F32Params p;
-};
-thread_local Waiting* t_collect = nullptr;  // while the pair's layers are run: the place for the next launch
+thread_local exhip_waiting<F32Params>* t_collect = nullptr;  // (exhip_conv2d_f32_pair)
 
 template <int MT, int NT, int WK, int R, int MODE, bool PAIRS, bool SLOW>
 int go(exhip_ctx* ctx, F32Params& p, int kblocks) {
@@ -782,35 +776,16 @@ extern "C" int exhip_conv2d_f32_placed(exhip_ctx* ctx, const exhip_conv_desc* d,
     return run_conv_f32(ctx, d, place, x, wp, bias, residual, y, y_f32_nchw);
 }
 
-static int run_pair(exhip_ctx* ctx, int (*layer)(exhip_ctx*, const void*), const void* first, const void* second) {
-    Waiting w[2];
-    int rc = 0;
-    for (int i = 0; i < 2 && !rc; ++i) {
-        t_collect = &w[i];
-        rc = layer(ctx, i ? second : first);
-        t_collect = nullptr;
-    }
-    // (a layer that ran by itself is done; it reads nothing of the other's)
-    if (!rc && w[0].kind >= 0 && w[1].kind >= 0 && (long long)w[0].groups + w[1].groups < (1ll << 31)) {
-        const F32Two q = {{w[0].kind, w[1].kind}, {w[0].groups, w[1].groups}};
-        hipLaunchKernelGGL(conv_f32_two_kernel, dim3(w[0].groups + w[1].groups), dim3(256), 0, ctx->stream, w[0].p, w[1].p, q);
-        EXHIP_LAUNCH_CHECK();
-        return 0;
-    }
-    for (Waiting& one : w) {
-        if (one.kind < 0) continue;
-        void* args[] = {&one.p};
-        EXHIP_CHECK(hipLaunchKernel(one.kernel, dim3(one.groups), dim3(256), args, 0, ctx->stream));
-        EXHIP_LAUNCH_CHECK();
-    }
-    return rc;
-}
-
 extern "C" int exhip_conv2d_f32_pair(exhip_ctx* ctx, const exhip_conv_f32_call* a, const exhip_conv_f32_call* b) {
     EXHIP_REQUIRE(ctx && a && b && a->d && a->place && b->d && b->place, "exhip_conv2d_f32_pair: NULL argument");
     auto layer = [](exhip_ctx* on, const void* call) {
         const auto* c = static_cast<const exhip_conv_f32_call*>(call);
         return exhip_conv2d_f32_placed(on, c->d, c->place, c->x, c->w_packed, c->bias, c->residual, c->y, c->y_nchw);
     };
-    return run_pair(ctx, layer, a, b);
+    return exhip_run_pair(ctx, &t_collect, layer, a, b, [ctx](const exhip_waiting<F32Params>* w) {
+        const F32Two q = {{w[0].kind, w[1].kind}, {w[0].groups, w[1].groups}};
+        hipLaunchKernelGGL(conv_f32_two_kernel, dim3(w[0].groups + w[1].groups), dim3(256), 0, ctx->stream, w[0].p, w[1].p, q);
+        EXHIP_LAUNCH_CHECK();
+        return 0;
+    });
 }

@@ -14,9 +14,8 @@
 // under a run of pixels, 16 * CS channels at a time, and takes the nine taps from there; a split in registers would cost every wave 44
 // vector instructions per 32 pixels, tap and step. Weight fragments come straight from memory, three taps ahead.
 //
-// A group's pixels are neighbours in a list of the output's vertical strips, row by row (a strip of a 13 x 13 map is the map). So ragged maps
-// waste no lanes, small maps of several images share groups, and what a run needs of the input are whole rows of a strip, one after
-// another, whatever the run begins with. WK waves share a run's steps, their sums meet in LDS in a fixed order.
+// A group's pixels are neighbours in a list of the output's vertical strips, row by row (strips.h; a strip of a 13 x 13 map is the map). WK waves share a run's
+// steps, their sums meet in LDS in a fixed order.
 //
 // Bounded by the matrix unit on large maps (128 -> 128 at 16 x 80 x 80 183 us, 165 TFLOP/s of float32 work, conv_f32_kernel 223) and by a group's chain of
 // loads, split and products on small ones: us, conv_f32_kernel and this one, launches queued from Python, 64 -> 64 on one 56 x 56 map 6.7, 5.5, at 160 x 160 23.5, 18.6,
@@ -36,6 +35,7 @@
 
 #include "conv_f32.h"
 #include "conv_f32_epilogue.h"
+#include "strips.h"
 
 namespace {
 
@@ -50,10 +50,8 @@ constexpr int kLdsLimit = 160 * 1024;
 
 struct ThirdsParams {
     F32Params f;
-    unsigned total;                // pixels of the list (strips of a ragged width count their missing columns)
-    unsigned strip_w, strips;
-    exhip_divisor by_fast, by_strip_w, by_height, by_strips, by_rows, by_cols;
-    int staged_rows, staged_cols;  // input rows of a map and columns of a strip with their border
+    exhip_strip_list list;
+    exhip_divisor by_fast;
     int chunks;                    // 16 * CS channels each
     int table_b, buffer_b;         // bytes of the tables in front of the staged pixels, and of a buffer of those
     float floor, post_floor;       // `plain`: what the activation and the ReLU behind the shortcut cut off at, -inf: nothing
@@ -75,21 +73,6 @@ __device__ __forceinline__ void split_thirds(v4f x, v2u& h, v2u& m, v2u& l) {
         b -= __uint_as_float(m[i] & 0xffff0000u);
         l[i] = bf16_pair(a, b);
     }
-}
-
-// The pixel at a place of the list: its number in the output (p.pixels or more: none), its row of all staged ones and its column of the strip.
-struct Where {
-    unsigned pix;
-    int row, x;
-};
-__device__ __forceinline__ Where where(const ThirdsParams& p, unsigned at) {
-    const unsigned in = at < p.total ? at : p.total - 1, row = p.by_strip_w(in), map = p.by_height(row), img = p.by_strips(map);
-    const unsigned col = in - row * p.strip_w, y = row - map * (unsigned)p.f.out_h, x = (map - img * p.strips) * p.strip_w + col;
-    Where w;
-    w.row = (int)(map * (unsigned)p.staged_rows + y);
-    w.x = (int)col;
-    w.pix = at < p.total && x < (unsigned)p.f.out_w ? (img * (unsigned)p.f.out_h + y) * (unsigned)p.f.out_w + x : 0xffffffffu;
-    return w;
 }
 
 constexpr unsigned kLeast = 0x0c000000;  // 2^-103: every third of a larger float32 is a normal number
@@ -368,16 +351,11 @@ __global__ __launch_bounds__(64 * WK * WP, OCC) void conv3x3_thirds_kernel(const
 
     // the staged rows: those under the run's first pixel to those under its last
     const unsigned run0 = tile * RUN;
-    const int first_row = __builtin_amdgcn_readfirstlane(where(q, run0).row), last_row = __builtin_amdgcn_readfirstlane(where(q, run0 + RUN - 1).row) + 2;
-    const int staged = (last_row - first_row + 1) * q.staged_cols;
+    const int first_row = __builtin_amdgcn_readfirstlane(q.list.where<1>(run0, p.out_h, p.out_w).row);
+    const int last_row = __builtin_amdgcn_readfirstlane(q.list.where<1>(run0 + RUN - 1, p.out_h, p.out_w).row) + 2;
+    const int staged = (last_row - first_row + 1) * q.list.staged_cols;
     if (threadIdx.x == 0) *again = 0;
-    for (int i = threadIdx.x; i < staged; i += THREADS) {
-        const unsigned r = q.by_cols((unsigned)i), row = (unsigned)first_row + r, map = q.by_rows(row), img = q.by_strips(map);
-        const int c = i - (int)r * q.staged_cols;
-        const int y = (int)(row - map * (unsigned)q.staged_rows) - p.pad_t, x = (int)((map - img * q.strips) * q.strip_w) + c - p.pad_l;
-        const bool in = (unsigned)y < (unsigned)p.in_h && (unsigned)x < (unsigned)p.in_w;
-        table[i] = in ? ((img * (unsigned)p.in_h + (unsigned)y) * (unsigned)p.in_w + (unsigned)x) * (unsigned)p.xs_b : kOutOfRange;
-    }
+    for (int i = threadIdx.x; i < staged; i += THREADS) table[i] = q.list.staged_pixel<1>(i, first_row, p.in_h, p.in_w, p.pad_t, p.pad_l, p.xs_b, kOutOfRange);
     __syncthreads();
     v4f x[BATCH];
     const int my_piece = threadIdx.x % PIECES, my_pixel = threadIdx.x / PIECES;
@@ -412,11 +390,11 @@ __global__ __launch_bounds__(64 * WK * WP, OCC) void conv3x3_thirds_kernel(const
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
         const int at = (side * NT + n) * 32 + (lane & 31);
-        const Where w = where(q, run0 + at);
+        const auto w = q.list.where<1>(run0 + at, p.out_h, p.out_w);
         if (part == 0) pixels[at] = w.pix;
-        b_at[n] = stage + ((w.row - first_row) * q.staged_cols + w.x) * PITCH + half * 16;
+        b_at[n] = stage + ((w.row - first_row) * q.list.staged_cols + w.x) * PITCH + half * 16;
     }
-    const int tap_row = q.staged_cols * PITCH;
+    const int tap_row = q.list.staged_cols * PITCH;
     v16f acc[MT][NT], low[MT][NT];
 #pragma unroll
     for (int m = 0; m < MT; ++m)
@@ -569,39 +547,11 @@ __global__ __launch_bounds__(64 * WK * WP, OCC) void conv3x3_thirds_kernel(const
 
 std::mutex g_attr_mutex;
 
-// A launch's strips and form.
+// A launch's form and strips.
 struct Plan {
     int form = -1;
-    unsigned width = 0, strips = 0;
-    int staged = 0;  // pixels that a group stages at most
-    long long tiles = 0;
+    exhip_strips strips;
 };
-
-// The strips for runs of `run` pixels: of all widths that split the map evenly the one whose groups, weighed with what they stage, are least,
-// among those of at most `most` staged pixels where there are any.
-// `wide`: strips of a column that does not exist beside the map's only one.
-void choose_strips(const F32Params& p, long long images, int run, int most, bool wide, Plan* plan) {
-    double best_cost = 0;
-    for (int width = wide ? 2 : p.out_w;;) {
-        const int count = (p.out_w + width - 1) / width;
-        if (!wide) width = (p.out_w + count - 1) / count;  // the narrowest of that many
-        const long long tiles = ((long long)count * width * p.out_h * images + run - 1) / run;
-        // rows that a run touches beside its first, maps that it enters beside its first, and their rows and columns with the border
-        const int rows = run % width == 0 ? run / width - 1 : (run + width - 2) / width;
-        const int crossed = (int)std::min<long long>((rows + p.out_h - 1) / p.out_h, images * count - 1);
-        const int staged = (rows + 2 * crossed + 3) * (width + 2);
-        const double cost = (staged > most ? 1e18 * staged : 0.) + (double)tiles * (run + 0.2 * staged);
-        if (plan->width == 0 || cost < best_cost) {
-            plan->width = (unsigned)width;
-            plan->strips = (unsigned)count;
-            plan->staged = staged;
-            plan->tiles = tiles;
-            best_cost = cost;
-        }
-        if (wide || (width <= 4 && (width == 1 || plan->staged <= most))) break;
-        --width;
-    }
-}
 
 constexpr int kForms = 5;
 struct Shape {
@@ -664,10 +614,9 @@ const Plan& plan_of(const F32Params& p, long long images, int kblocks, int tile)
         for (int tries = 0; tries < 3; ++tries) {
             const int form = tries ? 0 : chosen, buffers = p.csteps > kForm[form].cs ? 2 : 1;
             const Sizes s(kForm[form]);
-            e.plan = Plan();
             e.plan.form = form;
-            choose_strips(p, images, s.run, s.most(buffers), tries == 2, &e.plan);
-            if (s.lds(e.plan.staged, buffers) <= kLdsLimit) break;
+            e.plan.strips = exhip_choose_strips(p.out_h, p.out_w, 1, images, s.run, s.most(buffers), tries == 2);
+            if (s.lds(e.plan.strips.staged, buffers) <= kLdsLimit) break;
         }
         e.images = images;
     }
@@ -680,25 +629,16 @@ int go(exhip_ctx* ctx, ThirdsParams& q, const Plan& plan, long long images, int 
     const Sizes s(f);
     F32Params& p = q.f;
     q.chunks = (p.csteps + f.cs - 1) / f.cs;
-    const int lds = s.lds(plan.staged, q.chunks > 1 ? 2 : 1);
-    EXHIP_REQUIRE(lds <= kLdsLimit, "conv: %d pixels to stage", plan.staged);
-    q.strip_w = plan.width;
-    q.strips = plan.strips;
-    q.total = (unsigned)((long long)plan.width * plan.strips * p.out_h * images);
-    q.staged_rows = p.out_h + 2;
-    q.staged_cols = (int)plan.width + 2;
-    q.by_strip_w.set(plan.width);
-    q.by_strips.set(plan.strips);
-    q.by_height.set((unsigned)p.out_h);
-    q.by_rows.set((unsigned)q.staged_rows);
-    q.by_cols.set((unsigned)q.staged_cols);
-    q.table_b = s.table_bytes(plan.staged);
-    q.buffer_b = (plan.staged + 1) * s.pitch;
-    const long long groups = (kblocks + f.mt - 1) / f.mt, items = plan.tiles * groups;
+    const int lds = s.lds(plan.strips.staged, q.chunks > 1 ? 2 : 1);
+    EXHIP_REQUIRE(lds <= kLdsLimit, "conv: %d pixels to stage", plan.strips.staged);
+    q.list.set(plan.strips, p.out_h, 1, images);
+    q.table_b = s.table_bytes(plan.strips.staged);
+    q.buffer_b = (plan.strips.staged + 1) * s.pitch;
+    const long long groups = (kblocks + f.mt - 1) / f.mt, items = plan.strips.tiles * groups;
     EXHIP_REQUIRE(items < (1ll << 31) - 4, "conv: grid too large");
     p.items = (unsigned)items;
     p.tiles_fast = p.w_bytes > (4u << 20) && p.w_bytes > p.x_bytes;  // (conv_f32_kernel)
-    p.fast = (unsigned)(p.tiles_fast ? plan.tiles : groups);
+    p.fast = (unsigned)(p.tiles_fast ? plan.strips.tiles : groups);
     q.by_fast.set(p.fast);
     auto kernel = conv3x3_thirds_kernel<f.mt, f.nt, f.wk, f.wp, f.cs, f.occ, SLOW>;
     {

@@ -29,6 +29,7 @@
 
 #include "conv_pw_epilogue.h"
 #include "conv_staged.h"
+#include "pair.h"
 
 namespace {
 
@@ -495,7 +496,7 @@ __device__ __forceinline__ void split_group(const PwParams& p, char* lds_all, un
                 __builtin_amdgcn_raw_buffer_store_b64(o, tile_view(p.y_q, tile * 32, p.kstride, kb * 32, rows), pw_lane_offset(row, p.kstride, ch, k_end - kb * 32), 0, 0);
             }
         } else {
-            const v4u o = {round_pair(v[0], v[1]), round_pair(v[2], v[3]), round_pair(v[4], v[5]), round_pair(v[6], v[7])};
+            const v4u o = {exhip_round_pair(v[0], v[1]), exhip_round_pair(v[2], v[3]), exhip_round_pair(v[4], v[5]), exhip_round_pair(v[6], v[7])};
             __builtin_amdgcn_raw_buffer_store_b128(o, tile_view(p.y, tile * 32, p.kstride * 2, kb * 64, rows), pw_lane_offset(row, p.kstride * 2, ch * 2, (k_end - kb * 32) * 2), 0, 0);
         }
     }
@@ -679,7 +680,7 @@ __global__ __launch_bounds__(256, 3) void dw_pw_kernel(const PwParams p) {
                         if (p.dw_act == 3) res[e] = res[e] <= 6.f ? res[e] : 0.f;
                     }
                 }
-                const v2i o = {(int)round_pair(res[0], res[1]), (int)round_pair(res[2], res[3])};
+                const v2i o = {(int)exhip_round_pair(res[0], res[1]), (int)exhip_round_pair(res[2], res[3])};
                 *reinterpret_cast<v2i*>(mid + (st * PX + px) * mid_pitch + g * 8) = o;
             }
         };
@@ -965,14 +966,7 @@ int run_stem(exhip_ctx* ctx, const exhip_pw_geom& g, const exhip_pw_taps& t, int
     return vec ? go_stem<DT, 2, true>(ctx, p, lds) : go_stem<DT, 2, false>(ctx, p, lds);
 }
 
-// A launch that waits for another one to share it with (exhip_pw_pair).
-struct Waiting {
-    int kind = -1, dt = 0;
-    unsigned groups = 0;
-    const void* kernel = nullptr;
-    PwParams p;
-};
-thread_local Waiting* t_collect = nullptr;  // while the pair's layers are run: the place for the next launch
+thread_local exhip_waiting<PwParams>* t_collect = nullptr;  // (exhip_pw_pair)
 
 // U > 0: the kernel with U k-steps a request round, 100 + U in pairs; U < 0: the split form, -kSplit a k-step at a time, -2 * kSplit in pairs
 template <int DT, int MT, int NT, int U, bool TAPS, typename EP>
@@ -1434,16 +1428,8 @@ bool exhip_pw_splits_f16(long long pixels, int c_bytes, int k, int k_stride, int
 }
 
 int exhip_pw_pair(exhip_ctx* ctx, int (*layer)(exhip_ctx*, const void*), const void* first, const void* second) {
-    Waiting w[2];
-    int rc = 0;
-    for (int i = 0; i < 2 && !rc; ++i) {
-        t_collect = &w[i];
-        rc = layer(ctx, i ? second : first);
-        t_collect = nullptr;
-    }
-    // (a layer that ran by itself is done; it reads nothing of the other's)
-    const bool fits = (long long)w[0].groups + w[1].groups < (1ll << 31);
-    if (!rc && w[0].kind >= 0 && w[1].kind >= 0 && w[0].dt == w[1].dt && fits) {
+    return exhip_run_pair(ctx, &t_collect, layer, first, second, [ctx](const exhip_waiting<PwParams>* w) {
+        if (w[0].dt != w[1].dt) return EXHIP_ERR_UNSUPPORTED;
         PwTwo q;
         for (int i = 0; i < 2; ++i) q.p[i] = w[i].p, q.kind[i] = w[i].kind, q.groups[i] = w[i].groups;
         const dim3 grid(w[0].groups + w[1].groups);
@@ -1451,12 +1437,5 @@ int exhip_pw_pair(exhip_ctx* ctx, int (*layer)(exhip_ctx*, const void*), const v
         else hipLaunchKernelGGL(conv_pw_two_kernel<EXHIP_F16>, grid, dim3(256), 0, ctx->stream, q);
         EXHIP_LAUNCH_CHECK();
         return 0;
-    }
-    for (Waiting& one : w) {
-        if (one.kind < 0) continue;
-        void* args[] = {&one.p};
-        EXHIP_CHECK(hipLaunchKernel(one.kernel, dim3(one.groups), dim3(256), args, 0, ctx->stream));
-        EXHIP_LAUNCH_CHECK();
-    }
-    return rc;
+    });
 }

@@ -121,21 +121,13 @@ __device__ __forceinline__ void read_parameters(const char* lds, int which, int 
     }
 }
 
-// Two float32 values rounded to nearest-even halves, one instruction. (Written out: left to itself the compiler may round a
-// product to half in one step, which is another value than the float32 product rounded.)
-__device__ __forceinline__ unsigned round_pair(float lo, float hi) {
-    unsigned d;
-    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(d) : "v"(lo), "v"(hi));
-    return d;
-}
-
 // ROUND: the layer behind reads the halves that the layer in front of it stored.
 template <bool ROUND, int N>
 __device__ __forceinline__ void stored(float (&v)[N]) {
     if constexpr (ROUND) {
 #pragma unroll
         for (int e = 0; e < N; e += 2) {
-            const unsigned d = round_pair(v[e], v[e + 1]);
+            const unsigned d = exhip_round_pair(v[e], v[e + 1]);
             v[e] = exhip_h2f((uint16_t)(d & 0xffff));
             v[e + 1] = exhip_h2f((uint16_t)(d >> 16));
         }
@@ -334,7 +326,7 @@ __device__ __forceinline__ void pw_epilogue(const PwParams& p, const ACC (&acc)[
                 constexpr int pitch = MT * 64 + 16;
                 v4i o[2];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) o[e >> 2][e & 3] = (int)round_pair(v[2 * e], v[2 * e + 1]);
+                for (int e = 0; e < 8; ++e) o[e >> 2][e & 3] = (int)exhip_round_pair(v[2 * e], v[2 * e + 1]);
                 *reinterpret_cast<v4i*>(tile + row * pitch + m * 64 + half * 32) = o[0];
                 *reinterpret_cast<v4i*>(tile + row * pitch + m * 64 + half * 32 + 16) = o[1];
             }

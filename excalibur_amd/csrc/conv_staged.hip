@@ -3,7 +3,7 @@
 // The tapped form of conv_pw.hip reads every pixel up to nine times through a CU's address path, a KiB and a half for each MFMA: 96 cycles of L1 for 32 of the matrix unit.
 // The lean kernel (conv_i8_lean.hip) stages patches of up to 256 pixels x 64 channels, one a CU: a launch of 300 patches is two rounds, maps that patches do not divide
 // waste lanes, and four waves that all wait for the same barrier hide nothing from each other. Here a group's 64 to 256 pixels are neighbours
-// in a list of the output's vertical strips, row by row, whatever map they belong to (as in conv_f32_thirds.hip), three groups share a CU, and
+// in a list of the output's vertical strips, row by row, whatever map they belong to (strips.h), three groups share a CU, and
 // up to four waves share a run's sums where the launch is small. Pixels come from LDS (64 x 64 a wave: half a KiB for each MFMA, as
 // much of the weights from the caches, a filter row's six k-steps ahead); a run's input is staged 64 to 256 bytes a pixel at a time, the
 // next piece on its way into registers meanwhile. At stride 2 a staged row holds its even columns first, so that neighbouring lanes read neighbouring pixels.
@@ -20,6 +20,7 @@
 
 #include "conv_pw_epilogue.h"
 #include "conv_staged.h"
+#include "strips.h"
 
 namespace {
 
@@ -27,30 +28,12 @@ constexpr int kLdsLimit = 160 * 1024;
 
 struct StagedParams {
     PwParams f;
-    unsigned total;                // pixels of the list (strips of a ragged width count their missing columns)
-    unsigned strip_w, strips;
-    exhip_divisor by_groups, by_strip_w, by_height, by_strips, by_rows, by_cols;
-    int staged_rows, staged_cols;  // input rows of a map and columns of a strip with their border
+    exhip_divisor by_groups;
+    exhip_strip_list list;
     int subs, chunks;              // pieces of 64 bytes of a pixel, and what is staged of them at a time
     int tap_w, half_w;             // bytes of the weights from a tap to the next one, and from a piece's first half to its second
     int table_b;                   // bytes of the table in front of the staged pixels
 };
-
-// The pixel at a place of the list: its number in the output (or none), its first row of all staged ones and its column of the strip.
-struct Where {
-    unsigned pix;
-    int row, x;
-};
-template <int S>
-__device__ __forceinline__ Where where(const StagedParams& p, unsigned at) {
-    const unsigned in = at < p.total ? at : p.total - 1, row = p.by_strip_w(in), map = p.by_height(row), img = p.by_strips(map);
-    const unsigned col = in - row * p.strip_w, y = row - map * (unsigned)p.f.out_h, x = (map - img * p.strips) * p.strip_w + col;
-    Where w;
-    w.row = (int)(map * (unsigned)p.staged_rows + y * S);
-    w.x = (int)col;
-    w.pix = at < p.total && x < (unsigned)p.f.out_w ? (img * (unsigned)p.f.out_h + y) * (unsigned)p.f.out_w + x : 0xffffffffu;
-    return w;
-}
 
 // Rows of 32 pixels anywhere in the output from an LDS tile to memory: CHUNKS 16-byte pieces a row, neighbouring lanes on neighbouring pieces.
 template <int CHUNKS>
@@ -140,7 +123,7 @@ __device__ __forceinline__ void scattered_epilogue(const PwParams& p, const ACC 
                 constexpr int pitch = MT * 64 + 16;
                 v4i o[2];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) o[e >> 2][e & 3] = (int)round_pair(v[2 * e], v[2 * e + 1]);
+                for (int e = 0; e < 8; ++e) o[e >> 2][e & 3] = (int)exhip_round_pair(v[2 * e], v[2 * e + 1]);
                 *reinterpret_cast<v4i*>(tile + row * pitch + m * 64 + half * 32) = o[0];
                 *reinterpret_cast<v4i*>(tile + row * pitch + m * 64 + half * 32 + 16) = o[1];
             }
@@ -191,17 +174,11 @@ __global__ __launch_bounds__(64 * WK * WP, 3) void conv3x3_staged_kernel(const S
 
     // the staged rows: those under the run's first pixel to those under its last
     const unsigned run0 = tile * RUN;
-    const int first_row = __builtin_amdgcn_readfirstlane(where<S>(q, run0).row), last_row = __builtin_amdgcn_readfirstlane(where<S>(q, run0 + RUN - 1).row) + 2;
-    const int staged = (last_row - first_row + 1) * q.staged_cols;
-    const int even_cols = (q.staged_cols + 1) >> 1;  // S == 2: a row's even columns first, so that neighbouring pixels' taps are neighbours
-    for (int i = threadIdx.x; i < staged; i += THREADS) {
-        const unsigned r = q.by_cols((unsigned)i), row = (unsigned)first_row + r, map = q.by_rows(row), img = q.by_strips(map);
-        int c = i - (int)r * q.staged_cols;
-        if constexpr (S == 2) c = c < even_cols ? 2 * c : 2 * (c - even_cols) + 1;
-        const int y = (int)(row - map * (unsigned)q.staged_rows) - p.pad_t, x = (int)((map - img * q.strips) * q.strip_w) * S + c - p.pad_l;
-        const bool in = (unsigned)y < (unsigned)p.in_h && (unsigned)x < (unsigned)p.in_w;
-        table[i] = in ? (int)(((img * (unsigned)p.in_h + (unsigned)y) * (unsigned)p.in_w + (unsigned)x) * (unsigned)p.xs_b) : kOutOfRange;
-    }
+    const int first_row = __builtin_amdgcn_readfirstlane(q.list.template where<S>(run0, p.out_h, p.out_w).row);
+    const int last_row = __builtin_amdgcn_readfirstlane(q.list.template where<S>(run0 + RUN - 1, p.out_h, p.out_w).row) + 2;
+    const int staged = (last_row - first_row + 1) * q.list.staged_cols;
+    const int even_cols = (q.list.staged_cols + 1) >> 1;  // S == 2: a row's even columns come first
+    for (int i = threadIdx.x; i < staged; i += THREADS) table[i] = (int)q.list.template staged_pixel<S>(i, first_row, p.in_h, p.in_w, p.pad_t, p.pad_l, p.xs_b, kOutOfRange);
     __syncthreads();
     v4i x[BATCH];
     const int my_piece = threadIdx.x % PIECES, my_pixel = threadIdx.x / PIECES;
@@ -239,11 +216,11 @@ __global__ __launch_bounds__(64 * WK * WP, 3) void conv3x3_staged_kernel(const S
     unsigned pix[NT];
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
-        const Where w = where<S>(q, run0 + (side * NT + n) * 32 + (lane & 31));
+        const auto w = q.list.template where<S>(run0 + (side * NT + n) * 32 + (lane & 31), p.out_h, p.out_w);
         pix[n] = w.pix;
-        b_at[n] = stage + ((w.row - first_row) * q.staged_cols + w.x) * PITCH + half * 16;
+        b_at[n] = stage + ((w.row - first_row) * q.list.staged_cols + w.x) * PITCH + half * 16;
     }
-    const int tap_row = q.staged_cols * PITCH, tap_col[3] = {0, S == 2 ? even_cols * PITCH : PITCH, S == 2 ? PITCH : 2 * PITCH};
+    const int tap_row = q.list.staged_cols * PITCH, tap_col[3] = {0, S == 2 ? even_cols * PITCH : PITCH, S == 2 ? PITCH : 2 * PITCH};
     typedef typename std::conditional<DT == EXHIP_I8, v16i, v16f>::type acc_t;
     typedef typename std::conditional<DT == EXHIP_I8, v4i, v4f>::type four_t;
     acc_t acc[MT][NT];
@@ -380,37 +357,8 @@ __global__ __launch_bounds__(64 * WK * WP, 3) void conv3x3_staged_kernel(const S
 
 std::mutex g_attr_mutex;
 
-struct Strips {
-    int width = 0, count = 0, staged = 0;
-    long long tiles = 0;
-};
-
 // Staged pixels with which three groups share a CU, as many as their registers allow.
 int most_staged(int pitch) { return (kLdsLimit / 3 - 1280 - 16) / (pitch + 4); }
-
-// The strips for runs of `run` pixels: of all widths that split the map evenly the one whose groups, weighed with what they stage, are least, among those of
-// at most `most` staged pixels where there are any.
-Strips choose_strips(const PwParams& p, long long images, int run, int most) {
-    Strips best;
-    double best_cost = 0;
-    for (int width = p.out_w;;) {
-        const int count = (p.out_w + width - 1) / width;
-        width = (p.out_w + count - 1) / count;  // the narrowest of that many
-        const long long tiles = ((long long)count * width * p.out_h * images + run - 1) / run;
-        // rows that a run touches beside its first, maps that it enters beside its first, and their rows and columns with the border
-        const int rows = run % width == 0 ? run / width - 1 : (run + width - 2) / width;
-        const int crossed = (int)std::min<long long>((rows + p.out_h - 1) / p.out_h, images * count - 1);
-        const int staged = (rows * p.stride + crossed * (3 - p.stride) + 3) * ((width - 1) * p.stride + 3);
-        const double cost = (staged > most ? 1e18 * staged : 0.) + (double)tiles * (run + 0.2 * staged);
-        if (best.width == 0 || cost < best_cost) {
-            best.width = width; best.count = count; best.staged = staged; best.tiles = tiles;
-            best_cost = cost;
-        }
-        if (width <= 4 && (width == 1 || best.staged <= most)) break;
-        --width;
-    }
-    return best;
-}
 
 struct Launch {
     unsigned groups;
@@ -448,7 +396,7 @@ constexpr Form kForm[2][kForms] = {{{1, 4, 1}, {2, 2, 2}, {4, 1, 4}}, {{1, 4, 1}
 
 struct Plan {
     int form = -1;
-    Strips strips;
+    exhip_strips strips;
     double time = 0;  // us
 };
 
@@ -469,7 +417,7 @@ Plan choose(int dt, const PwParams& p, long long images, int subs, int kblocks) 
     Plan best;
     for (int i = 0; i < kForms; ++i) {
         const Form& f = kForm[p.stride - 1][i];
-        const Strips s = choose_strips(p, images, f.run(), most_staged(f.pitch()));
+        const exhip_strips s = exhip_choose_strips(p.out_h, p.out_w, p.stride, images, f.run(), most_staged(f.pitch()));
         const int lds = (f.lds(dt, s.staged) + 1279) / 1280 * 1280;
         if (lds > kLdsLimit) continue;
         const long long groups = s.tiles * ((kblocks + 1) / 2), slots = 256ll * std::min(kLdsLimit / lds, 3), full = groups / slots;
@@ -491,20 +439,14 @@ Plan choose(int dt, const PwParams& p, long long images, int subs, int kblocks) 
 }
 
 template <int DT, int S, int WK, int WP, int SUBS>
-int go(exhip_ctx* ctx, StagedParams& q, long long images, int kblocks, const Strips& s) {
+int go(exhip_ctx* ctx, StagedParams& q, long long images, int kblocks, const exhip_strips& s) {
     constexpr int MT = kMt, NT = kNt, WAVES = WK * WP;
     PwParams& p = q.f;
     q.chunks = (q.subs + SUBS - 1) / SUBS;
     q.table_b = (s.staged * 4 + 15) / 16 * 16;
     const int lds = Form{WK, WP, SUBS}.lds(DT, s.staged);
     if (lds > kLdsLimit) return EXHIP_ERR_UNSUPPORTED;
-    q.strip_w = (unsigned)s.width;
-    q.strips = (unsigned)s.count;
-    q.total = (unsigned)((long long)s.width * s.count * p.out_h * images);
-    q.staged_rows = (p.out_h - 1) * S + 3;
-    q.staged_cols = (s.width - 1) * S + 3;
-    q.by_strip_w.set((unsigned)s.width); q.by_strips.set((unsigned)s.count); q.by_height.set((unsigned)p.out_h);
-    q.by_rows.set((unsigned)q.staged_rows); q.by_cols.set((unsigned)q.staged_cols);
+    q.list.set(s, p.out_h, S, images);
     p.ch_groups = (unsigned)((kblocks + MT - 1) / MT);
     q.by_groups.set(p.ch_groups);
     const long long items = s.tiles * p.ch_groups;
@@ -534,7 +476,7 @@ int go(exhip_ctx* ctx, StagedParams& q, long long images, int kblocks, const Str
 }
 
 template <int DT, int S, int FORM>
-int go_form(exhip_ctx* ctx, StagedParams& q, long long images, int kblocks, const Strips& s) {
+int go_form(exhip_ctx* ctx, StagedParams& q, long long images, int kblocks, const exhip_strips& s) {
     constexpr Form f = kForm[S - 1][FORM];
     return go<DT, S, f.wk, f.wp, f.subs>(ctx, q, images, kblocks, s);
 }
@@ -629,7 +571,7 @@ int exhip_conv3x3_staged(exhip_ctx* ctx, int dt, const void* pw_params, long lon
     if (option > 1) {
         plan.form = std::min(option - 2, kForms - 1);
         const Form& f = kForm[p.stride - 1][plan.form];
-        plan.strips = choose_strips(p, images, f.run(), most_staged(f.pitch()));
+        plan.strips = exhip_choose_strips(p.out_h, p.out_w, p.stride, images, f.run(), most_staged(f.pitch()));
     } else {
         plan = plan_of(dt, p, images, subs, kblocks);
         if (plan.form < 0) return EXHIP_ERR_UNSUPPORTED;

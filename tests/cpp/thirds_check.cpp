@@ -23,8 +23,8 @@ bool small_maps() {
                         const Plan plan = plan_of(p, images, 2, tile);
                         ++plans;
                         const Sizes s(kForm[plan.form]);
-                        if (s.lds(plan.staged, csteps > kForm[plan.form].cs ? 2 : 1) > kLdsLimit)
-                            return printf("%lld images of %d x %d, %d steps, option %d: %d pixels staged in form %d\n", images, h, w, csteps, tile, plan.staged, plan.form), false;
+                        if (s.lds(plan.strips.staged, csteps > kForm[plan.form].cs ? 2 : 1) > kLdsLimit)
+                            return printf("%lld images of %d x %d, %d steps, option %d: %d pixels staged in form %d\n", images, h, w, csteps, tile, plan.strips.staged, plan.form), false;
                     }
                 }
     printf("%lld plans\n", plans);
