@@ -753,7 +753,7 @@ static int run_conv_f32(exhip_ctx* ctx, const exhip_conv_desc* d, const exhip_co
         p.y_nchw = y_nchw ? y_nchw + n0 * per_image * d->k : nullptr;
         // 1x1 layers of whole 64-byte pieces take the pixels in pairs of steps: 512 -> 256 on one 20 x 20 map 6.05 -> 5.44 us, 1024 -> 512 on
         // three 13 x 13 maps 9.1 -> 8.3. With a filter the products bound the chain, and the detour through LDS only lengthens it
-        // (64 -> 64 3x3 on one 160 x 160 map 23.6 us, 25.2 in pairs, 15.4 in thirds).
+        // (64 -> 64 3x3 on one 160 x 160 map 23.6 us, 25.2 in pairs, 18.8 in thirds).
         const bool point = d->kh == 1 && d->kw == 1 && !d->pt && !d->pb && !d->pl && !d->pr;
         const int go_rc = thirds                ? exhip_conv_f32_thirds_run(ctx, {&p, n, write_blocks})
                           : pair                  ? pick<kPair, false>(ctx, p, write_blocks)

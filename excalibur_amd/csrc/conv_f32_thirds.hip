@@ -17,14 +17,15 @@
 // A group's pixels are neighbours in a list of the output's vertical strips, row by row (strips.h; a strip of a 13 x 13 map is the map). WK waves share a run's
 // steps, their sums meet in LDS in a fixed order.
 //
-// Bounded by the matrix unit on large maps (128 -> 128 at 16 x 80 x 80 183 us, 165 TFLOP/s of float32 work, conv_f32_kernel 223) and by a group's chain of
-// loads, split and products on small ones: us, conv_f32_kernel and this one, launches queued from Python, 64 -> 64 on one 56 x 56 map 6.7, 5.5, at 160 x 160 23.5, 18.6,
-// 128 -> 128 at 80 x 80 22.5, 17.7, 512 -> 512 at 20 x 20 24.8, 21.4; over 62 layers 1.08 times as fast on average (with six products 1.20).
+// Bounded by the matrix unit on large maps (128 -> 128 at 16 x 80 x 80 185 us, 164 TFLOP/s of float32 work, conv_f32_kernel 226) and by a group's chain of
+// loads, split and products on small ones: us, conv_f32_kernel and this one, launches queued from Python, 64 -> 64 on one 56 x 56 map 6.7, 5.4, at 160 x 160 23.4, 18.8,
+// 128 -> 128 at 80 x 80 22.5, 17.8, 512 -> 512 at 20 x 20 24.9, 19.1. Over 62 layers 1.13 times as fast on average, 1.58 at most (112 -> 16 at 22 x 78 x 76), and
+// slower where there is little to split for: maps of one pixel .78 to .84, 16 channels in a few groups .80 to .84, launches of a few groups .92 to .95.
 //
 // What thirds do not hold: a third of an infinity is NaN, as is one times the zero third of a finite weight; below 2^-103 a last third is no normal number, below
 // 2^-110 it is cut off, and products below 2^-112 lose their smaller parts. A group that stages a value or finds a sum of that kind computes its
 // tile again with float32 products (float32_sums), whose results it gets, all of them; a weight of that kind is packed as a NaN that calls for them (split_weight).
-// Such a group takes 2.5 to 4 times as long.
+// Such a group takes 2.5 to 3.5 times as long (512 -> 512 at 20 x 20 all NaN 64 us, 128 -> 128 at 4 x 80 x 80 54 -> 184 to 199).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -573,10 +574,8 @@ private:
 
 // The form that a model of the launch says is shortest, in microseconds: 2.5 for the launch; per round of groups on 256 CUs 1.5 for a group's
 // start, 0.2 for every four channels of a pixel that a thread finishes and 0.09 for every chunk; the products at 0.019 each, all of a SIMD's or
-// a group's where it is alone; or the weights at 14.6 TB/s where that is longer. Its constants are fitted to 83 layers from 1 x 11 x 11 to 37
-// GFLOP in these forms (11 % off on average); its choice is 2 % slower than the fastest on average, and 1.49 times as fast as the float32
-// products (conv_f32_kernel), which no more than noise beats anywhere. Wave tiles of 64 x 64, 32 x 64 and eight waves to 64 x 32 or 64 x 64 are
-// within 3 % of these or slower on all of the layers but four.
+// a group's where it is alone; or the weights at 14.6 TB/s where that is longer. Its choice is 1.5 % slower than the fastest of these forms on average, over 62 layers
+// from 1 x 11 x 11 to 37 GFLOP.
 int choose_form(const F32Params& p, long long pixels, int kblocks) {
     int best = 0;
     double best_cost = 0;

@@ -242,8 +242,9 @@ int exhip_dw_pw_f16(exhip_ctx* ctx, const exhip_depthwise_desc* dw, const exhip_
 int exhip_bottleneck_f16(exhip_ctx* ctx, const exhip_conv_desc* first, const void* w_first, const float* bias_first, const exhip_depthwise_desc* dw,
                          const exhip_conv_desc* last, const void* w_last, const float* bias_last, const uint16_t* residual_nhwc, uint16_t* y_nhwc);
 
-/* Two layers of which neither reads what the other writes: the values of exhip_conv2d_i8 / exhip_conv2d_f16 for each, pointwise ones with the same kind of
- * layers behind them in one launch. An error is that of the first layer that has one; the other may have run. */
+/* Two layers of which neither reads what the other writes: the values of exhip_conv2d_i8 / exhip_conv2d_f16 for each, in one launch where both are pointwise
+ * and have behind them, int8: a BatchNorm with LeakyReLU and int8 results; fp16: nothing, not even an activation. Two launches otherwise.
+ * An error is that of the first layer that has one; the other may have run. */
 typedef struct exhip_conv_i8_call {
     const exhip_conv_desc* d;
     const int8_t* x;
