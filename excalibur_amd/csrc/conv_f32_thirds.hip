@@ -20,7 +20,7 @@
 // Bounded by the matrix unit on large maps (128 -> 128 at 16 x 80 x 80 185 us, 164 TFLOP/s of float32 work, conv_f32_kernel 226) and by a group's chain of
 // loads, split and products on small ones: us, conv_f32_kernel and this one, launches queued from Python, 64 -> 64 on one 56 x 56 map 6.7, 5.4, at 160 x 160 23.4, 18.8,
 // 128 -> 128 at 80 x 80 22.5, 17.8, 512 -> 512 at 20 x 20 24.9, 19.1. Over 62 layers 1.13 times as fast on average, 1.58 at most (112 -> 16 at 22 x 78 x 76), and
-// slower where there is little to split for: maps of one pixel .78 to .84, 16 channels in a few groups .80 to .84, launches of a few groups .92 to .95.
+// slower where there is little to split for: maps of one pixel .79 to .85, 16 channels in a few groups .81 to .87, 32 and 80 channels there .92 to .99.
 //
 // What thirds do not hold: a third of an infinity is NaN, as is one times the zero third of a finite weight; below 2^-103 a last third is no normal number, below
 // 2^-110 it is cut off, and products below 2^-112 lose their smaller parts. A group that stages a value or finds a sum of that kind computes its
@@ -565,8 +565,12 @@ struct Sizes {
     explicit Sizes(const Shape& f) : run(32 * f.nt * f.wp), pitch(f.cs * 96 + 16), waves(f.wk * f.wp), f_(f) {}
     int table_bytes(int staged) const { return ((run + kParams * f_.mt * 32 + 4 + staged) * 4 + 15) / 16 * 16; }
     int lds(int staged, int buffers) const { return table_bytes(staged) + std::max((staged + 1) * pitch * buffers, waves * f_.mt * f_.nt * 4096); }
-    // staged pixels with which as many groups share a CU as its registers allow
-    int most(int buffers) const { return (kLdsLimit / std::max(f_.occ * 4 / waves, 1) - table_bytes(0) - 16 - pitch * buffers) / (pitch * buffers + 4); }
+    // staged pixels with which as many of `items` groups share a CU as its registers allow. With room for three where a CU gets one, strips were so narrow that the columns
+    // a map does not have made a second round: 128 -> 128 at 3 x 26 x 26 264 groups for 256, 10.1 us, now 8.2; 512 -> 512 at 3 x 13 x 13 29.5, now 24.8.
+    int most(int buffers, long long items) const {
+        const int resident = (int)std::min<long long>(std::max(f_.occ * 4 / waves, 1), (items + 255) / 256);
+        return (kLdsLimit / resident - table_bytes(0) - 16 - pitch * buffers) / (pitch * buffers + 4);
+    }
 
 private:
     const Shape f_;
@@ -582,8 +586,8 @@ int choose_form(const F32Params& p, long long pixels, int kblocks) {
     for (int i = 0; i < kForms; ++i) {
         const Shape& f = kForm[i];
         const int waves = f.wk * f.wp, blocks = f.mt * f.nt, steps = (p.csteps + f.wk - 1) / f.wk, units = std::max(1, blocks * 4 / f.wk);
-        const int resident = std::max(1, f.occ * 4 / waves), slots = waves > 4 ? 240 : 256;  // (256 groups of eight waves took a second round)
-        const long long items = (pixels + 32 * f.nt * f.wp - 1) / (32 * f.nt * f.wp) * ((kblocks + f.mt - 1) / f.mt), each = (items + slots - 1) / slots;
+        const int resident = std::max(1, f.occ * 4 / waves);
+        const long long items = (pixels + 32 * f.nt * f.wp - 1) / (32 * f.nt * f.wp) * ((kblocks + f.mt - 1) / f.mt), each = (items + 255) / 256;
         const double products = steps * 9 * blocks * 8 * 0.0191, rounds = (double)((each + resident - 1) / resident);
         const double time = rounds * (1.5 + 0.2 * units + 0.09 * ((p.csteps + f.cs - 1) / f.cs - 1)) + std::max(each * (waves / 4) * products, rounds * products);
         const double cost = std::max(time, (double)items * f.mt * p.csteps * kStepBytes / 14.6e6);
@@ -613,8 +617,9 @@ const Plan& plan_of(const F32Params& p, long long images, int kblocks, int tile)
         for (int tries = 0; tries < 3; ++tries) {
             const int form = tries ? 0 : chosen, buffers = p.csteps > kForm[form].cs ? 2 : 1;
             const Sizes s(kForm[form]);
+            const long long groups = (kblocks + kForm[form].mt - 1) / kForm[form].mt, items = ((long long)p.out_h * p.out_w * images + s.run - 1) / s.run * groups;
             e.plan.form = form;
-            e.plan.strips = exhip_choose_strips(p.out_h, p.out_w, 1, images, s.run, s.most(buffers), tries == 2);
+            e.plan.strips = exhip_choose_strips(p.out_h, p.out_w, 1, images, s.run, s.most(buffers, items), groups, tries == 2);
             if (s.lds(e.plan.strips.staged, buffers) <= kLdsLimit) break;
         }
         e.images = images;

@@ -418,7 +418,7 @@ Plan choose(int dt, const PwParams& p, long long images, int subs, int kblocks) 
     Plan best;
     for (int i = 0; i < kForms; ++i) {
         const Form& f = kForm[p.stride - 1][i];
-        const exhip_strips s = exhip_choose_strips(p.out_h, p.out_w, p.stride, images, f.run(), most_staged(f.pitch()));
+        const exhip_strips s = exhip_choose_strips(p.out_h, p.out_w, p.stride, images, f.run(), most_staged(f.pitch()), 0);
         const int lds = (f.lds(dt, s.staged) + 1279) / 1280 * 1280;
         if (lds > kLdsLimit) continue;
         const long long groups = s.tiles * ((kblocks + 1) / 2), slots = 256ll * std::min(kLdsLimit / lds, 3), full = groups / slots;
@@ -572,7 +572,7 @@ int exhip_conv3x3_staged(exhip_ctx* ctx, int dt, const void* pw_params, long lon
     if (option > 1) {
         plan.form = std::min(option - 2, kForms - 1);
         const Form& f = kForm[p.stride - 1][plan.form];
-        plan.strips = exhip_choose_strips(p.out_h, p.out_w, p.stride, images, f.run(), most_staged(f.pitch()));
+        plan.strips = exhip_choose_strips(p.out_h, p.out_w, p.stride, images, f.run(), most_staged(f.pitch()), 0);
     } else {
         plan = plan_of(dt, p, images, subs, kblocks);
         if (plan.form < 0) return EXHIP_ERR_UNSUPPORTED;

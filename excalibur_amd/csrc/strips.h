@@ -13,8 +13,9 @@ struct exhip_strips {
 };
 
 // The strips for runs of `run` pixels: of all widths that split the map evenly the one whose runs, weighed with what they stage, are least, among those of at most `most`
-// staged pixels where there are any. `wide`: strips of a column that does not exist beside the map's only one.
-inline exhip_strips exhip_choose_strips(int out_h, int out_w, int stride, long long images, int run, int most, bool wide = false) {
+// staged pixels where there are any. `groups`: of each run, where what counts is the runs that one of 256 CUs gets (0: all of them). `wide`: strips of a column that does
+// not exist beside the map's only one.
+inline exhip_strips exhip_choose_strips(int out_h, int out_w, int stride, long long images, int run, int most, long long groups, bool wide = false) {
     exhip_strips best;
     double best_cost = 0;
     for (int width = wide ? 2 : out_w;;) {
@@ -25,7 +26,7 @@ inline exhip_strips exhip_choose_strips(int out_h, int out_w, int stride, long l
         const int rows = run % width == 0 ? run / width - 1 : (run + width - 2) / width;
         const int crossed = (int)std::min<long long>((rows + out_h - 1) / out_h, images * count - 1);
         const int staged = (rows * stride + crossed * (3 - stride) + 3) * ((width - 1) * stride + 3);
-        const double cost = (staged > most ? 1e18 * staged : 0.) + (double)tiles * (run + 0.2 * staged);
+        const double cost = (staged > most ? 1e18 * staged : 0.) + (double)(groups ? (tiles * groups + 255) / 256 : tiles) * (run + 0.2 * staged);
         if (best.width == 0 || cost < best_cost) {
             best.width = width; best.count = count; best.staged = staged; best.tiles = tiles;
             best_cost = cost;

@@ -1,5 +1,5 @@
-// The float32 kernel of bfloat16 thirds on the CPU: every layer of maps up to 40 x 40 has a form whose staged pixels LDS holds; and every load of every form, over
-// all channel counts from 16 to 512, lies inside its operand.
+// The float32 kernel of bfloat16 thirds on the CPU: every layer of maps up to 40 x 40 has a form whose staged pixels LDS holds, and as few groups as a CU each where
+// its pixels are that few; and every load of every form, over all channel counts from 16 to 512, lies inside its operand.
 #include <strict.h>
 #include <sys/mman.h>
 
@@ -29,6 +29,34 @@ bool small_maps() {
                 }
     printf("%lld plans\n", plans);
     return true;
+}
+
+// Strips of columns that a map does not have make runs: not more of them than there are CUs where the pixels alone need no more and strips that divide the map lie in LDS.
+bool one_round() {
+    int layers = 0;
+    for (int h = 8; h <= 64; ++h)
+        for (int w = h - 3; w <= h + 3; ++w)
+            for (int images = 1; images <= 4; ++images)
+                for (int kblocks : {1, 2, 4, 8, 16})
+                    for (int tile = 1; tile <= kForms; ++tile) {
+                        F32Params p = {};
+                        p.out_h = h; p.out_w = w; p.csteps = 8;
+                        const Plan plan = plan_of(p, images, kblocks, tile);
+                        const Shape& f = kForm[plan.form];
+                        const Sizes s(f);
+                        const long long groups = (kblocks + f.mt - 1) / f.mt, runs = ((long long)h * w * images + s.run - 1) / s.run;
+                        bool fits = false;
+                        for (int width = 4; width <= w; ++width) {
+                            const int rows = (s.run + width - 2) / width, staged = (rows + (rows + h - 1) / h * 2 + 3) * (width + 2);
+                            fits |= w % width == 0 && s.lds(staged, p.csteps > f.cs ? 2 : 1) <= kLdsLimit;
+                        }
+                        if (!fits || runs * groups > 256) continue;
+                        ++layers;
+                        if (plan.strips.tiles * groups > 256)
+                            return printf("%d images of %d x %d, %d blocks, form %d: %lld groups for %lld\n", images, h, w, kblocks, plan.form, plan.strips.tiles * groups, runs * groups), false;
+                    }
+    printf("%d layers of one round\n", layers);
+    return layers > 1000;
 }
 
 // `count` values whose last one is the last before an unreadable page
@@ -65,7 +93,7 @@ bool layer(int n, int h, int w, int c, int k, int tile, bool twice) {
 }  // namespace
 
 int main() {
-    if (!small_maps()) return 1;
+    if (!small_maps() || !one_round()) return 1;
     for (int tile = 1; tile <= kForms; ++tile)
         for (int c = 16; c <= 512; c += 16)
             if (!layer(c % 5 == 1 ? 2 : 1, 3, c % 3 ? 5 : 4, c, c % 7 ? 40 : 64, tile, false) || (c % 48 == 32 && (!layer(2, 3, 4, c, 40, tile, true) || !layer(33, 1, 1, c, 40, tile, false)))) return 1;  // (twice: sums that thirds do not hold)
