@@ -578,7 +578,7 @@ private:
 
 // The form that a model of the launch says is shortest, in microseconds: 2.5 for the launch; per round of groups on 256 CUs 1.5 for a group's
 // start, 0.2 for every four channels of a pixel that a thread finishes and 0.09 for every chunk; the products at 0.019 each, all of a SIMD's or
-// a group's where it is alone; or the weights at 14.6 TB/s where that is longer. Its choice is 1.5 % slower than the fastest of these forms on average, over 62 layers
+// a group's where it is alone; or the weights at 14.6 TB/s where that is longer. Its choice is 1 % slower than the fastest of these forms on average, over 62 layers
 // from 1 x 11 x 11 to 37 GFLOP.
 int choose_form(const F32Params& p, long long pixels, int kblocks) {
     int best = 0;
